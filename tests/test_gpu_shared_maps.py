@@ -1,0 +1,87 @@
+"""What layers leave on a map for the layers after them (tile plan, rows forms, re-ordered lists): read from a
+stream other than the one that made it, while that one is still busy, and from inside a captured graph."""
+import numpy as np
+import pytest
+import torch
+
+from helpers import kaiming_weight, normal_features
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def _surface(n, seed):
+    """n distinct voxels of three planes that meet, in random order."""
+    side = int(np.ceil(np.sqrt(n / 2.0))) + 2
+    uv = np.stack(np.meshgrid(np.arange(side), np.arange(side), indexing="ij"), -1).reshape(-1, 2)
+    z = np.zeros((len(uv), 1), dtype=np.int64)
+    c = np.unique(np.concatenate([np.hstack([uv, z]), np.hstack([uv[:, :1], z, uv[:, 1:]]), np.hstack([z, uv])]), axis=0)
+    c = c[np.random.default_rng(seed).permutation(len(c))[:n]]
+    return torch.as_tensor(np.hstack([np.zeros((len(c), 1), dtype=np.int64), c]).astype(np.int32), device=DEV)
+
+
+def _map(c, out=None, stride=1, ksize=3):
+    from warpconvnet_amd.geometry.coords.search.torch_discrete import generate_kernel_map
+    return generate_kernel_map(c, c if out is None else out, (stride,) * 3, (ksize,) * 3)
+
+
+def _occupy(big):
+    """Some 10 ms of work in front of whatever the current stream is given next."""
+    for _ in range(8):
+        big = torch.mm(big, big)
+    return big
+
+
+def _on_two_streams(call):
+    """call() behind a long queue on one stream, and at once on another: both results."""
+    big = torch.zeros(8192, 8192, device=DEV)
+    a, b = torch.cuda.Stream(), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(a):
+        _occupy(big)
+        first = call()
+    assert not a.query()  # still busy
+    with torch.cuda.stream(b):
+        second = call()
+    torch.cuda.synchronize()
+    return first, second
+
+
+def test_a_tile_plan_serves_layers_on_other_streams():
+    from warpconvnet_amd._lib import lib
+    from warpconvnet_amd.nn.functional.sparse_conv import sparse_conv_forward
+    c = _surface(40_000, 1)
+    n, km = len(c), _map(c)
+    x = normal_features(n, 128, seed=1, dtype=torch.float16).to(DEV)
+    w = kaiming_weight(27, 128, 256, seed=2, dtype=torch.float16).to(DEV)
+    want = sparse_conv_forward(x, w, _map(c.clone()), n)
+    assert lib().wcn_conv_last_kernel().decode().startswith("conv_fwd_tiles<")
+    for got in _on_two_streams(lambda: sparse_conv_forward(x, w, km, n)):
+        assert torch.equal(got, want)
+    assert km._tile_plan is not None
+
+
+def test_a_tile_plan_in_a_captured_graph():
+    """A plan made before the capture, on another stream, is read by the graph; one that would be made inside the
+    capture stays the graph's own.  Every replay gives the eager result."""
+    from warpconvnet_amd.nn.functional.sparse_conv import sparse_conv_forward
+    c = _surface(40_000, 3)
+    n = len(c)
+    x = normal_features(n, 128, seed=1, dtype=torch.float16).to(DEV)
+    w = kaiming_weight(27, 128, 256, seed=2, dtype=torch.float16).to(DEV)
+    for planned in (True, False):
+        km = _map(c)
+        if planned:
+            sparse_conv_forward(x, w, km, n)
+            assert km._tile_plan is not None
+        graph = torch.cuda.CUDAGraph()
+        torch.cuda.synchronize()
+        with torch.cuda.graph(graph):
+            out = sparse_conv_forward(x, w, km, n)
+        assert (km._tile_plan is not None) == planned
+        for i in range(3):
+            x.copy_(normal_features(n, 128, seed=10 + i, dtype=torch.float16))
+            want = sparse_conv_forward(x, w, _map(c), n)
+            graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(out, want), (planned, i)

@@ -9,6 +9,7 @@
 #include <torch/csrc/autograd/function.h>
 #include <torch/csrc/autograd/functions/utils.h>
 #include <torch/csrc/autograd/saved_variable.h>
+#include <c10/core/impl/VirtualGuardImpl.h>
 #include <c10/hip/HIPStream.h>
 #include <hip/hip_runtime_api.h>
 
@@ -52,6 +53,49 @@ int dtype_code(at::ScalarType t) {
 Tensor bytes_on(size_t n, const Tensor& like) {
   return at::empty({static_cast<int64_t>(n < 256 ? 256 : n)}, at::TensorOptions().dtype(at::kByte).device(like.device()));
 }
+
+/* Where a piece of device data that outlives its call was made, and the event behind the kernels that made it.  A call on
+ * another stream waits for them, and the allocator learns of that stream, so that memory given back by the object is not
+ * handed out again while that stream still reads it.  What is made inside a capture is kept by nobody: its
+ * kernels run when the graph is replayed, not now. */
+struct MadeOn {
+  void* stream;
+  hipEvent_t event = nullptr;
+  explicit MadeOn(void* s) : stream(s) {
+    if (hipEventCreateWithFlags(&event, hipEventDisableTiming) != hipSuccess ||
+        hipEventRecord(event, static_cast<hipStream_t>(s)) != hipSuccess) {
+      if (event) (void)hipEventDestroy(event);
+      throw std::runtime_error("an event behind kept device data could not be recorded");
+    }
+  }
+  MadeOn(const MadeOn&) = delete;
+  ~MadeOn() { (void)hipEventDestroy(event); }
+
+  static bool capturing(void* s) {
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    return hipStreamIsCapturing(static_cast<hipStream_t>(s), &status) == hipSuccess && status != hipStreamCaptureStatusNone;
+  }
+
+  // `data` is about to be read by work on the current stream of its device
+  void before_use(std::initializer_list<const Tensor*> data) const {
+    const Tensor& first = **data.begin();
+    void* s = stream_of(first);
+    if (s == stream) return;
+    if (!capturing(s)) {
+      if (hipStreamWaitEvent(static_cast<hipStream_t>(s), event, 0) != hipSuccess)
+        throw std::runtime_error("hipStreamWaitEvent failed");
+    } else {  // a graph cannot wait for work outside it: the host does
+      hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+      (void)hipThreadExchangeStreamCaptureMode(&mode);
+      const hipError_t waited = hipEventSynchronize(event);
+      (void)hipThreadExchangeStreamCaptureMode(&mode);
+      if (waited != hipSuccess) throw std::runtime_error("hipEventSynchronize failed");
+    }
+    const c10::Stream reader = c10::impl::VirtualGuardImpl(first.device().type()).getStream(first.device());
+    for (const Tensor* t : data)
+      if (t->defined()) t->record_stream(reader);
+  }
+};
 
 std::string shape_text(const Tensor& t) {
   std::string s = "(";
@@ -322,7 +366,7 @@ Tensor prepared_tiles(const py::object& weight_obj, const Tensor& weight, const 
 }
 
 /* Tile plan of a builder's map (wcn_tile_plan_build), kept on the map object: the layers over a map share
- * it.  Undefined where another contraction is to be taken, or the map is none the plan can be made from.  Where the plan
+ * it, on whichever stream they run.  Undefined where another contraction is to be taken, or the map is none the plan can be made from.  Where the plan
  * does not pay for itself in the calls that are known to come it is made for the second layer that would use it. */
 Tensor tile_plan(const py::object& km, const MapRef& map, int64_t n_in, int64_t num_out, int code, int32_t c_in, int32_t c_out,
                  int32_t calls) {
@@ -332,7 +376,11 @@ Tensor tile_plan(const py::object& km, const MapRef& map, int64_t n_in, int64_t 
   py::object kept = km.attr("_tile_plan");
   if (!kept.is_none()) {
     py::tuple t = kept.cast<py::tuple>();
-    if (t[1].cast<int64_t>() == n_in && t[2].cast<int64_t>() == num_out) return t[0].cast<Tensor>();
+    if (t[1].cast<int64_t>() == n_in && t[2].cast<int64_t>() == num_out) {
+      const Tensor plan = t[0].cast<Tensor>();
+      t[3].cast<const MadeOn*>()->before_use({&plan});
+      return plan;
+    }
   }
   py::object dev = km.attr("_device_offsets");
   if (dev.is_none() || !flag(km, "_out_ascend") || !flag(km, "_from_builder")) return Tensor();
@@ -343,14 +391,15 @@ Tensor tile_plan(const py::object& km, const MapRef& map, int64_t n_in, int64_t 
     km.attr("_tiles_wanted") = true;
     return Tensor();
   }
+  void* stream = stream_of(map.in_maps);
   const Tensor plan = bytes_on(wcn_tile_plan_bytes(num_out, map.K), map.in_maps);
   const Tensor ws = bytes_on(wcn_tile_plan_workspace_bytes(num_out, map.K, map.pairs()), map.in_maps);
   check(wcn_tile_plan_build(map.in_maps.const_data_ptr<int32_t>(), map.out_maps.const_data_ptr<int32_t>(),
                             dev.cast<Tensor>().const_data_ptr<int64_t>(), groups, map.K, static_cast<int32_t>(map.identity),
                             n_in, num_out, map.pairs(), plan.mutable_data_ptr(), static_cast<size_t>(plan.numel()),
-                            ws.mutable_data_ptr(), static_cast<size_t>(ws.numel()), stream_of(map.in_maps)),
+                            ws.mutable_data_ptr(), static_cast<size_t>(ws.numel()), stream),
         "wcn_tile_plan_build");
-  km.attr("_tile_plan") = py::make_tuple(plan, n_in, num_out);
+  if (!MadeOn::capturing(stream)) km.attr("_tile_plan") = py::make_tuple(plan, n_in, num_out, std::make_shared<MadeOn>(stream));
   return plan;
 }
 
@@ -1040,6 +1089,7 @@ Tensor pool_autograd(const Tensor& features, const py::object& km, int64_t num_o
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
+  py::class_<MadeOn, std::shared_ptr<MadeOn>>(m, "MadeOn");
   py::class_<PreparedWeight, std::shared_ptr<PreparedWeight>>(m, "PreparedWeight");
   m.def("batch_rows", &batch_rows);
   m.def("table_build", &table_build);

@@ -48,7 +48,7 @@ class IntSearchResult:
     _keys_unique = False
     # rows forms made of the map (csrc/wcn_host.cpp: rows_form), by what they group
     _rows_forms = None
-    # tile plan of the contraction (csrc/wcn_host.cpp: tile_plan): (plan, rows in, rows out)
+    # tile plan of the contraction (csrc/wcn_host.cpp: tile_plan): (plan, rows in, rows out, where and when made)
     _tile_plan = None
     _forward_map = None    # the map this one is the exchange of (a transposed convolution's)
     _tiles_wanted = False  # a layer has been over the map that would have used the plan
