@@ -85,3 +85,26 @@ def test_a_tile_plan_in_a_captured_graph():
             graph.replay()
             torch.cuda.synchronize()
             assert torch.equal(out, want), (planned, i)
+
+
+def test_rows_forms_serve_layers_on_other_streams():
+    from warpconvnet_amd.geometry.coords.ops.stride import stride_coords
+    from warpconvnet_amd.nn.functional.sparse_conv_depth import spatially_sparse_depthwise_conv
+    c = _surface(40_000, 5)
+    coarse = stride_coords(c, (2, 2, 2))[0]
+    n, m = len(c), len(coarse)
+    x = normal_features(n, 32, seed=1, dtype=torch.float16).to(DEV)
+    w = kaiming_weight(8, 32, 1, seed=2, dtype=torch.float16)[..., 0].to(DEV)
+    gy = normal_features(m, 32, seed=3, dtype=torch.float16).to(DEV)
+
+    def step(km):  # the forward reads the form by output row, the input gradient the one by input row
+        xg = x.clone().requires_grad_(True)
+        out = spatially_sparse_depthwise_conv(xg, w, km, m)
+        out.backward(gy)
+        return out.detach(), xg.grad
+
+    want = step(_map(c, coarse, 2, 2))
+    km = _map(c.clone(), coarse, 2, 2)
+    for got in _on_two_streams(lambda: step(km)):
+        assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+    assert len(km._rows_forms) == 2

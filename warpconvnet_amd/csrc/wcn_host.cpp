@@ -800,7 +800,7 @@ Tensor conv_autograd(const Tensor& features, const py::object& weight_obj, const
 
 /* The rows form of a map (wcn_map_rows_build) by output row or, with the lists exchanged, by input row.
  * It depends on the map alone and is kept on the map object: the layers and the backward passes that
- * share a map share it.  A builder's map comes with what the one-pass build reads. */
+ * share a map share it, on whichever stream they run.  A builder's map comes with what the one-pass build reads. */
 Tensor rows_form(const py::object& km, const MapRef& map, bool by_out, int64_t num_rows) {
   const Tensor &gathered = by_out ? map.in_maps : map.out_maps, &grouping = by_out ? map.out_maps : map.in_maps;
   py::object kept = km.attr("_rows_forms");
@@ -811,8 +811,14 @@ Tensor rows_form(const py::object& km, const MapRef& map, bool by_out, int64_t n
   py::dict forms = kept.cast<py::dict>();
   const py::tuple key = py::make_tuple(reinterpret_cast<uintptr_t>(grouping.const_data_ptr()),
                                        reinterpret_cast<uintptr_t>(gathered.const_data_ptr()), num_rows);
-  if (forms.contains(key)) return forms[key].cast<Tensor>();
+  if (forms.contains(key)) {
+    py::tuple t = forms[key].cast<py::tuple>();
+    const Tensor rows = t[0].cast<Tensor>();
+    t[1].cast<const MadeOn*>()->before_use({&rows});
+    return rows;
+  }
   const int64_t pairs = map.pairs();
+  void* stream = stream_of(gathered);
   const Tensor ws = bytes_on(wcn_map_rows_workspace_bytes(num_rows, map.K, pairs), gathered);
   const int32_t* groups = nullptr;
   py::object dev = km.attr("_device_offsets");
@@ -821,13 +827,13 @@ Tensor rows_form(const py::object& km, const MapRef& map, bool by_out, int64_t n
   if (groups)
     check(wcn_map_rows_build_grouped(gathered.const_data_ptr<int32_t>(), grouping.const_data_ptr<int32_t>(),
                                      dev.cast<Tensor>().const_data_ptr<int64_t>(), groups, map.K, num_rows, pairs,
-                                     ws.mutable_data_ptr(), static_cast<size_t>(ws.numel()), stream_of(gathered)),
+                                     ws.mutable_data_ptr(), static_cast<size_t>(ws.numel()), stream),
           "wcn_map_rows_build_grouped");
   else
     check(wcn_map_rows_build(gathered.const_data_ptr<int32_t>(), grouping.const_data_ptr<int32_t>(), map.host_offsets(),
-                             map.K, num_rows, ws.mutable_data_ptr(), static_cast<size_t>(ws.numel()), stream_of(gathered)),
+                             map.K, num_rows, ws.mutable_data_ptr(), static_cast<size_t>(ws.numel()), stream),
           "wcn_map_rows_build");
-  forms[key] = ws;
+  if (!MadeOn::capturing(stream)) forms[key] = py::make_tuple(ws, std::make_shared<MadeOn>(stream));
   return ws;
 }
 

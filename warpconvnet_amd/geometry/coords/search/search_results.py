@@ -46,7 +46,7 @@ class IntSearchResult:
     # pairs come from one look-up per (offset, output row) / over a table that reported no repeated key
     _from_builder = False
     _keys_unique = False
-    # rows forms made of the map (csrc/wcn_host.cpp: rows_form), by what they group
+    # rows forms made of the map (csrc/wcn_host.cpp: rows_form), by what they group, each with where and when it was made
     _rows_forms = None
     # tile plan of the contraction (csrc/wcn_host.cpp: tile_plan): (plan, rows in, rows out, where and when made)
     _tile_plan = None
