@@ -108,3 +108,27 @@ def test_rows_forms_serve_layers_on_other_streams():
     for got in _on_two_streams(lambda: step(km)):
         assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
     assert len(km._rows_forms) == 2
+
+
+def test_reordered_lists_serve_layers_on_other_streams():
+    """The lists by output row of a map made by hand, and those by input row for its input gradient."""
+    from warpconvnet_amd.geometry.coords.search.search_results import IntSearchResult
+    from warpconvnet_amd.nn.functional.sparse_conv import sparse_conv_backward, sparse_conv_forward
+    c = _surface(40_000, 7)
+    n, km = len(c), _map(c)
+    x = normal_features(n, 64, seed=1, dtype=torch.float16).to(DEV)
+    w = kaiming_weight(27, 64, 64, seed=2, dtype=torch.float16).to(DEV)
+
+    def by_hand():  # the pairs of a symmetric map with in and out exchanged, and no word of their order
+        m = IntSearchResult(km.out_maps, km.in_maps, km.offsets, km.identity_map_index)
+        m._from_builder = m._keys_unique = True
+        return m
+
+    def step(m):
+        return sparse_conv_forward(x, w, m, n), sparse_conv_backward(x, x, w, m, need_weight_grad=False)[0]
+
+    want = step(by_hand())
+    shared = by_hand()
+    for got in _on_two_streams(lambda: step(shared)):
+        assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
+    assert shared._by_out is not None and shared._by_in is not None

@@ -1095,7 +1095,13 @@ Tensor pool_autograd(const Tensor& features, const py::object& km, int64_t num_o
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
-  py::class_<MadeOn, std::shared_ptr<MadeOn>>(m, "MadeOn");
+  py::class_<MadeOn, std::shared_ptr<MadeOn>>(m, "MadeOn")
+      .def("before_use", [](const MadeOn& made, const Tensor& a, const Tensor& b, const Tensor& c) { made.before_use({&a, &b, &c}); });
+  // behind what the current stream of a tensor's device has been given; None inside a capture
+  m.def("made_now", [](const Tensor& t) {
+    void* stream = stream_of(t);
+    return MadeOn::capturing(stream) ? nullptr : std::make_shared<MadeOn>(stream);
+  });
   py::class_<PreparedWeight, std::shared_ptr<PreparedWeight>>(m, "PreparedWeight");
   m.def("batch_rows", &batch_rows);
   m.def("table_build", &table_build);

@@ -32,8 +32,8 @@ class IntSearchResult:
     # The pair lists re-ordered once for the contraction, kept with the map: ascending in out_maps
     # (`_by_out`, for the forward product over a map whose out_maps does not ascend: the map of a
     # transposed convolution) and ascending in in_maps (`_by_in`, for the input gradient over a map
-    # that is not symmetric).  Each is (first list, second list, group-start table, row count) or None
-    # until first needed.
+    # that is not symmetric).  Each is (first list, second list, group-start table, row count, where
+    # and when made) or None until first needed.
     _by_out = None
     _by_in = None
     # every output row occurs in exactly one pair (the map of a transposed convolution that undoes a

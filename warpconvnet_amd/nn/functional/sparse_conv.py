@@ -90,6 +90,7 @@ def _pairs_sorted(km: IntSearchResult, by: str, num_rows: int):
     Returns (gathered-side list, ascending-side list, group-start tensor)."""
     kept = km._by_out if by == "out" else km._by_in
     if kept is not None and kept[3] == num_rows:
+        kept[4].before_use(*kept[:3])  # the lists may have been made on another stream
         return kept[:3]
     gathered, ascending = (km.in_maps, km.out_maps) if by == "out" else (km.out_maps, km.in_maps)
     K = len(km)
@@ -124,12 +125,10 @@ def _pairs_sorted(km: IntSearchResult, by: str, num_rows: int):
                 raise ValueError(what)
             warnings.warn(what + "; the input gradient keeps the pair with the lowest row", RuntimeWarning,
                           stacklevel=3)
-    kept = (g_sorted, a_sorted, groups, num_rows)
-    if by == "out":
-        km._by_out = kept
-    else:
-        km._by_in = kept
-    return kept[:3]
+    made = native().made_now(groups)
+    if made is not None:  # (inside a capture the lists are the graph's own)
+        setattr(km, "_by_out" if by == "out" else "_by_in", (g_sorted, a_sorted, groups, num_rows, made))
+    return g_sorted, a_sorted, groups
 
 
 def sparse_conv_forward(in_features: Tensor, weight: Tensor, kernel_map: IntSearchResult,
