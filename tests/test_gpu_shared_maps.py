@@ -132,3 +132,28 @@ def test_reordered_lists_serve_layers_on_other_streams():
     for got in _on_two_streams(lambda: step(shared)):
         assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])
     assert shared._by_out is not None and shared._by_in is not None
+
+
+def test_kept_weight_tiles_serve_other_streams_and_are_not_kept_from_a_capture():
+    """Tiles made behind a busy queue and read from another stream; tiles that a capture makes are the graph's own."""
+    from warpconvnet_amd.nn.functional.sparse_conv import sparse_conv_forward
+    c = _surface(3_000, 9)
+    n, km = len(c), _map(c)
+    x = normal_features(n, 64, seed=1, dtype=torch.float16).to(DEV)
+    w0 = kaiming_weight(27, 64, 64, seed=2, dtype=torch.float16).to(DEV)
+    want = sparse_conv_forward(x, w0, km, n)
+    w = w0.clone()
+    for got in _on_two_streams(lambda: sparse_conv_forward(x, w, km, n, keep_prepared_weight=True)):
+        assert torch.equal(got, want)
+    w = w0.clone()
+    graph = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph):
+        out = sparse_conv_forward(x, w, km, n, keep_prepared_weight=True)
+    assert not hasattr(w, "_wcn_prepared")
+    for i in range(3):
+        assert torch.equal(sparse_conv_forward(x, w, km, n, keep_prepared_weight=True), want)
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want), i

@@ -319,11 +319,7 @@ struct PreparedWeight {
   at::ScalarType weight_dtype{}, dtype{};
   std::vector<int64_t> shape;
   Tensor tiles;
-  void* stream = nullptr;
-  hipEvent_t made = nullptr;  // behind the kernel that made the tiles: another stream waits for it
-  ~PreparedWeight() {
-    if (made) (void)hipEventDestroy(made);
-  }
+  std::unique_ptr<MadeOn> made;
 };
 
 /* The kernels' tiles of a weight, kept on the tensor object as `_wcn_prepared` = (what they were made
@@ -338,29 +334,27 @@ Tensor prepared_tiles(const py::object& weight_obj, const Tensor& weight, const 
     auto* p = kept[py::int_(0)].cast<PreparedWeight*>();
     if (p->version == version && p->data == weight.const_data_ptr() && p->weight_dtype == weight.scalar_type() &&
         p->dtype == dtype && p->c_in == c_in && weight.sizes().equals(p->shape)) {
-      if (p->stream != stream && hipStreamWaitEvent(static_cast<hipStream_t>(stream), p->made, 0) != hipSuccess)
-        throw std::runtime_error("hipStreamWaitEvent failed");
+      p->made->before_use({&p->tiles});
       return p->tiles;
     }
   }
   const Tensor w = make_w();
   const int32_t K = static_cast<int32_t>(w.size(0)), ci = static_cast<int32_t>(w.size(1)), co = static_cast<int32_t>(w.size(2));
   const size_t nbytes = wcn_conv_prepared_weight_bytes(K, ci, co, dtype_code(dtype));
-  auto p = std::make_shared<PreparedWeight>();
-  p->tiles = at::empty({static_cast<int64_t>(nbytes)}, at::TensorOptions().dtype(at::kByte).device(w.device()));
+  const Tensor tiles = at::empty({static_cast<int64_t>(nbytes)}, at::TensorOptions().dtype(at::kByte).device(w.device()));
   check(wcn_conv_prepare_weight(w.const_data_ptr(), dtype_code(w.scalar_type()), K, ci, co, dtype_code(dtype),
-                                p->tiles.mutable_data_ptr(), nbytes, stream),
+                                tiles.mutable_data_ptr(), nbytes, stream),
         "wcn_conv_prepare_weight");
-  if (hipEventCreateWithFlags(&p->made, hipEventDisableTiming) != hipSuccess ||
-      hipEventRecord(p->made, static_cast<hipStream_t>(stream)) != hipSuccess)
-    throw std::runtime_error("an event behind the weight's tiles could not be recorded");
+  if (MadeOn::capturing(stream)) return tiles;
+  auto p = std::make_shared<PreparedWeight>();
+  p->tiles = tiles;
+  p->made = std::make_unique<MadeOn>(stream);
   p->version = version;
   p->data = weight.const_data_ptr();
   p->weight_dtype = weight.scalar_type();
   p->dtype = dtype;
   p->c_in = c_in;
   p->shape = weight.sizes().vec();
-  p->stream = stream;
   if (py::hasattr(weight_obj, "__dict__")) weight_obj.attr("_wcn_prepared") = py::make_tuple(p, p->tiles);
   return p->tiles;
 }
