@@ -157,3 +157,27 @@ def test_kept_weight_tiles_serve_other_streams_and_are_not_kept_from_a_capture()
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, want), i
+
+
+def test_a_map_given_back_while_another_stream_reads_it():
+    """A layer waits in a busy queue; the map, made on the default stream, is dropped and memory of its sizes is taken
+    and overwritten there."""
+    from warpconvnet_amd.nn.functional.sparse_conv import sparse_conv_forward
+    c = _surface(40_000, 11)
+    n = len(c)
+    x = normal_features(n, 64, seed=1, dtype=torch.float16).to(DEV)
+    w = kaiming_weight(27, 64, 64, seed=2, dtype=torch.float16).to(DEV)
+    want = sparse_conv_forward(x, w, _map(c.clone()), n)
+    big = torch.zeros(8192, 8192, device=DEV)
+    side = torch.cuda.Stream()
+    km = _map(c)
+    sizes = [t.untyped_storage().nbytes() for t in (km.in_maps, km.out_maps, km._group_start[0])]
+    torch.cuda.synchronize()
+    with torch.cuda.stream(side):
+        _occupy(big)
+        got = sparse_conv_forward(x, w, km, n)
+    assert not side.query()
+    del km
+    taken = [torch.empty(s, dtype=torch.uint8, device=DEV).zero_() for s in sizes for _ in range(2)]
+    torch.cuda.synchronize()
+    assert len(taken) == 6 and torch.equal(got, want)

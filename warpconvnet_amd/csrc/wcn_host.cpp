@@ -60,8 +60,9 @@ Tensor bytes_on(size_t n, const Tensor& like) {
  * kernels run when the graph is replayed, not now. */
 struct MadeOn {
   void* stream;
-  hipEvent_t event = nullptr;
-  explicit MadeOn(void* s) : stream(s) {
+  hipEvent_t event = nullptr;  // null where the host has waited for the kernels
+  explicit MadeOn(void* s, bool complete = false) : stream(s) {
+    if (complete) return;
     if (hipEventCreateWithFlags(&event, hipEventDisableTiming) != hipSuccess ||
         hipEventRecord(event, static_cast<hipStream_t>(s)) != hipSuccess) {
       if (event) (void)hipEventDestroy(event);
@@ -69,7 +70,9 @@ struct MadeOn {
     }
   }
   MadeOn(const MadeOn&) = delete;
-  ~MadeOn() { (void)hipEventDestroy(event); }
+  ~MadeOn() {
+    if (event) (void)hipEventDestroy(event);
+  }
 
   static bool capturing(void* s) {
     hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
@@ -81,7 +84,8 @@ struct MadeOn {
     const Tensor& first = **data.begin();
     void* s = stream_of(first);
     if (s == stream) return;
-    if (!capturing(s)) {
+    if (!event) {
+    } else if (!capturing(s)) {
       if (hipStreamWaitEvent(static_cast<hipStream_t>(s), event, 0) != hipSuccess)
         throw std::runtime_error("hipStreamWaitEvent failed");
     } else {  // a graph cannot wait for work outside it: the host does
@@ -192,7 +196,7 @@ py::tuple stride_cells(const py::object& table, const Int3& stride, bool want_bo
  * assumed size (`per_row` pairs a row), one wait for the offsets; with more pairs than assumed the
  * emit pass has written nothing and runs again into exact buffers.  Returns (in_maps, out_maps,
  * offsets int64, offsets int32, group starts (bytes) and their address, offsets in device memory, table
- * flags). */
+ * flags, where and when they were made). */
 py::tuple kernel_map(const py::object& table, const Tensor& out4, const Int3& ks, const Int3& st,
                      const std::optional<Int3>& dilation, const std::optional<Int3>& centre, double per_row,
                      int64_t keep_workspace_bytes) {
@@ -211,6 +215,7 @@ py::tuple kernel_map(const py::object& table, const Tensor& out4, const Int3& ks
   // a set mapped onto itself can also be probed block by block (opt-in; same results, a little slower)
   const char* probe = std::getenv("WCN_KMAP_PROBE");
   Tensor kept;
+  auto made = std::make_shared<MadeOn>(stream, true);
   int64_t begin = 0;
   while (true) {
     TableRef t(table);
@@ -257,11 +262,13 @@ py::tuple kernel_map(const py::object& table, const Tensor& out4, const Int3& ks
       in_buf = at::empty({total}, out4.options());
       out_buf = at::empty({total}, out4.options());
       fill(total, in_buf, out_buf);
+      made = std::make_shared<MadeOn>(stream);
     } else if (2 * total <= assumed && (assumed - total) * 4 > (int64_t{32} << 20)) {
       // far fewer pairs than assumed, more than 32 MiB of each buffer unused: exact copies, so that the
       // map does not hold the large buffers
       in_buf = in_buf.narrow(0, 0, total).clone();
       out_buf = out_buf.narrow(0, 0, total).clone();
+      made = std::make_shared<MadeOn>(stream);
     } else {
       in_buf = in_buf.narrow(0, 0, total);
       out_buf = out_buf.narrow(0, 0, total);
@@ -273,7 +280,8 @@ py::tuple kernel_map(const py::object& table, const Tensor& out4, const Int3& ks
   Tensor groups = kept.narrow(0, begin, kept.numel() - begin);
   const auto address = reinterpret_cast<uintptr_t>(groups.const_data_ptr());
   return py::make_tuple(in_buf, out_buf, offsets, offsets32, groups, address,
-                        kept.narrow(0, 0, 8 * (int64_t{K} + 1)).view(at::kLong), wcn_kmap_last_table_flags());
+                        kept.narrow(0, 0, 8 * (int64_t{K} + 1)).view(at::kLong), wcn_kmap_last_table_flags(),
+                        made);
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -298,6 +306,13 @@ struct MapRef {
     K = static_cast<int32_t>(offsets.numel() - 1);
     py::object id = km.attr("identity_map_index");
     if (!id.is_none()) identity = id.cast<int64_t>();
+    // a builder's lists, with the workspace's head behind them (offsets and group starts)
+    py::object made = km.attr("_made");
+    if (!made.is_none()) {
+      py::object head = km.attr("_device_offsets");
+      const Tensor h = head.is_none() ? Tensor() : head.cast<Tensor>();
+      made.cast<const MadeOn*>()->before_use({&in_maps, &out_maps, &h});
+    }
   }
   const int64_t* host_offsets() const { return offsets.const_data_ptr<int64_t>(); }
   int64_t pairs() const { return host_offsets()[K]; }

@@ -84,7 +84,7 @@ def _kernel_map_from_table(table: TorchHashTable, out_coords: Tensor, kernel_siz
     M = out4.shape[0]
     ks, st = _pad_kernel_args(kernel_size, 1), _pad_kernel_args(stride, 1)
     shape_key = (tuple(ks), tuple(st), M.bit_length())
-    in_maps, out_maps, offsets64, offsets, groups, address, device_offsets, flags = native().kernel_map(
+    in_maps, out_maps, offsets64, offsets, groups, address, device_offsets, flags, made = native().kernel_map(
         table, out4, ks, st, None if dilation is None else _pad_kernel_args(dilation, 1),
         None if dilation is None else _pad_kernel_args(centres, 0), _PAIRS_PER_ROW.get(shape_key, 8.0),
         _KEEP_WORKSPACE_BYTES)
@@ -95,6 +95,7 @@ def _kernel_map_from_table(table: TorchHashTable, out_coords: Tensor, kernel_siz
     result._out_ascend = True  # pairs ascend in output row inside every offset
     result._group_start = (groups, address, (K, M))
     result._device_offsets = device_offsets
+    result._made = made
     result._keys_unique = (flags & 1) == 0
     return result
 

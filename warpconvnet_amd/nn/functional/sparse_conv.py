@@ -287,6 +287,7 @@ def generate_output_coords_and_kernel_map(
         kernel_map._keys_unique = forward_map._keys_unique
         kernel_map._from_builder = forward_map._from_builder
         kernel_map._device_offsets = forward_map._device_offsets
+        kernel_map._made = forward_map._made
         kernel_map._forward_map = forward_map
         # kernel as large as the stride, no dilation, a forward map of the builder's over fine voxels
         # without repeats: every fine row has its one parent, at one offset
