@@ -1,0 +1,89 @@
+"""What the layers' native host side takes and refuses, against the torch operations it stands for: biases of other
+shapes, types, places and alignments, weights in host memory."""
+import numpy as np
+import pytest
+import torch
+
+from helpers import kaiming_weight, normal_features
+from warpconvnet_amd.utils import synthetic
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def _voxels(n, c, dtype, seed=3, extent=24):
+    from warpconvnet_amd.geometry.types.voxels import Voxels
+    bc = synthetic.random_cloud(seed, n, extent)
+    x = normal_features(len(bc), c, seed=seed, dtype=dtype).to(DEV)
+    return Voxels(torch.as_tensor(np.ascontiguousarray(bc[:, 1:]), device=DEV), x, offsets=torch.tensor([0, len(bc)]))
+
+
+def _biases(c_out, n):
+    """Everything that `out + bias` takes, by name."""
+    g = torch.Generator().manual_seed(5)
+    full = torch.randn(c_out + 1, generator=g).to(DEV)
+    return {"one value": full[:1].clone(), "row": full[None, :c_out].clone(), "per row": torch.randn(n, c_out, generator=g).to(DEV),
+            "host scalar": torch.tensor(0.25), "fp64": full[:c_out].double(), "misaligned": full.half()[1:],
+            "misaligned fp32": full[1:], "strided": torch.randn(c_out, 2, generator=g).to(DEV)[:, 0]}
+
+
+@pytest.mark.parametrize("grad", [True, False], ids=["gradients", "inference"])
+@pytest.mark.parametrize("c_in,c_out,stride", [(32, 64, 1), (32, 32, 2)], ids=["k3", "up_sampling"])
+def test_convolution_biases_are_what_an_addition_takes(c_in, c_out, stride, grad):
+    """k3: the general contraction; up_sampling: the one for maps with one pair per output row."""
+    from warpconvnet_amd.nn.functional.sparse_conv import spatially_sparse_conv
+    vox = _voxels(3000, c_in, torch.float16)
+    w = kaiming_weight(27 if stride == 1 else 8, c_in, c_out, seed=2, dtype=torch.float16).to(DEV)
+    coarse = None
+    if stride == 2:
+        coarse = spatially_sparse_conv(vox, kaiming_weight(8, c_in, c_in, seed=1, dtype=torch.float16).to(DEV), 2, stride=2)
+
+    def layer(weight, bias):
+        if coarse is None:
+            return spatially_sparse_conv(vox, weight, 3, bias=bias).feature_tensor
+        return spatially_sparse_conv(coarse, weight, 2, stride=2, bias=bias, transposed=True,
+                                     output_spatially_sparse_tensor=vox).feature_tensor
+
+    gy = normal_features(len(vox), c_out, seed=9, dtype=torch.float16).to(DEV)
+    for name, b in _biases(c_out, len(vox)).items():
+        wg, wr = (w.clone().requires_grad_(grad) for _ in range(2))
+        bg, br = (b.clone().requires_grad_(grad) if name == "one value" else b for _ in range(2))
+        got = layer(wg, bg)
+        want = layer(wr, None) + br.half()
+        # without gradients a (c_out) bias goes into the sums: one rounding instead of two (2^-11 of a value of at most 8 each)
+        assert float((got.detach().float() - want.detach().float()).abs().max()) <= (0.0 if grad else 2 * 2 ** -11 * 8), name
+        if grad:
+            got.backward(gy)
+            want.backward(gy)
+            assert torch.equal(wg.grad, wr.grad), name
+            if bg.requires_grad:
+                assert bg.grad.shape == b.shape and torch.equal(bg.grad, br.grad), name
+    for bad in (torch.zeros(c_out - 1, device=DEV), torch.zeros(c_out + 1, device=DEV), torch.zeros(c_out)):
+        with pytest.raises(RuntimeError):
+            layer(w.clone().requires_grad_(grad), bad)
+    with pytest.raises((ValueError, RuntimeError)):
+        layer(w.cpu().requires_grad_(grad), None)
+
+
+@pytest.mark.parametrize("grad", [True, False], ids=["gradients", "inference"])
+def test_depthwise_biases_are_what_an_addition_takes(grad):
+    from warpconvnet_amd.geometry.coords.search.torch_discrete import generate_kernel_map
+    from warpconvnet_amd.nn.functional.sparse_conv_depth import spatially_sparse_depthwise_conv
+    vox = _voxels(3000, 32, torch.float16)
+    c, n = vox.batch_indexed_coordinates, len(vox)
+    km = generate_kernel_map(c, c, (1, 1, 1), (3, 3, 3))
+    w = kaiming_weight(27, 32, 1, seed=2, dtype=torch.float16)[..., 0].to(DEV)
+    for name, b in _biases(32, n).items():
+        bg, br = (b.clone().requires_grad_(grad) if name == "one value" else b for _ in range(2))
+        got = spatially_sparse_depthwise_conv(vox.feature_tensor, w, km, n, bias=bg)
+        want = spatially_sparse_depthwise_conv(vox.feature_tensor, w, km, n) + br.half()
+        assert torch.equal(got, want), name
+        if bg.requires_grad:
+            got.sum().backward()
+            want.sum().backward()
+            assert torch.equal(bg.grad, br.grad)
+    for bad in (torch.zeros(31, device=DEV), torch.zeros(33, device=DEV), torch.zeros(32)):
+        with pytest.raises(RuntimeError):
+            spatially_sparse_depthwise_conv(vox.feature_tensor, w, km, n, bias=bad)
+    with pytest.raises(ValueError):
+        spatially_sparse_depthwise_conv(vox.feature_tensor, w.cpu(), km, n)

@@ -414,6 +414,17 @@ Tensor tile_plan(const py::object& km, const MapRef& map, int64_t n_in, int64_t 
 
 bool aligned16(const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; }
 
+void check_weight_device(const Tensor& weight, const Tensor& features) {
+  if (weight.device() != features.device())
+    throw py::value_error("weight is on " + weight.device().str() + ", the features on " + features.device().str());
+}
+
+/* Whether a bias is what the kernels read: (c_out) values on the features' device.  Any other (one value for all channels, a
+ * row of its own per output row, a scalar in host memory, a wrong length) is added, or refused, by torch behind them. */
+bool kernel_bias(const Tensor& bias, const Tensor& features, int64_t c_out) {
+  return bias.dim() == 1 && bias.size(0) == c_out && bias.device() == features.device();
+}
+
 /* out = act(sum_k scatter(X[in_k] @ W[k]) + bias + residual), see sparse_conv_forward.  `graph`: the form for
  * a layer whose gradients will be asked for: no residual, no clamp, and the bias, whatever its type, is added to the rounded
  * sums. */
@@ -426,6 +437,7 @@ Tensor conv_forward(const Tensor& features, const py::object& weight_obj, const 
   if (!features.is_cuda()) throw py::value_error("in_features must be on a GPU device, got " + features.device().str());
   if (features.dim() != 2 || weight.dim() != 3 || weight.size(1) != features.size(1))
     throw py::value_error("shape mismatch: features " + shape_text(features) + ", weight " + shape_text(weight));
+  check_weight_device(weight, features);
   MapRef map(km);
   const int32_t K = static_cast<int32_t>(weight.size(0)), c_out = static_cast<int32_t>(weight.size(2));
   if (map.K != K)
@@ -440,8 +452,17 @@ Tensor conv_forward(const Tensor& features, const py::object& weight_obj, const 
     if (!t || !t->defined()) return Tensor();
     return (t->scalar_type() == dtype && t->is_contiguous()) ? *t : t->to(dtype).contiguous();
   };
+  if (bias && bias->defined() && !kernel_bias(*bias, features, c_out)) {
+    if (graph) throw py::value_error("bias has shape " + shape_text(*bias) + ", the output " + std::to_string(c_out) + " channels");
+    Tensor out = conv_forward(features, weight_obj, km, num_out, std::nullopt, compute_dtype, std::nullopt, false, keep_tiles,
+                              pairs_sorted, false);
+    out = out + bias->to(out.scalar_type());
+    if (residual) out = out + residual->to(out.scalar_type());
+    return relu ? at::relu(out) : out;
+  }
   // (graph) an fp32 bias goes to the library as it is, any other in the features' type
-  const Tensor b = graph && bias && bias->scalar_type() == at::kFloat ? bias->contiguous() : as_rows(bias);
+  Tensor b = graph && bias && bias->scalar_type() == at::kFloat ? bias->contiguous() : as_rows(bias);
+  if (b.defined() && !aligned16(b.const_data_ptr())) b = b.clone();
   const int b_code = b.defined() ? dtype_code(b.scalar_type()) : code;
   // Rows that are not whole 16-byte vectors (the 3-channel input of a network's stem) would take the
   // library's slow general kernel: the channels are zero-padded instead, and the weight's with them.
@@ -715,6 +736,7 @@ py::tuple conv_backward(const Tensor& grad_output, const Tensor& in_features, co
       grad_output.size(1) != weight.size(2))
     throw py::value_error("shape mismatch: features " + shape_text(in_features) + ", grad_output " + shape_text(grad_output) +
                           ", weight " + shape_text(weight) + ", " + std::to_string(g.map.K) + " offsets");
+  check_weight_device(weight, in_features);
   auto r = backward(grad_output, in_features, weight, g, dtype, need_x, need_w,
                     [&]() { return sorted_by_in(km, pairs_sorted, in_features.size(0)); });
   return py::make_tuple(r.first.defined() ? py::cast(r.first) : py::none(), r.second.defined() ? py::cast(r.second) : py::none());
@@ -779,10 +801,10 @@ Tensor conv_autograd(const Tensor& features, const py::object& weight_obj, const
                      const py::object& pairs_sorted) {
   const Tensor weight = weight_obj.cast<Tensor>();
   // a product in another type than the features' comes back in theirs before the bias is added
-  const bool has_bias = bias && bias->defined();
+  const bool given = bias && bias->defined(), has_bias = given && kernel_bias(*bias, features, weight.size(-1));
   const bool inside = !compute_dtype || *compute_dtype == features.scalar_type();
-  Tensor out = conv_forward(features, weight_obj, km, num_out, inside ? bias : std::nullopt, compute_dtype, std::nullopt, false,
-                            false, pairs_sorted, true);
+  Tensor out = conv_forward(features, weight_obj, km, num_out, inside && has_bias ? bias : std::nullopt, compute_dtype, std::nullopt,
+                            false, false, pairs_sorted, true);
   if (has_bias && !inside) {
     at::AutoDispatchBelowADInplaceOrView guard;
     out.add_(bias->scalar_type() == out.scalar_type() ? *bias : bias->to(out.scalar_type()));
@@ -800,7 +822,7 @@ Tensor conv_autograd(const Tensor& features, const py::object& weight_obj, const
   node->km_ = std::make_unique<HeldObject>(km);
   node->sorted_ = std::make_unique<HeldObject>(pairs_sorted);
   torch::autograd::set_history(out, node);
-  return out;
+  return given && !has_bias ? out + bias->to(out.scalar_type()) : out;
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -893,19 +915,19 @@ Tensor depthwise_rows(const Tensor& x, const Tensor& w, const Tensor& rows, cons
   return out;
 }
 
-Tensor depthwise_out(const Tensor& features, const Tensor& weight, const std::optional<Tensor>& bias, const RowsMap& m,
-                     int64_t num_out, at::ScalarType dtype) {
+Tensor depthwise_out(const Tensor& features, const Tensor& weight, const Tensor& bias, const RowsMap& m, int64_t num_out,
+                     at::ScalarType dtype) {
   at::AutoDispatchBelowADInplaceOrView guard;
   const Tensor x = features.to(dtype).contiguous();
-  const bool has_bias = bias && bias->defined(), fuse = has_bias && dtype == features.scalar_type();
+  const bool has_bias = bias.defined(), fuse = has_bias && dtype == features.scalar_type();
   Tensor out;
   if (num_out == 0 || x.size(0) == 0)
     out = at::zeros({num_out, x.size(1)}, x.options());
   else
     out = depthwise_rows(x, depthwise_weight(weight, dtype), m.by_out, m.map, num_out, false,
-                         fuse ? bias->to(dtype).contiguous() : Tensor());
+                         fuse ? bias.to(dtype).contiguous() : Tensor());
   out = out.to(features.scalar_type());
-  if (has_bias && (!fuse || num_out == 0 || x.size(0) == 0)) out.add_(bias->to(out.scalar_type()));
+  if (has_bias && (!fuse || num_out == 0 || x.size(0) == 0)) out.add_(bias.to(out.scalar_type()));
   return out;
 }
 
@@ -952,6 +974,7 @@ void check_depthwise(const Tensor& features, const Tensor& weight, const RowsMap
   if (features.dim() != 2 || weight.dim() != 2 || weight.size(1) != features.size(1) || weight.size(0) != m.map.K)
     throw py::value_error("shape mismatch: features " + shape_text(features) + ", weight " + shape_text(weight) + ", " +
                           std::to_string(m.map.K) + " offsets");
+  check_weight_device(weight, features);
 }
 
 Tensor depthwise_forward(const Tensor& features, const Tensor& weight, const py::object& km, int64_t num_out,
@@ -960,7 +983,7 @@ Tensor depthwise_forward(const Tensor& features, const Tensor& weight, const py:
   check_rows_features(features, dtype, "in_features");
   const RowsMap m(km, features.size(0), num_out);
   check_depthwise(features, weight, m);
-  return depthwise_out(features, weight, std::nullopt, m, num_out, dtype);
+  return depthwise_out(features, weight, Tensor(), m, num_out, dtype);
 }
 
 py::tuple depthwise_backward(const Tensor& grad_output, const Tensor& in_features, const Tensor& weight, const py::object& km,
@@ -1013,9 +1036,11 @@ Tensor depthwise_autograd(const Tensor& features, const Tensor& weight, const st
   check_rows_features(features, dtype, "in_features");
   auto m = std::make_unique<RowsMap>(km, features.size(0), num_out);
   check_depthwise(features, weight, *m);
-  Tensor out = depthwise_out(features, weight, bias, *m, num_out, dtype);
-  const Tensor b = bias.value_or(Tensor());
-  if (!in_graph({&features, &weight, &b})) return out;
+  const bool given = bias && bias->defined(), has_bias = given && kernel_bias(*bias, features, weight.size(1));
+  const Tensor b = has_bias ? *bias : Tensor();
+  Tensor out = depthwise_out(features, weight, b, *m, num_out, dtype);
+  auto with_bias = [&]() { return given && !has_bias ? out + bias->to(out.scalar_type()) : out; };
+  if (!in_graph({&features, &weight, &b})) return with_bias();
   auto node = std::shared_ptr<DepthwiseBackward>(new DepthwiseBackward(), torch::autograd::deleteNode);
   node->set_next_edges(b.defined() ? torch::autograd::collect_next_edges(features, weight, b)
                                    : torch::autograd::collect_next_edges(features, weight));
@@ -1026,7 +1051,7 @@ Tensor depthwise_autograd(const Tensor& features, const Tensor& weight, const st
   if (b.defined()) node->bias_dtype_ = b.scalar_type();
   node->map_ = std::move(m);
   torch::autograd::set_history(out, node);
-  return out;
+  return with_bias();
 }
 
 struct PoolBackward : public torch::autograd::Node {
