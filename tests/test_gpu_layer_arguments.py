@@ -87,3 +87,29 @@ def test_depthwise_biases_are_what_an_addition_takes(grad):
             spatially_sparse_depthwise_conv(vox.feature_tensor, w, km, n, bias=bad)
     with pytest.raises(ValueError):
         spatially_sparse_depthwise_conv(vox.feature_tensor, w.cpu(), km, n)
+
+
+def test_forward_mode_tangents_are_refused_and_those_of_a_bias_carried():
+    from torch.autograd import forward_ad
+    from warpconvnet_amd.nn.functional.sparse_conv import spatially_sparse_conv
+    from warpconvnet_amd.nn.functional.sparse_conv_depth import spatially_sparse_depthwise_conv
+    from warpconvnet_amd.nn.functional.sparse_pool import sparse_max_pool
+    vox = _voxels(500, 32, torch.float32)
+    x, n = vox.feature_tensor, len(vox)
+    w = kaiming_weight(27, 32, 32, seed=2).to(DEV).requires_grad_(True)
+    wd = kaiming_weight(27, 32, 1, seed=2)[..., 0].to(DEV)
+    b = torch.randn(32, device=DEV)
+    spatially_sparse_conv(vox, w, 3)
+    km = next(iter(vox.cache.values()))
+    with forward_ad.dual_level():
+        dx, dw, dwd, db = (forward_ad.make_dual(t.detach(), torch.ones_like(t)) for t in (x, w, wd, b))
+        dual = vox.replace(batched_features=dx)
+        for call in (lambda: spatially_sparse_conv(dual, w, 3), lambda: spatially_sparse_conv(vox, dw.requires_grad_(True), 3),
+                     lambda: spatially_sparse_depthwise_conv(dx, wd, km, n), lambda: spatially_sparse_depthwise_conv(x, dwd, km, n),
+                     lambda: sparse_max_pool(dual, 2)):
+            with pytest.raises(NotImplementedError):
+                call()
+        for out in (spatially_sparse_conv(vox, w, 3, bias=db).feature_tensor,
+                    spatially_sparse_depthwise_conv(x, wd, km, n, bias=db)):
+            tangent = forward_ad.unpack_dual(out).tangent
+            assert tangent is not None and bool((tangent == 1).all())

@@ -419,10 +419,19 @@ void check_weight_device(const Tensor& weight, const Tensor& features) {
     throw py::value_error("weight is on " + weight.device().str() + ", the features on " + features.device().str());
 }
 
+bool has_tangent(const Tensor& t) { return t.defined() && t._fw_grad(/*level=*/0).defined(); }
+
+// The layers' graph nodes have gradients and no forward-mode derivative: a tangent would be lost without a word.
+void refuse_tangents(std::initializer_list<const Tensor*> tensors, const char* layer) {
+  for (const Tensor* t : tensors)
+    if (has_tangent(*t)) TORCH_CHECK_NOT_IMPLEMENTED(false, layer, " has no forward-mode derivative (jvp)");
+}
+
 /* Whether a bias is what the kernels read: (c_out) values on the features' device.  Any other (one value for all channels, a
- * row of its own per output row, a scalar in host memory, a wrong length) is added, or refused, by torch behind them. */
+ * row of its own per output row, a scalar in host memory, a wrong length), and one with a forward-mode tangent, is added, or
+ * refused, by torch behind them. */
 bool kernel_bias(const Tensor& bias, const Tensor& features, int64_t c_out) {
-  return bias.dim() == 1 && bias.size(0) == c_out && bias.device() == features.device();
+  return bias.dim() == 1 && bias.size(0) == c_out && bias.device() == features.device() && !has_tangent(bias);
 }
 
 /* out = act(sum_k scatter(X[in_k] @ W[k]) + bias + residual), see sparse_conv_forward.  `graph`: the form for
@@ -800,6 +809,7 @@ Tensor conv_autograd(const Tensor& features, const py::object& weight_obj, const
                      const py::object& km, int64_t num_out, const std::optional<at::ScalarType>& compute_dtype,
                      const py::object& pairs_sorted) {
   const Tensor weight = weight_obj.cast<Tensor>();
+  refuse_tangents({&features, &weight}, "the sparse convolution");
   // a product in another type than the features' comes back in theirs before the bias is added
   const bool given = bias && bias->defined(), has_bias = given && kernel_bias(*bias, features, weight.size(-1));
   const bool inside = !compute_dtype || *compute_dtype == features.scalar_type();
@@ -1034,6 +1044,7 @@ Tensor depthwise_autograd(const Tensor& features, const Tensor& weight, const st
                           const py::object& km, int64_t num_out, const std::optional<at::ScalarType>& compute_dtype) {
   const at::ScalarType dtype = compute_dtype.value_or(features.scalar_type());
   check_rows_features(features, dtype, "in_features");
+  refuse_tangents({&features, &weight}, "the sparse depthwise convolution");
   auto m = std::make_unique<RowsMap>(km, features.size(0), num_out);
   check_depthwise(features, weight, *m);
   const bool given = bias && bias->defined(), has_bias = given && kernel_bias(*bias, features, weight.size(1));
@@ -1096,6 +1107,7 @@ struct PoolBackward : public torch::autograd::Node {
 /* Pooling over a map (mode as in wcn_sparse_pool_fwd), with its gradient as one graph node. */
 Tensor pool_autograd(const Tensor& features, const py::object& km, int64_t num_out, int32_t mode, bool single_in) {
   check_rows_features(features, features.scalar_type(), "features");
+  refuse_tangents({&features}, "sparse pooling");
   auto m = std::make_unique<RowsMap>(km, features.size(0), num_out);
   const bool graph = in_graph({&features});
   const int32_t c = static_cast<int32_t>(features.size(1));
