@@ -374,14 +374,16 @@ int wcn_sparse_conv_fwd_single_graph(const void* features, int64_t num_in, int32
  * the offsets reversed.  The bias is in the feature dtype or (forms other than 1) fp32, of which its
  * rounding to the feature dtype is taken; bias_after_rounding != 0 adds it to the rounded sums.  Workspace: for
  * forms other than 1, wcn_conv_prepared_weight_bytes(num_offsets, c_in, c_out, dtype) bytes.
- * wcn_conv_tiles_supported: 0 where this contraction does not take the problem or another is faster, 1 where
- * it is the one to take over a plan that is there, 2 where a plan pays for itself over many calls, 3 where it
- * does in the `calls` that are known to come. */
+ * wcn_conv_tiles_supported: 0 where this contraction does not take the problem or another is faster, 2 where a plan
+ * pays for itself over many calls, 3 where it does in the `calls` that are known to come. */
 size_t wcn_tile_plan_bytes(int64_t num_out, int32_t num_offsets);
 
-/* 1 where wcn_sparse_conv_fwd sums slices of the input channels separately (few output rows, wide ones): its
- * results differ in the last bits from those of wcn_sparse_conv_fwd_tiled there, and are the same elsewhere. */
-int wcn_conv_sums_slices(int64_t num_out, int32_t c_in, int32_t c_out, int32_t dtype);
+/* 1 where the kernel that a call over the pair lists would take adds up a row's products in the order of
+ * wcn_sparse_conv_fwd_tiled (ascending offset, then channel), so that the results are the same bits.  0 for the kernels of
+ * small maps, of narrow rows and of sliced input channels.  after_rounding: the call is wcn_sparse_conv_fwd_graph, which never
+ * takes the kernel for small maps. */
+int wcn_conv_tiles_same_sums(int32_t dtype, int32_t num_offsets, int32_t c_in, int32_t c_out, int64_t num_in, int64_t num_out,
+                             int64_t num_pairs, int32_t identity_offset, int32_t after_rounding);
 
 size_t wcn_tile_plan_workspace_bytes(int64_t num_out, int32_t num_offsets, int64_t num_pairs);
 

@@ -103,3 +103,49 @@ def test_layers_over_one_map_take_the_plan_and_give_the_same_bits():
     assert lib().wcn_conv_last_kernel().decode().startswith("conv_fwd_tiles<")
     want, _ = sparse_conv_backward(gy, x, w, bare, need_weight_grad=False)
     assert float((gx.float() - want.float()).norm() / want.float().norm()) <= 1e-3
+
+
+@pytest.mark.parametrize("dtype,c_in,c_out,n", [
+    (torch.float16, 64, 64, 40_000),     # the pair-packed kernel stands behind the plan
+    (torch.bfloat16, 128, 128, 20_000),  # the one for small maps: its waves' sums are added last
+    (torch.bfloat16, 128, 128, 40_000),  # the one for wide rows
+    (torch.float16, 32, 32, 40_000),     # narrow rows: small maps, and beyond them the kernel that starts with the
+    (torch.float16, 24, 32, 90_000),     # identity's product
+    (torch.float16, 320, 64, 90_000),    # the ring kernel: channels outside the offsets
+    (torch.bfloat16, 512, 32, 34_000)],  # the same with its slices apart
+    ids=["f16_64_64", "bf16_128_128_small", "bf16_128_128", "f16_32_32", "f16_24_32", "f16_320_64", "bf16_512_32"])
+def test_results_do_not_depend_on_the_layers_before(dtype, c_in, c_out, n):
+    """The same layer three times over one map, then over a map that a wider layer has left its plan on: the same
+    bits each time, with and without gradients, and in the input gradient."""
+    from warpconvnet_amd.geometry.types.voxels import Voxels
+    from warpconvnet_amd.nn.functional.sparse_conv import sparse_conv_backward, sparse_conv_forward, spatially_sparse_conv
+    coords = torch.as_tensor(_surface(n, 12)[:, 1:].copy(), device=DEV)
+    x = normal_features(n, c_in, seed=1, dtype=dtype).to(DEV)
+    wide = normal_features(n, 256, seed=1, dtype=dtype).to(DEV)
+    w = kaiming_weight(27, c_in, c_out, seed=2, dtype=dtype).to(DEV)
+    res = normal_features(n, c_out, seed=4, dtype=dtype).to(DEV)
+    gy = normal_features(n, c_out, seed=3, dtype=dtype).to(DEV)
+    w_wide = kaiming_weight(27, 256, 256, seed=5, dtype=dtype).to(DEV)
+
+    def fresh():
+        return Voxels(coords, x, offsets=torch.tensor([0, n]))
+
+    def calls(vox):
+        plain = spatially_sparse_conv(vox, w, 3, residual=res, relu=True).feature_tensor
+        km = next(iter(vox.cache.values()))
+        wg = w.clone().requires_grad_(True)
+        graph = spatially_sparse_conv(vox, wg, 3).feature_tensor.detach()
+        gx, _ = sparse_conv_backward(gy, x, w, km, need_weight_grad=False)
+        return km, (plain, graph, gx)
+
+    vox = fresh()
+    km, first = calls(vox)
+    for _ in range(2):
+        assert all(torch.equal(a, b) for a, b in zip(calls(vox)[1], first))
+    vox = fresh()
+    calls(vox)  # (leaves the map in the cache)
+    km = next(iter(vox.cache.values()))
+    km._tile_plan = None
+    sparse_conv_forward(wide, w_wide, km, n)
+    assert km._tile_plan is not None
+    assert all(torch.equal(a, b) for a, b in zip(calls(vox)[1], first))

@@ -91,7 +91,7 @@ SIGNATURES = {
     "wcn_tile_plan_bytes": (_sz, [_i64, _i32]),
     "wcn_tile_plan_workspace_bytes": (_sz, [_i64, _i32, _i64]),
     "wcn_tile_plan_build": (ctypes.c_int, [_vp, _vp, _vp, _vp, _i32, _i32, _i64, _i64, _i64, _vp, _sz, _vp, _sz, _vp]),
-    "wcn_conv_sums_slices": (ctypes.c_int, [_i64, _i32, _i32, _i32]),
+    "wcn_conv_tiles_same_sums": (ctypes.c_int, [_i32, _i32, _i32, _i32, _i64, _i64, _i64, _i32, _i32]),
     "wcn_conv_tiles_supported": (ctypes.c_int, [_i32, _i32, _i32, _i32, _i64, _i64p, _i32, _i32]),
     "wcn_sparse_conv_fwd_graph": (ctypes.c_int, [_vp, _i64, _i32, _i32, _vp, _i32, _i32, _i32, _vp, _i32, _vp, _vp,
                                                  _i64p, _i32, _i32, _vp, _vp, _i64, _vp, _sz, _vp]),

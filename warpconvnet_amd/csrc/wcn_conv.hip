@@ -1866,9 +1866,29 @@ int wcn_sparse_conv_fwd_single_graph(const void* features, int64_t num_in, int32
                     in_maps, out_maps, host_offsets, nullptr, 0, out, num_out, workspace, workspace_bytes, stream);
 }
 
-int wcn_conv_sums_slices(int64_t num_out, int32_t c_in, int32_t c_out, int32_t dtype) {
-  if (num_out < 0 || c_in < 1 || c_out < 1 || dtype < 0 || dtype > 2) return 0;
-  return conv_wants_split(num_out, (int)round_up(c_in, ck_of(dtype)), (int)round_up(c_out, TN), ck_of(dtype)) ? 1 : 0;
+int wcn_conv_tiles_same_sums(int32_t dtype, int32_t num_offsets, int32_t c_in, int32_t c_out, int64_t num_in, int64_t num_out,
+                             int64_t num_pairs, int32_t identity_offset, int32_t after_rounding) {
+  if (dtype < 0 || dtype > 2 || num_offsets < 1 || c_in < 1 || c_out < 1 || num_in < 0 || num_out < 0) return 0;
+  if (!wcn_conv_tiles_takes(dtype, num_offsets, c_in, c_out)) return 0;
+  static const int32_t some = 0;  // (the rules look at whether there are group starts, not at them)
+  ConvArgs a = {};
+  a.K = num_offsets;
+  a.c_in = c_in;
+  a.c_out = c_out;
+  a.c_in_pad = round_up(c_in, ck_of(dtype));
+  a.c_out_pad = round_up(c_out, TN);
+  a.num_in = num_in;
+  a.num_out = num_out;
+  a.num_pairs = num_pairs;
+  a.identity = identity_offset;
+  a.G = (num_out + 63) / 64;
+  a.group_start = &some;
+  a.vec_in = a.vec_out = 1;
+  a.split = conv_wants_split(num_out, a.c_in_pad, a.c_out_pad, ck_of(dtype)) ? 1 : 0;
+  // in the order of conv_run and launch_conv; the ring kernel walks the channels outside the offsets
+  if (!after_rounding && wcn_conv_split_takes(a, dtype)) return 0;
+  if (wcn_conv_dense_takes(a, dtype)) return 1;
+  return !wcn_conv_group_takes(a, dtype) && wcn_conv_pack_takes(a, dtype) ? 1 : 0;
 }
 
 int wcn_conv_tiles_supported(int32_t dtype, int32_t num_offsets, int32_t c_in, int32_t c_out, int64_t num_out,

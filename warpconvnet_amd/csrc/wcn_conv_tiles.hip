@@ -293,8 +293,9 @@ bool wcn_conv_tiles_takes(int dtype, int num_offsets, int c_in, int c_out) {
 //    300,000    82 ->  41   255 ->  80    294 ->  91   854 -> 279
 //  1,000,000   203 -> 117
 // Few rows: the longest tile (all offsets, 0.7 us each per 64 channels) is the time, and the kernel for small maps deals
-// its offsets to several waves.  Narrow rows (32 -> 32: 30 -> 24 at 170 k) gain less than a plan costs: they use one
-// that is there.  Pairs spread evenly over the offsets (volume-filling noise): a tile has pairs in two thirds of them,
+// its offsets to several waves.  Narrow rows (32 -> 32: 30 -> 24 at 170 k) gain less than a plan costs, and their kernel adds
+// the identity's product first: taken over a plan that a wider layer has left, a layer's last bits would tell what ran
+// before it (over 4 x 250 k voxels, ten such layers in a network's pass: 1 %).  Pairs spread evenly over the offsets (volume-filling noise): a tile has pairs in two thirds of them,
 // whatever the order of the rows, and such maps stay with the other kernels.  A plan takes about 20 us and 0.07 per thousand
 // rows; a call saves about 40 ps per pair and 64 x 128 channels (60 with the few offsets of a strided kernel: 96 -> 128,
 // 2x2x2, 300 k -> 162 k rows 65 -> 29 us), and `calls` calls over the map are expected.
@@ -309,7 +310,7 @@ int wcn_conv_tiles_worth(int K, int c_in, int c_out, int64_t num_out, const int6
   // effective number of offsets: 26 of 26 for noise, 25 for spheres, 17 to 22 for rooms
   if (squares <= 0.0 || (K > 12 && sum * sum / squares > 0.98 * (K - (identity >= 0 ? 1 : 0)))) return 0;
   if (num_out < (K <= 12 || (c_in >= 64 && c_out > 64) ? 16384 : 32768)) return 0;
-  if (c_in <= 32 && c_out <= 32) return c_in > 16 && c_out > 16 ? 1 : 0;
+  if (c_in <= 32 && c_out <= 32) return 0;
   const double saved = (double)host_offsets[K] * (K <= 12 ? 60e-6 : 40e-6) * ((double)c_in * c_out / 8192.0);
   return saved * calls > 20.0 + 70e-6 * num_out ? 3 : 2;
 }

@@ -376,12 +376,18 @@ Tensor prepared_tiles(const py::object& weight_obj, const Tensor& weight, const 
 
 /* Tile plan of a builder's map (wcn_tile_plan_build), kept on the map object: the layers over a map share
  * it, on whichever stream they run.  Undefined where another contraction is to be taken, or the map is none the plan can be made from.  Where the plan
- * does not pay for itself in the calls that are known to come it is made for the second layer that would use it. */
+ * does not pay for itself in the calls that are known to come it is made for the second layer that would use it; which
+ * layers came before must not show in the results, so such a plan is for the products alone that have the same bits
+ * without one.  Inside a graph (`graph`) that holds for every plan: a sum that rounds to the other side is nothing by itself, but
+ * behind a ReLU it switches a gradient off or on. */
 Tensor tile_plan(const py::object& km, const MapRef& map, int64_t n_in, int64_t num_out, int code, int32_t c_in, int32_t c_out,
-                 int32_t calls) {
+                 int32_t calls, bool graph) {
   const int worth = wcn_conv_tiles_supported(code, map.K, c_in, c_out, num_out, map.host_offsets(),
                                              static_cast<int32_t>(map.identity), calls);
   if (!worth) return Tensor();
+  if ((graph || worth < 3) && !wcn_conv_tiles_same_sums(code, map.K, c_in, c_out, n_in, num_out, map.pairs(),
+                                                        static_cast<int32_t>(map.identity), graph ? 1 : 0))
+    return Tensor();
   py::object kept = km.attr("_tile_plan");
   if (!kept.is_none()) {
     py::tuple t = kept.cast<py::tuple>();
@@ -395,7 +401,6 @@ Tensor tile_plan(const py::object& km, const MapRef& map, int64_t n_in, int64_t 
   if (dev.is_none() || !flag(km, "_out_ascend") || !flag(km, "_from_builder")) return Tensor();
   const int32_t* groups = group_starts(km.attr("_group_start"), map.K, num_out);
   if (!groups) return Tensor();
-  if (worth < 2) return Tensor();
   if (worth < 3 && !flag(km, "_tiles_wanted")) {
     km.attr("_tiles_wanted") = true;
     return Tensor();
@@ -531,10 +536,8 @@ Tensor conv_forward(const Tensor& features, const py::object& weight_obj, const 
           "wcn_sparse_conv_fwd_single");
     return finish();
   }
-  // inside a graph a map's plan changes no bit of the results (see conv_run)
-  const bool same_sums = !graph || !wcn_conv_sums_slices(num_out, c_in, c_out, code);
-  if (num_out > 0 && n_in > 0 && aligned16(px) && aligned16(po) && aligned16(pr) && same_sums) {
-    if (const Tensor plan = tile_plan(km, map, n_in, num_out, code, c_in, c_out, graph ? 2 : 1); plan.defined()) {
+  if (num_out > 0 && n_in > 0 && aligned16(px) && aligned16(po) && aligned16(pr)) {
+    if (const Tensor plan = tile_plan(km, map, n_in, num_out, code, c_in, c_out, graph ? 2 : 1, graph); plan.defined()) {
       Tensor w, ws;
       size_t nbytes = 0;
       if (keep_tiles) {
@@ -645,13 +648,13 @@ struct GradMap {
     // that a transposed convolution's map is the exchange of
     py::object forward = km.attr("_forward_map");
     if (symmetric && n_in > 0) {
-      plan = tile_plan(km, map, n_in, n_in, code, c_out, c_in, 1);
+      plan = tile_plan(km, map, n_in, n_in, code, c_out, c_in, 1, false);
       plan_form = 3;
     } else if (!forward.is_none() && n_in > 0 && n_out > 0) {
       const MapRef f(forward);
       if (f.out_maps.const_data_ptr() == map.in_maps.const_data_ptr() && f.in_maps.const_data_ptr() == map.out_maps.const_data_ptr() &&
           f.identity < 0 && map.identity < 0)
-        plan = tile_plan(forward, f, n_out, n_in, code, c_out, c_in, 1);
+        plan = tile_plan(forward, f, n_out, n_in, code, c_out, c_in, 1, false);
       plan_form = 2;
     }
   }
