@@ -107,17 +107,17 @@ def test_conv_stride1_matches_oracle(oracle, name, dtype, c_in, c_out, n, batch,
     assert rel_err(got, ref) <= TOL[dtype], name
 
 
-NARROW_CASES = [
-    # name, dtype, c_in, c_out, kernel, voxels (0: a full 14^3 cube, runs of up to 64 pairs), extent
-    ("bf16_32_32", torch.bfloat16, 32, 32, (3, 3, 3), 9000, 26),          # twelve waves: 54 KB of weights
-    ("f16_24_32", torch.float16, 24, 32, (3, 3, 3), 5000, 22),            # the last quarter of the k-step is padding
-    ("bf16_8_16", torch.bfloat16, 8, 16, (3, 3, 3), 5000, 22),            # 16-channel k-step, one block of output channels
-    ("f16_12_20", torch.float16, 12, 20, (3, 3, 3), 5000, 22),            # output rows that are not whole 16-byte vectors
-    ("f16_16_16_k5", torch.float16, 16, 16, (5, 5, 5), 4000, 24),         # more than 64 offsets, 16-channel k-step
-    ("f16_32_16_k357", torch.float16, 32, 16, (3, 5, 7), 4000, 24),       # 105 offsets of 32 channels: 105 KB of weights
-    ("bf16_16_16_k2", torch.bfloat16, 16, 16, (2, 2, 2), 5000, 22),       # no identity offset
-    ("f16_16_32_cube", torch.float16, 16, 32, (3, 3, 3), 0, 14),          # every run full: four blocks per offset and group
-    ("bf16_32_32_sparse", torch.bfloat16, 32, 32, (3, 3, 3), 3000, 60),   # nearly every run empty
+NARROW_CASES = [  # maps of 44,000 (2x2x2), 54,000 (3x3x3), 72,000 and more rows: smaller ones go to the kernel for small maps
+    # name, dtype, c_in, c_out, kernel, voxels (0: a full 39^3 cube, runs of up to 64 pairs), extent
+    ("bf16_32_32", torch.bfloat16, 32, 32, (3, 3, 3), 36000, 46),         # twelve waves: 54 KB of weights
+    ("f16_24_32", torch.float16, 24, 32, (3, 3, 3), 36000, 46),           # the last quarter of the k-step is padding
+    ("bf16_8_16", torch.bfloat16, 8, 16, (3, 3, 3), 36000, 46),           # 16-channel k-step, one block of output channels
+    ("f16_12_20", torch.float16, 12, 20, (3, 3, 3), 36000, 46),           # output rows that are not whole 16-byte vectors
+    ("f16_16_16_k5", torch.float16, 16, 16, (5, 5, 5), 48000, 60),        # more than 64 offsets, 16-channel k-step
+    ("f16_32_16_k357", torch.float16, 32, 16, (3, 5, 7), 48000, 60),      # 105 offsets of 32 channels: 105 KB of weights
+    ("bf16_16_16_k2", torch.bfloat16, 16, 16, (2, 2, 2), 30000, 46),      # no identity offset
+    ("f16_16_32_cube", torch.float16, 16, 32, (3, 3, 3), 0, 39),          # every run full: four blocks per offset and group
+    ("bf16_32_32_sparse", torch.bfloat16, 32, 32, (3, 3, 3), 30000, 130),  # nearly every run empty
 ]
 
 
@@ -139,7 +139,10 @@ def test_narrow_layers_take_the_group_kernel_and_match_the_oracle(oracle, name, 
     w = kaiming_weight(K, c_in, c_out, seed=22, dtype=dtype)
     bias = (torch.randn(c_out, generator=torch.Generator().manual_seed(23)) * 0.1).to(dtype)
     out = spatially_sparse_conv(_voxels(items, x), w.to(DEV), ksize, bias=bias.to(DEV))
-    assert lib().wcn_conv_last_kernel().decode().startswith("conv_fwd_group<"), lib().wcn_conv_last_kernel()
+    code = {torch.float16: "f16", torch.bfloat16: "bf16"}[dtype]
+    instance = (code, (c_out + 15) // 16, "true" if c_in <= 16 else "false", 1 if K <= 64 else 2)
+    assert lib().wcn_conv_last_kernel().decode().startswith("conv_fwd_group<%s, %d, %s, %d," % instance), \
+        lib().wcn_conv_last_kernel()
     got = out.feature_tensor.float().cpu().numpy()
     want, _ = _oracle_out(oracle, x, w, bc, bc, ksize, (1, 1, 1), bias)
     assert rel_err(got, want) <= TOL[dtype], name
@@ -151,11 +154,12 @@ def test_narrow_layers_take_the_group_kernel_and_match_the_oracle(oracle, name, 
 
 FUSED_CASES = [
     # name, dtype, c_in, c_out, voxels, extent, kernel whose launcher takes it
-    ("group", torch.bfloat16, 32, 32, 6000, 24, "conv_fwd_group"),
-    ("pack", torch.float16, 64, 64, 6000, 24, "conv_fwd_pack"),
-    ("pack_f32", torch.float32, 32, 24, 4000, 22, "conv_fwd_pack"),
-    ("dense", torch.bfloat16, 128, 128, 30000, 64, "conv_fwd_dense"),
-    ("ring_split", torch.float16, 256, 256, 1500, 16, "conv_fwd_ring"),
+    ("group", torch.bfloat16, 32, 32, 70000, 64, "conv_fwd_group<"),
+    ("pack", torch.float16, 64, 64, 50000, 56, "conv_fwd_pack<"),
+    ("pack_f32", torch.float32, 32, 24, 46000, 56, "conv_fwd_pack<"),
+    ("dense", torch.bfloat16, 128, 128, 30000, 64, "conv_fwd_dense<"),
+    ("ring_split", torch.float16, 256, 256, 12000, 32, "conv_fwd_ring<"),
+    ("small", torch.float16, 64, 64, 6000, 24, "conv_fwd_small<"),
     ("odd_widths", torch.float32, 7, 13, 3000, 20, "conv_fwd"),  # whichever kernel takes the padded rows
 ]
 
@@ -686,7 +690,7 @@ def test_dilated_convolution_matches_oracle(oracle):
 
 
 CHOICE_CASES = [
-    # name, dtype, c_in, c_out, voxels, kernel: shapes the wide-row, narrow-row and pair-packed kernels take by default
+    # name, dtype, c_in, c_out, voxels, kernel: by default the kernels for small maps and (the 128 -> 128 one) for wide rows
     ("f16_16_16", torch.float16, 16, 16, 6000, (3, 3, 3)),
     ("bf16_32_32_k5", torch.bfloat16, 32, 32, 3000, (5, 5, 5)),
     ("f16_64_64", torch.float16, 64, 64, 6000, (3, 3, 3)),
@@ -699,7 +703,7 @@ CHOICE_CASES = [
 @pytest.mark.parametrize("name,dtype,c_in,c_out,n,ksize", CHOICE_CASES, ids=[c[0] for c in CHOICE_CASES])
 def test_the_kernels_behind_the_environment_switch_agree(oracle, monkeypatch, name, dtype, c_in, c_out, n, ksize):
     """WCN_CONV_KERNEL=ring keeps every shape on the ring kernel (the documented fallback),
-    WCN_CONV_KERNEL=pack skips the kernels for narrow and for wide rows: all three choices against
+    WCN_CONV_KERNEL=pack skips the kernels for small maps, narrow and wide rows: all three choices against
     the oracle, and against each other within two roundings of the element type."""
     from warpconvnet_amd._lib import lib
     from warpconvnet_amd.geometry.coords.search.torch_discrete import generate_kernel_map

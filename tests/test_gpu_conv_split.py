@@ -49,14 +49,14 @@ def _run(oracle, dtype, c_in, c_out, rows, extent, ksize, stride=(1, 1, 1), resi
     ids=["bf16_32_32", "f16_40_72", "f16_72_20", "bf16_256_192", "f32_32_64", "f32_68_24", "f16_16_16_k5"])
 def test_small_maps_match_the_oracle(oracle, dtype, c_in, c_out, ksize, residual, rows):
     got, want, kernel = _run(oracle, dtype, c_in, c_out, rows, 12, ksize, residual=residual)
-    assert kernel.startswith(("conv_fwd_group<", "conv_fwd_pack_split<", "conv_fwd_ring_split<")), kernel
+    assert kernel.startswith("conv_fwd_small<"), kernel
     assert torch.equal(got[0], got[1])  # kept tiles and tiles made in the call, and one order of additions
     assert rel_err(got[0].double().cpu().numpy(), want) <= TOL[dtype]
 
 
 def test_small_strided_map_without_identity(oracle):
     got, want, kernel = _run(oracle, torch.float16, 64, 64, 900, 14, (3, 3, 3), stride=(2, 2, 2))
-    assert kernel.startswith("conv_fwd_pack_split<"), kernel
+    assert kernel.startswith("conv_fwd_small<"), kernel
     assert torch.equal(got[0], got[1]) and rel_err(got[0].double().cpu().numpy(), want) <= 1e-2
 
 
