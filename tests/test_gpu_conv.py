@@ -79,7 +79,8 @@ CONV_CASES = [
 
 @pytest.mark.parametrize("name,dtype,c_in,c_out,n,batch,ksize", CONV_CASES,
                          ids=[c[0] for c in CONV_CASES])
-def test_conv_stride1_matches_oracle(oracle, name, dtype, c_in, c_out, n, batch, ksize):
+def test_conv_stride1_matches_oracle(oracle, monkeypatch, name, dtype, c_in, c_out, n, batch, ksize):
+    from warpconvnet_amd._lib import lib
     from warpconvnet_amd.nn.functional.sparse_conv import spatially_sparse_conv
     from oracle.explicit_conv import explicit_gemm_forward
     items = [synthetic.random_cloud(10 + b, n, 26)[:, 1:] for b in range(batch)]
@@ -100,6 +101,11 @@ def test_conv_stride1_matches_oracle(oracle, name, dtype, c_in, c_out, n, batch,
     # (a 1x1x1 kernel is a torch matmul followed by a torch add, as in the reference,
     # sparse_conv.py:1715-1721: two roundings, felt where product and bias cancel)
     assert elementwise_rel_err(got, want) <= (5e-2 if K == 1 else ELEM_TOL[dtype]), name
+    if K > 1:  # most of these maps are small: the same on the pair-packed and ring kernels, which larger ones go to
+        monkeypatch.setenv("WCN_CONV_KERNEL", "pack")
+        behind = spatially_sparse_conv(vox, w.to(DEV), ksize, bias=bias.to(DEV)).feature_tensor.float().cpu().numpy()
+        assert lib().wcn_conv_last_kernel().decode().startswith(("conv_fwd_pack<", "conv_fwd_ring<", "conv_fwd<"))
+        assert rel_err(behind, want) <= TOL[dtype] and elementwise_rel_err(behind, want) <= ELEM_TOL[dtype], name
     # the reference's own operation order (per-offset rounding) on the CPU, same tolerance
     ref = explicit_gemm_forward(x.float() if dtype != torch.float32 else x, w.float(),
                                 torch.as_tensor(im), torch.as_tensor(om), off, iden, len(bc))
