@@ -615,6 +615,14 @@ struct AssignLds {
   uint32_t wave[8];
 };
 
+// What the wave's lanes wrote to LDS before is there for what they read behind this (no instruction: a wave's LDS
+// accesses are in order; the compiler may not hand a lane its own store back, or swap the two).
+__device__ __forceinline__ void wave_lds_order() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 template <int STEPS, class Src, typename KeyT>
 __device__ __forceinline__ void assign_rows(const Src& src, int64_t n, const KeyLayout& L, int buckets, int stride,
                                             int part, AssignLds& S, const KeyT* __restrict__ bounds,
@@ -671,6 +679,7 @@ __device__ __forceinline__ void assign_rows(const Src& src, int64_t n, const Key
       const bool live = wave_first + 64u * (r0 + r) + lane <= last;
       int rank = 0, together = 1;
       if (live) s_lane[d] = (uint8_t)lane;
+      wave_lds_order();
       const uint32_t before = s_count[d];
       unsigned long long met = __ballot(live && s_lane[d] != (uint8_t)lane);
       while (met != 0) {
@@ -682,6 +691,7 @@ __device__ __forceinline__ void assign_rows(const Src& src, int64_t n, const Key
         }
         met &= ~same;
       }
+      wave_lds_order();  // every lane has read both words
       if (live && rank == 0) s_count[d] = (uint16_t)(before + (uint32_t)together);
       packed[r0 + r] = d | (before + (uint32_t)rank) << 16;
     }
