@@ -149,3 +149,41 @@ def test_results_do_not_depend_on_the_layers_before(dtype, c_in, c_out, n):
     sparse_conv_forward(wide, w_wide, km, n)
     assert km._tile_plan is not None
     assert all(torch.equal(a, b) for a, b in zip(calls(vox)[1], first))
+
+
+def _with_infinities(w):
+    """An infinite, a NaN and (fp32: of fp16 features) a too large weight in three offsets that few rows have pairs in."""
+    w = w.clone()
+    w[2, 3, 7], w[11, 0, 0], w[20, 5, 9] = float("inf"), float("nan"), 1e6 if w.dtype == torch.float32 else -float("inf")
+    return w
+
+
+@pytest.mark.parametrize("kernel,dtype,c_in,c_out,n", [
+    ("tiles", torch.float16, 64, 64, 5003), ("tiles", torch.bfloat16, 128, 256, 5003), ("tiles", torch.float16, 40, 24, 700),
+    ("tiles", torch.float16, 96, 96, 3000), ("small", torch.float16, 64, 64, 5003), ("small", torch.bfloat16, 32, 32, 700),
+    ("small", torch.float32, 32, 64, 3000)])
+@pytest.mark.parametrize("wide_weight", [False, True], ids=["", "fp32_weight"])
+def test_infinite_weights_reach_only_rows_with_pairs_in_their_offsets(oracle, kernel, dtype, c_in, c_out, n, wide_weight):
+    """A place without a pair multiplies zeros, and zero times infinity is no zero: those rows stay as they are."""
+    from warpconvnet_amd._lib import lib
+    from warpconvnet_amd.geometry.coords.search.torch_discrete import generate_kernel_map
+    from warpconvnet_amd.nn.functional.sparse_conv import sparse_conv_forward
+    bc = _surface(n, n)
+    c = torch.as_tensor(bc, device=DEV)
+    km = generate_kernel_map(c, c, (1, 1, 1), (3, 3, 3))
+    x = normal_features(n, c_in, seed=1, dtype=dtype)
+    w = _with_infinities(kaiming_weight(27, c_in, c_out, seed=2, dtype=torch.float32 if wide_weight else dtype))
+    im, om, off, iden = oracle.kernel_map(bc, bc, (3, 3, 3), (1, 1, 1))
+    want = oracle.explicit_conv_f64(x.double().numpy(), w.to(dtype).double().numpy(), im, om, off, iden, n)
+    some = np.isfinite(want)
+    assert 0.01 < (~some).any(axis=1).mean() < 0.9
+    xd, wd = x.to(DEV), w.to(DEV)
+    if kernel == "tiles":
+        got = _tiled(km, xd, wd, 0, n, c_out)
+    else:
+        got = sparse_conv_forward(xd, wd, km, n)
+        assert lib().wcn_conv_last_kernel().decode().startswith("conv_fwd_small<")
+    got = got.double().cpu().numpy()
+    assert np.array_equal(np.isfinite(got), some) and np.array_equal(np.isnan(got), np.isnan(want))
+    assert rel_err(got[some], want[some]) <= (1e-5 if dtype == torch.float32 else 1e-2)
+    assert np.array_equal(got[np.isinf(want)], want[np.isinf(want)])

@@ -51,6 +51,8 @@ struct TileCfg {
   static constexpr int NB = (B_LOADS + WAVES - 1) / WAVES;            // ... of a wave
   static constexpr int SUM_STRIDE = TN * 4 + 16;          // bytes of a row of sums in LDS
   static constexpr int RING_BYTES = D * (A_BYTES + B_BYTES), SUM_BYTES = 64 * SUM_STRIDE;
+  static constexpr int NAN_AT = RING_BYTES - 16;          // a word per wave: whether it has a NaN among its sums
+  static_assert(SUM_BYTES <= NAN_AT, "the sums are put in rows beside these words");
   static int lds(int K) { return std::max(RING_BYTES + (K + 1) / 2 * 1024, SUM_BYTES); }
 };
 
@@ -126,19 +128,21 @@ __global__ void __launch_bounds__(256, 2) conv_fwd_tiles(ConvArgs a, WcnTilePlan
   };
 
   f32x4 acc[4][NBW];
+  // A place without a pair multiplies zeros, and zero times an infinite or NaN weight is NaN: a tile that ends with one among its
+  // sums is gone through again with such products left out.
+  for (bool masked = false;; masked = true) {
 #pragma unroll
-  for (int rb = 0; rb < 4; ++rb)
+    for (int rb = 0; rb < 4; ++rb)
 #pragma unroll
-    for (int cb = 0; cb < NBW; ++cb) acc[rb][cb] = (f32x4){0.f, 0.f, 0.f, 0.f};
-
-  if (S > 0) {
+      for (int cb = 0; cb < NBW; ++cb) acc[rb][cb] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    if (S == 0) break;
     // the rows' numbers, offset by offset, as they lie in the plan: 1 KiB per load, two offsets (the plan has room behind
     // its last)
     const char* const nbr = (const char*)(plan.nbr + tile * K * TM) + lane * 16;
     for (int i = wave; i < (n_off + 1) / 2; i += C::WAVES) to_lds(nbr + i * 1024, lds0 + C::RING_BYTES + i * 1024);
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
     // step s multiplies what buffer s % D holds; it was asked for D - 1 steps before
-    Cursor qa{0, 0}, qb{0, 0};
+    Cursor qa{0, 0}, qb{0, 0}, qm{0, 0};
     uint32_t rest = all;  // offsets from qb's on
     int kb = __builtin_ctz(rest), steps_b = 0;
     auto fetch = [&](int buf) {
@@ -170,16 +174,44 @@ __global__ void __launch_bounds__(256, 2) conv_fwd_tiles(ConvArgs a, WcnTilePlan
         for (int rb = 0; rb < 4; ++rb) x[rb] = *reinterpret_cast<const V*>(A + at(rb * 16 + c));
 #pragma unroll
         for (int cb = 0; cb < NBW; ++cb) w[cb] = *reinterpret_cast<const V*>(B + at(cb * 16 + c));
+        if (!masked) {
 #pragma unroll
-        for (int cb = 0; cb < NBW; ++cb)
+          for (int cb = 0; cb < NBW; ++cb)
 #pragma unroll
-          for (int rb = 0; rb < 4; ++rb) acc[rb][cb] = Mma<T>::mma(w[cb], x[rb], acc[rb][cb]);
+            for (int rb = 0; rb < 4; ++rb) acc[rb][cb] = Mma<T>::mma(w[cb], x[rb], acc[rb][cb]);
+        } else {
+#pragma unroll
+          for (int rb = 0; rb < 4; ++rb) {
+            const bool pair = table[qm.j * TM + wr * 64 + rb * 16 + c] >= 0;
+#pragma unroll
+            for (int cb = 0; cb < NBW; ++cb) {
+              const f32x4 sum = Mma<T>::mma(w[cb], x[rb], acc[rb][cb]);
+#pragma unroll
+              for (int e = 0; e < 4; ++e) acc[rb][cb][e] = pair ? sum[e] : acc[rb][cb][e];
+            }
+          }
+        }
       }
+      if (masked) next(qm);
       buf = buf == D - 1 ? 0 : buf + 1;
       // what the next step multiplies has landed, here and, behind the barrier, everywhere
       asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((D - 2) * (C::NA + C::NB)) : "memory");
     }
     asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
+    if (masked) break;
+    bool nan = false;
+#pragma unroll
+    for (int rb = 0; rb < 4; ++rb)
+#pragma unroll
+      for (int cb = 0; cb < NBW; ++cb)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) nan |= acc[rb][cb][e] != acc[rb][cb][e];
+    uint32_t* const words = reinterpret_cast<uint32_t*>(tiles_smem + C::NAN_AT);
+    const bool any = __ballot(nan) != 0ull;
+    if (lane == 0) words[wave] = any ? 1u : 0u;
+    __syncthreads();
+    const u32x4 w = *reinterpret_cast<const u32x4*>(words);
+    if (__builtin_amdgcn_readfirstlane(w[0] | w[1] | w[2] | w[3]) == 0u) break;
   }
 
   // ---- the sums in rows through LDS, 64 rows at a time, then bias, residual, clamp, one rounding, whole 16-byte stores ----
