@@ -187,3 +187,25 @@ def test_infinite_weights_reach_only_rows_with_pairs_in_their_offsets(oracle, ke
     assert np.array_equal(np.isfinite(got), some) and np.array_equal(np.isnan(got), np.isnan(want))
     assert rel_err(got[some], want[some]) <= (1e-5 if dtype == torch.float32 else 1e-2)
     assert np.array_equal(got[np.isinf(want)], want[np.isinf(want)])
+
+
+def test_no_plan_for_an_input_gradient_nobody_asks_for():
+    """512 -> 64 with gradients: the forward product takes no plan (its slices are summed apart), the input gradient
+    does, where there is one."""
+    from warpconvnet_amd.geometry.types.voxels import Voxels
+    from warpconvnet_amd.nn.functional.sparse_conv import sparse_conv_backward, spatially_sparse_conv
+    n = 40_000
+    coords = torch.as_tensor(_surface(n, 14)[:, 1:].copy(), device=DEV)
+    w = kaiming_weight(27, 512, 64, seed=2, dtype=torch.float16).to(DEV).requires_grad_(True)
+    gy = normal_features(n, 64, seed=3, dtype=torch.float16).to(DEV)
+    for wanted in (False, True):
+        x = normal_features(n, 512, seed=1, dtype=torch.float16).to(DEV).requires_grad_(wanted)
+        vox = Voxels(coords, x, offsets=torch.tensor([0, n]))
+        out = spatially_sparse_conv(vox, w, 3).feature_tensor
+        km = next(iter(vox.cache.values()))
+        assert (km._tile_plan is not None) == wanted
+        out.backward(gy)
+        assert (x.grad is not None) == wanted
+        km._tile_plan = None
+        sparse_conv_backward(gy, x.detach(), w.detach(), km, need_input_grad=wanted)
+        assert (km._tile_plan is not None) == wanted

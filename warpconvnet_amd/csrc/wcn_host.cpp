@@ -631,7 +631,7 @@ struct GradMap {
   Tensor device_offsets;                   // undefined where the map has none in device memory
   Tensor plan;                             // tile plan, where the input gradient is taken over one,
   int32_t plan_form = 3;                   // and the form the weight is read in
-  GradMap(const py::object& km, int64_t n_in, int64_t n_out, int code, int32_t c_in, int32_t c_out)
+  GradMap(const py::object& km, int64_t n_in, int64_t n_out, int code, int32_t c_in, int32_t c_out, bool need_x)
       : map(km),
         symmetric(flag(km, "_symmetric") && flag(km, "_out_ascend") && n_in == n_out),
         in_ascend(flag(km, "_in_ascend")),
@@ -647,6 +647,7 @@ struct GradMap {
     // the input gradient walks the rows of a symmetric map itself, with the offsets reversed, or those of the forward map
     // that a transposed convolution's map is the exchange of
     py::object forward = km.attr("_forward_map");
+    if (!need_x) return;
     if (symmetric && n_in > 0) {
       plan = tile_plan(km, map, n_in, n_in, code, c_out, c_in, 1, false);
       plan_form = 3;
@@ -743,7 +744,7 @@ py::tuple conv_backward(const Tensor& grad_output, const Tensor& in_features, co
   const at::ScalarType dtype = compute_dtype.value_or(in_features.scalar_type());
   if (dtype_code(dtype) < 0) throw py::type_error(std::string("unsupported feature dtype ") + c10::toString(dtype));
   GradMap g(km, in_features.size(0), grad_output.size(0), dtype_code(dtype), static_cast<int32_t>(in_features.size(1)),
-            static_cast<int32_t>(grad_output.size(1)));
+            static_cast<int32_t>(grad_output.size(1)), need_x);
   if (weight.dim() != 3 || g.map.K != weight.size(0) || in_features.size(1) != weight.size(1) ||
       grad_output.size(1) != weight.size(2))
     throw py::value_error("shape mismatch: features " + shape_text(in_features) + ", grad_output " + shape_text(grad_output) +
@@ -831,7 +832,8 @@ Tensor conv_autograd(const Tensor& features, const py::object& weight_obj, const
   node->has_bias_ = has_bias;
   if (has_bias) node->bias_dtype_ = bias->scalar_type();
   node->map_ = std::make_unique<GradMap>(km, features.size(0), num_out, dtype_code(node->dtype_),
-                                         static_cast<int32_t>(weight.size(1)), static_cast<int32_t>(weight.size(2)));
+                                         static_cast<int32_t>(weight.size(1)), static_cast<int32_t>(weight.size(2)),
+                                         features.requires_grad());
   node->km_ = std::make_unique<HeldObject>(km);
   node->sorted_ = std::make_unique<HeldObject>(pairs_sorted);
   torch::autograd::set_history(out, node);
