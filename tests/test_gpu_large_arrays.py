@@ -324,3 +324,29 @@ def test_points_to_voxels_of_120_million_points():
         assert float(per_voxel[:, col].double().sum()) == float(marks[:, col].double().sum())
     last = csr_indices[int(csr_offsets[m - 1]):]   # the last voxel's points: beyond element 2^31 of `marks`
     assert torch.equal(per_voxel[m - 1], marks[last].sum(dim=0))
+
+
+def test_tile_plans_beyond_the_size_that_stays_with_a_map():
+    """64 -> 128 over three planes of 10.8 M voxels: the plan (1.2 GB) is made by every call that it pays in and given
+    back, and not by one that it does not (64 -> 16); the results are those without a plan, bit for bit."""
+    from warpconvnet_amd.geometry.coords.search.torch_discrete import generate_kernel_map
+    from warpconvnet_amd.nn.functional.sparse_conv import sparse_conv_forward
+    side = 1900
+    a, b = torch.meshgrid(torch.arange(1, side + 1, device=DEV), torch.arange(1, side + 1, device=DEV), indexing="ij")
+    a, b, z = a.reshape(-1), b.reshape(-1), torch.zeros(side * side, dtype=torch.long, device=DEV)
+    planes = torch.cat([torch.stack(p, dim=1) for p in ((z, a, b, z), (z, a, z, b), (z, z, a, b))])
+    coords = planes.int().contiguous()
+    n = len(coords)
+    km = generate_kernel_map(coords, coords, (1, 1, 1), (3, 3, 3))
+    x = torch.randn(n, 64, device=DEV, dtype=torch.float16)
+    w = kaiming_weight(27, 64, 128, seed=8, dtype=torch.float16).to(DEV)
+    got = sparse_conv_forward(x, w, km, n)
+    assert lib().wcn_conv_last_kernel().decode().startswith("conv_fwd_tiles<"), lib().wcn_conv_last_kernel()
+    assert km._tile_plan is None
+    for _ in range(2):
+        narrower = sparse_conv_forward(x, w[:, :, :16].contiguous(), km, n)
+        assert not lib().wcn_conv_last_kernel().decode().startswith("conv_fwd_tiles<")
+    assert torch.equal(narrower, got[:, :16])
+    km._group_start = None  # without it there is no plan, and the call finds the group starts itself
+    assert torch.equal(sparse_conv_forward(x, w, km, n), got)
+    assert lib().wcn_conv_last_kernel().decode().startswith("conv_fwd_pack<")

@@ -374,17 +374,24 @@ Tensor prepared_tiles(const py::object& weight_obj, const Tensor& weight, const 
   return p->tiles;
 }
 
+// Plans up to this size stay with their map (4 bytes per row and offset: three times the lists of a map of a scene's
+// surface).  27 offsets of 10 M rows: what one 16-bit activation of 64 channels takes there.
+constexpr size_t kKeepPlanBytes = size_t{1} << 30;
+
 /* Tile plan of a builder's map (wcn_tile_plan_build), kept on the map object: the layers over a map share
  * it, on whichever stream they run.  Undefined where another contraction is to be taken, or the map is none the plan can be made from.  Where the plan
  * does not pay for itself in the calls that are known to come it is made for the second layer that would use it; which
  * layers came before must not show in the results, so such a plan is for the products alone that have the same bits
  * without one.  Inside a graph (`graph`) that holds for every plan: a sum that rounds to the other side is nothing by itself, but
- * behind a ReLU it switches a gradient off or on. */
+ * behind a ReLU it switches a gradient off or on.  A plan of more than kKeepPlanBytes is made by the calls that repay it
+ * alone, and goes with them. */
 Tensor tile_plan(const py::object& km, const MapRef& map, int64_t n_in, int64_t num_out, int code, int32_t c_in, int32_t c_out,
                  int32_t calls, bool graph) {
+  const size_t plan_bytes = wcn_tile_plan_bytes(num_out, map.K);
+  const bool keep = plan_bytes <= kKeepPlanBytes;
   const int worth = wcn_conv_tiles_supported(code, map.K, c_in, c_out, num_out, map.host_offsets(),
-                                             static_cast<int32_t>(map.identity), calls);
-  if (!worth) return Tensor();
+                                             static_cast<int32_t>(map.identity), keep ? calls : 1);
+  if (!worth || (!keep && worth < 3)) return Tensor();
   if ((graph || worth < 3) && !wcn_conv_tiles_same_sums(code, map.K, c_in, c_out, n_in, num_out, map.pairs(),
                                                         static_cast<int32_t>(map.identity), graph ? 1 : 0))
     return Tensor();
@@ -406,14 +413,14 @@ Tensor tile_plan(const py::object& km, const MapRef& map, int64_t n_in, int64_t 
     return Tensor();
   }
   void* stream = stream_of(map.in_maps);
-  const Tensor plan = bytes_on(wcn_tile_plan_bytes(num_out, map.K), map.in_maps);
+  const Tensor plan = bytes_on(plan_bytes, map.in_maps);
   const Tensor ws = bytes_on(wcn_tile_plan_workspace_bytes(num_out, map.K, map.pairs()), map.in_maps);
   check(wcn_tile_plan_build(map.in_maps.const_data_ptr<int32_t>(), map.out_maps.const_data_ptr<int32_t>(),
                             dev.cast<Tensor>().const_data_ptr<int64_t>(), groups, map.K, static_cast<int32_t>(map.identity),
                             n_in, num_out, map.pairs(), plan.mutable_data_ptr(), static_cast<size_t>(plan.numel()),
                             ws.mutable_data_ptr(), static_cast<size_t>(ws.numel()), stream),
         "wcn_tile_plan_build");
-  if (!MadeOn::capturing(stream)) km.attr("_tile_plan") = py::make_tuple(plan, n_in, num_out, std::make_shared<MadeOn>(stream));
+  if (keep && !MadeOn::capturing(stream)) km.attr("_tile_plan") = py::make_tuple(plan, n_in, num_out, std::make_shared<MadeOn>(stream));
   return plan;
 }
 
