@@ -172,6 +172,18 @@ def test_voxels_construction_offsets_and_batch_index():
         Voxels(torch.cat(coords).float(), torch.cat(feats), offsets=vox.offsets)
 
 
+def test_voxels_replace_refuses_rows_that_do_not_match_the_offsets():
+    from warpconvnet_amd.geometry.types.voxels import Voxels
+    vox = Voxels(torch.zeros(5, 3, dtype=torch.int32), torch.zeros(5, 2), offsets=torch.tensor([0, 2, 5]))
+    with pytest.raises(AssertionError):
+        vox.replace(batched_features=torch.zeros(4, 2))
+    vox.offsets[-1] = 6  # the rows of coordinates and features agree, the offsets with neither
+    with pytest.raises(AssertionError):
+        vox.replace(batched_features=torch.zeros(5, 2))
+    with pytest.raises(AssertionError):
+        vox._with_features(vox.batched_coordinates, torch.zeros(5, 2), None)
+
+
 def test_voxels_replace_keeps_extra_attributes_and_cache():
     """reference: tests/types/test_voxels.py:189-239 and geometry.py:313-347."""
     from warpconvnet_amd.geometry.coords.search.cache import IntSearchCache

@@ -41,8 +41,9 @@ class Voxels(Geometry):
     def _with_features(self, coords: IntCoords, features: Tensor, tensor_stride) -> "Voxels":
         """replace(batched_coordinates=coords, batched_features=features, tensor_stride=...) for (N, C)
         features of the coordinates' device: what every layer ends with, without the constructors'
-        checks of what a layer has just made."""
-        if type(self) is not Voxels or features.shape[0] != coords.batched_tensor.shape[0]:
+        conversions.  Rows that do not agree go to the constructors, which refuse them."""
+        rows = features.shape[0]
+        if type(self) is not Voxels or rows != coords.batched_tensor.shape[0] or rows != coords.offsets.tolist()[-1]:
             return self.replace(batched_coordinates=coords, batched_features=features, tensor_stride=tensor_stride)
         feats = CatFeatures.__new__(CatFeatures)
         feats.batched_tensor, feats.offsets = features, coords.offsets
