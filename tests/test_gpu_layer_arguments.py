@@ -113,3 +113,23 @@ def test_forward_mode_tangents_are_refused_and_those_of_a_bias_carried():
                     spatially_sparse_depthwise_conv(x, wd, km, n, bias=db)):
             tangent = forward_ad.unpack_dual(out).tangent
             assert tangent is not None and bool((tangent == 1).all())
+
+
+def test_errors_inside_a_backward_pass_are_the_package_s_own():
+    """The map's host offsets no longer ascend when the gradient is asked for: the library refuses them, on a thread of the
+    autograd engine, before anything is launched."""
+    from warpconvnet_amd._lib import WcnError
+    from warpconvnet_amd.nn.functional.sparse_conv import spatially_sparse_conv
+    vox = _voxels(500, 32, torch.float32)
+    x = vox.feature_tensor.clone().requires_grad_(True)
+    out = spatially_sparse_conv(vox.replace(batched_features=x), kaiming_weight(27, 32, 32, seed=2).to(DEV), 3)
+    offsets = next(iter(out.cache.values()))._offsets64
+    out = out.feature_tensor
+    right = offsets.clone()
+    offsets[3] = offsets[-1] + 1
+    with pytest.raises(WcnError) as failed:
+        out.backward(torch.ones_like(out), retain_graph=True)
+    assert failed.value.status == -1
+    offsets.copy_(right)
+    out.backward(torch.ones_like(out))
+    assert x.grad is not None

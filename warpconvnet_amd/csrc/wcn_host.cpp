@@ -6,6 +6,7 @@
 // kernel map was built), so that a network over one scan left the GPU idle for two thirds of the
 // time.  Everything here is what those Python functions did, on the same library entries.
 #include <torch/extension.h>
+#include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/function.h>
 #include <torch/csrc/autograd/functions/utils.h>
 #include <torch/csrc/autograd/saved_variable.h>
@@ -30,15 +31,21 @@ using Int3 = std::array<int32_t, 3>;
 
 void* stream_of(const Tensor& t) { return c10::hip::getCurrentHIPStream(t.get_device()).stream(); }
 
-// A failed call becomes the package's own exception; on a thread of the autograd engine, which has
-// no Python frame to raise it in, an ordinary one with the same text.
+// A failed call becomes the package's own exception, also on a thread of the autograd engine, which hands it to the thread
+// that called backward().
 void check(int status, const char* where) {
   if (status == WCN_OK) return;
-  if (PyGILState_Check()) {
+  const bool python_thread = PyGILState_Check();
+  py::gil_scoped_acquire locked;
+  try {
     py::module_::import("warpconvnet_amd._lib").attr("check")(status, where);
+  } catch (py::error_already_set& e) {
+    if (python_thread) throw;
+    e.restore();
+    python_error error;
+    error.persist();
+    throw error;
   }
-  throw std::runtime_error(std::string(where) + ": " + wcn_status_string(status) + " (status " +
-                           std::to_string(status) + ")");
 }
 
 int dtype_code(at::ScalarType t) {
