@@ -293,6 +293,27 @@ int wcn_sparse_conv_fwd_prepared(const void* features, int64_t num_in, int32_t c
                                  int64_t num_out, void* workspace, size_t workspace_bytes,
                                  void* stream);
 
+/* wcn_conv_prepare_weight makes the weight's tiles in two orders, of which a call reads one: in rows (half 0; also what
+ * wcn_sparse_conv_fwd_single and _tiled read) or as the kernel for small maps loads them (half 1).  A caller that keeps tiles
+ * for long makes the halves it needs, each of wcn_conv_prepared_weight_bytes / 2 bytes: wcn_conv_prepared_half says which
+ * one a map's rows ask for (features_aligned: the features are 16-byte aligned), wcn_sparse_conv_fwd_prepared_halves takes
+ * them, the one that is not read may be null. */
+int wcn_conv_prepared_half(int32_t dtype, int32_t num_offsets, int32_t c_in, int32_t c_out, int64_t num_out,
+                           int32_t features_aligned);
+
+int wcn_conv_prepare_weight_half(const void* weight, int32_t weight_dtype, int32_t num_offsets, int32_t c_in,
+                                 int32_t c_out, int32_t dtype, int32_t half, void* prepared, size_t prepared_bytes,
+                                 void* stream);
+
+int wcn_sparse_conv_fwd_prepared_halves(const void* features, int64_t num_in, int32_t c_in, int32_t dtype,
+                                        const void* half0_or_null, const void* half1_or_null, int32_t num_offsets,
+                                        int32_t c_out, const void* bias_or_null, const int32_t* in_maps,
+                                        const int32_t* out_maps, const int64_t* host_offsets,
+                                        const int64_t* device_offsets, int32_t identity_offset,
+                                        const int32_t* group_start, const void* residual_or_null, int32_t relu,
+                                        void* out, int64_t num_out, void* workspace, size_t workspace_bytes,
+                                        void* stream);
+
 /* The forward contraction over a map in which EVERY OUTPUT ROW HAS EXACTLY ONE PAIR
  * (host_offsets[num_offsets] == num_out, which is checked, and no output row twice, which the caller
  * vouches for): the transposed convolution that undoes a strided convolution whose kernel is as large

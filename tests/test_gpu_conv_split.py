@@ -72,3 +72,26 @@ def test_larger_maps_keep_their_kernels(oracle, dtype, c_in, c_out, rows, extent
     got, want, name = _run(oracle, dtype, c_in, c_out, rows, extent, ksize, residual=True)
     assert name.startswith(kernel), name
     assert torch.equal(got[0], got[1]) and rel_err(got[0].double().cpu().numpy(), want) <= TOL[dtype]
+
+
+def test_kept_tiles_are_those_that_are_read():
+    """One weight over a small map, a large one and the small one again: a half of the tiles for each kind of map, made
+    when first asked for and found again, with the bits of the calls that make their own."""
+    from warpconvnet_amd._lib import lib
+    from warpconvnet_amd.geometry.coords.search.torch_discrete import generate_kernel_map
+    from warpconvnet_amd.nn.functional.sparse_conv import sparse_conv_forward
+    w = kaiming_weight(27, 64, 64, seed=2, dtype=torch.float16).to(DEV)
+    half = lib().wcn_conv_prepared_weight_bytes(27, 64, 64, 1) // 2
+    seen = []
+    for n, extent in ((3000, 20), (60_000, 60), (3000, 20), (60_000, 60)):
+        c = torch.as_tensor(np.ascontiguousarray(synthetic.random_cloud(3, n, extent)), device=DEV)
+        km = generate_kernel_map(c, c, (1, 1, 1), (3, 3, 3))
+        x = normal_features(len(c), 64, seed=4, dtype=torch.float16).to(DEV)
+        before = torch.cuda.memory_allocated()
+        kept = sparse_conv_forward(x, w, km, len(c), keep_prepared_weight=True)
+        seen.append((lib().wcn_conv_last_kernel().decode().startswith("conv_fwd_small<"),
+                     torch.cuda.memory_allocated() - before - (kept.numel() * 2 + 511) // 512 * 512))
+        assert torch.equal(kept, sparse_conv_forward(x, w, km, len(c)))
+        del kept
+    assert [small for small, _ in seen] == [True, False, True, False]
+    assert [bytes_ for _, bytes_ in seen] == [half, half, 0, 0]

@@ -52,6 +52,10 @@ SIGNATURES = {
     "wcn_conv_prepared_weight_bytes": (_sz, [_i32, _i32, _i32, _i32]),
     "wcn_conv_prepared_workspace_bytes": (_sz, [_i64, _i32, _i32, _i32, _i32]),
     "wcn_conv_prepare_weight": (ctypes.c_int, [_vp, _i32, _i32, _i32, _i32, _i32, _vp, _sz, _vp]),
+    "wcn_conv_prepared_half": (ctypes.c_int, [_i32, _i32, _i32, _i32, _i64, _i32]),
+    "wcn_conv_prepare_weight_half": (ctypes.c_int, [_vp, _i32, _i32, _i32, _i32, _i32, _i32, _vp, _sz, _vp]),
+    "wcn_sparse_conv_fwd_prepared_halves": (ctypes.c_int, [_vp, _i64, _i32, _i32, _vp, _vp, _i32, _i32, _vp, _vp, _vp,
+                                                           _i64p, _vp, _i32, _vp, _vp, _i32, _vp, _i64, _vp, _sz, _vp]),
     "wcn_sparse_conv_fwd_prepared": (ctypes.c_int, [_vp, _i64, _i32, _i32, _vp, _sz, _i32, _i32, _vp, _vp,
                                                     _vp, _i64p, _vp, _i32, _vp, _vp, _i32, _vp, _i64,
                                                     _vp, _sz, _vp]),

@@ -1452,15 +1452,15 @@ static int conv_run(const void* features, int64_t num_in, int32_t c_in, int32_t 
                     int flip_offsets, bool no_copy_commands, void* stream,
                     const void* residual_or_null = nullptr, int relu = 0,
                     const int64_t* device_offsets_of_prepared = nullptr, int bias_dtype = -1,
-                    int bias_after_rounding = 0) {
-  // With device_offsets_of_prepared, `weight` is the tiles wcn_conv_prepare_weight made and the
-  // call enqueues nothing but the contraction.
+                    int bias_after_rounding = 0, const void* prepared_operands = nullptr) {
+  // With device_offsets_of_prepared, `weight` and `prepared_operands` are the two halves that wcn_conv_prepare_weight makes
+  // (the one that is not read may be null) and the call enqueues nothing but the contraction.
   const bool prepared = device_offsets_of_prepared != nullptr;
   if (dtype < 0 || dtype > 2 || (!prepared && weight_dtype != dtype && weight_dtype != WCN_DTYPE_F32))
     return WCN_ERR_INVALID_ARGUMENT;
   if (prepared && (!out_maps_ascend || !group_start_or_null)) return WCN_ERR_INVALID_ARGUMENT;
   if (num_in < 0 || num_out < 0 || num_offsets < 1 || num_offsets > WCN_MAX_OFFSETS || c_in < 1 ||
-      c_out < 1 || !weight || (!workspace && !prepared) || !host_offsets)
+      c_out < 1 || (!weight && !prepared_operands) || (!workspace && !prepared) || !host_offsets)
     return WCN_ERR_INVALID_ARGUMENT;
   if (num_in >= (1ll << 31) || num_out >= (1ll << 31)) return WCN_ERR_INVALID_ARGUMENT;
   if (identity_offset >= num_offsets) return WCN_ERR_INVALID_ARGUMENT;
@@ -1530,6 +1530,7 @@ static int conv_run(const void* features, int64_t num_in, int32_t c_in, int32_t 
   // gradient off or on, and those of one layer then differ by half their size from what any other
   // size of map gives.  In training it would save 4 % of a stage on 10,000 voxels.
   const bool small = !bias_after_rounding && kernel_choice() == 0 && wcn_conv_split_takes(a, dtype);
+  if (prepared && !(small ? prepared_operands : weight)) return WCN_ERR_INVALID_ARGUMENT;
   a.Wf = nullptr;
   if (small && !prepared) {
     a.Wf = w.Wt;
@@ -1553,7 +1554,7 @@ static int conv_run(const void* features, int64_t num_in, int32_t c_in, int32_t 
     void* zero_page_address = nullptr;
     if (const int st = static_zero_page(&zero_page_address)) return st;
     a.Wt = weight;
-    a.Wf = (const char*)weight + tile_bytes(num_offsets, c_in, c_out, dtype);
+    a.Wf = prepared_operands;
     a.zeros = zero_page_address;
     a.offsets = device_offsets_of_prepared;
   } else {
@@ -1735,21 +1736,22 @@ size_t wcn_conv_prepared_weight_bytes(int32_t num_offsets, int32_t c_in, int32_t
   return 2 * tile_bytes(num_offsets, c_in, c_out, dtype);
 }
 
-int wcn_conv_prepare_weight(const void* weight, int32_t weight_dtype, int32_t num_offsets, int32_t c_in,
-                            int32_t c_out, int32_t dtype, void* prepared, size_t prepared_bytes,
-                            void* stream) {
-  const size_t need = wcn_conv_prepared_weight_bytes(num_offsets, c_in, c_out, dtype);
-  if (need == 0 || !weight || !prepared || (weight_dtype != dtype && weight_dtype != WCN_DTYPE_F32))
+// halves: 1 the tiles in rows, 2 in the order of the kernel for small maps, 3 both
+static int prepare_weight(const void* weight, int32_t weight_dtype, int32_t num_offsets, int32_t c_in, int32_t c_out,
+                          int32_t dtype, int halves, void* prepared, size_t prepared_bytes, void* stream) {
+  const size_t half = wcn_conv_prepared_weight_bytes(num_offsets, c_in, c_out, dtype) / 2;
+  if (half == 0 || !weight || !prepared || (weight_dtype != dtype && weight_dtype != WCN_DTYPE_F32))
     return WCN_ERR_INVALID_ARGUMENT;
-  if (prepared_bytes < need) return WCN_ERR_WORKSPACE;
+  if (prepared_bytes < (halves == 3 ? 2 : 1) * half) return WCN_ERR_WORKSPACE;
   ConvArgs a = {};
   a.K = num_offsets;
   a.c_in = c_in;
   a.c_out = c_out;
   a.c_in_pad = round_up(c_in, ck_of(dtype));
   a.c_out_pad = round_up(c_out, TN);
-  a.Wt = prepared;  // zeros and offsets stay null: the kernel then writes the tiles only
-  a.Wf = (char*)prepared + need / 2;
+  // zeros and offsets stay null: the kernel then writes the tiles only
+  if (halves & 1) a.Wt = prepared;
+  if (halves & 2) a.Wf = (char*)prepared + (halves & 1 ? half : 0);
   hipStream_t s = (hipStream_t)stream;
   switch (dtype) {
     case WCN_DTYPE_F32: launch_prep<float>(a, weight, weight_dtype, dtype, 0, 0, nullptr, s); break;
@@ -1757,6 +1759,47 @@ int wcn_conv_prepare_weight(const void* weight, int32_t weight_dtype, int32_t nu
     default: launch_prep<__bf16>(a, weight, weight_dtype, dtype, 0, 0, nullptr, s); break;
   }
   return hipGetLastError() == hipSuccess ? WCN_OK : WCN_ERR_LAUNCH;
+}
+
+int wcn_conv_prepare_weight(const void* weight, int32_t weight_dtype, int32_t num_offsets, int32_t c_in,
+                            int32_t c_out, int32_t dtype, void* prepared, size_t prepared_bytes,
+                            void* stream) {
+  return prepare_weight(weight, weight_dtype, num_offsets, c_in, c_out, dtype, 3, prepared, prepared_bytes, stream);
+}
+
+int wcn_conv_prepare_weight_half(const void* weight, int32_t weight_dtype, int32_t num_offsets, int32_t c_in,
+                                 int32_t c_out, int32_t dtype, int32_t half, void* prepared, size_t prepared_bytes,
+                                 void* stream) {
+  if (half != 0 && half != 1) return WCN_ERR_INVALID_ARGUMENT;
+  return prepare_weight(weight, weight_dtype, num_offsets, c_in, c_out, dtype, 1 << half, prepared, prepared_bytes, stream);
+}
+
+int wcn_conv_prepared_half(int32_t dtype, int32_t num_offsets, int32_t c_in, int32_t c_out, int64_t num_out,
+                           int32_t features_aligned) {
+  if (dtype < 0 || dtype > 2 || num_offsets < 1 || c_in < 1 || c_out < 1 || num_out < 1 || kernel_choice() != 0) return 0;
+  ConvArgs a = {};
+  a.K = num_offsets;
+  a.c_in = c_in;
+  a.c_out = c_out;
+  a.num_out = num_out;
+  a.G = (num_out + 63) / 64;
+  a.vec_in = features_aligned && (size_t)c_in * elem_size(dtype) % 16 == 0 ? 1 : 0;
+  return wcn_conv_split_takes(a, dtype) ? 1 : 0;
+}
+
+int wcn_sparse_conv_fwd_prepared_halves(const void* features, int64_t num_in, int32_t c_in, int32_t dtype,
+                                        const void* half0_or_null, const void* half1_or_null, int32_t num_offsets,
+                                        int32_t c_out, const void* bias_or_null, const int32_t* in_maps,
+                                        const int32_t* out_maps, const int64_t* host_offsets,
+                                        const int64_t* device_offsets, int32_t identity_offset,
+                                        const int32_t* group_start, const void* residual_or_null, int32_t relu,
+                                        void* out, int64_t num_out, void* workspace, size_t workspace_bytes,
+                                        void* stream) {
+  if (residual_or_null && residual_or_null == out) return WCN_ERR_INVALID_ARGUMENT;
+  if (!device_offsets || !group_start) return WCN_ERR_INVALID_ARGUMENT;
+  return conv_run(features, num_in, c_in, dtype, half0_or_null, dtype, num_offsets, c_out, bias_or_null, in_maps, out_maps,
+                  host_offsets, identity_offset, 1, group_start, out, num_out, workspace, workspace_bytes, 0, 0, true,
+                  stream, residual_or_null, relu, device_offsets, -1, 0, half1_or_null);
 }
 
 int wcn_sparse_conv_fwd_prepared(const void* features, int64_t num_in, int32_t c_in, int32_t dtype,
@@ -1768,15 +1811,13 @@ int wcn_sparse_conv_fwd_prepared(const void* features, int64_t num_in, int32_t c
                                  const void* residual_or_null, int32_t relu, void* out,
                                  int64_t num_out, void* workspace, size_t workspace_bytes,
                                  void* stream) {
-  if (residual_or_null && residual_or_null == out) return WCN_ERR_INVALID_ARGUMENT;
-  if (!device_offsets || !group_start) return WCN_ERR_INVALID_ARGUMENT;
   const size_t need = wcn_conv_prepared_weight_bytes(num_offsets, c_in, c_out, dtype);
-  if (need == 0) return WCN_ERR_INVALID_ARGUMENT;
+  if (need == 0 || !prepared_weight) return WCN_ERR_INVALID_ARGUMENT;
   if (prepared_bytes < need) return WCN_ERR_WORKSPACE;
-  return conv_run(features, num_in, c_in, dtype, prepared_weight, dtype, num_offsets, c_out,
-                  bias_or_null, in_maps, out_maps, host_offsets, identity_offset, 1, group_start, out,
-                  num_out, workspace, workspace_bytes, 0, 0, true, stream, residual_or_null, relu,
-                  device_offsets);
+  return wcn_sparse_conv_fwd_prepared_halves(features, num_in, c_in, dtype, prepared_weight,
+                                             (const char*)prepared_weight + need / 2, num_offsets, c_out, bias_or_null, in_maps,
+                                             out_maps, host_offsets, device_offsets, identity_offset, group_start,
+                                             residual_or_null, relu, out, num_out, workspace, workspace_bytes, stream);
 }
 
 int wcn_conv_single_supported(int32_t dtype, int32_t c_in, int32_t c_out, int32_t num_offsets) {

@@ -340,45 +340,50 @@ struct PreparedWeight {
   const void* data = nullptr;
   at::ScalarType weight_dtype{}, dtype{};
   std::vector<int64_t> shape;
-  Tensor tiles;
-  std::unique_ptr<MadeOn> made;
+  Tensor tiles[2];  // by half (wcn_conv_prepared_half), each made when it is first asked for
+  std::unique_ptr<MadeOn> made[2];
 };
 
-/* The kernels' tiles of a weight, kept on the tensor object as `_wcn_prepared` = (what they were made
- * from, tiles).  make_w(): the weight as the contraction would receive it. */
+/* One half of the kernels' tiles of a weight, kept on the tensor object as `_wcn_prepared` = (what they were made
+ * from and the halves, the first of them).  make_w(): the weight as the contraction would receive it. */
 template <typename F>
 Tensor prepared_tiles(const py::object& weight_obj, const Tensor& weight, const F& make_w, at::ScalarType dtype,
-                      int64_t c_in) {
+                      int64_t c_in, int half) {
   const int64_t version = weight._version();
   void* stream = stream_of(weight);
   py::object kept = py::getattr(weight_obj, "_wcn_prepared", py::none());
+  std::shared_ptr<PreparedWeight> same;
   if (!kept.is_none()) {
-    auto* p = kept[py::int_(0)].cast<PreparedWeight*>();
+    auto p = kept[py::int_(0)].cast<std::shared_ptr<PreparedWeight>>();
     if (p->version == version && p->data == weight.const_data_ptr() && p->weight_dtype == weight.scalar_type() &&
         p->dtype == dtype && p->c_in == c_in && weight.sizes().equals(p->shape)) {
-      p->made->before_use({&p->tiles});
-      return p->tiles;
+      if (p->tiles[half].defined()) {
+        p->made[half]->before_use({&p->tiles[half]});
+        return p->tiles[half];
+      }
+      same = std::move(p);
     }
   }
   const Tensor w = make_w();
   const int32_t K = static_cast<int32_t>(w.size(0)), ci = static_cast<int32_t>(w.size(1)), co = static_cast<int32_t>(w.size(2));
-  const size_t nbytes = wcn_conv_prepared_weight_bytes(K, ci, co, dtype_code(dtype));
+  const size_t nbytes = wcn_conv_prepared_weight_bytes(K, ci, co, dtype_code(dtype)) / 2;
   const Tensor tiles = at::empty({static_cast<int64_t>(nbytes)}, at::TensorOptions().dtype(at::kByte).device(w.device()));
-  check(wcn_conv_prepare_weight(w.const_data_ptr(), dtype_code(w.scalar_type()), K, ci, co, dtype_code(dtype),
-                                tiles.mutable_data_ptr(), nbytes, stream),
-        "wcn_conv_prepare_weight");
+  check(wcn_conv_prepare_weight_half(w.const_data_ptr(), dtype_code(w.scalar_type()), K, ci, co, dtype_code(dtype), half,
+                                     tiles.mutable_data_ptr(), nbytes, stream),
+        "wcn_conv_prepare_weight_half");
   if (MadeOn::capturing(stream)) return tiles;
-  auto p = std::make_shared<PreparedWeight>();
-  p->tiles = tiles;
-  p->made = std::make_unique<MadeOn>(stream);
+  auto p = same ? same : std::make_shared<PreparedWeight>();
+  p->tiles[half] = tiles;
+  p->made[half] = std::make_unique<MadeOn>(stream);
+  if (same) return tiles;
   p->version = version;
   p->data = weight.const_data_ptr();
   p->weight_dtype = weight.scalar_type();
   p->dtype = dtype;
   p->c_in = c_in;
   p->shape = weight.sizes().vec();
-  if (py::hasattr(weight_obj, "__dict__")) weight_obj.attr("_wcn_prepared") = py::make_tuple(p, p->tiles);
-  return p->tiles;
+  if (py::hasattr(weight_obj, "__dict__")) weight_obj.attr("_wcn_prepared") = py::make_tuple(p, tiles);
+  return tiles;
 }
 
 // Plans up to this size stay with their map (4 bytes per row and offset: three times the lists of a map of a scene's
@@ -529,7 +534,7 @@ Tensor conv_forward(const Tensor& features, const py::object& weight_obj, const 
     Tensor w, ws;
     size_t nbytes = 0;
     if (keep_tiles) {
-      w = prepared_tiles(weight_obj, weight, make_w, dtype, c_in);
+      w = prepared_tiles(weight_obj, weight, make_w, dtype, c_in, 0);
     } else {
       w = make_w();
       nbytes = wcn_conv_prepared_weight_bytes(K, c_in, c_out, code);
@@ -555,7 +560,7 @@ Tensor conv_forward(const Tensor& features, const py::object& weight_obj, const 
       Tensor w, ws;
       size_t nbytes = 0;
       if (keep_tiles) {
-        w = prepared_tiles(weight_obj, weight, make_w, dtype, c_in);
+        w = prepared_tiles(weight_obj, weight, make_w, dtype, c_in, 0);
       } else {
         w = make_w();
         nbytes = wcn_conv_prepared_weight_bytes(K, c_in, c_out, code);
@@ -584,7 +589,9 @@ Tensor conv_forward(const Tensor& features, const py::object& weight_obj, const 
   const int32_t* out_maps = map.out_maps.const_data_ptr<int32_t>();
   const int32_t iden = static_cast<int32_t>(map.identity);
   if (keep_tiles && groups != nullptr && num_out > 0) {
-    const Tensor tiles = prepared_tiles(weight_obj, weight, make_w, dtype, c_in);
+    const int half = wcn_conv_prepared_half(code, K, c_in, c_out, num_out, aligned16(px) ? 1 : 0);
+    const Tensor tiles = prepared_tiles(weight_obj, weight, make_w, dtype, c_in, half);
+    const void* const pt = tiles.const_data_ptr();
     py::object dev = km.attr("_device_offsets");
     if (dev.is_none() || dev.cast<Tensor>().device() != x.device() || dev.cast<Tensor>().numel() != K + 1) {
       dev = py::cast(map.offsets.to(x.device()));
@@ -594,10 +601,11 @@ Tensor conv_forward(const Tensor& features, const py::object& weight_obj, const 
     const size_t nbytes = wcn_conv_prepared_workspace_bytes(num_out, K, c_in, c_out, code);
     Tensor ws;
     if (nbytes) ws = bytes_on(nbytes, x);
-    check(wcn_sparse_conv_fwd_prepared(px, n_in, c_in, code, tiles.const_data_ptr(), static_cast<size_t>(tiles.numel()), K,
-                                       c_out, pb, in_maps, out_maps, map.host_offsets(),
-                                       static_cast<const int64_t*>(device_offsets.const_data_ptr()), iden, groups, pr,
-                                       relu ? 1 : 0, po, num_out, nbytes ? ws.mutable_data_ptr() : nullptr, nbytes, stream),
+    check(wcn_sparse_conv_fwd_prepared_halves(px, n_in, c_in, code, half == 0 ? pt : nullptr, half == 1 ? pt : nullptr, K,
+                                              c_out, pb, in_maps, out_maps, map.host_offsets(),
+                                              static_cast<const int64_t*>(device_offsets.const_data_ptr()), iden, groups, pr,
+                                              relu ? 1 : 0, po, num_out, nbytes ? ws.mutable_data_ptr() : nullptr, nbytes,
+                                              stream),
           "wcn_sparse_conv_fwd_prepared");
     return finish();
   }
