@@ -181,3 +181,33 @@ def test_a_map_given_back_while_another_stream_reads_it():
     taken = [torch.empty(s, dtype=torch.uint8, device=DEV).zero_() for s in sizes for _ in range(2)]
     torch.cuda.synchronize()
     assert len(taken) == 6 and torch.equal(got, want)
+
+
+def test_copies_and_files_of_voxels_with_maps():
+    """copy.deepcopy and pickle of a tensor whose cache holds maps with everything the layers left on them: the copy
+    makes its own and gives the same results after the original is gone."""
+    import copy
+    import pickle
+    from warpconvnet_amd.geometry.types.voxels import Voxels
+    from warpconvnet_amd.nn.functional.sparse_conv import spatially_sparse_conv
+    from warpconvnet_amd.nn.functional.sparse_pool import sparse_max_pool
+    rows = _surface(40_000, 13)
+    x = normal_features(len(rows), 128, seed=1, dtype=torch.float16).to(DEV)
+    w = kaiming_weight(27, 128, 256, seed=2, dtype=torch.float16).to(DEV)
+    w_up = kaiming_weight(8, 128, 32, seed=3, dtype=torch.float16).to(DEV)
+
+    def use(vox):
+        pooled = sparse_max_pool(vox, 2)
+        up = spatially_sparse_conv(pooled, w_up, 2, stride=2, transposed=True, output_spatially_sparse_tensor=vox)
+        return (spatially_sparse_conv(vox, w, 3).feature_tensor, pooled.feature_tensor, up.feature_tensor)
+
+    vox = Voxels(rows[:, 1:].contiguous(), x, offsets=torch.tensor([0, len(rows)]))
+    want = use(vox)
+    copies = [copy.deepcopy(vox), pickle.loads(pickle.dumps(vox))]
+    del vox
+    taken = [torch.full((1 << 24,), 0x7f, dtype=torch.uint8, device=DEV) for _ in range(16)]
+    for other in copies:
+        assert other.cache and all(km._group_start is None and km._made is None for km in other.cache.values())
+        for _ in range(2):
+            assert all(torch.equal(a, b) for a, b in zip(use(other), want))
+    del taken

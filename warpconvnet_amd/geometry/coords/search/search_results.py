@@ -71,6 +71,13 @@ class IntSearchResult:
         self.identity_map_index, self._offsets64 = identity_map_index, offsets64
         return self
 
+    # what belongs to this object's memory, device and process: copies and files go without, and make their own
+    _OWN = ("_group_start", "_in_group_start", "_device_offsets", "_made", "_by_out", "_by_in", "_rows_forms", "_tile_plan",
+            "_forward_map", "_tiles_wanted")
+
+    def __getstate__(self):
+        return {name: value for name, value in self.__dict__.items() if name not in self._OWN}
+
     @torch.no_grad()
     def __getitem__(self, idx: int) -> Tuple[Tensor, Tensor]:
         start, end = int(self.offsets[idx]), int(self.offsets[idx + 1])
