@@ -128,21 +128,35 @@ __global__ void __launch_bounds__(256, 2) conv_fwd_tiles(ConvArgs a, WcnTilePlan
   };
 
   f32x4 acc[4][NBW];
-  // A place without a pair multiplies zeros, and zero times an infinite or NaN weight is NaN: a tile that ends with one among its
-  // sums is gone through again with such products left out.
-  for (bool masked = false;; masked = true) {
+  auto clear = [&]() {
 #pragma unroll
     for (int rb = 0; rb < 4; ++rb)
 #pragma unroll
       for (int cb = 0; cb < NBW; ++cb) acc[rb][cb] = (f32x4){0.f, 0.f, 0.f, 0.f};
-    if (S == 0) break;
+  };
+  // the operands of 32 channels of a step out of a buffer
+  auto operands = [&](int buf, int ks, V (&x)[4], V (&w)[NBW]) {
+    const char* const A = tiles_smem + buf * C::A_BYTES + wr * (64 * KC * 2);
+    const char* const B = tiles_smem + D * C::A_BYTES + buf * C::B_BYTES + wc * (16 * NBW * KC * 2);
+    auto at = [&](int row) {
+      const int p = ks * 4 + g;
+      return row * (KC * 2) + (KC == 64 ? p ^ ((row >> 1) & 7) : p ^ ((row >> 2) & 3)) * 16;
+    };
+#pragma unroll
+    for (int rb = 0; rb < 4; ++rb) x[rb] = *reinterpret_cast<const V*>(A + at(rb * 16 + c));
+#pragma unroll
+    for (int cb = 0; cb < NBW; ++cb) w[cb] = *reinterpret_cast<const V*>(B + at(cb * 16 + c));
+  };
+  clear();
+
+  if (S > 0) {
     // the rows' numbers, offset by offset, as they lie in the plan: 1 KiB per load, two offsets (the plan has room behind
     // its last)
     const char* const nbr = (const char*)(plan.nbr + tile * K * TM) + lane * 16;
     for (int i = wave; i < (n_off + 1) / 2; i += C::WAVES) to_lds(nbr + i * 1024, lds0 + C::RING_BYTES + i * 1024);
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
     // step s multiplies what buffer s % D holds; it was asked for D - 1 steps before
-    Cursor qa{0, 0}, qb{0, 0}, qm{0, 0};
+    Cursor qa{0, 0}, qb{0, 0};
     uint32_t rest = all;  // offsets from qb's on
     int kb = __builtin_ctz(rest), steps_b = 0;
     auto fetch = [&](int buf) {
@@ -161,44 +175,23 @@ __global__ void __launch_bounds__(256, 2) conv_fwd_tiles(ConvArgs a, WcnTilePlan
     int buf = 0;
     for (int s = 0; s < S; ++s) {
       fetch(buf == 0 ? D - 1 : buf - 1);
-      const char* const A = tiles_smem + buf * C::A_BYTES + wr * (64 * KC * 2);
-      const char* const B = tiles_smem + D * C::A_BYTES + buf * C::B_BYTES + wc * (16 * NBW * KC * 2);
 #pragma unroll
       for (int ks = 0; ks < KC / 32; ++ks) {
         V x[4], w[NBW];
-        auto at = [&](int row) {
-          const int p = ks * 4 + g;
-          return row * (KC * 2) + (KC == 64 ? p ^ ((row >> 1) & 7) : p ^ ((row >> 2) & 3)) * 16;
-        };
+        operands(buf, ks, x, w);
 #pragma unroll
-        for (int rb = 0; rb < 4; ++rb) x[rb] = *reinterpret_cast<const V*>(A + at(rb * 16 + c));
+        for (int cb = 0; cb < NBW; ++cb)
 #pragma unroll
-        for (int cb = 0; cb < NBW; ++cb) w[cb] = *reinterpret_cast<const V*>(B + at(cb * 16 + c));
-        if (!masked) {
-#pragma unroll
-          for (int cb = 0; cb < NBW; ++cb)
-#pragma unroll
-            for (int rb = 0; rb < 4; ++rb) acc[rb][cb] = Mma<T>::mma(w[cb], x[rb], acc[rb][cb]);
-        } else {
-#pragma unroll
-          for (int rb = 0; rb < 4; ++rb) {
-            const bool pair = table[qm.j * TM + wr * 64 + rb * 16 + c] >= 0;
-#pragma unroll
-            for (int cb = 0; cb < NBW; ++cb) {
-              const f32x4 sum = Mma<T>::mma(w[cb], x[rb], acc[rb][cb]);
-#pragma unroll
-              for (int e = 0; e < 4; ++e) acc[rb][cb][e] = pair ? sum[e] : acc[rb][cb][e];
-            }
-          }
-        }
+          for (int rb = 0; rb < 4; ++rb) acc[rb][cb] = Mma<T>::mma(w[cb], x[rb], acc[rb][cb]);
       }
-      if (masked) next(qm);
       buf = buf == D - 1 ? 0 : buf + 1;
       // what the next step multiplies has landed, here and, behind the barrier, everywhere
       asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((D - 2) * (C::NA + C::NB)) : "memory");
     }
     asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
-    if (masked) break;
+
+    // A place without a pair has multiplied zeros, and zero times an infinite or NaN weight is NaN: a tile with one among its
+    // sums is gone through again, a step at a time, with such products left out.
     bool nan = false;
 #pragma unroll
     for (int rb = 0; rb < 4; ++rb)
@@ -210,8 +203,38 @@ __global__ void __launch_bounds__(256, 2) conv_fwd_tiles(ConvArgs a, WcnTilePlan
     const bool any = __ballot(nan) != 0ull;
     if (lane == 0) words[wave] = any ? 1u : 0u;
     __syncthreads();
-    const u32x4 w = *reinterpret_cast<const u32x4*>(words);
-    if (__builtin_amdgcn_readfirstlane(w[0] | w[1] | w[2] | w[3]) == 0u) break;
+    const u32x4 found = *reinterpret_cast<const u32x4*>(words);
+    if (__builtin_amdgcn_readfirstlane(found[0] | found[1] | found[2] | found[3]) != 0u) {
+      clear();
+      Cursor q{0, 0};
+      rest = all;
+#pragma nounroll
+      for (int s = 0; s < S; ++s) {
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");  // the buffer (and the words above) have been read
+        fetch_weights(__builtin_ctz(rest), q.chunk, 0);
+        fetch_rows(q, 0);
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        bool pair[4];
+#pragma unroll
+        for (int rb = 0; rb < 4; ++rb) pair[rb] = table[q.j * TM + wr * 64 + rb * 16 + c] >= 0;
+#pragma unroll
+        for (int ks = 0; ks < KC / 32; ++ks) {
+          V x[4], w[NBW];
+          operands(0, ks, x, w);
+#pragma unroll
+          for (int cb = 0; cb < NBW; ++cb)
+#pragma unroll
+            for (int rb = 0; rb < 4; ++rb) {
+              const f32x4 with = Mma<T>::mma(w[cb], x[rb], acc[rb][cb]);
+#pragma unroll
+              for (int e = 0; e < 4; ++e) acc[rb][cb][e] = pair[rb] ? with[e] : acc[rb][cb][e];
+            }
+        }
+        next(q);
+        if (q.chunk == 0) rest &= rest - 1u;
+      }
+      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    }
   }
 
   // ---- the sums in rows through LDS, 64 rows at a time, then bias, residual, clamp, one rounding, whole 16-byte stores ----
