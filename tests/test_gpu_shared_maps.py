@@ -211,3 +211,20 @@ def test_copies_and_files_of_voxels_with_maps():
         for _ in range(2):
             assert all(torch.equal(a, b) for a, b in zip(use(other), want))
     del taken
+
+
+def test_a_coordinate_table_nobody_has_waited_for_is_its_stream_s_own():
+    from warpconvnet_amd.geometry.coords.search.torch_discrete import _table_of
+    from warpconvnet_amd.geometry.coords.search.torch_hashmap import HashMethod
+    c = _surface(3_000, 17)
+    torch.cuda.synchronize()
+    first = _table_of(c, HashMethod.CITY, c.device)
+    assert _table_of(c, HashMethod.CITY, c.device) is first
+    with torch.cuda.stream(torch.cuda.Stream()):
+        own = _table_of(c, HashMethod.CITY, c.device)
+        assert own is not first
+        km = _map(c)  # waits
+        assert own._checked
+    assert _table_of(c, HashMethod.CITY, c.device) is own
+    other = _map(c.clone())
+    assert torch.equal(km.in_maps, other.in_maps) and torch.equal(km.out_maps, other.out_maps)

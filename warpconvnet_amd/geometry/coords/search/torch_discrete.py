@@ -19,6 +19,7 @@ import torch
 from torch import Tensor
 
 from ...._lib import host as native
+from ...._lib import stream_ptr
 from ....utils.ntuple import ntuple
 from .search_results import IntSearchResult
 from .torch_hashmap import HashMethod, TorchHashTable, _four_columns
@@ -104,10 +105,13 @@ def _table_of(coords: Tensor, hash_method: HashMethod, device) -> TorchHashTable
     """The coordinate table of an input tensor, built once per tensor object: the maps of
     different kernels over the same input rows (the 3x3x3 and the strided 2x2x2 map of one
     resolution of a network) share it.  It is kept on the tensor object together with the
-    tensor's version counter, so an in-place change of the coordinates rebuilds it.  (The
-    reference builds a new table in every call, torch_discrete.py:398-401.)"""
+    tensor's version counter, so an in-place change of the coordinates rebuilds it, and with the
+    stream that builds it: until somebody has waited for the table (a map's builder does, with the
+    interpreter free for other threads), it is for that stream alone.  (The reference builds a new
+    table in every call, torch_discrete.py:398-401.)"""
     kept = getattr(coords, "_wcn_table", None)
-    if kept is not None and kept[0] == coords._version:
+    stream = stream_ptr(coords.device).value if coords.is_cuda else None
+    if kept is not None and kept[0] == coords._version and (kept[1]._checked or kept[2] == stream):
         return kept[1]
     # built from an alias of the tensor (same storage, another Python object): the table keeps its
     # keys alive, and keeping the table on `coords` itself would otherwise close a reference
@@ -118,7 +122,7 @@ def _table_of(coords: Tensor, hash_method: HashMethod, device) -> TorchHashTable
         table = TorchHashTable.from_keys(coords.detach(), hash_method=hash_method, device=device,
                                          _defer_check=True)
     try:
-        coords._wcn_table = (coords._version, table)
+        coords._wcn_table = (coords._version, table, stream)
     except AttributeError:
         pass
     return table
