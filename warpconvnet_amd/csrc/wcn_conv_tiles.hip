@@ -17,9 +17,9 @@
 // padding; the 16-byte piece p of row r sits at p ^ (bits of r), which is arranged on the source side: a lane
 // fetches the piece that belongs where its data lands.
 //
-// What bounds it: the way of both operands into LDS (16 TB/s over the chip at 128 x 128: a step of 64 channels takes
-// a CU 0.45 us, its multiplications 0.2), and for few rows the longest tile.  Tried: 256-row tiles of eight waves
-// (a quarter to a half less weight traffic, one workgroup per CU: 10 to 30 % slower), deeper buffers with fewer workgroups
+// What bounds it: the way of both operands out of the L2 into LDS (256 -> 256 over 39 k rows 10 TB/s with the matrix pipes 36 %
+// busy, 64 -> 64 over 157 k 16 TB/s; behind the L2 it moves 2 to 5), and for few rows the longest tile.  Tried: 256-row
+// tiles of eight waves (a quarter to a half less weight traffic, one workgroup per CU: 10 to 30 % slower), deeper buffers with fewer workgroups
 // (the same or slower).  Tiles in descending length (the plan's order) instead of ascending: 128 -> 128 over 170 k rows
 // 116 -> 84 us, 256 -> 256 over 39 k rows 138 -> 89.
 #include <algorithm>

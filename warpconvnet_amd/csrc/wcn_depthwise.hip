@@ -19,7 +19,8 @@ using namespace wcn_rows;
 // is X[m] * W[identity] for every m < num_in and its pairs are ignored (sparse_conv_depth.py:163-165).
 // The bias is added to the rounded sum, as a separate addition behind the call would.
 //
-// Bound by the latency and then the rate of the gathered rows (a gather alone of these rows: 40 us).  LDS_W: the
+// Bound by the rate of the gathered rows (4.3 TB/s behind the L2; a gather alone of these rows: 40 us) and by the LDS that
+// the weights come from (two thirds of its cycles, most of them bank conflicts).  LDS_W: the
 // weight, as fp32, in LDS for the life of the workgroup, which takes many rows; read from memory instead, the
 // rows of a wave asked for eight different weight rows per entry, two 16-byte loads each beside the one of the
 // feature row.  Eight entries in flight and the next row's mask on its way: 500 k rows of 64 fp16
