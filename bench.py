@@ -273,9 +273,9 @@ def secondary_configs(dev, steps, warmup):
         "gathered_GBps": 2 * 64 * (L3 + n) / (t_dw * 1e-3) / 1e9}
     del km3
     # a consumer of the same strided map: 2x2x2 stride-2 max pooling of 64 fp16 channels
-    from warpconvnet_amd.nn.functional.sparse_pool import _SparsePoolFunction
+    from warpconvnet_amd._lib import host
     xp = torch.randn(n, 64, generator=torch.Generator().manual_seed(6)).to(torch.float16).to(dev)
-    t_pool, _ = timed(lambda: _SparsePoolFunction.apply(xp, km, m, 2))
+    t_pool, _ = timed(lambda: host().pool_autograd(xp, km, m, 2, True))
     pool_bytes = 2 * 64 * (n + m) + 4 * (n + m)
     out["max pooling 2x2x2 s2 over the configs[2] map, 64 channels fp16 (warm map)"] = {
         "num_voxels": n, "num_coarse": m, "call_ms": t_pool,

@@ -478,3 +478,19 @@ def test_take_rows_in_pieces_equals_plain_indexing(monkeypatch):
     mask = torch.arange(50) % 2 == 0
     assert torch.equal(gather.take_rows(src, mask), src[mask])
     assert torch.equal(gather.take_rows(src[:, 0], index), src[:, 0][index])
+
+
+def test_what_the_benchmark_and_the_entry_points_import_is_there():
+    """Their rarer options import inside functions: every name they take from the package exists."""
+    import ast
+    import importlib
+    for name in ("bench.py", "__graft_entry__.py", os.path.join("perf", "cases.py")):
+        found = 0
+        for node in ast.walk(ast.parse(open(os.path.join(ROOT, name)).read())):
+            if isinstance(node, ast.ImportFrom) and (node.module or "").startswith("warpconvnet_amd"):
+                module = importlib.import_module(node.module)
+                for alias in node.names:
+                    found += 1
+                    if not hasattr(module, alias.name):
+                        importlib.import_module(f"{node.module}.{alias.name}")
+        assert found > 0
