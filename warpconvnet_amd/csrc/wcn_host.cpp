@@ -203,7 +203,7 @@ py::tuple stride_cells(const py::object& table, const Int3& stride, bool want_bo
  * assumed size (`per_row` pairs a row), one wait for the offsets; with more pairs than assumed the
  * emit pass has written nothing and runs again into exact buffers.  Returns (in_maps, out_maps,
  * offsets int64, offsets int32, group starts (bytes) and their address, offsets in device memory, table
- * flags, where and when they were made). */
+ * flags, where (and, with work behind the wait, when) the lists were made). */
 py::tuple kernel_map(const py::object& table, const Tensor& out4, const Int3& ks, const Int3& st,
                      const std::optional<Int3>& dilation, const std::optional<Int3>& centre, double per_row,
                      int64_t keep_workspace_bytes) {
@@ -222,7 +222,7 @@ py::tuple kernel_map(const py::object& table, const Tensor& out4, const Int3& ks
   // a set mapped onto itself can also be probed block by block (opt-in; same results, a little slower)
   const char* probe = std::getenv("WCN_KMAP_PROBE");
   Tensor kept;
-  auto made = std::make_shared<MadeOn>(stream, true);
+  std::shared_ptr<MadeOn> made;  // where work on the lists was enqueued behind the wait
   int64_t begin = 0;
   while (true) {
     TableRef t(table);
@@ -288,7 +288,7 @@ py::tuple kernel_map(const py::object& table, const Tensor& out4, const Int3& ks
   const auto address = reinterpret_cast<uintptr_t>(groups.const_data_ptr());
   return py::make_tuple(in_buf, out_buf, offsets, offsets32, groups, address,
                         kept.narrow(0, 0, 8 * (int64_t{K} + 1)).view(at::kLong), wcn_kmap_last_table_flags(),
-                        made);
+                        made ? py::cast(made) : py::reinterpret_steal<py::object>(PyLong_FromVoidPtr(stream)));
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -313,13 +313,17 @@ struct MapRef {
     K = static_cast<int32_t>(offsets.numel() - 1);
     py::object id = km.attr("identity_map_index");
     if (!id.is_none()) identity = id.cast<int64_t>();
-    // a builder's lists, with the workspace's head behind them (offsets and group starts)
+    // A builder's lists, and the workspace's head with offsets and group starts, on another stream than the builder's.  `_made` is
+    // that stream where the host has waited for the lists.
     py::object made = km.attr("_made");
-    if (!made.is_none()) {
+    if (made.is_none()) return;
+    auto elsewhere = [&](const MadeOn& m) {
       py::object head = km.attr("_device_offsets");
       const Tensor h = head.is_none() ? Tensor() : head.cast<Tensor>();
-      made.cast<const MadeOn*>()->before_use({&in_maps, &out_maps, &h});
-    }
+      m.before_use({&in_maps, &out_maps, &h});
+    };
+    if (!PyLong_Check(made.ptr())) elsewhere(*made.cast<const MadeOn*>());
+    else if (void* const stream = PyLong_AsVoidPtr(made.ptr()); stream != stream_of(in_maps)) elsewhere(MadeOn(stream, true));
   }
   const int64_t* host_offsets() const { return offsets.const_data_ptr<int64_t>(); }
   int64_t pairs() const { return host_offsets()[K]; }

@@ -101,6 +101,10 @@ def _kernel_map_from_table(table: TorchHashTable, out_coords: Tensor, kernel_siz
     return result
 
 
+def _stream_of(t: Tensor):
+    return stream_ptr(t.device).value if t.is_cuda else None
+
+
 def _table_of(coords: Tensor, hash_method: HashMethod, device) -> TorchHashTable:
     """The coordinate table of an input tensor, built once per tensor object: the maps of
     different kernels over the same input rows (the 3x3x3 and the strided 2x2x2 map of one
@@ -110,8 +114,7 @@ def _table_of(coords: Tensor, hash_method: HashMethod, device) -> TorchHashTable
     interpreter free for other threads), it is for that stream alone.  (The reference builds a new
     table in every call, torch_discrete.py:398-401.)"""
     kept = getattr(coords, "_wcn_table", None)
-    stream = stream_ptr(coords.device).value if coords.is_cuda else None
-    if kept is not None and kept[0] == coords._version and (kept[1]._checked or kept[2] == stream):
+    if kept is not None and kept[0] == coords._version and (kept[1]._checked or kept[2] == _stream_of(coords)):
         return kept[1]
     # built from an alias of the tensor (same storage, another Python object): the table keeps its
     # keys alive, and keeping the table on `coords` itself would otherwise close a reference
@@ -122,7 +125,7 @@ def _table_of(coords: Tensor, hash_method: HashMethod, device) -> TorchHashTable
         table = TorchHashTable.from_keys(coords.detach(), hash_method=hash_method, device=device,
                                          _defer_check=True)
     try:
-        coords._wcn_table = (coords._version, table, stream)
+        coords._wcn_table = (coords._version, table, _stream_of(coords))
     except AttributeError:
         pass
     return table
