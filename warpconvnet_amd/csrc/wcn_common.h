@@ -229,6 +229,14 @@ __device__ __forceinline__ int wcn_rank_below(unsigned long long mask, uint32_t 
   return __popcll(mask & ((1ull << bit) - 1ull));
 }
 
+// Workgroups go to the eight XCDs in turn (blockIdx % 8), each with an L2 of its own.  For kernels whose
+// neighbouring tiles write into the same lines (a few bytes each) or read them: the tile of workgroup `b` of `n` so that an
+// XCD works through one stretch of tiles, and the pieces of a line meet in its L2.
+__device__ __forceinline__ int wcn_xcd_tile(int b, int n) {
+  const int xcd = b & 7, each = n >> 3, more = n & 7;
+  return xcd * each + (xcd < more ? xcd : more) + (b >> 3);
+}
+
 __device__ __forceinline__ int wcn_lane() { return (int)(threadIdx.x & 63); }
 
 // Inclusive prefix sum over the 64 lanes of a wave: shifts inside rows of 16 lanes, then the last lane of

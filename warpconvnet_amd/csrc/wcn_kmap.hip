@@ -3,12 +3,12 @@
 // The reference materialises a dense (K, M) table of probe results and compacts it with several
 // passes (torch_discrete.py:80-157).  Here one thread owns one output voxel and resolves its K
 // offsets in registers; a wave's 64 voxels form a "group".  The probe pass stores, per offset and
-// group, the 64-bit mask of lanes that hit and its popcount, and the hit lanes park the input
-// rows they found in the group's stretch of a scratch table, packed offset by offset and in lane
-// order (one contiguous piece per group, for the emit pass to read back).  A row-wise
-// exclusive scan turns the counts into start positions; the emit pass then reads masks, starts
-// and parked rows -- no table probes -- and every hit lane writes its pair at start + (number of
-// hits in lower lanes).  Because groups are 64 consecutive output rows and lanes ascend within a
+// group, the number of lanes that hit, and parks what they found in the group's stretch of a
+// scratch table, packed offset by offset and in lane order (one contiguous piece per group, for the
+// emit pass to read back): the input row, and a tag of offset and lane.  A row-wise
+// exclusive scan turns the counts into start positions; the emit pass then reads starts, tags
+// and parked rows -- no table probes -- and writes pair p of a group at p + (start of its offset -
+// hits of the group in the offsets before).  Because groups are 64 consecutive output rows and lanes ascend within a
 // group, pairs come out in ascending output index for each offset, exactly the reference's order
 // (discrete_kernels.cu:183-213).
 #include "wcn_common.h"
@@ -33,8 +33,8 @@ struct KmapWorkspace {  // host-computed addresses inside a kmap workspace
   int32_t* ticket;      // arrival counter of the scan's workgroups (zeroed by the probe pass)
   int32_t* groups;      // (K+1, G+1): rows 0..K-1 per-offset hit counts of each 64-row group, row K
                         // all hits of the group; after the scan, exclusive prefix sums
-  unsigned long long* hits;  // (G, K): lanes of the group that hit, per offset
   int32_t* found;       // (G, 64 K): input rows found by the hit lanes of a group, packed offset by offset
+  uint16_t* tags;       // (G, 64 K): offset << 6 | lane of each of them
   int64_t G;            // number of 64-row groups
 };
 
@@ -50,10 +50,11 @@ inline size_t kmap_layout(void* base, int64_t num_out, int32_t K, KmapWorkspace*
   off += 256;
   if (w) w->groups = (int32_t*)(p + off);
   off += wcn_align256(sizeof(int32_t) * (size_t)(K + 1) * (size_t)(G + 1));
-  if (w) w->hits = (unsigned long long*)(p + off);
-  off += wcn_align256(sizeof(unsigned long long) * (size_t)K * (size_t)G);
   if (w) w->found = (int32_t*)(p + off);
   off += wcn_align256(sizeof(int32_t) * (size_t)K * (size_t)G * 64);
+  static_assert(WCN_MAX_OFFSETS <= 1024, "offset and lane share 16 bits");
+  if (w) w->tags = (uint16_t*)(p + off);
+  off += wcn_align256(sizeof(uint16_t) * (size_t)K * (size_t)G * 64);
   if (w) w->G = G;
   return off;
 }
@@ -64,8 +65,8 @@ inline int grid_for(int64_t n, int block) {
 }
 
 struct KmapProbe {      // what the probe pass leaves for the scan and the emit pass
-  unsigned long long* hits;
   int32_t* found;
+  uint16_t* tags;
   int32_t* ticket;      // set to zero
 };
 
@@ -115,12 +116,12 @@ __global__ void __launch_bounds__(256) kmap_pass(const WcnTableHeader* __restric
         }
         const unsigned long long hits = __ballot(found >= 0);
         const int cnt = __popcll(hits);
-        if (lane == 0) {
-          groups[(int64_t)k * (G + 1) + group] = cnt;
-          o.hits[group * g.K + k] = hits;
+        if (lane == 0) groups[(int64_t)k * (G + 1) + group] = cnt;
+        if (found >= 0) {  // hits of a group are parked contiguously: offset by offset, in lane order
+          const int64_t at = group * (64 * (int64_t)g.K) + group_hits + __popcll(hits & ((1ull << lane) - 1ull));
+          o.found[at] = found;
+          o.tags[at] = (uint16_t)(k << 6 | lane);
         }
-        if (found >= 0)  // hits of a group are parked contiguously: offset by offset, in lane order
-          o.found[group * (64 * (int64_t)g.K) + group_hits + __popcll(hits & ((1ull << lane) - 1ull))] = found;
         group_hits += cnt;
       }
     }
@@ -131,9 +132,16 @@ __global__ void __launch_bounds__(256) kmap_pass(const WcnTableHeader* __restric
 // ---- fixed-size kernel: compile-time kernel size, every dimension spans at most 2 blocks -------
 // Phase 1 requests the (up to) 8 block slots the neighbourhood can touch, all at once, so their
 // memory latencies overlap (3x3x3 over 2 k rows 12.6 -> 9.4 us, over 1 M 89 -> 83, 5x5x5 over 1 M 245 -> 231, against
-// eight conditional requests that waited for one another); phase 2 derives the hit bit of each of the K offsets from the cached
-// masks (no memory traffic); phase 3 reads the hit rows from `perm`, again as independent loads,
-// and leaves masks, counts and rows for the emit pass.
+// eight conditional requests that waited for one another), and keeps them in LDS as half blocks: 32 bits of
+// occupancy and the position of their first voxel in `perm`.
+// Phase 2 takes the KZ offsets of a (x, y) row of the kernel out of the two words that hold them, and appends a tag
+// (offset, lane) per hit to the wave's list, in the order in which pairs are parked.
+// Phase 3 empties the list 64 hits at a time, a lane per HIT: position in `perm` from the half block of the hit's own row, the row
+// from there, and both stores full.  Phases 2 and 3 alternate over a few rows of the kernel, so that the list
+// stays short; a round's row is stored when the next round's has been requested.
+// Against a mask, a rank and two predicated accesses per offset and lane: 3x3x3 over 1 M rows of rooms 85.5 -> 79.5 us, 5x5x5
+// 228 -> 187 (2,990 vector instructions a wave where 27 and 125 offsets' worth of 64-bit ranks took most of the time).  What bounds it
+// now: instruction issue (29 % of the wave cycles) and the texture addresser (61 % busy), both with scattered requests.
 template <int KX, int KY, int KZ>
 __global__ void __launch_bounds__(256) kmap_pass_fixed(const WcnTableHeader* __restrict__ hdr,
                                                        const WcnSlot* __restrict__ slots,
@@ -143,16 +151,19 @@ __global__ void __launch_bounds__(256) kmap_pass_fixed(const WcnTableHeader* __r
                                                        int64_t num_out, KmapGeom g,
                                                        int32_t* __restrict__ groups, int64_t G,
                                                        KmapProbe o) {
-  constexpr int K = KX * KY * KZ;
+  constexpr int K = KX * KY * KZ, ROWS = KX * KY;
   static_assert(KX <= 5 && KY <= 5 && KZ <= 5, "a kernel of up to five voxels spans at most two blocks per dimension");
-  __shared__ unsigned long long s_mask[8][256];
-  __shared__ int32_t s_base[8][256];
+  constexpr int TURN = 10 / KZ < ROWS ? 10 / KZ : ROWS;  // rows of the kernel between two visits to the list
+  constexpr int LIST = 64 * TURN * KZ + 64;              // all of them hit, and up to 63 left over
+  __shared__ uint2 s_half[16][256];  // [block * 2 + upper half of x][thread]: occupancy, position of the first voxel
+  __shared__ uint16_t s_list[4][LIST];
+  __shared__ uint8_t s_sub[256];     // place of the first neighbour in its block: x | y << 2 | z << 4
+  __shared__ int32_t s_count[4][K + 1];
   const int tid = threadIdx.x;
-  const int64_t m = (int64_t)blockIdx.x * blockDim.x + tid;
+  const int64_t m = (int64_t)wcn_xcd_tile((int)blockIdx.x, (int)gridDim.x) * 256 + tid;
   if (m == 0) *o.ticket = 0;
   const int64_t group = m >> 6;  // wave-uniform
-  if (group >= G) return;
-  const int lane = wcn_lane();
+  const int lane = wcn_lane(), wave = tid >> 6;
   const bool live = m < num_out;
   const WcnLayout L = wcn_make_layout(hdr);
   const int4 c = out_coords[live ? m : num_out - 1];
@@ -162,6 +173,7 @@ __global__ void __launch_bounds__(256) kmap_pass_fixed(const WcnTableHeader* __r
                           (uint32_t)c.w * (uint32_t)g.sz - (uint32_t)g.cz - L.amin[3]};
   const bool usable = live & (bool)L.ok & (rb <= L.span[0]);
   constexpr int KD[3] = {KX, KY, KZ};
+  s_sub[tid] = (uint8_t)((r0[0] & 3u) | ((r0[1] & 3u) << 2) | ((r0[2] & 3u) << 4));
 
   // candidate block coordinates per dimension: the block of the first neighbour and the next one
   uint32_t cand[3][2];
@@ -207,84 +219,167 @@ __global__ void __launch_bounds__(256) kmap_pass_fixed(const WcnTableHeader* __r
     const unsigned long long k0 = ((unsigned long long)lo[e].y << 32) | lo[e].x;
     const bool same = need[e] && k0 == key[e];
     if (need[e] && !same && k0 != WCN_EMPTY_KEY) walk |= 1u << e;
-    s_mask[e][tid] = same ? ((unsigned long long)lo[e].w << 32) | lo[e].z : 0ull;
-    s_base[e][tid] = same ? hi[e] : 0;
+    s_half[2 * e][tid] = make_uint2(same ? lo[e].z : 0u, (uint32_t)hi[e]);
+    s_half[2 * e + 1][tid] = make_uint2(same ? lo[e].w : 0u, (uint32_t)hi[e] + (uint32_t)__popc(lo[e].z));
   }
   while (walk != 0) {
     const int e = __ffs((int)walk) - 1;
     walk &= walk - 1;
     const unsigned long long wanted = block_key(e);
     int32_t base = 0;
-    s_mask[e][tid] = wcn_lookup_block_from(slots, cap_mask, wanted, (wcn_mix(wanted, cap_mask) + 1) & cap_mask, 1, &base);
-    s_base[e][tid] = base;
+    const unsigned long long mask =
+        wcn_lookup_block_from(slots, cap_mask, wanted, (wcn_mix(wanted, cap_mask) + 1) & cap_mask, 1, &base);
+    s_half[2 * e][tid] = make_uint2((uint32_t)mask, (uint32_t)base);
+    s_half[2 * e + 1][tid] = make_uint2((uint32_t)(mask >> 32), (uint32_t)base + (uint32_t)__popc((uint32_t)mask));
   }
-  // no barrier: every thread reads back only its own column
+  // no barrier: a wave reads back only what it has written itself (its lanes' columns, its list)
+  auto written = [] {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  };
+  written();
 
-  // Offsets are handled NI planes (values of the slowest kernel index) at a time: all of a small
-  // kernel at once, one plane of KY x KZ offsets at a time for 4x4x4 and 5x5x5 (the per-offset
-  // positions and rows live in registers).
-  constexpr int NI = K <= 32 ? KX : 1, PER = NI * KY * KZ;
-  static_assert(PER <= 32, "one plane fits a 32-bit hit mask");
-  int group_hits = 0;
+  int32_t* const found = o.found + group * (64 * (int64_t)K);
+  uint16_t* const tags = o.tags + group * (64 * (int64_t)K);
+  uint16_t* const list = s_list[wave];
+  int count[2] = {0, 0};
+  int pending = 0, parked = 0;  // hits in the list, hits parked (the same in all lanes)
+  int32_t last = 0;             // what the last round has found, not stored yet
+  int last_at = -1;
+  auto empty = [&](int first, int n) {  // n <= 64 hits of the list from `first` on
+    const bool mine = lane < n;
+    const uint32_t t = list[first + (mine ? lane : 0)];
+    const int k = (int)(t >> 6), src = (wave << 6) | (int)(t & 63u);
+    const uint32_t sub = s_sub[src];
+    const uint32_t ax = (sub & 3u) + (uint32_t)(k / (KY * KZ)), ay = ((sub >> 2) & 3u) + (uint32_t)(k / KZ % KY),
+                   az = (sub >> 4) + (uint32_t)(k % KZ);
+    const uint2 half = s_half[((ax >> 2) << 3) | ((ay >> 2) << 2) | ((az >> 2) << 1) | ((ax >> 1) & 1u)][src];
+    const uint32_t bit = ((ax & 1u) << 4) | ((ay & 3u) << 2) | (az & 3u);
+    const uint32_t at = half.y + (uint32_t)__popc(__builtin_amdgcn_ubfe(half.x, 0u, bit));
+    const int32_t row = perm[mine ? at : 0u];
+    if (mine) tags[parked + lane] = (uint16_t)t;
+    if (last_at >= 0) found[last_at] = last;
+    last = row;
+    last_at = mine ? parked + lane : -1;
+    parked += n;
+  };
 #pragma nounroll
-  for (int i0 = 0; i0 < KX; i0 += NI) {
-    uint32_t hm = 0;
-    int32_t pos[PER];
-    {
-      int q = 0;
+  for (int row0 = 0; row0 < ROWS; row0 += TURN) {
 #pragma unroll
-      for (int di = 0; di < NI; ++di) {
+    for (int r = 0; r < TURN; ++r) {
+      const int row = row0 + r;
+      if (ROWS % TURN != 0 && row >= ROWS) break;
+      const uint32_t ax = (r0[0] & 3u) + (uint32_t)(row / KY), ay = (r0[1] & 3u) + (uint32_t)(row % KY);
+      const uint32_t e = ((ax >> 2) << 3) | ((ay >> 2) << 2) | ((ax >> 1) & 1u), bit = ((ax & 1u) << 4) | ((ay & 3u) << 2);
+      const uint32_t near = __builtin_amdgcn_ubfe(s_half[e][tid].x, bit, 4u), far = __builtin_amdgcn_ubfe(s_half[e + 2][tid].x, bit, 4u);
+      const uint32_t hit = (near | (far << 4)) >> (r0[2] & 3u);
 #pragma unroll
-        for (int j = 0; j < KY; ++j) {
-#pragma unroll
-          for (int kk = 0; kk < KZ; ++kk, ++q) {
-            const uint32_t ax = (r0[0] & 3u) + (uint32_t)(i0 + di), ay = (r0[1] & 3u) + j, az = (r0[2] & 3u) + kk;
-            const int e = (int)(((ax >> 2) << 2) | ((ay >> 2) << 1) | (az >> 2));
-            const uint32_t bit = ((ax & 3u) << 4) | ((ay & 3u) << 2) | (az & 3u);
-            const unsigned long long mk = s_mask[e][tid];
-            const uint32_t hit = (uint32_t)((mk >> bit) & 1ull);
-            hm |= hit << q;
-            pos[q] = s_base[e][tid] + wcn_rank_below(mk, bit);
-          }
-        }
+      for (int kk = 0; kk < KZ; ++kk) {
+        const unsigned long long hits = __ballot((hit >> kk) & 1u);
+        if ((hit >> kk) & 1u)
+          list[pending + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(hits >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)hits, 0u))] =
+              (uint16_t)((row * KZ + kk) << 6 | lane);
+        const int n = __popcll(hits);
+        pending += n;
+        const int k = row * KZ + kk;  // lane k % 64 keeps the count
+        if (K <= 64 || k < 64) count[0] = lane == k ? n : count[0];
+        else count[1] = lane == k - 64 ? n : count[1];
       }
     }
-
-    int32_t found[PER];
-#pragma unroll
-    for (int q = 0; q < PER; ++q) found[q] = ((hm >> q) & 1u) ? perm[pos[q]] : -1;
-
-    // lane q keeps the lanes that hit with offset q: two stores for all of them
-    uint32_t mine_lo = 0, mine_hi = 0;
-    int32_t* const parked = o.found + group * (64 * (int64_t)K) + group_hits;
-    int before = 0;
-#pragma unroll
-    for (int q = 0; q < PER; ++q) {
-      const bool hit = (hm >> q) & 1u;
-      const unsigned long long hits = __ballot(hit);
-      mine_lo = lane == q ? (uint32_t)hits : mine_lo;
-      mine_hi = lane == q ? (uint32_t)(hits >> 32) : mine_hi;
-      if (hit)  // hits of a group are parked contiguously: offset by offset, in lane order
-        parked[before + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(hits >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)hits, 0u))] = found[q];
-      before += __popcll(hits);
-    }
-    group_hits += before;
-    if (lane < PER) {
-      const int k = i0 * KY * KZ + lane;
-      o.hits[group * K + k] = ((unsigned long long)mine_hi << 32) | mine_lo;
-      groups[(int64_t)k * (G + 1) + group] = __popc(mine_lo) + __popc(mine_hi);
+    written();
+    int first = 0;
+    for (; pending >= 64; pending -= 64, first += 64) empty(first, 64);
+    if (first > 0 && pending > 0) {  // what is left moves to the front
+      const uint16_t t = list[first + lane];
+      written();
+      list[lane] = t;
+      written();
     }
   }
-  if (lane == 0) groups[(int64_t)K * (G + 1) + group] = group_hits;
+  if (pending > 0) empty(0, pending);
+  if (last_at >= 0) found[last_at] = last;
+  if (lane < K) s_count[wave][lane] = count[0];
+  if (K > 64 && 64 + lane < K) s_count[wave][64 + lane] = count[1];
+  if (lane == 0) s_count[wave][K] = parked;
+  __syncthreads();
+  // the counts of four neighbouring groups lie beside each other
+  const int there = (int)(G - (group - wave) < 4 ? G - (group - wave) : 4);
+  for (int i = tid; i < 4 * (K + 1); i += 256)
+    if ((i & 3) < there) groups[(int64_t)(i >> 2) * (G + 1) + (group - wave) + (i & 3)] = s_count[i & 3][i >> 2];
 }
 
-// Emit pass: pair lists from the masks, scanned counts and parked rows of the probe pass, a lane per
+// Emit pass: pair lists from the scanned counts and what the probe pass has parked, a lane per
 // PAIR.  The parked rows of a group already lie in the order of its pairs (offset by offset, in lane
-// order), so for 64 offsets at a time (lane j fetches mask and start of offset k0 + j) lane p of a
-// round takes pair p, p + 64, ... of those offsets, finds the offset it belongs to (binary search
-// over the running counts the lanes hold), its rank there, and from rank and mask the output row.
-// A group's ~270 pairs of a 3x3x3 map cost five rounds of one load and two stores where a walk over
-// the offsets costs one load and two stores of a few lanes each per offset (5x5x5: 154 -> 85 us).
+// order), so pair p of the group goes to p + (start of its offset in the lists - hits of the group in the
+// offsets before); tag and row are read side by side, four rounds in flight.  The starts of a workgroup's neighbouring groups are
+// fetched together (they lie beside each other, one piece per offset).
+// LDS: 8 * EMIT_GROUPS + 4 * (EMIT_GROUPS + 1) bytes per offset.  Against a search for the pair's offset and lane in the hit masks, and
+// workgroups in turn over the XCDs (eight runs of 22 bytes and more meet in a line): 3x3x3 over 1 M rows 23.7 -> 20 us,
+// 5x5x5 60 -> 47.5, of which the XCDs' stretches are 1 and 8.
+template <int EMIT_GROUPS>
+__global__ void __launch_bounds__(64 * EMIT_GROUPS) kmap_emit(const int32_t* __restrict__ found,
+                                                              const uint16_t* __restrict__ tags,
+                                                              const int32_t* __restrict__ groups,
+                                                              const int64_t* __restrict__ offsets, int K,
+                                                              int64_t G, int64_t pair_capacity,
+                                                              int32_t* __restrict__ in_maps,
+                                                              int32_t* __restrict__ out_maps) {
+  // offsets[K] = number of pairs, offsets[K + 1] = table status bits (written by the scan): the
+  // pass may have been enqueued before the host has seen either, so it checks them itself
+  if (offsets[K] > pair_capacity || offsets[K + 1] != 0) return;
+  extern __shared__ __attribute__((aligned(16))) char emit_lds[];
+  int64_t* const s_shift = reinterpret_cast<int64_t*>(emit_lds);              // [EMIT_GROUPS][K]
+  int32_t* const s_start = reinterpret_cast<int32_t*>(s_shift + EMIT_GROUPS * K);  // [K][EMIT_GROUPS + 1]
+  const int64_t first = (int64_t)wcn_xcd_tile((int)blockIdx.x, (int)gridDim.x) * EMIT_GROUPS;
+  const int lane = wcn_lane(), wave = (int)(threadIdx.x >> 6);
+  for (int i = (int)threadIdx.x; i < K * (EMIT_GROUPS + 1); i += 64 * EMIT_GROUPS) {
+    const int k = i / (EMIT_GROUPS + 1), j = i % (EMIT_GROUPS + 1);
+    const int64_t g = first + j < G ? first + j : G;  // entry G holds the offset's total
+    s_start[i] = groups[(int64_t)k * (G + 1) + g];
+  }
+  __syncthreads();
+  const int64_t group = first + wave;
+  if (group >= G) return;
+  int total = 0;
+  for (int k0 = 0; k0 < K; k0 += 64) {
+    const int k = k0 + lane;
+    int n = 0, start = 0;
+    if (k < K) {
+      start = s_start[k * (EMIT_GROUPS + 1) + wave];
+      n = s_start[k * (EMIT_GROUPS + 1) + wave + 1] - start;
+    }
+    const int incl = wcn_wave_inclusive_sum(n);
+    if (k < K) s_shift[wave * K + k] = offsets[k] + start - (total + incl - n);
+    total += __shfl(incl, 63, 64);
+  }
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  const int32_t* const rows = found + group * (64 * (int64_t)K);
+  const uint16_t* const of = tags + group * (64 * (int64_t)K);
+  constexpr int AHEAD = 4;
+  for (int p0 = 0; p0 < total; p0 += 64 * AHEAD) {
+    int32_t row[AHEAD];
+    uint32_t tag[AHEAD];
+#pragma unroll
+    for (int u = 0; u < AHEAD; ++u) {
+      const int p = p0 + 64 * u + lane;
+      row[u] = rows[p < total ? p : 0];
+      tag[u] = of[p < total ? p : 0];
+    }
+#pragma unroll
+    for (int u = 0; u < AHEAD; ++u) {
+      const int p = p0 + 64 * u + lane;
+      if (p < total) {
+        const int64_t dst = s_shift[wave * K + (int)(tag[u] >> 6)] + p;
+        in_maps[dst] = row[u];
+        out_maps[dst] = (int32_t)(group * 64) + (int32_t)(tag[u] & 63u);
+      }
+    }
+  }
+}
+
 __device__ __forceinline__ int kmap_nth_set_bit(unsigned long long mask, int r) {  // position of the r-th set bit (r counts from 0)
   uint32_t w = (uint32_t)mask;
   int pos = 0;
@@ -307,56 +402,6 @@ __device__ __forceinline__ int kmap_nth_set_bit(unsigned long long mask, int r) 
     }
   }
   return pos;
-}
-
-__global__ void __launch_bounds__(256) kmap_emit_flat(const unsigned long long* __restrict__ hits,
-                                                      const int32_t* __restrict__ found,
-                                                      const int32_t* __restrict__ groups,
-                                                      const int64_t* __restrict__ offsets, int K,
-                                                      int64_t G, int64_t pair_capacity,
-                                                      int32_t* __restrict__ in_maps,
-                                                      int32_t* __restrict__ out_maps) {
-  const int64_t m = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int64_t group = m >> 6;  // wave-uniform
-  if (group >= G) return;
-  // offsets[K] = number of pairs, offsets[K + 1] = table status bits (written by the scan): the
-  // pass may have been enqueued before the host has seen either, so it checks them itself
-  if (offsets[K] > pair_capacity || offsets[K + 1] != 0) return;
-  const int lane = wcn_lane();
-  const int32_t* parked = found + group * (64 * (int64_t)K);
-  for (int k0 = 0; k0 < K; k0 += 64) {  // 64 offsets at a time, a lane per offset
-    unsigned long long h = 0ull;
-    long long st = 0;
-    if (k0 + lane < K) {
-      h = hits[group * K + k0 + lane];
-      st = offsets[k0 + lane] + groups[(int64_t)(k0 + lane) * (G + 1) + group];
-    }
-    const int cnt = __popcll(h);
-    const int incl = wcn_wave_inclusive_sum(cnt);  // pairs of these offsets up to and including this lane's
-    const int total = __shfl(incl, 63, 64);
-    for (int p0 = 0; p0 < total; p0 += 64) {
-      const int p = p0 + lane;
-      const bool live = p < total;
-      // first offset whose running count exceeds p (lanes past the last offset hold the total: never chosen by a live p)
-      int lo = 0, hi = 63;
-#pragma unroll
-      for (int step = 0; step < 6; ++step) {
-        const int mid = (lo + hi) >> 1;
-        const int v = __shfl(incl, mid, 64);
-        if (v <= p) lo = mid + 1; else hi = mid;
-      }
-      const int k = lo;
-      const unsigned long long hk = __shfl(h, k, 64);
-      const long long sk = __shfl(st, k, 64);
-      const int rank = p - (__shfl(incl, k, 64) - __popcll(hk));
-      if (live) {
-        const long long dst = sk + rank;
-        in_maps[dst] = parked[p];
-        out_maps[dst] = (int32_t)(group * 64 + kmap_nth_set_bit(hk, rank));
-      }
-    }
-    parked += total;  // the next 64 offsets' rows follow
-  }
 }
 
 // In-place exclusive prefix sum of each row of `groups` (one workgroup per row, G+1 entries; the
@@ -986,7 +1031,7 @@ void launch_probe(const WcnTableView& v, const int32_t* out_coords, int64_t num_
                   const KmapGeom& g, const KmapWorkspace& w, hipStream_t s) {
   const dim3 grid(grid_for(num_out, 256)), block(256);
   const uint32_t cap_mask = (uint32_t)(v.capacity - 1);
-  const KmapProbe o = {w.hits, w.found, w.ticket};
+  const KmapProbe o = {w.found, w.tags, w.ticket};
   if (is_fixed_size(g, 3, 3, 3)) {
     hipLaunchKernelGGL((kmap_pass_fixed<3, 3, 3>), grid, block, 0, s, v.hdr, v.slots, cap_mask,
                        v.perm, (const int4*)out_coords, num_out, g, w.groups, w.G, o);
@@ -1004,10 +1049,15 @@ void launch_probe(const WcnTableView& v, const int32_t* out_coords, int64_t num_
 
 void launch_emit(int64_t num_out, const KmapGeom& g, const KmapWorkspace& w, int64_t pair_capacity,
                  int32_t* in_maps, int32_t* out_maps, hipStream_t s) {
-  const dim3 grid(grid_for(num_out, 256)), block(256);
+  // eight groups a workgroup (100 bytes of LDS per offset), two where that would be more than 32 KB
   const int64_t* offsets = (const int64_t*)w.result;
-  hipLaunchKernelGGL(kmap_emit_flat, grid, block, 0, s, w.hits, w.found, w.groups, offsets, g.K,
-                     w.G, pair_capacity, in_maps, out_maps);
+  if (g.K <= 320) {
+    hipLaunchKernelGGL(kmap_emit<8>, dim3(grid_for(num_out, 512)), dim3(512), 100u * (unsigned)g.K, s, w.found, w.tags,
+                       w.groups, offsets, g.K, w.G, pair_capacity, in_maps, out_maps);
+  } else {
+    hipLaunchKernelGGL(kmap_emit<2>, dim3(grid_for(num_out, 128)), dim3(128), 28u * (unsigned)g.K, s, w.found, w.tags,
+                       w.groups, offsets, g.K, w.G, pair_capacity, in_maps, out_maps);
+  }
 }
 
 // ---- strided output coordinates -----------------------------------------------------------------

@@ -38,10 +38,10 @@ __device__ __forceinline__ uint32_t bin_of(const int4 c, uint32_t bin_mask) {
 struct PartRange {
   int64_t lo, hi;
 };
-__device__ __forceinline__ PartRange part_range(int64_t n_keys) {
+__device__ __forceinline__ PartRange part_range(int64_t n_keys, int part) {
   const int64_t chunk = (n_keys + gridDim.x - 1) / gridDim.x;
   PartRange r;
-  r.lo = (int64_t)blockIdx.x * chunk;
+  r.lo = (int64_t)part * chunk;
   r.hi = r.lo + chunk < n_keys ? r.lo + chunk : n_keys;
   return r;
 }
@@ -60,12 +60,12 @@ __global__ void __launch_bounds__(1024) table_hist(const int4* __restrict__ keys
   extern __shared__ int s_cnt[];  // [bins]
   __shared__ int s_mn[16][4];
   __shared__ int s_mx[16][4];
-  const int tid = threadIdx.x, parts = gridDim.x, part = blockIdx.x;
+  const int tid = threadIdx.x, parts = gridDim.x, part = wcn_xcd_tile((int)blockIdx.x, parts);
   for (int b = tid; b < bins; b += 1024) s_cnt[b] = 0;
   __syncthreads();
   int mn[4] = {INT32_MAX, INT32_MAX, INT32_MAX, INT32_MAX};
   int mx[4] = {INT32_MIN, INT32_MIN, INT32_MIN, INT32_MIN};
-  const PartRange r = part_range(n_keys);
+  const PartRange r = part_range(n_keys, part);
   const uint32_t bin_mask = (uint32_t)bins - 1u;
   constexpr int PER = 4;  // keys a thread has in flight together
   for (int64_t i0 = r.lo + tid; i0 < r.hi; i0 += 1024 * PER) {
@@ -143,7 +143,8 @@ __global__ void __launch_bounds__(256) table_colscan(int32_t* __restrict__ hist,
 
 // Every key and its row to its place in its bin.  Each workgroup scans the bin totals into bin
 // starts for itself (1024 x BPT numbers); workgroup 0 also stores them for the next pass,
-// merges the parts' bounding boxes and writes the header.
+// merges the parts' bounding boxes and writes the header.  Parts that follow one another run on one XCD: their pieces
+// of a bin (eight keys of 1 M: 128 bytes, 32 of rows) follow one another too (1 M keys: 25 -> 21.5 us).
 template <int BPT>
 __global__ void __launch_bounds__(1024) table_scatter(const int4* __restrict__ keys, int64_t n_keys,
                                                       int32_t bins, const int32_t* __restrict__ hist,
@@ -157,8 +158,8 @@ __global__ void __launch_bounds__(1024) table_scatter(const int4* __restrict__ k
   extern __shared__ int s_cur[];  // [bins]
   __shared__ int s_wave[16];
   const int tid = threadIdx.x, lane = wcn_lane(), wave = tid >> 6;
-  const int parts = gridDim.x, part = blockIdx.x;
-  const PartRange r = part_range(n_keys);
+  const int parts = gridDim.x, part = wcn_xcd_tile((int)blockIdx.x, parts);
+  const PartRange r = part_range(n_keys, part);
   constexpr int PER = 4;
   int4 c[PER];  // the first keys are requested before anything else
 #pragma unroll
