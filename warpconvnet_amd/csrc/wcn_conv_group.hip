@@ -23,6 +23,7 @@
 //   * the additions of a row happen in a fixed order: results are bitwise reproducible.
 #include <algorithm>
 #include <mutex>
+#include <type_traits>
 
 #include "wcn_common.h"
 #include "wcn_conv_args.h"
@@ -37,18 +38,24 @@ constexpr int GROUP_ENTRIES = 16;  // blocks whose pair-list entries are on thei
 
 typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
 typedef short s16x4 __attribute__((ext_vector_type(4)));
+typedef float f32x8 __attribute__((ext_vector_type(8), aligned(16)));
 
 // MFMA operands of a block of 16 pairs: 8 channels per lane (16x16x32) or, for rows of at most 16
-// channels, 4 (16x16x16).
+// channels, 4 (16x16x16).  fp32: the same channels per lane, one 16x16x4 product for the first channel of
+// every lane, one for the second, and so on.
 template <typename T, bool HALF_K>
 struct GroupOp;
 template <typename T>
-struct GroupOp<T, false> {
+struct GroupOpWide {
   typedef typename Mma<T>::V V;
   static constexpr int PER_LANE = 8;
   static __device__ __forceinline__ V zero() { return Mma<T>::zero(); }
   static __device__ __forceinline__ f32x4 mma(V a, V b, f32x4 c) { return Mma<T>::mma(a, b, c); }
 };
+template <>
+struct GroupOp<_Float16, false> : GroupOpWide<_Float16> {};
+template <>
+struct GroupOp<__bf16, false> : GroupOpWide<__bf16> {};
 template <>
 struct GroupOp<_Float16, true> {
   typedef f16x4 V;
@@ -68,6 +75,17 @@ struct GroupOp<__bf16, true> {
   }
 };
 
+template <bool HALF_K>
+struct GroupOp<float, HALF_K> {
+  typedef typename std::conditional<HALF_K, f32x4, f32x8>::type V;
+  static constexpr int PER_LANE = HALF_K ? 4 : 8;
+  static __device__ __forceinline__ V zero() { return (V)(0.f); }
+  static __device__ __forceinline__ f32x4 mma(V a, V b, f32x4 c) {
+#pragma unroll
+    for (int e = 0; e < PER_LANE; ++e) c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[e], b[e], c, 0, 0, 0);
+    return c;
+  }
+};
 // NCB: 16-channel blocks of output; NCH: 64s of kernel offsets; WAVES: groups in work per workgroup
 template <typename T, int NCB, bool HALF_K, int NCH, int WAVES>
 __global__ void __launch_bounds__(WAVES * 64) conv_fwd_group(ConvArgs a) {
@@ -104,6 +122,16 @@ __global__ void __launch_bounds__(WAVES * 64) conv_fwd_group(ConvArgs a) {
   // 16 bytes each, so that the 16 rows one instruction touches spread over the banks and an
   // address is one shift-and-add away from the row number
   auto granule = [&](int r, int gi) -> f32x4* { return reinterpret_cast<f32x4*>(acc) + gi * 65 + r; };
+  // fp32 rows of other than 16 or 32 channels: what such a lane has read is cleared before the product, bit by bit (an
+  // infinite feature stays infinite; 16-bit rows keep the NaN of infinity times a zero of padding).
+  const uint32_t keep = has_c ? ~0u : 0u;
+  auto existing = [&](V x) -> V {
+    if constexpr (std::is_same<T, float>::value) {
+#pragma unroll
+      for (int e = 0; e < PER; ++e) x[e] = __uint_as_float(__float_as_uint(x[e]) & keep);
+    }
+    return x;
+  };
   // 8 (4) channels of input row idx.  No lane is switched off and nothing is replaced by zeros
   // afterwards (a select fed by a load is turned into a branch around the load, and the straight
   // line is gone): a pair that does not exist reads row 0 and adds its product to the spare row of
@@ -122,7 +150,7 @@ __global__ void __launch_bounds__(WAVES * 64) conv_fwd_group(ConvArgs a) {
       sum[cb] = *at[cb];
     }
 #pragma unroll
-    for (int cb = 0; cb < NCB; ++cb) sum[cb] = Op::mma(s_w[(k * NCB + cb) * 64 + lane], xv, sum[cb]);
+    for (int cb = 0; cb < NCB; ++cb) sum[cb] = Op::mma(s_w[(k * NCB + cb) * 64 + lane], existing(xv), sum[cb]);
 #pragma unroll
     for (int cb = 0; cb < NCB; ++cb) *at[cb] = sum[cb];
   };
@@ -233,7 +261,7 @@ __global__ void __launch_bounds__(WAVES * 64) conv_fwd_group(ConvArgs a) {
           }
         }
         f32x4 d = (f32x4){0.f, 0.f, 0.f, 0.f};
-        if (with_identity) d = Op::mma(s_w[(a.identity * NCB + cb) * 64 + lane], xv, d);
+        if (with_identity) d = Op::mma(s_w[(a.identity * NCB + cb) * 64 + lane], existing(xv), d);
         if (!here) d = (f32x4){0.f, 0.f, 0.f, 0.f};
         *granule(rb * 16 + pr, cb * 4 + kg) = d + (f32x4){start[0], start[1], start[2], start[3]};
       }
@@ -315,7 +343,9 @@ __global__ void __launch_bounds__(WAVES * 64) conv_fwd_group(ConvArgs a) {
           T t[8];
 #pragma unroll
           for (int e = 0; e < 8; ++e) t[e] = from_float<T>(v[e]);
-          *reinterpret_cast<u32x4*>(dst) = *reinterpret_cast<const u32x4*>(t);
+#pragma unroll
+          for (int e = 0; e < 8; e += 16 / (int)sizeof(T))
+            *reinterpret_cast<u32x4*>(dst + e) = *reinterpret_cast<const u32x4*>(t + e);
         } else {
 #pragma unroll
           for (int e = 0; e < 8; ++e)
@@ -376,12 +406,22 @@ int launch_group_waves(const ConvArgs& a, hipStream_t s) {
 // sums per wave).  The instances for 32 input channels under more than 64 offsets do not stay
 // within the 128 registers of sixteen waves (one has weights that fit LDS for no such kernel anyway,
 // the other would spill a few registers): they are built for twelve waves only.
+// fp32 weights are twice as large: those of 5x5x5 16 -> 16 leave room for eight waves.
+template <typename T, bool HALF_K>
+constexpr int group_fewest_waves() {
+  return std::is_same<T, float>::value && HALF_K ? 8 : 12;
+}
+
 template <typename T, int NCB, bool HALF_K, int NCH>
 int launch_group_chunks(const ConvArgs& a, hipStream_t s) {
-  if constexpr (!(!HALF_K && NCH == 2)) {
+  constexpr bool fp32 = std::is_same<T, float>::value;
+  if constexpr (fp32 ? HALF_K && NCH == 1 : HALF_K || NCH == 1) {
     if (group_lds<T, NCB, HALF_K>(a.K, 16) <= GROUP_LDS_MAX) return launch_group_waves<T, NCB, HALF_K, NCH, 16>(a, s);
   }
-  return launch_group_waves<T, NCB, HALF_K, NCH, 12>(a, s);
+  if constexpr (fp32 && HALF_K && NCB == 2 && NCH == 1) {
+    if (group_lds<T, NCB, HALF_K>(a.K, 12) <= GROUP_LDS_MAX) return launch_group_waves<T, NCB, HALF_K, NCH, 12>(a, s);
+  }
+  return launch_group_waves<T, NCB, HALF_K, NCH, group_fewest_waves<T, HALF_K>()>(a, s);
 }
 
 template <typename T, int NCB, bool HALF_K>
@@ -394,34 +434,49 @@ int launch_group(const ConvArgs& a, hipStream_t s) {
   if (a.c_in <= 16) {
     return a.c_out <= 16 ? launch_group_instance<T, 1, true>(a, s) : launch_group_instance<T, 2, true>(a, s);
   }
-  return a.c_out <= 16 ? launch_group_instance<T, 1, false>(a, s) : launch_group_instance<T, 2, false>(a, s);
+  if (a.c_out <= 16) return launch_group_instance<T, 1, false>(a, s);
+  if constexpr (!std::is_same<T, float>::value) return launch_group_instance<T, 2, false>(a, s);
+  return WCN_ERR_INVALID_ARGUMENT;  // wcn_conv_group_takes says so
+}
+
+template <typename T, int NCB, bool HALF_K>
+bool group_instance_fits(int K) {
+  return group_lds<T, NCB, HALF_K>(K, group_fewest_waves<T, HALF_K>()) <= GROUP_LDS_MAX;
 }
 
 template <typename T>
 bool group_fits(const ConvArgs& a) {
-  const bool half_k = a.c_in <= 16;
-  const size_t lds = a.c_out <= 16 ? (half_k ? group_lds<T, 1, true>(a.K, 12) : group_lds<T, 1, false>(a.K, 12))
-                                   : (half_k ? group_lds<T, 2, true>(a.K, 12) : group_lds<T, 2, false>(a.K, 12));
-  return lds <= GROUP_LDS_MAX;
+  if (a.c_in <= 16) return a.c_out <= 16 ? group_instance_fits<T, 1, true>(a.K) : group_instance_fits<T, 2, true>(a.K);
+  if (a.c_out <= 16) return group_instance_fits<T, 1, false>(a.K);
+  return !std::is_same<T, float>::value && group_instance_fits<T, 2, false>(a.K);
 }
 
 }  // namespace
 
-// 16-bit rows of whole 16-byte pieces (8-byte pieces for rows of at most 16 channels), at most 32
-// channels on either side, all weight tiles and the waves' sums within LDS, a feature matrix that
+// Rows of whole 16-byte pieces (16-bit rows of at most 16 channels: 8-byte pieces; fp32 rows of more than 16: 32-byte
+// pieces, a lane's channels), at most 32 channels on either side, all weight tiles and the waves' sums within LDS, a feature matrix that
 // 32-bit byte offsets reach, a map that comes with its group starts (pairs ascending in output row
 // inside every offset).
+//
+// fp32 (us a call over 3x3x3 maps of rooms and of a cloud, this kernel / the pair-packed one; 60 k, 250 k, 1 M rows):
+//   16 -> 16   24, 21 / 34, 32     30, 28 / 49, 43     110, 103 / 163, 145
+//   32 -> 16   31, 28 / 41, 39     54, 50 / 62, 55     142, 139 / 216, 195
+//   32 -> 32   35, 31 / 42, 39     86, 76 / 67, 61     254, 250 / 221, 201
+//   5x5x5 16 -> 16 over 100 k and 1 M: 51, 48 / 108, 114 and 320, 407 / 539, 573
+// What bounds it: a wave's groups one after the other, 25-30 us each whatever the number of waves beside it (two waves a group,
+// sixteen output channels each: the same).  32 -> 32 leaves LDS for six waves, which is faster in the first round only: not taken.
 bool wcn_conv_group_takes(const ConvArgs& a, int dtype) {
-  if (dtype != WCN_DTYPE_F16 && dtype != WCN_DTYPE_BF16) return false;
+  const bool fp32 = dtype == WCN_DTYPE_F32;
   if (!a.vec_in || a.split || !a.group_start || a.G <= 0 || a.num_pairs <= 0) return false;
-  if (a.c_in > 32 || a.c_out > 32 || (a.c_in <= 16 && a.c_in % 4 != 0)) return false;
-  if ((uint64_t)a.num_in * (uint64_t)a.c_in * 2u >= (1ull << 32)) return false;
+  if (a.c_in > 32 || a.c_out > 32 || a.c_in % (a.c_in <= 16 ? 4 : 8) != 0) return false;
+  if ((uint64_t)a.num_in * (uint64_t)a.c_in * (fp32 ? 4u : 2u) >= (1ull << 32)) return false;
   if (a.K > 128 || (int64_t)a.K * (a.G + 1) >= (1ll << 31) || a.num_pairs >= (1ll << 30) ||
       a.num_in > (1ll << 24))
     return false;
-  return dtype == WCN_DTYPE_F16 ? group_fits<_Float16>(a) : group_fits<__bf16>(a);
+  return fp32 ? group_fits<float>(a) : dtype == WCN_DTYPE_F16 ? group_fits<_Float16>(a) : group_fits<__bf16>(a);
 }
 
 int wcn_conv_group_launch(const ConvArgs& a, int dtype, hipStream_t s) {
+  if (dtype == WCN_DTYPE_F32) return launch_group<float>(a, s);
   return dtype == WCN_DTYPE_F16 ? launch_group<_Float16>(a, s) : launch_group<__bf16>(a, s);
 }
