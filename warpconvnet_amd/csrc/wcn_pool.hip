@@ -197,13 +197,11 @@ __global__ void __launch_bounds__(256) pool_bwd_spread(const T* __restrict__ dY,
 // ---- rows form of a builder's map ---------------------------------------------------------------
 //
 // Pairs that ascend in output row inside every offset, once per (offset, row), with their 64-row
-// group starts: a workgroup makes the rows of a group by itself.  The group's first entry is the sum of
-// its starts over the offsets (lane = offset), a row's bits are set in LDS, and a pair's place follows
-// from the bits below its own.  The offsets are dealt to the four waves, an offset's pairs (at most 64) to the
-// lanes of its wave, eight offsets in flight; up to 32 offsets their numbers stay in registers between the two passes.
-// One pass over the lists instead of two with atomics, two clears, two counts and a scan: 500 k rows of a 3x3x3 map 88
-// -> 15 us.  (A wave per group and the pairs dealt to its lanes without gaps, by binary search over the
-// running counts, took 17 us for any map up to 300 k rows: a chain of shuffles and loads.)
+// group starts: a wave makes the rows of a group by itself.  The group's first entry is the sum of
+// its starts over the offsets (lane = offset).  The runs of its offsets are laid end to end and dealt to the lanes without gaps: every
+// offset marks where its run begins, and the running maximum of the marks is a pair's offset.  A row's bits are set in LDS, a
+// pair's place follows from the bits below its own; the numbers of the first 384 pairs (of some 270 on surfaces) stay in registers between the two.
+// Groups that follow one another go to one XCD: their runs follow one another in the lists.
 constexpr int GROUPED_WORDS = 4;  // up to 128 offsets
 
 template <bool ONE>  // at most 32 offsets
@@ -216,87 +214,111 @@ __global__ void __launch_bounds__(256) rows_from_groups(const int32_t* __restric
                                                         int32_t* __restrict__ row_ptr,
                                                         int32_t* __restrict__ row_in,
                                                         int32_t* __restrict__ clear, int clear_words) {
-  constexpr int W = 4, U = 8, WORDS = ONE ? 1 : GROUPED_WORDS;
-  __shared__ uint32_t s_mask[64][WORDS + (ONE ? 0 : 1)];
-  __shared__ int32_t s_first[64];
-  const int tid = threadIdx.x, lane = wcn_lane();
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  constexpr int WORDS = ONE ? 1 : GROUPED_WORDS, OFFSETS = 32 * WORDS, CHUNK = 384, ROUNDS = CHUNK / 64;
+  __shared__ uint32_t s_mask[4][64][WORDS + (ONE ? 0 : 1)];
+  __shared__ int32_t s_first[4][64];
+  __shared__ int32_t s_shift[4][OFFSETS];  // the place of an offset's first pair in the lists, less its place among the group's
+  __shared__ int32_t s_begin[4][OFFSETS];  // the latter
+  __shared__ uint8_t s_mark[4][CHUNK];     // of CHUNK of the group's pairs: offset + 1 where a run begins
+  const int tid = threadIdx.x, lane = wcn_lane(), wave = tid >> 6;
   if (blockIdx.x == 0)  // counters of whatever follows on the stream
     for (int i = tid; i < clear_words; i += 256) clear[i] = 0;
-  const int64_t group = blockIdx.x, row0 = group * 64;
-  if (tid < 64)
+  const int64_t group = (int64_t)wcn_xcd_tile((int)blockIdx.x, (int)gridDim.x) * 4 + wave, row0 = group * 64;
+  if (group >= G) return;
+  auto written = [] {  // what this wave has put into LDS is there for all its lanes
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  };
 #pragma unroll
-    for (int w = 0; w < WORDS; ++w) s_mask[tid][w] = 0u;
-  // lane k looks after offset k (and 64 + k)
-  int n[2] = {0, 0}, first[2] = {0, 0}, before = 0;
+  for (int w = 0; w < WORDS; ++w) s_mask[wave][lane][w] = 0u;
+  int before = 0, total = 0;
 #pragma unroll
-  for (int h = 0; h < (ONE ? 1 : 2); ++h) {
+  for (int h = 0; h < (ONE ? 1 : 2); ++h) {  // lane k looks after offset k (and 64 + k)
     const int k = lane + 64 * h;
+    int n = 0, first = 0;
     if (k < K) {
       const int32_t* g = gs + (int64_t)k * (G + 1) + group;
       const int b = g[0], cnt = g[1] - b;
       const int64_t start = offsets[k] + b;
       before += b;
-      n[h] = cnt < 0 || cnt > 64 || start < 0 || start + cnt > pairs ? 0 : cnt;  // inconsistent table: contribute nothing
-      first[h] = (int)start;
+      n = cnt < 0 || cnt > 64 || start < 0 || start + cnt > pairs ? 0 : cnt;  // inconsistent table: contribute nothing
+      first = (int)start;
     }
+    const int incl = wcn_wave_inclusive_sum(n);
+    if (k < OFFSETS) {
+      s_begin[wave][k] = n > 0 ? total + incl - n : -1;
+      s_shift[wave][k] = first - (total + incl - n);
+    }
+    total += __shfl(incl, 63, 64);
   }
-  // the numbers of offsets wave + W * (j0 .. j0 + U - 1); lanes past an offset's last pair read that one again
-  int at[U], cnt[U], in[U];
-  int64_t row[U];
-  auto request = [&](int j0, bool want_in) {
+  const int base = __shfl(wcn_wave_inclusive_sum(before), 63, 64);
+  int carry = 0;  // the offset (+ 1) of the last pair before the chunk
+  int k[ROUNDS], in[ROUNDS];
+  int64_t row[ROUNDS];
+  auto request = [&](int p0) {  // pairs p0 .. p0 + CHUNK - 1 of the group
+    uint32_t* const marks = reinterpret_cast<uint32_t*>(s_mark[wave]);
+    for (int i = lane; i < CHUNK / 4; i += 64) marks[i] = 0u;
+    written();
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int k = wave + W * (j0 + u);
-      cnt[u] = k >= K ? 0 : k < 64 ? __builtin_amdgcn_readlane(n[0], k & 63) : __builtin_amdgcn_readlane(n[1], k & 63);
-      const int start = k < 64 ? __builtin_amdgcn_readlane(first[0], k & 63) : __builtin_amdgcn_readlane(first[1], k & 63);
-      at[u] = cnt[u] > 0 ? start + (lane < cnt[u] ? lane : cnt[u] - 1) : 0;
+    for (int h = 0; h < (ONE ? 1 : 2); ++h) {
+      const int o = lane + 64 * h;
+      const int at = o < K ? s_begin[wave][o] - p0 : -1;
+      if (at >= 0 && at < CHUNK && s_begin[wave][o] >= 0) s_mark[wave][at] = (uint8_t)(o + 1);
     }
-    if (pairs > 0) {
+    written();
 #pragma unroll
-      for (int u = 0; u < U; ++u) row[u] = grouping[at[u]];
-      if (want_in)
-#pragma unroll
-        for (int u = 0; u < U; ++u) in[u] = gathered[at[u]];
+    for (int u = 0; u < ROUNDS; ++u) {
+      int v = max((int)s_mark[wave][u * 64 + lane], lane == 0 ? carry : 0);
+      // running maximum over the lanes, as wcn_wave_inclusive_sum
+      v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false));
+      v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false));
+      v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false));
+      v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false));
+      v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false));
+      v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false));
+      carry = __builtin_amdgcn_readlane(v, 63);
+      const int p = p0 + u * 64 + lane;
+      k[u] = p < total ? v - 1 : -1;
+      const int at = p < total ? p + s_shift[wave][v - 1] : 0;
+      row[u] = pairs > 0 ? grouping[at] : 0;
+      in[u] = pairs > 0 ? gathered[at] : 0;
     }
 #pragma unroll
-    for (int u = 0; u < U; ++u) row[u] = lane < cnt[u] ? row[u] - row0 : -1;
+    for (int u = 0; u < ROUNDS; ++u) row[u] = k[u] >= 0 ? row[u] - row0 : -1;
   };
-  __syncthreads();
-  for (int j0 = 0; wave + W * j0 < K; j0 += U) {
-    request(j0, ONE);
+  for (int p0 = 0; p0 < total; p0 += CHUNK) {
+    request(p0);
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int k = wave + W * (j0 + u);
-      if ((uint64_t)row[u] < 64u) atomicOr(&s_mask[row[u]][k >> 5], 1u << (k & 31));
-    }
+    for (int u = 0; u < ROUNDS; ++u)
+      if ((uint64_t)row[u] < 64u) atomicOr(&s_mask[wave][row[u]][ONE ? 0 : k[u] >> 5], 1u << (k[u] & 31));
   }
-  __syncthreads();
-  if (wave == 0) {
-    const int base = __shfl(wcn_wave_inclusive_sum(before), 63, 64);
-    int mine = 0;
+  written();
+  int mine = 0;
 #pragma unroll
-    for (int w = 0; w < WORDS; ++w) mine += __popc(s_mask[lane][w]);
-    const int incl = wcn_wave_inclusive_sum(mine);
-    s_first[lane] = base + incl - mine;
-    if (row0 + lane < num_rows) {
-      row_ptr[row0 + lane] = base + incl - mine;
+  for (int w = 0; w < WORDS; ++w) mine += __popc(s_mask[wave][lane][w]);
+  const int incl = wcn_wave_inclusive_sum(mine);
+  s_first[wave][lane] = base + incl - mine;
+  if (row0 + lane < num_rows) {
+    row_ptr[row0 + lane] = base + incl - mine;
 #pragma unroll
-      for (int w = 0; w < WORDS; ++w)
-        if (w < words) row_mask[(row0 + lane) * words + w] = s_mask[lane][w];
-      if (row0 + lane == num_rows - 1) row_ptr[num_rows] = base + incl;
-    }
+    for (int w = 0; w < WORDS; ++w)
+      if (w < words) row_mask[(row0 + lane) * words + w] = s_mask[wave][lane][w];
+    if (row0 + lane == num_rows - 1) row_ptr[num_rows] = base + incl;
   }
-  __syncthreads();
-  for (int j0 = 0; wave + W * j0 < K; j0 += U) {
-    if (!ONE) request(j0, true);
+  written();
+  const bool again = total > CHUNK;
+  carry = 0;
+  for (int p0 = 0; p0 < total; p0 += CHUNK) {
+    if (again) request(p0);
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int k = wave + W * (j0 + u);
+    for (int u = 0; u < ROUNDS; ++u) {
       if ((uint64_t)row[u] >= 64u) continue;
-      int rank = __popc(s_mask[row[u]][k >> 5] & ((1u << (k & 31)) - 1u));
-      for (int w = 0; w < (k >> 5); ++w) rank += __popc(s_mask[row[u]][w]);
-      const int64_t dst = (int64_t)s_first[row[u]] + rank;
+      const uint32_t* const mask = s_mask[wave][row[u]];
+      int rank = __popc(mask[ONE ? 0 : k[u] >> 5] & ((1u << (k[u] & 31)) - 1u));
+      if (!ONE)
+        for (int w = 0; w < (k[u] >> 5); ++w) rank += __popc(mask[w]);
+      const int64_t dst = (int64_t)s_first[wave][row[u]] + rank;
       if (dst < pairs) row_in[dst] = in[u];
     }
   }
@@ -610,7 +632,7 @@ int wcn_rows_from_groups(const int32_t* gathered_rows, const int32_t* grouping_r
   if (num_rows == 0) return WCN_OK;
   WcnRowsView v;
   wcn_rows_layout(workspace, num_rows, num_offsets, num_pairs, &v);
-  hipLaunchKernelGGL((num_offsets <= 32 ? rows_from_groups<true> : rows_from_groups<false>), dim3((unsigned)v.G), dim3(256), 0, s, gathered_rows,
+  hipLaunchKernelGGL((num_offsets <= 32 ? rows_from_groups<true> : rows_from_groups<false>), dim3((unsigned)((v.G + 3) / 4)), dim3(256), 0, s, gathered_rows,
                      grouping_rows, device_offsets, group_start, num_offsets, v.words, num_rows, v.G, num_pairs, v.row_mask,
                      v.row_ptr, v.row_in, clear, clear_words);
   WCN_LAUNCH_CHECK();
