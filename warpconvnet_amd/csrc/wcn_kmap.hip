@@ -1146,37 +1146,35 @@ __global__ void __launch_bounds__(256) stride_pick(const int4* __restrict__ coar
 // of 4), so its voxels are bits of one slot's mask, their rows stand next to each other in perm, and
 // the cell's representative is the lowest of them.  No table over the coarse rows is needed: one
 // slot look-up and at most sx * sy * sz loads of perm per row.  LOG: log2 of the strides.
-template <bool FILL>
-__global__ void __launch_bounds__(256) stride_pick_cells(const int4* __restrict__ coords, int64_t n,
-                                                         const WcnTableHeader* __restrict__ hdr,
-                                                         const WcnSlot* __restrict__ slots,
-                                                         uint32_t cap_mask,
-                                                         const int32_t* __restrict__ perm,
-                                                         int lx, int ly, int lz,
-                                                         int32_t* __restrict__ groups, int64_t G,
-                                                         unsigned long long* __restrict__ picked,
-                                                         int4* __restrict__ out_coords,
-                                                         int32_t* __restrict__ first_index) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+//
+// Two launches.  The counting one leaves a group's representatives as a mask, their number per 256 rows, and where the fine
+// rows of every batch item begin (a row whose batch id differs from the row's before it).  In the filling one a
+// workgroup adds up the counts before its own (up to CELLS_PARTS of them: 16 KB out of the L2; beyond, a scan in between
+// does), and the first one finds from the masks how many coarse rows lie before an item's first fine row, which together with
+// the number of rows and the table's status is what the host waits for.  (Counts scanned, totals, rows and a search of the
+// rows for every batch id, each in a launch of its own: 34 us of kernels and 4 gaps over 456 k rows.)
+constexpr int CELLS_PARTS = 4096;  // of 256 rows
+
+__global__ void __launch_bounds__(256) stride_count_cells(const int4* __restrict__ coords, int64_t n,
+                                                          const WcnTableHeader* __restrict__ hdr,
+                                                          const WcnSlot* __restrict__ slots,
+                                                          uint32_t cap_mask,
+                                                          const int32_t* __restrict__ perm,
+                                                          int lx, int ly, int lz,
+                                                          int32_t* __restrict__ counts,
+                                                          unsigned long long* __restrict__ picked,
+                                                          int32_t* __restrict__ item_row) {
+  __shared__ int32_t s_count[4];
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
   const int64_t group = i >> 6;
-  if (group >= G) return;
-  const int lane = wcn_lane();
-  if (FILL) {
-    // the counting pass left the group's representatives as a mask: no second look-up
-    const unsigned long long wins = picked[group];
-    if ((wins >> lane) & 1ull) {
-      const int4 c = coords[i];
-      const int64_t pos = (int64_t)groups[group] + __popcll(wins & ((1ull << lane) - 1ull));
-      out_coords[pos] = make_int4(c.x, floor_div(c.y, 1 << lx), floor_div(c.z, 1 << ly), floor_div(c.w, 1 << lz));
-      first_index[pos] = (int32_t)i;
-    }
-    return;
-  }
+  const int lane = wcn_lane(), wave = threadIdx.x >> 6;
   bool winner = false;
-  int4 c = make_int4(0, 0, 0, 0);
   if (i < n) {
     const WcnLayout L = wcn_make_layout(hdr);
-    c = coords[i];
+    const int4 c = coords[i];
+    const int before = i > 0 ? coords[i - 1].x : -1;
+    // (the host reads what comes of these only for rows whose batch column does not descend)
+    for (int b = before < 0 ? 0 : before + 1; b <= c.x && b < STRIDE_BATCH_MARKS; ++b) item_row[b] = (int32_t)i;
     uint32_t r[4];
     if (L.ok && wcn_relative(L, c.x, c.y, c.z, c.w, r)) {
       int32_t base = 0;
@@ -1200,8 +1198,111 @@ __global__ void __launch_bounds__(256) stride_pick_cells(const int4* __restrict_
   }
   const unsigned long long wins = __ballot(winner);
   if (lane == 0) {
-    groups[group] = __popcll(wins);
-    picked[group] = wins;
+    if (i < n) picked[group] = wins;
+    s_count[wave] = __popcll(wins);
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) counts[blockIdx.x] = s_count[0] + s_count[1] + s_count[2] + s_count[3];
+}
+
+struct StrideResult {
+  int64_t* result;   // as StrideWorkspace::result
+  int64_t* mailbox;  // pinned host memory (or null): the same words behind a sequence word
+  int64_t sequence;
+};
+
+template <bool SCANNED>  // counts: exclusive prefix sums, their total behind the last
+__global__ void __launch_bounds__(256) stride_fill_cells(const int4* __restrict__ coords, int64_t n,
+                                                         const WcnTableHeader* __restrict__ hdr,
+                                                         int lx, int ly, int lz,
+                                                         const int32_t* __restrict__ counts,
+                                                         const unsigned long long* __restrict__ picked,
+                                                         const int32_t* __restrict__ item_row,
+                                                         int4* __restrict__ out_coords,
+                                                         int32_t* __restrict__ first_index, StrideResult res) {
+  constexpr int PER = CELLS_PARTS / 256;
+  __shared__ int32_t s_wave[4];
+  __shared__ int32_t s_before[SCANNED ? 1 : CELLS_PARTS + 1];  // (first workgroup) coarse rows before a part
+  const int tid = threadIdx.x, lane = wcn_lane(), wave = tid >> 6;
+  const int part = (int)blockIdx.x, parts = (int)gridDim.x;
+  const int64_t i = (int64_t)part * 256 + tid, group = i >> 6;
+  const int4 c = coords[i < n ? i : n - 1];
+  unsigned long long wins[4];
+#pragma unroll
+  for (int w = 0; w < 4; ++w) wins[w] = ((int64_t)part * 4 + w) * 64 < n ? picked[(int64_t)part * 4 + w] : 0ull;
+  int before = SCANNED ? counts[part] : 0;
+  if (!SCANNED) {  // the sum of the counts before this part's
+    int sum = 0;
+#pragma unroll
+    for (int t = 0; t < PER; ++t) {
+      const int p = t * 256 + tid;
+      sum += p < part ? counts[p] : 0;
+    }
+    sum = wcn_wave_inclusive_sum(sum);
+    if (lane == 63) s_wave[wave] = sum;
+    __syncthreads();
+    before = s_wave[0] + s_wave[1] + s_wave[2] + s_wave[3];
+  }
+#pragma unroll
+  for (int w = 0; w < 4; ++w)
+    if (w < wave) before += __popcll(wins[w]);
+  const unsigned long long mine = wave == 0 ? wins[0] : wave == 1 ? wins[1] : wave == 2 ? wins[2] : wins[3];
+  if (i < n && ((mine >> lane) & 1ull)) {
+    const int64_t pos = (int64_t)before + __popcll(mine & ((1ull << lane) - 1ull));
+    out_coords[pos] = make_int4(c.x, floor_div(c.y, 1 << lx), floor_div(c.z, 1 << ly), floor_div(c.w, 1 << lz));
+    first_index[pos] = (int32_t)i;
+  }
+  if (part != 0) return;
+  if (!SCANNED) {
+    __syncthreads();  // s_wave has been read
+    int v[PER], sum = 0;
+#pragma unroll
+    for (int t = 0; t < PER; ++t) {
+      const int p = tid * PER + t;
+      v[t] = p < parts ? counts[p] : 0;
+      sum += v[t];
+    }
+    const int incl = wcn_wave_inclusive_sum(sum);
+    if (lane == 63) s_wave[wave] = incl;
+    __syncthreads();
+    int run = incl - sum;
+    for (int w = 0; w < wave; ++w) run += s_wave[w];
+#pragma unroll
+    for (int t = 0; t < PER; ++t) {
+      if (tid * PER + t <= parts) s_before[tid * PER + t] = run;
+      run += v[t];
+    }
+    if (tid == 255 && parts == CELLS_PARTS) s_before[CELLS_PARTS] = run;
+    __syncthreads();
+  }
+  const int64_t total = SCANNED ? counts[parts] : s_before[SCANNED ? 0 : parts];
+  const int last_item = coords[n - 1].x;
+  auto put = [&](int at, int64_t v) {
+    res.result[at] = v;
+    if (res.mailbox) res.mailbox[1 + at] = v;
+  };
+  for (int b = tid; b < STRIDE_BATCH_MARKS; b += 256) {
+    int64_t rows = total;
+    if (b <= last_item) {
+      int64_t r = item_row[b];
+      r = r < 0 ? 0 : r > n ? n : r;
+      if (r < n) {
+        const int p = (int)(r >> 8);
+        rows = SCANNED ? counts[p] : s_before[SCANNED ? 0 : p];
+        for (int64_t g = (int64_t)p * 4; g < r >> 6; ++g) rows += __popcll(picked[g]);
+        rows += __popcll(picked[r >> 6] & ((1ull << (r & 63)) - 1ull));
+      }
+    }
+    put(4 + b, rows);
+  }
+  if (tid == 0) {
+    put(0, total);
+    put(1, hdr->status);
+  }
+  if (res.mailbox) {  // everything is in the mailbox before the word that the host polls
+    __threadfence_system();
+    __syncthreads();
+    if (tid == 0) __hip_atomic_store(&res.mailbox[0], res.sequence, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
   }
 }
 
@@ -1210,6 +1311,11 @@ __global__ void stride_finish(int64_t* __restrict__ result, const int32_t* __res
   if (threadIdx.x != 0 || blockIdx.x != 0) return;
   result[0] = groups[G];
   result[1] = hdr->status;
+}
+
+// (no rows at all)
+__global__ void __launch_bounds__(1024) stride_no_rows(int64_t* __restrict__ result, const WcnTableHeader* __restrict__ hdr) {
+  for (int b = threadIdx.x; b < 4 + STRIDE_BATCH_MARKS; b += 1024) result[b] = b == 1 ? hdr->status : 0;
 }
 
 // Where the coarse rows of each batch item begin, for rows whose batch column does not descend
@@ -1484,8 +1590,9 @@ int wcn_stride_unique(const int32_t* coords, int64_t n, const int32_t host_strid
 size_t wcn_stride_unique_cells_workspace_bytes(int64_t n) {
   if (n < 0) return 0;
   return wcn_align256(sizeof(int64_t) * (size_t)(4 + STRIDE_BATCH_MARKS)) +
-         wcn_align256(sizeof(int32_t) * (size_t)((n + 63) / 64 + 1)) +
-         wcn_align256(sizeof(unsigned long long) * (size_t)((n + 63) / 64));
+         wcn_align256(sizeof(int32_t) * (size_t)((n + 255) / 256 + 1)) +
+         wcn_align256(sizeof(unsigned long long) * (size_t)((n + 63) / 64)) +
+         wcn_align256(sizeof(int32_t) * (size_t)STRIDE_BATCH_MARKS);
 }
 
 int wcn_stride_unique_cells(const void* table, int64_t n_keys, int64_t capacity, const int32_t* coords,
@@ -1505,28 +1612,49 @@ int wcn_stride_unique_cells(const void* table, int64_t n_keys, int64_t capacity,
   wcn_table_layout(const_cast<void*>(table), n_keys, capacity, &v);
   // the result block first, as in the workspace of wcn_stride_unique (the read calls find it there)
   int64_t* result = (int64_t*)workspace;
-  int32_t* groups = (int32_t*)((char*)workspace + wcn_align256(sizeof(int64_t) * (size_t)(4 + STRIDE_BATCH_MARKS)));
-  const int64_t G = (n + 63) / 64;
-  unsigned long long* picked = (unsigned long long*)((char*)groups + wcn_align256(sizeof(int32_t) * (size_t)(G + 1)));
+  int32_t* counts = (int32_t*)((char*)workspace + wcn_align256(sizeof(int64_t) * (size_t)(4 + STRIDE_BATCH_MARKS)));
+  const int64_t parts = (n + 255) / 256;
+  unsigned long long* picked = (unsigned long long*)((char*)counts + wcn_align256(sizeof(int32_t) * (size_t)(parts + 1)));
+  int32_t* item_row = (int32_t*)((char*)picked + wcn_align256(sizeof(unsigned long long) * (size_t)((n + 63) / 64)));
   const uint32_t cap_mask = (uint32_t)(capacity - 1);
-  if (n > 0) {
-    hipLaunchKernelGGL(stride_pick_cells<false>, dim3(grid_for(n, 256)), dim3(256), 0, s, (const int4*)coords,
-                       n, v.hdr, v.slots, cap_mask, v.perm, lg[0], lg[1], lg[2], groups, G, picked,
-                       (int4*)nullptr, (int32_t*)nullptr);
+  g_pending_sequence = 0;
+  g_pending_result = nullptr;
+  if (n == 0) {
+    hipLaunchKernelGGL(stride_no_rows, dim3(1), dim3(1024), 0, s, result, v.hdr);
+    WCN_LAUNCH_CHECK();
+    return WCN_OK;
   }
-  {
+  hipLaunchKernelGGL(stride_count_cells, dim3((unsigned)parts), dim3(256), 0, s, (const int4*)coords, n, v.hdr, v.slots, cap_mask,
+                     v.perm, lg[0], lg[1], lg[2], counts, picked, item_row);
+  // as the kernel map's result: into this thread's mailbox, where the read calls pick it up
+  StrideResult res = {result, nullptr, 0};
+  if (wcn_mailbox_begin(&res.mailbox, &res.sequence) != WCN_OK) res = {result, nullptr, 0};
+  if (parts <= CELLS_PARTS) {
+    hipLaunchKernelGGL(stride_fill_cells<false>, dim3((unsigned)parts), dim3(256), 0, s, (const int4*)coords, n, v.hdr, lg[0],
+                       lg[1], lg[2], counts, picked, item_row, (int4*)out_coords, first_index, res);
+  } else {
     const KmapFinish none = {nullptr, nullptr, nullptr, 0, nullptr, 0};
-    hipLaunchKernelGGL(kmap_scan_rows, dim3(1), dim3(1024), 0, s, groups, G, result + 2, none);
-  }
-  hipLaunchKernelGGL(stride_finish, dim3(1), dim3(64), 0, s, result, groups, G, v.hdr);
-  if (n > 0) {
-    hipLaunchKernelGGL(stride_pick_cells<true>, dim3(grid_for(n, 256)), dim3(256), 0, s, (const int4*)coords,
-                       n, v.hdr, v.slots, cap_mask, v.perm, lg[0], lg[1], lg[2], groups, G, picked,
-                       (int4*)out_coords, first_index);
-    hipLaunchKernelGGL(stride_batch_bounds, dim3(1), dim3(1024), 0, s, (const int4*)out_coords, result);
+    hipLaunchKernelGGL(kmap_scan_rows, dim3(1), dim3(1024), 0, s, counts, parts, result + 2, none);
+    hipLaunchKernelGGL(stride_fill_cells<true>, dim3((unsigned)parts), dim3(256), 0, s, (const int4*)coords, n, v.hdr, lg[0],
+                       lg[1], lg[2], counts, picked, item_row, (int4*)out_coords, first_index, res);
   }
   WCN_LAUNCH_CHECK();
+  if (res.mailbox) {
+    if (wcn_mailbox_mark(s) != WCN_OK) return WCN_ERR_LAUNCH;
+    g_pending_sequence = res.sequence;
+    g_pending_result = result;
+  }
   return WCN_OK;
+}
+
+// From the mailbox a wcn_stride_unique_cells call of this thread armed, once its rows are written too, otherwise from the device copy.
+static int stride_read(const int64_t* result, int64_t* host, size_t bytes, hipStream_t stream) {
+  const int64_t sequence = g_pending_result == (const void*)result ? g_pending_sequence : 0;
+  if (sequence != 0) {
+    g_pending_sequence = 0;
+    if (wcn_mailbox_end(host, bytes, sequence, true) == WCN_OK) return WCN_OK;
+  }
+  return wcn_read_small(host, result, bytes, stream);
 }
 
 int wcn_stride_unique_read_bounds(const void* workspace, int64_t n, int64_t capacity,
@@ -1535,7 +1663,7 @@ int wcn_stride_unique_read_bounds(const void* workspace, int64_t n, int64_t capa
   StrideWorkspace w;
   stride_layout(const_cast<void*>(workspace), n, capacity, &w);
   int64_t tmp[4 + STRIDE_BATCH_MARKS];
-  if (wcn_read_small(tmp, w.result, sizeof(tmp), (hipStream_t)stream) != WCN_OK) return WCN_ERR_LAUNCH;
+  if (stride_read(w.result, tmp, sizeof(tmp), (hipStream_t)stream) != WCN_OK) return WCN_ERR_LAUNCH;
   *host_count = tmp[0];
   for (int b = 0; b < STRIDE_BATCH_MARKS; ++b) host_bounds[b] = n > 0 ? tmp[4 + b] : 0;
   return wcn_table_status_from_bits((int32_t)tmp[1]);
@@ -1547,7 +1675,7 @@ int wcn_stride_unique_read_count(const void* workspace, int64_t n, int64_t capac
   StrideWorkspace w;
   stride_layout(const_cast<void*>(workspace), n, capacity, &w);
   int64_t tmp[2];
-  if (wcn_read_small(tmp, w.result, sizeof(tmp), (hipStream_t)stream) != WCN_OK) return WCN_ERR_LAUNCH;
+  if (stride_read(w.result, tmp, sizeof(tmp), (hipStream_t)stream) != WCN_OK) return WCN_ERR_LAUNCH;
   *host_count = tmp[0];
   return wcn_table_status_from_bits((int32_t)tmp[1]);
 }

@@ -890,12 +890,12 @@ int wcn_mailbox_mark(hipStream_t stream) {
   return hipEventRecord(g_box_done, stream) == hipSuccess ? WCN_OK : WCN_ERR_LAUNCH;
 }
 
-int wcn_mailbox_end(void* host_dst, size_t payload_bytes, int64_t sequence) {
+int wcn_mailbox_end(void* host_dst, size_t payload_bytes, int64_t sequence, bool kernel_over) {
   if (!g_box || !g_box_done || payload_bytes + 8 > kMailboxBytes) return WCN_ERR_INVALID_ARGUMENT;
   volatile int64_t* word0 = g_box;
   BoundedPoll poll;
   for (;;) {
-    if (*word0 == sequence) break;
+    if (!kernel_over && *word0 == sequence) break;
     const hipError_t e = hipEventQuery(g_box_done);
     if (e == hipErrorNotReady) {
       if (!poll.again()) return WCN_ERR_LAUNCH;
