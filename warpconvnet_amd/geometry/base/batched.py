@@ -50,7 +50,7 @@ class BatchedTensor:
             f"Offsets must be a cpu IntTensor or cpu LongTensor, got {self.offsets}"
         assert not self.offsets.requires_grad, "Offsets must not require grad"
         assert isinstance(self.batched_tensor, Tensor)
-        assert int(self.offsets[-1]) == self.batched_tensor.shape[0], \
+        assert self.offsets.tolist()[-1] == self.batched_tensor.shape[0], \
             f"Offsets {self.offsets.tolist()} do not match {self.batched_tensor.shape[0]} rows"
 
     @property

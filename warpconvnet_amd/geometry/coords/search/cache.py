@@ -36,6 +36,14 @@ class IntSearchCacheKey:
                      str(stride_mode), bool(skip_symmetric_kernel_map), _as_tuple(in_offsets),
                      _as_tuple(out_offsets))
 
+    @classmethod
+    def _over(cls, kernel_size: Tuple[int, ...], kernel_dilation: Tuple[int, ...], stride_mode: str, offsets) -> "IntSearchCacheKey":
+        """The key of a map of a coordinate set onto itself, from tuples as they are."""
+        key = cls.__new__(cls)
+        rows = _as_tuple(offsets)
+        key._all = (kernel_size, kernel_dilation, False, False, stride_mode, False, rows, rows)
+        return key
+
     kernel_size = property(lambda self: self._all[0])
     kernel_dilation = property(lambda self: self._all[1])
     transposed = property(lambda self: self._all[2])

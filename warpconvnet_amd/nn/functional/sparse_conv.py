@@ -315,6 +315,34 @@ def generate_output_coords_and_kernel_map(
 # Public entry point
 # ------------------------------------------------------------------------------------------------
 
+def _over_kept_map(voxels: Voxels, weight: Tensor, kernel_size, kernel_dilation, stride_mode, bias, residual, relu,
+                   compute_dtype, keep_prepared_weight) -> Optional[Voxels]:
+    """A stride-1 layer without gradients over a map that a layer before it has left: what spatially_sparse_conv does
+    then, without the questions that only other layers ask (16 us of the host per layer -> 8; a network's layers over one
+    scan run for 7 to 20 us each).  None where the layer is no such one."""
+    cache = voxels._extra_attributes.get("_cache")
+    coords = voxels.batched_coordinates
+    if cache is None or type(coords) is not IntCoords or coords._batch_indexed is None or torch.is_autocast_enabled():
+        return None
+    features, offsets = voxels.batched_features.batched_tensor, voxels.batched_features.offsets
+    rows = coords._batch_indexed.shape[0]
+    if rows == 0 or features.shape[0] == 0:
+        return None
+    if isinstance(residual, Voxels):
+        residual = residual.feature_tensor
+    if torch.is_grad_enabled() and (features.requires_grad or weight.requires_grad
+                                    or (residual is not None and residual.requires_grad)):
+        return None
+    kernel_map = cache.get(IntSearchCacheKey._over(kernel_size, kernel_dilation, _MODE_TEXT[stride_mode], offsets))
+    if kernel_map is None:
+        return None
+    out = native().conv_forward(features, weight, kernel_map, rows, bias,
+                                compute_dtype if compute_dtype is not None else features.dtype, residual, relu,
+                                keep_prepared_weight, _pairs_sorted)
+    stride = coords.tensor_stride
+    return voxels._with_features(coords, out, stride if stride is not None else (1,) * len(kernel_size))
+
+
 def spatially_sparse_conv(
     input_sparse_tensor: Voxels,
     weight: Tensor,
@@ -358,6 +386,13 @@ def spatially_sparse_conv(
     _kernel_size = ntuple(kernel_size, ndim=ndim)
     _kernel_dilation = ntuple(kernel_dilation, ndim=ndim)
     _stride = ntuple(stride, ndim=ndim)
+
+    if (output_spatially_sparse_tensor is None and not transposed and not generative and _stride == (1,) * ndim
+            and order is POINT_ORDERING.RANDOM and _kernel_size != _stride and type(input_sparse_tensor) is Voxels):
+        out = _over_kept_map(input_sparse_tensor, weight, _kernel_size, _kernel_dilation, stride_mode, bias, residual, relu,
+                             compute_dtype, keep_prepared_weight)
+        if out is not None:
+            return out
 
     if isinstance(residual, Voxels):
         residual = residual.feature_tensor
