@@ -17,9 +17,11 @@
 //     channels)), W[k]^T the A operand, so that a lane ends up with 4 consecutive output channels of
 //     one pair and hands that pair's row of sums to the MFMA as its C operand: one 16-byte LDS read
 //     and write per 16 channels.  Pairs that do not exist read row 0 and add into a spare row;
-//   * requests run a fixed distance ahead of the multiplications (the rows 8 blocks, the pair-list
+//   * requests run a fixed distance ahead of the multiplications (the rows 2 blocks, the pair-list
 //     entries 16), in a ring whose 16 steps are written out: plain loads, and the compiler's own
-//     waits for them come out exact because the start-up issues its requests in the loop's order;
+//     waits for them come out exact because the start-up issues its requests in the loop's order.  (Entries and rows ahead, us over 1 M
+//     rows for 3x3x3 32 -> 32, 16 -> 16 and 5x5x5 16 -> 16: 16 and 8 blocks 96.9, 65.1, 208; 16 and 4 95.7, 63.5, 208; 16 and 2
+//     96.7, 63.3, 179; 8 and 4 96.0, 62.6, 198; 8 and 2 96.7, 65.2, 178: past the latency, what is asked for beyond a list's end is lost.)
 //   * the additions of a row happen in a fixed order: results are bitwise reproducible.
 #include <algorithm>
 #include <mutex>
@@ -33,7 +35,7 @@ using namespace wcn_mma;
 
 namespace {
 
-constexpr int GROUP_AHEAD = 8;     // blocks of 16 pairs whose gathered rows are on their way
+constexpr int GROUP_AHEAD = 2;     // blocks of 16 pairs whose gathered rows are on their way
 constexpr int GROUP_ENTRIES = 16;  // blocks whose pair-list entries are on their way or held
 
 typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
@@ -294,16 +296,16 @@ __global__ void __launch_bounds__(WAVES * 64) conv_fwd_group(ConvArgs a) {
     turn_page(0);
 #pragma unroll
     for (int u = 0; u < GROUP_ENTRIES; ++u) {
-      if (u >= GROUP_AHEAD) request_rows(u - GROUP_AHEAD, u - GROUP_AHEAD);
+      if (u >= GROUP_ENTRIES - GROUP_AHEAD) request_rows(u - (GROUP_ENTRIES - GROUP_AHEAD), u - (GROUP_ENTRIES - GROUP_AHEAD));
       request_entries(u, u);
       __builtin_amdgcn_sched_barrier(0);
     }
-    static_assert(GROUP_ENTRIES == 16 && GROUP_AHEAD == 8, "the turn below is written out for a ring of 16 and 8");
+    static_assert(GROUP_ENTRIES == 16 && GROUP_ENTRIES % GROUP_AHEAD == 0 && GROUP_AHEAD < GROUP_ENTRIES, "the turn below is written out for a ring of 16");
     for (int t0 = 0; t0 < blocks; t0 += GROUP_ENTRIES) {
       const int ask = t0 + GROUP_ENTRIES;  // the first block whose entries this turn requests
       if ((ask & 63) == 0) turn_page(ask >> 6);
       const int todo = blocks - t0, on_page = ask & 63;
-      // one block: multiply it, request the rows of the block 8 further on (whose entries have
+      // one block: multiply it, request the rows of the block 2 further on (whose entries have
       // arrived) and the entries of the block 16 further on (into the slot just multiplied).
       // Written out rather than left to the unroller: the turn ends at the list's last block from
       // any of its 16 places, and the register of every slot has to be fixed at compile time.
@@ -463,7 +465,7 @@ bool group_fits(const ConvArgs& a) {
 //   32 -> 16   31, 28 / 41, 39     54, 50 / 62, 55     142, 139 / 216, 195
 //   32 -> 32   35, 31 / 42, 39     86, 76 / 67, 61     254, 250 / 221, 201
 //   5x5x5 16 -> 16 over 100 k and 1 M: 51, 48 / 108, 114 and 320, 407 / 539, 573
-// What bounds it: a wave's groups one after the other, 25-30 us each whatever the number of waves beside it (two waves a group,
+// (with rows requested 8 blocks ahead).  What bounds it: a wave's groups one after the other, 25-30 us each whatever the number of waves beside it (two waves a group,
 // sixteen output channels each: the same).  32 -> 32 leaves LDS for six waves, which is faster in the first round only: not taken.
 bool wcn_conv_group_takes(const ConvArgs& a, int dtype) {
   const bool fp32 = dtype == WCN_DTYPE_F32;
