@@ -84,6 +84,12 @@ size_t wcn_table_bytes(int64_t n_keys, int64_t capacity);
 int wcn_table_build(const int32_t* keys, int64_t n_keys, void* table, int64_t capacity,
                     void* stream);
 
+/* wcn_batch_indexed_rows of (n_rows, 3) coordinates into `rows` (n_rows, 4; 16-byte aligned) and wcn_table_build over them in
+ * one call, which takes a launch and a pass over the coordinates less.  host_batch_offsets: batch_size + 1 <= 65
+ * offsets that ascend from 0 to n_rows >= 1. */
+int wcn_table_build_items(const int32_t* coords, int64_t n_rows, const int64_t* host_batch_offsets, int32_t batch_size,
+                          int32_t* rows, void* table, int64_t capacity, void* stream);
+
 /* results[i] = row index of queries[i] (num_queries, 4) among the keys, or -1. */
 int wcn_table_query(const void* table, int64_t n_keys, int64_t capacity, const int32_t* queries,
                     int64_t num_queries, int32_t* results, void* stream);

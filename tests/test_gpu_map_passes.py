@@ -34,3 +34,48 @@ def test_solid_cubes_and_ragged_ends(oracle, ksize, stride, rows):
     assert np.array_equal(got.offsets.numpy().astype(np.int64), want[2])
     assert np.array_equal(got.in_maps.cpu().numpy(), want[0])
     assert np.array_equal(got.out_maps.cpu().numpy(), want[1])
+
+
+@pytest.mark.parametrize("sizes", [(1,), (64, 0, 1), (255, 257), (16384,), (16385,), (4096, 0, 0, 4097, 9000), tuple([7] * 64)],
+                         ids=lambda v: f"{len(v)}_{sum(v)}")
+def test_rows_and_table_by_the_same_launches(sizes):
+    """The batch column, and the table over the rows, for few keys and many, empty items and the most items that
+    travel with a launch; a second tensor of the same rows takes the launches of their own."""
+    from warpconvnet_amd.geometry.coords.integer import IntCoords
+    from warpconvnet_amd.geometry.coords.search.torch_discrete import rows_with_table
+    n = sum(sizes)
+    rng = np.random.default_rng(n)
+    xyz = np.unique(rng.integers(-60, 60, size=(3 * n + 100, 3)), axis=0)
+    xyz = torch.as_tensor(rng.permutation(xyz)[:n].astype(np.int32), device=DEV)
+    offsets = torch.as_tensor(np.concatenate([[0], np.cumsum(sizes)]))
+    coords, plain = IntCoords(xyz, offsets), IntCoords(xyz, offsets)
+    rows = rows_with_table(coords)
+    assert torch.equal(rows, plain.batch_indexed_coordinates) and rows_with_table(coords) is rows
+    table = rows._wcn_table[1]
+    want = torch.arange(n, dtype=torch.int32, device=DEV)
+    assert torch.equal(table.search(rows), want) and torch.equal(plain.hashmap.search(rows), want)
+    absent = rows + torch.tensor([0, 500, 0, 0], dtype=torch.int32, device=DEV)
+    assert (table.search(absent) == -1).all()
+
+
+@pytest.mark.parametrize("stride", [(2, 2, 2), (4, 1, 2)], ids=lambda v: "x".join(map(str, v)))
+@pytest.mark.parametrize("sizes", [(1,), (256,), (300, 0, 0, 513), (64, 192, 1, 0), (9000, 3), (1_100_000, 5)],
+                         ids=lambda v: f"{len(v)}_{sum(v)}")
+def test_strided_rows_and_their_batch_offsets(sizes, stride):
+    """Items that end inside a group, a workgroup's rows and beyond the parts that are added up without a scan."""
+    from warpconvnet_amd.geometry.coords.ops.stride import stride_coords
+    n = sum(sizes)
+    rng = np.random.default_rng(n)
+    edge = max(3, int(round((2.5 * n) ** (1 / 3))))
+    cells = rng.permutation(edge ** 3)[:n] if max(sizes) <= edge ** 3 else None
+    assert cells is not None
+    xyz = np.stack([cells // edge ** 2, cells // edge % edge, cells % edge], axis=1).astype(np.int32) - 7
+    item = np.repeat(np.arange(len(sizes)), sizes).astype(np.int32)
+    rows = np.concatenate([item[:, None], xyz], axis=1)
+    coarse = np.concatenate([item[:, None], xyz // np.asarray(stride)], axis=1)
+    _, first = np.unique(coarse, axis=0, return_index=True)
+    want = coarse[np.sort(first)]
+    got, offsets = stride_coords(torch.as_tensor(rows, device=DEV), stride, batch_sorted=True)
+    assert np.array_equal(got.cpu().numpy(), want)
+    counts = np.bincount(want[:, 0], minlength=len(sizes))[: int(want[-1, 0]) + 1]
+    assert offsets.tolist() == np.concatenate([[0], np.cumsum(counts)]).tolist()

@@ -23,6 +23,7 @@ SIGNATURES = {
     "wcn_table_default_capacity": (_i64, [_i64]),
     "wcn_table_bytes": (_sz, [_i64, _i64]),
     "wcn_table_build": (ctypes.c_int, [_vp, _i64, _vp, _i64, _vp]),
+    "wcn_table_build_items": (ctypes.c_int, [_vp, _i64, _i64p, _i32, _vp, _vp, _i64, _vp]),
     "wcn_table_query": (ctypes.c_int, [_vp, _i64, _i64, _vp, _i64, _vp, _vp]),
     "wcn_table_read_status": (ctypes.c_int, [_vp, _i32p, _vp]),
     "wcn_kmap_workspace_bytes": (_sz, [_i64, _i32]),

@@ -254,6 +254,33 @@ __device__ __forceinline__ int wcn_wave_inclusive_sum(int v) {
 
 #endif  // __HIPCC__
 
+// Where the rows of every batch item begin; handed over in a launch's arguments.
+struct WcnItemStarts {
+  int64_t start[WCN_VOXEL_MAX_BATCH + 1];
+};
+// From batch_size + 1 host offsets: false if there are none, too many, or they do not ascend from 0 to num_rows.
+static inline bool wcn_item_starts(const int64_t* host_offsets, int32_t batch_size, int64_t num_rows, WcnItemStarts* out) {
+  if (!host_offsets || batch_size < 1 || batch_size > WCN_VOXEL_MAX_BATCH || host_offsets[0] != 0) return false;
+  for (int b = 0; b <= batch_size; ++b) {
+    if (b > 0 && host_offsets[b] < host_offsets[b - 1]) return false;
+    out->start[b] = host_offsets[b];
+  }
+  for (int b = batch_size + 1; b <= WCN_VOXEL_MAX_BATCH; ++b) out->start[b] = num_rows;
+  return host_offsets[batch_size] == num_rows;
+}
+
+#ifdef __HIPCC__
+// The item of row i: `start` in LDS (lanes search at different places).
+__device__ __forceinline__ int wcn_item_of(const int64_t* start, int batch_size, int64_t i) {
+  int lo = 0, hi = batch_size;  // the item lies in [lo, hi)
+  while (hi - lo > 1) {
+    const int mid = (lo + hi) >> 1;
+    if (start[mid] <= i) lo = mid; else hi = mid;
+  }
+  return lo;
+}
+#endif
+
 // Small device-to-host reads (map offsets, table status, row counts): copied into pinned memory
 // and awaited by polling an event, which returns within a few microseconds of the copy's end (a
 // blocking stream synchronisation wakes the host tens of microseconds later).  One staging buffer

@@ -142,6 +142,19 @@ std::pair<Tensor, int64_t> table_build(const Tensor& keys4, int64_t slots) {
   return {table, slots};
 }
 
+/* (rows, table workspace, slot count): batch_rows and table_build of (n, 3) coordinates in one. */
+py::tuple batch_rows_table(const Tensor& coords, const std::vector<int64_t>& offsets) {
+  at::AutoDispatchBelowADInplaceOrView guard;
+  const Tensor c = coords.contiguous();
+  const int64_t n = c.size(0), slots = wcn_table_default_capacity(n);
+  Tensor rows = at::empty({n, 4}, c.options());
+  Tensor table = bytes_on(wcn_table_bytes(n, slots), c);
+  check(wcn_table_build_items(c.const_data_ptr<int32_t>(), n, offsets.data(), static_cast<int32_t>(offsets.size() - 1),
+                              rows.mutable_data_ptr<int32_t>(), table.mutable_data_ptr(), slots, stream_of(c)),
+        "wcn_table_build_items");
+  return py::make_tuple(rows, table, slots);
+}
+
 struct TableRef {  // what the builder reads of a TorchHashTable object
   Tensor raw, keys;
   int64_t slots;
@@ -1180,6 +1193,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   });
   py::class_<PreparedWeight, std::shared_ptr<PreparedWeight>>(m, "PreparedWeight");
   m.def("batch_rows", &batch_rows);
+  m.def("batch_rows_table", &batch_rows_table);
   m.def("table_build", &table_build);
   m.def("stride_cells", &stride_cells);
   m.def("kernel_map", &kernel_map);

@@ -22,6 +22,8 @@
 #include <mutex>
 #include <thread>
 
+#include <algorithm>
+
 #include "wcn_common.h"
 
 namespace {
@@ -53,11 +55,23 @@ constexpr int SMALL_BINS = 4096;
 
 // Keys per bin of one part of the keys, the part's bounding box; the part's share of the slots is
 // set to empty on the way (each slot is two 16-byte stores, {EMPTY, 0} and {0, 0, 0, 0}).
+// ITEMS: the keys are made here too, [batch item, x, y, z] of three columns, and written on the way (the launch that did nothing else
+// took 7.7 us over 1 M rows; with this pass 11.4 + 7.7 -> 14.8; few keys: 2.4 + 2.1 -> 2.4 and a launch less).
+struct KeysOfItems {
+  const int32_t* coords;  // (n, 3)
+  int4* rows;
+  WcnItemStarts starts;
+  int32_t batch_size;
+};
+
+template <bool ITEMS>
 __global__ void __launch_bounds__(1024) table_hist(const int4* __restrict__ keys, int64_t n_keys,
                                                    int32_t bins, int32_t* __restrict__ hist,
                                                    int32_t* __restrict__ part_box,
-                                                   WcnSlot* __restrict__ slots, int64_t capacity) {
+                                                   WcnSlot* __restrict__ slots, int64_t capacity, KeysOfItems of) {
   extern __shared__ int s_cnt[];  // [bins]
+  __shared__ int64_t s_start[ITEMS ? WCN_VOXEL_MAX_BATCH + 1 : 1];
+  if (ITEMS && threadIdx.x <= WCN_VOXEL_MAX_BATCH) s_start[threadIdx.x] = of.starts.start[threadIdx.x];
   __shared__ int s_mn[16][4];
   __shared__ int s_mx[16][4];
   const int tid = threadIdx.x, parts = gridDim.x, part = wcn_xcd_tile((int)blockIdx.x, parts);
@@ -72,11 +86,17 @@ __global__ void __launch_bounds__(1024) table_hist(const int4* __restrict__ keys
     int4 c[PER];
 #pragma unroll
     for (int t = 0; t < PER; ++t) {
-      const int64_t i = i0 + t * 1024;
-      c[t] = keys[i < r.hi ? i : i0];
+      const int64_t i = i0 + t * 1024 < r.hi ? i0 + t * 1024 : i0;
+      if (ITEMS) c[t] = make_int4(0, of.coords[3 * i], of.coords[3 * i + 1], of.coords[3 * i + 2]);
+      else c[t] = keys[i];
     }
 #pragma unroll
     for (int t = 0; t < PER; ++t) {
+      if (ITEMS) {
+        const int64_t i = i0 + t * 1024 < r.hi ? i0 + t * 1024 : i0;
+        c[t].x = wcn_item_of(s_start, of.batch_size, i);
+        of.rows[i] = c[t];
+      }
       if (i0 + t * 1024 < r.hi) atomicAdd(&s_cnt[bin_of(c[t], bin_mask)], 1);
       mn[0] = min(mn[0], c[t].x); mx[0] = max(mx[0], c[t].x);
       mn[1] = min(mn[1], c[t].y); mx[1] = max(mx[1], c[t].y);
@@ -523,9 +543,17 @@ __global__ void __launch_bounds__(1024) table_bins(WcnTableHeader* __restrict__ 
 constexpr int64_t SMALL_KEYS = 16384;
 constexpr int SMALL_KEY_BINS = 64;  // more bins (a table that was grown) would read the keys too often
 
+template <bool ITEMS>  // the keys are made on the way, as in table_hist
 __global__ void __launch_bounds__(256) table_clear(uint4* __restrict__ raw, int64_t items, WcnTableHeader* __restrict__ hdr,
-                                                   int32_t n_keys, int32_t bins, int64_t stats_offset) {
+                                                   int32_t n_keys, int32_t bins, int64_t stats_offset, KeysOfItems of) {
   const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (ITEMS) {
+    __shared__ int64_t s_start[WCN_VOXEL_MAX_BATCH + 1];
+    if (threadIdx.x <= WCN_VOXEL_MAX_BATCH) s_start[threadIdx.x] = of.starts.start[threadIdx.x];
+    __syncthreads();
+    if (i < n_keys)
+      of.rows[i] = make_int4(wcn_item_of(s_start, of.batch_size, i), of.coords[3 * i], of.coords[3 * i + 1], of.coords[3 * i + 2]);
+  }
   if (i < items) raw[i] = (i & 1) ? make_uint4(0u, 0u, 0u, 0u) : make_uint4(0xFFFFFFFFu, 0xFFFFFFFFu, 0u, 0u);
   if (i == 0) {
     hdr->num_blocks = 0;
@@ -678,7 +706,7 @@ inline int grid_for(int64_t n, int block, int cap = 0x7fffffff) {
 // LDS beyond the default limit: lifted once per device and kernel.
 static int allow_lds(const void* kernel, size_t bytes, int which) {
   static std::mutex mu;
-  static bool allowed[6][64] = {};
+  static bool allowed[7][64] = {};
   int device = 0;
   if (hipGetDevice(&device) != hipSuccess || device < 0 || device >= 64) return WCN_ERR_LAUNCH;
   std::lock_guard<std::mutex> hold(mu);
@@ -691,17 +719,18 @@ static int allow_lds(const void* kernel, size_t bytes, int which) {
 
 // Enqueue the build kernels.  Shared with the strided-coordinate path, which also wants the slot of
 // every key (`want_slot_of`).
-int wcn_table_build_impl(const int32_t* keys, int64_t n_keys, const WcnTableView& v,
-                         bool want_slot_of, hipStream_t s) {
+static int table_build_from(const int32_t* keys, int64_t n_keys, const WcnTableView& v, const KeysOfItems* items,
+                            bool want_slot_of, hipStream_t s) {
   const uint32_t cap_mask = (uint32_t)(v.capacity - 1);
   const int4* k4 = (const int4*)keys;
   if (v.bins < 1 || v.bins > WCN_MAX_BINS || (v.bins & (v.bins - 1))) return WCN_ERR_INVALID_ARGUMENT;
   if (n_keys >= 1 && n_keys <= SMALL_KEYS && v.bins <= SMALL_KEY_BINS) {
     auto small = want_slot_of ? table_small<true> : table_small<false>;
     if (allow_lds((const void*)small, sizeof(SmallLds), want_slot_of ? 4 : 3) != WCN_OK) return WCN_ERR_LAUNCH;
-    const int64_t items = 2 * v.capacity, stats = (int64_t)((const char*)v.bin_stats - (const char*)v.hdr);
-    hipLaunchKernelGGL(table_clear, dim3((unsigned)((items + 255) / 256)), dim3(256), 0, s, (uint4*)v.slots, items, v.hdr,
-                       (int32_t)n_keys, v.bins, stats);
+    const int64_t words = 2 * v.capacity, stats = (int64_t)((const char*)v.bin_stats - (const char*)v.hdr);
+    const int64_t clears = std::max(words, n_keys);
+    hipLaunchKernelGGL((items ? table_clear<true> : table_clear<false>), dim3((unsigned)((clears + 255) / 256)), dim3(256), 0, s,
+                       (uint4*)v.slots, words, v.hdr, (int32_t)n_keys, v.bins, stats, items ? *items : KeysOfItems{});
     hipLaunchKernelGGL(small, dim3(v.bins), dim3(1024), sizeof(SmallLds), s, k4, (int32_t)n_keys, v.bins, v.hdr,
                        v.slots, cap_mask, v.bin_start, v.order_tag, v.order_row, v.block_list, v.perm, v.slot_of,
                        v.bin_stats);
@@ -711,15 +740,16 @@ int wcn_table_build_impl(const int32_t* keys, int64_t n_keys, const WcnTableView
   const bool many_bins = v.bins > SMALL_BINS;
   const size_t counters = sizeof(int) * (size_t)v.bins;
   auto scatter = many_bins ? table_scatter<WCN_MAX_BINS / 1024> : table_scatter<SMALL_BINS / 1024>;
+  auto hist = items ? table_hist<true> : table_hist<false>;
   auto fn = want_slot_of ? table_bins<true> : table_bins<false>;
   if (allow_lds((const void*)fn, sizeof(BinLds), want_slot_of ? 1 : 0) != WCN_OK) return WCN_ERR_LAUNCH;
   if (many_bins) {
     const size_t most = sizeof(int) * WCN_MAX_BINS;
-    if (allow_lds((const void*)table_hist, most, 2) != WCN_OK || allow_lds((const void*)scatter, most, 5) != WCN_OK)
+    if (allow_lds((const void*)hist, most, items ? 6 : 2) != WCN_OK || allow_lds((const void*)scatter, most, 5) != WCN_OK)
       return WCN_ERR_LAUNCH;
   }
-  hipLaunchKernelGGL(table_hist, dim3(v.parts), dim3(1024), counters, s, k4, n_keys, v.bins, v.hist,
-                     v.part_box, v.slots, v.capacity);
+  hipLaunchKernelGGL(hist, dim3(v.parts), dim3(1024), counters, s, k4, n_keys, v.bins, v.hist,
+                     v.part_box, v.slots, v.capacity, items ? *items : KeysOfItems{});
   hipLaunchKernelGGL(table_colscan, dim3((v.bins + 3) / 4), dim3(256), 0, s, v.hist, v.bins,
                      v.parts, v.bin_total);
   hipLaunchKernelGGL(scatter, dim3(v.parts), dim3(1024), counters, s, k4, n_keys, v.bins, v.hist,
@@ -731,6 +761,10 @@ int wcn_table_build_impl(const int32_t* keys, int64_t n_keys, const WcnTableView
                      v.block_list, v.perm, v.slot_of, v.bin_stats);
   WCN_LAUNCH_CHECK();
   return WCN_OK;
+}
+
+int wcn_table_build_impl(const int32_t* keys, int64_t n_keys, const WcnTableView& v, bool want_slot_of, hipStream_t s) {
+  return table_build_from(keys, n_keys, v, nullptr, want_slot_of, s);
 }
 
 
@@ -973,6 +1007,17 @@ int wcn_table_build(const int32_t* keys, int64_t n_keys, void* table, int64_t ca
   WcnTableView v;
   wcn_table_layout(table, n_keys, capacity, &v);
   return wcn_table_build_impl(keys, n_keys, v, false, (hipStream_t)stream);
+}
+
+int wcn_table_build_items(const int32_t* coords, int64_t n_rows, const int64_t* host_batch_offsets, int32_t batch_size,
+                          int32_t* rows, void* table, int64_t capacity, void* stream) {
+  KeysOfItems of = {coords, (int4*)rows, {}, batch_size};
+  if (!table || n_rows < 1 || n_rows >= (1ll << 31) || !coords || !rows || (uintptr_t)rows % 16 != 0 || !is_pow2(capacity) ||
+      capacity < 64 || capacity > (1ll << 31) || !wcn_item_starts(host_batch_offsets, batch_size, n_rows, &of.starts))
+    return WCN_ERR_INVALID_ARGUMENT;
+  WcnTableView v;
+  wcn_table_layout(table, n_rows, capacity, &v);
+  return table_build_from(rows, n_rows, v, &of, false, (hipStream_t)stream);
 }
 
 int wcn_table_query(const void* table, int64_t n_keys, int64_t capacity, const int32_t* queries,

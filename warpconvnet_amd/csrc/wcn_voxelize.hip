@@ -164,9 +164,7 @@ size_t unique_layout(void* base, int64_t n, UniqueView* v) {
 // ---- where the rows come from -------------------------------------------------------------------
 // torch divides a float tensor by a host scalar as a multiplication with the scalar's reciprocal
 // (taken in double, rounded to float); the product is floored and converted to int32 the same way.
-struct BatchStarts {
-  int64_t start[WCN_VOXEL_MAX_BATCH + 1];
-};
+typedef WcnItemStarts BatchStarts;
 
 struct ItemHint {
   int item;       // of a row,
@@ -251,11 +249,7 @@ __global__ void __launch_bounds__(256) batch_indexed_rows(const int32_t* __restr
   __syncthreads();
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
-  int lo = 0, hi = batch_size;  // the item lies in [lo, hi)
-  while (hi - lo > 1) {
-    const int mid = (lo + hi) >> 1;
-    if (s_start[mid] <= i) lo = mid; else hi = mid;
-  }
+  const int lo = wcn_item_of(s_start, batch_size, i);
   if (dims == 3) {
     const int32_t* c = coords + 3 * i;
     reinterpret_cast<int4*>(rows)[i] = make_int4(lo, c[0], c[1], c[2]);
@@ -1373,16 +1367,9 @@ int wcn_voxel_rows(const float* points, int64_t num_points, const int64_t* host_
 int wcn_batch_indexed_rows(const int32_t* coords, int64_t num_rows, int32_t dims,
                            const int64_t* host_batch_offsets, int32_t batch_size, int32_t* rows,
                            void* stream) {
-  if (num_rows < 0 || dims < 1 || batch_size < 1 || batch_size > WCN_VOXEL_MAX_BATCH ||
-      !host_batch_offsets)
-    return WCN_ERR_INVALID_ARGUMENT;
   BatchStarts starts;
-  for (int b = 0; b <= batch_size; ++b) {
-    starts.start[b] = host_batch_offsets[b];
-    if (b > 0 && starts.start[b] < starts.start[b - 1]) return WCN_ERR_INVALID_ARGUMENT;
-  }
-  for (int b = batch_size + 1; b <= WCN_VOXEL_MAX_BATCH; ++b) starts.start[b] = num_rows;
-  if (starts.start[0] != 0 || starts.start[batch_size] != num_rows) return WCN_ERR_INVALID_ARGUMENT;
+  if (num_rows < 0 || dims < 1 || !wcn_item_starts(host_batch_offsets, batch_size, num_rows, &starts))
+    return WCN_ERR_INVALID_ARGUMENT;
   if (num_rows == 0) return WCN_OK;
   if (!coords || !rows) return WCN_ERR_INVALID_ARGUMENT;
   hipLaunchKernelGGL(batch_indexed_rows, dim3((unsigned)((num_rows + 255) / 256)), dim3(256), 0,

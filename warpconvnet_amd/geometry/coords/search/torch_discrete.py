@@ -21,6 +21,7 @@ from torch import Tensor
 from ...._lib import host as native
 from ...._lib import stream_ptr
 from ....utils.ntuple import ntuple
+from ..ops.batch_index import _BY_VALUE_BATCHES
 from .search_results import IntSearchResult
 from .torch_hashmap import HashMethod, TorchHashTable, _four_columns
 
@@ -129,6 +130,20 @@ def _table_of(coords: Tensor, hash_method: HashMethod, device) -> TorchHashTable
     except AttributeError:
         pass
     return table
+
+
+def rows_with_table(coords) -> Tensor:
+    """batch_indexed_coordinates of an IntCoords whose table the caller is about to need: where neither exists yet,
+    rows and table are made by the same launches, and the table is kept as _table_of keeps it."""
+    if coords._batch_indexed is None:
+        t, host = coords.batched_tensor, coords.offsets.tolist()
+        if (t.is_cuda and t.dtype == torch.int32 and t.ndim == 2 and t.shape[1] == 3 and t.shape[0] > 0
+                and 2 <= len(host) <= _BY_VALUE_BATCHES + 1 and host[0] == 0 and host[-1] == t.shape[0]):
+            with torch.no_grad():
+                rows, table, slots = native().batch_rows_table(t, host)
+            rows._wcn_table = (rows._version, TorchHashTable._over(rows.detach(), table, slots), _stream_of(rows))
+            coords._batch_indexed = rows
+    return coords.batch_indexed_coordinates
 
 
 @torch.no_grad()

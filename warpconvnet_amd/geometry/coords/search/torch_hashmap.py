@@ -147,13 +147,20 @@ class TorchHashTable:
     @classmethod
     def _deferred(cls, rows: Tensor) -> "TorchHashTable":
         """from_keys(rows, _defer_check=True) of (N, 4) contiguous int32 rows on a GPU."""
+        obj = cls._over(rows)
+        obj._build(0)
+        return obj
+
+    @classmethod
+    def _over(cls, rows: Tensor, table: Optional[Tensor] = None, slots: int = 0) -> "TorchHashTable":
+        """The object around a table of (N, 4) rows that the library has made, or is about to make."""
         obj = cls.__new__(cls)
         obj._capacity = max(16, 2 * rows.shape[0])
         obj._hash_method_enum = HashMethod.CITY
         obj._device = rows.device
         obj._vector_keys = obj._keys4 = rows
         obj._key_dim = 4
-        obj._build(0)
+        obj._table, obj._slots, obj._checked = table, slots, False
         return obj
 
     # -- query ---------------------------------------------------------------------------------

@@ -30,7 +30,7 @@ from ...geometry.coords.ops.serialization import POINT_ORDERING, encode
 from ...geometry.coords.ops.stride import stride_coords
 from ...geometry.coords.search.cache import IntSearchCache, IntSearchCacheKey
 from ...geometry.coords.search.search_results import IntSearchResult
-from ...geometry.coords.search.torch_discrete import generate_kernel_map
+from ...geometry.coords.search.torch_discrete import generate_kernel_map, rows_with_table
 from ...geometry.types.voxels import Voxels
 from ...utils.ntuple import ntuple
 from ...utils.gather import take_rows
@@ -232,7 +232,9 @@ def generate_output_coords_and_kernel_map(
     if strided and stride_mode == STRIDED_CONV_MODE.REDUCE_AND_STRIDE:
         raise ValueError("REDUCE_AND_STRIDE reaches the map builder with stride 1 (the functional "
                          "entry point pools the input by the stride first)")
-    in_coords = input_sparse_tensor.batch_indexed_coordinates
+    # (a transposed layer looks its inputs up from the output rows: its table is not over these)
+    in_coords = (input_sparse_tensor.batch_indexed_coordinates if transposed or type(input_sparse_tensor.batched_coordinates) is not IntCoords
+                 else rows_with_table(input_sparse_tensor.batched_coordinates))
 
     # output coordinates: given, expanded (generative), strided, or the input's (sparse_conv.py:1843-1886)
     if output_spatially_sparse_tensor is not None:

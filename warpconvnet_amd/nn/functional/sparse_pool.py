@@ -16,7 +16,7 @@ from ..._lib import host as native
 from ...geometry.coords.integer import IntCoords
 from ...geometry.coords.ops.stride import stride_coords
 from ...geometry.coords.search.cache import IntSearchCache, IntSearchCacheKey
-from ...geometry.coords.search.torch_discrete import generate_kernel_map
+from ...geometry.coords.search.torch_discrete import generate_kernel_map, rows_with_table
 from ...geometry.types.voxels import Voxels
 from ...ops.reductions import REDUCTIONS
 from ...utils.ntuple import ntuple
@@ -44,7 +44,8 @@ def sparse_reduce(voxels: Voxels, kernel_size: Union[int, Tuple[int, ...]],
         in_tensor_stride = ntuple(1, ndim=ndim)
     out_tensor_stride = tuple(o * s for o, s in zip(stride, in_tensor_stride))
 
-    in_coords = voxels.batch_indexed_coordinates
+    in_coords = (rows_with_table(voxels.batched_coordinates) if type(voxels.batched_coordinates) is IntCoords
+                 else voxels.batch_indexed_coordinates)
     out_coords, out_offsets = stride_coords(in_coords, stride, order=order, batch_sorted=True)
     from .sparse_conv import STRIDED_CONV_MODE
     key = IntSearchCacheKey(kernel_size=kernel_size, kernel_dilation=ntuple(1, ndim=ndim),
