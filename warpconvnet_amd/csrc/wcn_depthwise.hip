@@ -19,12 +19,14 @@ using namespace wcn_rows;
 // is X[m] * W[identity] for every m < num_in and its pairs are ignored (sparse_conv_depth.py:163-165).
 // The bias is added to the rounded sum, as a separate addition behind the call would.
 //
-// Bound by the rate of the gathered rows (4.3 TB/s behind the L2; a gather alone of these rows: 40 us) and by the LDS that
-// the weights come from (two thirds of its cycles, most of them bank conflicts).  LDS_W: the
+// Bound by the rate of the gathered rows (a gather alone of these rows: 40 us) and by the LDS that
+// the weights come from.  (A piece's eight weights side by side, its two 16-byte reads 32 bytes from its neighbour's: two thirds of
+// the LDS's cycles, most of them bank conflicts, and 71.6 us below; the halves apart: 64.2.  Rows padded by 16, 32, 64
+// bytes on top: the same.)  LDS_W: the
 // weight, as fp32, in LDS for the life of the workgroup, which takes many rows; read from memory instead, the
 // rows of a wave asked for eight different weight rows per entry, two 16-byte loads each beside the one of the
 // feature row.  Eight entries in flight and the next row's mask on its way: 500 k rows of 64 fp16
-// channels, 4.2 entries a row, 258 -> 75 us (four entries: 77; with a branch around each load: 107).
+// channels, 4.2 entries a row, 258 -> 75 us at the time (four entries: 77; with a branch around each load: 107).
 template <typename T, typename WT, bool LDS_W, bool VEC>
 __global__ void __launch_bounds__(256) depthwise_rows(const T* __restrict__ X, int64_t num_in, int channels,
                                                       RowTiling tiling, const WT* __restrict__ W, int K, int identity,
@@ -33,12 +35,15 @@ __global__ void __launch_bounds__(256) depthwise_rows(const T* __restrict__ X, i
                                                       const int32_t* __restrict__ row_in, int64_t num_out,
                                                       const T* __restrict__ bias, T* __restrict__ out) {
   constexpr int N = Piece<T>::N, U = 8;
-  extern __shared__ float s_w[];  // K rows of pieces * N
-  const int padded = tiling.pieces * N;
+  // The first four channels of every piece, then the last four: in either, K rows of 16 bytes per piece, so that the
+  // pieces of a row lie side by side.
+  extern __shared__ __attribute__((aligned(16))) float s_w[];
+  const int pitch = tiling.pieces * 4;
   if (LDS_W) {
+    const int padded = tiling.pieces * N;
     for (int i = threadIdx.x; i < K * padded; i += 256) {
       const int k = i / padded, c = i % padded;
-      s_w[i] = c < channels ? to_float(W[(int64_t)k * channels + c]) : 0.f;
+      s_w[(c % N / 4 * K + k) * pitch + c / N * 4 + c % 4] = c < channels ? to_float(W[(int64_t)k * channels + c]) : 0.f;
     }
     __syncthreads();
   }
@@ -61,7 +66,10 @@ __global__ void __launch_bounds__(256) depthwise_rows(const T* __restrict__ X, i
       for (int j = 0; j < N; ++j) acc[j] = 0.f;
       auto add = [&](const Piece<T>& x, int k) {
         if (LDS_W) {
-          const float* w = s_w + k * padded + c0;
+          float w[N];
+#pragma unroll
+          for (int h = 0; h < N / 4; ++h)
+            *reinterpret_cast<f32x4*>(w + 4 * h) = *reinterpret_cast<const f32x4*>(s_w + (h * K + k) * pitch + piece * 4);
 #pragma unroll
           for (int j = 0; j < N; ++j) acc[j] += to_float(x.v[j]) * w[j];
         } else {
@@ -288,7 +296,7 @@ int wcn_sparse_depthwise_fwd_fused(const void* features, int64_t num_in, int32_t
   wcn_rows_layout(const_cast<void*>(rows_by_out), num_out, num_offsets, num_pairs, &v);
   const bool vec = rows_are_vectors(features, channels, dtype) && rows_are_vectors(out, channels, dtype);
   const RowTiling t = row_tiling(channels, dtype);
-  const size_t lds = sizeof(float) * (size_t)num_offsets * t.pieces * (dtype == WCN_DTYPE_F32 ? 4 : 8);
+  const size_t lds = sizeof(float) * (size_t)num_offsets * (t.pieces * 4) * (dtype == WCN_DTYPE_F32 ? 1 : 2);
   // up to 32 KB a CU still holds five workgroups; more of them than one pass over the chip only make more copies
   const bool lds_w = lds <= 32768;
   const int64_t need = (num_out + t.rows - 1) / t.rows;
