@@ -14,9 +14,10 @@
 // once for every 64 channels of the other side.)  Piece p (16 bytes) of row r sits at p ^ f(r), f even, so that the sixteen
 // 32-byte runs of a transposing read lie in different banks; the source side arranges it.
 //
-// What bounds it: the gathered rows (6 to 7 TB/s behind the L2, which hits 7 to 15 %; matrix pipes 12 to 22 %) and, for a few thousand pairs per offset, the partial sums (64 KB per chunk).
+// What bounds it: the gathered rows (6 to 7 TB/s behind the L2; matrix pipes 12 to 22 %) and, for a few thousand pairs per offset, the partial sums (64 KB per chunk).
 // A stage of 3x3x3 96 -> 96 over 300 k rows and 128 -> 128 over 170 k with its 2x2x2 layers, bf16, all four weight gradients:
-// 667 -> 285 us (91, 107, 30 and 29, reductions 27).
+// 667 -> 285 us (91, 107, 30 and 29, reductions 27); with the rows of dY shared in the XCDs' L2s (wgrad_first_chunk) 232 (74, 80, 25 and
+// 28), where every row of dY came from behind the L2 for every offset.
 #include <algorithm>
 #include <mutex>
 
@@ -42,32 +43,49 @@ struct WgradTileArgs {
   const int64_t* offsets;  // (K + 1), device
   float* partial;          // (chunks, c_in_pad, c_out_pad)
   int64_t num_in, num_out, identity_rows;
-  int32_t K, c_in, c_out, c_in_pad, c_out_pad, identity, pairs_per_chunk, chunks, tiles_in, tiles_out;
+  int32_t K, c_in, c_out, c_in_pad, c_out_pad, identity, pairs_per_chunk, chunks, tiles_in, tiles_out;  // chunks: most on an XCD
 };
 
 __device__ __forceinline__ void to_lds(const char* g, uint32_t lds_off) {
   asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(g), "s"(lds_off) : "memory");
 }
 
-// The offset that a chunk belongs to and the chunks before it: the first 64 offsets by a scan over the lanes, then the next.
-__device__ __forceinline__ int chunk_offset(const int64_t* __restrict__ offsets, int K, int identity, int64_t identity_rows,
-                                            int per, int chunk, int* before) {
-  int base = 0;
+// Which chunks of an offset (W of them, in the order of its pairs) an XCD works on: those of about an eighth of the pairs, the
+// same eighth for all offsets, so that the rows of dY (which ascend inside every offset) that its workgroups read at a time are the
+// same few thousand and come out of its L2 for all offsets but the first.  The rounding differs from offset to offset, so
+// that no XCD gets the odd chunk of all of them.
+__host__ __device__ inline int wgrad_first_chunk(int xcd, int chunks, int k) {
+  const int64_t at = (int64_t)xcd * chunks - (5 * k & 7);
+  return at <= 0 ? 0 : (int)((at + 7) / 8);
+}
+
+struct WgradChunk {
+  int k, chunk, chunks, before;  // offset, number among its chunks, how many it has, and those of the offsets before it
+};
+// The q-th chunk of an XCD: a lane per offset, 64 offsets at a time.
+__device__ __forceinline__ WgradChunk chunk_of(const int64_t* __restrict__ offsets, int K, int identity, int64_t identity_rows,
+                                               int per, int xcd, int q) {
+  int here = 0, all = 0;
   for (int k0 = 0; k0 < K; k0 += 64) {
     const int k = k0 + wcn_lane();
     int64_t n = k < K ? offsets[k + 1] - offsets[k] : 0;
     if (k == identity) n = identity_rows;
-    const int mine = (int)((n + per - 1) / per);
-    const int incl = wcn_wave_inclusive_sum(mine);
-    const int past = __popcll(__ballot(base + incl <= chunk));  // offsets that end at or before the chunk
+    const int W = (int)((n + per - 1) / per);
+    const int j0 = wgrad_first_chunk(xcd, W, k), mine = wgrad_first_chunk(xcd + 1, W, k) - j0;
+    const int incl = wcn_wave_inclusive_sum(mine), incl_all = wcn_wave_inclusive_sum(W);
+    const int past = __popcll(__ballot(here + incl <= q));  // offsets whose chunks here end at or before this one
     if (past < 64) {
-      *before = base + __shfl(incl - mine, past, 64);
-      return k0 + past;
+      WgradChunk c;
+      c.k = k0 + past;
+      c.chunk = __shfl(j0, past, 64) + q - (here + __shfl(incl - mine, past, 64));
+      c.chunks = __shfl(W, past, 64);
+      c.before = all + __shfl(incl_all - W, past, 64);
+      return c;
     }
-    base += __shfl(incl, 63, 64);
+    here += __shfl(incl, 63, 64);
+    all += __shfl(incl_all, 63, 64);
   }
-  *before = base;
-  return K;
+  return {K, 0, 1, all};
 }
 
 template <int N>
@@ -95,19 +113,22 @@ __global__ void __launch_bounds__(256, 2) conv_wgrad_tiles(WgradTileArgs a) {
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   // the tiles of a chunk follow one another on one XCD (blockIdx % 8): they gather the same rows
   const int tiles = a.tiles_in * a.tiles_out, b8 = (int)blockIdx.x >> 3;
-  const int chunk = (b8 / tiles) * 8 + ((int)blockIdx.x & 7), tile = b8 % tiles;
-  if (chunk >= a.chunks) return;
+  const int xcd = (int)blockIdx.x & 7, tile = b8 % tiles;
   const int ci0 = tile / a.tiles_out * I::T, co0 = tile % a.tiles_out * O::T;
-  int before = 0;
-  const int k = __builtin_amdgcn_readfirstlane(
-      chunk_offset(a.offsets, a.K, a.identity, a.identity_rows, a.pairs_per_chunk, chunk, &before));
+  const WgradChunk at_chunk = chunk_of(a.offsets, a.K, a.identity, a.identity_rows, a.pairs_per_chunk, xcd, b8 / tiles);
+  const int k = __builtin_amdgcn_readfirstlane(at_chunk.k);
   if (k >= a.K) return;
-  before = __builtin_amdgcn_readfirstlane(before);
+  const int W = __builtin_amdgcn_readfirstlane(at_chunk.chunks), j = __builtin_amdgcn_readfirstlane(at_chunk.chunk);
+  const int chunk = __builtin_amdgcn_readfirstlane(at_chunk.before) + j;
   const bool ident = k == a.identity;
   const int64_t n_k = ident ? a.identity_rows : a.offsets[k + 1] - a.offsets[k];
-  const int64_t first = (int64_t)(chunk - before) * a.pairs_per_chunk;
-  const int count = (int)(n_k - first < a.pairs_per_chunk ? n_k - first : a.pairs_per_chunk);
-  const int64_t pbase = a.offsets[k] + first;
+  // The steps of an XCD's chunks of the offset are dealt to them in turn: all its workgroups move through their eighth together.
+  const int j0 = wgrad_first_chunk(xcd, W, k), abreast = wgrad_first_chunk(xcd + 1, W, k) - j0;
+  const uint32_t all_steps = (uint32_t)((n_k + KP - 1) / KP), each = all_steps / (uint32_t)W, odd = all_steps - each * (uint32_t)W;
+  auto steps_before = [&](uint32_t c) { return (int64_t)each * c + odd * c / (uint32_t)W; };  // of chunk c; W < 65,536
+  const int64_t step0 = steps_before((uint32_t)j0) + (j - j0), step1 = steps_before((uint32_t)(j0 + abreast));
+  const int my_steps = step1 > step0 ? (int)((step1 - step0 + abreast - 1) / abreast) : 0;
+  const int64_t pbase = a.offsets[k];
   const uint32_t in_bytes = (uint32_t)a.c_in * 2u, out_bytes = (uint32_t)a.c_out * 2u;
   const char* const zeros = (const char*)wgrad_zeros + lane * 16;
 
@@ -165,15 +186,16 @@ __global__ void __launch_bounds__(256, 2) conv_wgrad_tiles(WgradTileArgs a) {
 #pragma unroll
     for (int y = 0; y < NO; ++y) acc[x][y] = (f32x4){0.f, 0.f, 0.f, 0.f};
 
-  for (int seg = 0; seg < count; seg += SEGMENT) {
-    const int here = count - seg < SEGMENT ? count - seg : SEGMENT;
-    const int steps = (here + KP - 1) / KP;
+  constexpr int SEG_STEPS = SEGMENT / KP;
+  for (int seg = 0; seg < my_steps; seg += SEG_STEPS) {
+    const int steps = my_steps - seg < SEG_STEPS ? my_steps - seg : SEG_STEPS;
     // the rows' numbers; a pair that is not there, or names rows that are not, adds nothing
     for (int p = tid; p < (steps + 1) * KP && p < SEGMENT; p += 256) {
       int32_t rin = -1, rout = -1;
-      if (p < here) {
-        rin = ident ? (int32_t)(first + seg + p) : a.in_maps[pbase + seg + p];
-        rout = ident ? (int32_t)(first + seg + p) : a.out_maps[pbase + seg + p];
+      const int64_t pair = (step0 + (int64_t)(seg + p / KP) * abreast) * KP + p % KP;
+      if (p < steps * KP && pair < n_k) {
+        rin = ident ? (int32_t)pair : a.in_maps[pbase + pair];
+        rout = ident ? (int32_t)pair : a.out_maps[pbase + pair];
       }
       const bool there = (uint32_t)rin < (uint64_t)a.num_in && (uint32_t)rout < (uint64_t)a.num_out;
       s_in[p] = there ? rin : -1;
@@ -257,11 +279,13 @@ __global__ void __launch_bounds__(256) wgrad_tiles_reduce(WgradTileArgs a, WT* _
 inline int blocks_of(int c) { return c <= 32 ? 1 : c <= 64 ? 2 : c <= 96 ? 3 : 4; }  // 32-channel blocks of a tile
 inline int padded(int c) { return (c + 32 * blocks_of(c) - 1) / (32 * blocks_of(c)) * (32 * blocks_of(c)); }
 
-// Pairs per chunk: as many workgroups as the chip holds at once (two per CU with tiles of more than 64 channels on both
-// sides, else three), so that none is left for a second round; a multiple of a step and not fewer than 256.
+// Workgroups that the chip holds at once: two per CU with tiles of more than 64 channels on both sides, else three.
+inline int64_t wgrad_slots(int c_in, int c_out) { return blocks_of(c_in) > 2 && blocks_of(c_out) > 2 ? 512 : 768; }
+// Pairs per chunk: as many workgroups as that, so that none is left for a second round; a multiple of a step and not
+// fewer than 256.
 inline int64_t wgrad_pairs_per_chunk(int64_t pairs, int K, int c_in, int c_out) {
   const int64_t tiles = (int64_t)(padded(c_in) / (32 * blocks_of(c_in))) * (padded(c_out) / (32 * blocks_of(c_out)));
-  const int64_t slots = (blocks_of(c_in) > 2 && blocks_of(c_out) > 2 ? 512 : 768) / tiles;
+  const int64_t slots = wgrad_slots(c_in, c_out) / tiles;
   const int64_t want = std::max<int64_t>(64, std::max(slots / 2, slots - K / 2));  // half a chunk is lost per offset
   const int64_t p = std::max<int64_t>(256, (pairs + want - 1) / want);
   return std::min<int64_t>((p + KP - 1) / KP * KP, 1 << 30);
@@ -282,7 +306,7 @@ int launch_wgrad_tiles(const WgradTileArgs& a, hipStream_t s) {
       allowed[device] = true;
     }
   }
-  const int64_t grid = ((int64_t)a.chunks + 7) / 8 * 8 * a.tiles_in * a.tiles_out;
+  const int64_t grid = (int64_t)a.chunks * 8 * a.tiles_in * a.tiles_out;
   if (grid > INT32_MAX) return WCN_ERR_INVALID_ARGUMENT;
   if (grid > 0) hipLaunchKernelGGL((conv_wgrad_tiles<T, NI, NO>), dim3((unsigned)grid), dim3(256), lds, s, a);
   return WCN_OK;
@@ -338,16 +362,26 @@ int wcn_wgrad_tiles_launch(const void* features, int64_t num_in, int c_in, const
   a.c_in_pad = padded(c_in);
   a.c_out_pad = padded(c_out);
   a.identity = identity;
-  a.pairs_per_chunk = (int)wgrad_pairs_per_chunk(host_offsets[num_offsets] + a.identity_rows, num_offsets, c_in, c_out);
   a.tiles_in = a.c_in_pad / (32 * blocks_of(c_in));
   a.tiles_out = a.c_out_pad / (32 * blocks_of(c_out));
-  int64_t chunks = 0;  // the device computes the same numbers from the same inputs
-  for (int k = 0; k < num_offsets; ++k) {
-    const int64_t n = k == identity ? a.identity_rows : host_offsets[k + 1] - host_offsets[k];
-    chunks += (n + a.pairs_per_chunk - 1) / a.pairs_per_chunk;
+  // The device computes the same numbers from the same inputs.  Chunks get longer until every XCD holds its own at once.
+  int64_t per = wgrad_pairs_per_chunk(host_offsets[num_offsets] + a.identity_rows, num_offsets, c_in, c_out);
+  const int64_t room = wgrad_slots(c_in, c_out) / 8 / ((int64_t)a.tiles_in * a.tiles_out);
+  for (int turn = 0;; ++turn) {
+    int64_t here[8] = {}, most = 0;
+    for (int k = 0; k < num_offsets; ++k) {
+      const int64_t n = k == identity ? a.identity_rows : host_offsets[k + 1] - host_offsets[k];
+      const int64_t W = (n + per - 1) / per;  // fewer than 65,536: see wgrad_pairs_per_chunk
+      if (W >= 65536) return WCN_ERR_INVALID_ARGUMENT;
+      for (int x = 0; x < 8; ++x) here[x] += wgrad_first_chunk(x + 1, (int)W, k) - wgrad_first_chunk(x, (int)W, k);
+    }
+    for (int x = 0; x < 8; ++x) most = std::max(most, here[x]);
+    if (most > INT32_MAX / 8) return WCN_ERR_INVALID_ARGUMENT;
+    a.chunks = (int)most;
+    if (most <= room || turn == 16 || per >= (1 << 30)) break;
+    per = std::min<int64_t>((per + per / 24) / KP * KP + KP, 1 << 30);
   }
-  if (chunks > INT32_MAX) return WCN_ERR_INVALID_ARGUMENT;
-  a.chunks = (int)chunks;
+  a.pairs_per_chunk = (int)per;
   const int st = dtype == WCN_DTYPE_F16 ? launch_in<_Float16>(a, s) : launch_in<__bf16>(a, s);
   if (st != WCN_OK) return st;
   const dim3 grid((unsigned)((int64_t)num_offsets * (a.c_in_pad * a.c_out_pad / 256))), block(256);
