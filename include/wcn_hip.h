@@ -507,6 +507,16 @@ int wcn_sparse_conv_wgrad_mapped(const void* features, int64_t num_in, int32_t c
                                  int32_t identity_offset, void* grad_weight, int32_t weight_dtype,
                                  void* workspace, size_t workspace_bytes, void* stream);
 
+/* wcn_sparse_conv_wgrad_mapped and wcn_column_sums of grad_out (the gradient of a bias: c_out values of bias_dtype, with a workspace of
+ * wcn_column_sums_workspace_bytes(c_out)) in one call, the same results, which takes a launch less for 16-bit rows of
+ * whole 16-byte vectors. */
+int wcn_sparse_conv_wgrad_bias(const void* features, int64_t num_in, int32_t c_in, const void* grad_out, int64_t num_out,
+                               int32_t c_out, int32_t dtype, const int32_t* in_maps, const int32_t* out_maps,
+                               const int64_t* host_offsets, const int64_t* device_offsets_or_null, int32_t num_offsets,
+                               int32_t identity_offset, void* grad_weight, int32_t weight_dtype, void* workspace,
+                               size_t workspace_bytes, void* grad_bias, int32_t bias_dtype, void* bias_workspace,
+                               size_t bias_workspace_bytes, void* stream);
+
 /* ---------------------------------------------------------------------------------------------
  * Pooling over a kernel map.  Replaces the torch sort + torch_scatter.segment_csr reduction of
  * sparse_reduce (warpconvnet/nn/functional/sparse_pool.py:84-104, ops/reductions.py:38-56) and

@@ -110,6 +110,8 @@ SIGNATURES = {
     "wcn_conv_wgrad_workspace_bytes": (_sz, [_i32, _i32, _i32, _i64, _i64]),
     "wcn_sparse_conv_wgrad": (ctypes.c_int, [_vp, _i64, _i32, _vp, _i64, _i32, _i32, _vp, _vp, _i64p,
                                              _i32, _i32, _vp, _i32, _vp, _sz, _vp]),
+    "wcn_sparse_conv_wgrad_bias": (ctypes.c_int, [_vp, _i64, _i32, _vp, _i64, _i32, _i32, _vp, _vp, _i64p, _vp, _i32, _i32,
+                                                  _vp, _i32, _vp, _sz, _vp, _i32, _vp, _sz, _vp]),
     "wcn_sparse_conv_wgrad_mapped": (ctypes.c_int, [_vp, _i64, _i32, _vp, _i64, _i32, _i32, _vp, _vp, _i64p, _vp,
                                                     _i32, _i32, _vp, _i32, _vp, _sz, _vp]),
     "wcn_probe_gather_rows": (ctypes.c_int, [_vp, _i64, _i32, _vp, _i64, _vp, _vp]),

@@ -1,6 +1,7 @@
 // Column sums of a (rows, channels) array in fp32 (gfx950): the gradient of a layer's bias.
 #include <algorithm>
 
+#include "wcn_conv_args.h"
 #include "wcn_rows.h"
 
 namespace {
@@ -8,7 +9,6 @@ namespace {
 using namespace wcn_rows;
 
 constexpr int PARTS = 512;  // workgroups of the first pass: two per CU
-constexpr int FINISH = 8;   // partial sums in flight per thread of the second
 
 // A workgroup sums a stretch of rows, a thread per 16 bytes of channels, four rows in flight.  HBM-bound (5 TB/s): 500 k
 // rows of 64 fp16 channels (64 MB) in 12 + 4 us, where a generic column reduction took 34.
@@ -55,26 +55,8 @@ __global__ void __launch_bounds__(256) column_sums(const T* __restrict__ X, int6
 }
 
 template <typename OT>
-__global__ void __launch_bounds__(1024) column_sums_finish(const float* __restrict__ partial, int parts, int channels,
-                                                           OT* __restrict__ out) {
-  __shared__ float s_sum[16][64];
-  const int lane = threadIdx.x & 63, stretch = threadIdx.x >> 6;
-  const int c = blockIdx.x * 64 + lane;
-  float sum = 0.f;
-  if (c < channels) {
-    for (int p = stretch; p < parts; p += 16 * FINISH) {
-      float v[FINISH];
-#pragma unroll
-      for (int i = 0; i < FINISH; ++i) v[i] = p + 16 * i < parts ? partial[(int64_t)(p + 16 * i) * channels + c] : 0.f;
-#pragma unroll
-      for (int i = 0; i < FINISH; ++i) sum += v[i];
-    }
-  }
-  s_sum[stretch][lane] = sum;
-  __syncthreads();
-  if (stretch != 0 || c >= channels) return;
-  for (int p = 1; p < 16; ++p) sum += s_sum[p][lane];
-  out[c] = from_float<OT>(sum);
+__global__ void __launch_bounds__(256) column_sums_finish(WcnColumnSums s) {
+  wcn_column_sums_finish<OT>(s, (int)blockIdx.x * 16, (OT*)s.out);
 }
 
 inline int column_parts(int64_t n, int rows) {  // at least four rows per thread in a part
@@ -82,6 +64,30 @@ inline int column_parts(int64_t n, int rows) {  // at least four rows per thread
 }
 
 }  // namespace
+
+int wcn_column_sums_first(const void* rows, int64_t num_rows, int dtype, WcnColumnSums* c, hipStream_t s) {
+  const RowTiling t = row_tiling(c->channels, dtype);
+  const bool vec = rows_are_vectors(rows, c->channels, dtype);
+  c->parts = column_parts(num_rows, t.rows);
+  const int64_t per = (num_rows + c->parts - 1) / c->parts;
+  auto first = [&](auto v) {
+    using T = decltype(v);
+    hipLaunchKernelGGL((vec ? column_sums<T, true> : column_sums<T, false>), dim3((unsigned)c->parts), dim3(256), 0, s,
+                       (const T*)rows, num_rows, c->channels, t, per, c->partial);
+  };
+  if (dtype == WCN_DTYPE_F32) first(float{}); else if (dtype == WCN_DTYPE_F16) first(_Float16{}); else first(__bf16{});
+  WCN_LAUNCH_CHECK();
+  return WCN_OK;
+}
+
+int wcn_column_sums_second(const WcnColumnSums& c, hipStream_t s) {
+  const dim3 grid((unsigned)((c.channels + 15) / 16)), block(256);
+  if (c.out_dtype == WCN_DTYPE_F32) hipLaunchKernelGGL(column_sums_finish<float>, grid, block, 0, s, c);
+  else if (c.out_dtype == WCN_DTYPE_F16) hipLaunchKernelGGL(column_sums_finish<_Float16>, grid, block, 0, s, c);
+  else hipLaunchKernelGGL(column_sums_finish<__bf16>, grid, block, 0, s, c);
+  WCN_LAUNCH_CHECK();
+  return WCN_OK;
+}
 
 extern "C" {
 
@@ -95,26 +101,9 @@ int wcn_column_sums(const void* rows, int64_t num_rows, int32_t channels, int32_
       (num_rows > 0 && !rows))
     return WCN_ERR_INVALID_ARGUMENT;
   if (workspace_bytes < wcn_column_sums_workspace_bytes(channels)) return WCN_ERR_WORKSPACE;
-  hipStream_t s = (hipStream_t)stream;
-  float* partial = (float*)workspace;
-  const RowTiling t = row_tiling(channels, dtype);
-  const bool vec = rows_are_vectors(rows, channels, dtype);
-  const int parts = column_parts(num_rows, t.rows);
-  const int64_t per = (num_rows + parts - 1) / parts;
-  auto first = [&](auto v) {
-    using T = decltype(v);
-    hipLaunchKernelGGL((vec ? column_sums<T, true> : column_sums<T, false>), dim3((unsigned)parts), dim3(256), 0, s, (const T*)rows, num_rows, channels, t, per,
-                       partial);
-  };
-  auto second = [&](auto v) {
-    using OT = decltype(v);
-    hipLaunchKernelGGL(column_sums_finish<OT>, dim3((unsigned)((channels + 63) / 64)), dim3(1024), 0, s,
-                       (const float*)partial, parts, channels, (OT*)out);
-  };
-  if (dtype == WCN_DTYPE_F32) first(float{}); else if (dtype == WCN_DTYPE_F16) first(_Float16{}); else first(__bf16{});
-  if (out_dtype == WCN_DTYPE_F32) second(float{}); else if (out_dtype == WCN_DTYPE_F16) second(_Float16{}); else second(__bf16{});
-  WCN_LAUNCH_CHECK();
-  return WCN_OK;
+  WcnColumnSums c = {(float*)workspace, 0, channels, out, out_dtype};
+  const int st = wcn_column_sums_first(rows, num_rows, dtype, &c, (hipStream_t)stream);
+  return st != WCN_OK ? st : wcn_column_sums_second(c, (hipStream_t)stream);
 }
 
 }  // extern "C"

@@ -70,6 +70,43 @@ struct WcnSingleTiles {  // tiles of 256 pairs of one offset, in offset order
 bool wcn_conv_single_takes(int dtype, int c_in, int c_out, int num_offsets);
 int wcn_conv_single_launch(const ConvArgs& a, int dtype, const int64_t* host_offsets, hipStream_t stream);
 
+// Column sums of a (rows, channels) array: the first pass, `parts` fp32 partial sums per channel, and what the second is to do
+// with them (wcn_colsum.hip; the gradient of a bias).
+struct WcnColumnSums {
+  float* partial;  // (parts, channels)
+  int32_t parts, channels;
+  void* out;
+  int32_t out_dtype;
+};
+int wcn_column_sums_first(const void* rows, int64_t num_rows, int dtype, WcnColumnSums* c, hipStream_t stream);  // sets parts
+int wcn_column_sums_second(const WcnColumnSums& c, hipStream_t stream);
+
+#ifdef __HIPCC__
+// The second pass by 256 threads for 16 channels from c0 on: parts p, p + 16, ... to thread p / 16, eight in flight, their
+// sixteen sums added in order.
+template <typename OT>
+__device__ __forceinline__ void wcn_column_sums_finish(const WcnColumnSums& s, int c0, OT* out) {
+  __shared__ float s_sum[16][16];
+  constexpr int AHEAD = 8;
+  const int at = threadIdx.x & 15, stretch = threadIdx.x >> 4, c = c0 + at;
+  float sum = 0.f;
+  if (c < s.channels) {
+    for (int p = stretch; p < s.parts; p += 16 * AHEAD) {
+      float v[AHEAD];
+#pragma unroll
+      for (int i = 0; i < AHEAD; ++i) v[i] = p + 16 * i < s.parts ? s.partial[(int64_t)(p + 16 * i) * s.channels + c] : 0.f;
+#pragma unroll
+      for (int i = 0; i < AHEAD; ++i) sum += v[i];
+    }
+  }
+  s_sum[stretch][at] = sum;
+  __syncthreads();
+  if (stretch != 0 || c >= s.channels) return;
+  for (int p = 1; p < 16; ++p) sum += s_sum[p][at];
+  out[c] = (OT)sum;
+}
+#endif
+
 // The weight gradient of 16-bit rows of whole vectors (wcn_conv_wgrad.hip): whether it takes a problem, the bytes of its
 // partial sums (pairs with the identity's rows), and its launch.
 bool wcn_wgrad_tiles_takes(int dtype, int c_in, int c_out, const void* features, const void* grad_out);
@@ -77,7 +114,7 @@ size_t wcn_wgrad_tiles_partial_bytes(int num_offsets, int c_in, int c_out, int64
 int wcn_wgrad_tiles_launch(const void* features, int64_t num_in, int c_in, const void* grad_out, int64_t num_out, int c_out,
                            int dtype, const int32_t* in_maps, const int32_t* out_maps, const int64_t* host_offsets,
                            const int64_t* device_offsets, int num_offsets, int identity, void* grad_weight,
-                           int weight_dtype, float* partial, hipStream_t stream);
+                           int weight_dtype, float* partial, const WcnColumnSums* columns_or_null, hipStream_t stream);
 
 #endif  // WCN_CONV_ARGS_H_
 

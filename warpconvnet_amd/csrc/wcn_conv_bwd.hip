@@ -340,12 +340,12 @@ size_t wcn_conv_wgrad_workspace_bytes(int32_t num_offsets, int32_t c_in, int32_t
   return wgrad_layout(nullptr, num_offsets, c_in, c_out, num_pairs + identity_rows, nullptr);
 }
 
-int wcn_sparse_conv_wgrad_mapped(const void* features, int64_t num_in, int32_t c_in, const void* grad_out,
+static int wgrad_run(const void* features, int64_t num_in, int32_t c_in, const void* grad_out,
                           int64_t num_out, int32_t c_out, int32_t dtype, const int32_t* in_maps,
                           const int32_t* out_maps, const int64_t* host_offsets,
                           const int64_t* device_offsets_or_null, int32_t num_offsets, int32_t identity_offset, void* grad_weight,
                           int32_t weight_dtype, void* workspace, size_t workspace_bytes,
-                          void* stream) {
+                          const WcnColumnSums* columns, void* stream) {
   if (dtype < 0 || dtype > 2 || (weight_dtype != dtype && weight_dtype != WCN_DTYPE_F32))
     return WCN_ERR_INVALID_ARGUMENT;
   if (num_in < 0 || num_out < 0 || num_offsets < 1 || num_offsets > WCN_MAX_OFFSETS || c_in < 1 ||
@@ -371,7 +371,7 @@ int wcn_sparse_conv_wgrad_mapped(const void* features, int64_t num_in, int32_t c
     return WCN_ERR_LAUNCH;
   if (wcn_wgrad_tiles_takes(dtype, c_in, c_out, features, grad_out))
     return wcn_wgrad_tiles_launch(features, num_in, c_in, grad_out, num_out, c_out, dtype, in_maps, out_maps, host_offsets,
-                                  w.offsets, num_offsets, identity_offset, grad_weight, weight_dtype, w.partial, s);
+                                  w.offsets, num_offsets, identity_offset, grad_weight, weight_dtype, w.partial, columns, s);
   const int ppc = (int)plan_pairs_per_chunk(L + identity_rows, c_in, c_out);
   int64_t chunks = 0;  // the device computes the same numbers from the same inputs
   for (int k = 0; k < num_offsets; ++k) {
@@ -428,6 +428,37 @@ int wcn_sparse_conv_wgrad_mapped(const void* features, int64_t num_in, int32_t c
   }
   WCN_LAUNCH_CHECK();
   return WCN_OK;
+}
+
+int wcn_sparse_conv_wgrad_mapped(const void* features, int64_t num_in, int32_t c_in, const void* grad_out,
+                          int64_t num_out, int32_t c_out, int32_t dtype, const int32_t* in_maps,
+                          const int32_t* out_maps, const int64_t* host_offsets,
+                          const int64_t* device_offsets_or_null, int32_t num_offsets, int32_t identity_offset, void* grad_weight,
+                          int32_t weight_dtype, void* workspace, size_t workspace_bytes,
+                          void* stream) {
+  return wgrad_run(features, num_in, c_in, grad_out, num_out, c_out, dtype, in_maps, out_maps, host_offsets,
+                   device_offsets_or_null, num_offsets, identity_offset, grad_weight, weight_dtype, workspace, workspace_bytes,
+                   nullptr, stream);
+}
+
+int wcn_sparse_conv_wgrad_bias(const void* features, int64_t num_in, int32_t c_in, const void* grad_out, int64_t num_out,
+                               int32_t c_out, int32_t dtype, const int32_t* in_maps, const int32_t* out_maps,
+                               const int64_t* host_offsets, const int64_t* device_offsets_or_null, int32_t num_offsets,
+                               int32_t identity_offset, void* grad_weight, int32_t weight_dtype, void* workspace,
+                               size_t workspace_bytes, void* grad_bias, int32_t bias_dtype, void* bias_workspace,
+                               size_t bias_workspace_bytes, void* stream) {
+  if (!grad_bias || !bias_workspace || bias_dtype < 0 || bias_dtype > 2 || dtype < 0 || dtype > 2 || c_out < 1 || num_out < 0 ||
+      (num_out > 0 && !grad_out))
+    return WCN_ERR_INVALID_ARGUMENT;
+  if (bias_workspace_bytes < wcn_column_sums_workspace_bytes(c_out)) return WCN_ERR_WORKSPACE;
+  const bool joined = c_in >= 1 && wcn_wgrad_tiles_takes(dtype, c_in, c_out, features, grad_out);
+  WcnColumnSums c = {(float*)bias_workspace, 0, c_out, grad_bias, bias_dtype};
+  int st = wcn_column_sums_first(grad_out, num_out, dtype, &c, (hipStream_t)stream);
+  if (st != WCN_OK) return st;
+  st = wgrad_run(features, num_in, c_in, grad_out, num_out, c_out, dtype, in_maps, out_maps, host_offsets,
+                 device_offsets_or_null, num_offsets, identity_offset, grad_weight, weight_dtype, workspace, workspace_bytes,
+                 joined ? &c : nullptr, stream);
+  return st != WCN_OK || joined ? st : wcn_column_sums_second(c, (hipStream_t)stream);
 }
 
 int wcn_sparse_conv_wgrad(const void* features, int64_t num_in, int32_t c_in, const void* grad_out,

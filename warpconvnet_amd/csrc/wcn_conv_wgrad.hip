@@ -238,9 +238,18 @@ __global__ void __launch_bounds__(256, 2) conv_wgrad_tiles(WgradTileArgs a) {
 
 // dW[k] = the offset's chunks added up, rounded once: a workgroup owns 256 consecutive values of the padded plane, its
 // waves the chunks c = j, j + 4, ..., eight loads in flight, combined as (0 + 1) + (2 + 3).
+// Workgroups behind those (`columns.parts` > 0) finish the bias's gradient, which would be a launch of its own (4.6 us over 96
+// channels).
 template <typename WT>
-__global__ void __launch_bounds__(256) wgrad_tiles_reduce(WgradTileArgs a, WT* __restrict__ dW) {
+__global__ void __launch_bounds__(256) wgrad_tiles_reduce(WgradTileArgs a, WT* __restrict__ dW, int planes, WcnColumnSums columns) {
   __shared__ f32x4 part[4][64];
+  if ((int)blockIdx.x >= planes) {
+    const int c0 = ((int)blockIdx.x - planes) * 16;
+    if (columns.out_dtype == WCN_DTYPE_F32) wcn_column_sums_finish(columns, c0, (float*)columns.out);
+    else if (columns.out_dtype == WCN_DTYPE_F16) wcn_column_sums_finish(columns, c0, (_Float16*)columns.out);
+    else wcn_column_sums_finish(columns, c0, (__bf16*)columns.out);
+    return;
+  }
   const int plane = a.c_in_pad * a.c_out_pad, slices = plane / 256;
   const int k = blockIdx.x / slices, slice = blockIdx.x % slices;
   const int j = threadIdx.x >> 6, e = threadIdx.x & 63;
@@ -345,7 +354,7 @@ size_t wcn_wgrad_tiles_partial_bytes(int num_offsets, int c_in, int c_out, int64
 int wcn_wgrad_tiles_launch(const void* features, int64_t num_in, int c_in, const void* grad_out, int64_t num_out, int c_out,
                            int dtype, const int32_t* in_maps, const int32_t* out_maps, const int64_t* host_offsets,
                            const int64_t* device_offsets, int num_offsets, int identity, void* grad_weight,
-                           int weight_dtype, float* partial, hipStream_t s) {
+                           int weight_dtype, float* partial, const WcnColumnSums* columns, hipStream_t s) {
   WgradTileArgs a;
   a.X = features;
   a.dY = grad_out;
@@ -384,13 +393,15 @@ int wcn_wgrad_tiles_launch(const void* features, int64_t num_in, int c_in, const
   a.pairs_per_chunk = (int)per;
   const int st = dtype == WCN_DTYPE_F16 ? launch_in<_Float16>(a, s) : launch_in<__bf16>(a, s);
   if (st != WCN_OK) return st;
-  const dim3 grid((unsigned)((int64_t)num_offsets * (a.c_in_pad * a.c_out_pad / 256))), block(256);
+  const int planes = num_offsets * (a.c_in_pad * a.c_out_pad / 256);
+  const WcnColumnSums sums = columns ? *columns : WcnColumnSums{};
+  const dim3 grid((unsigned)(planes + (sums.channels + 15) / 16)), block(256);
   if (weight_dtype == WCN_DTYPE_F32)
-    hipLaunchKernelGGL(wgrad_tiles_reduce<float>, grid, block, 0, s, a, (float*)grad_weight);
+    hipLaunchKernelGGL(wgrad_tiles_reduce<float>, grid, block, 0, s, a, (float*)grad_weight, planes, sums);
   else if (dtype == WCN_DTYPE_F16)
-    hipLaunchKernelGGL(wgrad_tiles_reduce<_Float16>, grid, block, 0, s, a, (_Float16*)grad_weight);
+    hipLaunchKernelGGL(wgrad_tiles_reduce<_Float16>, grid, block, 0, s, a, (_Float16*)grad_weight, planes, sums);
   else
-    hipLaunchKernelGGL(wgrad_tiles_reduce<__bf16>, grid, block, 0, s, a, (__bf16*)grad_weight);
+    hipLaunchKernelGGL(wgrad_tiles_reduce<__bf16>, grid, block, 0, s, a, (__bf16*)grad_weight, planes, sums);
   WCN_LAUNCH_CHECK();
   return WCN_OK;
 }

@@ -700,10 +700,12 @@ struct GradMap {
 };
 
 /* (dX or undefined, dW or undefined), see sparse_conv_backward.  sorted(): the lists ascending in
- * input row, asked for only where the map needs re-ordering. */
+ * input row, asked for only where the map needs re-ordering.  `grad_bias`: filled with the sums of grad_output's rows
+ * (which are then of the features' type) beside dW. */
 template <typename F>
 std::pair<Tensor, Tensor> backward(const Tensor& grad_output, const Tensor& in_features, const Tensor& weight,
-                                   const GradMap& g, at::ScalarType dtype, bool need_x, bool need_w, const F& sorted) {
+                                   const GradMap& g, at::ScalarType dtype, bool need_x, bool need_w, const F& sorted,
+                                   Tensor* grad_bias = nullptr) {
   const int code = dtype_code(dtype);
   const int32_t K = g.map.K, c_in = static_cast<int32_t>(weight.size(1)), c_out = static_cast<int32_t>(weight.size(2));
   const Tensor x = in_features.to(dtype).contiguous(), gy = grad_output.to(dtype).contiguous();
@@ -753,12 +755,23 @@ std::pair<Tensor, Tensor> backward(const Tensor& grad_output, const Tensor& in_f
     grad_w = at::empty({K, c_in, c_out}, w.options());
     const int64_t identity_rows = iden >= 0 ? std::min(n_in, n_out) : 0;
     Tensor ws = bytes_on(wcn_conv_wgrad_workspace_bytes(K, c_in, c_out, pairs, identity_rows), x);
-    check(wcn_sparse_conv_wgrad_mapped(x.const_data_ptr(), n_in, c_in, pgy, n_out, c_out, code,
-                                g.map.in_maps.const_data_ptr<int32_t>(), g.map.out_maps.const_data_ptr<int32_t>(),
-                                g.map.host_offsets(),
-                                g.device_offsets.defined() ? g.device_offsets.const_data_ptr<int64_t>() : nullptr, K, iden, grad_w.mutable_data_ptr(), wcode, ws.mutable_data_ptr(),
-                                static_cast<size_t>(ws.numel()), stream),
-          "wcn_sparse_conv_wgrad");
+    const int64_t* device_offsets = g.device_offsets.defined() ? g.device_offsets.const_data_ptr<int64_t>() : nullptr;
+    const int32_t *in_maps = g.map.in_maps.const_data_ptr<int32_t>(), *out_maps = g.map.out_maps.const_data_ptr<int32_t>();
+    const size_t nbytes = static_cast<size_t>(ws.numel());
+    if (grad_bias) {
+      Tensor sums = bytes_on(wcn_column_sums_workspace_bytes(c_out), x);
+      check(wcn_sparse_conv_wgrad_bias(x.const_data_ptr(), n_in, c_in, pgy, n_out, c_out, code, in_maps, out_maps,
+                                       g.map.host_offsets(), device_offsets, K, iden, grad_w.mutable_data_ptr(), wcode,
+                                       ws.mutable_data_ptr(), nbytes, grad_bias->mutable_data_ptr(),
+                                       dtype_code(grad_bias->scalar_type()), sums.mutable_data_ptr(),
+                                       static_cast<size_t>(sums.numel()), stream),
+            "wcn_sparse_conv_wgrad_bias");
+    } else {
+      check(wcn_sparse_conv_wgrad_mapped(x.const_data_ptr(), n_in, c_in, pgy, n_out, c_out, code, in_maps, out_maps,
+                                         g.map.host_offsets(), device_offsets, K, iden, grad_w.mutable_data_ptr(), wcode,
+                                         ws.mutable_data_ptr(), nbytes, stream),
+            "wcn_sparse_conv_wgrad");
+    }
     grad_w = grad_w.to(weight.scalar_type());
   }
   return {grad_x, grad_w};
@@ -822,15 +835,18 @@ struct ConvBackward : public torch::autograd::Node {
     const Tensor x = x_.unpack(shared_from_this()), w = w_.unpack(shared_from_this());
     at::NoGradGuard no_grad;
     const bool need_x = task_should_compute_output(0), need_w = task_should_compute_output(1);
+    const bool need_b = has_bias_ && task_should_compute_output(2);
+    const bool joined = need_b && need_w && grads[0].scalar_type() == dtype_ && dtype_code(bias_dtype_) >= 0;
+    if (joined) out[2] = at::empty({grads[0].size(1)}, grads[0].options().dtype(bias_dtype_));
     if (need_x || need_w) {
       auto r = backward(grads[0], x, w, *map_, dtype_, need_x, need_w, [&]() {
         py::gil_scoped_acquire locked;
         return sorted_by_in(km_->o, sorted_->o, x.size(0));
-      });
+      }, joined ? &out[2] : nullptr);
       out[0] = r.first;
       out[1] = r.second;
     }
-    if (has_bias_ && task_should_compute_output(2)) out[2] = column_sums(grads[0], bias_dtype_);
+    if (need_b && !joined) out[2] = column_sums(grads[0], bias_dtype_);
     return out;
   }
   void release_variables() override {
