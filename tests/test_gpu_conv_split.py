@@ -95,3 +95,35 @@ def test_kept_tiles_are_those_that_are_read():
         del kept
     assert [small for small, _ in seen] == [True, False, True, False]
     assert [bytes_ for _, bytes_ in seen] == [half, half, 0, 0]
+
+
+# (dtype, C_in, C_out, rows, instance): sixteen, thirty-two or sixty-four channels a tile, as long as every tile has one of the 256 CUs,
+# and eight or sixteen waves (from 100 units on)
+_TILES = [(torch.bfloat16, 32, 32, 4096, "1, 8"), (torch.bfloat16, 32, 32, 4097, "2, 8"), (torch.bfloat16, 64, 64, 2080, "2, 8"),
+          (torch.float16, 128, 128, 1024, "1, 16"), (torch.float16, 128, 128, 1025, "2, 16"),
+          (torch.float16, 128, 128, 2049, "4, 16"), (torch.float16, 120, 100, 4097, "4, 8"),
+          (torch.float32, 64, 40, 2048, "1, 16"), (torch.float32, 64, 72, 2049, "2, 16"), (torch.float32, 16, 20, 60, "1, 8"),
+          (torch.float32, 64, 64, 4097, "4, 8")]
+
+
+@pytest.mark.parametrize("infinite", [False, True], ids=["finite", "infinite_weight"])
+@pytest.mark.parametrize("dtype,c_in,c_out,rows,tile", _TILES, ids=[f"{t[1]}_{t[2]}_{t[3]}_{t[4].replace(', ', 'x')}" for t in _TILES])
+def test_tiles_get_wider_when_the_cus_are_taken(oracle, dtype, c_in, c_out, rows, tile, infinite):
+    from warpconvnet_amd._lib import lib
+    from warpconvnet_amd.geometry.coords.search.torch_discrete import generate_kernel_map
+    from warpconvnet_amd.nn.functional.sparse_conv import sparse_conv_forward
+    bc = synthetic.random_cloud(11, 2 * rows, max(8, int(round((3 * rows) ** (1 / 3)))))[:rows]
+    assert len(bc) == rows
+    c = torch.as_tensor(np.ascontiguousarray(bc), device=DEV)
+    km = generate_kernel_map(c, c, (1, 1, 1), (3, 3, 3))
+    x, w = normal_features(rows, c_in, seed=6, dtype=dtype), kaiming_weight(27, c_in, c_out, seed=7, dtype=dtype)
+    if infinite:
+        w[2, 3, 7], w[20, 5, 9] = float("inf"), float("nan")
+    im, om, off, iden = oracle.kernel_map(bc, bc, (3, 3, 3))
+    with np.errstate(invalid="ignore"):
+        want = oracle.explicit_conv_f64(x.double().numpy(), w.double().numpy(), im, om, off, iden, rows)
+    got = sparse_conv_forward(x.to(DEV), w.to(DEV), km, rows).double().cpu().numpy()
+    text = {torch.bfloat16: "bf16", torch.float16: "f16", torch.float32: "float"}[dtype]
+    assert lib().wcn_conv_last_kernel().decode() == f"conv_fwd_small<{text}, {tile}>"
+    assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(got[np.isinf(want)], want[np.isinf(want)])
+    assert rel_err(np.where(np.isfinite(want), got, 0.0), np.where(np.isfinite(want), want, 0.0)) <= TOL[dtype]
