@@ -625,6 +625,14 @@ int wcn_sparse_depthwise_wgrad_grouped(const void* features, int64_t num_in, con
                                        int32_t weight_dtype, void* workspace, size_t workspace_bytes,
                                        void* stream);
 
+/* The convolution of one voxel: out = rows @ weight + bias, (num_rows, c_out) of the rows' type (16-bit), fp32 sums, one
+ * rounding.  weight: (c_in, c_out) of the rows' type, as stored; all pointers 16-byte aligned, rows dense.
+ * wcn_pointwise_takes: whether the call is one the kernel is made for (WCN_ERR_INVALID_ARGUMENT otherwise). */
+int32_t wcn_pointwise_takes(int64_t num_rows, int32_t c_in, int32_t c_out, int32_t dtype);
+
+int wcn_pointwise_fwd(const void* rows, int64_t num_rows, int32_t c_in, int32_t dtype, const void* weight, int32_t c_out,
+                      const void* bias_or_null, void* out, void* stream);
+
 /* out[c] = sum over the rows of rows[., c], in fp32, rounded once to out_dtype: the gradient of a bias. */
 size_t wcn_column_sums_workspace_bytes(int32_t channels);
 

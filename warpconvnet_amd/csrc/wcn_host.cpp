@@ -10,6 +10,9 @@
 #include <torch/csrc/autograd/function.h>
 #include <torch/csrc/autograd/functions/utils.h>
 #include <torch/csrc/autograd/saved_variable.h>
+#include <ATen/PythonTorchFunctionTLS.h>
+#include <ATen/autocast_mode.h>
+#include <c10/core/DeviceGuard.h>
 #include <c10/core/impl/VirtualGuardImpl.h>
 #include <c10/hip/HIPStream.h>
 #include <hip/hip_runtime_api.h>
@@ -641,6 +644,42 @@ Tensor conv_forward(const Tensor& features, const py::object& weight_obj, const 
   return finish();
 }
 
+bool in_graph(std::initializer_list<const Tensor*> tensors);
+
+/* Whether a tensor is plain device memory of this call's: no wrapper of a transform, a mode or a subclass. */
+bool plain_rows(const Tensor& t) {
+  const c10::DispatchKeySet keys = t.key_set() - c10::autograd_dispatch_keyset_with_ADInplaceOrView - c10::autocast_dispatch_keyset;
+  return keys == c10::DispatchKeySet(c10::DispatchKey::CUDA) && t.is_contiguous() && aligned16(t.const_data_ptr()) && !has_tangent(t);
+}
+
+/* The layer of one voxel and stride 1, outside any graph: features @ weight[0] + bias, or an undefined tensor where torch is to
+ * compute it: a call of another kind, or one that a transform, a trace or a mode has to see. */
+Tensor pointwise_forward(const Tensor& features, const Tensor& weight, const std::optional<Tensor>& bias) {
+  using c10::DispatchKey;
+  if (in_graph({&features, &weight, bias ? &*bias : &features}) || at::autocast::is_autocast_enabled(at::kCUDA)) return Tensor();
+  for (const DispatchKey key : {DispatchKey::Tracer, DispatchKey::FuncTorchDynamicLayerFrontMode, DispatchKey::Python,
+                                DispatchKey::PythonDispatcher, DispatchKey::Functionalize})
+    if (c10::impl::tls_is_dispatch_key_included(key)) return Tensor();
+  if (at::impl::torch_function_mode_enabled()) return Tensor();
+  const int code = dtype_code(features.scalar_type());
+  if (features.dim() != 2 || weight.dim() != 3 || weight.size(0) != 1 || weight.size(1) != features.size(1) ||
+      weight.scalar_type() != features.scalar_type() || weight.device() != features.device() || !plain_rows(features) ||
+      !plain_rows(weight))
+    return Tensor();
+  if (weight.size(1) > INT32_MAX || weight.size(2) > INT32_MAX) return Tensor();
+  const int32_t c_in = static_cast<int32_t>(weight.size(1)), c_out = static_cast<int32_t>(weight.size(2));
+  if (!wcn_pointwise_takes(features.size(0), c_in, c_out, code)) return Tensor();
+  const bool has_bias = bias && bias->defined();
+  if (has_bias && (!kernel_bias(*bias, features, c_out) || bias->scalar_type() != features.scalar_type() || !plain_rows(*bias)))
+    return Tensor();
+  const c10::DeviceGuard device(features.device());
+  Tensor out = at::empty({features.size(0), c_out}, features.options());
+  check(wcn_pointwise_fwd(features.const_data_ptr(), features.size(0), c_in, code, weight.const_data_ptr(), c_out,
+                          has_bias ? bias->const_data_ptr() : nullptr, out.mutable_data_ptr(), stream_of(features)),
+        "wcn_pointwise_fwd");
+  return out;
+}
+
 /* Sums over the rows, in fp32: the gradient of a bias. */
 Tensor column_sums(const Tensor& rows, at::ScalarType out_dtype) {
   if (dtype_code(out_dtype) < 0 || dtype_code(rows.scalar_type()) < 0) return rows.sum(0, false, out_dtype);
@@ -1217,6 +1256,10 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
                            const std::optional<Tensor>& bias, const std::optional<at::ScalarType>& compute_dtype,
                            const std::optional<Tensor>& residual, bool relu, bool keep_tiles, const py::object& pairs_sorted) {
     return conv_forward(features, weight, km, num_out, bias, compute_dtype, residual, relu, keep_tiles, pairs_sorted, false);
+  });
+  m.def("pointwise_forward", [](const Tensor& features, const Tensor& weight, const std::optional<Tensor>& bias) -> py::object {
+    const Tensor out = pointwise_forward(features, weight, bias);
+    return out.defined() ? py::cast(out) : py::none();
   });
   m.def("conv_backward", &conv_backward);
   m.def("conv_autograd", &conv_autograd);

@@ -406,7 +406,13 @@ def spatially_sparse_conv(
 
     if math.prod(_kernel_size) == 1 and math.prod(_stride) == 1:
         features = input_sparse_tensor.feature_tensor
-        if bias is not None:  # one library call, one rounding
+        out_features = None
+        if type(features) is Tensor and type(weight) in (Tensor, torch.nn.Parameter) and features.is_cuda \
+                and not torch.compiler.is_compiling():
+            out_features = native().pointwise_forward(features, weight, bias)
+        if out_features is not None:
+            pass
+        elif bias is not None:  # one library call, one rounding
             out_features = torch.addmm(bias.to(features.dtype), features, weight[0])
         else:
             out_features = features @ weight[0]
