@@ -62,7 +62,7 @@ int wcn_conv_tiles_launch(const ConvArgs& a, int dtype, const WcnTilePlan& plan,
 // takes a problem's shape, and its launch over pair lists in any order (`host_offsets`: the K + 1
 // offsets; X, Wt, bias, residual, relu, out, the lists and the sizes are read from `a`).
 constexpr int WCN_SINGLE_MAX_OFFSETS = 64;
-struct WcnSingleTiles {  // tiles of 256 pairs of one offset, in offset order
+struct WcnSingleTiles {  // tiles of 64 to 256 pairs of one offset, in offset order
   int32_t first_tile[WCN_SINGLE_MAX_OFFSETS + 1];
   int32_t first_pair[WCN_SINGLE_MAX_OFFSETS + 1];
   int32_t total;

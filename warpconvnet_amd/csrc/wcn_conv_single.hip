@@ -6,13 +6,18 @@
 //
 // Nothing is accumulated across pairs, so there are no sums to keep anywhere, no phases and no order
 // the pairs of an offset have to be in: the lists are taken as they are (a forward map with its
-// lists exchanged is not re-ordered first), cut into tiles of 256 pairs of one offset.  A workgroup
+// lists exchanged is not re-ordered first), cut into tiles of 64 to 256 pairs of one offset.  A workgroup
 // of four waves walks a contiguous stretch of tiles with W[k]^T of the current offset in LDS (loaded
-// again when the offset changes); a wave takes 64 pairs as four blocks of 16.  The product is
-// transposed: W[k]^T is the A operand (rows = output channels, read from LDS), the gathered rows
+// again when the offset changes); a wave takes one to four blocks of 16 pairs, whose list entries it has asked for a tile
+// ahead.  The product is transposed: W[k]^T is the A operand (rows = output channels, read from LDS), the gathered rows
 // are the B operand and go from memory straight into registers in operand layout (lane = pair,
-// 8 channels), so a lane ends up with 4 consecutive output channels of one pair and stores them
-// with one 8-byte store.  Output channels are walked 64 at a time with the gathered rows kept.
+// 8 channels), so a lane ends up with 4 consecutive output channels of one pair in each of two 16-channel blocks;
+// neighbouring quarters of the wave exchange halves and store 16 bytes.  Output channels are walked 32 at a time with the
+// gathered rows kept.
+// What bounds it: the way of a wave's rows and stores through memory, so the number of waves in flight: 128 registers and fewer
+// leave four a SIMD (64 channels at a time with four blocks of rows took 130 to 244: one to three).  bf16, kernel and stride 2, us:
+// 32 -> 32 over 1,000,000 fine rows 52 -> 41, 64 -> 32 over 550,000 40 -> 25, 128 -> 64 over 130,000 24 -> 18; over the
+// levels of one scan of 60,000 voxels (where smaller tiles make more workgroups) 256 -> 128 23 -> 13, 128 -> 64 12 -> 8.
 // Replaces the same reference path as the other kernels (sparse_conv.py:495-544 + the native GEMMs
 // it calls) for this kind of map.
 #include <algorithm>
@@ -26,34 +31,61 @@ namespace {
 
 using namespace wcn_mma;
 
-constexpr int SINGLE_WAVES = 4, SINGLE_BPW = 4;               // waves per workgroup, 16-pair blocks per wave
-constexpr int SINGLE_TILE = SINGLE_WAVES * SINGLE_BPW * 16;   // pairs per tile
+constexpr int SINGLE_WAVES = 4;
+// 16-pair blocks of a wave: what leaves four waves a SIMD (128 registers)
+constexpr int single_bpw(int ks) { return ks <= 2 ? 4 : ks <= 4 ? 2 : 1; }
+constexpr int single_tile(int ks) { return SINGLE_WAVES * single_bpw(ks) * 16; }  // pairs per tile
 
 // KS: 32-channel steps of the gathered rows (c_in = 32 KS)
 template <typename T, int KS>
-__global__ void __launch_bounds__(SINGLE_WAVES * 64) conv_fwd_single(ConvArgs a, WcnSingleTiles tt) {
+__global__ void __launch_bounds__(SINGLE_WAVES * 64, 4) conv_fwd_single(ConvArgs a, WcnSingleTiles tt) {
   typedef typename Mma<T>::V V;
   extern __shared__ __attribute__((aligned(16))) unsigned char single_smem[];
+  constexpr int BPW = single_bpw(KS), TILE = single_tile(KS);
   constexpr int ROW_BYTES = KS * 64 + 16;  // a row of W[k]^T (c_in values) plus 16 bytes: the operand reads of
                                            // 16 consecutive rows then fall into distinct banks
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int p = lane & 15, kg = lane >> 4;
   const int ncb = (a.c_out + 15) / 16;     // 16-channel blocks of output channels
-  const int wrows = ncb * 16;              // rows of W[k]^T that are used (the tiles are zero padded beyond c_out)
+  const int npairs = (ncb + 1) / 2;        // pairs of them
   const T* __restrict__ X = (const T*)a.X;
   const T* __restrict__ Wt = (const T*)a.Wt;
   T* __restrict__ out = (T*)a.out;
   const int per_wg = (tt.total + (int)gridDim.x - 1) / (int)gridDim.x;
   const int t_begin = (int)blockIdx.x * per_wg;
   const int t_end = t_begin + per_wg < tt.total ? t_begin + per_wg : tt.total;
+  if (t_begin >= t_end) return;  // (the whole workgroup)
+  // the entries of this lane's pairs of a tile in offset `of`; a place without a pair: -1
+  auto entries = [&](int tile, int of, int32_t (&irow)[BPW], int32_t (&orow)[BPW]) {
+    const int run_end = tt.first_pair[of + 1];
+    const int p0 = tt.first_pair[of] + (tile - tt.first_tile[of]) * TILE + wave * (BPW * 16) + p;
+#pragma unroll
+    for (int b = 0; b < BPW; ++b) {
+      const bool live = p0 + b * 16 < run_end;
+      irow[b] = live ? a.in_maps[p0 + b * 16] : -1;
+      orow[b] = live ? a.out_maps[p0 + b * 16] : -1;
+    }
+  };
   int k = 0, loaded = -1;
+  while (k + 1 < a.K && t_begin >= tt.first_tile[k + 1]) ++k;  // tiles ascend in offset
+  int32_t irow[BPW], orow[BPW];
+  entries(t_begin, k, irow, orow);
   for (int tile = t_begin; tile < t_end; ++tile) {
-    while (k + 1 < a.K && tile >= tt.first_tile[k + 1]) ++k;  // tiles ascend in offset
+    // the wave's rows, in MFMA operand layout
+    V B[BPW][KS];
+#pragma unroll
+    for (int b = 0; b < BPW; ++b) {
+      const bool ok = (uint32_t)irow[b] < (uint64_t)a.num_in && (uint32_t)orow[b] < (uint64_t)a.num_out;
+      if (!ok) orow[b] = -1;
+      const T* row = X + (int64_t)(ok ? irow[b] : 0) * a.c_in + kg * 8;
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) B[b][ks] = *reinterpret_cast<const V*>(row + ks * 32);
+    }
     if (k != loaded) {
       __syncthreads();  // everybody has finished with the previous offset's tile
       const u32x4* src = reinterpret_cast<const u32x4*>(Wt + (int64_t)k * a.c_out_pad * a.c_in_pad);
-      const int pieces = wrows * KS * 4;  // 16-byte pieces: KS * 4 per row
+      const int pieces = ncb * 16 * KS * 4;  // 16-byte pieces: KS * 4 per row (the tiles are zero padded beyond c_out)
       for (int i = tid; i < pieces; i += SINGLE_WAVES * 64) {
         const int row = i / (KS * 4), part = i % (KS * 4);
         *reinterpret_cast<u32x4*>(single_smem + row * ROW_BYTES + part * 16) =
@@ -62,70 +94,73 @@ __global__ void __launch_bounds__(SINGLE_WAVES * 64) conv_fwd_single(ConvArgs a,
       __syncthreads();
       loaded = k;
     }
-    const int run_end = tt.first_pair[k + 1];
-    const int p0 = tt.first_pair[k] + (tile - tt.first_tile[k]) * SINGLE_TILE + wave * (SINGLE_BPW * 16);
-    if (p0 >= run_end) continue;  // wave-uniform: this wave's share of the offset's last tile is empty
-    // the wave's pairs and their rows, in MFMA operand layout
-    int32_t orow[SINGLE_BPW];
-    V B[SINGLE_BPW][KS];
-#pragma unroll
-    for (int b = 0; b < SINGLE_BPW; ++b) {
-      const int pi = p0 + b * 16 + p;
-      const bool live = pi < run_end;
-      const int32_t irow = live ? a.in_maps[pi] : -1;
-      orow[b] = live ? a.out_maps[pi] : -1;
-      const bool ok = live && (uint32_t)irow < (uint64_t)a.num_in && (uint32_t)orow[b] < (uint64_t)a.num_out;
-      if (!ok) orow[b] = -1;
-      const T* row = X + (int64_t)(ok ? irow : 0) * a.c_in + kg * 8;
-#pragma unroll
-      for (int ks = 0; ks < KS; ++ks)
-        B[b][ks] = ok ? *reinterpret_cast<const V*>(row + ks * 32) : Mma<T>::zero();
+    int32_t next_irow[BPW], next_orow[BPW];  // asked for a tile ahead
+    if (tile + 1 < t_end) {
+      while (k + 1 < a.K && tile + 1 >= tt.first_tile[k + 1]) ++k;
+      entries(tile + 1, k, next_irow, next_orow);
     }
-    // 64 output channels at a time
-    for (int cg = 0; cg * 4 < ncb; ++cg) {
-      f32x4 acc[SINGLE_BPW][4];
+    for (int cp = 0; cp < npairs; ++cp) {
+      f32x4 acc[2][BPW];
 #pragma unroll
-      for (int b = 0; b < SINGLE_BPW; ++b)
+      for (int h = 0; h < 2; ++h)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) acc[b][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+        for (int b = 0; b < BPW; ++b) acc[h][b] = (f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
       for (int ks = 0; ks < KS; ++ks) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const int cb = cg * 4 + j;
-          if (cb < ncb) {  // uniform
-            const V A = *reinterpret_cast<const V*>(single_smem + (cb * 16 + p) * ROW_BYTES + (ks * 32 + kg * 8) * 2);
+        for (int h = 0; h < 2; ++h) {
+          if (h == 0 || cp * 2 + 1 < ncb) {  // uniform
+            const V A = *reinterpret_cast<const V*>(single_smem + (cp * 32 + h * 16 + p) * ROW_BYTES + (ks * 32 + kg * 8) * 2);
 #pragma unroll
-            for (int b = 0; b < SINGLE_BPW; ++b) acc[b][j] = Mma<T>::mma(A, B[b][ks], acc[b][j]);
+            for (int b = 0; b < BPW; ++b) acc[h][b] = Mma<T>::mma(A, B[b][ks], acc[h][b]);
           }
         }
       }
-      // lane (p, kg) holds channels cb * 16 + 4 kg .. + 3 of pair p of every block
+      // Lane (p, kg) holds channels 4 kg .. + 3 of pair p in both blocks; lanes kg and kg ^ 1 exchange four, so that each has
+      // eight of one block and stores 16 bytes.
+      float bias[2][4] = {};
+      if (a.bias) {
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int col = (cg * 4 + j) * 16 + 4 * kg;
-        if (col < a.c_out) {  // c_out is a multiple of 8: all four or none
-          float bias[4] = {0.f, 0.f, 0.f, 0.f};
-          if (a.bias) load_floats<T, 4>((const T*)a.bias + col, bias);
-#pragma unroll
-          for (int b = 0; b < SINGLE_BPW; ++b) {
-            if (orow[b] >= 0) {
-              float r[4] = {0.f, 0.f, 0.f, 0.f};
-              if (a.residual) load_floats<T, 4>((const T*)a.residual + (int64_t)orow[b] * a.c_out + col, r);
-              T t[4];
-#pragma unroll
-              for (int e = 0; e < 4; ++e) {
-                float f = acc[b][j][e];
-                if (a.bias_rounded) f = to_float(from_float<T>(f));
-                f = f + bias[e] + r[e];
-                if (a.relu) f = f < 0.f ? 0.f : f;
-                t[e] = from_float<T>(f);
-              }
-              *reinterpret_cast<uint2*>(out + (int64_t)orow[b] * a.c_out + col) = *reinterpret_cast<const uint2*>(t);
-            }
-          }
-        }
+        for (int h = 0; h < 2; ++h)
+          if (cp * 32 + h * 16 + 4 * kg < a.c_out) load_floats<T, 4>((const T*)a.bias + cp * 32 + h * 16 + 4 * kg, bias[h]);
       }
+      const int col = cp * 32 + (kg & 1) * 16 + (kg >> 1) * 8;
+#pragma unroll
+      for (int b = 0; b < BPW; ++b) {
+        uint32_t half[2][2];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+          float r[4] = {0.f, 0.f, 0.f, 0.f};
+          if (a.residual && orow[b] >= 0 && cp * 32 + h * 16 + 4 * kg < a.c_out)
+            load_floats<T, 4>((const T*)a.residual + (int64_t)orow[b] * a.c_out + cp * 32 + h * 16 + 4 * kg, r);
+          T t[4];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            float f = acc[h][b][e];
+            if (a.bias_rounded) f = to_float(from_float<T>(f));
+            f = f + bias[h][e] + r[e];
+            if (a.relu) f = f < 0.f ? 0.f : f;
+            t[e] = from_float<T>(f);
+          }
+          const uint2 two = *reinterpret_cast<const uint2*>(t);
+          half[h][0] = two.x;
+          half[h][1] = two.y;
+        }
+        u32x4 eight;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          const auto swapped = __builtin_amdgcn_permlane16_swap(half[0][i], half[1][i], false, false);
+          eight[i] = swapped[0];
+          eight[2 + i] = swapped[1];
+        }
+        if (orow[b] >= 0 && col < a.c_out)  // c_out is a multiple of 8: all eight or none
+          *reinterpret_cast<u32x4*>(out + (int64_t)orow[b] * a.c_out + col) = eight;
+      }
+    }
+#pragma unroll
+    for (int b = 0; b < BPW; ++b) {
+      irow[b] = next_irow[b];
+      orow[b] = next_orow[b];
     }
   }
 }
@@ -163,9 +198,8 @@ int launch_single(const ConvArgs& a, const WcnSingleTiles& tt, hipStream_t s) {
       allowed[device] = true;
     }
   }
-  // workgroups per CU: what the registers admit (130 to 166 a lane for rows of up to 96 channels: three
-  // waves per SIMD; 180 for 128 channels: two; 214 and 244 beyond: one) and LDS holds
-  const int per_cu = std::max(1, std::min(KS <= 3 ? 3 : (KS <= 4 ? 2 : 1), (160 * 1024) / lds));
+  // workgroups per CU: four waves a SIMD, and what LDS holds
+  const int per_cu = std::max(1, std::min(4, (160 * 1024) / lds));
   const unsigned grid = (unsigned)std::min<int64_t>(tt.total, (int64_t)single_cus() * per_cu);
   hipLaunchKernelGGL((conv_fwd_single<T, KS>), dim3(grid), dim3(SINGLE_WAVES * 64), lds, s, a, tt);
   wcn_conv_note_kernel("conv_fwd_single<%s, %d>", wcn_type_text<T>(), KS);
@@ -199,11 +233,12 @@ bool wcn_conv_single_takes(int dtype, int c_in, int c_out, int num_offsets) {
 
 int wcn_conv_single_launch(const ConvArgs& a, int dtype, const int64_t* host_offsets, hipStream_t s) {
   WcnSingleTiles tt;
+  const int tile = single_tile(a.c_in / 32);
   int64_t tiles = 0;
   for (int k = 0; k < a.K; ++k) {
     tt.first_tile[k] = (int32_t)tiles;
     tt.first_pair[k] = (int32_t)host_offsets[k];
-    tiles += (host_offsets[k + 1] - host_offsets[k] + SINGLE_TILE - 1) / SINGLE_TILE;
+    tiles += (host_offsets[k + 1] - host_offsets[k] + tile - 1) / tile;
   }
   if (tiles > INT32_MAX || host_offsets[a.K] > INT32_MAX) return WCN_ERR_INVALID_ARGUMENT;
   for (int k = a.K; k <= WCN_SINGLE_MAX_OFFSETS; ++k) {
