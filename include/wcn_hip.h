@@ -155,14 +155,6 @@ int wcn_kmap_fill(const void* table, int64_t n_keys, int64_t capacity, const int
                   const void* workspace, int64_t pair_capacity, int32_t* in_maps,
                   int32_t* out_maps, void* stream);
 
-/* wcn_kmap_count (or, with dilation and centre, wcn_kmap_count_dilated) and wcn_kmap_fill behind it in one call, which takes a
- * launch less for maps of up to 65,536 output rows.  wcn_kmap_read_result then waits as after wcn_kmap_count; with more pairs than
- * pair_capacity nothing has been written to the lists, and wcn_kmap_fill into larger ones is all that is left to do. */
-int wcn_kmap_count_fill(const void* table, int64_t n_keys, int64_t capacity, const int32_t* out_coords,
-                        int64_t num_out, const int32_t host_kernel_size[3], const int32_t host_stride[3],
-                        const int32_t* host_dilation_or_null, const int32_t* host_centre_or_null, void* workspace,
-                        int64_t pair_capacity, int32_t* in_maps, int32_t* out_maps, void* stream);
-
 /* The map of a coordinate set onto itself (the stride-1 convolution: out_coords are the table's own
  * keys, in the same rows): the same results as wcn_kmap_count / wcn_kmap_fill with out_coords =
  * keys and stride 1, from a probe pass that walks the keys in the table's block order, where

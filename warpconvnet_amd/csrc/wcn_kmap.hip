@@ -35,12 +35,8 @@ struct KmapWorkspace {  // host-computed addresses inside a kmap workspace
                         // all hits of the group; after the scan, exclusive prefix sums
   int32_t* found;       // (G, 64 K): input rows found by the hit lanes of a group, packed offset by offset
   uint16_t* tags;       // (G, 64 K): offset << 6 | lane of each of them
-  int32_t* raw;         // (K+1, G+1), up to KMAP_FEW_GROUPS groups: the counts as the probe pass leaves them
   int64_t G;            // number of 64-row groups
 };
-
-// Up to that many groups (65,536 rows) a map can be emitted without a scan in between (kmap_emit_few).
-constexpr int KMAP_FEW_GROUPS = 1024;
 
 inline size_t kmap_layout(void* base, int64_t num_out, int32_t K, KmapWorkspace* w) {
   char* p = (char*)base;
@@ -59,8 +55,6 @@ inline size_t kmap_layout(void* base, int64_t num_out, int32_t K, KmapWorkspace*
   static_assert(WCN_MAX_OFFSETS <= 1024, "offset and lane share 16 bits");
   if (w) w->tags = (uint16_t*)(p + off);
   off += wcn_align256(sizeof(uint16_t) * (size_t)K * (size_t)G * 64);
-  if (w) w->raw = (int32_t*)(p + off);
-  if (G <= KMAP_FEW_GROUPS) off += wcn_align256(sizeof(int32_t) * (size_t)(K + 1) * (size_t)(G + 1));
   if (w) w->G = G;
   return off;
 }
@@ -323,33 +317,6 @@ __global__ void __launch_bounds__(256) kmap_pass_fixed(const WcnTableHeader* __r
 // LDS: 8 * EMIT_GROUPS + 4 * (EMIT_GROUPS + 1) bytes per offset.  Against a search for the pair's offset and lane in the hit masks, and
 // workgroups in turn over the XCDs (eight runs of 22 bytes and more meet in a line): 3x3x3 over 1 M rows 23.7 -> 20 us,
 // 5x5x5 60 -> 47.5, of which the XCDs' stretches are 1 and 8.
-// A wave's group: the shifts per offset are in LDS.
-__device__ __forceinline__ void kmap_emit_group(const int32_t* __restrict__ rows, const uint16_t* __restrict__ of,
-                                                const int64_t* shift, int total, int64_t group,
-                                                int32_t* __restrict__ in_maps, int32_t* __restrict__ out_maps) {
-  constexpr int AHEAD = 4;
-  const int lane = wcn_lane();
-  for (int p0 = 0; p0 < total; p0 += 64 * AHEAD) {
-    int32_t row[AHEAD];
-    uint32_t tag[AHEAD];
-#pragma unroll
-    for (int u = 0; u < AHEAD; ++u) {
-      const int p = p0 + 64 * u + lane;
-      row[u] = rows[p < total ? p : 0];
-      tag[u] = of[p < total ? p : 0];
-    }
-#pragma unroll
-    for (int u = 0; u < AHEAD; ++u) {
-      const int p = p0 + 64 * u + lane;
-      if (p < total) {
-        const int64_t dst = shift[tag[u] >> 6] + p;
-        in_maps[dst] = row[u];
-        out_maps[dst] = (int32_t)(group * 64) + (int32_t)(tag[u] & 63u);
-      }
-    }
-  }
-}
-
 template <int EMIT_GROUPS>
 __global__ void __launch_bounds__(64 * EMIT_GROUPS) kmap_emit(const int32_t* __restrict__ found,
                                                               const uint16_t* __restrict__ tags,
@@ -389,8 +356,28 @@ __global__ void __launch_bounds__(64 * EMIT_GROUPS) kmap_emit(const int32_t* __r
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-  kmap_emit_group(found + group * (64 * (int64_t)K), tags + group * (64 * (int64_t)K), s_shift + wave * K, total, group,
-                  in_maps, out_maps);
+  const int32_t* const rows = found + group * (64 * (int64_t)K);
+  const uint16_t* const of = tags + group * (64 * (int64_t)K);
+  constexpr int AHEAD = 4;
+  for (int p0 = 0; p0 < total; p0 += 64 * AHEAD) {
+    int32_t row[AHEAD];
+    uint32_t tag[AHEAD];
+#pragma unroll
+    for (int u = 0; u < AHEAD; ++u) {
+      const int p = p0 + 64 * u + lane;
+      row[u] = rows[p < total ? p : 0];
+      tag[u] = of[p < total ? p : 0];
+    }
+#pragma unroll
+    for (int u = 0; u < AHEAD; ++u) {
+      const int p = p0 + 64 * u + lane;
+      if (p < total) {
+        const int64_t dst = s_shift[wave * K + (int)(tag[u] >> 6)] + p;
+        in_maps[dst] = row[u];
+        out_maps[dst] = (int32_t)(group * 64) + (int32_t)(tag[u] & 63u);
+      }
+    }
+  }
 }
 
 __device__ __forceinline__ int kmap_nth_set_bit(unsigned long long mask, int r) {  // position of the r-th set bit (r counts from 0)
@@ -551,131 +538,6 @@ __global__ void __launch_bounds__(1024) kmap_scan_rows(int32_t* __restrict__ gro
     __threadfence_system();
     if (lane == 0) __hip_atomic_store(&fin.mailbox[0], fin.sequence, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
   }
-}
-
-// Scan and emit pass of a map of few groups in one launch: a workgroup adds up the counts of the groups before its own
-// (all of them: 110 KB at the most for 27 offsets, out of the L2) by itself, and leaves its part of the group starts.  One
-// workgroup, the first, has no groups and writes what the scan's last one writes.  Counts (`raw`) and group starts are different arrays, so nobody
-// reads what another has written.  3x3x3 over 1.8 k to 60 k rows: 5.0 to 6.5 us of a scan and a launch less, for 1 to 3
-// us more in the emit pass.
-__global__ void __launch_bounds__(512) kmap_emit_few(const int32_t* __restrict__ found, const uint16_t* __restrict__ tags,
-                                                     const int32_t* __restrict__ raw, int32_t* __restrict__ groups, int G,
-                                                     int64_t pair_capacity, int32_t* __restrict__ in_maps,
-                                                     int32_t* __restrict__ out_maps, KmapFinish fin) {
-  constexpr int GROUPS = 8;
-  const int K = fin.K;
-  extern __shared__ __attribute__((aligned(16))) char emit_lds[];
-  int64_t* const s_shift = reinterpret_cast<int64_t*>(emit_lds);              // [GROUPS][K]
-  int32_t* const s_count = reinterpret_cast<int32_t*>(s_shift + GROUPS * K);  // [K][GROUPS]
-  int32_t* const s_before = s_count + GROUPS * K;                             // [K]: pairs of the groups before
-  int32_t* const s_offset = s_before + K;                                     // [K + 1]: totals, then the lists' offsets
-  __shared__ int s_stat[2][8];
-  const bool tells = blockIdx.x == 0;
-  const int first = tells ? 0 : ((int)blockIdx.x - 1) * GROUPS;
-  const int tid = threadIdx.x, lane = wcn_lane(), wave = tid >> 6;
-  const int64_t status = fin.hdr->status;
-  for (int k = wave; k < K; k += 8) {
-    const int32_t* const row = raw + (int64_t)k * (G + 1);
-    int before = 0, all = 0;
-    for (int g0 = 0; g0 < G; g0 += 256) {
-      int v[4];
-#pragma unroll
-      for (int t = 0; t < 4; ++t) v[t] = g0 + t * 64 + lane < G ? row[g0 + t * 64 + lane] : 0;
-#pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        all += v[t];
-        before += g0 + t * 64 + lane < first ? v[t] : 0;
-      }
-    }
-    before = wcn_wave_inclusive_sum(before);
-    all = wcn_wave_inclusive_sum(all);
-    if (lane == 63) {
-      s_before[k] = before;
-      s_offset[k] = all;
-    }
-  }
-  for (int i = tid; i < (tells ? 0 : K * GROUPS); i += 512)
-    s_count[i] = first + i % GROUPS < G ? raw[(int64_t)(i / GROUPS) * (G + 1) + first + i % GROUPS] : 0;
-  if (tells) {  // occupied slots and distinct keys, as in kmap_scan_rows
-    const int32_t bins = fin.hdr->bins;
-    const int32_t* stats = reinterpret_cast<const int32_t*>(reinterpret_cast<const char*>(fin.hdr) + fin.hdr->stats_offset);
-    int voxels = 0, occupied = 0;
-    for (int i = tid; i < bins; i += 512) {
-      voxels += stats[2 * i];
-      occupied += stats[2 * i + 1];
-    }
-    voxels = wcn_wave_inclusive_sum(voxels);
-    occupied = wcn_wave_inclusive_sum(occupied);
-    if (lane == 63) {
-      s_stat[0][wave] = voxels;
-      s_stat[1][wave] = occupied;
-    }
-  }
-  __syncthreads();
-  int pairs = 0;  // fewer than 2^31: 65,536 rows and 320 offsets
-  if (wave == 0) {
-    for (int k0 = 0; k0 < K; k0 += 64) {
-      const int n = k0 + lane < K ? s_offset[k0 + lane] : 0;
-      const int incl = wcn_wave_inclusive_sum(n);
-      if (k0 + lane < K) s_offset[k0 + lane] = pairs + incl - n;
-      pairs += __shfl(incl, 63, 64);
-    }
-    if (lane == 0) s_offset[K] = pairs;
-  }
-  __syncthreads();
-  pairs = s_offset[K];
-  if (tells) {
-    auto put = [&](int at, int64_t v) {
-      fin.result[at] = v;
-      if (fin.mailbox) fin.mailbox[1 + at] = v;
-    };
-    for (int k = tid; k <= K; k += 512) put(k, s_offset[k]);
-    if (tid == 0) {
-      int voxels = 0, occupied = 0;
-      for (int w = 0; w < 8; ++w) {
-        voxels += s_stat[0][w];
-        occupied += s_stat[1][w];
-      }
-      put(K + 1, status);
-      put(K + 2, (int64_t)occupied | ((int64_t)(voxels != fin.hdr->num_keys ? 1 : 0) << 32));
-    }
-    if (fin.mailbox) {
-      __threadfence_system();
-      __syncthreads();
-      if (tid == 0) __hip_atomic_store(&fin.mailbox[0], fin.sequence, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
-    }
-    return;
-  }
-  const bool last = first + GROUPS >= G;
-  for (int i = tid; i < K * (GROUPS + 1); i += 512) {  // the group starts: of these groups and, from the last, the totals
-    const int k = i / (GROUPS + 1), j = i % (GROUPS + 1);
-    if (first + j < (last ? G + 1 : first + GROUPS)) {
-      int start = s_before[k];
-      for (int t = 0; t < j; ++t) start += s_count[k * GROUPS + t];
-      groups[(int64_t)k * (G + 1) + first + j] = start;
-    }
-  }
-  if (pairs > pair_capacity || status != 0) return;
-  const int group = first + wave;
-  if (group >= G) return;
-  int total = 0;
-  for (int k0 = 0; k0 < K; k0 += 64) {
-    const int k = k0 + lane;
-    int n = 0, start = 0;
-    if (k < K) {
-      start = s_offset[k] + s_before[k];
-      for (int t = 0; t < wave; ++t) start += s_count[k * GROUPS + t];
-      n = s_count[k * GROUPS + wave];
-    }
-    const int incl = wcn_wave_inclusive_sum(n);
-    if (k < K) s_shift[wave * K + k] = start - (total + incl - n);
-    total += __shfl(incl, 63, 64);
-  }
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-  kmap_emit_group(found + (int64_t)group * (64 * K), tags + (int64_t)group * (64 * K), s_shift + wave * K, total, group,
-                  in_maps, out_maps);
 }
 
 // ---- maps of a coordinate set onto itself (stride 1), probed block by block ----------------------
@@ -1166,22 +1028,22 @@ inline bool table_args_ok(const void* table, int64_t n_keys, int64_t capacity) {
 }
 
 void launch_probe(const WcnTableView& v, const int32_t* out_coords, int64_t num_out,
-                  const KmapGeom& g, const KmapWorkspace& w, int32_t* counts, hipStream_t s) {
+                  const KmapGeom& g, const KmapWorkspace& w, hipStream_t s) {
   const dim3 grid(grid_for(num_out, 256)), block(256);
   const uint32_t cap_mask = (uint32_t)(v.capacity - 1);
   const KmapProbe o = {w.found, w.tags, w.ticket};
   if (is_fixed_size(g, 3, 3, 3)) {
     hipLaunchKernelGGL((kmap_pass_fixed<3, 3, 3>), grid, block, 0, s, v.hdr, v.slots, cap_mask,
-                       v.perm, (const int4*)out_coords, num_out, g, counts, w.G, o);
+                       v.perm, (const int4*)out_coords, num_out, g, w.groups, w.G, o);
   } else if (is_fixed_size(g, 2, 2, 2)) {
     hipLaunchKernelGGL((kmap_pass_fixed<2, 2, 2>), grid, block, 0, s, v.hdr, v.slots, cap_mask,
-                       v.perm, (const int4*)out_coords, num_out, g, counts, w.G, o);
+                       v.perm, (const int4*)out_coords, num_out, g, w.groups, w.G, o);
   } else if (is_fixed_size(g, 5, 5, 5)) {
     hipLaunchKernelGGL((kmap_pass_fixed<5, 5, 5>), grid, block, 0, s, v.hdr, v.slots, cap_mask,
-                       v.perm, (const int4*)out_coords, num_out, g, counts, w.G, o);
+                       v.perm, (const int4*)out_coords, num_out, g, w.groups, w.G, o);
   } else {
     hipLaunchKernelGGL(kmap_pass, grid, block, 0, s, v.hdr, v.slots, cap_mask, v.perm,
-                       (const int4*)out_coords, num_out, g, counts, w.G, o);
+                       (const int4*)out_coords, num_out, g, w.groups, w.G, o);
   }
 }
 
@@ -1496,32 +1358,22 @@ size_t wcn_kmap_workspace_bytes(int64_t num_out, int32_t num_offsets) {
   return a > b ? a : b;
 }
 
-// Count pass and scan; with `fill` the emit pass too, into lists of `pair_capacity` places.
-struct KmapFill {
-  int64_t pair_capacity;
-  int32_t *in_maps, *out_maps;
-};
-
 static int kmap_count_impl(const void* table, int64_t n_keys, int64_t capacity, const int32_t* out_coords,
                            int64_t num_out, const int32_t host_kernel_size[3],
                            const int32_t host_stride[3], const int32_t* host_dilation,
-                           const int32_t* host_centre, void* workspace, const KmapFill* fill, void* stream) {
+                           const int32_t* host_centre, void* workspace, void* stream) {
   KmapGeom g;
   if (!make_geom(host_kernel_size, host_stride, host_dilation, host_centre, &g)) return WCN_ERR_INVALID_ARGUMENT;
   if (!table_args_ok(table, n_keys, capacity) || !workspace || num_out < 0 ||
       num_out >= (1ll << 31) || (num_out > 0 && !out_coords))
-    return WCN_ERR_INVALID_ARGUMENT;
-  if (fill && (fill->pair_capacity < 0 || (fill->pair_capacity > 0 && (!fill->in_maps || !fill->out_maps))))
     return WCN_ERR_INVALID_ARGUMENT;
   hipStream_t s = (hipStream_t)stream;
   WcnTableView v;
   wcn_table_layout(const_cast<void*>(table), n_keys, capacity, &v);
   KmapWorkspace w;
   kmap_layout(workspace, num_out, g.K, &w);
-  // (320 offsets: 33 KB of LDS; more do not occur in earnest)
-  const bool few = fill && w.G > 0 && w.G <= KMAP_FEW_GROUPS && g.K <= 320;
   if (w.G > 0) {
-    launch_probe(v, out_coords, num_out, g, w, few ? w.raw : w.groups, s);
+    launch_probe(v, out_coords, num_out, g, w, s);
   } else {
     hipLaunchKernelGGL(kmap_zero_ticket, dim3(1), dim3(1), 0, s, w.ticket);
   }
@@ -1538,21 +1390,12 @@ static int kmap_count_impl(const void* table, int64_t n_keys, int64_t capacity, 
   g_pending_sequence = sequence;
   g_pending_result = w.result;
   const KmapFinish fin = {w.result, w.ticket, v.hdr, g.K, box, sequence};
-  if (few) {
-    hipLaunchKernelGGL(kmap_emit_few, dim3(1 + grid_for(num_out, 512)), dim3(512), 104u * (unsigned)g.K + 8u, s, w.found, w.tags, w.raw,
-                       w.groups, (int)w.G, fill->pair_capacity, fill->in_maps, fill->out_maps, fin);
-  } else {
-    hipLaunchKernelGGL(kmap_scan_rows, dim3(g.K + 1), dim3(1024), 0, s, w.groups, w.G, w.row_total, fin);
-  }
+  hipLaunchKernelGGL(kmap_scan_rows, dim3(g.K + 1), dim3(1024), 0, s, w.groups, w.G, w.row_total, fin);
   WCN_LAUNCH_CHECK();
   if (box) {
     if (wcn_mailbox_mark(s) != WCN_OK) return WCN_ERR_LAUNCH;
   } else if (wcn_read_early_begin(w.result, sizeof(int64_t) * (size_t)(g.K + 3), s) != WCN_OK) {
     return WCN_ERR_LAUNCH;
-  }
-  if (fill && !few && num_out > 0 && fill->pair_capacity > 0) {
-    launch_emit(num_out, g, w, fill->pair_capacity, fill->in_maps, fill->out_maps, s);
-    WCN_LAUNCH_CHECK();
   }
   return WCN_OK;
 }
@@ -1561,7 +1404,7 @@ int wcn_kmap_count(const void* table, int64_t n_keys, int64_t capacity, const in
                    int64_t num_out, const int32_t host_kernel_size[3],
                    const int32_t host_stride[3], void* workspace, void* stream) {
   return kmap_count_impl(table, n_keys, capacity, out_coords, num_out, host_kernel_size, host_stride,
-                         nullptr, nullptr, workspace, nullptr, stream);
+                         nullptr, nullptr, workspace, stream);
 }
 
 int wcn_kmap_count_dilated(const void* table, int64_t n_keys, int64_t capacity, const int32_t* out_coords,
@@ -1570,17 +1413,7 @@ int wcn_kmap_count_dilated(const void* table, int64_t n_keys, int64_t capacity, 
                            const int32_t host_centre[3], void* workspace, void* stream) {
   if (!host_dilation || !host_centre) return WCN_ERR_INVALID_ARGUMENT;
   return kmap_count_impl(table, n_keys, capacity, out_coords, num_out, host_kernel_size, host_stride,
-                         host_dilation, host_centre, workspace, nullptr, stream);
-}
-
-int wcn_kmap_count_fill(const void* table, int64_t n_keys, int64_t capacity, const int32_t* out_coords,
-                        int64_t num_out, const int32_t host_kernel_size[3], const int32_t host_stride[3],
-                        const int32_t* host_dilation_or_null, const int32_t* host_centre_or_null, void* workspace,
-                        int64_t pair_capacity, int32_t* in_maps, int32_t* out_maps, void* stream) {
-  if ((host_dilation_or_null == nullptr) != (host_centre_or_null == nullptr)) return WCN_ERR_INVALID_ARGUMENT;
-  const KmapFill fill = {pair_capacity, in_maps, out_maps};
-  return kmap_count_impl(table, n_keys, capacity, out_coords, num_out, host_kernel_size, host_stride,
-                         host_dilation_or_null, host_centre_or_null, workspace, &fill, stream);
+                         host_dilation, host_centre, workspace, stream);
 }
 
 static bool self_size(const int32_t ks[3], int32_t* K) {
