@@ -103,7 +103,7 @@ _TILES = [(torch.bfloat16, 32, 32, 4096, "1, 8"), (torch.bfloat16, 32, 32, 4097,
           (torch.float16, 128, 128, 1024, "1, 16"), (torch.float16, 128, 128, 1025, "2, 16"),
           (torch.float16, 128, 128, 2049, "4, 16"), (torch.float16, 120, 100, 4097, "4, 8"),
           (torch.float32, 64, 40, 2048, "1, 16"), (torch.float32, 64, 72, 2049, "2, 16"), (torch.float32, 16, 20, 60, "1, 8"),
-          (torch.float32, 64, 64, 4097, "4, 8")]
+          (torch.float32, 64, 64, 4097, "4, 8"), (torch.float16, 32, 16, 8193, "1, 8"), (torch.float32, 64, 12, 8193, "1, 8")]
 
 
 @pytest.mark.parametrize("infinite", [False, True], ids=["finite", "infinite_weight"])
