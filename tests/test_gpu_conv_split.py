@@ -97,13 +97,14 @@ def test_kept_tiles_are_those_that_are_read():
     assert [bytes_ for _, bytes_ in seen] == [half, half, 0, 0]
 
 
-# (dtype, C_in, C_out, rows, instance): sixteen, thirty-two or sixty-four channels a tile, as long as every tile has one of the 256 CUs,
-# and eight or sixteen waves (from 100 units on)
+# (dtype, C_in, C_out, rows, instance): sixteen, thirty-two or sixty-four channels a tile, as long as every tile has one of the 256 CUs
+# (forty-eight where that leaves less over), and eight or sixteen waves (from 100 units on)
 _TILES = [(torch.bfloat16, 32, 32, 4096, "1, 8"), (torch.bfloat16, 32, 32, 4097, "2, 8"), (torch.bfloat16, 64, 64, 2080, "2, 8"),
           (torch.float16, 128, 128, 1024, "1, 16"), (torch.float16, 128, 128, 1025, "2, 16"),
           (torch.float16, 128, 128, 2049, "4, 16"), (torch.float16, 120, 100, 4097, "4, 8"),
           (torch.float32, 64, 40, 2048, "1, 16"), (torch.float32, 64, 72, 2049, "2, 16"), (torch.float32, 16, 20, 60, "1, 8"),
-          (torch.float32, 64, 64, 4097, "4, 8"), (torch.float16, 32, 16, 8193, "1, 8"), (torch.float32, 64, 12, 8193, "1, 8")]
+          (torch.float32, 64, 64, 4097, "4, 8"), (torch.float16, 32, 16, 8193, "1, 8"), (torch.float32, 64, 12, 8193, "1, 8"),
+          (torch.bfloat16, 96, 96, 4097, "3, 8"), (torch.float16, 64, 136, 2100, "3, 8"), (torch.float32, 48, 40, 8193, "3, 8")]
 
 
 @pytest.mark.parametrize("infinite", [False, True], ids=["finite", "infinite_weight"])
