@@ -128,3 +128,15 @@ def test_tiles_get_wider_when_the_cus_are_taken(oracle, dtype, c_in, c_out, rows
     assert lib().wcn_conv_last_kernel().decode() == f"conv_fwd_small<{text}, {tile}>"
     assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(got[np.isinf(want)], want[np.isinf(want)])
     assert rel_err(np.where(np.isfinite(want), got, 0.0), np.where(np.isfinite(want), want, 0.0)) <= TOL[dtype]
+
+
+@pytest.mark.parametrize("dtype,c_in,c_out,rows,extent,ksize,kernel", [
+    (torch.float32, 96, 96, 24_000, 60, (3, 3, 3), "conv_fwd_pack<float"), (torch.float32, 128, 40, 40_000, 60, (3, 3, 3), "conv_fwd_pack<float"),
+    (torch.float32, 36, 64, 45_000, 60, (3, 3, 3), "conv_fwd_pack<float"), (torch.float32, 160, 64, 12_000, 40, (3, 3, 3), "conv_fwd_small<float, 4, 8"),
+    (torch.float32, 64, 64, 2500, 30, (5, 5, 5), "conv_fwd_small<float, 2, 16"), (torch.float16, 256, 256, 12_000, 50, (3, 3, 3), "conv_fwd_ring<"),
+    (torch.float16, 128, 128, 12_000, 50, (2, 2, 2), "conv_fwd_small<f16, 4, 8")],
+    ids=["f32_three_slices", "f32_four_slices", "f32_part_of_a_slice", "f32_five_slices", "f32_k5", "f16_ring", "f16_k2"])
+def test_lines_between_the_kernels(oracle, dtype, c_in, c_out, rows, extent, ksize, kernel):
+    got, want, name = _run(oracle, dtype, c_in, c_out, rows, extent, ksize, residual=True)
+    assert name.startswith(kernel), name
+    assert torch.equal(got[0], got[1]) and rel_err(got[0].double().cpu().numpy(), want) <= TOL[dtype]

@@ -1530,7 +1530,16 @@ static int conv_run(const void* features, int64_t num_in, int32_t c_in, int32_t 
   a.vec_res = (a.residual && ((size_t)c_out * es) % 16 == 0 && ((uintptr_t)a.residual % 16) == 0) ? 1 : 0;
   a.flat_in = (c_in % ck_of(dtype) == 0 && (uint64_t)num_in * c_in * es < (1ull << 32)) ? 1 : 0;
   a.partial = w.partial;
-  a.split = (a.vec_in && w.partial != nullptr) ? 1 : 0;
+  // fp32 rows that the pair-packed kernel takes are not sliced (their workspace is as if they were): its steps are longer than the
+  // barrier between them, whatever the number of tiles.  us, sliced ring kernel / pair-packed, 3x3x3 on rooms:
+  //     rows      64->64      96->96     128->128     64->128     128->64
+  //     12,000   162 /  78   169 / 114   172 / 148   167 /  80   168 / 146
+  //     32,000   166 /  79   249 / 114   416 / 147   247 /  79   246 / 142
+  //     64,000   238 /  80       / 162       / 211       / 115   440 / 143
+  // (16-bit rows: 47 / 48 at 128 -> 128 and 12,000 rows, 64 / 87 at 256 -> 256 and 7,000.)
+  a.split = 0;
+  a.split = a.vec_in && w.partial != nullptr &&
+            !(dtype == WCN_DTYPE_F32 && kernel_choice() != 1 && wcn_conv_pack_takes(a, dtype));
   // The kernel for small maps (which reads the weight in an order of its own).  Not inside a graph: it adds the
   // offsets up in the order of its waves, every other kernel in ascending order.  A sum that comes out on the other
   // side of a rounding is nothing by itself, but behind a ReLU one such value in a million switches a
