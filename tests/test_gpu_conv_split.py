@@ -131,7 +131,7 @@ def test_tiles_get_wider_when_the_cus_are_taken(oracle, dtype, c_in, c_out, rows
 
 
 @pytest.mark.parametrize("dtype,c_in,c_out,rows,extent,ksize,kernel", [
-    (torch.float32, 96, 96, 24_000, 60, (3, 3, 3), "conv_fwd_pack<float"), (torch.float32, 128, 40, 40_000, 60, (3, 3, 3), "conv_fwd_pack<float"),
+    (torch.float32, 96, 96, 24_000, 60, (3, 3, 3), "conv_fwd_pack<float"), (torch.float32, 128, 40, 48_000, 60, (3, 3, 3), "conv_fwd_pack<float"),
     (torch.float32, 36, 64, 45_000, 60, (3, 3, 3), "conv_fwd_pack<float"), (torch.float32, 160, 64, 12_000, 40, (3, 3, 3), "conv_fwd_small<float, 4, 8"),
     (torch.float32, 64, 64, 2500, 30, (5, 5, 5), "conv_fwd_small<float, 2, 16"), (torch.float16, 256, 256, 12_000, 50, (3, 3, 3), "conv_fwd_ring<"),
     (torch.float16, 128, 128, 12_000, 50, (2, 2, 2), "conv_fwd_small<f16, 4, 8")],
