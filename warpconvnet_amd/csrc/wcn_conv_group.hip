@@ -1,4 +1,4 @@
-// Feature contraction for narrow layers (at most 32 channels in and out, 16-bit features): a wave
+// Feature contraction for narrow layers (at most 32 channels in and out; fp32: at most 16 on one side): a wave
 // owns a group of 64 output rows from the first kernel offset to the last.
 //
 //   out[m, :] = bias + sum_k X[in_k(m), :] @ W[k]
