@@ -1203,8 +1203,8 @@ template <typename T>
 int launch_conv(const ConvArgs& a, hipStream_t s) {
   constexpr int dtype = std::is_same<T, float>::value ? WCN_DTYPE_F32
                         : std::is_same<T, _Float16>::value ? WCN_DTYPE_F16 : WCN_DTYPE_BF16;
-  // Wide rows on both sides go to the output-stationary kernel of wcn_conv_dense.hip, 16-bit rows of
-  // at most 32 channels on both sides to the kernel of wcn_conv_group.hip, rows of up to four
+  // Wide rows on both sides go to the output-stationary kernel of wcn_conv_dense.hip, rows of at most 32
+  // channels on both sides (fp32: 16 on one of them) to the kernel of wcn_conv_group.hip, rows of up to four
   // k-slices to the pair-packed kernel.
   const int only = kernel_choice();
   const bool ring_only = only == 1;

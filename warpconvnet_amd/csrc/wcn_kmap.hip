@@ -920,7 +920,7 @@ __global__ void __launch_bounds__(SELF_CHUNK) self_emit(const uint32_t* __restri
   __shared__ int s_start[WAVES][K];     // pairs of offset k below the wave's first row
   __shared__ uint32_t s_hm[WAVES][64][WORDS];
   __shared__ int32_t s_ptr[WAVES][64];
-  // as in kmap_emit_flat; the group starts are written whatever the room for pairs (the caller keeps them)
+  // as in kmap_emit; the group starts are written whatever the room for pairs (the caller keeps them)
   if (offsets[K + 1] != 0) return;
   const bool room = offsets[K] <= pair_capacity;
   const int tid = threadIdx.x, lane = wcn_lane(), wave = tid >> 6;
