@@ -10,7 +10,9 @@
  *     first use and held until wcn_thread_release() or the end of the process; and, per process,
  *     the device-resident array behind wcn_sparse_conv_fwd_static;
  *   - per-thread state crosses calls in three places, all named where they are declared:
- *     wcn_kmap_count arms the result mailbox that the same thread's wcn_kmap_read_result collects,
+ *     wcn_kmap_count (_dilated, _self) and wcn_stride_unique_cells arm the result mailbox that the same
+ *     thread's wcn_kmap_read_result and wcn_stride_unique_read_* collect (the next call that writes such a
+ *     result, wcn_stride_unique among them, lets go of one that nobody has read),
  *     wcn_kmap_last_table_flags reports on that thread's last read, and
  *     wcn_conv_set_timing_events arms the thread's next contraction call;
  *   - a call that waits for the device (the *_read_* functions) polls with an upper bound of

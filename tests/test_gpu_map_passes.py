@@ -1,6 +1,8 @@
 """The map passes where their lists are full or nearly empty: every offset of every row hits (a solid
 cube), rows that end inside a group, a workgroup or a stretch of workgroups, and maps of more offsets
 than one workgroup of the emit pass takes for eight groups.  Bit-exact against the CPU oracle."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -79,3 +81,39 @@ def test_strided_rows_and_their_batch_offsets(sizes, stride):
     assert np.array_equal(got.cpu().numpy(), want)
     counts = np.bincount(want[:, 0], minlength=len(sizes))[: int(want[-1, 0]) + 1]
     assert offsets.tolist() == np.concatenate([[0], np.cumsum(counts)]).tolist()
+
+
+@pytest.mark.parametrize("bounds", [False, True], ids=["count", "bounds"])
+@pytest.mark.parametrize("left", ["count", "dilated", "self", "cells"])
+def test_a_result_that_nobody_read_is_not_the_next_one(left, bounds):
+    """A map (or strided rows) whose result is not read, as after an error in between, then strided rows of another kind in
+    the same workspace: their number is theirs."""
+    from warpconvnet_amd._lib import check, int3, lib, ptr, stream_ptr, workspace
+    from warpconvnet_amd.geometry.coords.search.torch_hashmap import TorchHashTable
+    dev = torch.device(DEV)
+    rows = torch.as_tensor(_cube(9), device=DEV)
+    n, L, s = len(rows), lib(), stream_ptr(dev)
+    table, _, slots = TorchHashTable.from_keys(rows)._raw()
+    out = torch.empty(n, 4, dtype=torch.int32, device=DEV)
+    first = torch.empty(n, dtype=torch.int32, device=DEV)
+    ws = workspace(max(L.wcn_kmap_workspace_bytes(n, 27), L.wcn_stride_unique_workspace_bytes(n, slots),
+                       L.wcn_stride_unique_cells_workspace_bytes(n)), dev)
+    k3, one, two, three = (int3((v,) * 3) for v in (3, 1, 2, 3))
+    if left == "count":
+        check(L.wcn_kmap_count(ptr(table), n, slots, ptr(rows), n, k3, one, ptr(ws), s), "count")
+    elif left == "dilated":
+        check(L.wcn_kmap_count_dilated(ptr(table), n, slots, ptr(rows), n, k3, one, two, one, ptr(ws), s), "count")
+    elif left == "self":
+        check(L.wcn_kmap_count_self(ptr(table), n, slots, k3, ptr(ws), s), "count")
+    else:
+        check(L.wcn_stride_unique_cells(ptr(table), n, slots, ptr(rows), two, ptr(ws), ptr(out), ptr(first), s), "cells")
+    torch.cuda.synchronize()
+    check(L.wcn_stride_unique(ptr(rows), n, three, ptr(ws), slots, ptr(out), ptr(first), s), "stride")
+    got, marks = ctypes.c_int64(-1), (ctypes.c_int64 * 1025)()
+    if bounds:
+        check(L.wcn_stride_unique_read_bounds(ptr(ws), n, slots, ctypes.byref(got), marks, s), "read")
+        assert marks[0] == 0 and marks[1] == 27 and marks[1024] == 27
+    else:
+        check(L.wcn_stride_unique_read_count(ptr(ws), n, slots, ctypes.byref(got), s), "read")
+    assert got.value == 27  # -3 .. 5 in cells of three
+    assert torch.equal(out[:27].unique(dim=0), torch.unique(torch.cat([rows[:, :1], rows[:, 1:] // 3], dim=1), dim=0))

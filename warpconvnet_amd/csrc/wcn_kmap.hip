@@ -1345,9 +1345,25 @@ void wcn_scan_rows_launch(int32_t* groups, int64_t G, int rows, int64_t* row_tot
 // what the last wcn_kmap_read_result of this host thread learned about the table (bit 0: some
 // key was inserted more than once)
 static thread_local int32_t g_last_table_flags = 0;
-// the mailbox write the last count call of this thread armed, and the result block it mirrors
-static thread_local int64_t g_pending_sequence = 0;
-static thread_local const void* g_pending_result = nullptr;
+// The mailbox write that this thread's last call armed, the result block it mirrors, and whose words they are: a map's and strided
+// rows' results may lie at one address, one workspace after the other.  Every call that writes a result block sets or clears it.
+enum class Pending { none, map, cells };
+static thread_local struct {
+  Pending kind = Pending::none;
+  int64_t sequence = 0;
+  const void* result = nullptr;
+} g_pending;
+
+static void set_pending(Pending kind, int64_t sequence, const void* result) {
+  g_pending = {sequence != 0 ? kind : Pending::none, sequence, result};
+}
+
+// The sequence of the mailbox write behind a result block, which is then collected; 0 if there is none.
+static int64_t take_pending(Pending kind, const void* result) {
+  if (g_pending.kind != kind || g_pending.result != result) return 0;
+  g_pending.kind = Pending::none;
+  return g_pending.sequence;
+}
 
 extern "C" {
 
@@ -1387,8 +1403,7 @@ static int kmap_count_impl(const void* table, int64_t n_keys, int64_t capacity, 
     box = nullptr;
     sequence = 0;
   }
-  g_pending_sequence = sequence;
-  g_pending_result = w.result;
+  set_pending(Pending::map, sequence, w.result);
   const KmapFinish fin = {w.result, w.ticket, v.hdr, g.K, box, sequence};
   hipLaunchKernelGGL(kmap_scan_rows, dim3(g.K + 1), dim3(1024), 0, s, w.groups, w.G, w.row_total, fin);
   WCN_LAUNCH_CHECK();
@@ -1457,8 +1472,7 @@ int wcn_kmap_count_self(const void* table, int64_t n_keys, int64_t capacity,
     box = nullptr;
     sequence = 0;
   }
-  g_pending_sequence = sequence;
-  g_pending_result = w.result;
+  set_pending(Pending::map, sequence, w.result);
   const KmapFinish fin = {w.result, w.ticket, v.hdr, K, box, sequence};
   hipLaunchKernelGGL(kmap_scan_rows, dim3(K), dim3(1024), 0, s, w.chunk, w.C, w.row_total, fin);
   WCN_LAUNCH_CHECK();
@@ -1503,8 +1517,7 @@ int wcn_kmap_read_result(const void* workspace, int64_t num_out, int32_t num_off
   const size_t bytes = sizeof(int64_t) * (size_t)(num_offsets + 3);
   // from the mailbox the count call armed; otherwise (another thread, a count call that failed
   // half-way) from the device copy
-  const int64_t sequence = g_pending_result == (const void*)w.result ? g_pending_sequence : 0;
-  if (sequence != 0) g_pending_sequence = 0;
+  const int64_t sequence = take_pending(Pending::map, w.result);
   if (sequence == 0 || wcn_mailbox_end(tmp, bytes, sequence) != WCN_OK) {
     if (wcn_read_early_end(tmp, w.result, bytes, (hipStream_t)stream) != WCN_OK) return WCN_ERR_LAUNCH;
   }
@@ -1559,6 +1572,7 @@ int wcn_stride_unique(const int32_t* coords, int64_t n, const int32_t host_strid
   hipStream_t s = (hipStream_t)stream;
   StrideWorkspace w;
   stride_layout(workspace, n, capacity, &w);
+  set_pending(Pending::none, 0, nullptr);  // the result comes from the device
   WcnTableView v;
   wcn_table_layout(w.table, n, capacity, &v);
   if (n > 0) {
@@ -1617,8 +1631,7 @@ int wcn_stride_unique_cells(const void* table, int64_t n_keys, int64_t capacity,
   unsigned long long* picked = (unsigned long long*)((char*)counts + wcn_align256(sizeof(int32_t) * (size_t)(parts + 1)));
   int32_t* item_row = (int32_t*)((char*)picked + wcn_align256(sizeof(unsigned long long) * (size_t)((n + 63) / 64)));
   const uint32_t cap_mask = (uint32_t)(capacity - 1);
-  g_pending_sequence = 0;
-  g_pending_result = nullptr;
+  set_pending(Pending::none, 0, nullptr);
   if (n == 0) {
     hipLaunchKernelGGL(stride_no_rows, dim3(1), dim3(1024), 0, s, result, v.hdr);
     WCN_LAUNCH_CHECK();
@@ -1641,19 +1654,15 @@ int wcn_stride_unique_cells(const void* table, int64_t n_keys, int64_t capacity,
   WCN_LAUNCH_CHECK();
   if (res.mailbox) {
     if (wcn_mailbox_mark(s) != WCN_OK) return WCN_ERR_LAUNCH;
-    g_pending_sequence = res.sequence;
-    g_pending_result = result;
+    set_pending(Pending::cells, res.sequence, result);
   }
   return WCN_OK;
 }
 
 // From the mailbox a wcn_stride_unique_cells call of this thread armed, once its rows are written too, otherwise from the device copy.
 static int stride_read(const int64_t* result, int64_t* host, size_t bytes, hipStream_t stream) {
-  const int64_t sequence = g_pending_result == (const void*)result ? g_pending_sequence : 0;
-  if (sequence != 0) {
-    g_pending_sequence = 0;
-    if (wcn_mailbox_end(host, bytes, sequence, true) == WCN_OK) return WCN_OK;
-  }
+  const int64_t sequence = take_pending(Pending::cells, result);
+  if (sequence != 0 && wcn_mailbox_end(host, bytes, sequence, true) == WCN_OK) return WCN_OK;
   return wcn_read_small(host, result, bytes, stream);
 }
 
