@@ -117,3 +117,41 @@ def test_a_result_that_nobody_read_is_not_the_next_one(left, bounds):
         check(L.wcn_stride_unique_read_count(ptr(ws), n, slots, ctypes.byref(got), s), "read")
     assert got.value == 27  # -3 .. 5 in cells of three
     assert torch.equal(out[:27].unique(dim=0), torch.unique(torch.cat([rows[:, :1], rows[:, 1:] // 3], dim=1), dim=0))
+
+
+@pytest.mark.parametrize("then", ["map", "cells"])
+def test_a_result_on_its_way_does_not_reach_the_next_one(oracle, then):
+    """A map's result that nobody reads, behind a long queue of another stream; results asked for meanwhile come from the
+    device, and later ones from the mailbox again."""
+    from warpconvnet_amd._lib import check, int3, lib, ptr, stream_ptr, workspace
+    from warpconvnet_amd.geometry.coords.ops.stride import stride_coords
+    from warpconvnet_amd.geometry.coords.search.torch_discrete import generate_kernel_map
+    from warpconvnet_amd.geometry.coords.search.torch_hashmap import TorchHashTable
+    dev, cube = torch.device(DEV), _cube(9)
+    rows = torch.as_tensor(cube, device=DEV)
+    n, L = len(rows), lib()
+    table, _, slots = TorchHashTable.from_keys(rows)._raw()
+    ws = workspace(L.wcn_kmap_workspace_bytes(n, 125), dev)
+    want = oracle.kernel_map(cube, cube, (3, 3, 3))
+    a = torch.randn(8192, 8192, device=DEV)
+    (a @ a).sum().item()
+    other = torch.cuda.Stream()
+    other.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(other):
+        for _ in range(20):
+            a = a @ a * 1e-4
+        check(L.wcn_kmap_count(ptr(table), n, slots, ptr(rows), n, int3((5, 5, 5)), int3((1, 1, 1)), ptr(ws), stream_ptr(dev)), "count")
+        done = torch.cuda.Event()
+        done.record()
+    for turn in range(3):
+        if then == "map":
+            got = generate_kernel_map(rows.clone(), rows, (1, 1, 1), (3, 3, 3))
+            assert np.array_equal(got.offsets.numpy().astype(np.int64), want[2])
+            assert np.array_equal(got.in_maps.cpu().numpy(), want[0]) and np.array_equal(got.out_maps.cpu().numpy(), want[1])
+        else:
+            coarse, offsets = stride_coords(rows.clone(), (2, 2, 2), batch_sorted=True)
+            assert offsets.tolist() == [0, 125] and len(coarse.unique(dim=0)) == 125
+        if turn == 0:
+            assert not done.query()  # the queue was longer than this
+        if turn == 1:
+            torch.cuda.synchronize()

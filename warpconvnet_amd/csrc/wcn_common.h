@@ -296,7 +296,8 @@ int wcn_read_early_end(void* host_dst, const void* device_src, size_t bytes, hip
 // 8-byte sequence word) and a fresh sequence number; the kernel writes the payload, a system-scope
 // fence, then the sequence number into word 0.  `end` polls word 0 (and `done`, an event recorded
 // after the kernel, so that a kernel that never wrote cannot stall the host: it then returns
-// WCN_ERR_LAUNCH and the caller reads the device copy instead) and copies the payload out; with `kernel_over` it
+// WCN_ERR_LAUNCH and the caller reads the device copy instead) and copies the payload out.  While a write that was armed
+// and not collected is on its way, `begin` returns WCN_ERR_LAUNCH: the caller reads the device copy.  With `kernel_over` it
 // waits for `done` in any case (the kernel writes more than the mailbox, and the caller takes it for written).
 int wcn_mailbox_begin(int64_t** device_visible_box, int64_t* sequence);
 int wcn_mailbox_mark(hipStream_t stream);  // records `done` behind the writing kernel

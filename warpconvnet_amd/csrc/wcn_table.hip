@@ -892,9 +892,19 @@ thread_local int64_t* g_box = nullptr;        // pinned, coherent, mapped
 thread_local hipEvent_t g_box_done = nullptr;
 thread_local int g_box_device = -1;
 thread_local int64_t g_box_sequence = 0;
+thread_local int64_t g_box_open = 0;  // the sequence of a write that is on its way and that nobody has collected
 }  // namespace
 
 int wcn_mailbox_begin(int64_t** device_visible_box, int64_t* sequence) {
+  // A write that nobody has collected (an error between a call and its read) may be on its way still, on another stream
+  // than this call's: its words would land among this call's.  Until it has landed there is no mailbox.
+  if (g_box_open != 0 && *(volatile int64_t*)g_box != g_box_open) {
+    const hipError_t earlier = hipPeekAtLastError();  // of the caller's launches: not to be lost
+    const hipError_t e = hipEventQuery(g_box_done);
+    if (e != hipSuccess && earlier == hipSuccess) (void)hipGetLastError();
+    if (e == hipErrorNotReady) return WCN_ERR_LAUNCH;
+  }
+  g_box_open = 0;
   int device = 0;
   if (hipGetDevice(&device) != hipSuccess) return WCN_ERR_LAUNCH;
   if (!g_box) {
@@ -920,8 +930,9 @@ int wcn_mailbox_begin(int64_t** device_visible_box, int64_t* sequence) {
 }
 
 int wcn_mailbox_mark(hipStream_t stream) {
-  if (!g_box_done) return WCN_ERR_LAUNCH;
-  return hipEventRecord(g_box_done, stream) == hipSuccess ? WCN_OK : WCN_ERR_LAUNCH;
+  if (!g_box_done || hipEventRecord(g_box_done, stream) != hipSuccess) return WCN_ERR_LAUNCH;
+  g_box_open = g_box_sequence;
+  return WCN_OK;
 }
 
 int wcn_mailbox_end(void* host_dst, size_t payload_bytes, int64_t sequence, bool kernel_over) {
@@ -942,6 +953,7 @@ int wcn_mailbox_end(void* host_dst, size_t payload_bytes, int64_t sequence, bool
   }
   __atomic_thread_fence(__ATOMIC_ACQUIRE);
   memcpy(host_dst, (const void*)(g_box + 1), payload_bytes);
+  if (g_box_open == sequence) g_box_open = 0;
   return WCN_OK;
 }
 
@@ -966,6 +978,7 @@ int wcn_thread_release(void) {
   g_small_done = g_early_done = g_box_done = nullptr;
   g_small_staging = g_early_staging = nullptr;
   g_box = nullptr;
+  g_box_open = 0;
   g_small_device = g_early_device = g_box_device = -1;
   g_early_src = nullptr;
   return st;
