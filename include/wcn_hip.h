@@ -485,6 +485,11 @@ int wcn_sparse_conv_dgrad(const void* grad_out, int64_t num_out, int32_t c_out, 
 size_t wcn_conv_wgrad_workspace_bytes(int32_t num_offsets, int32_t c_in, int32_t c_out,
                                       int64_t num_pairs, int64_t identity_rows);
 
+/* Pairs that a workgroup adds up for 16-bit rows of whole 16-byte vectors (host arithmetic; 0 for arguments that are none):
+ * with the order of a chunk's pairs, what decides the order of the additions. */
+int64_t wcn_conv_wgrad_chunk_pairs(const int64_t* host_offsets, int32_t num_offsets, int32_t identity_offset,
+                                   int64_t identity_rows, int32_t c_in, int32_t c_out);
+
 /* grad_weight is (K, c_in, c_out) in weight_dtype (the feature dtype or fp32). */
 int wcn_sparse_conv_wgrad(const void* features, int64_t num_in, int32_t c_in, const void* grad_out,
                           int64_t num_out, int32_t c_out, int32_t dtype, const int32_t* in_maps,

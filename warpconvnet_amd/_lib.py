@@ -108,6 +108,7 @@ SIGNATURES = {
                                                  _vp, _i32, _vp, _i64, _vp, _sz, _vp]),
     "wcn_morton_codes": (ctypes.c_int, [_vp, _i64, _i32, _i32, _vp, _i32p, _vp, _vp]),
     "wcn_conv_wgrad_workspace_bytes": (_sz, [_i32, _i32, _i32, _i64, _i64]),
+    "wcn_conv_wgrad_chunk_pairs": (_i64, [_i64p, _i32, _i32, _i64, _i32, _i32]),
     "wcn_sparse_conv_wgrad": (ctypes.c_int, [_vp, _i64, _i32, _vp, _i64, _i32, _i32, _vp, _vp, _i64p,
                                              _i32, _i32, _vp, _i32, _vp, _sz, _vp]),
     "wcn_sparse_conv_wgrad_bias": (ctypes.c_int, [_vp, _i64, _i32, _vp, _i64, _i32, _i32, _vp, _vp, _i64p, _vp, _i32, _i32,

@@ -300,6 +300,52 @@ inline int64_t wgrad_pairs_per_chunk(int64_t pairs, int K, int c_in, int c_out) 
   return std::min<int64_t>((p + KP - 1) / KP * KP, 1 << 30);
 }
 
+struct WgradChunking {
+  int64_t per, most;  // pairs per chunk; chunks of the XCD that has most of them (-1: too many to number)
+};
+
+// Where some XCD has more chunks than it holds at once, chunks get longer until none has, if a round of those takes less time
+// than the rounds that it replaces take with the chunks' mean length (an offset's last chunk is short).  Wide rows leave few workgroups
+// for a chunk's place: there a chunk per offset may be too many already.  us, 3x3x3 on rooms, bf16, first length / longer:
+//     256 -> 256  24,000 rows   66 /  52 (1.06 times as long)    3,000 rows   34 /  31 (1.2)
+//     256 -> 512  24,000       118 / 128 (1.95; two rounds of mean length are 1.7)     100,000   359 / 423 (1.98)
+//     512 -> 512  24,000       194 / 236 (none has fitted at 2.2)                      300,000   1,980 / 2,490
+//     384 -> 384  24,000       130 / 137
+// (1024 -> 1024 over 20,000 rows, whose partial sums are 270 MB, 690 / 610: a third less of them.)
+WgradChunking wgrad_chunking(const int64_t* host_offsets, int K, int identity, int64_t identity_rows, int c_in, int c_out) {
+  int64_t pairs = 0, chunks = 0;  // of all offsets
+  auto most_of = [&](int64_t per) -> int64_t {
+    int64_t here[8] = {}, most = 0;
+    pairs = chunks = 0;
+    for (int k = 0; k < K; ++k) {
+      const int64_t n = k == identity ? identity_rows : host_offsets[k + 1] - host_offsets[k];
+      const int64_t W = (n + per - 1) / per;
+      if (W >= 65536) return -1;  // see conv_wgrad_tiles
+      pairs += n;
+      chunks += W;
+      for (int x = 0; x < 8; ++x) here[x] += wgrad_first_chunk(x + 1, (int)W, k) - wgrad_first_chunk(x, (int)W, k);
+    }
+    for (int x = 0; x < 8; ++x) most = std::max(most, here[x]);
+    return most > INT32_MAX / 8 ? -1 : most;
+  };
+  const int64_t tiles = (int64_t)(padded(c_in) / (32 * blocks_of(c_in))) * (padded(c_out) / (32 * blocks_of(c_out)));
+  const int64_t room = wgrad_slots(c_in, c_out) / 8 / tiles;
+  WgradChunking first;
+  first.per = wgrad_pairs_per_chunk(host_offsets[K] + identity_rows, K, c_in, c_out);
+  first.most = most_of(first.per);
+  if (first.most <= room || room < 1) return first;
+  const int64_t limit = (first.most + room - 1) / room * pairs / chunks;
+  if (most_of(1 << 30) > room) return first;
+  int64_t per = first.per;
+  for (int turn = 0; turn < 16; ++turn) {
+    per = std::min<int64_t>((per + per / 24) / KP * KP + KP, 1 << 30);
+    if (per >= limit) break;
+    const int64_t most = most_of(per);
+    if (most <= room) return {per, most};
+  }
+  return first;
+}
+
 template <typename T, int NI, int NO>
 int launch_wgrad_tiles(const WgradTileArgs& a, hipStream_t s) {
   constexpr int lds = 2 * (Side<NI>::BYTES + Side<NO>::BYTES) + 2 * SEGMENT * 4;
@@ -346,6 +392,16 @@ bool wcn_wgrad_tiles_takes(int dtype, int c_in, int c_out, const void* features,
   return dtype != WCN_DTYPE_F32 && c_in % 8 == 0 && c_out % 8 == 0 && (uintptr_t)features % 16 == 0 && (uintptr_t)grad_out % 16 == 0;
 }
 
+extern "C" int64_t wcn_conv_wgrad_chunk_pairs(const int64_t* host_offsets, int32_t num_offsets, int32_t identity_offset,
+                                              int64_t identity_rows, int32_t c_in, int32_t c_out) {
+  if (!host_offsets || num_offsets < 1 || num_offsets > WCN_MAX_OFFSETS || c_in < 8 || c_out < 8 || c_in % 8 || c_out % 8 ||
+      identity_offset >= num_offsets || identity_rows < 0 || host_offsets[0] != 0 || host_offsets[num_offsets] > INT32_MAX)
+    return 0;
+  for (int k = 0; k < num_offsets; ++k)
+    if (host_offsets[k + 1] < host_offsets[k]) return 0;
+  return wgrad_chunking(host_offsets, num_offsets, identity_offset, identity_offset >= 0 ? identity_rows : 0, c_in, c_out).per;
+}
+
 size_t wcn_wgrad_tiles_partial_bytes(int num_offsets, int c_in, int c_out, int64_t pairs) {
   const int64_t chunks = pairs / wgrad_pairs_per_chunk(pairs, num_offsets, c_in, c_out) + num_offsets;
   return wcn_align256(sizeof(float) * (size_t)chunks * padded(c_in) * padded(c_out));
@@ -373,24 +429,11 @@ int wcn_wgrad_tiles_launch(const void* features, int64_t num_in, int c_in, const
   a.identity = identity;
   a.tiles_in = a.c_in_pad / (32 * blocks_of(c_in));
   a.tiles_out = a.c_out_pad / (32 * blocks_of(c_out));
-  // The device computes the same numbers from the same inputs.  Chunks get longer until every XCD holds its own at once.
-  int64_t per = wgrad_pairs_per_chunk(host_offsets[num_offsets] + a.identity_rows, num_offsets, c_in, c_out);
-  const int64_t room = wgrad_slots(c_in, c_out) / 8 / ((int64_t)a.tiles_in * a.tiles_out);
-  for (int turn = 0;; ++turn) {
-    int64_t here[8] = {}, most = 0;
-    for (int k = 0; k < num_offsets; ++k) {
-      const int64_t n = k == identity ? a.identity_rows : host_offsets[k + 1] - host_offsets[k];
-      const int64_t W = (n + per - 1) / per;  // fewer than 65,536: see wgrad_pairs_per_chunk
-      if (W >= 65536) return WCN_ERR_INVALID_ARGUMENT;
-      for (int x = 0; x < 8; ++x) here[x] += wgrad_first_chunk(x + 1, (int)W, k) - wgrad_first_chunk(x, (int)W, k);
-    }
-    for (int x = 0; x < 8; ++x) most = std::max(most, here[x]);
-    if (most > INT32_MAX / 8) return WCN_ERR_INVALID_ARGUMENT;
-    a.chunks = (int)most;
-    if (most <= room || turn == 16 || per >= (1 << 30)) break;
-    per = std::min<int64_t>((per + per / 24) / KP * KP + KP, 1 << 30);
-  }
-  a.pairs_per_chunk = (int)per;
+  // The device computes the same numbers from the same inputs.
+  const WgradChunking plan = wgrad_chunking(host_offsets, num_offsets, identity, a.identity_rows, c_in, c_out);
+  if (plan.most < 0) return WCN_ERR_INVALID_ARGUMENT;
+  a.chunks = (int)plan.most;
+  a.pairs_per_chunk = (int)plan.per;
   const int st = dtype == WCN_DTYPE_F16 ? launch_in<_Float16>(a, s) : launch_in<__bf16>(a, s);
   if (st != WCN_OK) return st;
   const int planes = num_offsets * (a.c_in_pad * a.c_out_pad / 256);
