@@ -134,8 +134,17 @@ def test_tiles_get_wider_when_the_cus_are_taken(oracle, dtype, c_in, c_out, rows
     (torch.float32, 96, 96, 24_000, 60, (3, 3, 3), "conv_fwd_pack<float"), (torch.float32, 128, 40, 48_000, 60, (3, 3, 3), "conv_fwd_pack<float"),
     (torch.float32, 36, 64, 45_000, 60, (3, 3, 3), "conv_fwd_pack<float"), (torch.float32, 160, 64, 12_000, 40, (3, 3, 3), "conv_fwd_small<float, 4, 8"),
     (torch.float32, 64, 64, 2500, 30, (5, 5, 5), "conv_fwd_small<float, 2, 16"), (torch.float16, 256, 256, 12_000, 50, (3, 3, 3), "conv_fwd_ring<"),
-    (torch.float16, 128, 128, 12_000, 50, (2, 2, 2), "conv_fwd_small<f16, 4, 8")],
-    ids=["f32_three_slices", "f32_four_slices", "f32_part_of_a_slice", "f32_five_slices", "f32_k5", "f16_ring", "f16_k2"])
+    (torch.float16, 128, 128, 12_000, 50, (2, 2, 2), "conv_fwd_small<f16, 4, 8"),
+    # narrow layers: what comes behind is the kernel of their own, or the pair-packed one where their weights are too many for it
+    (torch.float32, 16, 16, 49_000, 70, (5, 5, 5), "conv_fwd_small<float, 1, 8"), (torch.float32, 16, 16, 51_000, 70, (5, 5, 5), "conv_fwd_group<float, 1, true, 2"),
+    (torch.float32, 16, 16, 55_000, 70, (3, 3, 3), "conv_fwd_small<float, 1, 8"), (torch.float32, 16, 16, 58_000, 70, (3, 3, 3), "conv_fwd_group<float, 1, true, 1"),
+    (torch.float32, 32, 16, 44_000, 70, (3, 3, 3), "conv_fwd_small<float, 1, 8"), (torch.float32, 32, 16, 46_000, 70, (3, 3, 3), "conv_fwd_group<float, 1, false"),
+    (torch.float32, 12, 32, 48_000, 70, (3, 3, 3), "conv_fwd_small<float, 2, 8"), (torch.float32, 12, 32, 50_000, 70, (3, 3, 3), "conv_fwd_group<float, 2, true"),
+    (torch.bfloat16, 16, 32, 90_000, 90, (4, 4, 4), "conv_fwd_small<bf16, 2, 8"), (torch.bfloat16, 16, 32, 95_000, 90, (4, 4, 4), "conv_fwd_pack<"),
+    (torch.bfloat16, 16, 16, 66_000, 80, (4, 4, 4), "conv_fwd_group<bf16, 1, true")],
+    ids=["f32_three_slices", "f32_four_slices", "f32_part_of_a_slice", "f32_five_slices", "f32_k5", "f16_ring", "f16_k2", "f32_narrow_k5_below",
+         "f32_narrow_k5_above", "f32_narrow_below", "f32_narrow_above", "f32_32_16_below", "f32_32_16_above", "f32_12_32_below", "f32_12_32_above",
+         "bf16_narrow_k4_below", "bf16_narrow_k4_above", "bf16_narrow_k4_group"])
 def test_lines_between_the_kernels(oracle, dtype, c_in, c_out, rows, extent, ksize, kernel):
     got, want, name = _run(oracle, dtype, c_in, c_out, rows, extent, ksize, residual=True)
     assert name.startswith(kernel), name

@@ -119,6 +119,7 @@ int wcn_wgrad_tiles_launch(const void* features, int64_t num_in, int c_in, const
 #endif  // WCN_CONV_ARGS_H_
 
 // The contraction for narrow layers (wcn_conv_group.hip): a wave per group of 64 output rows.
+bool wcn_conv_group_shape(int dtype, int num_offsets, int c_in, int c_out);  // what it asks of the layer alone
 bool wcn_conv_group_takes(const ConvArgs& a, int dtype);
 int wcn_conv_group_launch(const ConvArgs& a, int dtype, hipStream_t stream);
 

@@ -447,10 +447,10 @@ bool group_instance_fits(int K) {
 }
 
 template <typename T>
-bool group_fits(const ConvArgs& a) {
-  if (a.c_in <= 16) return a.c_out <= 16 ? group_instance_fits<T, 1, true>(a.K) : group_instance_fits<T, 2, true>(a.K);
-  if (a.c_out <= 16) return group_instance_fits<T, 1, false>(a.K);
-  return !std::is_same<T, float>::value && group_instance_fits<T, 2, false>(a.K);
+bool group_fits(int K, int c_in, int c_out) {
+  if (c_in <= 16) return c_out <= 16 ? group_instance_fits<T, 1, true>(K) : group_instance_fits<T, 2, true>(K);
+  if (c_out <= 16) return group_instance_fits<T, 1, false>(K);
+  return !std::is_same<T, float>::value && group_instance_fits<T, 2, false>(K);
 }
 
 }  // namespace
@@ -467,15 +467,18 @@ bool group_fits(const ConvArgs& a) {
 //   5x5x5 16 -> 16 over 100 k and 1 M: 51, 48 / 108, 114 and 320, 407 / 539, 573
 // (with rows requested 8 blocks ahead).  What bounds it: a wave's groups one after the other, 25-30 us each whatever the number of waves beside it (two waves a group,
 // sixteen output channels each: the same).  32 -> 32 leaves LDS for six waves, which is faster in the first round only: not taken.
+bool wcn_conv_group_shape(int dtype, int K, int c_in, int c_out) {
+  if (K > 128 || c_in > 32 || c_out > 32 || c_in % (c_in <= 16 ? 4 : 8) != 0) return false;
+  return dtype == WCN_DTYPE_F32   ? group_fits<float>(K, c_in, c_out)
+         : dtype == WCN_DTYPE_F16 ? group_fits<_Float16>(K, c_in, c_out) : group_fits<__bf16>(K, c_in, c_out);
+}
+
 bool wcn_conv_group_takes(const ConvArgs& a, int dtype) {
   const bool fp32 = dtype == WCN_DTYPE_F32;
   if (!a.vec_in || a.split || !a.group_start || a.G <= 0 || a.num_pairs <= 0) return false;
-  if (a.c_in > 32 || a.c_out > 32 || a.c_in % (a.c_in <= 16 ? 4 : 8) != 0) return false;
   if ((uint64_t)a.num_in * (uint64_t)a.c_in * (fp32 ? 4u : 2u) >= (1ull << 32)) return false;
-  if (a.K > 128 || (int64_t)a.K * (a.G + 1) >= (1ll << 31) || a.num_pairs >= (1ll << 30) ||
-      a.num_in > (1ll << 24))
-    return false;
-  return fp32 ? group_fits<float>(a) : dtype == WCN_DTYPE_F16 ? group_fits<_Float16>(a) : group_fits<__bf16>(a);
+  if ((int64_t)a.K * (a.G + 1) >= (1ll << 31) || a.num_pairs >= (1ll << 30) || a.num_in > (1ll << 24)) return false;
+  return wcn_conv_group_shape(dtype, a.K, a.c_in, a.c_out);
 }
 
 int wcn_conv_group_launch(const ConvArgs& a, int dtype, hipStream_t s) {
