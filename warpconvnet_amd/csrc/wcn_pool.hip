@@ -219,7 +219,7 @@ __global__ void __launch_bounds__(256) rows_from_groups(const int32_t* __restric
   __shared__ int32_t s_first[4][64];
   __shared__ int32_t s_shift[4][OFFSETS];  // the place of an offset's first pair in the lists, less its place among the group's
   __shared__ int32_t s_begin[4][OFFSETS];  // the latter
-  __shared__ uint8_t s_mark[4][CHUNK];     // of CHUNK of the group's pairs: offset + 1 where a run begins
+  __shared__ uint32_t s_mark[4][CHUNK / 4];  // a byte for each of CHUNK of the group's pairs: offset + 1 where a run begins
   const int tid = threadIdx.x, lane = wcn_lane(), wave = tid >> 6;
   if (blockIdx.x == 0)  // counters of whatever follows on the stream
     for (int i = tid; i < clear_words; i += 256) clear[i] = 0;
@@ -257,19 +257,19 @@ __global__ void __launch_bounds__(256) rows_from_groups(const int32_t* __restric
   int k[ROUNDS], in[ROUNDS];
   int64_t row[ROUNDS];
   auto request = [&](int p0) {  // pairs p0 .. p0 + CHUNK - 1 of the group
-    uint32_t* const marks = reinterpret_cast<uint32_t*>(s_mark[wave]);
-    for (int i = lane; i < CHUNK / 4; i += 64) marks[i] = 0u;
+    uint8_t* const mark = reinterpret_cast<uint8_t*>(s_mark[wave]);
+    for (int i = lane; i < CHUNK / 4; i += 64) s_mark[wave][i] = 0u;
     written();
 #pragma unroll
     for (int h = 0; h < (ONE ? 1 : 2); ++h) {
       const int o = lane + 64 * h;
       const int at = o < K ? s_begin[wave][o] - p0 : -1;
-      if (at >= 0 && at < CHUNK && s_begin[wave][o] >= 0) s_mark[wave][at] = (uint8_t)(o + 1);
+      if (at >= 0 && at < CHUNK && s_begin[wave][o] >= 0) mark[at] = (uint8_t)(o + 1);
     }
     written();
 #pragma unroll
     for (int u = 0; u < ROUNDS; ++u) {
-      int v = max((int)s_mark[wave][u * 64 + lane], lane == 0 ? carry : 0);
+      int v = max((int)mark[u * 64 + lane], lane == 0 ? carry : 0);
       // running maximum over the lanes, as wcn_wave_inclusive_sum
       v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false));
       v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false));
