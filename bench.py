@@ -734,7 +734,7 @@ def main():
             # the bytes the survey's formula prices for it
             "map_build": {
                 "kernel": "table_hist + table_colscan + table_scatter + table_bins + " + map_kernels
-                          + " + kmap_scan_rows + " + ("kmap_emit_flat" if "kmap_pass" in map_kernels else "self_count + self_emit"),
+                          + " + kmap_scan_rows + " + ("kmap_emit<8>" if "kmap_pass" in map_kernels else "self_count + self_emit"),
                 "probe_kernel": map_kernels,
                 "bound": "hbm",
                 "achieved": map_bytes / (map_ms * 1e-3) / 1e9,

@@ -70,7 +70,7 @@ struct OffsetsByValue {
 // Wf holds the same values for the kernel that loads them straight into MFMA operands
 // (wcn_conv_split.hip): per offset, block of 16 n and 128-byte slice of c, the eight 16-byte pieces of
 // the slice one after the other, each for the 16 n: a wave's operand load is then 1 KiB in one piece.
-// A thread makes one 16-byte piece: n fastest over the threads, so that reads of W are coalesced.
+// A thread makes one 16-byte piece, a wave 16 n x 4 pieces of one k.
 template <typename T, typename WT>
 __global__ void __launch_bounds__(256) conv_prep_weight(const WT* __restrict__ W, int K, int c_in,
                                                         int c_out, int c_in_pad, int c_out_pad,

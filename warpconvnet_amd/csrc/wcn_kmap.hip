@@ -1225,7 +1225,7 @@ __global__ void __launch_bounds__(256) stride_fill_cells(const int4* __restrict_
   __shared__ int32_t s_before[SCANNED ? 1 : CELLS_PARTS + 1];  // (first workgroup) coarse rows before a part
   const int tid = threadIdx.x, lane = wcn_lane(), wave = tid >> 6;
   const int part = (int)blockIdx.x, parts = (int)gridDim.x;
-  const int64_t i = (int64_t)part * 256 + tid, group = i >> 6;
+  const int64_t i = (int64_t)part * 256 + tid;
   const int4 c = coords[i < n ? i : n - 1];
   unsigned long long wins[4];
 #pragma unroll

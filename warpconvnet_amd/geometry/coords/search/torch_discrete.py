@@ -79,9 +79,10 @@ def _kernel_map_from_table(table: TorchHashTable, out_coords: Tensor, kernel_siz
     network differ a lot: 4 pairs per voxel of a scene's surface at the finest level, 14 two levels
     down).  By-product the contraction reuses: the per-64-row group starts of every offset, (K, G + 1)
     int32, behind the map's K + 1 offsets as int64 at the head of the builder's workspace; that head
-    (about K * M / 16 bytes) is what stays with the map.  The probe results behind it are K * M * 4
-    bytes: above _KEEP_WORKSPACE_BYTES the head is copied and the workspace goes back to the allocator,
-    below, the map keeps the workspace as it is and the step has no copy in it."""
+    (about K * M / 16 bytes) is what stays with the map.  The probe results behind it (a row's number and a
+    tag for each) are K * M * 6 bytes: above _KEEP_WORKSPACE_BYTES (3x3x3: 1.6 M rows) the head is copied and
+    the workspace goes back to the allocator, below, the map keeps the workspace as it is and the step has no
+    copy in it."""
     out4 = _four_columns(out_coords)
     M = out4.shape[0]
     ks, st = _pad_kernel_args(kernel_size, 1), _pad_kernel_args(stride, 1)
