@@ -14,7 +14,7 @@
 // once for every 64 channels of the other side.)  Piece p (16 bytes) of row r sits at p ^ f(r), f even, so that the sixteen
 // 32-byte runs of a transposing read lie in different banks; the source side arranges it.
 //
-// What bounds it: the gathered rows (6 to 7 TB/s behind the L2; matrix pipes 12 to 22 %) and, for a few thousand pairs per offset, the partial sums (64 KB per chunk).
+// What bounds it: the gathered rows (5.4 to 6.4 TB/s behind the L2, which hits 24 to 44 %; matrix pipes 8 to 25 %) and, for a few thousand pairs per offset, the partial sums (64 KB per chunk).
 // A stage of 3x3x3 96 -> 96 over 300 k rows and 128 -> 128 over 170 k with its 2x2x2 layers, bf16, all four weight gradients:
 // 667 -> 285 us (91, 107, 30 and 29, reductions 27); with the rows of dY shared in the XCDs' L2s (wgrad_first_chunk) 232 (74, 80, 25 and
 // 28), where every row of dY came from behind the L2 for every offset.

@@ -141,7 +141,8 @@ __global__ void __launch_bounds__(256) kmap_pass(const WcnTableHeader* __restric
 // stays short; a round's row is stored when the next round's has been requested.
 // Against a mask, a rank and two predicated accesses per offset and lane: 3x3x3 over 1 M rows of rooms 85.5 -> 79.5 us, 5x5x5
 // 228 -> 187 (2,990 vector instructions a wave where 27 and 125 offsets' worth of 64-bit ranks took most of the time).  What bounds it
-// now: instruction issue (29 % of the wave cycles) and the texture addresser (61 % busy), both with scattered requests.
+// now: scattered requests (3x3x3 and 5x5x5: texture addresser 58 and 51 % busy, L1s waiting for the L2 54 and 57 % of the cycles, waves half
+// of theirs; vector issue slots 32 and 34 % used).
 template <int KX, int KY, int KZ>
 __global__ void __launch_bounds__(256) kmap_pass_fixed(const WcnTableHeader* __restrict__ hdr,
                                                        const WcnSlot* __restrict__ slots,
