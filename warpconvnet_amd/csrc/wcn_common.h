@@ -7,31 +7,44 @@
 #include "../../include/wcn_hip.h"
 
 #define WCN_WAVE 64
-#define WCN_MAX_PROBE 128  // linear-probe bound of the block table (insert and lookup)
 #define WCN_EMPTY_KEY 0xFFFFFFFFFFFFFFFFull
+#define WCN_EMPTY_TAG 0xFFFFFFFFu
 #define WCN_MAX_OFFSETS 1024  // kernel volume bound of the kernel-map kernels
 
-// Device-recorded conditions (TableHeader::status, a bit set).
+// Conditions of a table that its build records (a bit set).
 #define WCN_DEV_OVERFLOW 1
 #define WCN_DEV_RANGE 2
 
 // ---- coordinate table -------------------------------------------------------------------------
 // The table does not store one slot per voxel.  Space is cut into 4x4x4-voxel blocks; a slot
-// holds the packed block coordinate, a 64-bit occupancy mask of the block and the rank of its
+// holds a tag of the packed block coordinate, a 64-bit occupancy mask of the block and the rank of its
 // first voxel in `perm`, the list of input rows grouped by block.  A voxel's row index is
-// perm[base + popcount(mask below its bit)].  One 32-byte slot answers up to 64 probes.
-struct __attribute__((aligned(32))) WcnSlot {
-  unsigned long long key;   // packed (batch, bx, by, bz) relative to the bounding box, or EMPTY
+// perm[base + popcount(mask below its bit)].  One 16-byte slot, one request, answers up to 64 probes.
+// The tag is the block coordinate itself where that fits 31 bits (4096 x 4096 x 2048 voxels and 8 batch items do), else 31 bits
+// of a hash of it: then the coordinates lie beside the slots, 8 bytes each, and a look-up compares them too.
+// The slots come in regions of WCN_BIN_SLOTS, one per bin of the build: every block of a 16x16x16-voxel cell is in the
+// region that the cell's hash names, so a region is made by one workgroup, in LDS, and written from end to end: no slot is
+// cleared beforehand and none is claimed with an atomic.
+struct __attribute__((aligned(16))) WcnSlot {
+  uint32_t tag;             // or WCN_EMPTY_TAG
+  uint32_t base;            // first position of the block's voxels in perm, | WCN_SLOT_PASSED where the search for another goes on
   unsigned long long mask;  // bit (x&3)*16 + (y&3)*4 + (z&3)
-  int32_t base;             // first position of the block's voxels in perm
-  int32_t pad[3];
+};
+#define WCN_SLOT_PASSED 0x80000000u
+
+struct __attribute__((aligned(32))) WcnBlock {  // a line of a bin's block list
+  unsigned long long key;   // packed (batch, bx, by, bz) relative to the bounding box
+  unsigned long long mask;
+  int32_t base;
+  int32_t first;            // first entry of the block, counted from the bin's first
+  int32_t pad[2];
 };
 
 struct WcnTableHeader {  // first 256 bytes of a table workspace
   int32_t mn[4];         // bounding box of the keys, per column
   int32_t mx[4];
   int32_t num_blocks;    // occupied slots (valid after table_sum_stats)
-  int32_t status;        // WCN_DEV_* bits
+  int32_t status;        // WCN_DEV_* bits (valid after table_sum_stats)
   int32_t total;         // number of distinct keys (valid after table_sum_stats)
   int32_t num_keys;      // keys inserted; more keys than set bits (`total`) means some key came twice
   int32_t bins;          // bins of the build
@@ -46,7 +59,8 @@ static_assert(sizeof(WcnTableHeader) == 256, "header is 256 bytes");
 
 struct WcnTableView {  // host-computed addresses inside a table workspace
   WcnTableHeader* hdr;
-  WcnSlot* slots;
+  WcnSlot* slots;         // bins regions of WCN_BIN_SLOTS
+  unsigned long long* wide_keys;  // their block coordinates, where a tag does not hold them
   int32_t* perm;        // n_keys
   int32_t* slot_of;     // n_keys (slot of each key; written on request)
   // The keys in block order: every key once, the keys of one block next to each other, the blocks
@@ -54,16 +68,15 @@ struct WcnTableView {  // host-computed addresses inside a table workspace
   int32_t* order_tag;     // n_keys: (index of the entry's block in its bin's block list) << 6 | voxel bit
   int32_t* order_row;     // n_keys: input row of each entry
   // The blocks of bin b, in the order of its entries: block_list[bin_start[b] + j], j < blocks of
-  // the bin.  key, mask and base as in the table's slot; pad[0] = first entry of the block,
-  // counted from bin_start[b].
-  WcnSlot* block_list;    // n_keys places (a bin has at most as many blocks as keys)
+  // the bin.
+  WcnBlock* block_list;   // n_keys places (a bin has at most as many blocks as keys)
   // build scratch
   int32_t* bin_coords;    // (n_keys, 4) keys grouped by bin
   int32_t* bin_row;       // n_keys
   int32_t* hist;          // (bins, parts) keys of part w in bin b, then their exclusive prefix sums
   int32_t* bin_total;     // bins: keys per bin
   int32_t* bin_start;     // bins + 1
-  int32_t* bin_stats;     // (bins, 2): distinct keys and blocks of each bin
+  int32_t* bin_stats;     // (bins, 2): distinct keys of each bin; its blocks, | WCN_BIN_LOST where some found no place
   int32_t* part_box;      // (parts, 8) bounding box of each part's keys
   int64_t n_keys;
   int64_t capacity;
@@ -76,7 +89,8 @@ static inline size_t wcn_align256(size_t x) { return (x + 255) & ~(size_t)255; }
 // Keys are first grouped into bins of one to two thousand (a bin is a hash of the key's 16x16x16-voxel
 // cell, so the 4x4x4 blocks of a cell stay together); the bin count follows the slot count, so a
 // rebuild with more slots also re-deals the bins.
-#define WCN_BIN_SLOTS 2048      // distinct blocks a bin can hold (its table in LDS)
+#define WCN_BIN_SLOTS 2048      // slots of a bin's region: the distinct blocks it can hold
+#define WCN_BIN_LOST (1 << 30)
 #define WCN_PART_KEYS 4096      // keys per workgroup of the histogram and scatter passes
 #define WCN_MAX_BINS 32768      // a counter per bin in LDS during the build: 128 KB
 static inline int32_t wcn_table_bins(int64_t capacity) {
@@ -100,7 +114,9 @@ static inline size_t wcn_table_layout(void* base, int64_t n_keys, int64_t capaci
   if (v) v->hdr = (WcnTableHeader*)(p + off);
   off += 256;
   if (v) v->slots = (WcnSlot*)(p + off);
-  off += wcn_align256(sizeof(WcnSlot) * (size_t)capacity);
+  off += sizeof(WcnSlot) * WCN_BIN_SLOTS * (size_t)bins;
+  if (v) v->wide_keys = (unsigned long long*)(p + off);
+  off += sizeof(unsigned long long) * WCN_BIN_SLOTS * (size_t)bins;
   if (v) v->perm = (int32_t*)(p + off);
   off += wcn_align256(sizeof(int32_t) * (size_t)n_keys);
   if (v) v->slot_of = (int32_t*)(p + off);
@@ -109,8 +125,8 @@ static inline size_t wcn_table_layout(void* base, int64_t n_keys, int64_t capaci
   off += wcn_align256(sizeof(int32_t) * (size_t)n_keys);
   if (v) v->order_row = (int32_t*)(p + off);
   off += wcn_align256(sizeof(int32_t) * (size_t)n_keys);
-  if (v) v->block_list = (WcnSlot*)(p + off);
-  off += wcn_align256(sizeof(WcnSlot) * (size_t)n_keys);
+  if (v) v->block_list = (WcnBlock*)(p + off);
+  off += wcn_align256(sizeof(WcnBlock) * (size_t)n_keys);
   if (v) v->bin_coords = (int32_t*)(p + off);
   off += wcn_align256(sizeof(int32_t) * 4 * (size_t)n_keys);
   if (v) v->bin_row = (int32_t*)(p + off);
@@ -142,6 +158,7 @@ struct WcnLayout {
   uint32_t span[4];   // largest valid (coord - amin) per column
   uint32_t shift[4];  // left shift of each field in the key
   bool ok;            // all fields fit in 63 bits
+  bool wide;          // ... but not in 31
 };
 
 __device__ __forceinline__ WcnLayout wcn_make_layout(const WcnTableHeader* __restrict__ h) {
@@ -160,7 +177,9 @@ __device__ __forceinline__ WcnLayout wcn_make_layout(const WcnTableHeader* __res
   L.shift[2] = bits[3];
   L.shift[1] = bits[3] + bits[2];
   L.shift[0] = bits[3] + bits[2] + bits[1];
-  L.ok = (bits[0] + bits[1] + bits[2] + bits[3]) <= 63u;
+  const uint32_t total = bits[0] + bits[1] + bits[2] + bits[3];
+  L.ok = total <= 63u;
+  L.wide = total > 31u;
   return L;
 }
 
@@ -184,45 +203,99 @@ __device__ __forceinline__ uint32_t wcn_block_bit(const uint32_t r[4]) {
   return ((r[1] & 3u) << 4) | ((r[2] & 3u) << 2) | (r[3] & 3u);
 }
 
-// Slot of a block key: the key's two halves folded into one word, then the 32-bit finaliser of
-// MurmurHash3 (neighbouring block keys spread over the table; a third of the instructions of a
-// 64-bit mix, and every probe of the kernel-map passes pays for it).
-__device__ __forceinline__ uint32_t wcn_mix(unsigned long long k, uint32_t cap_mask) {
-  uint32_t h = (uint32_t)k ^ ((uint32_t)(k >> 32) * 0x9E3779B1u);
-  h ^= h >> 16;
-  h *= 0x85ebca6bu;
-  h ^= h >> 13;
-  h *= 0xc2b2ae35u;
-  h ^= h >> 16;
-  return h & cap_mask;
+// Hash of the 16x16x16-voxel cell that holds a block, from the block's absolute coordinates (block boundaries are multiples of
+// four in absolute coordinates: the table's origin is rounded down to one): the sum of a term per column, finalised.  One
+// multiplication does: bins and places are as even as with two (rooms, spheres, full cubes, grids of step 8 to 64).
+__device__ __forceinline__ uint32_t wcn_cell_batch(uint32_t batch) { return batch * 0x9E3779B1u; }
+__device__ __forceinline__ uint32_t wcn_cell_x(int32_t block) { return (uint32_t)(block >> 2) * 0x85EBCA77u; }
+__device__ __forceinline__ uint32_t wcn_cell_y(int32_t block) { return (uint32_t)(block >> 2) * 0xC2B2AE3Du; }
+__device__ __forceinline__ uint32_t wcn_cell_z(int32_t block) { return (uint32_t)(block >> 2) * 0x27D4EB2Fu; }
+__device__ __forceinline__ uint32_t wcn_cell_hash(uint32_t sum) {
+  sum ^= sum >> 16;
+  sum *= 0xC2B2AE35u;
+  return sum ^ (sum >> 15);
 }
 
-// Finds the slot of a block key.  Returns its mask (0 if the block is absent) and base.  Both
-// 16-byte halves of the 32-byte slot are requested together, so a hit costs one memory round trip.
-__device__ __forceinline__ unsigned long long wcn_lookup_block_from(
-    const WcnSlot* __restrict__ slots, uint32_t cap_mask, unsigned long long key, uint32_t h,
-    int first_probe, int32_t* base) {
-  for (int p = first_probe; p < WCN_MAX_PROBE; ++p) {
-    const uint4* raw = reinterpret_cast<const uint4*>(&slots[h]);
-    const uint4 lo = raw[0];
-    const uint4 hi = raw[1];
-    const unsigned long long k = ((unsigned long long)lo.y << 32) | lo.x;
-    if (k == key) {
-      *base = (int32_t)hi.x;
-      return ((unsigned long long)lo.w << 32) | lo.z;
+// Where a block is looked for: in its bin's region, first at its place in the line of 128 bytes of its 8x8x8-voxel cell (a
+// row's neighbourhood lies in 3.4 blocks but in 2 lines on average), then in another line (wcn_probe_slot).  The eight
+// lines of a larger cell, and a line's eight places, are turned by the larger cell's hash (exclusive or with the sum of a word per
+// dimension).  Lines that follow one another, and a search of the line's other places, were slower: the blocks
+// of a dense cell stand in each other's way (up to 50 slots looked at for the slowest lane of a wave, 2 this way).  A second place
+// anywhere in the region: 66 us for the probe pass of 1 M voxels of rooms instead of 59; the blocks of a cell that gives way to another
+// stay in one line this way.
+__device__ __forceinline__ uint32_t wcn_place_x(int32_t block) { return ((block & 2) ? 0x95u << 3 : 0u) | (uint32_t)(block & 1) << 2; }
+__device__ __forceinline__ uint32_t wcn_place_y(int32_t block) { return ((block & 2) ? 0x4Eu << 3 : 0u) | (uint32_t)(block & 1) << 1; }
+__device__ __forceinline__ uint32_t wcn_place_z(int32_t block) { return ((block & 2) ? 0x2Bu << 3 : 0u) | (uint32_t)(block & 1); }
+__device__ __forceinline__ uint32_t wcn_home_slot(uint32_t cell, uint32_t place, uint32_t bin_mask) {
+  return (cell & bin_mask) * WCN_BIN_SLOTS | (((cell >> 16) ^ place) & (WCN_BIN_SLOTS - 1));
+}
+static_assert(WCN_BIN_SLOTS == 2048 && WCN_MAX_BINS <= 32768, "places from bits 16 to 26 of the hash, bins from bits 0 to 14");
+__device__ __forceinline__ uint32_t wcn_home_slot_of(int32_t batch, int32_t bx, int32_t by, int32_t bz, uint32_t bin_mask) {
+  return wcn_home_slot(wcn_cell_hash(wcn_cell_batch((uint32_t)batch) + wcn_cell_x(bx) + wcn_cell_y(by) + wcn_cell_z(bz)),
+                       wcn_place_x(bx) ^ wcn_place_y(by) ^ wcn_place_z(bz), bin_mask);
+}
+// The p-th slot of the search: the same place of another line, then nine slots further and further; with p up to WCN_BIN_SLOTS
+// all of the region's.
+__device__ __forceinline__ uint32_t wcn_probe_slot(uint32_t home, int p) {
+  if (p == 0) return home;
+  return (home & ~(uint32_t)(WCN_BIN_SLOTS - 1)) | (((home ^ (0xB5u << 3)) + 9u * (uint32_t)(p - 1)) & (WCN_BIN_SLOTS - 1));
+}
+
+// What a slot's tag says of a block key (never WCN_EMPTY_TAG).
+__device__ __forceinline__ uint32_t wcn_block_tag(const WcnLayout& L, unsigned long long key) {
+  return L.wide ? ((uint32_t)(key ^ (key >> 31)) * 0x9E3779B1u) >> 1 : (uint32_t)key;
+}
+
+struct WcnTableRef {  // what a look-up reads
+  const WcnSlot* __restrict__ slots;
+  const unsigned long long* __restrict__ wide_keys;  // read only where the layout is wide
+  uint32_t bin_mask;
+};
+
+inline WcnTableRef wcn_table_ref(const WcnTableView& v) { return {v.slots, v.wide_keys, (uint32_t)v.bins - 1u}; }
+
+// Finds the slot of a block key from probe `p` on.  Returns its mask (0 if the block is absent) and base.
+__device__ __forceinline__ unsigned long long wcn_lookup_block_from(const WcnLayout& L, const WcnTableRef& t,
+                                                                    unsigned long long key, uint32_t home, int p,
+                                                                    int32_t* base) {
+  const uint32_t tag = wcn_block_tag(L, key);
+  for (; p <= WCN_BIN_SLOTS; ++p) {
+    const uint32_t h = wcn_probe_slot(home, p);
+    const uint4 s = *reinterpret_cast<const uint4*>(&t.slots[h]);
+    if (s.x == tag && (!L.wide || t.wide_keys[h] == key)) {
+      *base = (int32_t)(s.y & ~WCN_SLOT_PASSED);
+      return ((unsigned long long)s.w << 32) | s.z;
     }
-    if (k == WCN_EMPTY_KEY) break;
-    h = (h + 1) & cap_mask;
+    if (!(s.y & WCN_SLOT_PASSED)) break;
   }
   *base = 0;
   return 0ull;
 }
 
-__device__ __forceinline__ unsigned long long wcn_lookup_block(const WcnSlot* __restrict__ slots,
-                                                               uint32_t cap_mask,
-                                                               unsigned long long key,
+// The block at relative coordinates (batch, x, y, z in blocks) within the box.
+__device__ __forceinline__ uint32_t wcn_home_of_relative(const WcnLayout& L, uint32_t rb, uint32_t bx, uint32_t by, uint32_t bz,
+                                                          uint32_t bin_mask) {
+  return wcn_home_slot_of((int32_t)(rb + L.amin[0]), ((int32_t)L.amin[1] >> 2) + (int32_t)bx,
+                          ((int32_t)L.amin[2] >> 2) + (int32_t)by, ((int32_t)L.amin[3] >> 2) + (int32_t)bz, bin_mask);
+}
+// The block of a voxel at relative coordinates r.
+__device__ __forceinline__ unsigned long long wcn_lookup_block(const WcnLayout& L, const WcnTableRef& t, const uint32_t r[4],
                                                                int32_t* base) {
-  return wcn_lookup_block_from(slots, cap_mask, key, wcn_mix(key, cap_mask), 0, base);
+  return wcn_lookup_block_from(L, t, wcn_block_key(L, r), wcn_home_of_relative(L, r[0], r[1] >> 2, r[2] >> 2, r[3] >> 2, t.bin_mask),
+                               0, base);
+}
+
+// The table's WCN_DEV_* bits, by all `threads` (>= 64, a multiple of 64) of a workgroup; `shared`: 16 words of LDS.
+__device__ __forceinline__ int wcn_table_status(const WcnTableHeader* __restrict__ h, int tid, int threads, int32_t* shared) {
+  const int32_t* stats = reinterpret_cast<const int32_t*>(reinterpret_cast<const char*>(h) + h->stats_offset);
+  int lost = 0;
+  for (int b = tid; b < h->bins; b += threads) lost |= stats[2 * b + 1] & WCN_BIN_LOST;
+  const bool any = __ballot(lost != 0) != 0ull;
+  if ((tid & 63) == 0) shared[tid >> 6] = any ? 1 : 0;
+  __syncthreads();
+  int all = 0;
+  for (int w = 0; w < threads / 64; ++w) all |= shared[w];
+  return (all ? WCN_DEV_OVERFLOW : 0) | (h->num_keys > 0 && !wcn_make_layout(h).ok ? WCN_DEV_RANGE : 0);
 }
 
 __device__ __forceinline__ int wcn_rank_below(unsigned long long mask, uint32_t bit) {

@@ -28,7 +28,7 @@ struct KmapGeom {
 };
 
 struct KmapWorkspace {  // host-computed addresses inside a kmap workspace
-  int64_t* result;      // [0..K] offsets, [K+1] = table status bits, [K+2] = occupied slots | duplicates << 32
+  int64_t* result;      // [0..K] offsets, [K+1] = table status bits, [K+2] = occupied slots | duplicates << 32 | status << 33
   int64_t* row_total;   // [K+1] totals of the rows of `groups`
   int32_t* ticket;      // arrival counter of the scan's workgroups (zeroed by the probe pass)
   int32_t* groups;      // (K+1, G+1): rows 0..K-1 per-offset hit counts of each 64-row group, row K
@@ -74,8 +74,7 @@ struct KmapProbe {      // what the probe pass leaves for the scan and the emit 
 // Probe results are produced offset by offset; consecutive offsets differ in z (the fastest
 // digit) and mostly fall in the block of the previous probe, whose slot is kept in registers.
 __global__ void __launch_bounds__(256) kmap_pass(const WcnTableHeader* __restrict__ hdr,
-                                                 const WcnSlot* __restrict__ slots,
-                                                 uint32_t cap_mask,
+                                                 WcnTableRef table,
                                                  const int32_t* __restrict__ perm,
                                                  const int4* __restrict__ out_coords,
                                                  int64_t num_out, KmapGeom g,
@@ -108,7 +107,7 @@ __global__ void __launch_bounds__(256) kmap_pass(const WcnTableHeader* __restric
         if (usable && r[1] <= L.span[1] && r[2] <= L.span[2] && r[3] <= L.span[3]) {
           const unsigned long long key = wcn_block_key(L, r);
           if (key != cached_key) {
-            cached_mask = wcn_lookup_block(slots, cap_mask, key, &cached_base);
+            cached_mask = wcn_lookup_block(L, table, r, &cached_base);
             cached_key = key;
           }
           const uint32_t bit = wcn_block_bit(r);
@@ -133,30 +132,32 @@ __global__ void __launch_bounds__(256) kmap_pass(const WcnTableHeader* __restric
 // Phase 1 requests the (up to) 8 block slots the neighbourhood can touch, all at once, so their
 // memory latencies overlap (3x3x3 over 2 k rows 12.6 -> 9.4 us, over 1 M 89 -> 83, 5x5x5 over 1 M 245 -> 231, against
 // eight conditional requests that waited for one another), and keeps them in LDS as half blocks: 32 bits of
-// occupancy and the position of their first voxel in `perm`.
+// occupancy and the position of their first voxel in `perm`.  INSIDE: 2x2x2 neighbourhoods that begin at even places lie in one
+// block (270 k rows of rooms 15.5 -> 8 us).
 // Phase 2 takes the KZ offsets of a (x, y) row of the kernel out of the two words that hold them, and appends a tag
 // (offset, lane) per hit to the wave's list, in the order in which pairs are parked.
 // Phase 3 empties the list 64 hits at a time, a lane per HIT: position in `perm` from the half block of the hit's own row, the row
 // from there, and both stores full.  Phases 2 and 3 alternate over a few rows of the kernel, so that the list
 // stays short; a round's row is stored when the next round's has been requested.
 // Against a mask, a rank and two predicated accesses per offset and lane: 3x3x3 over 1 M rows of rooms 85.5 -> 79.5 us, 5x5x5
-// 228 -> 187 (2,990 vector instructions a wave where 27 and 125 offsets' worth of 64-bit ranks took most of the time).  What bounds it
-// now: scattered requests (3x3x3 and 5x5x5: texture addresser 58 and 51 % busy, L1s waiting for the L2 54 and 57 % of the cycles, waves half
-// of theirs; vector issue slots 32 and 34 % used).
-template <int KX, int KY, int KZ>
+// 228 -> 187 (2,990 vector instructions a wave where 27 and 125 offsets' worth of 64-bit ranks took most of the time).  What bound it
+// then were scattered requests (texture addresser 58 and 51 % busy, L1s waiting for the L2 54 and 57 % of the cycles): one of 16 bytes
+// for two of 16 and 4 changed nothing, slots of neighbouring blocks in one line (wcn_home_slot) and regions without displaced blocks
+// took 3x3x3 from 86 to 59 and 5x5x5 from 189 to 140.  An array asked with the number of a block that was not at its place lay in
+// memory, 32 bytes a lane written on every path: 5 us of both.
+template <int KX, int KY, int KZ, bool INSIDE>
 __global__ void __launch_bounds__(256) kmap_pass_fixed(const WcnTableHeader* __restrict__ hdr,
-                                                       const WcnSlot* __restrict__ slots,
-                                                       uint32_t cap_mask,
+                                                       WcnTableRef table,
                                                        const int32_t* __restrict__ perm,
                                                        const int4* __restrict__ out_coords,
                                                        int64_t num_out, KmapGeom g,
                                                        int32_t* __restrict__ groups, int64_t G,
                                                        KmapProbe o) {
-  constexpr int K = KX * KY * KZ, ROWS = KX * KY;
+  constexpr int K = KX * KY * KZ, ROWS = KX * KY, CAND = INSIDE ? 1 : 8;
   static_assert(KX <= 5 && KY <= 5 && KZ <= 5, "a kernel of up to five voxels spans at most two blocks per dimension");
   constexpr int TURN = 10 / KZ < ROWS ? 10 / KZ : ROWS;  // rows of the kernel between two visits to the list
   constexpr int LIST = 64 * TURN * KZ + 64;              // all of them hit, and up to 63 left over
-  __shared__ uint2 s_half[16][256];  // [block * 2 + upper half of x][thread]: occupancy, position of the first voxel
+  __shared__ uint2 s_half[INSIDE ? 2 : 16][256];  // [block * 2 + upper half of x][thread]: occupancy, position of the first voxel
   __shared__ uint16_t s_list[4][LIST];
   __shared__ uint8_t s_sub[256];     // place of the first neighbour in its block: x | y << 2 | z << 4
   __shared__ int32_t s_count[4][K + 1];
@@ -187,49 +188,80 @@ __global__ void __launch_bounds__(256) kmap_pass_fixed(const WcnTableHeader* __r
     cok[d][0] = cand[d][0] <= lim;
     cok[d][1] = (cand[d][1] <= lim) & (((r0[d] & 3u) + (uint32_t)(KD[d] - 1)) >= 4u);
   }
+  // candidate e's block coordinates where e is no constant (an array asked with it would lie in memory)
+  auto block_at = [&](int d, int e) { return (cand[d][0] + ((uint32_t)e >> (2 - d) & 1u)) & 0x3FFFFFFFu; };
   auto block_key = [&](int e) {
-    return ((unsigned long long)rb << L.shift[0]) |
-           ((unsigned long long)((e & 4) ? cand[0][1] : cand[0][0]) << L.shift[1]) |
-           ((unsigned long long)((e & 2) ? cand[1][1] : cand[1][0]) << L.shift[2]) |
-           (unsigned long long)((e & 1) ? cand[2][1] : cand[2][0]);
+    return ((unsigned long long)rb << L.shift[0]) | ((unsigned long long)block_at(0, e) << L.shift[1]) |
+           ((unsigned long long)block_at(1, e) << L.shift[2]) | (unsigned long long)block_at(2, e);
   };
-  unsigned long long key[8];
-  uint32_t hh[8];
-  bool need[8];
-  typedef uint32_t Half __attribute__((ext_vector_type(4)));
-  Half lo[8];
-  int32_t hi[8];  // only the base is needed of a slot's second half: a 4-byte load
+  uint32_t tag[CAND], home[CAND];
+  bool need[CAND];
+  typedef uint32_t Slot4 __attribute__((ext_vector_type(4)));
+  Slot4 slot[CAND];
 #pragma unroll
-  for (int e = 0; e < 8; ++e) {
-    need[e] = usable & cok[0][e >> 2] & cok[1][(e >> 1) & 1] & cok[2][e & 1];
-    key[e] = block_key(e);
-    hh[e] = need[e] ? wcn_mix(key[e], cap_mask) : 0u;
+  for (int e = 0; e < CAND; ++e) need[e] = usable & cok[0][e >> 2] & cok[1][(e >> 1) & 1] & cok[2][e & 1];
+  {
+    // the candidates' absolute block coordinates: terms of the cells' hash, and places in cell and line (wcn_home_slot)
+    uint32_t term[3][2], place[3][2];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int32_t x = ((int32_t)L.amin[1] >> 2) + (int32_t)cand[0][j], y = ((int32_t)L.amin[2] >> 2) + (int32_t)cand[1][j],
+                    z = ((int32_t)L.amin[3] >> 2) + (int32_t)cand[2][j];
+      term[0][j] = wcn_cell_batch((uint32_t)c.x) + wcn_cell_x(x);
+      term[1][j] = wcn_cell_y(y);
+      term[2][j] = wcn_cell_z(z);
+      place[0][j] = wcn_place_x(x);
+      place[1][j] = wcn_place_y(y);
+      place[2][j] = wcn_place_z(z);
+    }
+#pragma unroll
+    for (int e = 0; e < CAND; ++e) {
+      const int x = e >> 2, y = (e >> 1) & 1, z = e & 1;
+      home[e] = wcn_home_slot(wcn_cell_hash(term[0][x] + term[1][y] + term[2][z]), place[0][x] ^ place[1][y] ^ place[2][z],
+                              table.bin_mask);
+    }
+  }
+  if (!L.wide) {  // keys of 31 bits (one that lies in the box: the fields of another may overflow, and it is not asked for)
+    const uint32_t fx[2] = {rb << L.shift[0] | cand[0][0] << L.shift[1], rb << L.shift[0] | cand[0][1] << L.shift[1]};
+    const uint32_t fy[2] = {cand[1][0] << L.shift[2], cand[1][1] << L.shift[2]};
+#pragma unroll
+    for (int e = 0; e < CAND; ++e) tag[e] = fx[e >> 2] | fy[(e >> 1) & 1] | cand[2][e & 1];
+  } else {
+#pragma unroll
+    for (int e = 0; e < CAND; ++e) tag[e] = wcn_block_tag(L, block_key(e));
   }
   // Every lane reads, those without a need the table's first slot: behind a condition each of the eight
-  // requests waited for the one before it.
+  // requests waited for the one before it.  Blocks that another has put out of their place (one in twelve) are looked
+  // for at their second place, all together; the few that are not there either one after the other.
+  uint32_t left = 0;
 #pragma unroll
-  for (int e = 0; e < 8; ++e) {
-    lo[e] = *reinterpret_cast<const Half*>(&slots[hh[e]]);
-    hi[e] = slots[hh[e]].base;
+  for (int e = 0; e < CAND; ++e) left |= need[e] ? 1u << e : 0u;
+#pragma unroll
+  for (int round = 0; round < 2; ++round) {
+    if (round > 0 && __ballot(left != 0) == 0ull) break;
+#pragma unroll
+    for (int e = 0; e < CAND; ++e)
+      slot[e] = *reinterpret_cast<const Slot4*>(&table.slots[(left >> e) & 1u ? wcn_probe_slot(home[e], round) : 0u]);
+#pragma unroll
+    for (int e = 0; e < CAND; ++e) asm volatile("" : "+v"(slot[e]));
+#pragma unroll
+    for (int e = 0; e < CAND; ++e) {
+      bool same = (left >> e & 1u) & (slot[e].x == tag[e]);
+      if (L.wide && same) same = table.wide_keys[wcn_probe_slot(home[e], round)] == block_key(e);
+      if (same | !(slot[e].y & WCN_SLOT_PASSED)) left &= ~(1u << e);
+      if (round == 0 || same) {
+        const uint32_t base = slot[e].y & ~WCN_SLOT_PASSED;
+        s_half[2 * e][tid] = make_uint2(same ? slot[e].z : 0u, base);
+        s_half[2 * e + 1][tid] = make_uint2(same ? slot[e].w : 0u, base + (uint32_t)__popc(slot[e].z));
+      }
+    }
   }
-#pragma unroll
-  for (int e = 0; e < 8; ++e) asm volatile("" : "+v"(lo[e]), "+v"(hi[e]));
-  uint32_t walk = 0;  // collided on the first probe
-#pragma unroll
-  for (int e = 0; e < 8; ++e) {
-    const unsigned long long k0 = ((unsigned long long)lo[e].y << 32) | lo[e].x;
-    const bool same = need[e] && k0 == key[e];
-    if (need[e] && !same && k0 != WCN_EMPTY_KEY) walk |= 1u << e;
-    s_half[2 * e][tid] = make_uint2(same ? lo[e].z : 0u, (uint32_t)hi[e]);
-    s_half[2 * e + 1][tid] = make_uint2(same ? lo[e].w : 0u, (uint32_t)hi[e] + (uint32_t)__popc(lo[e].z));
-  }
-  while (walk != 0) {
-    const int e = __ffs((int)walk) - 1;
-    walk &= walk - 1;
-    const unsigned long long wanted = block_key(e);
+  while (left != 0) {
+    const int e = __ffs((int)left) - 1;
+    left &= left - 1;
     int32_t base = 0;
-    const unsigned long long mask =
-        wcn_lookup_block_from(slots, cap_mask, wanted, (wcn_mix(wanted, cap_mask) + 1) & cap_mask, 1, &base);
+    const uint32_t first = wcn_home_of_relative(L, rb, block_at(0, e), block_at(1, e), block_at(2, e), table.bin_mask);
+    const unsigned long long mask = wcn_lookup_block_from(L, table, block_key(e), first, 2, &base);
     s_half[2 * e][tid] = make_uint2((uint32_t)mask, (uint32_t)base);
     s_half[2 * e + 1][tid] = make_uint2((uint32_t)(mask >> 32), (uint32_t)base + (uint32_t)__popc((uint32_t)mask));
   }
@@ -255,7 +287,7 @@ __global__ void __launch_bounds__(256) kmap_pass_fixed(const WcnTableHeader* __r
     const uint32_t sub = s_sub[src];
     const uint32_t ax = (sub & 3u) + (uint32_t)(k / (KY * KZ)), ay = ((sub >> 2) & 3u) + (uint32_t)(k / KZ % KY),
                    az = (sub >> 4) + (uint32_t)(k % KZ);
-    const uint2 half = s_half[((ax >> 2) << 3) | ((ay >> 2) << 2) | ((az >> 2) << 1) | ((ax >> 1) & 1u)][src];
+    const uint2 half = s_half[INSIDE ? (ax >> 1) & 1u : ((ax >> 2) << 3) | ((ay >> 2) << 2) | ((az >> 2) << 1) | ((ax >> 1) & 1u)][src];
     const uint32_t bit = ((ax & 1u) << 4) | ((ay & 3u) << 2) | (az & 3u);
     const uint32_t at = half.y + (uint32_t)__popc(__builtin_amdgcn_ubfe(half.x, 0u, bit));
     const int32_t row = perm[mine ? at : 0u];
@@ -272,8 +304,8 @@ __global__ void __launch_bounds__(256) kmap_pass_fixed(const WcnTableHeader* __r
       const int row = row0 + r;
       if (ROWS % TURN != 0 && row >= ROWS) break;
       const uint32_t ax = (r0[0] & 3u) + (uint32_t)(row / KY), ay = (r0[1] & 3u) + (uint32_t)(row % KY);
-      const uint32_t e = ((ax >> 2) << 3) | ((ay >> 2) << 2) | ((ax >> 1) & 1u), bit = ((ax & 1u) << 4) | ((ay & 3u) << 2);
-      const uint32_t near = __builtin_amdgcn_ubfe(s_half[e][tid].x, bit, 4u), far = __builtin_amdgcn_ubfe(s_half[e + 2][tid].x, bit, 4u);
+      const uint32_t e = INSIDE ? (ax >> 1) & 1u : ((ax >> 2) << 3) | ((ay >> 2) << 2) | ((ax >> 1) & 1u), bit = ((ax & 1u) << 4) | ((ay & 3u) << 2);
+      const uint32_t near = __builtin_amdgcn_ubfe(s_half[e][tid].x, bit, 4u), far = INSIDE ? 0u : __builtin_amdgcn_ubfe(s_half[INSIDE ? 0 : e + 2][tid].x, bit, 4u);
       const uint32_t hit = (near | (far << 4)) >> (r0[2] & 3u);
 #pragma unroll
       for (int kk = 0; kk < KZ; ++kk) {
@@ -410,7 +442,7 @@ __device__ __forceinline__ int kmap_nth_set_bit(unsigned long long mask, int r) 
 __global__ void kmap_zero_ticket(int32_t* ticket) { *ticket = 0; }
 
 struct KmapFinish {  // null `result`: no finishing step
-  int64_t* result;              // [0..K] offsets, [K+1] table status bits, [K+2] occupied slots | duplicates << 32
+  int64_t* result;              // [0..K] offsets, [K+1] table status bits, [K+2] occupied slots | duplicates << 32 | status << 33
   int32_t* ticket;              // zero before the launch; left at zero
   const WcnTableHeader* hdr;
   int32_t K;
@@ -422,7 +454,7 @@ __global__ void __launch_bounds__(1024) kmap_scan_rows(int32_t* __restrict__ gro
                                                        int64_t* __restrict__ row_total,
                                                        KmapFinish fin) {
   __shared__ int s_wave[16];
-  __shared__ int s_stat[2][16];
+  __shared__ int s_stat[3][16];
   int32_t* row = groups + (int64_t)blockIdx.x * (G + 1);
   const int lane = wcn_lane(), wave = threadIdx.x >> 6;
   if (fin.result && blockIdx.x == 0) {
@@ -433,10 +465,13 @@ __global__ void __launch_bounds__(1024) kmap_scan_rows(int32_t* __restrict__ gro
     const int32_t bins = fin.hdr->bins;
     const int32_t* stats = reinterpret_cast<const int32_t*>(reinterpret_cast<const char*>(fin.hdr) + fin.hdr->stats_offset);
     int voxels = 0, occupied = 0;
+    bool lost = false;
     for (int i = threadIdx.x; i < bins; i += 1024) {
       voxels += stats[2 * i];
-      occupied += stats[2 * i + 1];
+      occupied += stats[2 * i + 1] & ~WCN_BIN_LOST;
+      lost |= (stats[2 * i + 1] & WCN_BIN_LOST) != 0;
     }
+    const bool any_lost = __ballot(lost) != 0ull;
 #pragma unroll
     for (int sft = 32; sft > 0; sft >>= 1) {
       voxels += __shfl_xor(voxels, sft, 64);
@@ -445,16 +480,19 @@ __global__ void __launch_bounds__(1024) kmap_scan_rows(int32_t* __restrict__ gro
     if (lane == 0) {
       s_stat[0][wave] = voxels;
       s_stat[1][wave] = occupied;
+      s_stat[2][wave] = any_lost ? WCN_DEV_OVERFLOW : 0;
     }
     __syncthreads();
     if (threadIdx.x == 0) {
       voxels = occupied = 0;
+      int status = fin.hdr->num_keys > 0 && !wcn_make_layout(fin.hdr).ok ? WCN_DEV_RANGE : 0;
       for (int w = 0; w < 16; ++w) {
         voxels += s_stat[0][w];
         occupied += s_stat[1][w];
+        status |= s_stat[2][w];
       }
       // written before this thread's ticket (and the fence in front of it) further down
-      fin.result[fin.K + 2] = (int64_t)occupied | ((int64_t)(voxels != fin.hdr->num_keys ? 1 : 0) << 32);
+      fin.result[fin.K + 2] = (int64_t)occupied | ((int64_t)(voxels != fin.hdr->num_keys ? 1 : 0) << 32) | (int64_t)status << 33;
     }
   }
   int64_t carry = 0;
@@ -521,9 +559,9 @@ __global__ void __launch_bounds__(1024) kmap_scan_rows(int32_t* __restrict__ gro
     run += __shfl(v, 63, 64);
   }
   if (lane == 0) {
-    const int64_t status = fin.hdr->status;
-    // occupied slots | duplicates << 32: left there by the first workgroup (see the top)
+    // occupied slots | duplicates << 32 | status << 33: left there by the first workgroup (see the top)
     const int64_t blocks = __hip_atomic_load(&fin.result[fin.K + 2], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const int64_t status = blocks >> 33;
     fin.result[0] = 0;
     fin.result[fin.K + 1] = status;
     if (fin.mailbox) {
@@ -656,11 +694,11 @@ constexpr int SELF_TILE = 32;
 constexpr int SELF_LIST = 1024;  // found rows fetched per turn of a workgroup
 template <int R>
 __global__ void __launch_bounds__(256) self_probe(const WcnTableHeader* __restrict__ hdr,
-                                                  const WcnSlot* __restrict__ slots, uint32_t cap_mask,
+                                                  WcnTableRef table,
                                                   const int32_t* __restrict__ perm,
                                                   const int32_t* __restrict__ bin_start,
                                                   const int32_t* __restrict__ bin_stats,
-                                                  const WcnSlot* __restrict__ block_list,
+                                                  const WcnBlock* __restrict__ block_list,
                                                   const int32_t* __restrict__ order_tag,
                                                   const int32_t* __restrict__ order_row,
                                                   uint32_t* __restrict__ hm_out,
@@ -679,7 +717,7 @@ __global__ void __launch_bounds__(256) self_probe(const WcnTableHeader* __restri
   const int tid = threadIdx.x, lane = wcn_lane(), wave = tid >> 6;
   if (blockIdx.x == 0 && blockIdx.y == 0 && tid == 0) *ticket = 0;
   const int bin = blockIdx.x;
-  const int lo = bin_start[bin], entries = bin_start[bin + 1] - lo, blocks = bin_stats[2 * bin + 1];
+  const int lo = bin_start[bin], entries = bin_start[bin + 1] - lo, blocks = bin_stats[2 * bin + 1] & ~WCN_BIN_LOST;
   const WcnLayout L = wcn_make_layout(hdr);
   if (!L.ok) return;
   const uint32_t lim[3] = {L.span[1] >> 2, L.span[2] >> 2, L.span[3] >> 2};
@@ -744,7 +782,7 @@ __global__ void __launch_bounds__(256) self_probe(const WcnTableHeader* __restri
         s_task[at++] = (uint16_t)((lane << 5) | n);
       }
       if (lane == 63) s_tasks = incl;
-      if (lane == 0) s_first[nblk] = j0 + nblk < blocks ? block_list[lo + j0 + nblk].pad[0] : entries;
+      if (lane == 0) s_first[nblk] = j0 + nblk < blocks ? block_list[lo + j0 + nblk].first : entries;
     }
     __syncthreads();
     // the tile's first round of entries is requested now and used in step 3
@@ -764,7 +802,9 @@ __global__ void __launch_bounds__(256) self_probe(const WcnTableHeader* __restri
                                       ((unsigned long long)(s_coord[t][2] + (uint32_t)dy) << L.shift[2]) |
                                       (unsigned long long)(s_coord[t][3] + (uint32_t)dz);
       int32_t base = 0;
-      s_nmask[t][n] = wcn_lookup_block(slots, cap_mask, nkey, &base);
+      const uint32_t home = wcn_home_of_relative(L, s_coord[t][0], s_coord[t][1] + (uint32_t)dx, s_coord[t][2] + (uint32_t)dy,
+                                                 s_coord[t][3] + (uint32_t)dz, table.bin_mask);
+      s_nmask[t][n] = wcn_lookup_block_from(L, table, nkey, home, 0, &base);
       s_nbase[t][n] = base;
     }
     __syncthreads();
@@ -1031,19 +1071,22 @@ inline bool table_args_ok(const void* table, int64_t n_keys, int64_t capacity) {
 void launch_probe(const WcnTableView& v, const int32_t* out_coords, int64_t num_out,
                   const KmapGeom& g, const KmapWorkspace& w, hipStream_t s) {
   const dim3 grid(grid_for(num_out, 256)), block(256);
-  const uint32_t cap_mask = (uint32_t)(v.capacity - 1);
+  const WcnTableRef table = wcn_table_ref(v);
   const KmapProbe o = {w.found, w.tags, w.ticket};
   if (is_fixed_size(g, 3, 3, 3)) {
-    hipLaunchKernelGGL((kmap_pass_fixed<3, 3, 3>), grid, block, 0, s, v.hdr, v.slots, cap_mask,
+    hipLaunchKernelGGL((kmap_pass_fixed<3, 3, 3, false>), grid, block, 0, s, v.hdr, table,
+                       v.perm, (const int4*)out_coords, num_out, g, w.groups, w.G, o);
+  } else if (is_fixed_size(g, 2, 2, 2) && g.sx % 2 == 0 && g.sy % 2 == 0 && g.sz % 2 == 0) {
+    hipLaunchKernelGGL((kmap_pass_fixed<2, 2, 2, true>), grid, block, 0, s, v.hdr, table,
                        v.perm, (const int4*)out_coords, num_out, g, w.groups, w.G, o);
   } else if (is_fixed_size(g, 2, 2, 2)) {
-    hipLaunchKernelGGL((kmap_pass_fixed<2, 2, 2>), grid, block, 0, s, v.hdr, v.slots, cap_mask,
+    hipLaunchKernelGGL((kmap_pass_fixed<2, 2, 2, false>), grid, block, 0, s, v.hdr, table,
                        v.perm, (const int4*)out_coords, num_out, g, w.groups, w.G, o);
   } else if (is_fixed_size(g, 5, 5, 5)) {
-    hipLaunchKernelGGL((kmap_pass_fixed<5, 5, 5>), grid, block, 0, s, v.hdr, v.slots, cap_mask,
+    hipLaunchKernelGGL((kmap_pass_fixed<5, 5, 5, false>), grid, block, 0, s, v.hdr, table,
                        v.perm, (const int4*)out_coords, num_out, g, w.groups, w.G, o);
   } else {
-    hipLaunchKernelGGL(kmap_pass, grid, block, 0, s, v.hdr, v.slots, cap_mask, v.perm,
+    hipLaunchKernelGGL(kmap_pass, grid, block, 0, s, v.hdr, table, v.perm,
                        (const int4*)out_coords, num_out, g, w.groups, w.G, o);
   }
 }
@@ -1127,8 +1170,8 @@ __global__ void __launch_bounds__(256) stride_pick(const int4* __restrict__ coar
       c = coarse[i];
       uint32_t r[4];
       wcn_relative(L, c.x, c.y, c.z, c.w, r);
-      const ulonglong2 km = *reinterpret_cast<const ulonglong2*>(&slots[h]);
-      const int64_t pos = (int64_t)slots[h].base + wcn_rank_below(km.y, wcn_block_bit(r));
+      const WcnSlot slot = slots[h];
+      const int64_t pos = (int64_t)(slot.base & ~WCN_SLOT_PASSED) + wcn_rank_below(slot.mask, wcn_block_bit(r));
       winner = pos >= 0 && pos < n && perm[pos] == (int32_t)i;
     }
   }
@@ -1158,8 +1201,7 @@ constexpr int CELLS_PARTS = 4096;  // of 256 rows
 
 __global__ void __launch_bounds__(256) stride_count_cells(const int4* __restrict__ coords, int64_t n,
                                                           const WcnTableHeader* __restrict__ hdr,
-                                                          const WcnSlot* __restrict__ slots,
-                                                          uint32_t cap_mask,
+                                                          WcnTableRef table,
                                                           const int32_t* __restrict__ perm,
                                                           int lx, int ly, int lz,
                                                           int32_t* __restrict__ counts,
@@ -1179,7 +1221,7 @@ __global__ void __launch_bounds__(256) stride_count_cells(const int4* __restrict
     uint32_t r[4];
     if (L.ok && wcn_relative(L, c.x, c.y, c.z, c.w, r)) {
       int32_t base = 0;
-      const unsigned long long mask = wcn_lookup_block(slots, cap_mask, wcn_block_key(L, r), &base);
+      const unsigned long long mask = wcn_lookup_block(L, table, r, &base);
       // the bits of the block that lie in this row's coarse cell
       const uint32_t x0 = (r[1] & 3u) >> lx << lx, y0 = (r[2] & 3u) >> ly << ly, z0 = (r[3] & 3u) >> lz << lz;
       const unsigned long long zs = ((1ull << (1 << lz)) - 1ull) << z0;          // within a row of 4 bits
@@ -1254,6 +1296,8 @@ __global__ void __launch_bounds__(256) stride_fill_cells(const int4* __restrict_
     first_index[pos] = (int32_t)i;
   }
   if (part != 0) return;
+  __shared__ int32_t s_lost[4];
+  const int status = wcn_table_status(hdr, tid, 256, s_lost);
   if (!SCANNED) {
     __syncthreads();  // s_wave has been read
     int v[PER], sum = 0;
@@ -1298,7 +1342,7 @@ __global__ void __launch_bounds__(256) stride_fill_cells(const int4* __restrict_
   }
   if (tid == 0) {
     put(0, total);
-    put(1, hdr->status);
+    put(1, status);
   }
   if (res.mailbox) {  // everything is in the mailbox before the word that the host polls
     __threadfence_system();
@@ -1307,16 +1351,20 @@ __global__ void __launch_bounds__(256) stride_fill_cells(const int4* __restrict_
   }
 }
 
-__global__ void stride_finish(int64_t* __restrict__ result, const int32_t* __restrict__ groups,
+__global__ void __launch_bounds__(1024) stride_finish(int64_t* __restrict__ result, const int32_t* __restrict__ groups,
                               int64_t G, const WcnTableHeader* __restrict__ hdr) {
-  if (threadIdx.x != 0 || blockIdx.x != 0) return;
+  __shared__ int32_t s_lost[16];
+  const int status = wcn_table_status(hdr, (int)threadIdx.x, 1024, s_lost);
+  if (threadIdx.x != 0) return;
   result[0] = groups[G];
-  result[1] = hdr->status;
+  result[1] = status;
 }
 
 // (no rows at all)
 __global__ void __launch_bounds__(1024) stride_no_rows(int64_t* __restrict__ result, const WcnTableHeader* __restrict__ hdr) {
-  for (int b = threadIdx.x; b < 4 + STRIDE_BATCH_MARKS; b += 1024) result[b] = b == 1 ? hdr->status : 0;
+  __shared__ int32_t s_lost[16];
+  const int status = wcn_table_status(hdr, (int)threadIdx.x, 1024, s_lost);
+  for (int b = threadIdx.x; b < 4 + STRIDE_BATCH_MARKS; b += 1024) result[b] = b == 1 ? status : 0;
 }
 
 // Where the coarse rows of each batch item begin, for rows whose batch column does not descend
@@ -1455,15 +1503,14 @@ int wcn_kmap_count_self(const void* table, int64_t n_keys, int64_t capacity,
   wcn_table_layout(const_cast<void*>(table), n_keys, capacity, &v);
   SelfWorkspace w;
   self_layout(workspace, n_keys, K, &w);
-  const uint32_t cap_mask = (uint32_t)(capacity - 1);
   // a bin of the usual size has about ten tiles; bins with more are walked in turns
   const dim3 pgrid((unsigned)v.bins, 8), cgrid((unsigned)w.C);
   if (K == 27) {
-    hipLaunchKernelGGL(self_probe<1>, pgrid, dim3(256), 0, s, v.hdr, v.slots, cap_mask, v.perm, v.bin_start,
+    hipLaunchKernelGGL(self_probe<1>, pgrid, dim3(256), 0, s, v.hdr, wcn_table_ref(v), v.perm, v.bin_start,
                        v.bin_stats, v.block_list, v.order_tag, v.order_row, w.hm, w.ptr, w.park, w.ticket);
     hipLaunchKernelGGL(self_count<27>, cgrid, dim3(SELF_CHUNK), 0, s, w.hm, n_keys, w.chunk, w.C);
   } else {
-    hipLaunchKernelGGL(self_probe<2>, pgrid, dim3(256), 0, s, v.hdr, v.slots, cap_mask, v.perm, v.bin_start,
+    hipLaunchKernelGGL(self_probe<2>, pgrid, dim3(256), 0, s, v.hdr, wcn_table_ref(v), v.perm, v.bin_start,
                        v.bin_stats, v.block_list, v.order_tag, v.order_row, w.hm, w.ptr, w.park, w.ticket);
     hipLaunchKernelGGL(self_count<125>, cgrid, dim3(SELF_CHUNK), 0, s, w.hm, n_keys, w.chunk, w.C);
   }
@@ -1591,7 +1638,7 @@ int wcn_stride_unique(const int32_t* coords, int64_t n, const int32_t host_strid
     const KmapFinish none = {nullptr, nullptr, nullptr, 0, nullptr, 0};
     hipLaunchKernelGGL(kmap_scan_rows, dim3(1), dim3(1024), 0, s, w.groups, w.G, w.result + 2, none);
   }
-  hipLaunchKernelGGL(stride_finish, dim3(1), dim3(64), 0, s, w.result, w.groups, w.G, v.hdr);
+  hipLaunchKernelGGL(stride_finish, dim3(1), dim3(1024), 0, s, w.result, w.groups, w.G, v.hdr);
   if (n > 0) {
     hipLaunchKernelGGL(stride_pick<true>, dim3(grid_for(n, 256)), dim3(256), 0, s,
                        (const int4*)w.coarse, n, v.hdr, v.slots, v.slot_of, v.perm, w.groups, w.G,
@@ -1631,14 +1678,13 @@ int wcn_stride_unique_cells(const void* table, int64_t n_keys, int64_t capacity,
   const int64_t parts = (n + 255) / 256;
   unsigned long long* picked = (unsigned long long*)((char*)counts + wcn_align256(sizeof(int32_t) * (size_t)(parts + 1)));
   int32_t* item_row = (int32_t*)((char*)picked + wcn_align256(sizeof(unsigned long long) * (size_t)((n + 63) / 64)));
-  const uint32_t cap_mask = (uint32_t)(capacity - 1);
   set_pending(Pending::none, 0, nullptr);
   if (n == 0) {
     hipLaunchKernelGGL(stride_no_rows, dim3(1), dim3(1024), 0, s, result, v.hdr);
     WCN_LAUNCH_CHECK();
     return WCN_OK;
   }
-  hipLaunchKernelGGL(stride_count_cells, dim3((unsigned)parts), dim3(256), 0, s, (const int4*)coords, n, v.hdr, v.slots, cap_mask,
+  hipLaunchKernelGGL(stride_count_cells, dim3((unsigned)parts), dim3(256), 0, s, (const int4*)coords, n, v.hdr, wcn_table_ref(v),
                      v.perm, lg[0], lg[1], lg[2], counts, picked, item_row);
   // as the kernel map's result: into this thread's mailbox, where the read calls pick it up
   StrideResult res = {result, nullptr, 0};

@@ -6,21 +6,25 @@
 // builds their masks with LDS atomics:
 //   table_hist     per part of the keys (a workgroup): keys per bin (LDS counters) and the part's
 //                  bounding box
-//   table_colscan  per bin (a wave): prefix sums over the parts; the last workgroup to finish turns
-//                  the bin totals into bin starts, merges the boxes and initialises the header
-//   table_scatter  per part: every key and its row to its place in its bin; clears the slots
-//   table_bins     per bin: block masks and entry counts in an LDS table, their prefix sums, one
-//                  64-bit CAS per BLOCK to claim a slot of the table in memory (mask and base are
-//                  plain stores), then per key: its place in block order and perm[base + rank] = row
+//   table_colscan  per bin (a wave): prefix sums over the parts
+//   table_scatter  per part: every key and its row to its place in its bin; the first workgroup merges the boxes and
+//                  writes the header
+//   table_bins     per bin: block masks and entry counts in an LDS table, their prefix sums; that table is the bin's
+//                  region of the table in memory; then per key: its place in block order and perm[base + rank] = row
+// Up to 16,384 keys one launch does all of it (table_small).
 //
 // HBM traffic per key: 16 B read twice (histogram, scatter), 20 B written and read (binned entry),
-// 20 B written (entry in block order) + 4 B (perm), plus 32 B per table slot to clear.
+// 20 B written (entry in block order) + 4 B (perm), plus 16 B per table slot.
+// What the regions gave over 1 M voxels of rooms (us, against slots of 32 bytes anywhere in the table, cleared by the first
+// launch and claimed with a 64-bit compare-and-swap per block): table_hist 13.6 -> 10.4, table_bins 29.4 -> 26, the probe passes
+// of a 3x3x3 map 86 -> 59 and of a 5x5x5 map 189 -> 140; 1,800 voxels: 14.4 in two launches -> 10.2 in one.
 #include <stdlib.h>
 #include <string.h>
 
 #include <chrono>
 #include <mutex>
 #include <thread>
+#include <type_traits>
 
 #include <algorithm>
 
@@ -28,13 +32,9 @@
 
 namespace {
 
-// Bin of a key: a hash of (batch, x >> 4, y >> 4, z >> 4).  Block boundaries are multiples of four
-// in absolute coordinates (the table's origin is rounded down to one), so a block never straddles
-// two cells.
+// Bin of a key (wcn_cell_* in wcn_common.h).
 __device__ __forceinline__ uint32_t bin_of(const int4 c, uint32_t bin_mask) {
-  const unsigned long long a = ((unsigned long long)(uint32_t)c.x << 32) | (uint32_t)(c.y >> 4);
-  const unsigned long long b = ((unsigned long long)(uint32_t)(c.z >> 4) << 32) | (uint32_t)(c.w >> 4);
-  return wcn_mix(a * 0x9E3779B97F4A7C15ull + b, bin_mask);
+  return wcn_cell_hash(wcn_cell_batch((uint32_t)c.x) + wcn_cell_x(c.y >> 2) + wcn_cell_y(c.z >> 2) + wcn_cell_z(c.w >> 2)) & bin_mask;
 }
 
 struct PartRange {
@@ -53,8 +53,7 @@ __device__ __forceinline__ PartRange part_range(int64_t n_keys, int part) {
 // scans BINS_PER_THREAD bin totals: 4 up to 4096 bins, 32 beyond.
 constexpr int SMALL_BINS = 4096;
 
-// Keys per bin of one part of the keys, the part's bounding box; the part's share of the slots is
-// set to empty on the way (each slot is two 16-byte stores, {EMPTY, 0} and {0, 0, 0, 0}).
+// Keys per bin of one part of the keys, the part's bounding box.
 // ITEMS: the keys are made here too, [batch item, x, y, z] of three columns, and written on the way (the launch that did nothing else
 // took 7.7 us over 1 M rows; with this pass 11.4 + 7.7 -> 14.8; few keys: 2.4 + 2.1 -> 2.4 and a launch less).
 struct KeysOfItems {
@@ -67,8 +66,7 @@ struct KeysOfItems {
 template <bool ITEMS>
 __global__ void __launch_bounds__(1024) table_hist(const int4* __restrict__ keys, int64_t n_keys,
                                                    int32_t bins, int32_t* __restrict__ hist,
-                                                   int32_t* __restrict__ part_box,
-                                                   WcnSlot* __restrict__ slots, int64_t capacity, KeysOfItems of) {
+                                                   int32_t* __restrict__ part_box, KeysOfItems of) {
   extern __shared__ int s_cnt[];  // [bins]
   __shared__ int64_t s_start[ITEMS ? WCN_VOXEL_MAX_BATCH + 1 : 1];
   if (ITEMS && threadIdx.x <= WCN_VOXEL_MAX_BATCH) s_start[threadIdx.x] = of.starts.start[threadIdx.x];
@@ -103,13 +101,6 @@ __global__ void __launch_bounds__(1024) table_hist(const int4* __restrict__ keys
       mn[2] = min(mn[2], c[t].z); mx[2] = max(mx[2], c[t].z);
       mn[3] = min(mn[3], c[t].w); mx[3] = max(mx[3], c[t].w);
     }
-  }
-  {
-    uint4* raw = reinterpret_cast<uint4*>(slots);
-    const int64_t items = 2 * capacity, chunk = (items + parts - 1) / parts;
-    const int64_t lo = (int64_t)part * chunk, hi = lo + chunk < items ? lo + chunk : items;
-    for (int64_t i = lo + tid; i < hi; i += 1024)
-      raw[i] = (i & 1) ? make_uint4(0u, 0u, 0u, 0u) : make_uint4(0xFFFFFFFFu, 0xFFFFFFFFu, 0u, 0u);
   }
 #pragma unroll
   for (int d = 0; d < 4; ++d) {
@@ -226,9 +217,6 @@ __global__ void __launch_bounds__(1024) table_scatter(const int4* __restrict__ k
       if (lane < 4) hdr->mn[lane] = acc;
       else if (lane < 8) hdr->mx[lane - 4] = acc;
       if (lane == 8) {
-        hdr->num_blocks = 0;
-        hdr->status = 0;
-        hdr->total = 0;
         hdr->num_keys = (int32_t)n_keys;
         hdr->bins = bins;
         hdr->stats_offset = stats_offset;
@@ -264,31 +252,46 @@ struct BinLds {
   unsigned long long mask[WCN_BIN_SLOTS];
   uint32_t cursor[WCN_BIN_SLOTS];   // entries of the block, then the next free place among them
   uint32_t base[WCN_BIN_SLOTS];     // voxels of the blocks before this one
-  int32_t where[WCN_BIN_SLOTS];     // the block's slot in the table in memory
   int32_t low[WCN_BIN_SLOTS];       // lowest row per voxel when keys repeat
   int32_t index[WCN_BIN_SLOTS];     // the block's number in the bin's block list
   int32_t part[3][16];
+  uint32_t passed[WCN_BIN_SLOTS / 32];  // slots that the search for a block that is there has gone on from
+  int32_t lost;                     // a block has found no place
 };
 
-// Entry e of the bin: claims / finds its block in the LDS table, sets its bit, counts itself.
-// Returns the block's place in the LDS table, or -1 if the table is full.
-__device__ __forceinline__ int bin_insert(BinLds* s, unsigned long long key, uint32_t bit) {
-  uint32_t h = wcn_mix(key, WCN_BIN_SLOTS - 1);
-  for (int p = 0; p < WCN_BIN_SLOTS; ++p) {
+// A key of the bin: claims / finds its block in the LDS table, sets its bit, counts itself.  The search goes as a look-up's
+// will.  Returns the block's place, or -1 if the table is full.
+__device__ __forceinline__ int bin_insert(BinLds* s, unsigned long long key, uint32_t home, uint32_t bit) {
+  for (int p = 0; p <= WCN_BIN_SLOTS; ++p) {
+    const uint32_t h = wcn_probe_slot(home, p);
     unsigned long long seen = s->key[h];
     if (seen == WCN_EMPTY_KEY) {
       seen = atomicCAS(&s->key[h], WCN_EMPTY_KEY, key);
-      if (seen == WCN_EMPTY_KEY) seen = key;
+      if (seen == WCN_EMPTY_KEY) {
+        seen = key;
+        for (int q = 0; q < p; ++q) {
+          const uint32_t on = wcn_probe_slot(home, q);
+          atomicOr(&s->passed[on >> 5], 1u << (on & 31u));
+        }
+      }
     }
     if (seen == key) {
       atomicOr(&s->mask[h], 1ull << bit);
       atomicAdd(&s->cursor[h], 1u);
       return (int)h;
     }
-    h = (h + 1) & (WCN_BIN_SLOTS - 1);
   }
   return -1;
 }
+__device__ __forceinline__ int bin_find(const BinLds* s, unsigned long long key, uint32_t home) {
+  for (int p = 0; p <= WCN_BIN_SLOTS; ++p) {
+    const uint32_t h = wcn_probe_slot(home, p);
+    if (s->key[h] == key) return (int)h;
+  }
+  return -1;
+}
+// Where the block of a key is looked for in its bin's region.
+__device__ __forceinline__ uint32_t home_in_bin(const int4 c) { return wcn_home_slot_of(c.x, c.y >> 2, c.z >> 2, c.w >> 2, 0u); }
 
 // Where a bin's entries [lo, hi) come from.
 struct BinEntries {  // as table_scatter left them
@@ -297,33 +300,34 @@ struct BinEntries {  // as table_scatter left them
   __device__ __forceinline__ int4 coords(int e) const { return keys[e]; }
   __device__ __forceinline__ int32_t row(int e) const { return rows[e]; }
 };
+template <class Keys>
 struct ListedEntries {  // the rows of a few keys, listed in LDS
-  const int4* __restrict__ keys;
+  Keys keys;
   const uint16_t* list;
   int lo;
-  __device__ __forceinline__ int4 coords(int e) const { return keys[list[e - lo]]; }
+  __device__ __forceinline__ int4 coords(int e) const { return keys(list[e - lo]); }
   __device__ __forceinline__ int32_t row(int e) const { return list[e - lo]; }
 };
 
-template <bool WANT_SLOT_OF, class Entries>
+template <bool WANT_SLOT_OF, int E, class Entries>
 __device__ __forceinline__ void build_bin(const Entries& in, int bin, int lo, int hi, const WcnLayout& L, BinLds* s,
-                                          WcnTableHeader* __restrict__ hdr, WcnSlot* __restrict__ slots,
-                                          uint32_t cap_mask, int32_t* __restrict__ order_tag,
-                                          int32_t* __restrict__ order_row, WcnSlot* __restrict__ block_list,
+                                          WcnSlot* __restrict__ slots, unsigned long long* __restrict__ wide_keys,
+                                          int32_t* __restrict__ order_tag,
+                                          int32_t* __restrict__ order_row, WcnBlock* __restrict__ block_list,
                                           int32_t* __restrict__ perm, int32_t* __restrict__ slot_of,
                                           int32_t* __restrict__ bin_stats) {
   const int tid = threadIdx.x, lane = wcn_lane(), wave = tid >> 6;
-  if (tid == 0) {
-    bin_stats[2 * bin] = 0;
-    bin_stats[2 * bin + 1] = 0;
+  uint4* const region = reinterpret_cast<uint4*>(slots + (size_t)bin * WCN_BIN_SLOTS);
+  if (lo >= hi) {
+    if (tid == 0) bin_stats[2 * bin] = bin_stats[2 * bin + 1] = 0;
+    for (int h = tid; h < WCN_BIN_SLOTS; h += 1024) region[h] = make_uint4(WCN_EMPTY_TAG, 0u, 0u, 0u);
+    return;
   }
-  if (lo >= hi) return;
   // A thread keeps its first E entries in registers from the first pass to the last (bins hold
   // one to two thousand keys: one or two entries per thread); entries beyond that are read again.
-  constexpr int E = 4;
   int4 c[E];
   int32_t row[E];
-  int where[E];
+  int where[E];  // place of the key's block << 6 | voxel bit, or -1
 #pragma unroll
   for (int t = 0; t < E; ++t) {
     const int e = lo + tid + t * 1024;
@@ -331,7 +335,7 @@ __device__ __forceinline__ void build_bin(const Entries& in, int bin, int lo, in
     c[t] = in.coords(e < hi ? e : lo);
   }
   if (!L.ok) {
-    if (tid == 0) atomicOr(&hdr->status, WCN_DEV_RANGE);
+    if (tid == 0) bin_stats[2 * bin] = bin_stats[2 * bin + 1] = 0;
     for (int e = lo + tid; e < hi; e += 1024) {
       if (WANT_SLOT_OF) slot_of[in.row(e)] = -1;
       order_row[e] = in.row(e);
@@ -343,8 +347,9 @@ __device__ __forceinline__ void build_bin(const Entries& in, int bin, int lo, in
     s->key[h] = WCN_EMPTY_KEY;
     s->mask[h] = 0ull;
     s->cursor[h] = 0u;
-    s->where[h] = -1;
   }
+  if (tid < WCN_BIN_SLOTS / 32) s->passed[tid] = 0u;
+  if (tid == 0) s->lost = 0;
   __syncthreads();
   // masks and entry counts
   bool lost = false;
@@ -354,17 +359,18 @@ __device__ __forceinline__ void build_bin(const Entries& in, int bin, int lo, in
     if (lo + tid + t * 1024 < hi) {
       uint32_t r[4];
       wcn_relative(L, c[t].x, c[t].y, c[t].z, c[t].w, r);  // always inside: the box was built from these keys
-      where[t] = bin_insert(s, wcn_block_key(L, r), wcn_block_bit(r));
-      lost |= where[t] < 0;
+      const int h = bin_insert(s, wcn_block_key(L, r), home_in_bin(c[t]), wcn_block_bit(r));
+      lost |= h < 0;
+      where[t] = h < 0 ? -1 : h << 6 | (int)wcn_block_bit(r);
     }
   }
   for (int e = lo + tid + E * 1024; e < hi; e += 1024) {
     const int4 ce = in.coords(e);
     uint32_t r[4];
     wcn_relative(L, ce.x, ce.y, ce.z, ce.w, r);
-    lost |= bin_insert(s, wcn_block_key(L, r), wcn_block_bit(r)) < 0;
+    lost |= bin_insert(s, wcn_block_key(L, r), home_in_bin(ce), wcn_block_bit(r)) < 0;
   }
-  if (lost) atomicOr(&hdr->status, WCN_DEV_OVERFLOW);  // more distinct blocks in this bin than its table holds
+  if (lost) s->lost = 1;  // more distinct blocks in this bin than its table holds
   __syncthreads();
   // Prefix sums over the table's slots, entries and voxels.  Thread t owns slots t, t + 1024, ...
   // and counts them as neighbours in the order of the sums (any fixed order will do, and this one
@@ -405,29 +411,18 @@ __device__ __forceinline__ void build_bin(const Entries& in, int bin, int lo, in
   const bool low_in_lds = total_v <= WCN_BIN_SLOTS;  // room for one word per voxel
   uint32_t re = (uint32_t)(be + ie) - se, rv = (uint32_t)(bv + iv) - sv;
   int rb = bb + ib - (int)sb;
-  // Every block claims a slot of the table in memory: one claimant per block in the whole grid,
-  // so the compare-and-swap only ever meets other blocks' keys.
-  int claimed = 0;
+  // The LDS table's places are the region's slots.
 #pragma unroll
   for (int t = 0; t < PER; ++t) {
     const int h = tid + t * 1024;
     s->cursor[h] = re;
     s->base[h] = rv;
-    if (bkey[t] != WCN_EMPTY_KEY) {
-      uint32_t g = wcn_mix(bkey[t], cap_mask);
-      int p = 0;
-      for (; p < WCN_MAX_PROBE; ++p) {
-        if (atomicCAS(&slots[g].key, WCN_EMPTY_KEY, bkey[t]) == WCN_EMPTY_KEY) break;
-        g = (g + 1) & cap_mask;
-      }
-      if (p < WCN_MAX_PROBE) {
-        slots[g].mask = bmask[t];
-        slots[g].base = lo + (int32_t)rv;
-        if (WANT_SLOT_OF) s->where[h] = (int32_t)g;
-        ++claimed;
-      } else {
-        atomicOr(&hdr->status, WCN_DEV_OVERFLOW);
-      }
+    const bool there = bkey[t] != WCN_EMPTY_KEY;
+    region[h] = there ? make_uint4(wcn_block_tag(L, bkey[t]), (uint32_t)(lo + (int32_t)rv) | (s->passed[h >> 5] >> (h & 31)) << 31, (uint32_t)bmask[t],
+                                    (uint32_t)(bmask[t] >> 32))
+                      : make_uint4(WCN_EMPTY_TAG, 0u, 0u, 0u);
+    if (there) {
+      if (L.wide) wide_keys[(size_t)bin * WCN_BIN_SLOTS + h] = bkey[t];
       // the block's line of the bin's block list (two 16-byte stores)
       uint4* line = reinterpret_cast<uint4*>(&block_list[lo + rb]);
       line[0] = make_uint4((uint32_t)bkey[t], (uint32_t)(bkey[t] >> 32), (uint32_t)bmask[t], (uint32_t)(bmask[t] >> 32));
@@ -438,7 +433,6 @@ __device__ __forceinline__ void build_bin(const Entries& in, int bin, int lo, in
     re += ne[t];
     rv += nv[t];
   }
-  (void)claimed;
   if (repeats) {
     if (low_in_lds) {
       for (int j = tid; j < total_v; j += 1024) s->low[j] = INT32_MAX;
@@ -449,19 +443,20 @@ __device__ __forceinline__ void build_bin(const Entries& in, int bin, int lo, in
   }
   __syncthreads();
   // every key to its place in block order; the row of every voxel into perm
-  auto place = [&](const int4 ce, int32_t rw, int h, int e) {
-    if (h < 0) {  // its block did not fit (overflow is flagged): the entry stays where it is
+  auto place = [&](int32_t rw, int where, int e) {
+    if (where < 0) {  // its block did not fit (overflow is flagged): the entry stays where it is
       order_tag[e] = 0;
       order_row[e] = rw;
       if (WANT_SLOT_OF) slot_of[rw] = -1;
       return;
     }
-    uint32_t r[4];
-    wcn_relative(L, ce.x, ce.y, ce.z, ce.w, r);
-    const int v = (int)s->base[h] + wcn_rank_below(s->mask[h], wcn_block_bit(r));
+    const int h = where >> 6;
+    const uint32_t bit = (uint32_t)where & 63u;
+    if (WANT_SLOT_OF) slot_of[rw] = bin * WCN_BIN_SLOTS + h;
+    const int v = (int)s->base[h] + wcn_rank_below(s->mask[h], bit);
     // without repeated keys the entries of a block are its voxels: block order is perm's order
     const int q = lo + (repeats ? (int)atomicAdd(&s->cursor[h], 1u) : v);
-    order_tag[q] = (s->index[h] << 6) | (int32_t)wcn_block_bit(r);
+    order_tag[q] = (s->index[h] << 6) | (int32_t)bit;
     order_row[q] = rw;
     if (!repeats) perm[lo + v] = rw;
     else if (low_in_lds) atomicMin(&s->low[v], rw);
@@ -470,67 +465,40 @@ __device__ __forceinline__ void build_bin(const Entries& in, int bin, int lo, in
 #pragma unroll
   for (int t = 0; t < E; ++t) {
     const int e = lo + tid + t * 1024;
-    if (e < hi) place(c[t], row[t], where[t], e);
+    if (e < hi) place(row[t], where[t], e);
   }
   for (int e = lo + tid + E * 1024; e < hi; e += 1024) {
     const int4 ce = in.coords(e);
     uint32_t r[4];
     wcn_relative(L, ce.x, ce.y, ce.z, ce.w, r);
-    const unsigned long long key = wcn_block_key(L, r);
-    uint32_t h = wcn_mix(key, WCN_BIN_SLOTS - 1);
-    int found = -1;
-    for (int p = 0; p < WCN_BIN_SLOTS && found < 0; ++p) {
-      if (s->key[h] == key) found = (int)h;
-      h = (h + 1) & (WCN_BIN_SLOTS - 1);
-    }
-    place(ce, in.row(e), found, e);
+    const int h = bin_find(s, wcn_block_key(L, r), home_in_bin(ce));
+    place(in.row(e), h < 0 ? -1 : h << 6 | (int)wcn_block_bit(r), e);
   }
   __syncthreads();
-  if (WANT_SLOT_OF) {  // the claims have landed: the slot of every key
-#pragma unroll
-    for (int t = 0; t < E; ++t) {
-      const int e = lo + tid + t * 1024;
-      if (e < hi && where[t] >= 0) slot_of[row[t]] = s->where[where[t]];
-    }
-    for (int e = lo + tid + E * 1024; e < hi; e += 1024) {
-      const int4 ce = in.coords(e);
-      uint32_t r[4];
-      wcn_relative(L, ce.x, ce.y, ce.z, ce.w, r);
-      const unsigned long long key = wcn_block_key(L, r);
-      uint32_t h = wcn_mix(key, WCN_BIN_SLOTS - 1);
-      for (int p = 0; p < WCN_BIN_SLOTS; ++p) {
-        if (s->key[h] == key) {
-          slot_of[in.row(e)] = s->where[h];
-          break;
-        }
-        h = (h + 1) & (WCN_BIN_SLOTS - 1);
-      }
-    }
-  }
   if (repeats && low_in_lds)
     for (int j = tid; j < total_v; j += 1024) perm[lo + j] = s->low[j];
   if (tid == 0) {
     bin_stats[2 * bin] = total_v;
-    bin_stats[2 * bin + 1] = total_b;
+    bin_stats[2 * bin + 1] = total_b | (s->lost ? WCN_BIN_LOST : 0);
   }
 }
 
-template <bool WANT_SLOT_OF>
-__global__ void __launch_bounds__(1024) table_bins(WcnTableHeader* __restrict__ hdr,
-                                                   WcnSlot* __restrict__ slots, uint32_t cap_mask,
+template <bool WANT_SLOT_OF, bool TWO>
+__global__ void __launch_bounds__(1024, TWO ? 8 : 4) table_bins(const WcnTableHeader* __restrict__ hdr,
+                                                   WcnSlot* __restrict__ slots, unsigned long long* __restrict__ wide_keys,
                                                    const int32_t* __restrict__ bin_start,
                                                    const int4* __restrict__ bin_coords,
                                                    const int32_t* __restrict__ bin_row,
                                                    int32_t* __restrict__ order_tag,
                                                    int32_t* __restrict__ order_row,
-                                                   WcnSlot* __restrict__ block_list,
+                                                   WcnBlock* __restrict__ block_list,
                                                    int32_t* __restrict__ perm,
                                                    int32_t* __restrict__ slot_of,
                                                    int32_t* __restrict__ bin_stats) {
   extern __shared__ __attribute__((aligned(16))) unsigned char bin_smem[];
   const BinEntries in{bin_coords, bin_row};
-  build_bin<WANT_SLOT_OF>(in, (int)blockIdx.x, bin_start[blockIdx.x], bin_start[blockIdx.x + 1], wcn_make_layout(hdr),
-                          reinterpret_cast<BinLds*>(bin_smem), hdr, slots, cap_mask, order_tag, order_row, block_list,
+  build_bin<WANT_SLOT_OF, TWO ? 3 : 4>(in, (int)blockIdx.x, bin_start[blockIdx.x], bin_start[blockIdx.x + 1], wcn_make_layout(hdr),
+                          reinterpret_cast<BinLds*>(bin_smem), slots, wide_keys, order_tag, order_row, block_list,
                           perm, slot_of, bin_stats);
 }
 
@@ -538,52 +506,53 @@ __global__ void __launch_bounds__(1024) table_bins(WcnTableHeader* __restrict__ 
 // The passes above are a chain of four launches of about five microseconds each, whatever there is to
 // do in them.  Up to SMALL_KEYS keys every workgroup of the last pass reads all of them (a quarter of a megabyte at
 // the most, out of its die's L2): it finds the box, lists the rows of its own bin and counts those of the bins before it.
-// What has to be done before the first of them starts is the clearing of the slots.  Over 2 k keys 18.1 us
-// and four launches before, 14.3 and two this way (layer 78.4 -> 75.4 us, a U-Net over 60 k voxels 1522 -> 1499).
+// Over 2 k keys 18.1 us and four launches before, 14.3 and two this way while the slots had to be cleared in a launch before it
+// (layer 78.4 -> 75.4 us, a U-Net over 60 k voxels 1522 -> 1499), one launch now.
 constexpr int64_t SMALL_KEYS = 16384;
 constexpr int SMALL_KEY_BINS = 64;  // more bins (a table that was grown) would read the keys too often
-
-template <bool ITEMS>  // the keys are made on the way, as in table_hist
-__global__ void __launch_bounds__(256) table_clear(uint4* __restrict__ raw, int64_t items, WcnTableHeader* __restrict__ hdr,
-                                                   int32_t n_keys, int32_t bins, int64_t stats_offset, KeysOfItems of) {
-  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (ITEMS) {
-    __shared__ int64_t s_start[WCN_VOXEL_MAX_BATCH + 1];
-    if (threadIdx.x <= WCN_VOXEL_MAX_BATCH) s_start[threadIdx.x] = of.starts.start[threadIdx.x];
-    __syncthreads();
-    if (i < n_keys)
-      of.rows[i] = make_int4(wcn_item_of(s_start, of.batch_size, i), of.coords[3 * i], of.coords[3 * i + 1], of.coords[3 * i + 2]);
-  }
-  if (i < items) raw[i] = (i & 1) ? make_uint4(0u, 0u, 0u, 0u) : make_uint4(0xFFFFFFFFu, 0xFFFFFFFFu, 0u, 0u);
-  if (i == 0) {
-    hdr->num_blocks = 0;
-    hdr->status = 0;
-    hdr->total = 0;
-    hdr->num_keys = n_keys;
-    hdr->bins = bins;
-    hdr->stats_offset = stats_offset;
-  }
-}
 
 struct SmallLds {
   BinLds bin;
   uint16_t list[SMALL_KEYS];
   WcnTableHeader box;
+  int64_t item_start[WCN_VOXEL_MAX_BATCH + 1];
   int part[16][10];  // per wave: least and greatest value of every column, keys of earlier bins
   int listed;
 };
 
-template <bool WANT_SLOT_OF>
-__global__ void __launch_bounds__(1024) table_small(const int4* __restrict__ keys, int32_t n_keys, int32_t bins,
-                                                    WcnTableHeader* __restrict__ hdr, WcnSlot* __restrict__ slots,
-                                                    uint32_t cap_mask, int32_t* __restrict__ bin_start,
+struct KeyRows {
+  const int4* __restrict__ keys;
+  __device__ __forceinline__ int4 operator()(int i) const { return keys[i]; }
+};
+struct KeyItems {  // made here, as in table_hist
+  const int32_t* __restrict__ coords;
+  const int64_t* start;
+  int32_t batch_size;
+  __device__ __forceinline__ int4 operator()(int i) const {
+    return make_int4(wcn_item_of(start, batch_size, i), coords[3 * i], coords[3 * i + 1], coords[3 * i + 2]);
+  }
+};
+
+template <bool WANT_SLOT_OF, bool ITEMS>
+__global__ void __launch_bounds__(1024) table_small(const int4* __restrict__ rows, KeysOfItems of, int32_t n_keys, int32_t bins,
+                                                    WcnTableHeader* __restrict__ hdr, int64_t stats_offset,
+                                                    WcnSlot* __restrict__ slots, unsigned long long* __restrict__ wide_keys,
+                                                    int32_t* __restrict__ bin_start,
                                                     int32_t* __restrict__ order_tag, int32_t* __restrict__ order_row,
-                                                    WcnSlot* __restrict__ block_list, int32_t* __restrict__ perm,
+                                                    WcnBlock* __restrict__ block_list, int32_t* __restrict__ perm,
                                                     int32_t* __restrict__ slot_of, int32_t* __restrict__ bin_stats) {
   extern __shared__ __attribute__((aligned(16))) unsigned char bin_smem[];
   SmallLds* s = reinterpret_cast<SmallLds*>(bin_smem);
   const int tid = threadIdx.x, lane = wcn_lane(), wave = tid >> 6, bin = (int)blockIdx.x;
   const uint32_t bin_mask = (uint32_t)bins - 1u;
+  typedef typename std::conditional<ITEMS, KeyItems, KeyRows>::type Keys;
+  Keys keys;
+  if constexpr (ITEMS) {
+    if (tid <= WCN_VOXEL_MAX_BATCH) s->item_start[tid] = of.starts.start[tid];
+    keys = Keys{of.coords, s->item_start, of.batch_size};
+  } else {
+    keys = Keys{rows};
+  }
   if (tid == 0) s->listed = 0;
   __syncthreads();
   int v[9] = {INT32_MAX, INT32_MAX, INT32_MAX, INT32_MAX, INT32_MIN, INT32_MIN, INT32_MIN, INT32_MIN, 0};
@@ -591,7 +560,7 @@ __global__ void __launch_bounds__(1024) table_small(const int4* __restrict__ key
   for (int i0 = tid; i0 < n_keys; i0 += 1024 * PER) {
     int4 c[PER];
 #pragma unroll
-    for (int t = 0; t < PER; ++t) c[t] = keys[i0 + t * 1024 < n_keys ? i0 + t * 1024 : i0];
+    for (int t = 0; t < PER; ++t) c[t] = keys(i0 + t * 1024 < n_keys ? i0 + t * 1024 : i0);
 #pragma unroll
     for (int t = 0; t < PER; ++t) {
       const int i = i0 + t * 1024;
@@ -601,6 +570,7 @@ __global__ void __launch_bounds__(1024) table_small(const int4* __restrict__ key
       v[3] = min(v[3], c[t].w); v[7] = max(v[7], c[t].w);
       const int b = (int)bin_of(c[t], bin_mask);
       const bool live = i < n_keys;
+      if (ITEMS && live && ((uint32_t)i >> 10 & bin_mask) == (uint32_t)bin) of.rows[i] = c[t];
       v[8] += live && b < bin ? 1 : 0;
       if (live && b == bin) s->list[atomicAdd(&s->listed, 1)] = (uint16_t)i;
     }
@@ -630,9 +600,14 @@ __global__ void __launch_bounds__(1024) table_small(const int4* __restrict__ key
   if (tid == 0) {
     bin_start[bin] = lo;
     if (bin == bins - 1) bin_start[bins] = n_keys;
+    if (bin == 0) {
+      hdr->num_keys = n_keys;
+      hdr->bins = bins;
+      hdr->stats_offset = stats_offset;
+    }
   }
-  const ListedEntries in{keys, s->list, lo};
-  build_bin<WANT_SLOT_OF>(in, bin, lo, hi, wcn_make_layout(&s->box), &s->bin, hdr, slots, cap_mask, order_tag, order_row,
+  const ListedEntries<Keys> in{keys, s->list, lo};
+  build_bin<WANT_SLOT_OF, 4>(in, bin, lo, hi, wcn_make_layout(&s->box), &s->bin, slots, wide_keys, order_tag, order_row,
                           block_list, perm, slot_of, bin_stats);
 }
 
@@ -642,10 +617,12 @@ __global__ void __launch_bounds__(1024) table_sum_stats(WcnTableHeader* __restri
   __shared__ int s_v[16], s_b[16];
   const int32_t bins = hdr->bins;
   const int32_t* bin_stats = reinterpret_cast<const int32_t*>(reinterpret_cast<const char*>(hdr) + hdr->stats_offset);
+  __shared__ int s_lost[16];
+  const int status = wcn_table_status(hdr, (int)threadIdx.x, 1024, s_lost);
   int v = 0, b = 0;
   for (int i = threadIdx.x; i < bins; i += 1024) {
     v += bin_stats[2 * i];
-    b += bin_stats[2 * i + 1];
+    b += bin_stats[2 * i + 1] & ~WCN_BIN_LOST;
   }
 #pragma unroll
   for (int s = 32; s > 0; s >>= 1) {
@@ -665,12 +642,12 @@ __global__ void __launch_bounds__(1024) table_sum_stats(WcnTableHeader* __restri
     }
     hdr->total = v;
     hdr->num_blocks = b;
+    hdr->status = status;
   }
 }
 
 __global__ void __launch_bounds__(256) table_query(const WcnTableHeader* __restrict__ hdr,
-                                                   const WcnSlot* __restrict__ slots,
-                                                   uint32_t cap_mask,
+                                                   WcnTableRef table,
                                                    const int32_t* __restrict__ perm,
                                                    const int4* __restrict__ queries,
                                                    int64_t num_queries,
@@ -683,7 +660,7 @@ __global__ void __launch_bounds__(256) table_query(const WcnTableHeader* __restr
   int32_t res = -1;
   if (L.ok && wcn_relative(L, c.x, c.y, c.z, c.w, r)) {
     int32_t base;
-    const unsigned long long mask = wcn_lookup_block(slots, cap_mask, wcn_block_key(L, r), &base);
+    const unsigned long long mask = wcn_lookup_block(L, table, r, &base);
     const uint32_t bit = wcn_block_bit(r);
     if ((mask >> bit) & 1ull) res = perm[base + wcn_rank_below(mask, bit)];
   }
@@ -706,7 +683,7 @@ inline int grid_for(int64_t n, int block, int cap = 0x7fffffff) {
 // LDS beyond the default limit: lifted once per device and kernel.
 static int allow_lds(const void* kernel, size_t bytes, int which) {
   static std::mutex mu;
-  static bool allowed[7][64] = {};
+  static bool allowed[11][64] = {};
   int device = 0;
   if (hipGetDevice(&device) != hipSuccess || device < 0 || device >= 64) return WCN_ERR_LAUNCH;
   std::lock_guard<std::mutex> hold(mu);
@@ -721,19 +698,17 @@ static int allow_lds(const void* kernel, size_t bytes, int which) {
 // every key (`want_slot_of`).
 static int table_build_from(const int32_t* keys, int64_t n_keys, const WcnTableView& v, const KeysOfItems* items,
                             bool want_slot_of, hipStream_t s) {
-  const uint32_t cap_mask = (uint32_t)(v.capacity - 1);
   const int4* k4 = (const int4*)keys;
   if (v.bins < 1 || v.bins > WCN_MAX_BINS || (v.bins & (v.bins - 1))) return WCN_ERR_INVALID_ARGUMENT;
+  const int64_t stats = (int64_t)((const char*)v.bin_stats - (const char*)v.hdr);
   if (n_keys >= 1 && n_keys <= SMALL_KEYS && v.bins <= SMALL_KEY_BINS) {
-    auto small = want_slot_of ? table_small<true> : table_small<false>;
-    if (allow_lds((const void*)small, sizeof(SmallLds), want_slot_of ? 4 : 3) != WCN_OK) return WCN_ERR_LAUNCH;
-    const int64_t words = 2 * v.capacity, stats = (int64_t)((const char*)v.bin_stats - (const char*)v.hdr);
-    const int64_t clears = std::max(words, n_keys);
-    hipLaunchKernelGGL((items ? table_clear<true> : table_clear<false>), dim3((unsigned)((clears + 255) / 256)), dim3(256), 0, s,
-                       (uint4*)v.slots, words, v.hdr, (int32_t)n_keys, v.bins, stats, items ? *items : KeysOfItems{});
-    hipLaunchKernelGGL(small, dim3(v.bins), dim3(1024), sizeof(SmallLds), s, k4, (int32_t)n_keys, v.bins, v.hdr,
-                       v.slots, cap_mask, v.bin_start, v.order_tag, v.order_row, v.block_list, v.perm, v.slot_of,
-                       v.bin_stats);
+    auto small = want_slot_of ? (items ? table_small<true, true> : table_small<true, false>)
+                              : (items ? table_small<false, true> : table_small<false, false>);
+    const int which = 7 + (want_slot_of ? 2 : 0) + (items ? 1 : 0);
+    if (allow_lds((const void*)small, sizeof(SmallLds), which) != WCN_OK) return WCN_ERR_LAUNCH;
+    hipLaunchKernelGGL(small, dim3(v.bins), dim3(1024), sizeof(SmallLds), s, k4, items ? *items : KeysOfItems{}, (int32_t)n_keys,
+                       v.bins, v.hdr, stats, v.slots, v.wide_keys, v.bin_start, v.order_tag, v.order_row, v.block_list, v.perm,
+                       v.slot_of, v.bin_stats);
     WCN_LAUNCH_CHECK();
     return WCN_OK;
   }
@@ -741,22 +716,24 @@ static int table_build_from(const int32_t* keys, int64_t n_keys, const WcnTableV
   const size_t counters = sizeof(int) * (size_t)v.bins;
   auto scatter = many_bins ? table_scatter<WCN_MAX_BINS / 1024> : table_scatter<SMALL_BINS / 1024>;
   auto hist = items ? table_hist<true> : table_hist<false>;
-  auto fn = want_slot_of ? table_bins<true> : table_bins<false>;
-  if (allow_lds((const void*)fn, sizeof(BinLds), want_slot_of ? 1 : 0) != WCN_OK) return WCN_ERR_LAUNCH;
+  const bool two = v.bins > 256;  // more than one per CU: 64 registers let two share it (fewer bins: 15.7 -> 22 us of 500 k voxels)
+  auto fn = want_slot_of ? (two ? table_bins<true, true> : table_bins<true, false>)
+                         : (two ? table_bins<false, true> : table_bins<false, false>);
+  if (allow_lds((const void*)fn, sizeof(BinLds), (want_slot_of ? 1 : 0) + (two ? 3 : 0)) != WCN_OK) return WCN_ERR_LAUNCH;
   if (many_bins) {
     const size_t most = sizeof(int) * WCN_MAX_BINS;
     if (allow_lds((const void*)hist, most, items ? 6 : 2) != WCN_OK || allow_lds((const void*)scatter, most, 5) != WCN_OK)
       return WCN_ERR_LAUNCH;
   }
   hipLaunchKernelGGL(hist, dim3(v.parts), dim3(1024), counters, s, k4, n_keys, v.bins, v.hist,
-                     v.part_box, v.slots, v.capacity, items ? *items : KeysOfItems{});
+                     v.part_box, items ? *items : KeysOfItems{});
   hipLaunchKernelGGL(table_colscan, dim3((v.bins + 3) / 4), dim3(256), 0, s, v.hist, v.bins,
                      v.parts, v.bin_total);
   hipLaunchKernelGGL(scatter, dim3(v.parts), dim3(1024), counters, s, k4, n_keys, v.bins, v.hist,
                      v.bin_total, v.bin_start, v.part_box, v.hdr,
-                     (int64_t)((const char*)v.bin_stats - (const char*)v.hdr), (int4*)v.bin_coords,
+                     stats, (int4*)v.bin_coords,
                      v.bin_row);
-  hipLaunchKernelGGL(fn, dim3(v.bins), dim3(1024), sizeof(BinLds), s, v.hdr, v.slots, cap_mask,
+  hipLaunchKernelGGL(fn, dim3(v.bins), dim3(1024), sizeof(BinLds), s, v.hdr, v.slots, v.wide_keys,
                      v.bin_start, (const int4*)v.bin_coords, v.bin_row, v.order_tag, v.order_row,
                      v.block_list, v.perm, v.slot_of, v.bin_stats);
   WCN_LAUNCH_CHECK();
@@ -1042,7 +1019,7 @@ int wcn_table_query(const void* table, int64_t n_keys, int64_t capacity, const i
   WcnTableView v;
   wcn_table_layout(const_cast<void*>(table), n_keys, capacity, &v);
   hipLaunchKernelGGL(table_query, dim3(grid_for(num_queries, 256)), dim3(256), 0,
-                     (hipStream_t)stream, v.hdr, v.slots, (uint32_t)(capacity - 1), v.perm,
+                     (hipStream_t)stream, v.hdr, wcn_table_ref(v), v.perm,
                      (const int4*)queries, num_queries, results);
   WCN_LAUNCH_CHECK();
   return WCN_OK;
