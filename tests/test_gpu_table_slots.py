@@ -71,3 +71,16 @@ def test_blocks_at_the_same_place_of_their_cells(n, step):
     table = TorchHashTable.from_keys(_dev(rows), device=DEV)
     assert np.array_equal(table.search(_dev(rows)).cpu().numpy(), np.arange(n, dtype=np.int32))
     assert (table.search(_dev(rows + np.array([0, 1, 0, 0], np.int32))).cpu().numpy() == -1).all()
+
+
+# (parts of 4096 keys x bins either side of what the scatter pass adds up by itself; 64, 8 and 4 lanes a bin)
+@pytest.mark.parametrize("n", [16_385, 131_073, 262_143, 262_145, 300_000])
+@pytest.mark.parametrize("repeats", [False, True])
+def test_tables_whose_scatter_pass_adds_up_the_histogram(n, repeats):
+    from warpconvnet_amd.geometry.coords.search.torch_hashmap import TorchHashTable
+    rng = np.random.default_rng(n)
+    cells = rng.choice(4 * 90 ** 3, n, replace=repeats)
+    rows = np.stack([cells // 90 ** 3, cells // 8100 % 90 - 31, cells // 90 % 90, cells % 90 - 60], axis=1).astype(np.int32)
+    _, first, back = np.unique(cells, return_index=True, return_inverse=True)
+    table = TorchHashTable.from_keys(_dev(rows), device=DEV)
+    assert np.array_equal(table.search(_dev(rows)).cpu().numpy(), first[back])

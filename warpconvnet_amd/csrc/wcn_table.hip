@@ -6,7 +6,7 @@
 // builds their masks with LDS atomics:
 //   table_hist     per part of the keys (a workgroup): keys per bin (LDS counters) and the part's
 //                  bounding box
-//   table_colscan  per bin (a wave): prefix sums over the parts
+//   table_colscan  per bin (a wave): prefix sums over the parts (up to some 260,000 keys table_scatter adds them up itself)
 //   table_scatter  per part: every key and its row to its place in its bin; the first workgroup merges the boxes and
 //                  writes the header
 //   table_bins     per bin: block masks and entry counts in an LDS table, their prefix sums; that table is the bin's
@@ -156,7 +156,13 @@ __global__ void __launch_bounds__(256) table_colscan(int32_t* __restrict__ hist,
 // starts for itself (1024 x BPT numbers); workgroup 0 also stores them for the next pass,
 // merges the parts' bounding boxes and writes the header.  Parts that follow one another run on one XCD: their pieces
 // of a bin (eight keys of 1 M: 128 bytes, 32 of rows) follow one another too (1 M keys: 25 -> 21.5 us).
-template <int BPT>
+// COUNTS: the histogram as table_hist leaves it (up to OWN_SUMS words): every workgroup adds up what it needs of it, the
+// bins' totals and the keys of earlier parts, and table_colscan is not launched: scatter and scan over 100 k keys 7.6 + 2.8 to 3.8 us
+// -> 7.7, over 24 k 5.9 + 4 -> 5.9, over 160 k 7.7 + 3 -> 9.  At 500 k keys (31 words a lane) it took what it saved: 11.7 + 4.6 -> 16.2.
+constexpr int64_t OWN_SUMS = 16384;
+constexpr int OWN_BINS = 256;
+
+template <int BPT, bool COUNTS>
 __global__ void __launch_bounds__(1024) table_scatter(const int4* __restrict__ keys, int64_t n_keys,
                                                       int32_t bins, const int32_t* __restrict__ hist,
                                                       const int32_t* __restrict__ bin_total,
@@ -171,19 +177,51 @@ __global__ void __launch_bounds__(1024) table_scatter(const int4* __restrict__ k
   const int tid = threadIdx.x, lane = wcn_lane(), wave = tid >> 6;
   const int parts = gridDim.x, part = wcn_xcd_tile((int)blockIdx.x, parts);
   const PartRange r = part_range(n_keys, part);
+  // (COUNTS) the lanes of a bin, 4 to 64, and the first of the parts that each of them looks after
+  const int lanes_log = COUNTS ? 10 - (31 - __builtin_clz(bins)) : 0, lanes = 1 << lanes_log;
+  const int own_bin = tid >> lanes_log, first = tid & (lanes - 1);
+  constexpr int AHEAD = 4;
+  int n[COUNTS ? AHEAD : 1];
+  if (COUNTS) {
+#pragma unroll
+    for (int t = 0; t < AHEAD; ++t) n[COUNTS ? t : 0] = hist[own_bin * parts + (first + t * lanes < parts ? first + t * lanes : 0)];
+  }
   constexpr int PER = 4;
-  int4 c[PER];  // the first keys are requested before anything else
+  int4 c[PER];  // the first keys are requested before anything else is waited for
 #pragma unroll
   for (int t = 0; t < PER; ++t) {
     const int64_t i = r.lo + tid + t * 1024;
     c[t] = i < r.hi ? keys[i] : make_int4(0, 0, 0, 0);
   }
   int v[BPT], mine[BPT], sum = 0;
+  __shared__ int2 s_bin[COUNTS ? OWN_BINS : 1];
+  if (COUNTS) {
+    int all = 0, before = 0;
+    for (int p0 = first; p0 < parts; p0 += AHEAD * lanes) {
+      if (p0 != first) {
+#pragma unroll
+        for (int t = 0; t < AHEAD; ++t) n[COUNTS ? t : 0] = hist[own_bin * parts + (p0 + t * lanes < parts ? p0 + t * lanes : 0)];
+      }
+#pragma unroll
+      for (int t = 0; t < AHEAD; ++t) {
+        const int p = p0 + t * lanes;
+        all += p < parts ? n[COUNTS ? t : 0] : 0;
+        before += p < part ? n[COUNTS ? t : 0] : 0;
+      }
+    }
+    for (int d = 1; d < lanes; d <<= 1) {
+      all += __shfl_xor(all, d, 64);
+      before += __shfl_xor(before, d, 64);
+    }
+    if (first == 0) s_bin[COUNTS ? own_bin : 0] = make_int2(all, before);
+    __syncthreads();
+  }
 #pragma unroll
   for (int t = 0; t < BPT; ++t) {
     const int b = tid * BPT + t;
-    v[t] = b < bins ? bin_total[b] : 0;
-    mine[t] = b < bins ? hist[(int64_t)b * parts + part] : 0;
+    const int2 own = COUNTS && b < bins ? s_bin[COUNTS ? b : 0] : make_int2(0, 0);
+    v[t] = COUNTS ? own.x : b < bins ? bin_total[b] : 0;
+    mine[t] = COUNTS ? own.y : b < bins ? hist[(int64_t)b * parts + part] : 0;
     sum += v[t];
   }
   const int incl = wcn_wave_inclusive_sum(sum);
@@ -714,7 +752,10 @@ static int table_build_from(const int32_t* keys, int64_t n_keys, const WcnTableV
   }
   const bool many_bins = v.bins > SMALL_BINS;
   const size_t counters = sizeof(int) * (size_t)v.bins;
-  auto scatter = many_bins ? table_scatter<WCN_MAX_BINS / 1024> : table_scatter<SMALL_BINS / 1024>;
+  const bool own_sums = v.bins <= OWN_BINS && (int64_t)v.bins * v.parts <= OWN_SUMS;
+  auto scatter = many_bins  ? table_scatter<WCN_MAX_BINS / 1024, false>
+                 : own_sums ? table_scatter<SMALL_BINS / 1024, true>
+                            : table_scatter<SMALL_BINS / 1024, false>;
   auto hist = items ? table_hist<true> : table_hist<false>;
   const bool two = v.bins > 256;  // more than one per CU: 64 registers let two share it (fewer bins: 15.7 -> 22 us of 500 k voxels)
   auto fn = want_slot_of ? (two ? table_bins<true, true> : table_bins<true, false>)
@@ -727,8 +768,9 @@ static int table_build_from(const int32_t* keys, int64_t n_keys, const WcnTableV
   }
   hipLaunchKernelGGL(hist, dim3(v.parts), dim3(1024), counters, s, k4, n_keys, v.bins, v.hist,
                      v.part_box, items ? *items : KeysOfItems{});
-  hipLaunchKernelGGL(table_colscan, dim3((v.bins + 3) / 4), dim3(256), 0, s, v.hist, v.bins,
-                     v.parts, v.bin_total);
+  if (!own_sums)
+    hipLaunchKernelGGL(table_colscan, dim3((v.bins + 3) / 4), dim3(256), 0, s, v.hist, v.bins,
+                       v.parts, v.bin_total);
   hipLaunchKernelGGL(scatter, dim3(v.parts), dim3(1024), counters, s, k4, n_keys, v.bins, v.hist,
                      v.bin_total, v.bin_start, v.part_box, v.hdr,
                      stats, (int4*)v.bin_coords,
