@@ -1,0 +1,110 @@
+"""Layers over small maps that are launched before the map's offsets have reached the host: the same bits as over the kept
+map, with every extra of the epilogue; lists that turn out too short, and calls that have to wait for the map."""
+import numpy as np
+import pytest
+import torch
+
+from helpers import kaiming_weight, normal_features
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def _voxels(n, c_in, dtype, seed=0):
+    from warpconvnet_amd.geometry.types.voxels import Voxels
+    rng = np.random.default_rng(seed)
+    side = int(np.ceil(np.sqrt(n / 0.5)))
+    cells = rng.permutation(side * side)[:n]
+    coords = np.stack([cells // side, cells % side, cells % 3 // 2], axis=1).astype(np.int32) - 7
+    return Voxels(torch.as_tensor(coords, device=DEV), normal_features(n, c_in, seed=seed, dtype=dtype).to(DEV),
+                  offsets=torch.tensor([0, n // 3, n]))
+
+
+def _spied(monkeypatch):
+    """What the layers that ran ahead of their maps have left: one entry per LayerAhead made."""
+    from warpconvnet_amd.nn.functional import sparse_conv as f
+    made = []
+    native = f.native()
+
+    class Spy:
+        def __getattr__(self, name):
+            if name != "LayerAhead":
+                return getattr(native, name)
+
+            def make(*args):
+                made.append(native.LayerAhead(*args))
+                return made[-1]
+            return make
+    monkeypatch.setattr(f, "native", lambda: Spy())
+    return made
+
+
+@pytest.mark.parametrize("n", [1, 31, 33, 1800, 5000])
+@pytest.mark.parametrize("dtype,c_in,c_out,kernel,stride", [
+    (torch.float16, 32, 64, 3, 1), (torch.bfloat16, 64, 64, 3, 1), (torch.float32, 32, 32, 3, 1), (torch.bfloat16, 64, 128, 2, 2),
+    (torch.float16, 16, 24, 5, 1), (torch.float16, 32, 32, 3, 2), (torch.bfloat16, 256, 256, 3, 1)])
+@pytest.mark.parametrize("extras", [False, True])
+def test_same_bits_as_over_the_kept_map(monkeypatch, n, dtype, c_in, c_out, kernel, stride, extras):
+    from warpconvnet_amd.nn.functional.sparse_conv import spatially_sparse_conv
+    made = _spied(monkeypatch)
+    w = kaiming_weight(kernel ** 3, c_in, c_out, seed=2, dtype=dtype).to(DEV)
+    vox = _voxels(n, c_in, dtype, seed=n)
+    kw = {"stride": stride}
+    if extras:
+        kw.update(bias=normal_features(1, c_out, seed=3, dtype=dtype)[0].to(DEV), relu=True, keep_prepared_weight=True)
+        if stride == 1:
+            kw["residual"] = normal_features(n, c_out, seed=4, dtype=dtype).to(DEV)
+    first = spatially_sparse_conv(vox, w, kernel, **kw).feature_tensor
+    assert len(made) == 1 and made[0].out is not None
+    again = spatially_sparse_conv(vox, w, kernel, **kw).feature_tensor
+    assert all(a.out is None for a in made[1:])  # the map is there
+    assert torch.equal(first, again)
+    # new voxels in the same rows: the layer's own map, and the bits of the first
+    assert torch.equal(first, spatially_sparse_conv(_voxels(n, c_in, dtype, seed=n), w, kernel, **kw).feature_tensor)
+
+
+def test_lists_that_turn_out_too_short(monkeypatch):
+    """27 pairs per voxel where ten are assumed: the layer that ran ahead has found no lists, and runs again."""
+    from warpconvnet_amd.geometry.coords.search import torch_discrete
+    from warpconvnet_amd.geometry.types.voxels import Voxels
+    from warpconvnet_amd.nn.functional.sparse_conv import spatially_sparse_conv
+    made = _spied(monkeypatch)
+    monkeypatch.setattr(torch_discrete, "_PAIRS_PER_ROW", {})
+    cube = np.stack(np.meshgrid(*[np.arange(20)] * 3, indexing="ij"), axis=-1).reshape(-1, 3).astype(np.int32)
+    n = len(cube)
+    x = normal_features(n, 64, seed=1, dtype=torch.float16).to(DEV)
+    w = kaiming_weight(27, 64, 64, seed=2, dtype=torch.float16).to(DEV)
+    vox = Voxels(torch.as_tensor(cube, device=DEV), x, offsets=torch.tensor([0, n]))
+    first = spatially_sparse_conv(vox, w, 3).feature_tensor
+    assert len(made) == 1 and made[0].out is None
+    km = next(iter(vox.cache.values()))
+    assert km.in_maps.shape[0] == (20 * 3 - 2) ** 3
+    assert torch.equal(first, spatially_sparse_conv(vox, w, 3).feature_tensor)
+    # the next map of this size assumes what this one held
+    vox = Voxels(torch.as_tensor(cube, device=DEV), x, offsets=torch.tensor([0, n]))
+    assert torch.equal(first, spatially_sparse_conv(vox, w, 3).feature_tensor)
+    assert made[-1].out is not None
+
+
+@pytest.mark.parametrize("case", ["columns", "fp32_bias", "one_bias", "half_weight", "residual_type", "three_channels", "converted"])
+def test_calls_that_wait_for_the_map(monkeypatch, case):
+    from warpconvnet_amd.nn.functional.sparse_conv import spatially_sparse_conv
+    made = _spied(monkeypatch)
+    n, c_in, c_out, dtype = 900, 3 if case == "three_channels" else 32, 32, torch.float16
+    vox = _voxels(n, c_in, dtype)
+    w = kaiming_weight(27, c_in, c_out, seed=2, dtype=torch.bfloat16 if case == "half_weight" else dtype).to(DEV)
+    kw = {}
+    if case == "columns":
+        wide = normal_features(n, 2 * c_in, seed=5, dtype=dtype).to(DEV)
+        vox = vox.replace(batched_features=wide[:, ::2])
+    elif case == "fp32_bias":
+        kw["bias"] = torch.randn(c_out, device=DEV)
+    elif case == "one_bias":
+        kw["bias"] = torch.ones(1, device=DEV, dtype=dtype)
+    elif case == "residual_type":
+        kw["residual"] = torch.randn(n, c_out, device=DEV)
+    elif case == "converted":
+        kw["compute_dtype"] = torch.bfloat16
+    first = spatially_sparse_conv(vox, w, 3, **kw).feature_tensor
+    assert len(made) == 1 and made[0].out is None
+    assert torch.equal(first, spatially_sparse_conv(vox, w, 3, **kw).feature_tensor)

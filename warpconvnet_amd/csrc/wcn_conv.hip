@@ -1459,7 +1459,7 @@ static int conv_run(const void* features, int64_t num_in, int32_t c_in, int32_t 
                     int flip_offsets, bool no_copy_commands, void* stream,
                     const void* residual_or_null = nullptr, int relu = 0,
                     const int64_t* device_offsets_of_prepared = nullptr, int bias_dtype = -1,
-                    int bias_after_rounding = 0, const void* prepared_operands = nullptr) {
+                    int bias_after_rounding = 0, const void* prepared_operands = nullptr, int64_t list_capacity = 0) {
   // With device_offsets_of_prepared, `weight` and `prepared_operands` are the two halves that wcn_conv_prepare_weight makes
   // (the one that is not read may be null) and the call enqueues nothing but the contraction.
   const bool prepared = device_offsets_of_prepared != nullptr;
@@ -1484,7 +1484,8 @@ static int conv_run(const void* features, int64_t num_in, int32_t c_in, int32_t 
   if (prepared) {
     // tiles, zeros, offsets and group starts all come from elsewhere: the workspace is the partial
     // sums of split input-channel slices, where the problem's shape asks for them, and nothing else
-    const size_t need = wcn_conv_prepared_workspace_bytes(num_out, num_offsets, c_in, c_out, dtype);
+    // (the kernel for small maps, which a call ahead of its map is for, adds its sums in LDS)
+    const size_t need = list_capacity > 0 ? 0 : wcn_conv_prepared_workspace_bytes(num_out, num_offsets, c_in, c_out, dtype);
     if (need > 0 && (!workspace || workspace_bytes < need)) return WCN_ERR_WORKSPACE;
     conv_layout(nullptr, num_out, num_offsets, c_in, c_out, dtype, -1, &w);
     w.partial = need > 0 ? (float*)workspace : nullptr;
@@ -1517,6 +1518,7 @@ static int conv_run(const void* features, int64_t num_in, int32_t c_in, int32_t 
   a.num_in = num_in;
   a.num_out = num_out;
   a.num_pairs = L;
+  a.list_capacity = list_capacity;
   a.G = w.G;
   a.K = num_offsets;
   a.c_in = c_in;
@@ -1547,6 +1549,7 @@ static int conv_run(const void* features, int64_t num_in, int32_t c_in, int32_t 
   // size of map gives.  In training it would save 4 % of a stage on 10,000 voxels.
   const bool small = !bias_after_rounding && kernel_choice() == 0 && wcn_conv_split_takes(a, dtype);
   if (prepared && !(small ? prepared_operands : weight)) return WCN_ERR_INVALID_ARGUMENT;
+  if (list_capacity > 0 && !small) return WCN_ERR_INVALID_ARGUMENT;
   a.Wf = nullptr;
   if (small && !prepared) {
     a.Wf = w.Wt;
@@ -1816,6 +1819,26 @@ int wcn_sparse_conv_fwd_prepared_halves(const void* features, int64_t num_in, in
   return conv_run(features, num_in, c_in, dtype, half0_or_null, dtype, num_offsets, c_out, bias_or_null, in_maps, out_maps,
                   host_offsets, identity_offset, 1, group_start, out, num_out, workspace, workspace_bytes, 0, 0, true,
                   stream, residual_or_null, relu, device_offsets, -1, 0, half1_or_null);
+}
+
+int wcn_sparse_conv_fwd_ahead(const void* features, int64_t num_in, int32_t c_in, int32_t dtype, const void* half1,
+                              int32_t num_offsets, int32_t c_out, const void* bias_or_null, const int32_t* in_maps,
+                              const int32_t* out_maps, int64_t pair_capacity, const int64_t* map_result,
+                              int32_t identity_offset, const int32_t* group_start, const void* residual_or_null, int32_t relu,
+                              void* out, int64_t num_out, void* stream) {
+  if (residual_or_null && residual_or_null == out) return WCN_ERR_INVALID_ARGUMENT;
+  if (!half1 || !map_result || !group_start || !in_maps || !out_maps || pair_capacity < 1 || num_offsets < 1 ||
+      num_offsets > WCN_MAX_OFFSETS)
+    return WCN_ERR_INVALID_ARGUMENT;
+  static const int64_t unknown[WCN_MAX_OFFSETS + 1] = {};  // the pairs: the kernel for small maps does not ask for them
+  return conv_run(features, num_in, c_in, dtype, nullptr, dtype, num_offsets, c_out, bias_or_null, in_maps, out_maps, unknown,
+                  identity_offset, 1, group_start, out, num_out, nullptr, 0, 0, 0, true, stream, residual_or_null, relu, map_result,
+                  -1, 0, half1, pair_capacity);
+}
+
+int wcn_conv_tiles_sized(int32_t dtype, int32_t num_offsets, int32_t c_in, int32_t c_out, int64_t num_out) {
+  return kernel_choice() == 0 && wcn_conv_tiles_takes(dtype, num_offsets, c_in, c_out) &&
+         wcn_conv_tiles_rows(num_offsets, c_in, c_out, num_out);
 }
 
 int wcn_sparse_conv_fwd_prepared(const void* features, int64_t num_in, int32_t c_in, int32_t dtype,

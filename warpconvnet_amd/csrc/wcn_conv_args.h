@@ -18,6 +18,8 @@ struct ConvArgs {
   void* out;
   int64_t num_in, num_out, G;
   int64_t num_pairs;           // all offsets together (known on the host)
+  int64_t list_capacity;       // > 0 (kernel for small maps): the lists of a builder that the host has not waited for.  They hold
+                               // what they should if offsets[K], the pairs, is at most this and offsets[K + 1], its status, 0
   int32_t K, c_in, c_out, c_in_pad, c_out_pad, identity;
   int32_t vec_in;   // feature rows are 16-byte aligned and a whole number of 16-byte vectors
   int32_t vec_out;  // same for output rows
@@ -54,6 +56,7 @@ int wcn_conv_split_launch(const ConvArgs& a, int dtype, hipStream_t stream);
 // The contraction over a tile plan (wcn_conv_tiles.hip): whether it takes a problem's shape, and its launch
 // (X, Wt, bias, residual, relu, out and the sizes are read from `a`).
 bool wcn_conv_tiles_takes(int dtype, int num_offsets, int c_in, int c_out);
+bool wcn_conv_tiles_rows(int num_offsets, int c_in, int c_out, int64_t num_out);  // enough rows for a plan, whatever the pairs
 int wcn_conv_tiles_worth(int num_offsets, int c_in, int c_out, int64_t num_out, const int64_t* host_offsets, int identity,
                          int calls);
 int wcn_conv_tiles_launch(const ConvArgs& a, int dtype, const WcnTilePlan& plan, hipStream_t stream);

@@ -364,10 +364,13 @@ int wcn_conv_tiles_worth(int K, int c_in, int c_out, int64_t num_out, const int6
   }
   // effective number of offsets: 26 of 26 for noise, 25 for spheres, 17 to 22 for rooms
   if (squares <= 0.0 || (K > 12 && sum * sum / squares > 0.98 * (K - (identity >= 0 ? 1 : 0)))) return 0;
-  if (num_out < (K <= 12 || (c_in >= 64 && c_out > 64) ? 16384 : 32768)) return 0;
-  if (c_in <= 32 && c_out <= 32) return 0;
+  if (!wcn_conv_tiles_rows(K, c_in, c_out, num_out)) return 0;
   const double saved = (double)host_offsets[K] * (K <= 12 ? 60e-6 : 40e-6) * ((double)c_in * c_out / 8192.0);
   return saved * calls > 20.0 + 70e-6 * num_out ? 3 : 2;
+}
+
+bool wcn_conv_tiles_rows(int K, int c_in, int c_out, int64_t num_out) {
+  return num_out >= (K <= 12 || (c_in >= 64 && c_out > 64) ? 16384 : 32768) && !(c_in <= 32 && c_out <= 32);
 }
 
 int wcn_conv_tiles_launch(const ConvArgs& a, int dtype, const WcnTilePlan& plan, hipStream_t s) {

@@ -215,6 +215,20 @@ py::tuple stride_cells(const py::object& table, const Int3& stride, bool want_bo
   }
 }
 
+/* A layer without gradients whose map is about to be made, for kernel_map to run between the map's launches and the wait for its
+ * offsets.  `out` stays undefined where the layer is none that can: it is then run behind the map, as any other. */
+struct LayerAhead {
+  Tensor features;
+  py::object weight;
+  std::optional<Tensor> bias, residual;
+  std::optional<at::ScalarType> compute_dtype;
+  bool relu = false, keep_tiles = false;
+  int64_t identity = -1;
+  Tensor out;
+  void launch(const Tensor& in_maps, const Tensor& out_maps, const void* map_result, const int32_t* groups, int32_t K,
+              int64_t num_out);
+};
+
 /* Kernel map of (m, 4) output rows over a coordinate table: count pass, emit pass into buffers of
  * assumed size (`per_row` pairs a row), one wait for the offsets; with more pairs than assumed the
  * emit pass has written nothing and runs again into exact buffers.  Returns (in_maps, out_maps,
@@ -222,7 +236,7 @@ py::tuple stride_cells(const py::object& table, const Int3& stride, bool want_bo
  * flags, where (and, with work behind the wait, when) the lists were made). */
 py::tuple kernel_map(const py::object& table, const Tensor& out4, const Int3& ks, const Int3& st,
                      const std::optional<Int3>& dilation, const std::optional<Int3>& centre, double per_row,
-                     int64_t keep_workspace_bytes) {
+                     int64_t keep_workspace_bytes, LayerAhead* ahead) {
   at::AutoDispatchBelowADInplaceOrView guard;
   const int64_t M = out4.size(0);
   const int32_t K = ks[0] * ks[1] * ks[2];
@@ -269,6 +283,8 @@ py::tuple kernel_map(const py::object& table, const Tensor& out4, const Int3& ks
     begin = reinterpret_cast<const char*>(wcn_kmap_group_start(w, M, K)) - static_cast<const char*>(w);
     kept = ws.narrow(0, 0, begin + 4 * int64_t{K} * ((M + 63) / 64 + 1));
     if (ws.numel() > keep_workspace_bytes) kept = kept.clone();
+    // what a layer needs of the map is on its way: with it behind, the GPU has work while the host takes the offsets in
+    if (ahead) ahead->launch(in_buf, out_buf, w, wcn_kmap_group_start(w, M, K), K, M);
     int status;
     {
       py::gil_scoped_release unlocked;
@@ -282,6 +298,7 @@ py::tuple kernel_map(const py::object& table, const Tensor& out4, const Int3& ks
     table.attr("_checked") = true;
     const int64_t total = host_offsets[K];
     if (total > assumed) {
+      if (ahead) ahead->out = Tensor();  // it has found no lists
       in_buf = at::empty({total}, out4.options());
       out_buf = at::empty({total}, out4.options());
       fill(total, in_buf, out_buf);
@@ -404,6 +421,54 @@ Tensor prepared_tiles(const py::object& weight_obj, const Tensor& weight, const 
   p->shape = weight.sizes().vec();
   if (py::hasattr(weight_obj, "__dict__")) weight_obj.attr("_wcn_prepared") = py::make_tuple(p, tiles);
   return tiles;
+}
+
+bool kernel_bias(const Tensor& bias, const Tensor& features, int64_t c_out);
+bool aligned16(const void* p);
+
+void LayerAhead::launch(const Tensor& in_maps, const Tensor& out_maps, const void* map_result, const int32_t* groups, int32_t K,
+                        int64_t num_out) {
+  out = Tensor();
+  const Tensor w = weight.cast<Tensor>();
+  const at::ScalarType dtype = features.scalar_type();
+  const int code = dtype_code(dtype);
+  // what conv_forward has to convert, copy, pad or refuse is left to it
+  if (code < 0 || !features.is_cuda() || features.dim() != 2 || w.dim() != 3 || w.size(0) != K || w.size(1) != features.size(1) ||
+      w.device() != features.device() || features.device() != in_maps.device() || !features.is_contiguous() || !w.is_contiguous() ||
+      (w.scalar_type() != dtype && w.scalar_type() != at::kFloat) || (compute_dtype && *compute_dtype != dtype) || num_out == 0 ||
+      features.size(0) == 0 || features.size(0) * features.element_size() == 0 || w.size(2) > INT32_MAX || w.size(1) > INT32_MAX)
+    return;
+  const int32_t c_in = static_cast<int32_t>(w.size(1)), c_out = static_cast<int32_t>(w.size(2));
+  const void* const px = features.const_data_ptr();
+  if (c_in * features.element_size() % 16 != 0 || !aligned16(px) || !wcn_conv_prepared_half(code, K, c_in, c_out, num_out, 1) ||
+      wcn_conv_tiles_sized(code, K, c_in, c_out, num_out))
+    return;
+  const bool has_bias = bias && bias->defined(), has_residual = residual && residual->defined();
+  if (has_bias && (!kernel_bias(*bias, features, c_out) || bias->scalar_type() != dtype || !bias->is_contiguous() ||
+                   !aligned16(bias->const_data_ptr())))
+    return;
+  if (has_residual && (residual->dim() != 2 || residual->size(0) != num_out || residual->size(1) != c_out || !residual->is_cuda() ||
+                       residual->device() != features.device() || residual->scalar_type() != dtype || !residual->is_contiguous()))
+    return;
+  void* stream = stream_of(features);
+  Tensor tiles;
+  if (keep_tiles) {
+    tiles = prepared_tiles(weight, w, [&]() { return w; }, dtype, c_in, 1);
+  } else {
+    const size_t nbytes = wcn_conv_prepared_weight_bytes(K, c_in, c_out, code) / 2;
+    tiles = bytes_on(nbytes, features);
+    check(wcn_conv_prepare_weight_half(w.const_data_ptr(), dtype_code(w.scalar_type()), K, c_in, c_out, code, 1,
+                                       tiles.mutable_data_ptr(), static_cast<size_t>(tiles.numel()), stream),
+          "wcn_conv_prepare_weight_half");
+  }
+  Tensor rows = at::empty({num_out, c_out}, features.options());
+  check(wcn_sparse_conv_fwd_ahead(px, features.size(0), c_in, code, tiles.const_data_ptr(), K, c_out,
+                                  has_bias ? bias->const_data_ptr() : nullptr, in_maps.const_data_ptr<int32_t>(),
+                                  out_maps.const_data_ptr<int32_t>(), in_maps.numel(), static_cast<const int64_t*>(map_result),
+                                  static_cast<int32_t>(identity), groups, has_residual ? residual->const_data_ptr() : nullptr,
+                                  relu ? 1 : 0, rows.mutable_data_ptr(), num_out, stream),
+        "wcn_sparse_conv_fwd_ahead");
+  out = rows;
 }
 
 // Plans up to this size stay with their map (4 bytes per row and offset: three times the lists of a map of a scene's
@@ -1252,7 +1317,17 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("batch_rows_table", &batch_rows_table);
   m.def("table_build", &table_build);
   m.def("stride_cells", &stride_cells);
-  m.def("kernel_map", &kernel_map);
+  py::class_<LayerAhead>(m, "LayerAhead")
+      .def(py::init([](const Tensor& features, const py::object& weight, const std::optional<Tensor>& bias,
+                       const std::optional<at::ScalarType>& compute_dtype, const std::optional<Tensor>& residual, bool relu,
+                       bool keep_tiles) {
+        return LayerAhead{features, weight, bias, residual, compute_dtype, relu, keep_tiles, -1, Tensor()};
+      }))
+      .def_property("identity", [](const LayerAhead& a) { return a.identity; },
+                    [](LayerAhead& a, std::optional<int64_t> k) { a.identity = k.value_or(-1); })
+      .def_property_readonly("out", [](const LayerAhead& a) { return a.out.defined() ? py::cast(a.out) : py::none(); });
+  m.def("kernel_map", &kernel_map, py::arg("table"), py::arg("rows"), py::arg("kernel_size"), py::arg("stride"), py::arg("dilation"),
+        py::arg("centre"), py::arg("per_row"), py::arg("keep_workspace_bytes"), py::arg("ahead") = py::none());
   m.def("conv_forward", [](const Tensor& features, const py::object& weight, const py::object& km, int64_t num_out,
                            const std::optional<Tensor>& bias, const std::optional<at::ScalarType>& compute_dtype,
                            const std::optional<Tensor>& residual, bool relu, bool keep_tiles, const py::object& pairs_sorted) {

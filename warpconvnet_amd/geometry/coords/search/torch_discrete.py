@@ -68,7 +68,7 @@ _PAIRS_PER_ROW = {}
 
 def _kernel_map_from_table(table: TorchHashTable, out_coords: Tensor, kernel_size, stride,
                            identity_map_index: Optional[int], dilation=None,
-                           centres=None) -> IntSearchResult:
+                           centres=None, ahead=None) -> IntSearchResult:
     """Count, emit and read the offsets in one native call (csrc/wcn_host.cpp: kernel_map), which also
     handles the device-reported table overflow by rebuilding the table with more slots.
 
@@ -84,13 +84,15 @@ def _kernel_map_from_table(table: TorchHashTable, out_coords: Tensor, kernel_siz
     the workspace goes back to the allocator, below, the map keeps the workspace as it is and the step has no
     copy in it."""
     out4 = _four_columns(out_coords)
+    if ahead is not None:
+        ahead.identity = identity_map_index
     M = out4.shape[0]
     ks, st = _pad_kernel_args(kernel_size, 1), _pad_kernel_args(stride, 1)
     shape_key = (tuple(ks), tuple(st), M.bit_length())
     in_maps, out_maps, offsets64, offsets, groups, address, device_offsets, flags, made = native().kernel_map(
         table, out4, ks, st, None if dilation is None else _pad_kernel_args(dilation, 1),
         None if dilation is None else _pad_kernel_args(centres, 0), _PAIRS_PER_ROW.get(shape_key, 8.0),
-        _KEEP_WORKSPACE_BYTES)
+        _KEEP_WORKSPACE_BYTES, ahead)
     if M > 0:
         _PAIRS_PER_ROW[shape_key] = in_maps.shape[0] / M
     K = offsets.shape[0] - 1
@@ -235,8 +237,11 @@ def generate_kernel_map(
     method: Literal["offset", "size"] = "size",
     hash_method: HashMethod = HashMethod.CITY,
     skip_symmetric_kernel_map: bool = False,
+    _ahead=None,
 ) -> IntSearchResult:
     """Kernel map between input and output coordinates (reference: torch_discrete.py:365-466).
+    `_ahead`: the layer that is to run over the map (csrc/wcn_host.cpp: LayerAhead), launched before the map's offsets
+    have reached the host where it can be.
 
     For every kernel offset k (enumerated with the last spatial dimension fastest) and output
     row m, the query out[m] * [1, stride] + offset_k is looked up among the inputs; hits become
@@ -285,7 +290,8 @@ def generate_kernel_map(
         elif all(d == 1 for d in dilation):
             dilation = centres = None
     result = _kernel_map_from_table(table, batch_indexed_out_coords, kernel_size, stride,
-                                    identity_map_index, dilation, centres)
+                                    identity_map_index, dilation, centres,
+                                    None if skip_symmetric_kernel_map else _ahead)
     same_set = (batch_indexed_in_coords.data_ptr() == batch_indexed_out_coords.data_ptr()
                 and batch_indexed_in_coords.shape == batch_indexed_out_coords.shape
                 and batch_indexed_in_coords.stride() == batch_indexed_out_coords.stride())

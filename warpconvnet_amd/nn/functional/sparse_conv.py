@@ -224,6 +224,7 @@ def generate_output_coords_and_kernel_map(
     output_spatially_sparse_tensor: Optional[Voxels],
     stride_mode: STRIDED_CONV_MODE = STRIDED_CONV_MODE.STRIDE_ONLY,
     order=POINT_ORDERING.RANDOM,
+    _ahead=None,
 ) -> Tuple[Tensor, Tensor, IntSearchResult]:
     """Output coordinates (given / strided / same as input), then the kernel map, through the
     cache on the input tensor (reference: sparse_conv.py:1808-1996).  A transposed convolution
@@ -300,7 +301,7 @@ def generate_output_coords_and_kernel_map(
     else:
         kernel_map = generate_kernel_map(in_coords, out_coords, stride, kernel_size,
                                          kernel_dilation, method=method,
-                                         skip_symmetric_kernel_map=False)
+                                         skip_symmetric_kernel_map=False, _ahead=_ahead)
         # kernel as large as the stride over voxels without repeats: every input row is in one pair
         kernel_map._single_in = bool(
             strided and tuple(kernel_size) == tuple(stride) and all(int(d) == 1 for d in kernel_dilation)
@@ -448,14 +449,19 @@ def spatially_sparse_conv(
     features = input_sparse_tensor.feature_tensor
     effective_compute_dtype = compute_dtype if compute_dtype is not None else features.dtype
 
+    needs_grad = torch.is_grad_enabled() and (features.requires_grad or weight.requires_grad)
+    needs_residual_grad = residual is not None and torch.is_grad_enabled() and residual.requires_grad
+    ahead = None
+    if not (needs_grad or needs_residual_grad or transposed) and features.is_cuda:
+        # a layer over a small map that has to be made first does not wait for the host to have read the map's offsets
+        ahead = native().LayerAhead(features, weight, bias, effective_compute_dtype, residual, relu, keep_prepared_weight)
     out_coords, out_offsets, kernel_map = generate_output_coords_and_kernel_map(
         input_sparse_tensor=input_sparse_tensor, kernel_size=_kernel_size,
         kernel_dilation=_kernel_dilation, stride=_stride, generative=generative,
         transposed=transposed, output_spatially_sparse_tensor=output_spatially_sparse_tensor,
-        stride_mode=stride_mode, order=order)
+        stride_mode=stride_mode, order=order, _ahead=ahead)
     num_out_coords = out_coords.shape[0]
 
-    needs_grad = torch.is_grad_enabled() and (features.requires_grad or weight.requires_grad)
     if needs_grad:
         if num_out_coords == 0 or features.shape[0] == 0:
             out_features = UnifiedSpatiallySparseConvFunction.apply(
@@ -474,13 +480,14 @@ def spatially_sparse_conv(
         out_features = after(out_features)
     else:
         # inference: bias, residual and clamp are fused into the contraction's epilogue
-        needs_residual_grad = residual is not None and torch.is_grad_enabled() and residual.requires_grad
         fused = not needs_residual_grad
-        out_features = sparse_conv_forward(features, weight, kernel_map, num_out_coords, bias=bias,
-                                           compute_dtype=effective_compute_dtype,
-                                           residual=residual if fused else None,
-                                           relu=relu and fused,
-                                           keep_prepared_weight=keep_prepared_weight)
+        out_features = ahead.out if ahead is not None else None
+        if out_features is None:
+            out_features = sparse_conv_forward(features, weight, kernel_map, num_out_coords, bias=bias,
+                                               compute_dtype=effective_compute_dtype,
+                                               residual=residual if fused else None,
+                                               relu=relu and fused,
+                                               keep_prepared_weight=keep_prepared_weight)
         if not fused:
             out_features = after(out_features)
 
