@@ -60,6 +60,22 @@ def test_other_calls_stay_with_the_library(dtype, c_in, c_out, rows):
     assert not lib().wcn_pointwise_takes(rows, c_in, c_out, {torch.float32: 0, torch.float16: 1, torch.bfloat16: 2}[dtype])
 
 
+@pytest.mark.parametrize("c_in,c_out,rows,own", [(128, 64, 1, True), (256, 128, 300, True), (192, 96, 32_767, True),
+                                                 (128, 128, 32_768, True), (128, 128, 32_769, False), (256, 128, 99_999, False)])
+def test_wide_rows_over_few_voxels(c_in, c_out, rows, own):
+    w = kaiming_weight(1, c_in, c_out, seed=4, dtype=torch.bfloat16).to(DEV)
+    vox = _voxels(rows, c_in, torch.bfloat16)
+    with torch.no_grad():
+        spatially_sparse_conv(_voxels(10, 32, torch.float16), kaiming_weight(1, 32, 16, seed=1, dtype=torch.float16).to(DEV),
+                              kernel_size=1)
+        before = _kernel()
+        got = spatially_sparse_conv(vox, w, kernel_size=1).feature_tensor
+    assert (_kernel() != before) == own
+    x64, w64 = vox.feature_tensor.double(), w[0].double()
+    want, sums = x64 @ w64, c_in * 2.0 ** -24 * (x64.abs() @ w64.abs())  # fp32 sums of c_in products, then one rounding
+    assert bool(((got.double() - want).abs() <= UNIT[torch.bfloat16] * (want.abs() + sums) + sums + 2.0 ** -25).all())
+
+
 def test_gradients_transforms_and_modes_see_the_product():
     w = kaiming_weight(1, 64, 32, seed=4, dtype=torch.float16).to(DEV)
     vox = _voxels(300, 64, torch.float16)
