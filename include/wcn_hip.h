@@ -322,18 +322,21 @@ int wcn_sparse_conv_fwd_prepared_halves(const void* features, int64_t num_in, in
                                         void* out, int64_t num_out, void* workspace, size_t workspace_bytes,
                                         void* stream);
 
-/* wcn_sparse_conv_fwd_prepared_halves for a shape that the kernel for small maps takes (wcn_conv_prepared_half: 1), over the lists of
- * a map builder that the host has not waited for: in_maps / out_maps of pair_capacity places each, as given to wcn_kmap_fill,
- * map_result the first words of its workspace (offsets and status) and group_start its table.  With more pairs than
- * places, or a status that is not 0, nothing is written to `out`: the caller, who learns that from wcn_kmap_read_result, calls
- * again.  wcn_conv_tiles_sized: whether a layer over so many rows may take a tile plan, whatever its pairs. */
-int wcn_sparse_conv_fwd_ahead(const void* features, int64_t num_in, int32_t c_in, int32_t dtype, const void* half1,
+/* wcn_sparse_conv_fwd_prepared_halves over the lists of a map builder that the host has not waited for: in_maps / out_maps of
+ * pair_capacity places each, as given to wcn_kmap_fill, map_result the first words of its workspace (offsets and status) and
+ * group_start its table.  With more pairs than places, or a status that is not 0, nothing is written to `out`: the caller, who
+ * learns that from wcn_kmap_read_result, calls again.  `half` is the half of the prepared weight that wcn_conv_ahead_half names for
+ * the layer (16-byte aligned feature rows): 1 or 0, or -1 where the choice of kernel depends on the map's pairs, or is one
+ * that needs more of them, and the call is refused.  pairs_expected (what the caller thinks they will be) decides about the height of
+ * a tile and nothing else. */
+int wcn_conv_ahead_half(int32_t dtype, int32_t num_offsets, int32_t c_in, int32_t c_out, int64_t num_in, int64_t num_out,
+                        int64_t pair_capacity);
+
+int wcn_sparse_conv_fwd_ahead(const void* features, int64_t num_in, int32_t c_in, int32_t dtype, const void* half,
                               int32_t num_offsets, int32_t c_out, const void* bias_or_null, const int32_t* in_maps,
-                              const int32_t* out_maps, int64_t pair_capacity, const int64_t* map_result,
+                              const int32_t* out_maps, int64_t pair_capacity, int64_t pairs_expected, const int64_t* map_result,
                               int32_t identity_offset, const int32_t* group_start, const void* residual_or_null,
                               int32_t relu, void* out, int64_t num_out, void* stream);
-
-int wcn_conv_tiles_sized(int32_t dtype, int32_t num_offsets, int32_t c_in, int32_t c_out, int64_t num_out);
 
 /* The forward contraction over a map in which EVERY OUTPUT ROW HAS EXACTLY ONE PAIR
  * (host_offsets[num_offsets] == num_out, which is checked, and no output row twice, which the caller

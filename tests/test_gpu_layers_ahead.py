@@ -1,4 +1,4 @@
-"""Layers over small maps that are launched before the map's offsets have reached the host: the same bits as over the kept
+"""Layers that are launched before the map's offsets have reached the host: the same bits as over the kept
 map, with every extra of the epilogue; lists that turn out too short, and calls that have to wait for the map."""
 import numpy as np
 import pytest
@@ -84,6 +84,67 @@ def test_lists_that_turn_out_too_short(monkeypatch):
     vox = Voxels(torch.as_tensor(cube, device=DEV), x, offsets=torch.tensor([0, n]))
     assert torch.equal(first, spatially_sparse_conv(vox, w, 3).feature_tensor)
     assert made[-1].out is not None
+
+
+def _kernel():
+    from warpconvnet_amd._lib import lib
+    return lib().wcn_conv_last_kernel().decode()
+
+
+@pytest.mark.parametrize("n,dtype,c_in,c_out,kernel,stride,name", [
+    (70_001, torch.float16, 32, 32, 3, 1, "group"), (240_000, torch.bfloat16, 16, 13, 3, 2, "group"), (140_000, torch.float16, 8, 8, 5, 1, "group"),
+    (200_000, torch.float32, 16, 13, 3, 2, "group"), (60_007, torch.float32, 32, 16, 3, 1, "group"),
+    (50_001, torch.float32, 32, 32, 3, 1, "pack"), (30_000, torch.float32, 128, 128, 3, 1, "pack"), (160_000, torch.float32, 40, 72, 2, 2, "pack"),
+    (64_000, torch.float16, 64, 20, 3, 1, "pack"), (90_031, torch.bfloat16, 32, 60, 3, 1, "pack")])
+@pytest.mark.parametrize("extras", [False, True])
+def test_narrow_and_packed_kernels_give_the_same_bits(monkeypatch, n, dtype, c_in, c_out, kernel, stride, name, extras):
+    from warpconvnet_amd.nn.functional.sparse_conv import spatially_sparse_conv
+    made = _spied(monkeypatch)
+    w = kaiming_weight(kernel ** 3, c_in, c_out, seed=2, dtype=dtype).to(DEV)
+    kw = {"stride": stride}
+    if extras:
+        kw.update(bias=normal_features(1, c_out, seed=3, dtype=dtype)[0].to(DEV), relu=True, keep_prepared_weight=True)
+        if stride == 1:
+            kw["residual"] = normal_features(n, c_out, seed=4, dtype=dtype).to(DEV)
+    vox = _voxels(n, c_in, dtype, seed=n)
+    first = spatially_sparse_conv(vox, w, kernel, **kw).feature_tensor
+    assert len(made) == 1 and made[0].out is not None
+    assert _kernel().startswith(f"conv_fwd_{name}<"), _kernel()
+    again = spatially_sparse_conv(vox, w, kernel, **kw).feature_tensor  # the pairs are known now
+    assert made[1:] == [] or made[-1].out is None
+    assert _kernel().startswith(f"conv_fwd_{name}<"), _kernel()
+    assert torch.equal(first, again)
+
+
+@pytest.mark.parametrize("dtype,c_in,c_out,name", [(torch.float16, 32, 32, "group"), (torch.float32, 32, 32, "pack")])
+def test_narrow_and_packed_kernels_find_no_lists(monkeypatch, dtype, c_in, c_out, name):
+    from warpconvnet_amd.geometry.coords.search import torch_discrete
+    from warpconvnet_amd.geometry.types.voxels import Voxels
+    from warpconvnet_amd.nn.functional.sparse_conv import spatially_sparse_conv
+    made = _spied(monkeypatch)
+    monkeypatch.setattr(torch_discrete, "_PAIRS_PER_ROW", {})
+    cube = np.stack(np.meshgrid(*[np.arange(40)] * 3, indexing="ij"), axis=-1).reshape(-1, 3).astype(np.int32)
+    n = len(cube)
+    x = normal_features(n, c_in, seed=1, dtype=dtype).to(DEV)
+    w = kaiming_weight(27, c_in, c_out, seed=2, dtype=dtype).to(DEV)
+    vox = Voxels(torch.as_tensor(cube, device=DEV), x, offsets=torch.tensor([0, n]))
+    first = spatially_sparse_conv(vox, w, 3).feature_tensor
+    assert len(made) == 1 and made[0].out is None
+    assert _kernel().startswith(f"conv_fwd_{name}<"), _kernel()
+    vox = Voxels(torch.as_tensor(cube, device=DEV), x, offsets=torch.tensor([0, n]))
+    assert torch.equal(first, spatially_sparse_conv(vox, w, 3).feature_tensor)
+    assert made[-1].out is not None
+
+
+@pytest.mark.parametrize("dtype,num_offsets,c_in,c_out,rows,capacity,half", [
+    (1, 27, 32, 64, 1000, 27_000, 1), (1, 27, 32, 32, 70_000, 10 ** 6, 0), (0, 27, 32, 32, 100_000, 10 ** 6, 0),
+    (1, 27, 64, 64, 32_768, 10 ** 6, -1),  # a tile plan may be taken: the pairs decide
+    (1, 27, 20, 32, 70_000, 10 ** 6, -1),  # rows of other than whole 16-byte vectors
+    (2, 200, 128, 128, 5000, 10 ** 6, -1),  # slices of channels over workgroups
+    (1, 27, 32, 32, 100_000_000, 1 << 30, -1)])  # more pairs than the kernels' offsets reach
+def test_half_of_the_weight(dtype, num_offsets, c_in, c_out, rows, capacity, half):
+    from warpconvnet_amd._lib import lib
+    assert lib().wcn_conv_ahead_half(dtype, num_offsets, c_in, c_out, rows, rows, capacity) == half
 
 
 @pytest.mark.parametrize("case", ["columns", "fp32_bias", "one_bias", "half_weight", "residual_type", "three_channels", "converted"])

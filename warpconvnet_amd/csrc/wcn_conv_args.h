@@ -18,8 +18,7 @@ struct ConvArgs {
   void* out;
   int64_t num_in, num_out, G;
   int64_t num_pairs;           // all offsets together (known on the host)
-  int64_t list_capacity;       // > 0 (kernel for small maps): the lists of a builder that the host has not waited for.  They hold
-                               // what they should if offsets[K], the pairs, is at most this and offsets[K + 1], its status, 0
+  int64_t list_capacity;       // > 0: the lists of a builder that the host has not waited for (num_pairs: its guess), see lists_absent
   int32_t K, c_in, c_out, c_in_pad, c_out_pad, identity;
   int32_t vec_in;   // feature rows are 16-byte aligned and a whole number of 16-byte vectors
   int32_t vec_out;  // same for output rows
@@ -36,6 +35,12 @@ struct ConvArgs {
   int32_t relu;
   int32_t bias_rounded;  // the bias is added to the rounded sums (kernels of tile plans and single pairs)
   int32_t vec_res;  // rows of `residual` are 16-byte aligned and a whole number of 16-byte vectors
+
+  // Lists that the host has not waited for hold what they should if offsets[K], the pairs, is at most their capacity and
+  // offsets[K + 1], the builder's status, 0.  Otherwise the kernel returns at once and the host launches again.
+  __device__ __forceinline__ bool lists_absent() const {
+    return list_capacity > 0 && (offsets[K] > list_capacity || offsets[K + 1] != 0);
+  }
 };
 
 

@@ -97,6 +97,7 @@ __global__ void __launch_bounds__(WAVES * 64) conv_fwd_group(ConvArgs a) {
   constexpr int ROWF = NCB * 16;  // floats per row of sums
   constexpr int ACC_FLOATS = 65 * ROWF;  // row 64: sums of pairs that do not exist
   extern __shared__ __attribute__((aligned(16))) unsigned char group_smem[];
+  if (a.lists_absent()) return;
   // LDS: the weight operands of all offsets, [k][cb][lane], then the sums of every wave
   V* __restrict__ s_w = reinterpret_cast<V*>(group_smem);
   const int K = a.K;

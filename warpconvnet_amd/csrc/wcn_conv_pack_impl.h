@@ -212,6 +212,7 @@ __global__ void __launch_bounds__((NW + 1) * 64) conv_fwd_pack(ConvArgs a, int n
   u32x4* const wbuf = (u32x4*)(smem + R * RS);               // 2 weight tiles
   int32_t* const s_plan = (int32_t*)(wbuf + 2 * WTILE);      // PLAN_SLOTS x {cnt[128], start[128]}
   float* const s_bias = (float*)(s_plan + PLAN_SLOTS * 256); // MAX_BIAS
+  if (a.lists_absent()) return;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int K = a.K;

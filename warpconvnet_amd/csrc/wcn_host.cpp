@@ -225,8 +225,8 @@ struct LayerAhead {
   bool relu = false, keep_tiles = false;
   int64_t identity = -1;
   Tensor out;
-  void launch(const Tensor& in_maps, const Tensor& out_maps, const void* map_result, const int32_t* groups, int32_t K,
-              int64_t num_out);
+  void launch(const Tensor& in_maps, const Tensor& out_maps, int64_t expected, const void* map_result, const int32_t* groups,
+              int32_t K, int64_t num_out);
 };
 
 /* Kernel map of (m, 4) output rows over a coordinate table: count pass, emit pass into buffers of
@@ -284,7 +284,7 @@ py::tuple kernel_map(const py::object& table, const Tensor& out4, const Int3& ks
     kept = ws.narrow(0, 0, begin + 4 * int64_t{K} * ((M + 63) / 64 + 1));
     if (ws.numel() > keep_workspace_bytes) kept = kept.clone();
     // what a layer needs of the map is on its way: with it behind, the GPU has work while the host takes the offsets in
-    if (ahead) ahead->launch(in_buf, out_buf, w, wcn_kmap_group_start(w, M, K), K, M);
+    if (ahead) ahead->launch(in_buf, out_buf, static_cast<int64_t>(per_row * M), w, wcn_kmap_group_start(w, M, K), K, M);
     int status;
     {
       py::gil_scoped_release unlocked;
@@ -426,8 +426,8 @@ Tensor prepared_tiles(const py::object& weight_obj, const Tensor& weight, const 
 bool kernel_bias(const Tensor& bias, const Tensor& features, int64_t c_out);
 bool aligned16(const void* p);
 
-void LayerAhead::launch(const Tensor& in_maps, const Tensor& out_maps, const void* map_result, const int32_t* groups, int32_t K,
-                        int64_t num_out) {
+void LayerAhead::launch(const Tensor& in_maps, const Tensor& out_maps, int64_t expected, const void* map_result,
+                        const int32_t* groups, int32_t K, int64_t num_out) {
   out = Tensor();
   const Tensor w = weight.cast<Tensor>();
   const at::ScalarType dtype = features.scalar_type();
@@ -440,9 +440,9 @@ void LayerAhead::launch(const Tensor& in_maps, const Tensor& out_maps, const voi
     return;
   const int32_t c_in = static_cast<int32_t>(w.size(1)), c_out = static_cast<int32_t>(w.size(2));
   const void* const px = features.const_data_ptr();
-  if (c_in * features.element_size() % 16 != 0 || !aligned16(px) || !wcn_conv_prepared_half(code, K, c_in, c_out, num_out, 1) ||
-      wcn_conv_tiles_sized(code, K, c_in, c_out, num_out))
-    return;
+  if (c_in * features.element_size() % 16 != 0 || !aligned16(px)) return;
+  const int half = wcn_conv_ahead_half(code, K, c_in, c_out, features.size(0), num_out, in_maps.numel());
+  if (half < 0) return;
   const bool has_bias = bias && bias->defined(), has_residual = residual && residual->defined();
   if (has_bias && (!kernel_bias(*bias, features, c_out) || bias->scalar_type() != dtype || !bias->is_contiguous() ||
                    !aligned16(bias->const_data_ptr())))
@@ -453,18 +453,18 @@ void LayerAhead::launch(const Tensor& in_maps, const Tensor& out_maps, const voi
   void* stream = stream_of(features);
   Tensor tiles;
   if (keep_tiles) {
-    tiles = prepared_tiles(weight, w, [&]() { return w; }, dtype, c_in, 1);
+    tiles = prepared_tiles(weight, w, [&]() { return w; }, dtype, c_in, half);
   } else {
     const size_t nbytes = wcn_conv_prepared_weight_bytes(K, c_in, c_out, code) / 2;
     tiles = bytes_on(nbytes, features);
-    check(wcn_conv_prepare_weight_half(w.const_data_ptr(), dtype_code(w.scalar_type()), K, c_in, c_out, code, 1,
+    check(wcn_conv_prepare_weight_half(w.const_data_ptr(), dtype_code(w.scalar_type()), K, c_in, c_out, code, half,
                                        tiles.mutable_data_ptr(), static_cast<size_t>(tiles.numel()), stream),
           "wcn_conv_prepare_weight_half");
   }
   Tensor rows = at::empty({num_out, c_out}, features.options());
   check(wcn_sparse_conv_fwd_ahead(px, features.size(0), c_in, code, tiles.const_data_ptr(), K, c_out,
                                   has_bias ? bias->const_data_ptr() : nullptr, in_maps.const_data_ptr<int32_t>(),
-                                  out_maps.const_data_ptr<int32_t>(), in_maps.numel(), static_cast<const int64_t*>(map_result),
+                                  out_maps.const_data_ptr<int32_t>(), in_maps.numel(), expected, static_cast<const int64_t*>(map_result),
                                   static_cast<int32_t>(identity), groups, has_residual ? residual->const_data_ptr() : nullptr,
                                   relu ? 1 : 0, rows.mutable_data_ptr(), num_out, stream),
         "wcn_sparse_conv_fwd_ahead");
