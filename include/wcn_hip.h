@@ -157,6 +157,14 @@ int wcn_kmap_fill(const void* table, int64_t n_keys, int64_t capacity, const int
                   const void* workspace, int64_t pair_capacity, int32_t* in_maps,
                   int32_t* out_maps, void* stream);
 
+/* wcn_kmap_count (with dilation and centre, which come together: wcn_kmap_count_dilated) and a wcn_kmap_fill into lists of
+ * assumed size, in one call: the same results, for maps of up to some 260,000 rows in one launch less.  wcn_kmap_read_result and, with
+ * more pairs than places, another wcn_kmap_fill follow as they would; the lists of a table that reports a problem hold nothing of use. */
+int wcn_kmap_count_fill(const void* table, int64_t n_keys, int64_t capacity, const int32_t* out_coords, int64_t num_out,
+                        const int32_t host_kernel_size[3], const int32_t host_stride[3], const int32_t* host_dilation_or_null,
+                        const int32_t* host_centre_or_null, void* workspace, int64_t pair_capacity, int32_t* in_maps,
+                        int32_t* out_maps, void* stream);
+
 /* The map of a coordinate set onto itself (the stride-1 convolution: out_coords are the table's own
  * keys, in the same rows): the same results as wcn_kmap_count / wcn_kmap_fill with out_coords =
  * keys and stride 1, from a probe pass that walks the keys in the table's block order, where

@@ -155,3 +155,61 @@ def test_a_result_on_its_way_does_not_reach_the_next_one(oracle, then):
             assert not done.query()  # the queue was longer than this
         if turn == 1:
             torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("kernel,stride,dilation", [(3, 1, 1), (3, 2, 1), (2, 2, 1), (2, 1, 1), (5, 1, 1), (3, 1, 2), ((1, 3, 2), 1, 1)])
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 256, 257, 511, 513, 2049, 30_011, 131_073, (1 << 18), (1 << 18) + 1])
+def test_one_call_leaves_what_two_leave(n, kernel, stride, dilation):
+    """wcn_kmap_count_fill against wcn_kmap_count and wcn_kmap_fill: offsets, status, group starts and lists, also where the lists
+    are too short and a fill follows."""
+    import math
+
+    from warpconvnet_amd._lib import check, int3, lib, ptr, stream_ptr, workspace
+    from warpconvnet_amd.geometry.coords.search.torch_hashmap import TorchHashTable
+    dev, L = torch.device(DEV), lib()
+    rng = np.random.default_rng(n)
+    side = int(np.ceil(np.sqrt(n / 0.6)))
+    cells = rng.permutation(side * side)[:n]
+    rows = torch.as_tensor(np.stack([cells % 2, cells // side - 40, cells % side, cells % 5 // 3], axis=1).astype(np.int32), device=DEV)
+    table, _, slots = TorchHashTable.from_keys(rows)._raw()
+    ks = (kernel,) * 3 if isinstance(kernel, int) else kernel
+    K, k3, st, dil, centre = math.prod(ks), int3(ks), int3((stride,) * 3), int3((dilation,) * 3), int3(tuple(k // 2 for k in ks))
+    s, groups = stream_ptr(dev), (n + 63) // 64
+
+    def run(fill):
+        ws = workspace(L.wcn_kmap_workspace_bytes(n, K), dev)
+        ws.fill_(0xEE)
+        ins, outs = (torch.full((K * n + 64,), -7, dtype=torch.int32, device=DEV) for _ in range(2))
+        fill(ws, ins, outs)
+        offsets = (ctypes.c_int64 * (K + 1))()
+        check(L.wcn_kmap_read_result(ptr(ws), n, K, offsets, s), "read")
+        begin = L.wcn_kmap_group_start(ptr(ws), n, K) - ws.data_ptr()
+        starts = ws[begin:begin + 4 * K * (groups + 1)].clone()
+        return list(offsets), L.wcn_kmap_last_table_flags(), starts, ins, outs, ws[:8 * (K + 3)].clone(), ws
+
+    def two(ws, ins, outs):
+        if dilation == 1:
+            check(L.wcn_kmap_count(ptr(table), n, slots, ptr(rows), n, k3, st, ptr(ws), s), "count")
+        else:
+            check(L.wcn_kmap_count_dilated(ptr(table), n, slots, ptr(rows), n, k3, st, dil, centre, ptr(ws), s), "count")
+        check(L.wcn_kmap_fill(ptr(table), n, slots, ptr(rows), n, k3, st, ptr(ws), K * n, ptr(ins), ptr(outs), s), "fill")
+
+    def one(capacity):
+        def fill(ws, ins, outs):
+            extra = (dil, centre) if dilation != 1 else (None, None)
+            check(L.wcn_kmap_count_fill(ptr(table), n, slots, ptr(rows), n, k3, st, *extra, ptr(ws), capacity, ptr(ins), ptr(outs), s),
+                  "count_fill")
+        return fill
+
+    want = run(two)
+    pairs = want[0][K]
+    got = run(one(K * n))
+    assert got[0] == want[0] and got[1] == want[1]
+    assert all(torch.equal(a, b) for a, b in zip(got[2:6], want[2:6]))
+    if pairs:
+        exact = run(one(pairs))
+        assert all(torch.equal(a, b) for a, b in zip(exact[2:6], want[2:6]))
+        short = run(one(pairs - 1))
+        assert short[0] == want[0] and torch.equal(short[2], want[2]) and bool((short[3] == -7).all()) and bool((short[4] == -7).all())
+        check(L.wcn_kmap_fill(ptr(table), n, slots, ptr(rows), n, k3, st, ptr(short[6]), K * n, ptr(short[3]), ptr(short[4]), s), "fill")
+        assert torch.equal(short[3], want[3]) and torch.equal(short[4], want[4])

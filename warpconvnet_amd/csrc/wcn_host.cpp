@@ -269,14 +269,13 @@ py::tuple kernel_map(const py::object& table, const Tensor& out4, const Int3& ks
     };
     if (blocks) {
       check(wcn_kmap_count_self(raw, n, t.slots, ks.data(), w, stream), "wcn_kmap_count_self");
-    } else if (!dilation) {
-      check(wcn_kmap_count(raw, n, t.slots, rows, M, ks.data(), st.data(), w, stream), "wcn_kmap_count");
+      fill(assumed, in_buf, out_buf);
     } else {
-      check(wcn_kmap_count_dilated(raw, n, t.slots, rows, M, ks.data(), st.data(), dilation->data(), centre->data(), w,
-                                   stream),
-            "wcn_kmap_count_dilated");
+      check(wcn_kmap_count_fill(raw, n, t.slots, rows, M, ks.data(), st.data(), dilation ? dilation->data() : nullptr,
+                                dilation ? centre->data() : nullptr, w, assumed, in_buf.mutable_data_ptr<int32_t>(),
+                                out_buf.mutable_data_ptr<int32_t>(), stream),
+            "wcn_kmap_count_fill");
     }
-    fill(assumed, in_buf, out_buf);
     // What stays with the map is the workspace's head: its K + 1 offsets and the group starts.  Up to
     // keep_workspace_bytes the workspace itself is kept; beyond, the head is copied, here, so that
     // nothing stands between the wait below and what the caller launches next.

@@ -35,8 +35,20 @@ struct KmapWorkspace {  // host-computed addresses inside a kmap workspace
                         // all hits of the group; after the scan, exclusive prefix sums
   int32_t* found;       // (G, 64 K): input rows found by the hit lanes of a group, packed offset by offset
   uint16_t* tags;       // (G, 64 K): offset << 6 | lane of each of them
+  uint16_t* counts;     // (K, C): hits per offset of the probe's workgroups of 256 rows (maps that kmap_starts_emit finishes)
   int64_t G;            // number of 64-row groups
+  int32_t C;            // number of the probe's workgroups, in whole 16-byte vectors of counts
 };
+
+// Up to so many rows the emit pass adds up the counts of all 256-row workgroups itself (kmap_starts_emit).  What every
+// workgroup reads grows with the rows, and so does the number of workgroups.  us of a call that makes a map, scan and emit pass / in one:
+//     rows      1,800      15,000     60,000     120,000    180,000    260,000    400,000     600,000     1,000,000
+//     2x2x2   16.8 15.7  17.2 16.1  18.1 16.5  18.1 17.0  18.8 16.8  19.2 17.7  22.1  20.1  26.9  24.5   36.3  36.1
+//     3x3x3   20.1 19.4  22.2 20.3  24.6 22.8  26.9 25.2  28.5 26.1  32.4 28.7  46.0  46.0  59.1  61.1   88.3 104.5
+//     5x5x5   38.5 35.6  40.6 37.5  44.4 40.7  51.0 44.7  57.1 56.3  63.2 61.2  92.7 111.4   124   156    192   292
+// (the emit pass overlaps the host's read here; with a layer behind it a map of 1,800 to 60,000 rows gains 4 to 5: scan 5.6 and emit
+// 5.4 us against 6.3 together.)
+constexpr int64_t KMAP_OWN_SUMS = 1 << 18;
 
 inline size_t kmap_layout(void* base, int64_t num_out, int32_t K, KmapWorkspace* w) {
   char* p = (char*)base;
@@ -55,7 +67,11 @@ inline size_t kmap_layout(void* base, int64_t num_out, int32_t K, KmapWorkspace*
   static_assert(WCN_MAX_OFFSETS <= 1024, "offset and lane share 16 bits");
   if (w) w->tags = (uint16_t*)(p + off);
   off += wcn_align256(sizeof(uint16_t) * (size_t)K * (size_t)G * 64);
+  const int64_t C = ((num_out + 255) / 256 + 7) / 8 * 8;
+  if (w) w->counts = (uint16_t*)(p + off);
+  if (num_out <= KMAP_OWN_SUMS) off += wcn_align256(sizeof(uint16_t) * (size_t)K * (size_t)C);
   if (w) w->G = G;
+  if (w) w->C = (int32_t)C;
   return off;
 }
 
@@ -68,6 +84,8 @@ struct KmapProbe {      // what the probe pass leaves for the scan and the emit 
   int32_t* found;
   uint16_t* tags;
   int32_t* ticket;      // set to zero
+  uint16_t* counts;     // (fixed sizes) null: not asked for
+  int32_t C;
 };
 
 // ---- generic kernel: any kernel size up to WCN_MAX_OFFSETS offsets -----------------------------
@@ -340,6 +358,8 @@ __global__ void __launch_bounds__(256) kmap_pass_fixed(const WcnTableHeader* __r
   const int there = (int)(G - (group - wave) < 4 ? G - (group - wave) : 4);
   for (int i = tid; i < 4 * (K + 1); i += 256)
     if ((i & 3) < there) groups[(int64_t)(i >> 2) * (G + 1) + (group - wave) + (i & 3)] = s_count[i & 3][i >> 2];
+  if (o.counts && tid < K)
+    o.counts[tid * o.C + (int)(group >> 2)] = (uint16_t)(s_count[0][tid] + s_count[1][tid] + s_count[2][tid] + s_count[3][tid]);
 }
 
 // Emit pass: pair lists from the scanned counts and what the probe pass has parked, a lane per
@@ -1037,6 +1057,194 @@ __global__ void __launch_bounds__(SELF_CHUNK) self_emit(const uint32_t* __restri
   }
 }
 
+// The scan and the emit pass of a small map in one: every workgroup adds up the counts of all of the probe's workgroups, which takes
+// the launch, and the wait for it, of kmap_scan_rows out of the chain.  It writes what the scan and the emit pass write
+// (but the starts of the row of all hits, which nothing reads): the first workgroup the offsets, the table's status and the host's
+// mailbox, and every one the starts of its own eight groups, in the place of their counts, which no other workgroup reads.
+// KL: counts of a wave's offsets requested together.
+template <int KL>
+__global__ void __launch_bounds__(512) kmap_starts_emit(const int32_t* __restrict__ found, const uint16_t* __restrict__ tags,
+                                                        int32_t* __restrict__ groups, const uint16_t* __restrict__ counts,
+                                                        int32_t blocks, int32_t C, int32_t K, int64_t G, int64_t pair_capacity,
+                                                        int32_t* __restrict__ in_maps, int32_t* __restrict__ out_maps,
+                                                        KmapFinish fin) {
+  constexpr int GROUPS = 8, MAX_K = 128;
+  __shared__ int32_t s_all[MAX_K], s_before[MAX_K];  // hits of an offset: of all workgroups, of those before this one
+  __shared__ int32_t s_base[MAX_K];                  // where its pairs begin in the lists
+  __shared__ int32_t s_start[MAX_K][GROUPS + 1];
+  __shared__ int32_t s_shift[GROUPS][MAX_K];
+  __shared__ int32_t s_stat[3][GROUPS];
+  __shared__ int32_t s_total;
+  const int tid = threadIdx.x, lane = wcn_lane(), wave = tid >> 6;
+  const int tile = wcn_xcd_tile((int)blockIdx.x, (int)gridDim.x);
+  const int64_t first = (int64_t)tile * GROUPS, group = first + wave;
+  const int own = tile * 2;  // the first of the probe's workgroups whose groups these are
+
+  // everything that needs no sum is requested first: the counts of this workgroup's groups, and the first parked pairs of
+  // every wave's group (of 64 K places, 512 and more)
+  int mine[2];
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+    const int i = tid + 512 * t, k = i >> 3;
+    mine[t] = k < K && first + (i & 7) < G ? groups[(int64_t)k * (G + 1) + first + (i & 7)] : 0;
+  }
+  const int64_t parked = (group < G ? group : 0) * (64 * (int64_t)K);
+  const int32_t* const rows = found + parked;
+  const uint16_t* const of = tags + parked;
+  constexpr int AHEAD = 4;
+  int32_t row[AHEAD];
+  uint32_t tag[AHEAD];
+#pragma unroll
+  for (int u = 0; u < AHEAD; ++u) {
+    row[u] = rows[64 * u + lane];
+    tag[u] = of[64 * u + lane];
+  }
+
+  // a wave looks after the offsets wave, wave + 8, ...; a lane takes eight counts at a time
+  typedef uint32_t Counts __attribute__((ext_vector_type(4)));
+  for (int k0 = wave; k0 < K; k0 += GROUPS * KL) {
+    int all[KL], before[KL];
+#pragma unroll
+    for (int j = 0; j < KL; ++j) all[j] = before[j] = 0;
+    for (int b0 = 0; b0 < blocks; b0 += 512) {
+      const int b = b0 + lane * 8, at = b < C ? b : 0;
+      Counts n[KL];
+#pragma unroll
+      for (int j = 0; j < KL; ++j) {
+        const int k = k0 + GROUPS * j < K ? k0 + GROUPS * j : k0;
+        n[j] = *reinterpret_cast<const Counts*>(counts + (int64_t)k * C + at);
+      }
+#pragma unroll
+      for (int j = 0; j < KL; ++j) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const int v = (int)((n[j][e >> 1] >> (16 * (e & 1))) & 0xFFFFu);
+          all[j] += b + e < blocks ? v : 0;
+          before[j] += b + e < own ? v : 0;
+        }
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < KL; ++j) {
+      const int a = wcn_wave_inclusive_sum(all[j]), p = wcn_wave_inclusive_sum(before[j]);
+      if (lane == 63 && k0 + GROUPS * j < K) {
+        s_all[k0 + GROUPS * j] = a;
+        s_before[k0 + GROUPS * j] = p;
+      }
+    }
+  }
+  if (tile == 0) {  // the table's status: the sums of its bins' counts
+    const int32_t bins = fin.hdr->bins;
+    const int32_t* stats = reinterpret_cast<const int32_t*>(reinterpret_cast<const char*>(fin.hdr) + fin.hdr->stats_offset);
+    int voxels = 0, occupied = 0;
+    bool lost = false;
+    for (int i = tid; i < bins; i += 512) {
+      voxels += stats[2 * i];
+      occupied += stats[2 * i + 1] & ~WCN_BIN_LOST;
+      lost |= (stats[2 * i + 1] & WCN_BIN_LOST) != 0;
+    }
+    voxels = wcn_wave_inclusive_sum(voxels);
+    occupied = wcn_wave_inclusive_sum(occupied);
+    const bool any_lost = __ballot(lost) != 0ull;
+    if (lane == 63) {
+      s_stat[0][wave] = voxels;
+      s_stat[1][wave] = occupied;
+      s_stat[2][wave] = any_lost ? WCN_DEV_OVERFLOW : 0;
+    }
+  }
+  __syncthreads();
+  if (wave == 0) {
+    int run = 0;
+    for (int k0 = 0; k0 < K; k0 += 64) {
+      const int k = k0 + lane, n = k < K ? s_all[k] : 0;
+      const int incl = run + wcn_wave_inclusive_sum(n);
+      if (k < K) {
+        s_base[k] = incl - n;
+        if (tile == 0) {
+          fin.result[k + 1] = incl;
+          if (fin.mailbox) fin.mailbox[1 + k + 1] = incl;
+        }
+      }
+      run = __shfl(incl, 63, 64);
+    }
+    if (lane == 0) s_total = run;
+    if (tile == 0) {
+      if (lane == 0) {
+        int voxels = 0, occupied = 0, status = fin.hdr->num_keys > 0 && !wcn_make_layout(fin.hdr).ok ? WCN_DEV_RANGE : 0;
+        for (int w = 0; w < GROUPS; ++w) {
+          voxels += s_stat[0][w];
+          occupied += s_stat[1][w];
+          status |= s_stat[2][w];
+        }
+        const int64_t all_bits =
+            (int64_t)occupied | ((int64_t)(voxels != fin.hdr->num_keys ? 1 : 0) << 32) | (int64_t)status << 33;
+        fin.result[0] = 0;
+        fin.result[K + 1] = status;
+        fin.result[K + 2] = all_bits;
+        if (fin.mailbox) {
+          fin.mailbox[1] = 0;
+          fin.mailbox[1 + K + 1] = status;
+          fin.mailbox[1 + K + 2] = all_bits;
+        }
+      }
+      if (fin.mailbox) {  // the host polls the sequence word, see kmap_scan_rows
+        __threadfence_system();
+        if (lane == 0) __hip_atomic_store(&fin.mailbox[0], fin.sequence, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+      }
+    }
+  }
+  // the starts of the groups, eight lanes an offset
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+    const int i = tid + 512 * t, k = i >> 3, j = i & 7;
+    int incl = mine[t];
+#pragma unroll
+    for (int d = 1; d < 8; d <<= 1) {
+      const int o = __shfl_up(incl, d, 8);
+      if (j >= d) incl += o;
+    }
+    if (k < K) {
+      const int start = s_before[k] + incl - mine[t];
+      s_start[k][j] = start;
+      if (j == 7) s_start[k][8] = start + mine[t];
+      if (first + j < G) groups[(int64_t)k * (G + 1) + first + j] = start;
+      if (tile == (int)gridDim.x - 1 && j == 7) groups[(int64_t)k * (G + 1) + G] = s_all[k];
+    }
+  }
+  __syncthreads();
+  if (s_total > pair_capacity || group >= G) return;
+  int total = 0;
+  for (int k0 = 0; k0 < K; k0 += 64) {
+    const int k = k0 + lane;
+    const int start = k < K ? s_start[k][wave] : 0, n = k < K ? s_start[k][wave + 1] - start : 0;
+    const int incl = wcn_wave_inclusive_sum(n);
+    if (k < K) s_shift[wave][k] = s_base[k] + start - (total + incl - n);
+    total += __shfl(incl, 63, 64);
+  }
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  for (int p0 = 0; p0 < total; p0 += 64 * AHEAD) {
+    if (p0 > 0) {
+#pragma unroll
+      for (int u = 0; u < AHEAD; ++u) {
+        const int p = p0 + 64 * u + lane;
+        row[u] = rows[p < total ? p : 0];
+        tag[u] = of[p < total ? p : 0];
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < AHEAD; ++u) {
+      const int p = p0 + 64 * u + lane;
+      if (p < total) {
+        const int dst = s_shift[wave][tag[u] >> 6] + p;
+        in_maps[dst] = row[u];
+        out_maps[dst] = (int32_t)(group * 64) + (int32_t)(tag[u] & 63u);
+      }
+    }
+  }
+}
+
 bool make_geom(const int32_t ks[3], const int32_t st[3], const int32_t* dil, const int32_t* centre,
                KmapGeom* g) {
   if (!ks || !st) return false;
@@ -1069,10 +1277,10 @@ inline bool table_args_ok(const void* table, int64_t n_keys, int64_t capacity) {
 }
 
 void launch_probe(const WcnTableView& v, const int32_t* out_coords, int64_t num_out,
-                  const KmapGeom& g, const KmapWorkspace& w, hipStream_t s) {
+                  const KmapGeom& g, const KmapWorkspace& w, hipStream_t s, bool counts = false) {
   const dim3 grid(grid_for(num_out, 256)), block(256);
   const WcnTableRef table = wcn_table_ref(v);
-  const KmapProbe o = {w.found, w.tags, w.ticket};
+  const KmapProbe o = {w.found, w.tags, w.ticket, counts ? w.counts : nullptr, w.C};
   if (is_fixed_size(g, 3, 3, 3)) {
     hipLaunchKernelGGL((kmap_pass_fixed<3, 3, 3, false>), grid, block, 0, s, v.hdr, table,
                        v.perm, (const int4*)out_coords, num_out, g, w.groups, w.G, o);
@@ -1089,6 +1297,24 @@ void launch_probe(const WcnTableView& v, const int32_t* out_coords, int64_t num_
     hipLaunchKernelGGL(kmap_pass, grid, block, 0, s, v.hdr, table, v.perm,
                        (const int4*)out_coords, num_out, g, w.groups, w.G, o);
   }
+}
+
+// Whether kmap_starts_emit finishes a map: one that kmap_pass_fixed probes (its workgroups leave their counts), with few enough of them.
+bool own_sums(const KmapGeom& g, int64_t num_out) {
+  return num_out > 0 && num_out <= KMAP_OWN_SUMS &&
+         (is_fixed_size(g, 3, 3, 3) || is_fixed_size(g, 2, 2, 2) || is_fixed_size(g, 5, 5, 5));
+}
+
+void launch_starts_emit(int64_t num_out, const KmapGeom& g, const KmapWorkspace& w, int64_t pair_capacity, int32_t* in_maps,
+                        int32_t* out_maps, const KmapFinish& fin, hipStream_t s) {
+  const dim3 grid(grid_for(num_out, 512)), block(512);
+  const int32_t blocks = (int32_t)((num_out + 255) / 256);
+  if (g.K <= 8)
+    hipLaunchKernelGGL(kmap_starts_emit<1>, grid, block, 0, s, w.found, w.tags, w.groups, w.counts, blocks, w.C, g.K, w.G,
+                       pair_capacity, in_maps, out_maps, fin);
+  else
+    hipLaunchKernelGGL(kmap_starts_emit<4>, grid, block, 0, s, w.found, w.tags, w.groups, w.counts, blocks, w.C, g.K, w.G,
+                       pair_capacity, in_maps, out_maps, fin);
 }
 
 void launch_emit(int64_t num_out, const KmapGeom& g, const KmapWorkspace& w, int64_t pair_capacity,
@@ -1426,19 +1652,22 @@ size_t wcn_kmap_workspace_bytes(int64_t num_out, int32_t num_offsets) {
 static int kmap_count_impl(const void* table, int64_t n_keys, int64_t capacity, const int32_t* out_coords,
                            int64_t num_out, const int32_t host_kernel_size[3],
                            const int32_t host_stride[3], const int32_t* host_dilation,
-                           const int32_t* host_centre, void* workspace, void* stream) {
+                           const int32_t* host_centre, void* workspace, void* stream, bool fill = false,
+                           int64_t pair_capacity = 0, int32_t* in_maps = nullptr, int32_t* out_maps = nullptr) {
   KmapGeom g;
   if (!make_geom(host_kernel_size, host_stride, host_dilation, host_centre, &g)) return WCN_ERR_INVALID_ARGUMENT;
   if (!table_args_ok(table, n_keys, capacity) || !workspace || num_out < 0 ||
       num_out >= (1ll << 31) || (num_out > 0 && !out_coords))
     return WCN_ERR_INVALID_ARGUMENT;
+  if (fill && (pair_capacity < 0 || (num_out > 0 && pair_capacity > 0 && (!in_maps || !out_maps)))) return WCN_ERR_INVALID_ARGUMENT;
   hipStream_t s = (hipStream_t)stream;
   WcnTableView v;
   wcn_table_layout(const_cast<void*>(table), n_keys, capacity, &v);
   KmapWorkspace w;
   kmap_layout(workspace, num_out, g.K, &w);
+  const bool together = fill && own_sums(g, num_out);
   if (w.G > 0) {
-    launch_probe(v, out_coords, num_out, g, w, s);
+    launch_probe(v, out_coords, num_out, g, w, s, together);
   } else {
     hipLaunchKernelGGL(kmap_zero_ticket, dim3(1), dim3(1), 0, s, w.ticket);
   }
@@ -1454,14 +1683,28 @@ static int kmap_count_impl(const void* table, int64_t n_keys, int64_t capacity, 
   }
   set_pending(Pending::map, sequence, w.result);
   const KmapFinish fin = {w.result, w.ticket, v.hdr, g.K, box, sequence};
-  hipLaunchKernelGGL(kmap_scan_rows, dim3(g.K + 1), dim3(1024), 0, s, w.groups, w.G, w.row_total, fin);
+  if (together) launch_starts_emit(num_out, g, w, pair_capacity, in_maps, out_maps, fin, s);
+  else hipLaunchKernelGGL(kmap_scan_rows, dim3(g.K + 1), dim3(1024), 0, s, w.groups, w.G, w.row_total, fin);
   WCN_LAUNCH_CHECK();
   if (box) {
     if (wcn_mailbox_mark(s) != WCN_OK) return WCN_ERR_LAUNCH;
   } else if (wcn_read_early_begin(w.result, sizeof(int64_t) * (size_t)(g.K + 3), s) != WCN_OK) {
     return WCN_ERR_LAUNCH;
   }
+  if (fill && !together && num_out > 0 && pair_capacity > 0) {
+    launch_emit(num_out, g, w, pair_capacity, in_maps, out_maps, s);
+    WCN_LAUNCH_CHECK();
+  }
   return WCN_OK;
+}
+
+int wcn_kmap_count_fill(const void* table, int64_t n_keys, int64_t capacity, const int32_t* out_coords, int64_t num_out,
+                        const int32_t host_kernel_size[3], const int32_t host_stride[3], const int32_t* host_dilation_or_null,
+                        const int32_t* host_centre_or_null, void* workspace, int64_t pair_capacity, int32_t* in_maps,
+                        int32_t* out_maps, void* stream) {
+  if (!host_dilation_or_null != !host_centre_or_null) return WCN_ERR_INVALID_ARGUMENT;
+  return kmap_count_impl(table, n_keys, capacity, out_coords, num_out, host_kernel_size, host_stride, host_dilation_or_null,
+                         host_centre_or_null, workspace, stream, true, pair_capacity, in_maps, out_maps);
 }
 
 int wcn_kmap_count(const void* table, int64_t n_keys, int64_t capacity, const int32_t* out_coords,
