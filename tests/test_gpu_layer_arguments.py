@@ -133,3 +133,22 @@ def test_errors_inside_a_backward_pass_are_the_package_s_own():
     offsets.copy_(right)
     out.backward(torch.ones_like(out))
     assert x.grad is not None
+
+
+@pytest.mark.parametrize("n", [63, 3000, 20_001])
+@pytest.mark.parametrize("dtype,c_in,c_out,kernel,name", [
+    (torch.float16, 32, 32, 3, "group"), (torch.bfloat16, 16, 24, 3, "group"), (torch.float32, 16, 13, 3, "group"), (torch.float16, 8, 9, 5, "group"),
+    (torch.float16, 32, 64, 3, "pack"), (torch.bfloat16, 64, 40, 3, "pack"), (torch.float32, 32, 32, 3, "pack"), (torch.float16, 64, 13, 3, "pack"),
+    (torch.bfloat16, 256, 128, 3, "ring")])
+def test_a_bias_is_added_to_the_rounded_product(n, dtype, c_in, c_out, kernel, name):
+    """A layer with gradients: the bits of the product and an addition behind it, in the kernel or as a launch of its own."""
+    from warpconvnet_amd._lib import lib
+    from warpconvnet_amd.nn.functional.sparse_conv import spatially_sparse_conv
+    vox = _voxels(n, c_in, dtype)
+    w = kaiming_weight(kernel ** 3, c_in, c_out, seed=2, dtype=torch.float32).to(DEV).requires_grad_(True)
+    weight = w if dtype == torch.float32 else w.to(dtype)
+    product = spatially_sparse_conv(vox, weight, kernel).feature_tensor
+    for b in (normal_features(1, c_out, seed=4, dtype=dtype)[0].to(DEV), normal_features(1, c_out, seed=4, dtype=torch.float32)[0].to(DEV)):
+        got = spatially_sparse_conv(vox, weight, kernel, bias=b).feature_tensor
+        assert lib().wcn_conv_last_kernel().decode().startswith(f"conv_fwd_{name}<")
+        assert torch.equal(got, product + b.to(dtype))

@@ -1514,7 +1514,7 @@ static int conv_run(const void* features, int64_t num_in, int32_t c_in, int32_t 
   a.bias = bias_or_null;
   a.residual = residual_or_null;
   a.relu = relu ? 1 : 0;
-  a.bias_rounded = 0;  // (that bias comes behind the kernel here)
+  a.bias_rounded = 0;
   a.out = out;
   a.num_in = num_in;
   a.num_out = num_out;
@@ -1565,13 +1565,7 @@ static int conv_run(const void* features, int64_t num_in, int32_t c_in, int32_t 
     bias_src = (const float*)bias_or_null;
     a.bias = w.bias;
   }
-  // a bias that is added to the rounded sums is added behind the kernel
-  const void* bias_behind = nullptr;
-  if (bias_or_null && bias_after_rounding) {
-    if (residual_or_null || relu) return WCN_ERR_INVALID_ARGUMENT;
-    bias_behind = a.bias;
-    a.bias = nullptr;
-  }
+  if (bias_or_null && bias_after_rounding && (residual_or_null || relu)) return WCN_ERR_INVALID_ARGUMENT;
   if (prepared) {
     void* zero_page_address = nullptr;
     if (const int st = static_zero_page(&zero_page_address)) return st;
@@ -1607,6 +1601,18 @@ static int conv_run(const void* features, int64_t num_in, int32_t c_in, int32_t 
     hipLaunchKernelGGL(conv_group_start, dim3((unsigned)((items + 255) / 256)), dim3(256), 0, s,
                        out_maps, (const int64_t*)w.offsets, num_offsets, w.G, w.group_start);
     a.group_start = w.group_start;
+  }
+  // A bias that is added to the rounded sums: the kernels for narrow rows and the pair-packed one round in between, behind any other it
+  // is a launch of its own (4 us and the wait for it, over 24,000 rows of 32 channels).
+  const void* bias_behind = nullptr;
+  if (bias_or_null && bias_after_rounding) {
+    const int only = kernel_choice();
+    const bool dense = only == 0 && wcn_conv_dense_takes(a, dtype);
+    a.bias_rounded = !dense && ((only == 0 && wcn_conv_group_takes(a, dtype)) || (only != 1 && wcn_conv_pack_takes(a, dtype)));
+    if (!a.bias_rounded) {
+      bias_behind = a.bias;
+      a.bias = nullptr;
+    }
   }
   if (small) {
     if (g_time_start) (void)hipEventRecord(g_time_start, s);

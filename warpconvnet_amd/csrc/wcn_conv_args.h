@@ -33,7 +33,7 @@ struct ConvArgs {
   // on the fp32 sums before the one rounding.
   const void* residual;
   int32_t relu;
-  int32_t bias_rounded;  // the bias is added to the rounded sums (kernels of tile plans and single pairs)
+  int32_t bias_rounded;  // the bias is added to the rounded sums (not in the kernels for small maps and wide rows and the ring)
   int32_t vec_res;  // rows of `residual` are 16-byte aligned and a whole number of 16-byte vectors
 
   // Lists that the host has not waited for hold what they should if offsets[K], the pairs, is at most their capacity and

@@ -335,6 +335,10 @@ __global__ void __launch_bounds__(WAVES * 64) conv_fwd_group(ConvArgs a) {
         const f32x4 hi4 = *granule(r, cpart * 2 + 1);
         float v[8] = {lo4[0], lo4[1], lo4[2], lo4[3], hi4[0], hi4[1], hi4[2], hi4[3]};
         const int col = cpart * 8;
+        if (a.bias_rounded) {
+#pragma unroll
+          for (int e = 0; e < 8; ++e) v[e] = to_float(from_float<T>(v[e]));
+        }
 #pragma unroll
         for (int e = 0; e < 8; ++e) v[e] += bias_v[e];
         if (a.relu) {  // (the residual went into the sums at the group's start)

@@ -597,6 +597,10 @@ __global__ void __launch_bounds__((NW + 1) * 64) conv_fwd_pack(ConvArgs a, int n
             *s0 = (f32x4){0.f, 0.f, 0.f, 0.f};
             *s1 = (f32x4){0.f, 0.f, 0.f, 0.f};
             float v[8] = {v0[0], v0[1], v0[2], v0[3], v1[0], v1[1], v1[2], v1[3]};
+            if (a.bias_rounded) {
+#pragma unroll
+              for (int e = 0; e < 8; ++e) v[e] = to_float(from_float<T>(v[e]));
+            }
 #pragma unroll
             for (int e = 0; e < 8; ++e) v[e] += bias_v[e];
             if (a.residual) {
