@@ -336,9 +336,20 @@ int wcn_sparse_conv_fwd_prepared_halves(const void* features, int64_t num_in, in
  * learns that from wcn_kmap_read_result, calls again.  `half` is the half of the prepared weight that wcn_conv_ahead_half names for
  * the layer (16-byte aligned feature rows): 1 or 0, or -1 where the choice of kernel depends on the map's pairs, or is one
  * that needs more of them, and the call is refused.  pairs_expected (what the caller thinks they will be) decides about the height of
- * a tile and nothing else. */
+ * a tile and nothing else.  wcn_sparse_conv_fwd_graph_ahead: the same for wcn_sparse_conv_fwd_graph, where
+ * wcn_conv_graph_ahead gives 1; the workspace is wcn_conv_workspace_bytes for no pairs and ascending lists. */
 int wcn_conv_ahead_half(int32_t dtype, int32_t num_offsets, int32_t c_in, int32_t c_out, int64_t num_in, int64_t num_out,
                         int64_t pair_capacity);
+
+int wcn_conv_graph_ahead(int32_t dtype, int32_t num_offsets, int32_t c_in, int32_t c_out, int64_t num_in, int64_t num_out,
+                         int64_t pair_capacity);
+
+int wcn_sparse_conv_fwd_graph_ahead(const void* features, int64_t num_in, int32_t c_in, int32_t dtype, const void* weight,
+                                    int32_t weight_dtype, int32_t num_offsets, int32_t c_out, const void* bias_or_null,
+                                    int32_t bias_dtype, const int32_t* in_maps, const int32_t* out_maps, int64_t pair_capacity,
+                                    int64_t pairs_expected, const int64_t* map_result, int32_t identity_offset,
+                                    const int32_t* group_start, void* out, int64_t num_out, void* workspace,
+                                    size_t workspace_bytes, void* stream);
 
 int wcn_sparse_conv_fwd_ahead(const void* features, int64_t num_in, int32_t c_in, int32_t dtype, const void* half,
                               int32_t num_offsets, int32_t c_out, const void* bias_or_null, const int32_t* in_maps,

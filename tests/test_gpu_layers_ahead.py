@@ -147,6 +147,60 @@ def test_half_of_the_weight(dtype, num_offsets, c_in, c_out, rows, capacity, hal
     assert lib().wcn_conv_ahead_half(dtype, num_offsets, c_in, c_out, rows, rows, capacity) == half
 
 
+@pytest.mark.parametrize("n,dtype,c_in,c_out,kernel,stride,ahead", [
+    (900, torch.float16, 32, 64, 3, 1, True), (24_000, torch.float16, 32, 32, 3, 1, True), (12_000, torch.float16, 32, 64, 2, 2, True),
+    (8000, torch.bfloat16, 64, 64, 3, 1, True), (5000, torch.float32, 16, 16, 3, 1, True), (9000, torch.float32, 32, 32, 3, 2, True),
+    (4000, torch.bfloat16, 256, 256, 3, 1, False), (40_000, torch.float16, 64, 64, 3, 1, False), (500, torch.float16, 3, 16, 3, 1, False)])
+@pytest.mark.parametrize("bias", [None, "own", "fp32", "per_row", "requires_grad"])
+@pytest.mark.parametrize("master", [False, True])
+def test_layers_with_gradients(monkeypatch, n, dtype, c_in, c_out, kernel, stride, ahead, bias, master):
+    """Product and gradients ahead of the map are those over the kept map, bit for bit."""
+    from warpconvnet_amd.geometry.types.voxels import Voxels
+    from warpconvnet_amd.nn.functional.sparse_conv import spatially_sparse_conv
+    made = _spied(monkeypatch)
+    vox = _voxels(n, c_in, dtype, seed=n)
+    w = kaiming_weight(kernel ** 3, c_in, c_out, seed=2, dtype=torch.float32 if master else dtype).to(DEV)
+    b = normal_features(1, c_out, seed=3, dtype=torch.float32)[0].to(DEV)
+    if bias in ("own", "requires_grad"):
+        b = b.to(dtype)
+
+    def step(vox, times):
+        x = vox.feature_tensor.detach().requires_grad_(True)
+        weight, extra = w.clone().requires_grad_(True), None if bias is None else b.clone().requires_grad_(bias == "requires_grad")
+        if bias == "per_row":
+            extra = b[None]
+        vox = vox.replace(batched_features=x)
+        for _ in range(times):  # (the first call of several makes the map)
+            out = spatially_sparse_conv(vox, weight, kernel, stride=stride, bias=extra).feature_tensor
+        gy = normal_features(len(out), c_out, seed=7, dtype=dtype).to(DEV)
+        wanted = [x, weight] + ([extra] if bias == "requires_grad" else [])
+        return [out.detach()] + list(torch.autograd.grad(out, wanted, gy))
+
+    first = step(vox, 1)
+    assert len(made) == 1 and (made[0].out is not None) == (ahead and bias != "per_row")
+    over_kept = step(_voxels(n, c_in, dtype, seed=n), 2)
+    assert made[-1].out is None
+    assert all(torch.equal(p, q) for p, q in zip(first, over_kept))
+
+
+def test_lists_too_short_for_a_layer_with_gradients(monkeypatch):
+    from warpconvnet_amd.geometry.coords.search import torch_discrete
+    from warpconvnet_amd.geometry.types.voxels import Voxels
+    from warpconvnet_amd.nn.functional.sparse_conv import spatially_sparse_conv
+    made = _spied(monkeypatch)
+    cube = np.stack(np.meshgrid(*[np.arange(20)] * 3, indexing="ij"), axis=-1).reshape(-1, 3).astype(np.int32)
+    n, got = len(cube), []
+    x = normal_features(n, 32, seed=1, dtype=torch.float16).to(DEV)
+    w = kaiming_weight(27, 32, 64, seed=2, dtype=torch.float32).to(DEV).requires_grad_(True)
+    b = torch.linspace(-1, 1, 64, device=DEV)
+    monkeypatch.setattr(torch_discrete, "_PAIRS_PER_ROW", {})
+    for assumed in ("too few", "enough"):
+        vox = Voxels(torch.as_tensor(cube, device=DEV), x, offsets=torch.tensor([0, n]))
+        got.append(spatially_sparse_conv(vox, w, 3, bias=b).feature_tensor)
+        assert (made[-1].out is None) == (assumed == "too few")
+    assert torch.equal(*got)
+
+
 @pytest.mark.parametrize("case", ["columns", "fp32_bias", "one_bias", "half_weight", "residual_type", "three_channels", "converted"])
 def test_calls_that_wait_for_the_map(monkeypatch, case):
     from warpconvnet_amd.nn.functional.sparse_conv import spatially_sparse_conv

@@ -61,6 +61,9 @@ SIGNATURES = {
     "wcn_sparse_conv_fwd_ahead": (ctypes.c_int, [_vp, _i64, _i32, _i32, _vp, _i32, _i32, _vp, _vp, _vp, _i64, _i64, _vp, _i32,
                                                  _vp, _vp, _i32, _vp, _i64, _vp]),
     "wcn_conv_ahead_half": (ctypes.c_int, [_i32, _i32, _i32, _i32, _i64, _i64, _i64]),
+    "wcn_conv_graph_ahead": (ctypes.c_int, [_i32, _i32, _i32, _i32, _i64, _i64, _i64]),
+    "wcn_sparse_conv_fwd_graph_ahead": (ctypes.c_int, [_vp, _i64, _i32, _i32, _vp, _i32, _i32, _i32, _vp, _i32, _vp, _vp, _i64, _i64,
+                                                       _vp, _i32, _vp, _vp, _i64, _vp, _sz, _vp]),
     "wcn_sparse_conv_fwd_prepared": (ctypes.c_int, [_vp, _i64, _i32, _i32, _vp, _sz, _i32, _i32, _vp, _vp,
                                                     _vp, _i64p, _vp, _i32, _vp, _vp, _i32, _vp, _i64,
                                                     _vp, _sz, _vp]),

@@ -1446,6 +1446,43 @@ size_t wcn_conv_prepared_workspace_bytes(int64_t num_out, int32_t num_offsets, i
   return wcn_align256(sizeof(float) * (size_t)(cip / ck_of(dtype)) * (size_t)num_out * cop);
 }
 
+// The kernels whose choice and launch follow from rows and channels alone: those for small maps and for narrow layers, and the
+// pair-packed one.  Where a tile plan could be taken the pairs decide (nearly all that the kernel for wide rows takes is among that),
+// and slices of channels over workgroups would need a workspace.  What a layer gains is the host's time between the map's
+// last kernel and its own launch, whatever its size.  us of a call that makes its map, launched behind the wait / ahead of it:
+//     3x3x3  32 -> 64 fp16,   1,800 voxels     67 / 59     (small maps)
+//     3x3x3  32 -> 32 fp32, 100,000 voxels    108 / 100    (pair-packed)
+//     3x3x3, stride 2, 16 -> 13 fp32, 456,000 178 / 174    (narrow)
+//     a training step over 24,000 voxels      610 / 565    (three layers, `graph`)
+// graph: never the kernel for small maps, whose order of sums depends on the size of the map (see conv_run).
+static int ahead_half(int32_t dtype, int32_t num_offsets, int32_t c_in, int32_t c_out, int64_t num_in, int64_t num_out,
+                      int64_t pair_capacity, bool graph) {
+  if (dtype < 0 || dtype > 2 || num_offsets < 1 || num_offsets > WCN_MAX_OFFSETS || c_in < 1 || c_out < 1 || num_in < 1 ||
+      num_out < 1 || pair_capacity < 1 || kernel_choice() != 0 || (size_t)c_in * elem_size(dtype) % 16 != 0)
+    return -1;
+  if (wcn_conv_tiles_takes(dtype, num_offsets, c_in, c_out) && wcn_conv_tiles_rows(num_offsets, c_in, c_out, num_out)) return -1;
+  static const int32_t some = 0;  // (the rules look at whether there are group starts, not at them)
+  ConvArgs a = {};
+  a.K = num_offsets;
+  a.c_in = c_in;
+  a.c_out = c_out;
+  a.c_in_pad = round_up(c_in, ck_of(dtype));
+  a.c_out_pad = round_up(c_out, TN);
+  a.num_in = num_in;
+  a.num_out = num_out;
+  a.num_pairs = pair_capacity;
+  a.identity = -1;
+  a.G = (num_out + 63) / 64;
+  a.group_start = &some;
+  a.vec_in = a.vec_out = 1;
+  // in the order of conv_run and launch_conv
+  if (!graph && wcn_conv_split_takes(a, dtype)) return 1;
+  if (conv_wants_split(num_out, a.c_in_pad, a.c_out_pad, ck_of(dtype)) && !(dtype == WCN_DTYPE_F32 && wcn_conv_pack_takes(a, dtype)))
+    return -1;
+  if (wcn_conv_dense_takes(a, dtype) || pair_capacity >= (1ll << 30)) return -1;
+  return wcn_conv_group_takes(a, dtype) || wcn_conv_pack_takes(a, dtype) ? 0 : -1;
+}
+
 // Shared body of the forward product and the input gradient.  weight_as_stored / flip_offsets
 // choose how the caller's weight becomes the kernels' tiles (see conv_prep_weight).  With
 // `no_copy_commands` the call enqueues kernels only (the offsets must then fit the kernel
@@ -1460,7 +1497,7 @@ static int conv_run(const void* features, int64_t num_in, int32_t c_in, int32_t 
                     const void* residual_or_null = nullptr, int relu = 0,
                     const int64_t* device_offsets_of_prepared = nullptr, int bias_dtype = -1,
                     int bias_after_rounding = 0, const void* prepared_operands = nullptr, int64_t list_capacity = 0,
-                    int64_t pairs_expected = 0) {
+                    int64_t pairs_expected = 0, const int64_t* map_result = nullptr) {
   // With device_offsets_of_prepared, `weight` and `prepared_operands` are the two halves that wcn_conv_prepare_weight makes
   // (the one that is not read may be null) and the call enqueues nothing but the contraction.
   const bool prepared = device_offsets_of_prepared != nullptr;
@@ -1498,8 +1535,9 @@ static int conv_run(const void* features, int64_t num_in, int32_t c_in, int32_t 
   }
   // Up to 127 offsets reach the device in the arguments of the weight preparation, which is the
   // first launch of the call: no copy command.
-  const bool offsets_by_value = num_offsets + 1 <= OFFSETS_BY_VALUE;
-  if (!offsets_by_value && !prepared) {
+  // (Ahead of its map a call has them in device memory.)
+  const bool offsets_by_value = num_offsets + 1 <= OFFSETS_BY_VALUE && !map_result;
+  if (!offsets_by_value && !prepared && !map_result) {
     if (no_copy_commands) return WCN_ERR_INVALID_ARGUMENT;
     if (hipMemcpyAsync(w.offsets, host_offsets, sizeof(int64_t) * (size_t)(num_offsets + 1),
                        hipMemcpyHostToDevice, s) != hipSuccess)
@@ -1507,7 +1545,7 @@ static int conv_run(const void* features, int64_t num_in, int32_t c_in, int32_t 
   }
 
   ConvArgs a;
-  a.offsets = w.offsets;
+  a.offsets = map_result ? map_result : w.offsets;
   a.X = features;
   a.Wt = w.Wt;
   a.zeros = w.zeros;
@@ -1550,8 +1588,8 @@ static int conv_run(const void* features, int64_t num_in, int32_t c_in, int32_t 
   // size of map gives.  In training it would save 4 % of a stage on 10,000 voxels.
   const bool small = !bias_after_rounding && kernel_choice() == 0 && wcn_conv_split_takes(a, dtype);
   if (prepared && !(small ? prepared_operands : weight)) return WCN_ERR_INVALID_ARGUMENT;
-  if (list_capacity > 0 && (!a.vec_in || wcn_conv_ahead_half(dtype, num_offsets, c_in, c_out, num_in, num_out, list_capacity) !=
-                                             (small ? 1 : 0)))
+  if (list_capacity > 0 && (!a.vec_in || ahead_half(dtype, num_offsets, c_in, c_out, num_in, num_out, list_capacity,
+                                                    bias_after_rounding != 0) != (small ? 1 : 0)))
     return WCN_ERR_INVALID_ARGUMENT;
   a.Wf = nullptr;
   if (small && !prepared) {
@@ -1830,39 +1868,14 @@ int wcn_sparse_conv_fwd_prepared_halves(const void* features, int64_t num_in, in
                   stream, residual_or_null, relu, device_offsets, -1, 0, half1_or_null);
 }
 
-// The kernels whose choice and launch follow from rows and channels alone: those for small maps and for narrow layers, and the
-// pair-packed one.  Where a tile plan could be taken the pairs decide (nearly all that the kernel for wide rows takes is among that),
-// and slices of channels over workgroups would need a workspace.  What a layer gains is the host's time between the map's
-// last kernel and its own launch, whatever its size.  us of a call that makes its map, launched behind the wait / ahead of it:
-//     3x3x3  32 -> 64 fp16,   1,800 voxels     67 / 59     (small maps)
-//     3x3x3  32 -> 32 fp32, 100,000 voxels    108 / 100    (pair-packed)
-//     3x3x3, stride 2, 16 -> 13 fp32, 456,000 178 / 174    (narrow)
 int wcn_conv_ahead_half(int32_t dtype, int32_t num_offsets, int32_t c_in, int32_t c_out, int64_t num_in, int64_t num_out,
                         int64_t pair_capacity) {
-  if (dtype < 0 || dtype > 2 || num_offsets < 1 || num_offsets > WCN_MAX_OFFSETS || c_in < 1 || c_out < 1 || num_in < 1 ||
-      num_out < 1 || pair_capacity < 1 || kernel_choice() != 0 || (size_t)c_in * elem_size(dtype) % 16 != 0)
-    return -1;
-  if (wcn_conv_tiles_takes(dtype, num_offsets, c_in, c_out) && wcn_conv_tiles_rows(num_offsets, c_in, c_out, num_out)) return -1;
-  static const int32_t some = 0;  // (the rules look at whether there are group starts, not at them)
-  ConvArgs a = {};
-  a.K = num_offsets;
-  a.c_in = c_in;
-  a.c_out = c_out;
-  a.c_in_pad = round_up(c_in, ck_of(dtype));
-  a.c_out_pad = round_up(c_out, TN);
-  a.num_in = num_in;
-  a.num_out = num_out;
-  a.num_pairs = pair_capacity;
-  a.identity = -1;
-  a.G = (num_out + 63) / 64;
-  a.group_start = &some;
-  a.vec_in = a.vec_out = 1;
-  // in the order of conv_run and launch_conv
-  if (wcn_conv_split_takes(a, dtype)) return 1;
-  if (conv_wants_split(num_out, a.c_in_pad, a.c_out_pad, ck_of(dtype)) && !(dtype == WCN_DTYPE_F32 && wcn_conv_pack_takes(a, dtype)))
-    return -1;
-  if (wcn_conv_dense_takes(a, dtype) || pair_capacity >= (1ll << 30)) return -1;
-  return wcn_conv_group_takes(a, dtype) || wcn_conv_pack_takes(a, dtype) ? 0 : -1;
+  return ahead_half(dtype, num_offsets, c_in, c_out, num_in, num_out, pair_capacity, false);
+}
+
+int wcn_conv_graph_ahead(int32_t dtype, int32_t num_offsets, int32_t c_in, int32_t c_out, int64_t num_in, int64_t num_out,
+                         int64_t pair_capacity) {
+  return ahead_half(dtype, num_offsets, c_in, c_out, num_in, num_out, pair_capacity, true) == 0 ? 1 : 0;
 }
 
 int wcn_sparse_conv_fwd_ahead(const void* features, int64_t num_in, int32_t c_in, int32_t dtype, const void* half,
@@ -1879,6 +1892,22 @@ int wcn_sparse_conv_fwd_ahead(const void* features, int64_t num_in, int32_t c_in
                   out_maps, unknown, identity_offset, 1, group_start, out, num_out, nullptr, 0, 0, 0, true, stream, residual_or_null,
                   relu, map_result, -1, 0, which == 1 ? half : nullptr, pair_capacity,
                   std::min(std::max<int64_t>(pairs_expected, 1), pair_capacity));
+}
+
+int wcn_sparse_conv_fwd_graph_ahead(const void* features, int64_t num_in, int32_t c_in, int32_t dtype, const void* weight,
+                                    int32_t weight_dtype, int32_t num_offsets, int32_t c_out, const void* bias_or_null,
+                                    int32_t bias_dtype, const int32_t* in_maps, const int32_t* out_maps, int64_t pair_capacity,
+                                    int64_t pairs_expected, const int64_t* map_result, int32_t identity_offset,
+                                    const int32_t* group_start, void* out, int64_t num_out, void* workspace,
+                                    size_t workspace_bytes, void* stream) {
+  if (bias_or_null && bias_dtype != dtype && bias_dtype != WCN_DTYPE_F32) return WCN_ERR_INVALID_ARGUMENT;
+  if (!map_result || !group_start || !in_maps || !out_maps ||
+      !wcn_conv_graph_ahead(dtype, num_offsets, c_in, c_out, num_in, num_out, pair_capacity))
+    return WCN_ERR_INVALID_ARGUMENT;
+  static const int64_t unknown[WCN_MAX_OFFSETS + 1] = {};  // the pairs
+  return conv_run(features, num_in, c_in, dtype, weight, weight_dtype, num_offsets, c_out, bias_or_null, in_maps, out_maps, unknown,
+                  identity_offset, 1, group_start, out, num_out, workspace, workspace_bytes, 0, 0, true, stream, nullptr, 0, nullptr,
+                  bias_dtype, 1, nullptr, pair_capacity, std::min(std::max<int64_t>(pairs_expected, 1), pair_capacity), map_result);
 }
 
 int wcn_sparse_conv_fwd_prepared(const void* features, int64_t num_in, int32_t c_in, int32_t dtype,

@@ -215,14 +215,14 @@ py::tuple stride_cells(const py::object& table, const Int3& stride, bool want_bo
   }
 }
 
-/* A layer without gradients whose map is about to be made, for kernel_map to run between the map's launches and the wait for its
+/* A layer whose map is about to be made (`graph`: one whose gradients will be asked for, as conv_forward's), for kernel_map to run between the map's launches and the wait for its
  * offsets.  `out` stays undefined where the layer is none that can: it is then run behind the map, as any other. */
 struct LayerAhead {
   Tensor features;
   py::object weight;
   std::optional<Tensor> bias, residual;
   std::optional<at::ScalarType> compute_dtype;
-  bool relu = false, keep_tiles = false;
+  bool relu = false, keep_tiles = false, graph = false;
   int64_t identity = -1;
   Tensor out;
   void launch(const Tensor& in_maps, const Tensor& out_maps, int64_t expected, const void* map_result, const int32_t* groups,
@@ -424,6 +424,7 @@ Tensor prepared_tiles(const py::object& weight_obj, const Tensor& weight, const 
 
 bool kernel_bias(const Tensor& bias, const Tensor& features, int64_t c_out);
 bool aligned16(const void* p);
+bool plain_rows(const Tensor& t);
 
 void LayerAhead::launch(const Tensor& in_maps, const Tensor& out_maps, int64_t expected, const void* map_result,
                         const int32_t* groups, int32_t K, int64_t num_out) {
@@ -435,21 +436,38 @@ void LayerAhead::launch(const Tensor& in_maps, const Tensor& out_maps, int64_t e
   if (code < 0 || !features.is_cuda() || features.dim() != 2 || w.dim() != 3 || w.size(0) != K || w.size(1) != features.size(1) ||
       w.device() != features.device() || features.device() != in_maps.device() || !features.is_contiguous() || !w.is_contiguous() ||
       (w.scalar_type() != dtype && w.scalar_type() != at::kFloat) || (compute_dtype && *compute_dtype != dtype) || num_out == 0 ||
-      features.size(0) == 0 || features.size(0) * features.element_size() == 0 || w.size(2) > INT32_MAX || w.size(1) > INT32_MAX)
+      features.size(0) == 0 || features.size(0) * features.element_size() == 0 || w.size(2) > INT32_MAX || w.size(1) > INT32_MAX ||
+      (graph && (!plain_rows(features) || !plain_rows(w))))
     return;
   const int32_t c_in = static_cast<int32_t>(w.size(1)), c_out = static_cast<int32_t>(w.size(2));
   const void* const px = features.const_data_ptr();
   if (c_in * features.element_size() % 16 != 0 || !aligned16(px)) return;
-  const int half = wcn_conv_ahead_half(code, K, c_in, c_out, features.size(0), num_out, in_maps.numel());
+  const int half = graph ? wcn_conv_graph_ahead(code, K, c_in, c_out, features.size(0), num_out, in_maps.numel()) - 1
+                         : wcn_conv_ahead_half(code, K, c_in, c_out, features.size(0), num_out, in_maps.numel());
   if (half < 0) return;
   const bool has_bias = bias && bias->defined(), has_residual = residual && residual->defined();
-  if (has_bias && (!kernel_bias(*bias, features, c_out) || bias->scalar_type() != dtype || !bias->is_contiguous() ||
-                   !aligned16(bias->const_data_ptr())))
+  if (has_bias && (!kernel_bias(*bias, features, c_out) || !bias->is_contiguous() ||
+                   (bias->scalar_type() != dtype && !(graph && bias->scalar_type() == at::kFloat)) ||
+                   !(graph ? plain_rows(*bias) : aligned16(bias->const_data_ptr()))))
     return;
   if (has_residual && (residual->dim() != 2 || residual->size(0) != num_out || residual->size(1) != c_out || !residual->is_cuda() ||
                        residual->device() != features.device() || residual->scalar_type() != dtype || !residual->is_contiguous()))
     return;
   void* stream = stream_of(features);
+  if (graph) {
+    Tensor rows = at::empty({num_out, c_out}, features.options());
+    const Tensor ws = bytes_on(wcn_conv_workspace_bytes(num_out, K, c_in, c_out, code, 0, 1), features);
+    check(wcn_sparse_conv_fwd_graph_ahead(px, features.size(0), c_in, code, w.const_data_ptr(), dtype_code(w.scalar_type()), K, c_out,
+                                          has_bias ? bias->const_data_ptr() : nullptr,
+                                          has_bias ? dtype_code(bias->scalar_type()) : code, in_maps.const_data_ptr<int32_t>(),
+                                          out_maps.const_data_ptr<int32_t>(), in_maps.numel(), expected,
+                                          static_cast<const int64_t*>(map_result), static_cast<int32_t>(identity), groups,
+                                          rows.mutable_data_ptr(), num_out, ws.mutable_data_ptr(), static_cast<size_t>(ws.numel()),
+                                          stream),
+          "wcn_sparse_conv_fwd_graph_ahead");
+    out = rows;
+    return;
+  }
   Tensor tiles;
   if (keep_tiles) {
     tiles = prepared_tiles(weight, w, [&]() { return w; }, dtype, c_in, half);
@@ -966,17 +984,18 @@ struct ConvBackward : public torch::autograd::Node {
 
 /* The contraction with its gradients as one graph node.  The bias is added to the rounded product, as
  * a separate addition behind the function would: fusing it into the sums moves values across the zero of
- * a following ReLU, whose gradient then differs. */
+ * a following ReLU, whose gradient then differs.  `ahead`: what a LayerAhead of the same arguments has left. */
 Tensor conv_autograd(const Tensor& features, const py::object& weight_obj, const std::optional<Tensor>& bias,
                      const py::object& km, int64_t num_out, const std::optional<at::ScalarType>& compute_dtype,
-                     const py::object& pairs_sorted) {
+                     const py::object& pairs_sorted, const std::optional<Tensor>& ahead) {
   const Tensor weight = weight_obj.cast<Tensor>();
   refuse_tangents({&features, &weight}, "the sparse convolution");
   // a product in another type than the features' comes back in theirs before the bias is added
   const bool given = bias && bias->defined(), has_bias = given && kernel_bias(*bias, features, weight.size(-1));
   const bool inside = !compute_dtype || *compute_dtype == features.scalar_type();
-  Tensor out = conv_forward(features, weight_obj, km, num_out, inside && has_bias ? bias : std::nullopt, compute_dtype, std::nullopt,
-                            false, false, pairs_sorted, true);
+  Tensor out = ahead ? *ahead
+                     : conv_forward(features, weight_obj, km, num_out, inside && has_bias ? bias : std::nullopt, compute_dtype,
+                                    std::nullopt, false, false, pairs_sorted, true);
   if (has_bias && !inside) {
     at::AutoDispatchBelowADInplaceOrView guard;
     out.add_(bias->scalar_type() == out.scalar_type() ? *bias : bias->to(out.scalar_type()));
@@ -1319,9 +1338,10 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   py::class_<LayerAhead>(m, "LayerAhead")
       .def(py::init([](const Tensor& features, const py::object& weight, const std::optional<Tensor>& bias,
                        const std::optional<at::ScalarType>& compute_dtype, const std::optional<Tensor>& residual, bool relu,
-                       bool keep_tiles) {
-        return LayerAhead{features, weight, bias, residual, compute_dtype, relu, keep_tiles, -1, Tensor()};
-      }))
+                       bool keep_tiles, bool graph) {
+        return LayerAhead{features, weight, bias, residual, compute_dtype, relu, keep_tiles, graph, -1, Tensor()};
+      }), py::arg("features"), py::arg("weight"), py::arg("bias"), py::arg("compute_dtype"), py::arg("residual"), py::arg("relu"),
+           py::arg("keep_tiles"), py::arg("graph") = false)
       .def_property("identity", [](const LayerAhead& a) { return a.identity; },
                     [](LayerAhead& a, std::optional<int64_t> k) { a.identity = k.value_or(-1); })
       .def_property_readonly("out", [](const LayerAhead& a) { return a.out.defined() ? py::cast(a.out) : py::none(); });
@@ -1337,7 +1357,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     return out.defined() ? py::cast(out) : py::none();
   });
   m.def("conv_backward", &conv_backward);
-  m.def("conv_autograd", &conv_autograd);
+  m.def("conv_autograd", &conv_autograd, py::arg("features"), py::arg("weight"), py::arg("bias"), py::arg("km"), py::arg("num_out"),
+        py::arg("compute_dtype"), py::arg("pairs_sorted"), py::arg("ahead") = py::none());
   m.def("depthwise_forward", &depthwise_forward);
   m.def("depthwise_backward", &depthwise_backward);
   m.def("depthwise_autograd", &depthwise_autograd);

@@ -452,9 +452,10 @@ def spatially_sparse_conv(
     needs_grad = torch.is_grad_enabled() and (features.requires_grad or weight.requires_grad)
     needs_residual_grad = residual is not None and torch.is_grad_enabled() and residual.requires_grad
     ahead = None
-    if not (needs_grad or needs_residual_grad or transposed) and features.is_cuda:
-        # a layer over a small map that has to be made first does not wait for the host to have read the map's offsets
-        ahead = native().LayerAhead(features, weight, bias, effective_compute_dtype, residual, relu, keep_prepared_weight)
+    if not transposed and features.is_cuda and (needs_grad or not needs_residual_grad):
+        # a layer whose map has to be made first does not wait for the host to have read the map's offsets
+        ahead = native().LayerAhead(features, weight, bias, effective_compute_dtype, None, False, False, True) if needs_grad \
+            else native().LayerAhead(features, weight, bias, effective_compute_dtype, residual, relu, keep_prepared_weight)
     out_coords, out_offsets, kernel_map = generate_output_coords_and_kernel_map(
         input_sparse_tensor=input_sparse_tensor, kernel_size=_kernel_size,
         kernel_dilation=_kernel_dilation, stride=_stride, generative=generative,
@@ -470,7 +471,8 @@ def spatially_sparse_conv(
                 out_features = out_features + bias.to(out_features.dtype)
         else:
             out_features = native().conv_autograd(features, weight, bias, kernel_map, num_out_coords,
-                                                  effective_compute_dtype, _pairs_sorted)
+                                                  effective_compute_dtype, _pairs_sorted,
+                                                  ahead.out if ahead is not None else None)
         out_features = after(out_features)
     elif num_out_coords == 0 or features.shape[0] == 0:
         out_features = torch.zeros((num_out_coords, weight.shape[-1]), dtype=features.dtype,
