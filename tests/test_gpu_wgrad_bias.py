@@ -51,3 +51,28 @@ def test_weight_and_bias_gradient_in_one_call(c_out, rows, dtype, bias_dtype, sh
     # fp32 sums: each addition rounds by 2^-24 of a partial sum, which is at most the sum of the magnitudes; then the bias's type
     bound = gy.double().abs().sum(0) * 2.0 ** -20 + want.abs() * {torch.float32: 0, torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8}[bias_dtype]
     assert ((gb.double() - want).abs() <= bound + 1e-7).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("c_in,c_out,rows,pairs", [(8, 8, 0, 0), (8, 8, 5, 0), (32, 32, 3000, 1), (64, 264, 70_001, 5000), (136, 64, 33_000, 64),
+                                                   (96, 96, 300_000, 20_000)])
+def test_column_sums_beside_any_weight_gradient(c_in, c_out, rows, pairs, dtype):
+    """The sums ride on the weight gradient's launches, also where that has no pair, and no row, to work on."""
+    g = torch.Generator().manual_seed(rows)
+    x = torch.randn(700, c_in, generator=g).to(dtype).to(DEV)
+    gy = torch.randn(rows, c_out, generator=g).to(dtype).to(DEV)
+    im = torch.randint(0, 700, (max(pairs, 1),), generator=g, dtype=torch.int32).to(DEV)
+    om = torch.randint(0, max(rows, 1), (max(pairs, 1),), generator=g, dtype=torch.int32).to(DEV)
+    host = (ctypes.c_int64 * 3)(0, pairs // 3, pairs)
+    L, s = lib(), stream_ptr(DEV)
+    ws = workspace(L.wcn_conv_wgrad_workspace_bytes(2, c_in, c_out, pairs, 0), DEV)
+    bws = workspace(L.wcn_column_sums_workspace_bytes(c_out), DEV)
+    gw, gw2 = (torch.full((2, c_in, c_out), 9.0, device=DEV) for _ in range(2))
+    gb, gb2 = (torch.full((c_out,), 9.0, device=DEV) for _ in range(2))
+    args = (ptr(x), 700, c_in, ptr(gy) if rows else None, rows, c_out, CODE[dtype], ptr(im), ptr(om), host, None, 2, -1)
+    check(L.wcn_sparse_conv_wgrad_bias(*args, ptr(gw), 0, ptr(ws), ws.numel(), ptr(gb), 0, ptr(bws), bws.numel(), s), "wgrad_bias")
+    check(L.wcn_sparse_conv_wgrad_mapped(*args, ptr(gw2), 0, ptr(ws), ws.numel(), s), "wgrad")
+    check(L.wcn_column_sums(ptr(gy) if rows else None, rows, c_out, CODE[dtype], ptr(gb2), 0, ptr(bws), bws.numel(), s), "sums")
+    assert torch.equal(gw, gw2) and torch.equal(gb, gb2)
+    assert pairs > 0 or not gw.any()
+    assert ((gb.double() - gy.double().sum(0)).abs() <= gy.double().abs().sum(0) * 2.0 ** -20 + 1e-7).all()

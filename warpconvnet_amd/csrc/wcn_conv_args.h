@@ -86,7 +86,8 @@ struct WcnColumnSums {
   void* out;
   int32_t out_dtype;
 };
-int wcn_column_sums_first(const void* rows, int64_t num_rows, int dtype, WcnColumnSums* c, hipStream_t stream);  // sets parts
+void wcn_column_sums_parts(int64_t num_rows, int dtype, WcnColumnSums* c);  // sets parts
+int wcn_column_sums_first(const void* rows, int64_t num_rows, int dtype, const WcnColumnSums& c, hipStream_t stream);
 int wcn_column_sums_second(const WcnColumnSums& c, hipStream_t stream);
 
 #ifdef __HIPCC__
@@ -116,7 +117,7 @@ __device__ __forceinline__ void wcn_column_sums_finish(const WcnColumnSums& s, i
 #endif
 
 // The weight gradient of 16-bit rows of whole vectors (wcn_conv_wgrad.hip): whether it takes a problem, the bytes of its
-// partial sums (pairs with the identity's rows), and its launch.
+// partial sums (pairs with the identity's rows), and its launch (with the column sums of grad_out, both passes).
 bool wcn_wgrad_tiles_takes(int dtype, int c_in, int c_out, const void* features, const void* grad_out);
 size_t wcn_wgrad_tiles_partial_bytes(int num_offsets, int c_in, int c_out, int64_t pairs);
 int wcn_wgrad_tiles_launch(const void* features, int64_t num_in, int c_in, const void* grad_out, int64_t num_out, int c_out,

@@ -453,7 +453,9 @@ int wcn_sparse_conv_wgrad_bias(const void* features, int64_t num_in, int32_t c_i
   if (bias_workspace_bytes < wcn_column_sums_workspace_bytes(c_out)) return WCN_ERR_WORKSPACE;
   const bool joined = c_in >= 1 && wcn_wgrad_tiles_takes(dtype, c_in, c_out, features, grad_out);
   WcnColumnSums c = {(float*)bias_workspace, 0, c_out, grad_bias, bias_dtype};
-  int st = wcn_column_sums_first(grad_out, num_out, dtype, &c, (hipStream_t)stream);
+  wcn_column_sums_parts(num_out, dtype, &c);
+  // (joined: both passes ride on the launches of the weight gradient)
+  int st = joined ? WCN_OK : wcn_column_sums_first(grad_out, num_out, dtype, c, (hipStream_t)stream);
   if (st != WCN_OK) return st;
   st = wgrad_run(features, num_in, c_in, grad_out, num_out, c_out, dtype, in_maps, out_maps, host_offsets,
                  device_offsets_or_null, num_offsets, identity_offset, grad_weight, weight_dtype, workspace, workspace_bytes,

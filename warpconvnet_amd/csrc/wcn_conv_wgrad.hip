@@ -18,12 +18,16 @@
 // A stage of 3x3x3 96 -> 96 over 300 k rows and 128 -> 128 over 170 k with its 2x2x2 layers, bf16, all four weight gradients:
 // 667 -> 285 us (91, 107, 30 and 29, reductions 27); with the rows of dY shared in the XCDs' L2s (wgrad_first_chunk) 232 (74, 80, 25 and
 // 28), where every row of dY came from behind the L2 for every offset.
+// The column sums of dY (a bias's gradient) are workgroups of the same launch, behind the others, where the last of those leave CUs
+// idle: these four and their column sums 206 + 39 us one after the other, 234 together; of a stage on 24,000 voxels of 32 and 64
+// channels, where most of a launch is its start and end, 28 + 22 and 31.
 #include <algorithm>
 #include <mutex>
 
 #include "wcn_common.h"
 #include "wcn_conv_args.h"
 #include "wcn_mma.h"
+#include "wcn_rows.h"
 
 namespace {
 
@@ -44,6 +48,7 @@ struct WgradTileArgs {
   float* partial;          // (chunks, c_in_pad, c_out_pad)
   int64_t num_in, num_out, identity_rows;
   int32_t K, c_in, c_out, c_in_pad, c_out_pad, identity, pairs_per_chunk, chunks, tiles_in, tiles_out;  // chunks: most on an XCD
+  int32_t grid;  // workgroups of the tiles
 };
 
 __device__ __forceinline__ void to_lds(const char* g, uint32_t lds_off) {
@@ -100,12 +105,16 @@ struct Side {  // one operand: a tile of 32 N channels in rows of S
 };
 
 template <typename T, int NI, int NO>
-__global__ void __launch_bounds__(256, 2) conv_wgrad_tiles(WgradTileArgs a) {
+__global__ void __launch_bounds__(256, 2) conv_wgrad_tiles(WgradTileArgs a, wcn_rows::ColumnPart columns) {
   typedef typename Mma<T>::V V;
   typedef Side<NI> I;
   typedef Side<NO> O;
   constexpr int STAGE = I::BYTES + O::BYTES;
   extern __shared__ __attribute__((aligned(16))) char wgrad_smem[];
+  if ((int)blockIdx.x >= a.grid) {  // the column sums of dY: workgroups of their own behind the others
+    wcn_rows::column_part<T, true>(columns, (int)blockIdx.x - a.grid, reinterpret_cast<float*>(wgrad_smem));
+    return;
+  }
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)wgrad_smem;
   int32_t* const s_in = reinterpret_cast<int32_t*>(wgrad_smem + 2 * STAGE);
   int32_t* const s_out = s_in + SEGMENT;
@@ -347,8 +356,9 @@ WgradChunking wgrad_chunking(const int64_t* host_offsets, int K, int identity, i
 }
 
 template <typename T, int NI, int NO>
-int launch_wgrad_tiles(const WgradTileArgs& a, hipStream_t s) {
+int launch_wgrad_tiles(WgradTileArgs a, const wcn_rows::ColumnPart& columns, int parts, hipStream_t s) {
   constexpr int lds = 2 * (Side<NI>::BYTES + Side<NO>::BYTES) + 2 * SEGMENT * 4;
+  static_assert(lds >= 256 * 9 * 4, "room for the column sums");
   const void* fn = (const void*)conv_wgrad_tiles<T, NI, NO>;
   {  // more than 64 KiB of dynamic LDS has to be allowed once per device and kernel
     static std::mutex mu;
@@ -362,27 +372,28 @@ int launch_wgrad_tiles(const WgradTileArgs& a, hipStream_t s) {
     }
   }
   const int64_t grid = (int64_t)a.chunks * 8 * a.tiles_in * a.tiles_out;
-  if (grid > INT32_MAX) return WCN_ERR_INVALID_ARGUMENT;
-  if (grid > 0) hipLaunchKernelGGL((conv_wgrad_tiles<T, NI, NO>), dim3((unsigned)grid), dim3(256), lds, s, a);
+  if (grid + parts > INT32_MAX) return WCN_ERR_INVALID_ARGUMENT;
+  a.grid = (int32_t)grid;
+  if (grid + parts > 0) hipLaunchKernelGGL((conv_wgrad_tiles<T, NI, NO>), dim3((unsigned)(grid + parts)), dim3(256), lds, s, a, columns);
   return WCN_OK;
 }
 
 template <typename T, int NI>
-int launch_out(const WgradTileArgs& a, hipStream_t s) {
+int launch_out(const WgradTileArgs& a, const wcn_rows::ColumnPart& c, int parts, hipStream_t s) {
   switch (blocks_of(a.c_out)) {
-    case 1: return launch_wgrad_tiles<T, NI, 1>(a, s);
-    case 2: return launch_wgrad_tiles<T, NI, 2>(a, s);
-    case 3: return launch_wgrad_tiles<T, NI, 3>(a, s);
-    default: return launch_wgrad_tiles<T, NI, 4>(a, s);
+    case 1: return launch_wgrad_tiles<T, NI, 1>(a, c, parts, s);
+    case 2: return launch_wgrad_tiles<T, NI, 2>(a, c, parts, s);
+    case 3: return launch_wgrad_tiles<T, NI, 3>(a, c, parts, s);
+    default: return launch_wgrad_tiles<T, NI, 4>(a, c, parts, s);
   }
 }
 template <typename T>
-int launch_in(const WgradTileArgs& a, hipStream_t s) {
+int launch_in(const WgradTileArgs& a, const wcn_rows::ColumnPart& c, int parts, hipStream_t s) {
   switch (blocks_of(a.c_in)) {
-    case 1: return launch_out<T, 1>(a, s);
-    case 2: return launch_out<T, 2>(a, s);
-    case 3: return launch_out<T, 3>(a, s);
-    default: return launch_out<T, 4>(a, s);
+    case 1: return launch_out<T, 1>(a, c, parts, s);
+    case 2: return launch_out<T, 2>(a, c, parts, s);
+    case 3: return launch_out<T, 3>(a, c, parts, s);
+    default: return launch_out<T, 4>(a, c, parts, s);
   }
 }
 
@@ -434,10 +445,12 @@ int wcn_wgrad_tiles_launch(const void* features, int64_t num_in, int c_in, const
   if (plan.most < 0) return WCN_ERR_INVALID_ARGUMENT;
   a.chunks = (int)plan.most;
   a.pairs_per_chunk = (int)plan.per;
-  const int st = dtype == WCN_DTYPE_F16 ? launch_in<_Float16>(a, s) : launch_in<__bf16>(a, s);
+  a.grid = 0;
+  const WcnColumnSums sums = columns ? *columns : WcnColumnSums{};
+  const wcn_rows::ColumnPart part = wcn_rows::column_part_of(grad_out, num_out, dtype, sums);
+  const int st = dtype == WCN_DTYPE_F16 ? launch_in<_Float16>(a, part, sums.parts, s) : launch_in<__bf16>(a, part, sums.parts, s);
   if (st != WCN_OK) return st;
   const int planes = num_offsets * (a.c_in_pad * a.c_out_pad / 256);
-  const WcnColumnSums sums = columns ? *columns : WcnColumnSums{};
   const dim3 grid((unsigned)(planes + (sums.channels + 15) / 16)), block(256);
   if (weight_dtype == WCN_DTYPE_F32)
     hipLaunchKernelGGL(wgrad_tiles_reduce<float>, grid, block, 0, s, a, (float*)grad_weight, planes, sums);

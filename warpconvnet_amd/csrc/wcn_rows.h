@@ -85,6 +85,61 @@ inline RowTiling row_tiling(int channels, int dtype) {
   return t;
 }
 
+// The first pass of column sums (WcnColumnSums) as a kernel reads it.  A workgroup of 256 threads sums a stretch of `per` rows,
+// a thread per 16 bytes of channels, four rows in flight.  s_sum: 256 (Piece<T>::N + 1) floats.
+struct ColumnPart {
+  const void* rows;
+  float* partial;
+  int64_t n, per;
+  RowTiling tiling;
+  int32_t channels;
+};
+template <class Sums>
+inline ColumnPart column_part_of(const void* rows, int64_t n, int dtype, const Sums& c) {
+  return {rows, c.partial, n, c.parts > 0 ? (n + c.parts - 1) / c.parts : 0, row_tiling(c.channels > 0 ? c.channels : 1, dtype), c.channels};
+}
+template <typename T, bool VEC>
+__device__ __forceinline__ void column_part(const ColumnPart& c, int part, float* s_sum) {
+  constexpr int N = Piece<T>::N, U = 4;
+  const T* const X = (const T*)c.rows;
+  const RowTiling tiling = c.tiling;
+  const int sub = (int)threadIdx.x / tiling.width, at = (int)threadIdx.x % tiling.width;
+  const int64_t begin = part * c.per, end = begin + c.per < c.n ? begin + c.per : c.n;
+  for (int p0 = 0; p0 < tiling.pieces; p0 += tiling.width) {
+    const int c0 = (p0 + at) * N;
+    float acc[N];
+#pragma unroll
+    for (int j = 0; j < N; ++j) acc[j] = 0.f;
+    if (sub < tiling.rows && p0 + at < tiling.pieces) {
+      for (int64_t m = begin + sub; m < end; m += U * tiling.rows) {
+        Piece<T> x[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const int64_t r = m + u * tiling.rows;
+          x[u] = load_raw<T, VEC>(X, r < end ? r : end - 1, c.channels, c0);
+          if (r >= end) x[u] = Piece<T>{};
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+          for (int j = 0; j < N; ++j) acc[j] += to_float(x[u].v[j]);
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < N; ++j) s_sum[threadIdx.x * (N + 1) + j] = acc[j];
+    __syncthreads();
+    if (sub == 0 && p0 + at < tiling.pieces) {
+      for (int l = 1; l < tiling.rows; ++l)
+#pragma unroll
+        for (int j = 0; j < N; ++j) acc[j] += s_sum[(l * tiling.width + at) * (N + 1) + j];
+#pragma unroll
+      for (int j = 0; j < N; ++j)
+        if (c0 + j < c.channels) c.partial[(int64_t)part * c.channels + c0 + j] = acc[j];
+    }
+    __syncthreads();
+  }
+}
+
 // Entries of one row of a rows form, U at a time in ascending offset: f(k[U], r[U], live[U]).  Where there are
 // fewer than U, or an entry is no row of the `limit` there are, live is false and r names a row that can be
 // read all the same (limit >= 1): the U row numbers are loaded without a branch between them, and so are the U feature
