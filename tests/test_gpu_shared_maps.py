@@ -228,3 +228,40 @@ def test_a_coordinate_table_nobody_has_waited_for_is_its_stream_s_own():
     assert _table_of(c, HashMethod.CITY, c.device) is own
     other = _map(c.clone())
     assert torch.equal(km.in_maps, other.in_maps) and torch.equal(km.out_maps, other.out_maps)
+
+
+@pytest.mark.parametrize("kernel,stride", [(2, 2), (3, 1), (3, 2), (5, 1)])
+@pytest.mark.parametrize("scene", ["cube", "sheet", "cloud", "one"])
+def test_rows_form_of_a_builders_map_is_that_of_its_lists(kernel, stride, scene):
+    """Groups of few pairs, of 384 and more (a chunk of a thin map) and of 1,024 and more (a chunk of a dense one), rows that end
+    inside a group: a depthwise layer over the one-pass form against the form made from the lists alone, bit for bit."""
+    from warpconvnet_amd.nn.functional.sparse_conv import native
+    from warpconvnet_amd.geometry.coords.ops.stride import stride_coords
+    from warpconvnet_amd.geometry.coords.search.torch_discrete import generate_kernel_map
+    rng = np.random.default_rng(kernel + stride)
+    if scene == "cube":
+        cells = np.stack(np.meshgrid(*[np.arange(23)] * 3, indexing="ij"), -1).reshape(-1, 3)
+    elif scene == "sheet":
+        cells = np.stack([rng.permutation(200 * 200)[:20_011] // 200, rng.permutation(200 * 200)[:20_011] % 200, np.zeros(20_011, int)], 1)
+    elif scene == "cloud":
+        at = rng.permutation(60 ** 3)[:9001]
+        cells = np.stack([at // 3600, at // 60 % 60, at % 60], 1)
+    else:
+        cells = np.zeros((1, 3), int)
+    cells = np.unique(cells, axis=0)
+    rows = torch.as_tensor(np.concatenate([np.zeros((len(cells), 1), int), cells], 1).astype(np.int32), device=DEV)
+    out = stride_coords(rows, (stride,) * 3)[0] if stride > 1 else rows
+    km = generate_kernel_map(rows, out, (stride,) * 3, (kernel,) * 3)
+    K, n, m = kernel ** 3, len(rows), len(out)
+    x = torch.randn(n, 8, device=DEV, generator=torch.Generator(DEV).manual_seed(1))
+    w = torch.randn(K, 8, device=DEV, generator=torch.Generator(DEV).manual_seed(2))
+    got = native().depthwise_forward(x, w, km, m, torch.float32)
+    km._rows_forms, km._from_builder = None, False
+    want = native().depthwise_forward(x, w, km, m, torch.float32)
+    assert torch.equal(got, want)
+    ins, outs, offsets = km.in_maps.long(), km.out_maps.long(), km.offsets.tolist()
+    sums = torch.zeros(m, 8, dtype=torch.float64, device=DEV)
+    for k in range(K):
+        at = slice(offsets[k], offsets[k + 1])
+        sums.index_add_(0, outs[at], x[ins[at]].double() * w[k].double())
+    assert float((got - sums).abs().max()) <= K * 2.0 ** -22 * 16  # K fp32 steps on sums of a few units

@@ -200,11 +200,16 @@ __global__ void __launch_bounds__(256) pool_bwd_spread(const T* __restrict__ dY,
 // group starts: a wave makes the rows of a group by itself.  The group's first entry is the sum of
 // its starts over the offsets (lane = offset).  The runs of its offsets are laid end to end and dealt to the lanes without gaps: every
 // offset marks where its run begins, and the running maximum of the marks is a pair's offset.  A row's bits are set in LDS, a
-// pair's place follows from the bits below its own; the numbers of the first 384 pairs (of some 270 on surfaces) stay in registers between the two.
-// Groups that follow one another go to one XCD: their runs follow one another in the lists.
+// pair's place follows from the bits below its own.  The numbers of a chunk of pairs stay in registers between the two, and where that is
+// all of the group's they go through LDS to their places, in runs.  A group with more asks for everything twice, a chunk after the other, so
+// maps of more than five pairs a row are dealt with 1,024 at a time; others with 384 (some 270 on surfaces), in half the registers.  Groups
+// that follow one another go to one XCD: their runs follow one another in the lists.  Bound by its chain of two reads and, of full
+// groups, by what one wave has to go through.  us, 384 and entries stored one by one / as it is: 3x3x3 over 157,000 rows of 12 pairs 19.7 / 13.8,
+// 37,000 of 13 17.7 / 13.2, 163,000 of 9 16.2 / 12.3; of 5 and fewer pairs: 300,000 9.2 / 8.1, 500,000 11.4 / 10.7, 2x2x2 163,000 6.0 / 5.7
+// (1,024 at a time, 84 registers: 11.4 and 15.3 over 300,000 and 500,000).
 constexpr int GROUPED_WORDS = 4;  // up to 128 offsets
 
-template <bool ONE>  // at most 32 offsets
+template <bool ONE, int CHUNK>  // ONE: at most 32 offsets; CHUNK: pairs of a group that are held at a time
 __global__ void __launch_bounds__(256) rows_from_groups(const int32_t* __restrict__ gathered,
                                                         const int32_t* __restrict__ grouping,
                                                         const int64_t* __restrict__ offsets,
@@ -214,11 +219,12 @@ __global__ void __launch_bounds__(256) rows_from_groups(const int32_t* __restric
                                                         int32_t* __restrict__ row_ptr,
                                                         int32_t* __restrict__ row_in,
                                                         int32_t* __restrict__ clear, int clear_words) {
-  constexpr int WORDS = ONE ? 1 : GROUPED_WORDS, OFFSETS = 32 * WORDS, CHUNK = 384, ROUNDS = CHUNK / 64;
+  constexpr int WORDS = ONE ? 1 : GROUPED_WORDS, OFFSETS = 32 * WORDS, ROUNDS = CHUNK / 64;
   __shared__ uint32_t s_mask[4][64][WORDS + (ONE ? 0 : 1)];
   __shared__ int32_t s_first[4][64];
   __shared__ int32_t s_shift[4][OFFSETS];  // the place of an offset's first pair in the lists, less its place among the group's
   __shared__ int32_t s_begin[4][OFFSETS];  // the latter
+  __shared__ int32_t s_in[4][CHUNK];         // the group's entries in their places
   __shared__ uint32_t s_mark[4][CHUNK / 4];  // a byte for each of CHUNK of the group's pairs: offset + 1 where a run begins
   const int tid = threadIdx.x, lane = wcn_lane(), wave = tid >> 6;
   if (blockIdx.x == 0)  // counters of whatever follows on the stream
@@ -254,11 +260,13 @@ __global__ void __launch_bounds__(256) rows_from_groups(const int32_t* __restric
   }
   const int base = __shfl(wcn_wave_inclusive_sum(before), 63, 64);
   int carry = 0;  // the offset (+ 1) of the last pair before the chunk
-  int k[ROUNDS], in[ROUNDS];
-  int64_t row[ROUNDS];
+  uint32_t tag[ROUNDS];  // a pair's row in the group and, from bit 8 on, its offset; ~0: none
+  int in[ROUNDS];
   auto request = [&](int p0) {  // pairs p0 .. p0 + CHUNK - 1 of the group
     uint8_t* const mark = reinterpret_cast<uint8_t*>(s_mark[wave]);
-    for (int i = lane; i < CHUNK / 4; i += 64) s_mark[wave][i] = 0u;
+#pragma unroll
+    for (int i = 0; i < CHUNK / 4; i += 64)
+      if (p0 + 4 * i < total && i + lane < CHUNK / 4) s_mark[wave][i + lane] = 0u;
     written();
 #pragma unroll
     for (int h = 0; h < (ONE ? 1 : 2); ++h) {
@@ -267,8 +275,11 @@ __global__ void __launch_bounds__(256) rows_from_groups(const int32_t* __restric
       if (at >= 0 && at < CHUNK && s_begin[wave][o] >= 0) mark[at] = (uint8_t)(o + 1);
     }
     written();
+    int row[ROUNDS];
 #pragma unroll
     for (int u = 0; u < ROUNDS; ++u) {
+      tag[u] = ~0u;
+      if (p0 + u * 64 >= total) continue;
       int v = max((int)mark[u * 64 + lane], lane == 0 ? carry : 0);
       // running maximum over the lanes, as wcn_wave_inclusive_sum
       v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false));
@@ -279,19 +290,23 @@ __global__ void __launch_bounds__(256) rows_from_groups(const int32_t* __restric
       v = max(v, __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false));
       carry = __builtin_amdgcn_readlane(v, 63);
       const int p = p0 + u * 64 + lane;
-      k[u] = p < total ? v - 1 : -1;
+      if (p < total) tag[u] = (uint32_t)(v - 1);
       const int at = p < total ? p + s_shift[wave][v - 1] : 0;
       row[u] = pairs > 0 ? grouping[at] : 0;
       in[u] = pairs > 0 ? gathered[at] : 0;
     }
 #pragma unroll
-    for (int u = 0; u < ROUNDS; ++u) row[u] = k[u] >= 0 ? row[u] - row0 : -1;
+    for (int u = 0; u < ROUNDS; ++u) {
+      if (p0 + u * 64 >= total) continue;
+      const int64_t r = row[u] - row0;
+      tag[u] = tag[u] != ~0u && (uint64_t)r < 64u ? tag[u] << 8 | (uint32_t)r : ~0u;
+    }
   };
   for (int p0 = 0; p0 < total; p0 += CHUNK) {
     request(p0);
 #pragma unroll
     for (int u = 0; u < ROUNDS; ++u)
-      if ((uint64_t)row[u] < 64u) atomicOr(&s_mask[wave][row[u]][ONE ? 0 : k[u] >> 5], 1u << (k[u] & 31));
+      if (tag[u] != ~0u) atomicOr(&s_mask[wave][tag[u] & 63u][ONE ? 0 : tag[u] >> 13], 1u << (tag[u] >> 8 & 31u));
   }
   written();
   int mine = 0;
@@ -313,15 +328,22 @@ __global__ void __launch_bounds__(256) rows_from_groups(const int32_t* __restric
     if (again) request(p0);
 #pragma unroll
     for (int u = 0; u < ROUNDS; ++u) {
-      if ((uint64_t)row[u] >= 64u) continue;
-      const uint32_t* const mask = s_mask[wave][row[u]];
-      int rank = __popc(mask[ONE ? 0 : k[u] >> 5] & ((1u << (k[u] & 31)) - 1u));
+      if (tag[u] == ~0u) continue;
+      const int row = (int)(tag[u] & 63u), k = (int)(tag[u] >> 8);
+      const uint32_t* const mask = s_mask[wave][row];
+      int rank = __popc(mask[ONE ? 0 : k >> 5] & ((1u << (k & 31)) - 1u));
       if (!ONE)
-        for (int w = 0; w < (k[u] >> 5); ++w) rank += __popc(mask[w]);
-      const int64_t dst = (int64_t)s_first[wave][row[u]] + rank;
-      if (dst < pairs) row_in[dst] = in[u];
+        for (int w = 0; w < (k >> 5); ++w) rank += __popc(mask[w]);
+      const int at = s_first[wave][row] - base + rank;
+      if (!again) s_in[wave][at] = in[u];
+      else if ((int64_t)base + at < pairs) row_in[(int64_t)base + at] = in[u];
     }
   }
+  if (again) return;
+  written();
+  const int held = __shfl(incl, 63, 64);  // of at most CHUNK pairs
+  for (int i = lane; i < held; i += 64)
+    if ((int64_t)base + i < pairs) row_in[(int64_t)base + i] = s_in[wave][i];
 }
 
 // ---- reduction over CSR segments (the point -> voxel pooling) -----------------------------------
@@ -632,7 +654,9 @@ int wcn_rows_from_groups(const int32_t* gathered_rows, const int32_t* grouping_r
   if (num_rows == 0) return WCN_OK;
   WcnRowsView v;
   wcn_rows_layout(workspace, num_rows, num_offsets, num_pairs, &v);
-  hipLaunchKernelGGL((num_offsets <= 32 ? rows_from_groups<true> : rows_from_groups<false>), dim3((unsigned)((v.G + 3) / 4)), dim3(256), 0, s, gathered_rows,
+  const bool many = num_pairs > 5 * num_rows;
+  hipLaunchKernelGGL((num_offsets <= 32 ? (many ? rows_from_groups<true, 1024> : rows_from_groups<true, 384>)
+                                       : many ? rows_from_groups<false, 1024> : rows_from_groups<false, 384>), dim3((unsigned)((v.G + 3) / 4)), dim3(256), 0, s, gathered_rows,
                      grouping_rows, device_offsets, group_start, num_offsets, v.words, num_rows, v.G, num_pairs, v.row_mask,
                      v.row_ptr, v.row_in, clear, clear_words);
   WCN_LAUNCH_CHECK();
