@@ -61,8 +61,8 @@ def _pad_kernel_args(values: Sequence[int], fill: int):
 # a map builder's workspace up to this size stays with its map (see _kernel_map_from_table)
 _KEEP_WORKSPACE_BYTES = 256 << 20
 
-# pairs per output row of the last map built for (kernel size, stride, size class of the row count):
-# sizes the buffers the pairs are emitted into before their number is known
+# pairs per output row of the last map built for (kernel size, stride, size class of the row count), by quarters of an octave of rows
+# and by whole ones (negative): sizes the buffers the pairs are emitted into before their number is known
 _PAIRS_PER_ROW = {}
 
 
@@ -88,13 +88,14 @@ def _kernel_map_from_table(table: TorchHashTable, out_coords: Tensor, kernel_siz
         ahead.identity = identity_map_index
     M = out4.shape[0]
     ks, st = _pad_kernel_args(kernel_size, 1), _pad_kernel_args(stride, 1)
-    shape_key = (tuple(ks), tuple(st), M.bit_length())
+    # (levels of a network lie within an octave: 1 M rows of 5 pairs and 553 k of 9, each of which made the other emit its pairs twice)
+    size, octave = (tuple(ks), tuple(st), (M ** 4).bit_length()), (tuple(ks), tuple(st), -M.bit_length())
     in_maps, out_maps, offsets64, offsets, groups, address, device_offsets, flags, made = native().kernel_map(
         table, out4, ks, st, None if dilation is None else _pad_kernel_args(dilation, 1),
-        None if dilation is None else _pad_kernel_args(centres, 0), _PAIRS_PER_ROW.get(shape_key, 8.0),
+        None if dilation is None else _pad_kernel_args(centres, 0), _PAIRS_PER_ROW.get(size, _PAIRS_PER_ROW.get(octave, 8.0)),
         _KEEP_WORKSPACE_BYTES, ahead)
     if M > 0:
-        _PAIRS_PER_ROW[shape_key] = in_maps.shape[0] / M
+        _PAIRS_PER_ROW[size] = _PAIRS_PER_ROW[octave] = in_maps.shape[0] / M
     K = offsets.shape[0] - 1
     result = IntSearchResult._of(in_maps, out_maps, offsets, identity_map_index, offsets64)
     result._out_ascend = True  # pairs ascend in output row inside every offset
