@@ -21,8 +21,11 @@ def _voxels(n, c_in, dtype, seed=0):
 
 
 def _spied(monkeypatch):
-    """What the layers that ran ahead of their maps have left: one entry per LayerAhead made."""
+    """What the layers that ran ahead of their maps have left: one entry per LayerAhead made.  The lists are sized as if no map had
+    been made before."""
+    from warpconvnet_amd.geometry.coords.search import torch_discrete
     from warpconvnet_amd.nn.functional import sparse_conv as f
+    monkeypatch.setattr(torch_discrete, "_PAIRS_PER_ROW", {})
     made = []
     native = f.native()
 

@@ -73,10 +73,10 @@ def test_blocks_at_the_same_place_of_their_cells(n, step):
     assert (table.search(_dev(rows + np.array([0, 1, 0, 0], np.int32))).cpu().numpy() == -1).all()
 
 
-# (parts of 4096 keys x bins either side of what the scatter pass adds up by itself; 64, 8 and 4 lanes a bin)
+# (one workgroup of the sort and more, 256 of them and more keys in each)
 @pytest.mark.parametrize("n", [16_385, 131_073, 262_143, 262_145, 300_000])
 @pytest.mark.parametrize("repeats", [False, True])
-def test_tables_whose_scatter_pass_adds_up_the_histogram(n, repeats):
+def test_tables_of_several_parts(n, repeats):
     from warpconvnet_amd.geometry.coords.search.torch_hashmap import TorchHashTable
     rng = np.random.default_rng(n)
     cells = rng.choice(4 * 90 ** 3, n, replace=repeats)
@@ -84,3 +84,42 @@ def test_tables_whose_scatter_pass_adds_up_the_histogram(n, repeats):
     _, first, back = np.unique(cells, return_index=True, return_inverse=True)
     table = TorchHashTable.from_keys(_dev(rows), device=DEV)
     assert np.array_equal(table.search(_dev(rows)).cpu().numpy(), first[back])
+
+
+@pytest.mark.parametrize("n,slots", [(16_385, 1 << 16), (262_144, 1 << 20), (262_145, 1 << 20), (20_000, 1 << 24), (70_001, 1 << 22),
+                                     (1 << 20, 1 << 21), ((1 << 20) + 1, 1 << 22), (1_300_007, 1 << 24)])
+@pytest.mark.parametrize("items", [False, True], ids=["rows", "items"])
+def test_parts_that_stay_in_registers_and_parts_that_do_not(n, slots, items):
+    """Up to 4,096 keys a part and more of them (read twice), up to 4,096 bins and more (not through LDS), rows given and made of
+    three columns and offsets; some keys twice, all of one corner in one bin."""
+    import ctypes
+
+    from warpconvnet_amd._lib import check, lib, ptr, stream_ptr
+    rng = np.random.default_rng(n)
+    cells = np.sort(rng.integers(0, 3, n)) * 10 ** 7 + rng.integers(0, 128 ** 3, n)
+    cells[: min(n // 4, 5000)] = np.arange(min(n // 4, 5000)) % 4096  # (16 x 16 x 16 voxels: one bin)
+    cells = np.sort(cells)
+    at = cells % 10 ** 7
+    rows = np.stack([cells // 10 ** 7, at % 16 + at // 4096 % 8 * 16 - 31, at // 16 % 16 + at // 32768 % 8 * 16,
+                     at // 256 % 16 + at // 262144 * 16 - 60], axis=1).astype(np.int32)
+    order = np.argsort(rows[:, 0], kind="stable")
+    rows = rows[order]
+    for b in range(3):  # no order inside an item
+        mine = np.flatnonzero(rows[:, 0] == b)
+        rows[mine] = rows[rng.permutation(mine)]
+    key = rows.astype(np.int64) @ np.array([10 ** 9, 10 ** 6, 10 ** 3, 1])
+    _, first, back = np.unique(key, return_index=True, return_inverse=True)
+    L, s = lib(), stream_ptr(torch.device(DEV))
+    table = torch.empty(L.wcn_table_bytes(n, slots), dtype=torch.uint8, device=DEV)
+    if items:
+        bounds = (ctypes.c_int64 * 4)(0, *np.cumsum(np.bincount(rows[:, 0], minlength=3)).tolist())
+        made = torch.empty(n, 4, dtype=torch.int32, device=DEV)
+        columns = _dev(rows[:, 1:])
+        check(L.wcn_table_build_items(ptr(columns), n, bounds, 3, ptr(made), ptr(table), slots, s), "build")
+        assert torch.equal(made, _dev(rows))
+    else:
+        made = _dev(rows)
+        check(L.wcn_table_build(ptr(made), n, ptr(table), slots, s), "build")
+    found = torch.empty(n, dtype=torch.int32, device=DEV)
+    check(L.wcn_table_query(ptr(table), n, slots, ptr(made), n, ptr(found), s), "query")
+    assert np.array_equal(found.cpu().numpy(), first[back])

@@ -71,17 +71,16 @@ struct WcnTableView {  // host-computed addresses inside a table workspace
   // the bin.
   WcnBlock* block_list;   // n_keys places (a bin has at most as many blocks as keys)
   // build scratch
-  int32_t* bin_coords;    // (n_keys, 4) keys grouped by bin
+  int32_t* bin_coords;    // (n_keys, 4) the keys of every part, grouped by bin within the part
   int32_t* bin_row;       // n_keys
-  int32_t* hist;          // (bins, parts) keys of part w in bin b, then their exclusive prefix sums
-  int32_t* bin_total;     // bins: keys per bin
+  int32_t* part_start;    // (bins + 1, parts): keys of part w in the bins before b
   int32_t* bin_start;     // bins + 1
   int32_t* bin_stats;     // (bins, 2): distinct keys of each bin; its blocks, | WCN_BIN_LOST where some found no place
   int32_t* part_box;      // (parts, 8) bounding box of each part's keys
   int64_t n_keys;
   int64_t capacity;
   int32_t bins;           // power of two
-  int32_t parts;          // workgroups of the histogram and scatter passes
+  int32_t parts;          // workgroups of the sort
 };
 
 static inline size_t wcn_align256(size_t x) { return (x + 255) & ~(size_t)255; }
@@ -91,7 +90,7 @@ static inline size_t wcn_align256(size_t x) { return (x + 255) & ~(size_t)255; }
 // rebuild with more slots also re-deals the bins.
 #define WCN_BIN_SLOTS 2048      // slots of a bin's region: the distinct blocks it can hold
 #define WCN_BIN_LOST (1 << 30)
-#define WCN_PART_KEYS 4096      // keys per workgroup of the histogram and scatter passes
+#define WCN_PART_KEYS 1024      // keys of a workgroup of the sort (more beyond 256 of them)
 #define WCN_MAX_BINS 32768      // a counter per bin in LDS during the build: 128 KB
 static inline int32_t wcn_table_bins(int64_t capacity) {
   int64_t b = capacity / 2048;
@@ -131,10 +130,8 @@ static inline size_t wcn_table_layout(void* base, int64_t n_keys, int64_t capaci
   off += wcn_align256(sizeof(int32_t) * 4 * (size_t)n_keys);
   if (v) v->bin_row = (int32_t*)(p + off);
   off += wcn_align256(sizeof(int32_t) * (size_t)n_keys);
-  if (v) v->hist = (int32_t*)(p + off);
-  off += wcn_align256(sizeof(int32_t) * (size_t)bins * (size_t)parts);
-  if (v) v->bin_total = (int32_t*)(p + off);
-  off += wcn_align256(sizeof(int32_t) * (size_t)bins);
+  if (v) v->part_start = (int32_t*)(p + off);
+  off += wcn_align256(sizeof(int32_t) * (size_t)(bins + 1) * (size_t)parts);
   if (v) v->bin_start = (int32_t*)(p + off);
   off += wcn_align256(sizeof(int32_t) * (size_t)(bins + 1));
   if (v) v->bin_stats = (int32_t*)(p + off);

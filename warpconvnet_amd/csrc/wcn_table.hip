@@ -1,23 +1,22 @@
 // Coordinate table of 4x4x4-voxel blocks: build and point queries (gfx950).
 //
-// Build pipeline (all on the caller's stream, no host round trip).  The keys are first grouped into
-// bins of one to two thousand (a bin is a hash of the key's 16x16x16-voxel cell, so every 4x4x4
-// block lies in exactly one bin); one workgroup per bin then sees all voxels of its blocks and
-// builds their masks with LDS atomics:
-//   table_hist     per part of the keys (a workgroup): keys per bin (LDS counters) and the part's
-//                  bounding box
-//   table_colscan  per bin (a wave): prefix sums over the parts (up to some 260,000 keys table_scatter adds them up itself)
-//   table_scatter  per part: every key and its row to its place in its bin; the first workgroup merges the boxes and
-//                  writes the header
-//   table_bins     per bin: block masks and entry counts in an LDS table, their prefix sums; that table is the bin's
-//                  region of the table in memory; then per key: its place in block order and perm[base + rank] = row
+// Build pipeline (all on the caller's stream, no host round trip).  The keys are grouped by bins of one to two thousand (a bin is
+// a hash of the key's 16x16x16-voxel cell, so every 4x4x4 block lies in exactly one bin); one workgroup per bin then sees all
+// voxels of its blocks and builds their masks with LDS atomics:
+//   table_sort     per part of the keys (a workgroup): the part's keys in the order of their bins, where each bin begins among them, and
+//                  the part's bounding box
+//   table_bins     per bin: its stretches of all parts, the box and the keys of the bins before; block masks and entry counts in
+//                  an LDS table, their prefix sums; that table is the bin's region of the table in memory; then per key: its
+//                  place in block order and perm[base + rank] = row
 // Up to 16,384 keys one launch does all of it (table_small).
 //
-// HBM traffic per key: 16 B read twice (histogram, scatter), 20 B written and read (binned entry),
-// 20 B written (entry in block order) + 4 B (perm), plus 16 B per table slot.
-// What the regions gave over 1 M voxels of rooms (us, against slots of 32 bytes anywhere in the table, cleared by the first
-// launch and claimed with a 64-bit compare-and-swap per block): table_hist 13.6 -> 10.4, table_bins 29.4 -> 26, the probe passes
-// of a 3x3x3 map 86 -> 59 and of a 5x5x5 map 189 -> 140; 1,800 voxels: 14.4 in two launches -> 10.2 in one.
+// HBM traffic per key: 16 B read (12 where the keys are made here, and 16 written), 20 B written and read (grouped entry), 8 B written
+// (entry in block order) + 4 B (perm), plus 16 B per table slot.
+// What it took over 1 M voxels of rooms, us: with bins laid out one behind the other (a launch for the parts' counts per bin 10.5, one for
+// their sums 4.9, the scatter 21.2, table_bins over contiguous entries 26) 62.6; as it is, 14.6 + 32.4, of which the stretches of
+// eight keys in 245 parts are 6.  456,000: 38.1 -> 30.2; 60,000 and 24,000 voxels of a network's levels 48.2 -> 40.6 together.  The regions written
+// whole against slots of 32 bytes anywhere in the table, cleared by the first launch and claimed with a 64-bit compare-and-swap per block:
+// the probe passes of a 3x3x3 map 86 -> 59 and of a 5x5x5 map 189 -> 140; 1,800 voxels: 14.4 in two launches -> 10.2 in one.
 #include <stdlib.h>
 #include <string.h>
 
@@ -48,14 +47,14 @@ __device__ __forceinline__ PartRange part_range(int64_t n_keys, int part) {
   return r;
 }
 
-// Bins: capacity / 2048, at most WCN_MAX_BINS.  The histogram and scatter passes keep one counter
-// per bin in LDS (dynamic: 4 bytes per bin, 128 KB at the most), and a thread of the scatter pass
-// scans BINS_PER_THREAD bin totals: 4 up to 4096 bins, 32 beyond.
+// Bins: capacity / 2048, at most WCN_MAX_BINS.  The sort keeps one counter per bin in LDS (dynamic: 4 bytes per bin, 128 KB at the
+// most), and a thread of it adds up BPT of them: 4 up to 4096 bins, 32 beyond.
 constexpr int SMALL_BINS = 4096;
 
-// Keys per bin of one part of the keys, the part's bounding box.
-// ITEMS: the keys are made here too, [batch item, x, y, z] of three columns, and written on the way (the launch that did nothing else
-// took 7.7 us over 1 M rows; with this pass 11.4 + 7.7 -> 14.8; few keys: 2.4 + 2.1 -> 2.4 and a launch less).
+// The keys of one part in the order of their bins, within the part's own stretch of memory; where each bin begins there, and the
+// part's bounding box.  A part of up to 4,096 keys (up to a million altogether) is read once.  What its workgroup writes lies in 80 KB,
+// in whole lines.
+// ITEMS: the keys are made here too, [batch item, x, y, z] of three columns, and written on the way.
 struct KeysOfItems {
   const int32_t* coords;  // (n, 3)
   int4* rows;
@@ -63,31 +62,32 @@ struct KeysOfItems {
   int32_t batch_size;
 };
 
-template <bool ITEMS>
-__global__ void __launch_bounds__(1024) table_hist(const int4* __restrict__ keys, int64_t n_keys,
-                                                   int32_t bins, int32_t* __restrict__ hist,
-                                                   int32_t* __restrict__ part_box, KeysOfItems of) {
-  extern __shared__ int s_cnt[];  // [bins]
+template <int BPT, bool ITEMS>
+__global__ void __launch_bounds__(1024) table_sort(const int4* __restrict__ keys, int64_t n_keys, int32_t bins,
+                                                   int32_t* __restrict__ part_start, int32_t* __restrict__ part_box,
+                                                   int4* __restrict__ bin_coords, int32_t* __restrict__ bin_row, KeysOfItems of) {
+  extern __shared__ __attribute__((aligned(16))) int s_cur[];  // [bins], then (BPT 4) the part's keys and their numbers in it
   __shared__ int64_t s_start[ITEMS ? WCN_VOXEL_MAX_BATCH + 1 : 1];
-  if (ITEMS && threadIdx.x <= WCN_VOXEL_MAX_BATCH) s_start[threadIdx.x] = of.starts.start[threadIdx.x];
-  __shared__ int s_mn[16][4];
-  __shared__ int s_mx[16][4];
-  const int tid = threadIdx.x, parts = gridDim.x, part = wcn_xcd_tile((int)blockIdx.x, parts);
-  for (int b = tid; b < bins; b += 1024) s_cnt[b] = 0;
-  __syncthreads();
-  int mn[4] = {INT32_MAX, INT32_MAX, INT32_MAX, INT32_MAX};
-  int mx[4] = {INT32_MIN, INT32_MIN, INT32_MIN, INT32_MIN};
+  __shared__ int s_mn[16][4], s_mx[16][4], s_wave[16];
+  const int tid = threadIdx.x, lane = wcn_lane(), wave = tid >> 6;
+  const int parts = gridDim.x, part = wcn_xcd_tile((int)blockIdx.x, parts);
   const PartRange r = part_range(n_keys, part);
   const uint32_t bin_mask = (uint32_t)bins - 1u;
+  if (ITEMS && tid <= WCN_VOXEL_MAX_BATCH) s_start[tid] = of.starts.start[tid];
+  for (int b = tid; b < bins; b += 1024) s_cur[b] = 0;
+  __syncthreads();
   constexpr int PER = 4;  // keys a thread has in flight together
+  auto load = [&](int64_t i) {
+    return ITEMS ? make_int4(0, of.coords[3 * i], of.coords[3 * i + 1], of.coords[3 * i + 2]) : keys[i];
+  };
+  const bool kept = r.hi - r.lo <= 1024 * PER;  // a thread's keys stay in registers
+  int4 c[PER];
+  int rank[PER] = {};
+  int mn[4] = {INT32_MAX, INT32_MAX, INT32_MAX, INT32_MAX};
+  int mx[4] = {INT32_MIN, INT32_MIN, INT32_MIN, INT32_MIN};
   for (int64_t i0 = r.lo + tid; i0 < r.hi; i0 += 1024 * PER) {
-    int4 c[PER];
 #pragma unroll
-    for (int t = 0; t < PER; ++t) {
-      const int64_t i = i0 + t * 1024 < r.hi ? i0 + t * 1024 : i0;
-      if (ITEMS) c[t] = make_int4(0, of.coords[3 * i], of.coords[3 * i + 1], of.coords[3 * i + 2]);
-      else c[t] = keys[i];
-    }
+    for (int t = 0; t < PER; ++t) c[t] = load(i0 + t * 1024 < r.hi ? i0 + t * 1024 : i0);
 #pragma unroll
     for (int t = 0; t < PER; ++t) {
       if (ITEMS) {
@@ -95,7 +95,7 @@ __global__ void __launch_bounds__(1024) table_hist(const int4* __restrict__ keys
         c[t].x = wcn_item_of(s_start, of.batch_size, i);
         of.rows[i] = c[t];
       }
-      if (i0 + t * 1024 < r.hi) atomicAdd(&s_cnt[bin_of(c[t], bin_mask)], 1);
+      if (i0 + t * 1024 < r.hi) rank[t] = atomicAdd(&s_cur[bin_of(c[t], bin_mask)], 1);
       mn[0] = min(mn[0], c[t].x); mx[0] = max(mx[0], c[t].x);
       mn[1] = min(mn[1], c[t].y); mx[1] = max(mx[1], c[t].y);
       mn[2] = min(mn[2], c[t].z); mx[2] = max(mx[2], c[t].z);
@@ -110,8 +110,7 @@ __global__ void __launch_bounds__(1024) table_hist(const int4* __restrict__ keys
       mx[d] = max(mx[d], __shfl_xor(mx[d], s, 64));
     }
   }
-  const int wave = tid >> 6;
-  if (wcn_lane() == 0) {
+  if (lane == 0) {
 #pragma unroll
     for (int d = 0; d < 4; ++d) {
       s_mn[wave][d] = mn[d];
@@ -119,7 +118,14 @@ __global__ void __launch_bounds__(1024) table_hist(const int4* __restrict__ keys
     }
   }
   __syncthreads();
-  for (int b = tid; b < bins; b += 1024) hist[(int64_t)b * parts + part] = s_cnt[b];
+  int v[BPT], sum = 0;
+#pragma unroll
+  for (int t = 0; t < BPT; ++t) {
+    v[t] = tid * BPT + t < bins ? s_cur[tid * BPT + t] : 0;
+    sum += v[t];
+  }
+  const int incl = wcn_wave_inclusive_sum(sum);
+  if (lane == 63) s_wave[wave] = incl;
   if (tid < 4) {
     int a = s_mn[0][tid], b = s_mx[0][tid];
     for (int w = 1; w < 16; ++w) {
@@ -129,103 +135,6 @@ __global__ void __launch_bounds__(1024) table_hist(const int4* __restrict__ keys
     part_box[part * 8 + tid] = a;
     part_box[part * 8 + 4 + tid] = b;
   }
-}
-
-// One wave per bin: hist[bin][0..parts) becomes its exclusive prefix sum, bin_total[bin] its sum.
-// All loads of a column are issued before the first is used (parts <= 256: four per lane).
-__global__ void __launch_bounds__(256) table_colscan(int32_t* __restrict__ hist, int32_t bins,
-                                                     int32_t parts, int32_t* __restrict__ bin_total) {
-  const int lane = wcn_lane(), wave = threadIdx.x >> 6;
-  const int bin = blockIdx.x * 4 + wave;
-  if (bin >= bins) return;
-  int32_t* col = hist + (int64_t)bin * parts;
-  int v[4];
-#pragma unroll
-  for (int t = 0; t < 4; ++t) v[t] = t * 64 + lane < parts ? col[t * 64 + lane] : 0;
-  int carry = 0;
-#pragma unroll
-  for (int t = 0; t < 4; ++t) {
-    const int incl = wcn_wave_inclusive_sum(v[t]);
-    if (t * 64 + lane < parts) col[t * 64 + lane] = carry + incl - v[t];
-    carry += __shfl(incl, 63, 64);
-  }
-  if (lane == 0) bin_total[bin] = carry;
-}
-
-// Every key and its row to its place in its bin.  Each workgroup scans the bin totals into bin
-// starts for itself (1024 x BPT numbers); workgroup 0 also stores them for the next pass,
-// merges the parts' bounding boxes and writes the header.  Parts that follow one another run on one XCD: their pieces
-// of a bin (eight keys of 1 M: 128 bytes, 32 of rows) follow one another too (1 M keys: 25 -> 21.5 us).
-// COUNTS: the histogram as table_hist leaves it (up to OWN_SUMS words): every workgroup adds up what it needs of it, the
-// bins' totals and the keys of earlier parts, and table_colscan is not launched: scatter and scan over 100 k keys 7.6 + 2.8 to 3.8 us
-// -> 7.7, over 24 k 5.9 + 4 -> 5.9, over 160 k 7.7 + 3 -> 9.  At 500 k keys (31 words a lane) it took what it saved: 11.7 + 4.6 -> 16.2.
-constexpr int64_t OWN_SUMS = 16384;
-constexpr int OWN_BINS = 256;
-
-template <int BPT, bool COUNTS>
-__global__ void __launch_bounds__(1024) table_scatter(const int4* __restrict__ keys, int64_t n_keys,
-                                                      int32_t bins, const int32_t* __restrict__ hist,
-                                                      const int32_t* __restrict__ bin_total,
-                                                      int32_t* __restrict__ bin_start,
-                                                      const int32_t* __restrict__ part_box,
-                                                      WcnTableHeader* __restrict__ hdr,
-                                                      int64_t stats_offset,
-                                                      int4* __restrict__ bin_coords,
-                                                      int32_t* __restrict__ bin_row) {
-  extern __shared__ int s_cur[];  // [bins]
-  __shared__ int s_wave[16];
-  const int tid = threadIdx.x, lane = wcn_lane(), wave = tid >> 6;
-  const int parts = gridDim.x, part = wcn_xcd_tile((int)blockIdx.x, parts);
-  const PartRange r = part_range(n_keys, part);
-  // (COUNTS) the lanes of a bin, 4 to 64, and the first of the parts that each of them looks after
-  const int lanes_log = COUNTS ? 10 - (31 - __builtin_clz(bins)) : 0, lanes = 1 << lanes_log;
-  const int own_bin = tid >> lanes_log, first = tid & (lanes - 1);
-  constexpr int AHEAD = 4;
-  int n[COUNTS ? AHEAD : 1];
-  if (COUNTS) {
-#pragma unroll
-    for (int t = 0; t < AHEAD; ++t) n[COUNTS ? t : 0] = hist[own_bin * parts + (first + t * lanes < parts ? first + t * lanes : 0)];
-  }
-  constexpr int PER = 4;
-  int4 c[PER];  // the first keys are requested before anything else is waited for
-#pragma unroll
-  for (int t = 0; t < PER; ++t) {
-    const int64_t i = r.lo + tid + t * 1024;
-    c[t] = i < r.hi ? keys[i] : make_int4(0, 0, 0, 0);
-  }
-  int v[BPT], mine[BPT], sum = 0;
-  __shared__ int2 s_bin[COUNTS ? OWN_BINS : 1];
-  if (COUNTS) {
-    int all = 0, before = 0;
-    for (int p0 = first; p0 < parts; p0 += AHEAD * lanes) {
-      if (p0 != first) {
-#pragma unroll
-        for (int t = 0; t < AHEAD; ++t) n[COUNTS ? t : 0] = hist[own_bin * parts + (p0 + t * lanes < parts ? p0 + t * lanes : 0)];
-      }
-#pragma unroll
-      for (int t = 0; t < AHEAD; ++t) {
-        const int p = p0 + t * lanes;
-        all += p < parts ? n[COUNTS ? t : 0] : 0;
-        before += p < part ? n[COUNTS ? t : 0] : 0;
-      }
-    }
-    for (int d = 1; d < lanes; d <<= 1) {
-      all += __shfl_xor(all, d, 64);
-      before += __shfl_xor(before, d, 64);
-    }
-    if (first == 0) s_bin[COUNTS ? own_bin : 0] = make_int2(all, before);
-    __syncthreads();
-  }
-#pragma unroll
-  for (int t = 0; t < BPT; ++t) {
-    const int b = tid * BPT + t;
-    const int2 own = COUNTS && b < bins ? s_bin[COUNTS ? b : 0] : make_int2(0, 0);
-    v[t] = COUNTS ? own.x : b < bins ? bin_total[b] : 0;
-    mine[t] = COUNTS ? own.y : b < bins ? hist[(int64_t)b * parts + part] : 0;
-    sum += v[t];
-  }
-  const int incl = wcn_wave_inclusive_sum(sum);
-  if (lane == 63) s_wave[wave] = incl;
   __syncthreads();
   int run = incl - sum;
   for (int w = 0; w < wave; ++w) run += s_wave[w];
@@ -233,52 +142,48 @@ __global__ void __launch_bounds__(1024) table_scatter(const int4* __restrict__ k
   for (int t = 0; t < BPT; ++t) {
     const int b = tid * BPT + t;
     if (b < bins) {
-      s_cur[b] = run + mine[t];
-      if (part == 0) bin_start[b] = run;
+      s_cur[b] = run;
+      part_start[(int64_t)b * parts + part] = run;
     }
     run += v[t];
   }
-  if (part == 0) {
-    if (tid == 0) bin_start[bins] = (int32_t)n_keys;
-    if (wave == 1) {  // the boxes: lane d + 8 j merges column d of parts j, j + 8, ...
-      const int d = lane & 7;
-      int acc = d < 4 ? INT32_MAX : INT32_MIN;
-      for (int p = lane >> 3; p < parts; p += 8) {
-        const int x = part_box[p * 8 + d];
-        acc = d < 4 ? min(acc, x) : max(acc, x);
-      }
-#pragma unroll
-      for (int s = 8; s < 64; s <<= 1) {
-        const int o = __shfl_xor(acc, s, 64);
-        acc = d < 4 ? min(acc, o) : max(acc, o);
-      }
-      if (lane < 4) hdr->mn[lane] = acc;
-      else if (lane < 8) hdr->mx[lane - 4] = acc;
-      if (lane == 8) {
-        hdr->num_keys = (int32_t)n_keys;
-        hdr->bins = bins;
-        hdr->stats_offset = stats_offset;
-      }
-    }
-  }
+  if (tid == 0) part_start[(int64_t)bins * parts + part] = r.hi > r.lo ? (int32_t)(r.hi - r.lo) : 0;
   __syncthreads();
-  const uint32_t bin_mask = (uint32_t)bins - 1u;
-  for (int64_t i0 = r.lo + tid; i0 < r.hi; i0 += 1024 * PER) {
-    if (i0 != r.lo + tid) {
+  auto put = [&](int64_t i, const int4 key, int at) {
+    bin_coords[r.lo + at] = key;
+    bin_row[r.lo + at] = (int32_t)i;
+  };
+  if (kept) {
+    // through LDS, for whole lines: written one by one a part's keys are as many requests (1 M voxels 19.8 us, 14.6 so)
+    int4* const s_key = reinterpret_cast<int4*>(s_cur + bins);
+    uint16_t* const s_row = reinterpret_cast<uint16_t*>(s_key + 1024 * PER);
 #pragma unroll
-      for (int t = 0; t < PER; ++t) {
-        const int64_t i = i0 + t * 1024;
-        c[t] = keys[i < r.hi ? i : i0];
+    for (int t = 0; t < PER; ++t) {
+      if (r.lo + tid + t * 1024 >= r.hi) continue;
+      const int at = s_cur[bin_of(c[t], bin_mask)] + rank[t];
+      if (BPT == 4) {
+        s_key[at] = c[t];
+        s_row[at] = (uint16_t)(tid + t * 1024);
+      } else {
+        put(r.lo + tid + t * 1024, c[t], at);
       }
     }
+    if (BPT != 4) return;
+    __syncthreads();
+#pragma unroll
+    for (int t = 0; t < PER; ++t)
+      if (r.lo + tid + t * 1024 < r.hi) put(r.lo + s_row[tid + t * 1024], s_key[tid + t * 1024], tid + t * 1024);
+    return;
+  }
+  for (int64_t i0 = r.lo + tid; i0 < r.hi; i0 += 1024 * PER) {
+#pragma unroll
+    for (int t = 0; t < PER; ++t) c[t] = load(i0 + t * 1024 < r.hi ? i0 + t * 1024 : i0);
 #pragma unroll
     for (int t = 0; t < PER; ++t) {
       const int64_t i = i0 + t * 1024;
-      if (i < r.hi) {
-        const int pos = atomicAdd(&s_cur[bin_of(c[t], bin_mask)], 1);
-        bin_coords[pos] = c[t];
-        bin_row[pos] = (int32_t)i;
-      }
+      if (i >= r.hi) continue;
+      if (ITEMS) c[t].x = wcn_item_of(s_start, of.batch_size, i);
+      put(i, c[t], atomicAdd(&s_cur[bin_of(c[t], bin_mask)], 1));
     }
   }
 }
@@ -331,21 +236,60 @@ __device__ __forceinline__ int bin_find(const BinLds* s, unsigned long long key,
 // Where the block of a key is looked for in its bin's region.
 __device__ __forceinline__ uint32_t home_in_bin(const int4 c) { return wcn_home_slot_of(c.x, c.y >> 2, c.z >> 2, c.w >> 2, 0u); }
 
-// Where a bin's entries [lo, hi) come from.
-struct BinEntries {  // as table_scatter left them
+// Where a bin's entries [lo, hi) come from: at(e) is what coords() and row() are asked with.
+constexpr int MAX_PARTS = 256;
+struct PartedEntries {  // as table_sort left them, a stretch in every part
   const int4* __restrict__ keys;
   const int32_t* __restrict__ rows;
-  __device__ __forceinline__ int4 coords(int e) const { return keys[e]; }
-  __device__ __forceinline__ int32_t row(int e) const { return rows[e]; }
+  const int32_t* first;  // [MAX_PARTS] LDS: entries of the bin in the parts before; INT32_MAX past the last part
+  const int32_t* shift;  // [MAX_PARTS] LDS: where the part's first lies, less that
+  int lo;
+  template <int N>
+  __device__ __forceinline__ void at(int (&e)[N]) const {  // N searches abreast
+    int part[N];
+#pragma unroll
+    for (int t = 0; t < N; ++t) part[t] = 0;
+#pragma nounroll
+    for (int step = MAX_PARTS / 2; step >= 1; step >>= 1) {
+#pragma unroll
+      for (int t = 0; t < N; ++t) part[t] += first[part[t] + step] <= e[t] - lo ? step : 0;
+    }
+#pragma unroll
+    for (int t = 0; t < N; ++t) e[t] += shift[part[t]] - lo;
+  }
+  __device__ __forceinline__ int at(int e) const {
+    int one[1] = {e};
+    at(one);
+    return one[0];
+  }
+  __device__ __forceinline__ int4 coords(int i) const { return keys[i]; }
+  __device__ __forceinline__ int32_t row(int i) const { return rows[i]; }
 };
 template <class Keys>
 struct ListedEntries {  // the rows of a few keys, listed in LDS
   Keys keys;
   const uint16_t* list;
   int lo;
-  __device__ __forceinline__ int4 coords(int e) const { return keys(list[e - lo]); }
-  __device__ __forceinline__ int32_t row(int e) const { return list[e - lo]; }
+  template <int N>
+  __device__ __forceinline__ void at(int (&e)[N]) const {
+#pragma unroll
+    for (int t = 0; t < N; ++t) e[t] = list[e[t] - lo];
+  }
+  __device__ __forceinline__ int at(int e) const { return list[e - lo]; }
+  __device__ __forceinline__ int4 coords(int i) const { return keys(i); }
+  __device__ __forceinline__ int32_t row(int i) const { return i; }
 };
+
+// The layout of a box in LDS, in scalar registers.
+__device__ __forceinline__ WcnLayout layout_of(const WcnTableHeader& box) {
+  WcnTableHeader h;
+#pragma unroll
+  for (int d = 0; d < 4; ++d) {
+    h.mn[d] = __builtin_amdgcn_readfirstlane(box.mn[d]);
+    h.mx[d] = __builtin_amdgcn_readfirstlane(box.mx[d]);
+  }
+  return wcn_make_layout(&h);
+}
 
 template <bool WANT_SLOT_OF, int E, class Entries>
 __device__ __forceinline__ void build_bin(const Entries& in, int bin, int lo, int hi, const WcnLayout& L, BinLds* s,
@@ -367,16 +311,20 @@ __device__ __forceinline__ void build_bin(const Entries& in, int bin, int lo, in
   int32_t row[E];
   int where[E];  // place of the key's block << 6 | voxel bit, or -1
 #pragma unroll
+  for (int t = 0; t < E; ++t) where[t] = lo + tid + t * 1024 < hi ? lo + tid + t * 1024 : lo;
+  in.at(where);
+#pragma unroll
   for (int t = 0; t < E; ++t) {
-    const int e = lo + tid + t * 1024;
-    row[t] = in.row(e < hi ? e : lo);
-    c[t] = in.coords(e < hi ? e : lo);
+    row[t] = in.row(where[t]);
+    c[t] = in.coords(where[t]);
   }
   if (!L.ok) {
     if (tid == 0) bin_stats[2 * bin] = bin_stats[2 * bin + 1] = 0;
+#pragma nounroll
     for (int e = lo + tid; e < hi; e += 1024) {
-      if (WANT_SLOT_OF) slot_of[in.row(e)] = -1;
-      order_row[e] = in.row(e);
+      const int32_t rw = in.row(in.at(e));
+      if (WANT_SLOT_OF) slot_of[rw] = -1;
+      order_row[e] = rw;
       order_tag[e] = 0;
     }
     return;
@@ -402,8 +350,9 @@ __device__ __forceinline__ void build_bin(const Entries& in, int bin, int lo, in
       where[t] = h < 0 ? -1 : h << 6 | (int)wcn_block_bit(r);
     }
   }
+#pragma nounroll
   for (int e = lo + tid + E * 1024; e < hi; e += 1024) {
-    const int4 ce = in.coords(e);
+    const int4 ce = in.coords(in.at(e));
     uint32_t r[4];
     wcn_relative(L, ce.x, ce.y, ce.z, ce.w, r);
     lost |= bin_insert(s, wcn_block_key(L, r), home_in_bin(ce), wcn_block_bit(r)) < 0;
@@ -505,12 +454,14 @@ __device__ __forceinline__ void build_bin(const Entries& in, int bin, int lo, in
     const int e = lo + tid + t * 1024;
     if (e < hi) place(row[t], where[t], e);
   }
+#pragma nounroll
   for (int e = lo + tid + E * 1024; e < hi; e += 1024) {
-    const int4 ce = in.coords(e);
+    const int i = in.at(e);
+    const int4 ce = in.coords(i);
     uint32_t r[4];
     wcn_relative(L, ce.x, ce.y, ce.z, ce.w, r);
     const int h = bin_find(s, wcn_block_key(L, r), home_in_bin(ce));
-    place(in.row(e), h < 0 ? -1 : h << 6 | (int)wcn_block_bit(r), e);
+    place(in.row(i), h < 0 ? -1 : h << 6 | (int)wcn_block_bit(r), e);
   }
   __syncthreads();
   if (repeats && low_in_lds)
@@ -521,10 +472,20 @@ __device__ __forceinline__ void build_bin(const Entries& in, int bin, int lo, in
   }
 }
 
+struct BinsLds {
+  BinLds bin;
+  WcnTableHeader box;
+  int32_t first[MAX_PARTS], shift[MAX_PARTS];
+  int32_t wave[2][4], part[16][8];
+};
+
+// A bin's keys in front of it, its own and where they lie follow from two rows of the parts' starts (the keys of a part in the bins
+// before are its start), the box from the parts' boxes: every workgroup finds both, and no launch stands between the sort and this one.
 template <bool WANT_SLOT_OF, bool TWO>
-__global__ void __launch_bounds__(1024, TWO ? 8 : 4) table_bins(const WcnTableHeader* __restrict__ hdr,
+__global__ void __launch_bounds__(1024, TWO ? 8 : 4) table_bins(WcnTableHeader* __restrict__ hdr, int64_t n_keys, int64_t stats_offset,
                                                    WcnSlot* __restrict__ slots, unsigned long long* __restrict__ wide_keys,
-                                                   const int32_t* __restrict__ bin_start,
+                                                   const int32_t* __restrict__ part_start, const int32_t* __restrict__ part_box,
+                                                   int32_t parts, int32_t* __restrict__ bin_start,
                                                    const int4* __restrict__ bin_coords,
                                                    const int32_t* __restrict__ bin_row,
                                                    int32_t* __restrict__ order_tag,
@@ -534,10 +495,65 @@ __global__ void __launch_bounds__(1024, TWO ? 8 : 4) table_bins(const WcnTableHe
                                                    int32_t* __restrict__ slot_of,
                                                    int32_t* __restrict__ bin_stats) {
   extern __shared__ __attribute__((aligned(16))) unsigned char bin_smem[];
-  const BinEntries in{bin_coords, bin_row};
-  build_bin<WANT_SLOT_OF, TWO ? 3 : 4>(in, (int)blockIdx.x, bin_start[blockIdx.x], bin_start[blockIdx.x + 1], wcn_make_layout(hdr),
-                          reinterpret_cast<BinLds*>(bin_smem), slots, wide_keys, order_tag, order_row, block_list,
-                          perm, slot_of, bin_stats);
+  BinsLds* const s = reinterpret_cast<BinsLds*>(bin_smem);
+  const int tid = threadIdx.x, lane = wcn_lane(), wave = tid >> 6, bin = (int)blockIdx.x;
+  int before = 0, n = 0, incl = 0;
+  if (tid < MAX_PARTS) {  // a thread per part
+    const int32_t* const at = part_start + (int64_t)bin * parts + (tid < parts ? tid : 0);
+    before = tid < parts ? at[0] : 0;
+    n = tid < parts ? at[parts] - before : 0;
+  }
+  // (columns of the boxes lane & 7: the values of a thread are of one column)
+  const int column = lane & 7;
+  int v = column < 4 ? INT32_MAX : INT32_MIN;
+#pragma unroll
+  for (int t = 0; t < MAX_PARTS * 8 / 1024; ++t) {
+    const int i = tid + t * 1024, x = part_box[i < parts * 8 ? i : column];
+    v = column < 4 ? min(v, x) : max(v, x);
+  }
+#pragma unroll
+  for (int d = 8; d < 64; d <<= 1) {
+    const int o = __shfl_xor(v, d, 64);
+    v = column < 4 ? min(v, o) : max(v, o);
+  }
+  if (lane < 8) s->part[wave][lane] = v;
+  if (tid < MAX_PARTS) {
+    incl = wcn_wave_inclusive_sum(n);
+    const int all_before = wcn_wave_inclusive_sum(before);
+    if (lane == 63) {
+      s->wave[0][wave] = incl;
+      s->wave[1][wave] = all_before;
+    }
+  }
+  __syncthreads();
+  if (tid < 8) {
+    int a = s->part[0][tid];
+    for (int w = 1; w < 16; ++w) a = tid < 4 ? min(a, s->part[w][tid]) : max(a, s->part[w][tid]);
+    *(tid < 4 ? &s->box.mn[tid] : &s->box.mx[tid - 4]) = a;
+    if (bin == 0) *(tid < 4 ? &hdr->mn[tid] : &hdr->mx[tid - 4]) = a;
+  }
+  if (tid < MAX_PARTS) {
+    int first = incl - n;
+    for (int w = 0; w < wave; ++w) first += s->wave[0][w];
+    const int64_t chunk = (n_keys + parts - 1) / parts;
+    s->first[tid] = tid < parts ? first : INT32_MAX;
+    s->shift[tid] = tid < parts ? (int32_t)(tid * chunk) + before - first : 0;
+  }
+  const int lo = __builtin_amdgcn_readfirstlane(s->wave[1][0] + s->wave[1][1] + s->wave[1][2] + s->wave[1][3]);
+  const int hi = __builtin_amdgcn_readfirstlane(lo + s->wave[0][0] + s->wave[0][1] + s->wave[0][2] + s->wave[0][3]);
+  if (tid == 0) {
+    bin_start[bin] = lo;
+    if (bin == (int)gridDim.x - 1) bin_start[bin + 1] = (int32_t)n_keys;
+    if (bin == 0) {
+      hdr->num_keys = (int32_t)n_keys;
+      hdr->bins = (int32_t)gridDim.x;
+      hdr->stats_offset = stats_offset;
+    }
+  }
+  __syncthreads();
+  const PartedEntries in{bin_coords, bin_row, s->first, s->shift, lo};
+  build_bin<WANT_SLOT_OF, TWO ? 2 : 4>(in, bin, lo, hi, layout_of(s->box), &s->bin, slots, wide_keys, order_tag, order_row,
+                          block_list, perm, slot_of, bin_stats);
 }
 
 // ---- few keys -----------------------------------------------------------------------------------
@@ -562,7 +578,7 @@ struct KeyRows {
   const int4* __restrict__ keys;
   __device__ __forceinline__ int4 operator()(int i) const { return keys[i]; }
 };
-struct KeyItems {  // made here, as in table_hist
+struct KeyItems {  // made here, as in table_sort
   const int32_t* __restrict__ coords;
   const int64_t* start;
   int32_t batch_size;
@@ -634,7 +650,7 @@ __global__ void __launch_bounds__(1024) table_small(const int4* __restrict__ row
     if (bin == 0 && tid < 8) *(tid < 4 ? &hdr->mn[tid] : &hdr->mx[tid - 4]) = a;
   }
   __syncthreads();
-  const int lo = s->box.total, hi = lo + s->listed;
+  const int lo = __builtin_amdgcn_readfirstlane(s->box.total), hi = __builtin_amdgcn_readfirstlane(lo + s->listed);
   if (tid == 0) {
     bin_start[bin] = lo;
     if (bin == bins - 1) bin_start[bins] = n_keys;
@@ -645,7 +661,7 @@ __global__ void __launch_bounds__(1024) table_small(const int4* __restrict__ row
     }
   }
   const ListedEntries<Keys> in{keys, s->list, lo};
-  build_bin<WANT_SLOT_OF, 4>(in, bin, lo, hi, wcn_make_layout(&s->box), &s->bin, slots, wide_keys, order_tag, order_row,
+  build_bin<WANT_SLOT_OF, 4>(in, bin, lo, hi, layout_of(s->box), &s->bin, slots, wide_keys, order_tag, order_row,
                           block_list, perm, slot_of, bin_stats);
 }
 
@@ -721,7 +737,7 @@ inline int grid_for(int64_t n, int block, int cap = 0x7fffffff) {
 // LDS beyond the default limit: lifted once per device and kernel.
 static int allow_lds(const void* kernel, size_t bytes, int which) {
   static std::mutex mu;
-  static bool allowed[11][64] = {};
+  static bool allowed[12][64] = {};
   int device = 0;
   if (hipGetDevice(&device) != hipSuccess || device < 0 || device >= 64) return WCN_ERR_LAUNCH;
   std::lock_guard<std::mutex> hold(mu);
@@ -751,32 +767,21 @@ static int table_build_from(const int32_t* keys, int64_t n_keys, const WcnTableV
     return WCN_OK;
   }
   const bool many_bins = v.bins > SMALL_BINS;
-  const size_t counters = sizeof(int) * (size_t)v.bins;
-  const bool own_sums = v.bins <= OWN_BINS && (int64_t)v.bins * v.parts <= OWN_SUMS;
-  auto scatter = many_bins  ? table_scatter<WCN_MAX_BINS / 1024, false>
-                 : own_sums ? table_scatter<SMALL_BINS / 1024, true>
-                            : table_scatter<SMALL_BINS / 1024, false>;
-  auto hist = items ? table_hist<true> : table_hist<false>;
+  auto sort = items ? (many_bins ? table_sort<WCN_MAX_BINS / 1024, true> : table_sort<SMALL_BINS / 1024, true>)
+                    : (many_bins ? table_sort<WCN_MAX_BINS / 1024, false> : table_sort<SMALL_BINS / 1024, false>);
   const bool two = v.bins > 256;  // more than one per CU: 64 registers let two share it (fewer bins: 15.7 -> 22 us of 500 k voxels)
   auto fn = want_slot_of ? (two ? table_bins<true, true> : table_bins<true, false>)
                          : (two ? table_bins<false, true> : table_bins<false, false>);
-  if (allow_lds((const void*)fn, sizeof(BinLds), (want_slot_of ? 1 : 0) + (two ? 3 : 0)) != WCN_OK) return WCN_ERR_LAUNCH;
-  if (many_bins) {
-    const size_t most = sizeof(int) * WCN_MAX_BINS;
-    if (allow_lds((const void*)hist, most, items ? 6 : 2) != WCN_OK || allow_lds((const void*)scatter, most, 5) != WCN_OK)
-      return WCN_ERR_LAUNCH;
-  }
-  hipLaunchKernelGGL(hist, dim3(v.parts), dim3(1024), counters, s, k4, n_keys, v.bins, v.hist,
-                     v.part_box, items ? *items : KeysOfItems{});
-  if (!own_sums)
-    hipLaunchKernelGGL(table_colscan, dim3((v.bins + 3) / 4), dim3(256), 0, s, v.hist, v.bins,
-                       v.parts, v.bin_total);
-  hipLaunchKernelGGL(scatter, dim3(v.parts), dim3(1024), counters, s, k4, n_keys, v.bins, v.hist,
-                     v.bin_total, v.bin_start, v.part_box, v.hdr,
-                     stats, (int4*)v.bin_coords,
-                     v.bin_row);
-  hipLaunchKernelGGL(fn, dim3(v.bins), dim3(1024), sizeof(BinLds), s, v.hdr, v.slots, v.wide_keys,
-                     v.bin_start, (const int4*)v.bin_coords, v.bin_row, v.order_tag, v.order_row,
+  if (allow_lds((const void*)fn, sizeof(BinsLds), (want_slot_of ? 1 : 0) + (two ? 3 : 0)) != WCN_OK) return WCN_ERR_LAUNCH;
+  // (up to 4096 bins beside the counters a part's keys, 16 and 2 bytes each)
+  const size_t sort_lds = sizeof(int) * (size_t)v.bins + (many_bins ? 0 : 4096 * 18);
+  if (allow_lds((const void*)sort, many_bins ? sizeof(int) * WCN_MAX_BINS : sizeof(int) * SMALL_BINS + 4096 * 18,
+                many_bins ? (items ? 6 : 2) : (items ? 11 : 5)) != WCN_OK)
+    return WCN_ERR_LAUNCH;
+  hipLaunchKernelGGL(sort, dim3(v.parts), dim3(1024), sort_lds, s, k4, n_keys, v.bins, v.part_start, v.part_box,
+                     (int4*)v.bin_coords, v.bin_row, items ? *items : KeysOfItems{});
+  hipLaunchKernelGGL(fn, dim3(v.bins), dim3(1024), sizeof(BinsLds), s, v.hdr, n_keys, stats, v.slots, v.wide_keys, v.part_start,
+                     v.part_box, v.parts, v.bin_start, (const int4*)v.bin_coords, v.bin_row, v.order_tag, v.order_row,
                      v.block_list, v.perm, v.slot_of, v.bin_stats);
   WCN_LAUNCH_CHECK();
   return WCN_OK;
