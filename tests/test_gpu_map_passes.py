@@ -158,7 +158,7 @@ def test_a_result_on_its_way_does_not_reach_the_next_one(oracle, then):
 
 
 @pytest.mark.parametrize("kernel,stride,dilation", [(3, 1, 1), (3, 2, 1), (2, 2, 1), (2, 1, 1), (5, 1, 1), (3, 1, 2), ((1, 3, 2), 1, 1)])
-@pytest.mark.parametrize("n", [1, 63, 64, 65, 256, 257, 511, 513, 2049, 30_011, 131_073, (1 << 18), (1 << 18) + 1])
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 256, 257, 511, 513, 2049, 30_011, 131_073, (1 << 18), (1 << 18) + 1, 700_003])
 def test_one_call_leaves_what_two_leave(n, kernel, stride, dilation):
     """wcn_kmap_count_fill against wcn_kmap_count and wcn_kmap_fill: offsets, status, group starts and lists, also where the lists
     are too short and a fill follows."""

@@ -38,6 +38,8 @@ struct KmapWorkspace {  // host-computed addresses inside a kmap workspace
   uint16_t* counts;     // (K, C): hits per offset of the probe's workgroups of 256 rows (maps that kmap_starts_emit finishes)
   int64_t G;            // number of 64-row groups
   int32_t C;            // number of the probe's workgroups, in whole 16-byte vectors of counts
+  int32_t* blocks;      // (K, B + 1): the same of larger maps; after the scan, exclusive prefix sums
+  int32_t B;            // number of the probe's workgroups
 };
 
 // Up to so many rows the emit pass adds up the counts of all 256-row workgroups itself (kmap_starts_emit).  What every
@@ -47,7 +49,7 @@ struct KmapWorkspace {  // host-computed addresses inside a kmap workspace
 //     3x3x3   20.1 19.4  22.2 20.3  24.6 22.8  26.9 25.2  28.5 26.1  32.4 28.7  46.0  46.0  59.1  61.1   88.3 104.5
 //     5x5x5   38.5 35.6  40.6 37.5  44.4 40.7  51.0 44.7  57.1 56.3  63.2 61.2  92.7 111.4   124   156    192   292
 // (the emit pass overlaps the host's read here; with a layer behind it a map of 1,800 to 60,000 rows gains 4 to 5: scan 5.6 and emit
-// 5.4 us against 6.3 together.)
+// 5.4 us against 6.3 together.)  Beyond, the counts are scanned first: 3x3x3 over 265,000 rows 37.6 35.6, 1 M 87.6 81.6.
 constexpr int64_t KMAP_OWN_SUMS = 1 << 18;
 
 inline size_t kmap_layout(void* base, int64_t num_out, int32_t K, KmapWorkspace* w) {
@@ -70,6 +72,10 @@ inline size_t kmap_layout(void* base, int64_t num_out, int32_t K, KmapWorkspace*
   const int64_t C = ((num_out + 255) / 256 + 7) / 8 * 8;
   if (w) w->counts = (uint16_t*)(p + off);
   if (num_out <= KMAP_OWN_SUMS) off += wcn_align256(sizeof(uint16_t) * (size_t)K * (size_t)C);
+  const int64_t B = (num_out + 255) / 256;
+  if (w) w->blocks = (int32_t*)(p + off);
+  if (num_out > KMAP_OWN_SUMS) off += wcn_align256(sizeof(int32_t) * (size_t)K * (size_t)(B + 1));
+  if (w) w->B = (int32_t)B;
   if (w) w->G = G;
   if (w) w->C = (int32_t)C;
   return off;
@@ -84,8 +90,10 @@ struct KmapProbe {      // what the probe pass leaves for the scan and the emit 
   int32_t* found;
   uint16_t* tags;
   int32_t* ticket;      // set to zero
-  uint16_t* counts;     // (fixed sizes) null: not asked for
+  uint16_t* counts;     // (fixed sizes) hits per offset of a workgroup, or null, and
   int32_t C;
+  int32_t* blocks;      // the same in 32 bits, or null
+  int32_t B;
 };
 
 // ---- generic kernel: any kernel size up to WCN_MAX_OFFSETS offsets -----------------------------
@@ -360,6 +368,8 @@ __global__ void __launch_bounds__(256) kmap_pass_fixed(const WcnTableHeader* __r
     if ((i & 3) < there) groups[(int64_t)(i >> 2) * (G + 1) + (group - wave) + (i & 3)] = s_count[i & 3][i >> 2];
   if (o.counts && tid < K)
     o.counts[tid * o.C + (int)(group >> 2)] = (uint16_t)(s_count[0][tid] + s_count[1][tid] + s_count[2][tid] + s_count[3][tid]);
+  if (o.blocks && tid < K)
+    o.blocks[(int64_t)tid * (o.B + 1) + (group >> 2)] = s_count[0][tid] + s_count[1][tid] + s_count[2][tid] + s_count[3][tid];
 }
 
 // Emit pass: pair lists from the scanned counts and what the probe pass has parked, a lane per
@@ -1062,17 +1072,21 @@ __global__ void __launch_bounds__(SELF_CHUNK) self_emit(const uint32_t* __restri
 // (but the starts of the row of all hits, which nothing reads): the first workgroup the offsets, the table's status and the host's
 // mailbox, and every one the starts of its own eight groups, in the place of their counts, which no other workgroup reads.
 // KL: counts of a wave's offsets requested together.
-template <int KL>
+// SCANNED (larger maps): kmap_scan_rows has made starts of the counts, a quarter of what the starts of all groups are (which these
+// workgroups make of them), and has written the rest.  Over 1 M rows of 3x3x3 and 5x5x5 scan and emit 14.2 + 20.6 and 19.3 + 49.4 us
+// with the starts of all groups scanned, 7.8 + 19.1 and 12.2 + 48.4 so.
+template <int KL, bool SCANNED>
 __global__ void __launch_bounds__(512) kmap_starts_emit(const int32_t* __restrict__ found, const uint16_t* __restrict__ tags,
                                                         int32_t* __restrict__ groups, const uint16_t* __restrict__ counts,
-                                                        int32_t blocks, int32_t C, int32_t K, int64_t G, int64_t pair_capacity,
+                                                        const int32_t* __restrict__ starts, int32_t blocks, int32_t C, int32_t K, int64_t G, int64_t pair_capacity,
                                                         int32_t* __restrict__ in_maps, int32_t* __restrict__ out_maps,
                                                         KmapFinish fin) {
   constexpr int GROUPS = 8, MAX_K = 128;
   __shared__ int32_t s_all[MAX_K], s_before[MAX_K];  // hits of an offset: of all workgroups, of those before this one
-  __shared__ int32_t s_base[MAX_K];                  // where its pairs begin in the lists
+  typedef typename std::conditional<SCANNED, int64_t, int32_t>::type Place;  // (few rows: few pairs)
+  __shared__ Place s_base[MAX_K];                    // where its pairs begin in the lists
   __shared__ int32_t s_start[MAX_K][GROUPS + 1];
-  __shared__ int32_t s_shift[GROUPS][MAX_K];
+  __shared__ Place s_shift[GROUPS][MAX_K];
   __shared__ int32_t s_stat[3][GROUPS];
   __shared__ int32_t s_total;
   const int tid = threadIdx.x, lane = wcn_lane(), wave = tid >> 6;
@@ -1100,9 +1114,16 @@ __global__ void __launch_bounds__(512) kmap_starts_emit(const int32_t* __restric
     tag[u] = of[64 * u + lane];
   }
 
+  if (SCANNED) {
+    for (int k = tid; k < K; k += 512) {
+      s_before[k] = starts[(int64_t)k * (blocks + 1) + own];
+      s_all[k] = starts[(int64_t)k * (blocks + 1) + blocks];
+      s_base[k] = (Place)fin.result[k];
+    }
+  }
   // a wave looks after the offsets wave, wave + 8, ...; a lane takes eight counts at a time
   typedef uint32_t Counts __attribute__((ext_vector_type(4)));
-  for (int k0 = wave; k0 < K; k0 += GROUPS * KL) {
+  for (int k0 = SCANNED ? K : wave; k0 < K; k0 += GROUPS * KL) {
     int all[KL], before[KL];
 #pragma unroll
     for (int j = 0; j < KL; ++j) all[j] = before[j] = 0;
@@ -1133,7 +1154,7 @@ __global__ void __launch_bounds__(512) kmap_starts_emit(const int32_t* __restric
       }
     }
   }
-  if (tile == 0) {  // the table's status: the sums of its bins' counts
+  if (!SCANNED && tile == 0) {  // the table's status: the sums of its bins' counts
     const int32_t bins = fin.hdr->bins;
     const int32_t* stats = reinterpret_cast<const int32_t*>(reinterpret_cast<const char*>(fin.hdr) + fin.hdr->stats_offset);
     int voxels = 0, occupied = 0;
@@ -1153,7 +1174,7 @@ __global__ void __launch_bounds__(512) kmap_starts_emit(const int32_t* __restric
     }
   }
   __syncthreads();
-  if (wave == 0) {
+  if (!SCANNED && wave == 0) {
     int run = 0;
     for (int k0 = 0; k0 < K; k0 += 64) {
       const int k = k0 + lane, n = k < K ? s_all[k] : 0;
@@ -1212,7 +1233,7 @@ __global__ void __launch_bounds__(512) kmap_starts_emit(const int32_t* __restric
     }
   }
   __syncthreads();
-  if (s_total > pair_capacity || group >= G) return;
+  if ((SCANNED ? fin.result[K] > pair_capacity || fin.result[K + 1] != 0 : s_total > pair_capacity) || group >= G) return;
   int total = 0;
   for (int k0 = 0; k0 < K; k0 += 64) {
     const int k = k0 + lane;
@@ -1237,7 +1258,7 @@ __global__ void __launch_bounds__(512) kmap_starts_emit(const int32_t* __restric
     for (int u = 0; u < AHEAD; ++u) {
       const int p = p0 + 64 * u + lane;
       if (p < total) {
-        const int dst = s_shift[wave][tag[u] >> 6] + p;
+        const Place dst = s_shift[wave][tag[u] >> 6] + p;
         in_maps[dst] = row[u];
         out_maps[dst] = (int32_t)(group * 64) + (int32_t)(tag[u] & 63u);
       }
@@ -1277,10 +1298,10 @@ inline bool table_args_ok(const void* table, int64_t n_keys, int64_t capacity) {
 }
 
 void launch_probe(const WcnTableView& v, const int32_t* out_coords, int64_t num_out,
-                  const KmapGeom& g, const KmapWorkspace& w, hipStream_t s, bool counts = false) {
+                  const KmapGeom& g, const KmapWorkspace& w, hipStream_t s, bool counts = false, bool blocks = false) {
   const dim3 grid(grid_for(num_out, 256)), block(256);
   const WcnTableRef table = wcn_table_ref(v);
-  const KmapProbe o = {w.found, w.tags, w.ticket, counts ? w.counts : nullptr, w.C};
+  const KmapProbe o = {w.found, w.tags, w.ticket, counts ? w.counts : nullptr, w.C, blocks ? w.blocks : nullptr, w.B};
   if (is_fixed_size(g, 3, 3, 3)) {
     hipLaunchKernelGGL((kmap_pass_fixed<3, 3, 3, false>), grid, block, 0, s, v.hdr, table,
                        v.perm, (const int4*)out_coords, num_out, g, w.groups, w.G, o);
@@ -1299,22 +1320,16 @@ void launch_probe(const WcnTableView& v, const int32_t* out_coords, int64_t num_
   }
 }
 
-// Whether kmap_starts_emit finishes a map: one that kmap_pass_fixed probes (its workgroups leave their counts), with few enough of them.
-bool own_sums(const KmapGeom& g, int64_t num_out) {
-  return num_out > 0 && num_out <= KMAP_OWN_SUMS &&
-         (is_fixed_size(g, 3, 3, 3) || is_fixed_size(g, 2, 2, 2) || is_fixed_size(g, 5, 5, 5));
+// Whether kmap_starts_emit finishes a map: one that kmap_pass_fixed probes (its workgroups leave their counts).
+bool leaves_counts(const KmapGeom& g, int64_t num_out) {
+  return num_out > 0 && (is_fixed_size(g, 3, 3, 3) || is_fixed_size(g, 2, 2, 2) || is_fixed_size(g, 5, 5, 5));
 }
 
 void launch_starts_emit(int64_t num_out, const KmapGeom& g, const KmapWorkspace& w, int64_t pair_capacity, int32_t* in_maps,
                         int32_t* out_maps, const KmapFinish& fin, hipStream_t s) {
-  const dim3 grid(grid_for(num_out, 512)), block(512);
-  const int32_t blocks = (int32_t)((num_out + 255) / 256);
-  if (g.K <= 8)
-    hipLaunchKernelGGL(kmap_starts_emit<1>, grid, block, 0, s, w.found, w.tags, w.groups, w.counts, blocks, w.C, g.K, w.G,
-                       pair_capacity, in_maps, out_maps, fin);
-  else
-    hipLaunchKernelGGL(kmap_starts_emit<4>, grid, block, 0, s, w.found, w.tags, w.groups, w.counts, blocks, w.C, g.K, w.G,
-                       pair_capacity, in_maps, out_maps, fin);
+  auto fn = num_out > KMAP_OWN_SUMS ? kmap_starts_emit<1, true> : g.K <= 8 ? kmap_starts_emit<1, false> : kmap_starts_emit<4, false>;
+  hipLaunchKernelGGL(fn, dim3(grid_for(num_out, 512)), dim3(512), 0, s, w.found, w.tags, w.groups, w.counts, w.blocks, w.B, w.C, g.K,
+                     w.G, pair_capacity, in_maps, out_maps, fin);
 }
 
 void launch_emit(int64_t num_out, const KmapGeom& g, const KmapWorkspace& w, int64_t pair_capacity,
@@ -1665,9 +1680,9 @@ static int kmap_count_impl(const void* table, int64_t n_keys, int64_t capacity, 
   wcn_table_layout(const_cast<void*>(table), n_keys, capacity, &v);
   KmapWorkspace w;
   kmap_layout(workspace, num_out, g.K, &w);
-  const bool together = fill && own_sums(g, num_out);
+  const bool own = fill && leaves_counts(g, num_out), together = own && num_out <= KMAP_OWN_SUMS;
   if (w.G > 0) {
-    launch_probe(v, out_coords, num_out, g, w, s, together);
+    launch_probe(v, out_coords, num_out, g, w, s, together, own && !together);
   } else {
     hipLaunchKernelGGL(kmap_zero_ticket, dim3(1), dim3(1), 0, s, w.ticket);
   }
@@ -1684,6 +1699,7 @@ static int kmap_count_impl(const void* table, int64_t n_keys, int64_t capacity, 
   set_pending(Pending::map, sequence, w.result);
   const KmapFinish fin = {w.result, w.ticket, v.hdr, g.K, box, sequence};
   if (together) launch_starts_emit(num_out, g, w, pair_capacity, in_maps, out_maps, fin, s);
+  else if (own) hipLaunchKernelGGL(kmap_scan_rows, dim3(g.K), dim3(1024), 0, s, w.blocks, (int64_t)w.B, w.row_total, fin);
   else hipLaunchKernelGGL(kmap_scan_rows, dim3(g.K + 1), dim3(1024), 0, s, w.groups, w.G, w.row_total, fin);
   WCN_LAUNCH_CHECK();
   if (box) {
@@ -1691,8 +1707,9 @@ static int kmap_count_impl(const void* table, int64_t n_keys, int64_t capacity, 
   } else if (wcn_read_early_begin(w.result, sizeof(int64_t) * (size_t)(g.K + 3), s) != WCN_OK) {
     return WCN_ERR_LAUNCH;
   }
-  if (fill && !together && num_out > 0 && pair_capacity > 0) {
-    launch_emit(num_out, g, w, pair_capacity, in_maps, out_maps, s);
+  if (fill && !together && num_out > 0 && (own || pair_capacity > 0)) {
+    if (own) launch_starts_emit(num_out, g, w, pair_capacity, in_maps, out_maps, fin, s);
+    else launch_emit(num_out, g, w, pair_capacity, in_maps, out_maps, s);
     WCN_LAUNCH_CHECK();
   }
   return WCN_OK;
