@@ -676,7 +676,7 @@ def main():
     map_bytes = 24 * n + 8 * cap + 16 * n + 8 * K * n + 8 * num_pairs
     achieved = conv_bytes / (conv_kernel_ms * 1e-3) / 1e9
     traffic_bytes, traffic_note = measured_traffic(TRAFFIC_FILE, conv_kernel)
-    map_kernels = ("kmap_pass_fixed<3, 3, 3>" if os.environ.get("WCN_KMAP_PROBE") != "blocks" else "self_probe<1>")
+    map_kernels = ("kmap_pass_fixed<3, 3, 3, false>" if os.environ.get("WCN_KMAP_PROBE") != "blocks" else "self_probe<1>")
     map_traffic_bytes, map_traffic_note = measured_traffic(MAP_TRAFFIC_FILE, map_kernels)
 
     result = {
@@ -730,11 +730,11 @@ def main():
             "algorithmic_bytes": conv_bytes,
             "measured_peaks": measured_peaks(dev),
             # the second half of the metric as a roofline line of its own: all kernels of the map
-            # build together (table: hist, colscan, scatter, bins; map: probe, scan, emit) against
+            # build together (table: sort, bins; map: probe, scan, emit) against
             # the bytes the survey's formula prices for it
             "map_build": {
-                "kernel": "table_hist + table_colscan + table_scatter + table_bins + " + map_kernels
-                          + " + kmap_scan_rows + " + ("kmap_emit<8>" if "kmap_pass" in map_kernels else "self_count + self_emit"),
+                "kernel": "table_sort + table_bins + " + map_kernels
+                          + " + kmap_scan_rows + " + ("kmap_starts_emit<1, true>" if "kmap_pass" in map_kernels else "self_count + self_emit"),
                 "probe_kernel": map_kernels,
                 "bound": "hbm",
                 "achieved": map_bytes / (map_ms * 1e-3) / 1e9,
