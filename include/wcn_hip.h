@@ -659,6 +659,17 @@ int wcn_sparse_depthwise_wgrad_grouped(const void* features, int64_t num_in, con
                                        int32_t weight_dtype, void* workspace, size_t workspace_bytes,
                                        void* stream);
 
+/* That and wcn_column_sums of grad_out (the gradient of a bias: `channels` values of bias_dtype, with a workspace of
+ * wcn_column_sums_workspace_bytes(channels)) in one call, the same results, in two launches less. */
+int wcn_sparse_depthwise_wgrad_grouped_bias(const void* features, int64_t num_in, const void* grad_out,
+                                            int64_t num_out, int32_t channels, int32_t dtype,
+                                            const int32_t* in_maps, const int32_t* out_maps,
+                                            const int64_t* device_offsets, const int32_t* group_start,
+                                            int32_t num_offsets, int32_t identity_offset, void* grad_weight,
+                                            int32_t weight_dtype, void* workspace, size_t workspace_bytes,
+                                            void* grad_bias, int32_t bias_dtype, void* bias_workspace,
+                                            size_t bias_workspace_bytes, void* stream);
+
 /* The convolution of one voxel: out = rows @ weight + bias, (num_rows, c_out) of the rows' type (16-bit), fp32 sums, one
  * rounding.  weight: (c_in, c_out) of the rows' type, as stored; all pointers 16-byte aligned, rows dense.
  * wcn_pointwise_takes: whether the call is one the kernel is made for (WCN_ERR_INVALID_ARGUMENT otherwise). */

@@ -98,6 +98,8 @@ SIGNATURES = {
     "wcn_depthwise_wgrad_grouped_workspace_bytes": (_sz, [_i32, _i32, _i64]),
     "wcn_sparse_depthwise_wgrad_grouped": (ctypes.c_int, [_vp, _i64, _vp, _i64, _i32, _i32, _vp, _vp, _vp, _vp,
                                                           _i32, _i32, _vp, _i32, _vp, _sz, _vp]),
+    "wcn_sparse_depthwise_wgrad_grouped_bias": (ctypes.c_int, [_vp, _i64, _vp, _i64, _i32, _i32, _vp, _vp, _vp, _vp, _i32, _i32,
+                                                               _vp, _i32, _vp, _sz, _vp, _i32, _vp, _sz, _vp]),
     "wcn_pointwise_takes": (_i32, [_i64, _i32, _i32, _i32]),
     "wcn_pointwise_fwd": (ctypes.c_int, [_vp, _i64, _i32, _i32, _vp, _i32, _vp, _vp, _vp]),
     "wcn_column_sums_workspace_bytes": (_sz, [_i32]),

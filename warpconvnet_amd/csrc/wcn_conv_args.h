@@ -91,15 +91,16 @@ int wcn_column_sums_first(const void* rows, int64_t num_rows, int dtype, const W
 int wcn_column_sums_second(const WcnColumnSums& c, hipStream_t stream);
 
 #ifdef __HIPCC__
-// The second pass by 256 threads for 16 channels from c0 on: parts p, p + 16, ... to thread p / 16, eight in flight, their
+// The second pass by a workgroup's first 256 threads for 16 channels from c0 on: parts p, p + 16, ... to thread p / 16, eight in flight, their
 // sixteen sums added in order.
 template <typename OT>
 __device__ __forceinline__ void wcn_column_sums_finish(const WcnColumnSums& s, int c0, OT* out) {
   __shared__ float s_sum[16][16];
   constexpr int AHEAD = 8;
+  const bool there = threadIdx.x < 256;
   const int at = threadIdx.x & 15, stretch = threadIdx.x >> 4, c = c0 + at;
   float sum = 0.f;
-  if (c < s.channels) {
+  if (there && c < s.channels) {
     for (int p = stretch; p < s.parts; p += 16 * AHEAD) {
       float v[AHEAD];
 #pragma unroll
@@ -108,7 +109,7 @@ __device__ __forceinline__ void wcn_column_sums_finish(const WcnColumnSums& s, i
       for (int i = 0; i < AHEAD; ++i) sum += v[i];
     }
   }
-  s_sum[stretch][at] = sum;
+  if (there) s_sum[stretch][at] = sum;
   __syncthreads();
   if (stretch != 0 || c >= s.channels) return;
   for (int p = 1; p < 16; ++p) sum += s_sum[p][at];

@@ -7,6 +7,7 @@
 // over a rows form of the map, a thread per (row, 16 bytes of channels), fp32 sums, one store.
 #include <algorithm>
 
+#include "wcn_conv_args.h"
 #include "wcn_rows.h"
 
 namespace {
@@ -120,6 +121,8 @@ __global__ void __launch_bounds__(256) depthwise_rows(const T* __restrict__ X, i
 // a range follow one another on one XCD: its dY rows (at most 8192, 1 MB of 64 fp16 channels) then come
 // out of that XCD's L2 for all offsets but the first.  Without them a range is a share of the offset's pairs.
 // Four pairs in flight per thread: 2.1 M pairs of 64 fp16 channels 117 + 57 (reduction) -> 88 + 10 us.
+// The column sums of dY (a bias's gradient) ride on this launch and the reduction's: over 500 k rows of 64 fp16 channels 85.0 + 12.7 and
+// 10.4 + 4.1 us one after the other, 90.7 and 10.7 together; a layer and a pooling forward and backward 531 -> 505 to 514 us.
 struct WgradRanges {
   const int32_t* gs;  // (K, G + 1) or null
   int64_t G;
@@ -138,9 +141,13 @@ __global__ void __launch_bounds__(256) depthwise_wgrad(const T* __restrict__ X, 
                                                        const int32_t* __restrict__ out_maps,
                                                        const int64_t* __restrict__ offsets, WgradRanges q, int K,
                                                        int identity, int64_t identity_rows,
-                                                       float* __restrict__ partial) {
+                                                       float* __restrict__ partial, int grid, ColumnPart columns) {
   constexpr int N = Piece<T>::N, U = 4;
   __shared__ float s_sum[256][N + 1];
+  if ((int)blockIdx.x >= grid) {  // the column sums of dY: workgroups of their own behind the others
+    column_part<T, VEC>(columns, (int)blockIdx.x - grid, &s_sum[0][0]);
+    return;
+  }
   // blockIdx % 8 is the XCD: range = 8 * (b / 8 / K) + b % 8
   const int places = wgrad_places(K, identity);
   const int t = blockIdx.x >> 3, place = t % places, range = (t / places) * 8 + (blockIdx.x & 7);
@@ -225,11 +232,20 @@ __global__ void __launch_bounds__(256) depthwise_wgrad(const T* __restrict__ X, 
   }
 }
 
-// dW[k][c] = the ranges' partial rows added up: 16 stretches side by side, then those in order.
+// dW[k][c] = the ranges' partial rows added up: 16 stretches side by side, then those in order.  From blockIdx.x = K on: the
+// second pass of the column sums, 16 channels each.
 template <typename WT>
 __global__ void __launch_bounds__(1024) depthwise_wgrad_reduce(const float* __restrict__ partial, int ranges,
-                                                               int K, int identity, int channels, WT* __restrict__ dW) {
+                                                               int K, int identity, int channels, WT* __restrict__ dW,
+                                                               WcnColumnSums columns) {
   __shared__ float s_sum[16][64];
+  if ((int)blockIdx.x >= K) {
+    const int c0 = (int)blockIdx.y * 64 + ((int)blockIdx.x - K) * 16;
+    if (columns.out_dtype == WCN_DTYPE_F32) wcn_column_sums_finish<float>(columns, c0, (float*)columns.out);
+    else if (columns.out_dtype == WCN_DTYPE_F16) wcn_column_sums_finish<_Float16>(columns, c0, (_Float16*)columns.out);
+    else wcn_column_sums_finish<__bf16>(columns, c0, (__bf16*)columns.out);
+    return;
+  }
   const int k = blockIdx.x, lane = threadIdx.x & 63, part = threadIdx.x >> 6;
   const int c = blockIdx.y * 64 + lane;
   float sum = 0.f;
@@ -340,19 +356,22 @@ size_t wcn_depthwise_wgrad_grouped_workspace_bytes(int32_t num_offsets, int32_t 
 static int depthwise_wgrad_launch(const void* features, int64_t num_in, const void* grad_out, int64_t num_out,
                                   int32_t channels, int32_t dtype, const int32_t* in_maps, const int32_t* out_maps,
                                   const int64_t* offsets, const WgradRanges& q, int32_t K, int32_t identity,
-                                  void* grad_weight, int32_t weight_dtype, float* partial, hipStream_t s) {
+                                  void* grad_weight, int32_t weight_dtype, float* partial, hipStream_t s,
+                                  const WcnColumnSums& columns = WcnColumnSums{}) {
   const int64_t identity_rows = identity >= 0 ? std::min(num_in, num_out) : 0;
   const bool vec = rows_are_vectors(features, channels, dtype) && rows_are_vectors(grad_out, channels, dtype);
   const int ranges = num_in == 0 || num_out == 0 ? 0 : q.ranges;  // 0: the sums are zeros
   const unsigned grid = (unsigned)((ranges + 7) / 8 * 8) * (unsigned)wgrad_places(K, identity);
+  const unsigned parts = (unsigned)columns.parts;
+  const ColumnPart part = column_part_of(grad_out, num_out, dtype, columns);
   with_types(dtype, weight_dtype, [&](auto a, auto b) {
     using T = decltype(a);
     using WT = decltype(b);
-    if (ranges > 0)
-      hipLaunchKernelGGL((vec ? depthwise_wgrad<T, true> : depthwise_wgrad<T, false>), dim3(grid), dim3(256), 0, s, (const T*)features, num_in, (const T*)grad_out,
-                       num_out, channels, in_maps, out_maps, offsets, q, K, identity, identity_rows, partial);
-    hipLaunchKernelGGL(depthwise_wgrad_reduce<WT>, dim3((unsigned)K, (unsigned)((channels + 63) / 64)), dim3(1024), 0, s,
-                       (const float*)partial, ranges, K, identity, channels, (WT*)grad_weight);
+    if (grid + parts > 0)
+      hipLaunchKernelGGL((vec ? depthwise_wgrad<T, true> : depthwise_wgrad<T, false>), dim3(grid + parts), dim3(256), 0, s, (const T*)features, num_in, (const T*)grad_out,
+                       num_out, channels, in_maps, out_maps, offsets, q, K, identity, identity_rows, partial, (int)grid, part);
+    hipLaunchKernelGGL(depthwise_wgrad_reduce<WT>, dim3((unsigned)K + (columns.channels > 0 ? 4u : 0u), (unsigned)((channels + 63) / 64)), dim3(1024), 0, s,
+                       (const float*)partial, ranges, K, identity, channels, (WT*)grad_weight, columns);
   });
   WCN_LAUNCH_CHECK();
   return WCN_OK;
@@ -387,11 +406,11 @@ int wcn_sparse_depthwise_wgrad(const void* features, int64_t num_in, const void*
                                 num_offsets, identity_offset, grad_weight, weight_dtype, partial, s);
 }
 
-int wcn_sparse_depthwise_wgrad_grouped(const void* features, int64_t num_in, const void* grad_out, int64_t num_out,
-                                       int32_t channels, int32_t dtype, const int32_t* in_maps, const int32_t* out_maps,
-                                       const int64_t* device_offsets, const int32_t* group_start, int32_t num_offsets,
-                                       int32_t identity_offset, void* grad_weight, int32_t weight_dtype,
-                                       void* workspace, size_t workspace_bytes, void* stream) {
+static int wgrad_grouped(const void* features, int64_t num_in, const void* grad_out, int64_t num_out,
+                         int32_t channels, int32_t dtype, const int32_t* in_maps, const int32_t* out_maps,
+                         const int64_t* device_offsets, const int32_t* group_start, int32_t num_offsets,
+                         int32_t identity_offset, void* grad_weight, int32_t weight_dtype,
+                         void* workspace, size_t workspace_bytes, const WcnColumnSums& columns, void* stream) {
   if (!types_ok(dtype, weight_dtype) || channels < 1 || num_in < 0 || num_out < 0 || !grad_weight || !workspace ||
       !device_offsets || !group_start || num_offsets < 1 || num_offsets > WCN_MAX_OFFSETS || identity_offset >= num_offsets ||
       (num_in > 0 && !features) || (num_out > 0 && !grad_out) || num_out > INT32_MAX)
@@ -402,7 +421,31 @@ int wcn_sparse_depthwise_wgrad_grouped(const void* features, int64_t num_in, con
                       wgrad_rows_per_range(num_out, num_offsets) / 64};
   return depthwise_wgrad_launch(features, num_in, grad_out, num_out, channels, dtype, in_maps, out_maps, device_offsets, q,
                                 num_offsets, identity_offset, grad_weight, weight_dtype, (float*)workspace,
-                                (hipStream_t)stream);
+                                (hipStream_t)stream, columns);
+}
+
+int wcn_sparse_depthwise_wgrad_grouped(const void* features, int64_t num_in, const void* grad_out, int64_t num_out,
+                                       int32_t channels, int32_t dtype, const int32_t* in_maps, const int32_t* out_maps,
+                                       const int64_t* device_offsets, const int32_t* group_start, int32_t num_offsets,
+                                       int32_t identity_offset, void* grad_weight, int32_t weight_dtype,
+                                       void* workspace, size_t workspace_bytes, void* stream) {
+  return wgrad_grouped(features, num_in, grad_out, num_out, channels, dtype, in_maps, out_maps, device_offsets, group_start,
+                       num_offsets, identity_offset, grad_weight, weight_dtype, workspace, workspace_bytes, WcnColumnSums{}, stream);
+}
+
+int wcn_sparse_depthwise_wgrad_grouped_bias(const void* features, int64_t num_in, const void* grad_out, int64_t num_out,
+                                            int32_t channels, int32_t dtype, const int32_t* in_maps, const int32_t* out_maps,
+                                            const int64_t* device_offsets, const int32_t* group_start, int32_t num_offsets,
+                                            int32_t identity_offset, void* grad_weight, int32_t weight_dtype,
+                                            void* workspace, size_t workspace_bytes, void* grad_bias, int32_t bias_dtype,
+                                            void* bias_workspace, size_t bias_workspace_bytes, void* stream) {
+  if (!types_ok(dtype, weight_dtype) || channels < 1 || num_out < 0 || bias_dtype < 0 || bias_dtype > 2 || !grad_bias || !bias_workspace)
+    return WCN_ERR_INVALID_ARGUMENT;
+  if (bias_workspace_bytes < wcn_column_sums_workspace_bytes(channels)) return WCN_ERR_WORKSPACE;
+  WcnColumnSums columns = {(float*)bias_workspace, 0, channels, grad_bias, bias_dtype};
+  wcn_column_sums_parts(num_out, dtype, &columns);
+  return wgrad_grouped(features, num_in, grad_out, num_out, channels, dtype, in_maps, out_maps, device_offsets, group_start,
+                       num_offsets, identity_offset, grad_weight, weight_dtype, workspace, workspace_bytes, columns, stream);
 }
 
 }  // extern "C"

@@ -1124,7 +1124,8 @@ Tensor depthwise_out(const Tensor& features, const Tensor& weight, const Tensor&
 }
 
 std::pair<Tensor, Tensor> depthwise_grads(const Tensor& grad_output, const Tensor& in_features, const Tensor& weight,
-                                          const RowsMap& m, at::ScalarType dtype, bool need_x, bool need_w) {
+                                          const RowsMap& m, at::ScalarType dtype, bool need_x, bool need_w,
+                                          Tensor* grad_bias = nullptr) {
   const Tensor x = in_features.to(dtype).contiguous(), gy = grad_output.to(dtype).contiguous();
   const Tensor w = depthwise_weight(weight, dtype);
   const int64_t n_in = x.size(0), n_out = gy.size(0);
@@ -1144,7 +1145,16 @@ std::pair<Tensor, Tensor> depthwise_grads(const Tensor& grad_output, const Tenso
     void* stream = stream_of(x);
     if (m.groups) {
       const Tensor ws = bytes_on(wcn_depthwise_wgrad_grouped_workspace_bytes(K, c, n_out), x);
-      check(wcn_sparse_depthwise_wgrad_grouped(x.const_data_ptr(), n_in, gy.const_data_ptr(), n_out, c, code, in_maps, out_maps,
+      if (grad_bias) {
+        const Tensor sums = bytes_on(wcn_column_sums_workspace_bytes(c), x);
+        check(wcn_sparse_depthwise_wgrad_grouped_bias(x.const_data_ptr(), n_in, gy.const_data_ptr(), n_out, c, code, in_maps, out_maps,
+                                                      m.device_offsets.const_data_ptr<int64_t>(), m.groups, K, iden,
+                                                      grad_w.mutable_data_ptr(), dtype_code(w.scalar_type()),
+                                                      ws.mutable_data_ptr(), static_cast<size_t>(ws.numel()),
+                                                      grad_bias->mutable_data_ptr(), dtype_code(grad_bias->scalar_type()),
+                                                      sums.mutable_data_ptr(), static_cast<size_t>(sums.numel()), stream),
+              "wcn_sparse_depthwise_wgrad_grouped_bias");
+      } else check(wcn_sparse_depthwise_wgrad_grouped(x.const_data_ptr(), n_in, gy.const_data_ptr(), n_out, c, code, in_maps, out_maps,
                                                m.device_offsets.const_data_ptr<int64_t>(), m.groups, K, iden,
                                                grad_w.mutable_data_ptr(), dtype_code(w.scalar_type()), ws.mutable_data_ptr(),
                                                static_cast<size_t>(ws.numel()), stream),
@@ -1199,10 +1209,13 @@ struct DepthwiseBackward : public torch::autograd::Node {
     TORCH_CHECK(map_ != nullptr, "Trying to backward through the graph a second time (the map was given back after the first)");
     const Tensor x = x_.unpack(shared_from_this()), w = w_.unpack(shared_from_this());
     at::NoGradGuard no_grad;
-    auto r = depthwise_grads(grads[0], x, w, *map_, dtype_, task_should_compute_output(0), task_should_compute_output(1));
+    const bool need_w = task_should_compute_output(1), need_b = has_bias_ && task_should_compute_output(2);
+    const bool joined = need_b && need_w && map_->groups && grads[0].scalar_type() == dtype_ && dtype_code(bias_dtype_) >= 0;
+    if (joined) out[2] = at::empty({grads[0].size(1)}, grads[0].options().dtype(bias_dtype_));
+    auto r = depthwise_grads(grads[0], x, w, *map_, dtype_, task_should_compute_output(0), need_w, joined ? &out[2] : nullptr);
     out[0] = r.first;
     out[1] = r.second;
-    if (has_bias_ && task_should_compute_output(2)) out[2] = column_sums(grads[0], bias_dtype_);
+    if (need_b && !joined) out[2] = column_sums(grads[0], bias_dtype_);
     return out;
   }
   void release_variables() override {
