@@ -165,6 +165,21 @@ int wcn_kmap_count_fill(const void* table, int64_t n_keys, int64_t capacity, con
                         const int32_t* host_centre_or_null, void* workspace, int64_t pair_capacity, int32_t* in_maps,
                         int32_t* out_maps, void* stream);
 
+/* wcn_kmap_count_fill and the wcn_kmap_fill that may follow with the workspace in two pieces: `head`, the first
+ * wcn_kmap_head_bytes of it (offsets, status and group starts: what wcn_kmap_read_result and wcn_kmap_group_start are given, and what
+ * stays with a map), and `parked`, the rest of its wcn_kmap_workspace_bytes, which nothing reads behind the last of these calls.
+ * Both 256-byte aligned. */
+size_t wcn_kmap_head_bytes(int64_t num_out, int32_t num_offsets);
+
+int wcn_kmap_count_fill_apart(const void* table, int64_t n_keys, int64_t capacity, const int32_t* out_coords, int64_t num_out,
+                              const int32_t host_kernel_size[3], const int32_t host_stride[3],
+                              const int32_t* host_dilation_or_null, const int32_t* host_centre_or_null, void* head, void* parked,
+                              int64_t pair_capacity, int32_t* in_maps, int32_t* out_maps, void* stream);
+
+int wcn_kmap_fill_apart(const void* table, int64_t n_keys, int64_t capacity, const int32_t* out_coords, int64_t num_out,
+                        const int32_t host_kernel_size[3], const int32_t host_stride[3], const void* head, const void* parked,
+                        int64_t pair_capacity, int32_t* in_maps, int32_t* out_maps, void* stream);
+
 /* The map of a coordinate set onto itself (the stride-1 convolution: out_coords are the table's own
  * keys, in the same rows): the same results as wcn_kmap_count / wcn_kmap_fill with out_coords =
  * keys and stride 1, from a probe pass that walks the keys in the table's block order, where

@@ -213,3 +213,34 @@ def test_one_call_leaves_what_two_leave(n, kernel, stride, dilation):
         assert short[0] == want[0] and torch.equal(short[2], want[2]) and bool((short[3] == -7).all()) and bool((short[4] == -7).all())
         check(L.wcn_kmap_fill(ptr(table), n, slots, ptr(rows), n, k3, st, ptr(short[6]), K * n, ptr(short[3]), ptr(short[4]), s), "fill")
         assert torch.equal(short[3], want[3]) and torch.equal(short[4], want[4])
+
+
+@pytest.mark.parametrize("kernel,stride,dilation", [(3, 1, 1), (2, 2, 1), (5, 1, 1), (3, 1, 2), ((1, 3, 2), 1, 1)])
+@pytest.mark.parametrize("n", [1, 65, 30_011, (1 << 18) + 1])
+@pytest.mark.parametrize("short", [False, True])
+def test_maps_whose_head_lies_apart(monkeypatch, n, kernel, stride, dilation, short):
+    """A workspace in two pieces (that of maps over a size) against one in one piece: lists, offsets and group starts, also where the
+    lists were taken for shorter than they are and are emitted again."""
+    from warpconvnet_amd.geometry.coords.search import torch_discrete
+    rng = np.random.default_rng(n)
+    side = int(np.ceil(np.sqrt(n / 0.6)))
+    cells = rng.permutation(side * side)[:n]
+    rows = torch.as_tensor(np.stack([cells * 0, cells // side, cells % side, cells % 5 // 3], axis=1).astype(np.int32), device=DEV)
+    ks = (kernel,) * 3 if isinstance(kernel, int) else kernel
+
+    def build(keep):
+        monkeypatch.setattr(torch_discrete, "_KEEP_WORKSPACE_BYTES", keep)
+        monkeypatch.setattr(torch_discrete, "_PAIRS_PER_ROW", torch_discrete._PAIRS_PER_ROW.__class__())
+        if short:
+            octave = (tuple(ks), (stride,) * 3, -n.bit_length())
+            torch_discrete._PAIRS_PER_ROW[octave] = 0.01
+        args = dict(kernel_dilation=(dilation,) * 3, method="offset") if dilation != 1 else {}
+        km = torch_discrete.generate_kernel_map(rows, rows, (stride,) * 3, ks, **args)
+        torch.cuda.synchronize()
+        return km
+
+    want, got = build(1 << 40), build(0)
+    assert torch.equal(got.in_maps, want.in_maps) and torch.equal(got.out_maps, want.out_maps)
+    assert torch.equal(got.offsets, want.offsets) and torch.equal(got._device_offsets, want._device_offsets)
+    starts = 4 * len(want) * ((n + 63) // 64 + 1)
+    assert torch.equal(got._group_start[0][:starts], want._group_start[0][:starts])

@@ -242,15 +242,26 @@ py::tuple kernel_map(const py::object& table, const Tensor& out4, const Int3& ks
   const int32_t K = ks[0] * ks[1] * ks[2];
   const int32_t* rows = out4.const_data_ptr<int32_t>();
   void* stream = stream_of(out4);
-  Tensor ws = bytes_on(wcn_kmap_workspace_bytes(M, K), out4);
+  // What stays with the map is the workspace's head: its K + 1 offsets and the group starts.  Up to keep_workspace_bytes the
+  // workspace itself is kept; beyond, the head is an allocation of its own and the rest is given back.  (Copied out of the
+  // workspace it was a copy and its launch between the map and the layer: 5x5x5 16 -> 16 over 1 M rows 435 us a call, 429 so.)
+  const size_t ws_bytes = wcn_kmap_workspace_bytes(M, K), head_bytes = wcn_kmap_head_bytes(M, K);
+  Tensor ws, parked;
+  // a set mapped onto itself can also be probed block by block (opt-in; same results, a little slower)
+  const char* probe = std::getenv("WCN_KMAP_PROBE");
+  const bool by_blocks = probe != nullptr && std::strcmp(probe, "blocks") == 0, large = static_cast<int64_t>(ws_bytes) > keep_workspace_bytes;
+  if (large && !by_blocks) {
+    ws = bytes_on(head_bytes, out4);
+    parked = bytes_on(ws_bytes - head_bytes, out4);
+  } else {
+    ws = bytes_on(ws_bytes, out4);
+  }
   void* w = ws.mutable_data_ptr();
   Tensor offsets = at::empty({K + 1}, at::kLong);
   int64_t* host_offsets = offsets.mutable_data_ptr<int64_t>();
   const int64_t assumed =
       std::min<int64_t>(K * M, std::max<int64_t>(static_cast<int64_t>(1.25 * per_row * M) + 4096, int64_t{1} << 16));
   Tensor in_buf = at::empty({assumed}, out4.options()), out_buf = at::empty({assumed}, out4.options());
-  // a set mapped onto itself can also be probed block by block (opt-in; same results, a little slower)
-  const char* probe = std::getenv("WCN_KMAP_PROBE");
   Tensor kept;
   std::shared_ptr<MadeOn> made;  // where work on the lists was enqueued behind the wait
   int64_t begin = 0;
@@ -258,30 +269,34 @@ py::tuple kernel_map(const py::object& table, const Tensor& out4, const Int3& ks
     TableRef t(table);
     const int64_t n = t.keys.size(0);
     const void* raw = t.raw.const_data_ptr();
-    const bool blocks = probe != nullptr && std::strcmp(probe, "blocks") == 0 && !dilation && st[0] == 1 && st[1] == 1 &&
+    const bool blocks = by_blocks && !dilation && st[0] == 1 && st[1] == 1 &&
                         st[2] == 1 && rows == t.keys.const_data_ptr<int32_t>() && M == n &&
                         wcn_kmap_self_supported(ks.data(), M);
     auto fill = [&](int64_t capacity, const Tensor& ins, const Tensor& outs) {
       int32_t *pi = ins.mutable_data_ptr<int32_t>(), *po = outs.mutable_data_ptr<int32_t>();
       check(blocks ? wcn_kmap_fill_self(M, ks.data(), w, capacity, pi, po, stream)
+            : parked.defined() ? wcn_kmap_fill_apart(raw, n, t.slots, rows, M, ks.data(), st.data(), w, parked.const_data_ptr(),
+                                                     capacity, pi, po, stream)
                    : wcn_kmap_fill(raw, n, t.slots, rows, M, ks.data(), st.data(), w, capacity, pi, po, stream),
             "wcn_kmap_fill");
     };
     if (blocks) {
       check(wcn_kmap_count_self(raw, n, t.slots, ks.data(), w, stream), "wcn_kmap_count_self");
       fill(assumed, in_buf, out_buf);
+    } else if (parked.defined()) {
+      check(wcn_kmap_count_fill_apart(raw, n, t.slots, rows, M, ks.data(), st.data(), dilation ? dilation->data() : nullptr,
+                                      dilation ? centre->data() : nullptr, w, parked.mutable_data_ptr(), assumed,
+                                      in_buf.mutable_data_ptr<int32_t>(), out_buf.mutable_data_ptr<int32_t>(), stream),
+            "wcn_kmap_count_fill_apart");
     } else {
       check(wcn_kmap_count_fill(raw, n, t.slots, rows, M, ks.data(), st.data(), dilation ? dilation->data() : nullptr,
                                 dilation ? centre->data() : nullptr, w, assumed, in_buf.mutable_data_ptr<int32_t>(),
                                 out_buf.mutable_data_ptr<int32_t>(), stream),
             "wcn_kmap_count_fill");
     }
-    // What stays with the map is the workspace's head: its K + 1 offsets and the group starts.  Up to
-    // keep_workspace_bytes the workspace itself is kept; beyond, the head is copied, here, so that
-    // nothing stands between the wait below and what the caller launches next.
     begin = reinterpret_cast<const char*>(wcn_kmap_group_start(w, M, K)) - static_cast<const char*>(w);
     kept = ws.narrow(0, 0, begin + 4 * int64_t{K} * ((M + 63) / 64 + 1));
-    if (ws.numel() > keep_workspace_bytes) kept = kept.clone();
+    if (large && !parked.defined()) kept = kept.clone();
     // what a layer needs of the map is on its way: with it behind, the GPU has work while the host takes the offsets in
     if (ahead) ahead->launch(in_buf, out_buf, static_cast<int64_t>(per_row * M), w, wcn_kmap_group_start(w, M, K), K, M);
     int status;

@@ -52,7 +52,8 @@ struct KmapWorkspace {  // host-computed addresses inside a kmap workspace
 // 5.4 us against 6.3 together.)  Beyond, the counts are scanned first: 3x3x3 over 265,000 rows 37.6 35.6, 1 M 87.6 81.6.
 constexpr int64_t KMAP_OWN_SUMS = 1 << 18;
 
-inline size_t kmap_layout(void* base, int64_t num_out, int32_t K, KmapWorkspace* w) {
+// parked: where everything behind the head (result to groups) lies, if apart from it.  head_bytes: what the head takes.
+inline size_t kmap_layout(void* base, int64_t num_out, int32_t K, KmapWorkspace* w, void* parked = nullptr, size_t* head_bytes = nullptr) {
   char* p = (char*)base;
   size_t off = 0;
   const int64_t G = (num_out + 63) / 64;
@@ -64,6 +65,8 @@ inline size_t kmap_layout(void* base, int64_t num_out, int32_t K, KmapWorkspace*
   off += 256;
   if (w) w->groups = (int32_t*)(p + off);
   off += wcn_align256(sizeof(int32_t) * (size_t)(K + 1) * (size_t)(G + 1));
+  if (head_bytes) *head_bytes = off;
+  if (parked) p = (char*)parked - off;
   if (w) w->found = (int32_t*)(p + off);
   off += wcn_align256(sizeof(int32_t) * (size_t)K * (size_t)G * 64);
   static_assert(WCN_MAX_OFFSETS <= 1024, "offset and lane share 16 bits");
@@ -1668,7 +1671,8 @@ static int kmap_count_impl(const void* table, int64_t n_keys, int64_t capacity, 
                            int64_t num_out, const int32_t host_kernel_size[3],
                            const int32_t host_stride[3], const int32_t* host_dilation,
                            const int32_t* host_centre, void* workspace, void* stream, bool fill = false,
-                           int64_t pair_capacity = 0, int32_t* in_maps = nullptr, int32_t* out_maps = nullptr) {
+                           int64_t pair_capacity = 0, int32_t* in_maps = nullptr, int32_t* out_maps = nullptr,
+                           void* parked = nullptr) {
   KmapGeom g;
   if (!make_geom(host_kernel_size, host_stride, host_dilation, host_centre, &g)) return WCN_ERR_INVALID_ARGUMENT;
   if (!table_args_ok(table, n_keys, capacity) || !workspace || num_out < 0 ||
@@ -1679,7 +1683,7 @@ static int kmap_count_impl(const void* table, int64_t n_keys, int64_t capacity, 
   WcnTableView v;
   wcn_table_layout(const_cast<void*>(table), n_keys, capacity, &v);
   KmapWorkspace w;
-  kmap_layout(workspace, num_out, g.K, &w);
+  kmap_layout(workspace, num_out, g.K, &w, parked);
   const bool own = fill && leaves_counts(g, num_out), together = own && num_out <= KMAP_OWN_SUMS;
   if (w.G > 0) {
     launch_probe(v, out_coords, num_out, g, w, s, together, own && !together);
@@ -1722,6 +1726,22 @@ int wcn_kmap_count_fill(const void* table, int64_t n_keys, int64_t capacity, con
   if (!host_dilation_or_null != !host_centre_or_null) return WCN_ERR_INVALID_ARGUMENT;
   return kmap_count_impl(table, n_keys, capacity, out_coords, num_out, host_kernel_size, host_stride, host_dilation_or_null,
                          host_centre_or_null, workspace, stream, true, pair_capacity, in_maps, out_maps);
+}
+
+size_t wcn_kmap_head_bytes(int64_t num_out, int32_t num_offsets) {
+  if (num_out < 0 || num_offsets < 1 || num_offsets > WCN_MAX_OFFSETS) return 0;
+  size_t head = 0;
+  kmap_layout(nullptr, num_out, num_offsets, nullptr, nullptr, &head);
+  return head;
+}
+
+int wcn_kmap_count_fill_apart(const void* table, int64_t n_keys, int64_t capacity, const int32_t* out_coords, int64_t num_out,
+                              const int32_t host_kernel_size[3], const int32_t host_stride[3],
+                              const int32_t* host_dilation_or_null, const int32_t* host_centre_or_null, void* head, void* parked,
+                              int64_t pair_capacity, int32_t* in_maps, int32_t* out_maps, void* stream) {
+  if (!host_dilation_or_null != !host_centre_or_null || !parked) return WCN_ERR_INVALID_ARGUMENT;
+  return kmap_count_impl(table, n_keys, capacity, out_coords, num_out, host_kernel_size, host_stride, host_dilation_or_null,
+                         host_centre_or_null, head, stream, true, pair_capacity, in_maps, out_maps, parked);
 }
 
 int wcn_kmap_count(const void* table, int64_t n_keys, int64_t capacity, const int32_t* out_coords,
@@ -1837,10 +1857,10 @@ int wcn_kmap_read_result(const void* workspace, int64_t num_out, int32_t num_off
   return WCN_OK;
 }
 
-int wcn_kmap_fill(const void* table, int64_t n_keys, int64_t capacity, const int32_t* out_coords,
-                  int64_t num_out, const int32_t host_kernel_size[3], const int32_t host_stride[3],
-                  const void* workspace, int64_t pair_capacity, int32_t* in_maps, int32_t* out_maps,
-                  void* stream) {
+static int kmap_fill_impl(const void* table, int64_t n_keys, int64_t capacity, const int32_t* out_coords,
+                          int64_t num_out, const int32_t host_kernel_size[3], const int32_t host_stride[3],
+                          const void* workspace, const void* parked, int64_t pair_capacity, int32_t* in_maps, int32_t* out_maps,
+                          void* stream) {
   KmapGeom g;
   if (!make_geom(host_kernel_size, host_stride, nullptr, nullptr, &g)) return WCN_ERR_INVALID_ARGUMENT;
   if (!table_args_ok(table, n_keys, capacity) || !workspace || num_out < 0 ||
@@ -1851,10 +1871,27 @@ int wcn_kmap_fill(const void* table, int64_t n_keys, int64_t capacity, const int
   WcnTableView v;
   wcn_table_layout(const_cast<void*>(table), n_keys, capacity, &v);
   KmapWorkspace w;
-  kmap_layout(const_cast<void*>(workspace), num_out, g.K, &w);
+  kmap_layout(const_cast<void*>(workspace), num_out, g.K, &w, const_cast<void*>(parked));
   launch_emit(num_out, g, w, pair_capacity, in_maps, out_maps, (hipStream_t)stream);
   WCN_LAUNCH_CHECK();
   return WCN_OK;
+}
+
+int wcn_kmap_fill(const void* table, int64_t n_keys, int64_t capacity, const int32_t* out_coords,
+                  int64_t num_out, const int32_t host_kernel_size[3], const int32_t host_stride[3],
+                  const void* workspace, int64_t pair_capacity, int32_t* in_maps, int32_t* out_maps,
+                  void* stream) {
+  return kmap_fill_impl(table, n_keys, capacity, out_coords, num_out, host_kernel_size, host_stride, workspace, nullptr,
+                        pair_capacity, in_maps, out_maps, stream);
+}
+
+int wcn_kmap_fill_apart(const void* table, int64_t n_keys, int64_t capacity, const int32_t* out_coords,
+                        int64_t num_out, const int32_t host_kernel_size[3], const int32_t host_stride[3],
+                        const void* head, const void* parked, int64_t pair_capacity, int32_t* in_maps, int32_t* out_maps,
+                        void* stream) {
+  if (!parked) return WCN_ERR_INVALID_ARGUMENT;
+  return kmap_fill_impl(table, n_keys, capacity, out_coords, num_out, host_kernel_size, host_stride, head, parked,
+                        pair_capacity, in_maps, out_maps, stream);
 }
 
 const int32_t* wcn_kmap_group_start(const void* workspace, int64_t num_out, int32_t num_offsets) {

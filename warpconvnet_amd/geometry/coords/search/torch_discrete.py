@@ -80,9 +80,8 @@ def _kernel_map_from_table(table: TorchHashTable, out_coords: Tensor, kernel_siz
     down).  By-product the contraction reuses: the per-64-row group starts of every offset, (K, G + 1)
     int32, behind the map's K + 1 offsets as int64 at the head of the builder's workspace; that head
     (about K * M / 16 bytes) is what stays with the map.  The probe results behind it (a row's number and a
-    tag for each) are K * M * 6 bytes: above _KEEP_WORKSPACE_BYTES (3x3x3: 1.6 M rows) the head is copied and
-    the workspace goes back to the allocator, below, the map keeps the workspace as it is and the step has no
-    copy in it."""
+    tag for each) are K * M * 6 bytes: above _KEEP_WORKSPACE_BYTES (3x3x3: 1.6 M rows) the head is an allocation
+    of its own and they go back to the allocator, below, the map keeps the workspace as it is."""
     out4 = _four_columns(out_coords)
     if ahead is not None:
         ahead.identity = identity_map_index
