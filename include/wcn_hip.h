@@ -134,8 +134,10 @@ int wcn_kmap_count_dilated(const void* table, int64_t n_keys, int64_t capacity,
                            const int32_t host_dilation[3], const int32_t host_centre[3],
                            void* workspace, void* stream);
 
-/* Waits for the stream.  host_offsets[K+1] receives the exclusive prefix sums of the per-offset
- * pair counts (host_offsets[K] = L).  Returns the table status or WCN_ERR_TOO_MANY_PAIRS. */
+/* Waits for the counts.  host_offsets[K+1] receives the exclusive prefix sums of the per-offset
+ * pair counts (host_offsets[K] = L).  Returns the table status or WCN_ERR_TOO_MANY_PAIRS.  The kernels that write the lists and
+ * the group starts may run on after it: work on the same stream is behind them, work on another has to wait for them (see
+ * wcn_kmap_take_event). */
 int wcn_kmap_read_result(const void* workspace, int64_t num_out, int32_t num_offsets,
                          int64_t* host_offsets, void* stream);
 
@@ -164,6 +166,13 @@ int wcn_kmap_count_fill(const void* table, int64_t n_keys, int64_t capacity, con
                         const int32_t host_kernel_size[3], const int32_t host_stride[3], const int32_t* host_dilation_or_null,
                         const int32_t* host_centre_or_null, void* workspace, int64_t pair_capacity, int32_t* in_maps,
                         int32_t* out_maps, void* stream);
+
+/* An event (hipEvent_t, without timing) behind the kernels of this host thread's last wcn_kmap_count_fill(_apart), once its result
+ * has been read from the same workspace (head): what work on another stream than the builder's has to wait for before it reads
+ * lists or group starts.  The caller's to destroy; asked for at most once.  Null where there is none (the result came the slow way,
+ * another call on this thread since): then an event recorded on the builder's stream now serves, as it does behind a wcn_kmap_fill
+ * that followed. */
+void* wcn_kmap_take_event(const void* workspace);
 
 /* wcn_kmap_count_fill and the wcn_kmap_fill that may follow with the workspace in two pieces: `head`, the first
  * wcn_kmap_head_bytes of it (offsets, status and group starts: what wcn_kmap_read_result and wcn_kmap_group_start are given, and what

@@ -183,6 +183,36 @@ def test_a_map_given_back_while_another_stream_reads_it():
     assert len(taken) == 6 and torch.equal(got, want)
 
 
+@pytest.mark.parametrize("rows,ksize,width,assumed", [(1_000_000, 5, 16, None),   # scan, then lists and group starts
+                                                      (200_000, 3, 16, None),     # all three in one launch
+                                                      (200_000, 3, 16, 0.1),      # lists filled behind the host's wait
+                                                      (1_000_000, 3, 16, 27.0)])  # copied there: far fewer than assumed
+def test_a_map_just_made_serves_layers_on_other_streams(rows, ksize, width, assumed):
+    """The host knows the counts of a map before its lists and group starts are complete: a layer on an idle stream, at once
+    and without a synchronisation, waits for them."""
+    from warpconvnet_amd._lib import host
+    from warpconvnet_amd.geometry.coords.search import torch_discrete
+    from warpconvnet_amd.nn.functional.sparse_conv import sparse_conv_forward
+    c = _surface(rows, 19)
+    n = len(c)
+    x = normal_features(n, width, seed=1, dtype=torch.float16).to(DEV)
+    w = kaiming_weight(ksize ** 3, width, width, seed=2, dtype=torch.float16).to(DEV)
+    want = sparse_conv_forward(x, w, _map(c, ksize=ksize), n)
+    a, b = torch.cuda.Stream(), torch.cuda.Stream()
+    for _ in range(4):
+        if assumed is not None:
+            torch_discrete._PAIRS_PER_ROW.update({k: assumed for k in torch_discrete._PAIRS_PER_ROW})
+        torch.cuda.synchronize()
+        with torch.cuda.stream(a):
+            km = _map(c, ksize=ksize)
+        with torch.cuda.stream(b):
+            got = sparse_conv_forward(x, w, km, n)
+        assert isinstance(km._made, host().MadeOn)
+        torch.cuda.synchronize()
+        assert torch.equal(got, want)
+        del km
+
+
 def test_copies_and_files_of_voxels_with_maps():
     """copy.deepcopy and pickle of a tensor whose cache holds maps with everything the layers left on them: the copy
     makes its own and gives the same results after the original is gone."""

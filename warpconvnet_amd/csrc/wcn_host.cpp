@@ -70,9 +70,9 @@ Tensor bytes_on(size_t n, const Tensor& like) {
  * kernels run when the graph is replayed, not now. */
 struct MadeOn {
   void* stream;
-  hipEvent_t event = nullptr;  // null where the host has waited for the kernels
-  explicit MadeOn(void* s, bool complete = false) : stream(s) {
-    if (complete) return;
+  hipEvent_t event = nullptr;
+  MadeOn(void* s, void* recorded) : stream(s), event(static_cast<hipEvent_t>(recorded)) {}
+  explicit MadeOn(void* s) : stream(s) {
     if (hipEventCreateWithFlags(&event, hipEventDisableTiming) != hipSuccess ||
         hipEventRecord(event, static_cast<hipStream_t>(s)) != hipSuccess) {
       if (event) (void)hipEventDestroy(event);
@@ -94,8 +94,7 @@ struct MadeOn {
     const Tensor& first = **data.begin();
     void* s = stream_of(first);
     if (s == stream) return;
-    if (!event) {
-    } else if (!capturing(s)) {
+    if (!capturing(s)) {
       if (hipStreamWaitEvent(static_cast<hipStream_t>(s), event, 0) != hipSuccess)
         throw std::runtime_error("hipStreamWaitEvent failed");
     } else {  // a graph cannot wait for work outside it: the host does
@@ -233,7 +232,7 @@ struct LayerAhead {
  * assumed size (`per_row` pairs a row), one wait for the offsets; with more pairs than assumed the
  * emit pass has written nothing and runs again into exact buffers.  Returns (in_maps, out_maps,
  * offsets int64, offsets int32, group starts (bytes) and their address, offsets in device memory, table
- * flags, where (and, with work behind the wait, when) the lists were made). */
+ * flags, where and when the lists were made). */
 py::tuple kernel_map(const py::object& table, const Tensor& out4, const Int3& ks, const Int3& st,
                      const std::optional<Int3>& dilation, const std::optional<Int3>& centre, double per_row,
                      int64_t keep_workspace_bytes, LayerAhead* ahead) {
@@ -263,7 +262,9 @@ py::tuple kernel_map(const py::object& table, const Tensor& out4, const Int3& ks
       std::min<int64_t>(K * M, std::max<int64_t>(static_cast<int64_t>(1.25 * per_row * M) + 4096, int64_t{1} << 16));
   Tensor in_buf = at::empty({assumed}, out4.options()), out_buf = at::empty({assumed}, out4.options());
   Tensor kept;
-  std::shared_ptr<MadeOn> made;  // where work on the lists was enqueued behind the wait
+  // The wait is for the counts: the lists and the group starts may be on their way still, so a call on another stream waits for the
+  // event behind the kernels that write them (the one that the counts' mailbox has anyway: no launch more).
+  std::shared_ptr<MadeOn> made;
   int64_t begin = 0;
   while (true) {
     TableRef t(table);
@@ -326,6 +327,8 @@ py::tuple kernel_map(const py::object& table, const Tensor& out4, const Int3& ks
     } else {
       in_buf = in_buf.narrow(0, 0, total);
       out_buf = out_buf.narrow(0, 0, total);
+      void* const behind = wcn_kmap_take_event(w);
+      made = behind ? std::make_shared<MadeOn>(stream, behind) : std::make_shared<MadeOn>(stream);
     }
     break;
   }
@@ -335,7 +338,7 @@ py::tuple kernel_map(const py::object& table, const Tensor& out4, const Int3& ks
   const auto address = reinterpret_cast<uintptr_t>(groups.const_data_ptr());
   return py::make_tuple(in_buf, out_buf, offsets, offsets32, groups, address,
                         kept.narrow(0, 0, 8 * (int64_t{K} + 1)).view(at::kLong), wcn_kmap_last_table_flags(),
-                        made ? py::cast(made) : py::reinterpret_steal<py::object>(PyLong_FromVoidPtr(stream)));
+                        made);
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -360,17 +363,14 @@ struct MapRef {
     K = static_cast<int32_t>(offsets.numel() - 1);
     py::object id = km.attr("identity_map_index");
     if (!id.is_none()) identity = id.cast<int64_t>();
-    // A builder's lists, and the workspace's head with offsets and group starts, on another stream than the builder's.  `_made` is
-    // that stream where the host has waited for the lists.
+    // A builder's lists, and the workspace's head with offsets and group starts, on another stream than the builder's.
     py::object made = km.attr("_made");
     if (made.is_none()) return;
-    auto elsewhere = [&](const MadeOn& m) {
-      py::object head = km.attr("_device_offsets");
-      const Tensor h = head.is_none() ? Tensor() : head.cast<Tensor>();
-      m.before_use({&in_maps, &out_maps, &h});
-    };
-    if (!PyLong_Check(made.ptr())) elsewhere(*made.cast<const MadeOn*>());
-    else if (void* const stream = PyLong_AsVoidPtr(made.ptr()); stream != stream_of(in_maps)) elsewhere(MadeOn(stream, true));
+    const MadeOn& m = *made.cast<const MadeOn*>();
+    if (m.stream == stream_of(in_maps)) return;
+    py::object head = km.attr("_device_offsets");
+    const Tensor h = head.is_none() ? Tensor() : head.cast<Tensor>();
+    m.before_use({&in_maps, &out_maps, &h});
   }
   const int64_t* host_offsets() const { return offsets.const_data_ptr<int64_t>(); }
   int64_t pairs() const { return host_offsets()[K]; }

@@ -1645,7 +1645,9 @@ static thread_local struct {
   Pending kind = Pending::none;
   int64_t sequence = 0;
   const void* result = nullptr;
+  bool filled = false;  // the event behind the write is behind the map's lists too
 } g_pending;
+static thread_local const void* g_filled = nullptr;  // the result block of such a map, from its read to wcn_kmap_take_event
 
 static void set_pending(Pending kind, int64_t sequence, const void* result) {
   g_pending = {sequence != 0 ? kind : Pending::none, sequence, result};
@@ -1706,17 +1708,23 @@ static int kmap_count_impl(const void* table, int64_t n_keys, int64_t capacity, 
   else if (own) hipLaunchKernelGGL(kmap_scan_rows, dim3(g.K), dim3(1024), 0, s, w.blocks, (int64_t)w.B, w.row_total, fin);
   else hipLaunchKernelGGL(kmap_scan_rows, dim3(g.K + 1), dim3(1024), 0, s, w.groups, w.G, w.row_total, fin);
   WCN_LAUNCH_CHECK();
-  if (box) {
-    if (wcn_mailbox_mark(s) != WCN_OK) return WCN_ERR_LAUNCH;
-  } else if (wcn_read_early_begin(w.result, sizeof(int64_t) * (size_t)(g.K + 3), s) != WCN_OK) {
-    return WCN_ERR_LAUNCH;
-  }
+  if (!box && wcn_read_early_begin(w.result, sizeof(int64_t) * (size_t)(g.K + 3), s) != WCN_OK) return WCN_ERR_LAUNCH;
+  bool emitted = true;
   if (fill && !together && num_out > 0 && (own || pair_capacity > 0)) {
     if (own) launch_starts_emit(num_out, g, w, pair_capacity, in_maps, out_maps, fin, s);
     else launch_emit(num_out, g, w, pair_capacity, in_maps, out_maps, s);
-    WCN_LAUNCH_CHECK();
+    emitted = hipGetLastError() == hipSuccess;
   }
-  return WCN_OK;
+  // behind all of the map's kernels: whoever reads the lists on another stream waits for this event (wcn_kmap_take_event)
+  if (box && wcn_mailbox_mark(s) != WCN_OK) return WCN_ERR_LAUNCH;
+  g_pending.filled = fill && box;
+  return emitted ? WCN_OK : WCN_ERR_LAUNCH;
+}
+
+void* wcn_kmap_take_event(const void* workspace) {
+  if (!workspace || g_filled != workspace) return nullptr;
+  g_filled = nullptr;
+  return wcn_mailbox_take_event();
 }
 
 int wcn_kmap_count_fill(const void* table, int64_t n_keys, int64_t capacity, const int32_t* out_coords, int64_t num_out,
@@ -1845,8 +1853,12 @@ int wcn_kmap_read_result(const void* workspace, int64_t num_out, int32_t num_off
   const size_t bytes = sizeof(int64_t) * (size_t)(num_offsets + 3);
   // from the mailbox the count call armed; otherwise (another thread, a count call that failed
   // half-way) from the device copy
+  const bool filled = g_pending.filled;
   const int64_t sequence = take_pending(Pending::map, w.result);
-  if (sequence == 0 || wcn_mailbox_end(tmp, bytes, sequence) != WCN_OK) {
+  g_filled = nullptr;
+  if (sequence != 0 && wcn_mailbox_end(tmp, bytes, sequence) == WCN_OK) {
+    if (filled) g_filled = w.result;
+  } else {
     if (wcn_read_early_end(tmp, w.result, bytes, (hipStream_t)stream) != WCN_OK) return WCN_ERR_LAUNCH;
   }
   for (int k = 0; k <= num_offsets; ++k) host_offsets[k] = tmp[k];

@@ -981,6 +981,14 @@ int wcn_mailbox_end(void* host_dst, size_t payload_bytes, int64_t sequence, bool
   return WCN_OK;
 }
 
+// The event behind the thread's last write, which has been collected, is the caller's from here on (the next write gets another).
+void* wcn_mailbox_take_event() {
+  if (g_box_open != 0) return nullptr;
+  void* const event = (void*)g_box_done;
+  g_box_done = nullptr;
+  return event;
+}
+
 int wcn_table_status_from_bits(int32_t bits) {
   if (bits & WCN_DEV_RANGE) return WCN_ERR_COORD_RANGE;
   if (bits & WCN_DEV_OVERFLOW) return WCN_ERR_TABLE_OVERFLOW;

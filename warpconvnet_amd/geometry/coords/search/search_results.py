@@ -21,7 +21,7 @@ class IntSearchResult:
     _out_ascend = False
     _group_start = None
     _device_offsets = None  # (K + 1) int64 copy of `offsets` in device memory, when the builder left one
-    _made = None            # the builder's stream (an address), or where and when work behind its wait was enqueued
+    _made = None            # where and when the builder made the lists: a call on another stream waits for that
     _offsets64 = None       # `offsets` as an int64 host tensor, made on first use where the builder left none
     # For the gradients: whether in_maps ascends inside every offset (the map of a transposed
     # convolution: a forward map with its lists exchanged), the group starts that belong to that order,
