@@ -213,6 +213,35 @@ def test_a_map_just_made_serves_layers_on_other_streams(rows, ksize, width, assu
         del km
 
 
+def test_maps_put_together_of_others_serve_layers_on_other_streams():
+    """Over four spatial dimensions the lists are joined behind the builder's wait; half a map has the whole one's lists."""
+    from warpconvnet_amd._lib import host
+    from warpconvnet_amd.geometry.coords.search.torch_discrete import generate_kernel_map
+    from warpconvnet_amd.nn.functional.sparse_conv import sparse_conv_forward
+    at = torch.as_tensor(np.random.default_rng(23).permutation(24 ** 4)[:60_000], device=DEV)
+    c = torch.stack([torch.zeros_like(at), at // 24 ** 3, at // 24 ** 2 % 24, at // 24 % 24, at % 24], 1).int()
+    n = len(c)
+    x = normal_features(n, 16, seed=1, dtype=torch.float16).to(DEV)
+    w = kaiming_weight(81, 16, 16, seed=2, dtype=torch.float16).to(DEV)
+    make = lambda **kw: generate_kernel_map(c, c, (1,) * 4, (3,) * 4, **kw)
+    want = sparse_conv_forward(x, w, make(), n)
+    a, b = torch.cuda.Stream(), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(a):
+        km = make()
+    with torch.cuda.stream(b):
+        got = sparse_conv_forward(x, w, km, n)
+    assert isinstance(km._made, host().MadeOn)
+    torch.cuda.synchronize()
+    assert torch.equal(got, want)
+    for half, whole in ((make(skip_symmetric_kernel_map=True), km),
+                        (generate_kernel_map(c[:, :4].contiguous(), c[:, :4].contiguous(), (1,) * 3, (3,) * 3,
+                                             skip_symmetric_kernel_map=True), None)):
+        assert isinstance(half._made, host().MadeOn) and half.in_maps.shape[0] == int(half.offsets[-1])
+        if whole is not None:
+            assert torch.equal(half.in_maps, whole.in_maps[:len(half.in_maps)]) and len(half) == 40
+
+
 def test_copies_and_files_of_voxels_with_maps():
     """copy.deepcopy and pickle of a tensor whose cache holds maps with everything the layers left on them: the copy
     makes its own and gives the same results after the original is gone."""

@@ -218,13 +218,18 @@ def _kernel_map_more_dims(in_coords: Tensor, out_coords: Tensor, stride, kernel_
     result._out_ascend = True
     result._from_builder = True
     result._keys_unique = all(getattr(m, "_keys_unique", False) for m in maps)
-    if skip_symmetric_kernel_map and is_odd:
-        half = K // 2
-        end = int(result.offsets[half])
-        result = IntSearchResult(result.in_maps[:end], result.out_maps[:end],
-                                 result.offsets[: half + 1].clone(), identity_map_index=identity_map_index)
-        result._out_ascend = True
-    return result
+    result._made = native().made_now(result.in_maps)  # (the lists have just been put together, on this stream)
+    return _half_of(result, K // 2) if skip_symmetric_kernel_map and is_odd else result
+
+
+def _half_of(result: IntSearchResult, half: int) -> IntSearchResult:
+    """The offsets before the centre (reference: torch_discrete.py:286-296): lists that are views of the whole map's."""
+    end = int(result.offsets[half])
+    first = IntSearchResult(result.in_maps[:end], result.out_maps[:end], result.offsets[: half + 1].clone(),
+                            identity_map_index=result.identity_map_index)
+    first._out_ascend = True
+    first._made = result._made
+    return first
 
 
 def generate_kernel_map(
@@ -298,12 +303,4 @@ def generate_kernel_map(
     result._from_builder = True  # pairs come from one lookup per (offset, output row)
     result._symmetric = bool(same_set and is_odd and all(s == 1 for s in stride)
                              and centres is None and getattr(result, "_keys_unique", False))
-    if skip_symmetric_kernel_map and is_odd:
-        # only the offsets before the centre are kept (torch_discrete.py:286-296)
-        half = int(np.prod(kernel_size)) // 2
-        end = int(result.offsets[half])
-        result = IntSearchResult(result.in_maps[:end], result.out_maps[:end],
-                                 result.offsets[: half + 1].clone(),
-                                 identity_map_index=identity_map_index)
-        result._out_ascend = True
-    return result
+    return _half_of(result, int(np.prod(kernel_size)) // 2) if skip_symmetric_kernel_map and is_odd else result
