@@ -226,17 +226,3 @@ def test_calls_that_wait_for_the_map(monkeypatch, case):
     first = spatially_sparse_conv(vox, w, 3, **kw).feature_tensor
     assert len(made) == 1 and made[0].out is None
     assert torch.equal(first, spatially_sparse_conv(vox, w, 3, **kw).feature_tensor)
-
-
-@pytest.mark.parametrize("grad", [False, True])
-@pytest.mark.parametrize("kernel,stride", [(3, 1), (2, 2)])
-def test_a_kept_map_asks_for_no_layer_ahead(monkeypatch, kernel, stride, grad):
-    """What a layer ahead of its map needs is put together behind the miss in the cache, not for every layer."""
-    from warpconvnet_amd.nn.functional.sparse_conv import spatially_sparse_conv
-    made = _spied(monkeypatch)
-    w = kaiming_weight(kernel ** 3, 32, 32, seed=2, dtype=torch.float16).to(DEV).requires_grad_(grad)
-    vox = _voxels(1800, 32, torch.float16, seed=1)
-    first = spatially_sparse_conv(vox, w, kernel, stride=stride).feature_tensor
-    assert len(made) == 1
-    again = spatially_sparse_conv(vox, w, kernel, stride=stride).feature_tensor
-    assert len(made) == 1 and torch.equal(first, again)

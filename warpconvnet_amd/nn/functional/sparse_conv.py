@@ -228,8 +228,7 @@ def generate_output_coords_and_kernel_map(
 ) -> Tuple[Tensor, Tensor, IntSearchResult]:
     """Output coordinates (given / strided / same as input), then the kernel map, through the
     cache on the input tensor (reference: sparse_conv.py:1808-1996).  A transposed convolution
-    reuses the cached forward map of the matching strided convolution with in/out exchanged.
-    `_ahead`: makes the layer that generate_kernel_map is given to launch; called where the cache has no map."""
+    reuses the cached forward map of the matching strided convolution with in/out exchanged."""
     strided = any(s != 1 for s in stride)
     if strided and stride_mode == STRIDED_CONV_MODE.REDUCE_AND_STRIDE:
         raise ValueError("REDUCE_AND_STRIDE reaches the map builder with stride 1 (the functional "
@@ -302,8 +301,7 @@ def generate_output_coords_and_kernel_map(
     else:
         kernel_map = generate_kernel_map(in_coords, out_coords, stride, kernel_size,
                                          kernel_dilation, method=method,
-                                         skip_symmetric_kernel_map=False,
-                                         _ahead=_ahead() if _ahead is not None else None)
+                                         skip_symmetric_kernel_map=False, _ahead=_ahead)
         # kernel as large as the stride over voxels without repeats: every input row is in one pair
         kernel_map._single_in = bool(
             strided and tuple(kernel_size) == tuple(stride) and all(int(d) == 1 for d in kernel_dilation)
@@ -454,20 +452,15 @@ def spatially_sparse_conv(
     needs_grad = torch.is_grad_enabled() and (features.requires_grad or weight.requires_grad)
     needs_residual_grad = residual is not None and torch.is_grad_enabled() and residual.requires_grad
     ahead = None
-
-    def layer_ahead():
-        """Asked for where the map has to be made: the layer does not wait for the host to have read the map's offsets."""
-        nonlocal ahead
+    if not transposed and features.is_cuda and (needs_grad or not needs_residual_grad):
+        # a layer whose map has to be made first does not wait for the host to have read the map's offsets
         ahead = native().LayerAhead(features, weight, bias, effective_compute_dtype, None, False, False, True) if needs_grad \
             else native().LayerAhead(features, weight, bias, effective_compute_dtype, residual, relu, keep_prepared_weight)
-        return ahead
-
-    can_go_ahead = not transposed and features.is_cuda and (needs_grad or not needs_residual_grad)
     out_coords, out_offsets, kernel_map = generate_output_coords_and_kernel_map(
         input_sparse_tensor=input_sparse_tensor, kernel_size=_kernel_size,
         kernel_dilation=_kernel_dilation, stride=_stride, generative=generative,
         transposed=transposed, output_spatially_sparse_tensor=output_spatially_sparse_tensor,
-        stride_mode=stride_mode, order=order, _ahead=layer_ahead if can_go_ahead else None)
+        stride_mode=stride_mode, order=order, _ahead=ahead)
     num_out_coords = out_coords.shape[0]
 
     if needs_grad:
