@@ -226,3 +226,22 @@ def test_calls_that_wait_for_the_map(monkeypatch, case):
     first = spatially_sparse_conv(vox, w, 3, **kw).feature_tensor
     assert len(made) == 1 and made[0].out is None
     assert torch.equal(first, spatially_sparse_conv(vox, w, 3, **kw).feature_tensor)
+
+
+def test_dilated_and_plain_layers_keep_their_own_estimates(monkeypatch):
+    """Over voxels of even places a row has one pair, and nine with a dilation of two: neither layer makes the other's lists too short."""
+    from warpconvnet_amd.geometry.types.voxels import Voxels
+    from warpconvnet_amd.nn.functional.sparse_conv import spatially_sparse_conv
+    made = _spied(monkeypatch)
+    cells = np.stack(np.meshgrid(np.arange(200), np.arange(200), [0], indexing="ij"), axis=-1).reshape(-1, 3).astype(np.int32) * 2
+    n = len(cells)
+    x = normal_features(n, 32, seed=1, dtype=torch.float16).to(DEV)
+    w = kaiming_weight(27, 32, 32, seed=2, dtype=torch.float16).to(DEV)
+    for turn in range(3):
+        for dilation, pairs in ((1, n), (2, (200 * 3 - 2) ** 2)):
+            vox = Voxels(torch.as_tensor(cells, device=DEV), x, offsets=torch.tensor([0, n]))
+            got = spatially_sparse_conv(vox, w, 3, kernel_dilation=dilation).feature_tensor
+            assert next(iter(vox.cache.values())).in_maps.shape[0] == pairs
+            if turn > 0:
+                assert made[-1].out is not None, dilation
+                assert torch.equal(got, spatially_sparse_conv(vox, w, 3, kernel_dilation=dilation).feature_tensor)

@@ -61,8 +61,9 @@ def _pad_kernel_args(values: Sequence[int], fill: int):
 # a map builder's workspace up to this size stays with its map (see _kernel_map_from_table)
 _KEEP_WORKSPACE_BYTES = 256 << 20
 
-# pairs per output row of the last map built for (kernel size, stride, size class of the row count), by quarters of an octave of rows
-# and by whole ones (negative): sizes the buffers the pairs are emitted into before their number is known
+# pairs per output row of the last map built for (kernel size, stride, dilation and centre where they are not the plain ones, size
+# class of the row count), by quarters of an octave of rows and by whole ones (negative): sizes the buffers the pairs are emitted into
+# before their number is known
 _PAIRS_PER_ROW = {}
 
 
@@ -87,12 +88,17 @@ def _kernel_map_from_table(table: TorchHashTable, out_coords: Tensor, kernel_siz
         ahead.identity = identity_map_index
     M = out4.shape[0]
     ks, st = _pad_kernel_args(kernel_size, 1), _pad_kernel_args(stride, 1)
+    dil = None if dilation is None else _pad_kernel_args(dilation, 1)
+    centre = None if dilation is None else _pad_kernel_args(centres, 0)
     # (levels of a network lie within an octave: 1 M rows of 5 pairs and 553 k of 9, each of which made the other emit its pairs twice)
-    size, octave = (tuple(ks), tuple(st), (M ** 4).bit_length()), (tuple(ks), tuple(st), -M.bit_length())
+    # A dilated kernel's pairs are another number than the plain one's (voxels of even places: 1 and 9 a row); until one has been
+    # built the plain one's have to do.
+    plain = (tuple(ks), tuple(st))
+    kind = plain if dil is None else plain + (tuple(dil), tuple(centre))
+    size, octave = kind + ((M ** 4).bit_length(),), kind + (-M.bit_length(),)
+    per_row = _PAIRS_PER_ROW.get(size, _PAIRS_PER_ROW.get(octave, _PAIRS_PER_ROW.get(plain + octave[-1:], 8.0)))
     in_maps, out_maps, offsets64, offsets, groups, address, device_offsets, flags, made = native().kernel_map(
-        table, out4, ks, st, None if dilation is None else _pad_kernel_args(dilation, 1),
-        None if dilation is None else _pad_kernel_args(centres, 0), _PAIRS_PER_ROW.get(size, _PAIRS_PER_ROW.get(octave, 8.0)),
-        _KEEP_WORKSPACE_BYTES, ahead)
+        table, out4, ks, st, dil, centre, per_row, _KEEP_WORKSPACE_BYTES, ahead)
     if M > 0:
         _PAIRS_PER_ROW[size] = _PAIRS_PER_ROW[octave] = in_maps.shape[0] / M
     K = offsets.shape[0] - 1
