@@ -494,3 +494,24 @@ def test_what_the_benchmark_and_the_entry_points_import_is_there():
                     if not hasattr(module, alias.name):
                         importlib.import_module(f"{node.module}.{alias.name}")
         assert found > 0
+
+
+@pytest.mark.parametrize("slots,after", [(4096, 1 << 17), (1 << 15, 1 << 17), (1 << 16, 1 << 18), (1 << 24, 1 << 26), (1 << 25, 1 << 27),
+                                         (1 << 26, None), (1 << 27, None), (1 << 30, None)])
+def test_a_table_grows_as_long_as_that_makes_more_bins(monkeypatch, slots, after):
+    """Up to 2^26 slots: there a rebuild would overflow in the same bins, however many keys there are."""
+    from warpconvnet_amd._lib import ERR_TABLE_OVERFLOW, WcnError, lib
+    from warpconvnet_amd.geometry.coords.search.torch_hashmap import TorchHashTable
+    builds = []
+    monkeypatch.setattr(TorchHashTable, "_build", lambda self, n: builds.append(n))
+    keys = torch.zeros(1, 4, dtype=torch.int32).expand(40_000_000, 4)  # (nothing reads them)
+    table = TorchHashTable._over(keys, None, slots)
+    n = 40_000_000
+    if after is None:
+        with pytest.raises(WcnError) as e:
+            table._grow()
+        assert e.value.status == ERR_TABLE_OVERFLOW and builds == []
+        assert lib().wcn_table_bytes(n, 1 << 26) == lib().wcn_table_bytes(n, slots)
+    else:
+        table._grow()
+        assert builds == [after] and lib().wcn_table_bytes(n, after) > lib().wcn_table_bytes(n, slots)

@@ -19,6 +19,9 @@ from ...._lib import ERR_TABLE_OVERFLOW, WcnError, check, lib, ptr, require_devi
 from ...._lib import host as native
 
 
+_LEAST_SLOTS, _MOST_SLOTS = 1 << 15, 1 << 26  # 16 to 32,768 bins of 2,048 slots, whatever the slot count says
+
+
 class HashMethod(enum.Enum):
     FNV1A = 0
     CITY = 1
@@ -96,13 +99,12 @@ class TorchHashTable:
         self._checked = False
 
     def _grow(self) -> None:
-        """Rebuild with four times the slots (after the device reported an overflow).  More slots
-        shorten the probe chains and, up to 2^26 slots, mean more bins during the build; beyond
-        that and four slots per key neither changes and the overflow is final."""
-        n = self._keys4.shape[0]
-        if self._slots >= (1 << 30) or (self._slots >= (1 << 26) and self._slots >= 4 * n):
+        """Rebuild with four times the slots (after the device reported an overflow: a bin with more distinct blocks
+        than its region has slots).  More slots mean more bins, from 2^15 up to 2^26 slots; beyond that a rebuild would be
+        the same table and the overflow is final."""
+        if self._slots >= _MOST_SLOTS:
             raise WcnError(ERR_TABLE_OVERFLOW, "wcn_table_build")
-        self._build(self._slots * 4)
+        self._build(max(self._slots, _LEAST_SLOTS) * 4)
 
     def _ensure_checked(self) -> None:
         """Read the device-side build status once (this waits for the stream)."""
