@@ -515,3 +515,42 @@ def test_a_table_grows_as_long_as_that_makes_more_bins(monkeypatch, slots, after
     else:
         table._grow()
         assert builds == [after] and lib().wcn_table_bytes(n, after) > lib().wcn_table_bytes(n, slots)
+
+
+@pytest.mark.parametrize("read", ["item", "iteration", "batch", "csr", "clone", "deepcopy", "pickle", "unpool"])
+def test_whoever_reads_a_map_s_lists_waits_for_them(read):
+    """The host knows a map's counts before its lists are complete: what torch does with the lists, on whichever stream, comes behind
+    the builder's event."""
+    import copy
+    import pickle
+    from types import SimpleNamespace
+    from warpconvnet_amd.geometry.coords.search.search_results import IntSearchResult
+    from warpconvnet_amd.nn.functional.sparse_pool import sparse_unpool
+
+    class Made:
+        waits = 0
+
+        def before_use(self, *lists):
+            assert lists[0] is km.in_maps and lists[1] is km.out_maps
+            Made.waits += 1
+
+    ints = lambda *v: torch.tensor(v, dtype=torch.int32)
+    km = IntSearchResult(ints(2, 0, 1), ints(0, 1, 1), torch.tensor([0, 1, 3]))
+    km._made = Made()
+    if read == "item":
+        assert [t.tolist() for t in km[1]] == [[0, 1], [1, 1]]
+    elif read == "iteration":
+        assert [t.tolist() for pair in km for t in pair] == [[2], [0], [0, 1], [1, 1]]
+    elif read == "batch":
+        assert km.get_batch(0, 2, "tensor")[0].tolist() == [[2, -1], [0, 1]]
+    elif read == "csr":
+        assert [t.tolist() for t in km.to_csr()] == [[2, 0, 1], [0, 1], [0, 1, 3]]
+    elif read in ("clone", "deepcopy", "pickle"):
+        other = {"clone": km.clone, "deepcopy": lambda: copy.deepcopy(km), "pickle": lambda: pickle.loads(pickle.dumps(km))}[read]()
+        assert other._made is None and other.in_maps.tolist() == [2, 0, 1] and other.out_maps.tolist() == [0, 1, 1]
+    else:
+        pooled = SimpleNamespace(num_spatial_dims=3, offsets=ints(0, 2), cache=SimpleNamespace(get=lambda key: km),
+                                 feature_tensor=torch.tensor([[1.], [2.]]))
+        fine = SimpleNamespace(offsets=ints(0, 3), replace=lambda batched_features: batched_features)
+        assert sparse_unpool(pooled, fine, 2, 2).tolist() == [[2.], [2.], [1.]]
+    assert Made.waits > 0

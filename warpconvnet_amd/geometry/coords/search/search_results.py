@@ -75,13 +75,22 @@ class IntSearchResult:
     _OWN = ("_group_start", "_in_group_start", "_device_offsets", "_made", "_by_out", "_by_in", "_rows_forms", "_tile_plan",
             "_forward_map", "_tiles_wanted")
 
+    def _lists(self) -> Tuple[Tensor, Tensor]:
+        """in_maps and out_maps for operations on the current stream, which may be another than the builder's: the host's wait
+        for a map is one for its counts, and the lists may be on their way still."""
+        if self._made is not None:
+            self._made.before_use(self.in_maps, self.out_maps, self.out_maps)
+        return self.in_maps, self.out_maps
+
     def __getstate__(self):
+        self._lists()  # (about to be copied)
         return {name: value for name, value in self.__dict__.items() if name not in self._OWN}
 
     @torch.no_grad()
     def __getitem__(self, idx: int) -> Tuple[Tensor, Tensor]:
         start, end = int(self.offsets[idx]), int(self.offsets[idx + 1])
-        return self.in_maps[start:end], self.out_maps[start:end]
+        in_maps, out_maps = self._lists()
+        return in_maps[start:end], out_maps[start:end]
 
     def __len__(self) -> int:
         return len(self.offsets) - 1
@@ -117,14 +126,15 @@ class IntSearchResult:
     @torch.no_grad()
     def to_csr(self) -> Tuple[Tensor, Tensor, Tensor]:
         """(in indices sorted by out index, unique out indices, CPU row offsets)."""
-        out_sorted, order = torch.sort(self.out_maps)
+        in_maps, out_maps = self._lists()
+        out_sorted, order = torch.sort(out_maps)
         unique_out, counts = torch.unique(out_sorted, return_counts=True, sorted=True)
         offsets = torch.cat([torch.zeros(1, dtype=torch.int32), torch.cumsum(counts.cpu(), dim=0)])
-        return self.in_maps[order], unique_out, offsets
+        return in_maps[order], unique_out, offsets
 
     def clone(self) -> "IntSearchResult":
-        return IntSearchResult(self.in_maps.clone(), self.out_maps.clone(), self.offsets.clone(),
-                               self.identity_map_index)
+        in_maps, out_maps = self._lists()
+        return IntSearchResult(in_maps.clone(), out_maps.clone(), self.offsets.clone(), self.identity_map_index)
 
     @property
     def device(self):

@@ -98,7 +98,7 @@ def sparse_unpool(pooled_voxels: Voxels, unpooled_voxels: Voxels, kernel_size, s
     assert pooled_voxels.cache is not None
     kernel_map = pooled_voxels.cache.get(key)
     assert kernel_map is not None
-    unpooled_maps, pooled_maps = kernel_map.in_maps, kernel_map.out_maps
+    unpooled_maps, pooled_maps = kernel_map._lists()
     perm = torch.argsort(unpooled_maps)
     rep_feats = take_rows(pooled_voxels.feature_tensor, pooled_maps[perm].long())
     if concat_unpooled_voxels:
