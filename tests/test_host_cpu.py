@@ -554,3 +554,33 @@ def test_whoever_reads_a_map_s_lists_waits_for_them(read):
         fine = SimpleNamespace(offsets=ints(0, 3), replace=lambda batched_features: batched_features)
         assert sparse_unpool(pooled, fine, 2, 2).tolist() == [[2.], [2.], [1.]]
     assert Made.waits > 0
+
+
+def test_strided_rows_give_up_where_more_slots_make_no_more_bins(monkeypatch):
+    """The table over coarse rows of any stride is rebuilt as a coordinate table is: not where it would overflow in the same bins."""
+    import importlib
+    from warpconvnet_amd._lib import ERR_TABLE_OVERFLOW, WcnError
+    stride = importlib.import_module("warpconvnet_amd.geometry.coords.ops.stride")
+    builds = []
+
+    class Library:
+        wcn_table_default_capacity = staticmethod(lambda n: 1024)
+        wcn_stride_unique_workspace_bytes = staticmethod(lambda n, slots: 256)
+        wcn_stride_unique_read_count = staticmethod(lambda *a: ERR_TABLE_OVERFLOW)
+        wcn_stride_unique_read_bounds = staticmethod(lambda *a: ERR_TABLE_OVERFLOW)
+
+        @staticmethod
+        def wcn_stride_unique(coords, n, st, ws, slots, *rest):
+            builds.append(slots)
+            return 0
+
+    monkeypatch.setattr(stride, "lib", lambda: Library)
+    monkeypatch.setattr(stride, "stream_ptr", lambda device: None)
+    monkeypatch.setattr(stride, "workspace", lambda n, device: torch.empty(n, dtype=torch.uint8))
+    monkeypatch.setattr(stride, "_four_columns", lambda rows: rows)
+    for batch_sorted in (False, True):
+        builds.clear()
+        with pytest.raises(WcnError) as e:
+            stride._unique_floor_div(torch.zeros(10, 4, dtype=torch.int32), (3, 3, 3), batch_sorted)
+        assert e.value.status == ERR_TABLE_OVERFLOW
+        assert builds == [1024, 1 << 17, 1 << 19, 1 << 21, 1 << 23, 1 << 25, 1 << 27]

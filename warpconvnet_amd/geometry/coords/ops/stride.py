@@ -9,7 +9,7 @@ from torch import Tensor
 from ...._lib import ERR_TABLE_OVERFLOW, check, int3, lib, ptr, stream_ptr, workspace
 from ...._lib import host as native
 from .batch_index import offsets_from_batch_index
-from ..search.torch_hashmap import _four_columns
+from ..search.torch_hashmap import _four_columns, more_slots
 
 
 def stride_coords(batch_indexed_coords: Tensor, stride: Tuple[int, ...],
@@ -86,8 +86,8 @@ def _unique_floor_div(batch_indexed_coords: Tensor, stride: Tuple[int, ...], bat
         check(L.wcn_stride_unique(ptr(coords), n, st, ptr(ws), slots, ptr(out), ptr(first),
                                   stream_ptr(device)), "wcn_stride_unique")
         status = read(ws, slots)
-        if status == ERR_TABLE_OVERFLOW and slots < (1 << 30):
-            slots *= 4
+        if status == ERR_TABLE_OVERFLOW:
+            slots = more_slots(slots)
             continue
         check(status, "wcn_stride_unique")
         break

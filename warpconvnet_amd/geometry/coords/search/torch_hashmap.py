@@ -22,6 +22,15 @@ from ...._lib import host as native
 _LEAST_SLOTS, _MOST_SLOTS = 1 << 15, 1 << 26  # 16 to 32,768 bins of 2,048 slots, whatever the slot count says
 
 
+def more_slots(slots: int) -> int:
+    """Slots of the rebuild after the device reported an overflow (a bin with more distinct blocks than its region has
+    slots): four times as many.  More slots mean more bins, from 2^15 up to 2^26 slots; beyond that a rebuild would be the same table
+    and the overflow is final."""
+    if slots >= _MOST_SLOTS:
+        raise WcnError(ERR_TABLE_OVERFLOW, "wcn_table_build")
+    return max(slots, _LEAST_SLOTS) * 4
+
+
 class HashMethod(enum.Enum):
     FNV1A = 0
     CITY = 1
@@ -99,12 +108,7 @@ class TorchHashTable:
         self._checked = False
 
     def _grow(self) -> None:
-        """Rebuild with four times the slots (after the device reported an overflow: a bin with more distinct blocks
-        than its region has slots).  More slots mean more bins, from 2^15 up to 2^26 slots; beyond that a rebuild would be
-        the same table and the overflow is final."""
-        if self._slots >= _MOST_SLOTS:
-            raise WcnError(ERR_TABLE_OVERFLOW, "wcn_table_build")
-        self._build(max(self._slots, _LEAST_SLOTS) * 4)
+        self._build(more_slots(self._slots))
 
     def _ensure_checked(self) -> None:
         """Read the device-side build status once (this waits for the stream)."""
