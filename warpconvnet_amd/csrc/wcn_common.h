@@ -54,9 +54,6 @@ struct WcnTableHeader {  // first 256 bytes of a table workspace
 };
 static_assert(sizeof(WcnTableHeader) == 256, "header is 256 bytes");
 
-// Valid once the bins' counts have been summed into the header: every distinct key set one bit.
-#define WCN_HAS_DUPLICATES(hdr) ((hdr)->total != (hdr)->num_keys)
-
 struct WcnTableView {  // host-computed addresses inside a table workspace
   WcnTableHeader* hdr;
   WcnSlot* slots;         // bins regions of WCN_BIN_SLOTS

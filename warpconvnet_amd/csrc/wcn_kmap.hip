@@ -29,10 +29,9 @@ struct KmapGeom {
 
 struct KmapWorkspace {  // host-computed addresses inside a kmap workspace
   int64_t* result;      // [0..K] offsets, [K+1] = table status bits, [K+2] = occupied slots | duplicates << 32 | status << 33
-  int64_t* row_total;   // [K+1] totals of the rows of `groups`
+  int64_t* row_total;   // [K] totals of the scanned rows
   int32_t* ticket;      // arrival counter of the scan's workgroups (zeroed by the probe pass)
-  int32_t* groups;      // (K+1, G+1): rows 0..K-1 per-offset hit counts of each 64-row group, row K
-                        // all hits of the group; after the scan, exclusive prefix sums
+  int32_t* groups;      // (K, G+1): per-offset hit counts of each 64-row group; after the scan, exclusive prefix sums
   int32_t* found;       // (G, 64 K): input rows found by the hit lanes of a group, packed offset by offset
   uint16_t* tags;       // (G, 64 K): offset << 6 | lane of each of them
   uint16_t* counts;     // (K, C): hits per offset of the probe's workgroups of 256 rows (maps that kmap_starts_emit finishes)
@@ -60,11 +59,11 @@ inline size_t kmap_layout(void* base, int64_t num_out, int32_t K, KmapWorkspace*
   if (w) w->result = (int64_t*)(p + off);
   off += wcn_align256(sizeof(int64_t) * (size_t)(K + 3));
   if (w) w->row_total = (int64_t*)(p + off);
-  off += wcn_align256(sizeof(int64_t) * (size_t)(K + 1));
+  off += wcn_align256(sizeof(int64_t) * (size_t)K);
   if (w) w->ticket = (int32_t*)(p + off);
   off += 256;
   if (w) w->groups = (int32_t*)(p + off);
-  off += wcn_align256(sizeof(int32_t) * (size_t)(K + 1) * (size_t)(G + 1));
+  off += wcn_align256(sizeof(int32_t) * (size_t)K * (size_t)(G + 1));
   if (head_bytes) *head_bytes = off;
   if (parked) p = (char*)parked - off;
   if (w) w->found = (int32_t*)(p + off);
@@ -154,7 +153,6 @@ __global__ void __launch_bounds__(256) kmap_pass(const WcnTableHeader* __restric
       }
     }
   }
-  if (lane == 0) groups[(int64_t)g.K * (G + 1) + group] = group_hits;
 }
 
 // ---- fixed-size kernel: compile-time kernel size, every dimension spans at most 2 blocks -------
@@ -189,7 +187,7 @@ __global__ void __launch_bounds__(256) kmap_pass_fixed(const WcnTableHeader* __r
   __shared__ uint2 s_half[INSIDE ? 2 : 16][256];  // [block * 2 + upper half of x][thread]: occupancy, position of the first voxel
   __shared__ uint16_t s_list[4][LIST];
   __shared__ uint8_t s_sub[256];     // place of the first neighbour in its block: x | y << 2 | z << 4
-  __shared__ int32_t s_count[4][K + 1];
+  __shared__ int32_t s_count[4][K];
   const int tid = threadIdx.x;
   const int64_t m = (int64_t)wcn_xcd_tile((int)blockIdx.x, (int)gridDim.x) * 256 + tid;
   if (m == 0) *o.ticket = 0;
@@ -363,11 +361,10 @@ __global__ void __launch_bounds__(256) kmap_pass_fixed(const WcnTableHeader* __r
   if (last_at >= 0) found[last_at] = last;
   if (lane < K) s_count[wave][lane] = count[0];
   if (K > 64 && 64 + lane < K) s_count[wave][64 + lane] = count[1];
-  if (lane == 0) s_count[wave][K] = parked;
   __syncthreads();
   // the counts of four neighbouring groups lie beside each other
   const int there = (int)(G - (group - wave) < 4 ? G - (group - wave) : 4);
-  for (int i = tid; i < 4 * (K + 1); i += 256)
+  for (int i = tid; i < 4 * K; i += 256)
     if ((i & 3) < there) groups[(int64_t)(i >> 2) * (G + 1) + (group - wave) + (i & 3)] = s_count[i & 3][i >> 2];
   if (o.counts && tid < K)
     o.counts[tid * o.C + (int)(group >> 2)] = (uint16_t)(s_count[0][tid] + s_count[1][tid] + s_count[2][tid] + s_count[3][tid]);
@@ -470,8 +467,6 @@ __device__ __forceinline__ int kmap_nth_set_bit(unsigned long long mask, int r) 
   return pos;
 }
 
-// In-place exclusive prefix sum of each row of `groups` (one workgroup per row, G+1 entries; the
-// last entry receives the row total).
 __global__ void kmap_zero_ticket(int32_t* ticket) { *ticket = 0; }
 
 struct KmapFinish {  // null `result`: no finishing step
@@ -483,6 +478,8 @@ struct KmapFinish {  // null `result`: no finishing step
   int64_t sequence;
 };
 
+// In-place exclusive prefix sum of each row of `groups` (one workgroup per row, G+1 entries; the
+// last entry receives the row total).
 __global__ void __launch_bounds__(1024) kmap_scan_rows(int32_t* __restrict__ groups, int64_t G,
                                                        int64_t* __restrict__ row_total,
                                                        KmapFinish fin) {
@@ -560,9 +557,7 @@ __global__ void __launch_bounds__(1024) kmap_scan_rows(int32_t* __restrict__ gro
   }
   __shared__ int s_last;
   if (threadIdx.x == 0) {
-    // a row of the per-offset counts holds at most M < 2^31 pairs; the row of all hits can
-    // exceed int32, which the host turns into WCN_ERR_TOO_MANY_PAIRS
-    row[G] = (int32_t)carry;
+    row[G] = (int32_t)carry;  // (an offset's pairs are at most its output rows, < 2^31; callers with other rows see to it)
     row_total[blockIdx.x] = carry;
     s_last = 0;
     if (fin.result) {
@@ -623,7 +618,7 @@ struct SelfWorkspace {
   int64_t* result;      // as KmapWorkspace (same places: the read-result call serves both)
   int64_t* row_total;
   int32_t* ticket;
-  int32_t* groups;      // (K+1, G+1): the finished group starts of every offset (written by the emit pass)
+  int32_t* groups;      // (K, G+1): the finished group starts of every offset (written by the emit pass)
   uint32_t* hm;         // (num_out, words) hit masks per row
   int32_t* ptr;         // num_out: index into park of the row's first found row
   int32_t* park;        // (num_out, K) at most: found rows, row by row of a tile, offsets ascending
@@ -641,11 +636,11 @@ inline size_t self_layout(void* base, int64_t num_out, int32_t K, SelfWorkspace*
   if (w) w->result = (int64_t*)(p + off);
   off += wcn_align256(sizeof(int64_t) * (size_t)(K + 3));
   if (w) w->row_total = (int64_t*)(p + off);
-  off += wcn_align256(sizeof(int64_t) * (size_t)(K + 1));
+  off += wcn_align256(sizeof(int64_t) * (size_t)K);
   if (w) w->ticket = (int32_t*)(p + off);
   off += 256;
   if (w) w->groups = (int32_t*)(p + off);
-  off += wcn_align256(sizeof(int32_t) * (size_t)(K + 1) * (size_t)(G + 1));
+  off += wcn_align256(sizeof(int32_t) * (size_t)K * (size_t)(G + 1));
   if (w) w->hm = (uint32_t*)(p + off);
   off += wcn_align256(sizeof(uint32_t) * (size_t)words * (size_t)num_out);
   if (w) w->ptr = (int32_t*)(p + off);
@@ -1071,9 +1066,8 @@ __global__ void __launch_bounds__(SELF_CHUNK) self_emit(const uint32_t* __restri
 }
 
 // The scan and the emit pass of a small map in one: every workgroup adds up the counts of all of the probe's workgroups, which takes
-// the launch, and the wait for it, of kmap_scan_rows out of the chain.  It writes what the scan and the emit pass write
-// (but the starts of the row of all hits, which nothing reads): the first workgroup the offsets, the table's status and the host's
-// mailbox, and every one the starts of its own eight groups, in the place of their counts, which no other workgroup reads.
+// the launch, and the wait for it, of kmap_scan_rows out of the chain.  It writes what the scan and the emit pass write:
+// the first workgroup the offsets, the table's status and the host's mailbox, and every one the starts of its own eight groups, in the place of their counts, which no other workgroup reads.
 // KL: counts of a wave's offsets requested together.
 // SCANNED (larger maps): kmap_scan_rows has made starts of the counts, a quarter of what the starts of all groups are (which these
 // workgroups make of them), and has written the rest.  Over 1 M rows of 3x3x3 and 5x5x5 scan and emit 14.2 + 20.6 and 19.3 + 49.4 us
@@ -1706,7 +1700,7 @@ static int kmap_count_impl(const void* table, int64_t n_keys, int64_t capacity, 
   const KmapFinish fin = {w.result, w.ticket, v.hdr, g.K, box, sequence};
   if (together) launch_starts_emit(num_out, g, w, pair_capacity, in_maps, out_maps, fin, s);
   else if (own) hipLaunchKernelGGL(kmap_scan_rows, dim3(g.K), dim3(1024), 0, s, w.blocks, (int64_t)w.B, w.row_total, fin);
-  else hipLaunchKernelGGL(kmap_scan_rows, dim3(g.K + 1), dim3(1024), 0, s, w.groups, w.G, w.row_total, fin);
+  else hipLaunchKernelGGL(kmap_scan_rows, dim3(g.K), dim3(1024), 0, s, w.groups, w.G, w.row_total, fin);
   WCN_LAUNCH_CHECK();
   if (!box && wcn_read_early_begin(w.result, sizeof(int64_t) * (size_t)(g.K + 3), s) != WCN_OK) return WCN_ERR_LAUNCH;
   bool emitted = true;
