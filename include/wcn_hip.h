@@ -10,9 +10,10 @@
  *     first use and held until wcn_thread_release() or the end of the process; and, per process,
  *     the device-resident array behind wcn_sparse_conv_fwd_static;
  *   - per-thread state crosses calls in three places, all named where they are declared:
- *     wcn_kmap_count (_dilated, _self) and wcn_stride_unique_cells arm the result mailbox that the same
+ *     wcn_kmap_count (_dilated, _self, _fill, _fill_apart) and wcn_stride_unique_cells arm the result mailbox that the same
  *     thread's wcn_kmap_read_result and wcn_stride_unique_read_* collect (the next call that writes such a
- *     result, wcn_stride_unique among them, lets go of one that nobody has read),
+ *     result, wcn_stride_unique among them, lets go of one that nobody has read; behind a read wcn_kmap_take_event
+ *     hands out the event that belongs to it),
  *     wcn_kmap_last_table_flags reports on that thread's last read, and
  *     wcn_conv_set_timing_events arms the thread's next contraction call;
  *   - a call that waits for the device (the *_read_* functions) polls with an upper bound of
@@ -21,7 +22,7 @@
  *   - `stream` is a hipStream_t passed as void*; all work is enqueued on it and, unless stated,
  *     the call returns without waiting for the device;
  *   - the return value is a status: 0 = success, negative = error (wcn_status_string());
- *   - conditions only the device can see (probe limit of the coordinate table exceeded,
+ *   - conditions only the device can see (a bin of the coordinate table with more blocks than slots,
  *     coordinate range too wide to pack, more than 2^31-1 pairs) are recorded in the table
  *     header / result block and surface through wcn_kmap_read_result(), wcn_table_read_status();
  *   - coordinates are rows [batch, x, y, z] of int32; index outputs are int32, bit-exact with the
@@ -50,7 +51,7 @@ extern "C" {
 #define WCN_OK 0
 #define WCN_ERR_INVALID_ARGUMENT (-1)  /* null pointer, bad size, unsupported dtype ...        */
 #define WCN_ERR_LAUNCH (-2)            /* the HIP runtime refused a launch or a copy           */
-#define WCN_ERR_TABLE_OVERFLOW (-3)    /* probe limit exceeded: rebuild with a larger capacity */
+#define WCN_ERR_TABLE_OVERFLOW (-3)    /* a bin has more blocks than slots: rebuild with a larger capacity (of use up to 2^26) */
 #define WCN_ERR_COORD_RANGE (-4)       /* bounding box of the keys cannot be packed in 63 bits */
 #define WCN_ERR_TOO_MANY_PAIRS (-5)    /* kernel map would hold more than 2^31-1 pairs         */
 #define WCN_ERR_WORKSPACE (-6)         /* workspace smaller than the *_bytes() query demands   */

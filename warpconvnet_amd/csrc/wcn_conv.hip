@@ -1450,10 +1450,11 @@ size_t wcn_conv_prepared_workspace_bytes(int64_t num_out, int32_t num_offsets, i
 // pair-packed one.  Where a tile plan could be taken the pairs decide (nearly all that the kernel for wide rows takes is among that),
 // and slices of channels over workgroups would need a workspace.  What a layer gains is the host's time between the map's
 // last kernel and its own launch, whatever its size.  us of a call that makes its map, launched behind the wait / ahead of it:
-//     3x3x3  32 -> 64 fp16,   1,800 voxels     67 / 59     (small maps)
-//     3x3x3  32 -> 32 fp32, 100,000 voxels    108 / 100    (pair-packed)
-//     3x3x3, stride 2, 16 -> 13 fp32, 456,000 178 / 174    (narrow)
-//     a training step over 24,000 voxels      610 / 565    (three layers, `graph`)
+//     3x3x3  32 -> 64 fp16,   1,800 voxels     71 / 63     (small maps)
+//     3x3x3  32 -> 32 fp32, 100,000 voxels    102 / 94     (pair-packed)
+//     3x3x3, stride 2, 16 -> 13 fp32, 456,000 173 / 168    (narrow)
+// (two runs of one side differ by 3 to 8 %.  A U-Net over 60,000 voxels 1,277 / 1,229 and, with `graph`, a training step over 24,000
+// voxels 588 / 519, of which runs differ by 6 and 17 %.)
 // graph: never the kernel for small maps, whose order of sums depends on the size of the map (see conv_run).
 static int ahead_half(int32_t dtype, int32_t num_offsets, int32_t c_in, int32_t c_out, int64_t num_in, int64_t num_out,
                       int64_t pair_capacity, bool graph) {

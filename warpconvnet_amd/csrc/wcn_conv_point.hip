@@ -202,11 +202,15 @@ extern "C" {
 
 // 16-bit rows, whole 16-byte vectors on both sides, of 32 to 96 channels, 128, 192 or 256, whose weight fits twice into the LDS of
 // a CU.  Up to 96 channels on both sides whatever the number of rows, wider ones up to 32,768 rows and from 100,000 on.  Between
-// the two a weight of 16 KB and more is as long on its way into every workgroup's LDS as the library takes for all of it, and the
-// GPU is what such a call waits for.  Below them both take less time than the host needs for a layer, so the host's part decides:
-// around a library product called from Python the GPU stands idle for 56 to 75 us.  A U-Net over one scan of 120,000 points, which
-// has two such layers: 1,340 us with the library's product, 1,272 with this one.  us on the GPU here / the library's matrix product,
-// bf16:
+// the two a weight of 16 KB and more is as long on its way into every workgroup's LDS as the library takes for all of it, and where the
+// GPU is what a network waits for the library's product is the one that is 1 to 6 us shorter.  Where the host is, this one is, at any
+// size: a library product is called through Python.  us of a layer with a bias called alone, bf16, here / by the library's product:
+//     rows            1,000        30,000       60,000       90,000
+//     128 -> 64      20 / 36      20 / 38      22 / 38      26 / 47
+//     128 -> 128     21 / 36      22 / 37      26 / 40      30 / 51
+//     256 -> 128     21 / 36      27 / 38      32 / 42      37 / 56
+// (A U-Net over 60,000 voxels, with two such layers of fewer than 32,768 rows: 1,267 / 1,385 us,
+// of which two runs of one side differ by 9 %.)  us on the GPU here / the library's matrix product, bf16:
 //     rows      32->32      64->32      64->64      96->96      128->64     128->128    192->96     256->128
 //      1,000    3 /   4     3 /  4      4 /   4     5 /   5     5 /   4     7 /   5     6 /   6     8 /   6
 //     30,000    4 /  22     4 /  6      5 /  19     6 /  27     6 /   8     8 /   7     9 /  12    13 /   9

@@ -557,11 +557,12 @@ __global__ void __launch_bounds__(1024, TWO ? 8 : 4) table_bins(WcnTableHeader* 
 }
 
 // ---- few keys -----------------------------------------------------------------------------------
-// The passes above are a chain of four launches of about five microseconds each, whatever there is to
-// do in them.  Up to SMALL_KEYS keys every workgroup of the last pass reads all of them (a quarter of a megabyte at
-// the most, out of its die's L2): it finds the box, lists the rows of its own bin and counts those of the bins before it.
-// Over 2 k keys 18.1 us and four launches before, 14.3 and two this way while the slots had to be cleared in a launch before it
-// (layer 78.4 -> 75.4 us, a U-Net over 60 k voxels 1522 -> 1499), one launch now.
+// Of few keys the two launches above are mostly start, end and the wait between them.  Up to SMALL_KEYS keys one launch does both:
+// every workgroup reads all of them (a quarter of a megabyte at the most, out of its die's L2), finds the box, lists the rows of its
+// own bin and counts those of the bins before it.  What each reads grows with the keys, and the list takes LDS.  us of a build,
+// spheres, two launches / one:
+//     keys        500         2,000        8,000        12,000       16,384       20,000       24,000       30,000
+//             14.0 /  9.1  14.7 / 10.1  15.6 / 11.9  15.9 / 13.4  16.9 / 15.4  17.8 / 17.1  18.6 / 18.9  19.7 / 22.7
 constexpr int64_t SMALL_KEYS = 16384;
 constexpr int SMALL_KEY_BINS = 64;  // more bins (a table that was grown) would read the keys too often
 
@@ -1021,7 +1022,7 @@ const char* wcn_status_string(int status) {
     case WCN_OK: return "success";
     case WCN_ERR_INVALID_ARGUMENT: return "invalid argument";
     case WCN_ERR_LAUNCH: return "HIP launch or copy failed";
-    case WCN_ERR_TABLE_OVERFLOW: return "coordinate table probe limit exceeded (capacity too small)";
+    case WCN_ERR_TABLE_OVERFLOW: return "a bin of the coordinate table holds more blocks than it has slots (capacity too small)";
     case WCN_ERR_COORD_RANGE: return "coordinate bounding box does not fit the 63-bit block key";
     case WCN_ERR_TOO_MANY_PAIRS: return "kernel map exceeds 2^31-1 pairs";
     case WCN_ERR_WORKSPACE: return "workspace too small";
@@ -1030,9 +1031,9 @@ const char* wcn_status_string(int status) {
 }
 
 int64_t wcn_table_default_capacity(int64_t n_keys) {
-  // Blocks hold up to 64 voxels; surface-like data fills ~10 per block.  One slot per two keys
-  // keeps the load factor under 0.5 unless almost every voxel is alone in its block, in which
-  // case the build reports WCN_ERR_TABLE_OVERFLOW and the caller retries with 4x the slots.
+  // Blocks hold up to 64 voxels; surface-like data fills ~10 per block.  The power of two above the key count makes bins of one
+  // to two thousand keys (2,048 slots each): a bin overflows only where almost every voxel is alone in its block and more than
+  // the average falls to it; the build then reports WCN_ERR_TABLE_OVERFLOW and the caller retries with 4x the slots.
   int64_t want = n_keys + 1;
   int64_t cap = 1024;
   while (cap < want) cap <<= 1;
