@@ -244,3 +244,36 @@ def test_maps_whose_head_lies_apart(monkeypatch, n, kernel, stride, dilation, sh
     assert torch.equal(got.offsets, want.offsets) and torch.equal(got._device_offsets, want._device_offsets)
     starts = 4 * len(want) * ((n + 63) // 64 + 1)
     assert torch.equal(got._group_start[0][:starts], want._group_start[0][:starts])
+
+
+@pytest.mark.parametrize("since", ["cells", "count", "stride", "release"])
+def test_the_event_of_a_map_is_not_that_of_a_later_call(since):
+    """wcn_kmap_take_event is asked after the same thread has made something else: the event is behind that by then, maybe on
+    another stream, and none is handed out."""
+    from warpconvnet_amd._lib import check, int3, lib, ptr, stream_ptr, workspace
+    from warpconvnet_amd.geometry.coords.search.torch_hashmap import TorchHashTable
+    dev, L = torch.device(DEV), lib()
+    rows = torch.as_tensor(_cube(9), device=DEV)
+    n, s = len(rows), stream_ptr(dev)
+    table, _, slots = TorchHashTable.from_keys(rows)._raw()
+    k3, one, two, three = (int3((v,) * 3) for v in (3, 1, 2, 3))
+    ws, other = (workspace(max(L.wcn_kmap_workspace_bytes(n, 27), L.wcn_stride_unique_workspace_bytes(n, slots),
+                               L.wcn_stride_unique_cells_workspace_bytes(n)), dev) for _ in range(2))
+    ins, outs = (torch.empty(27 * n, dtype=torch.int32, device=DEV) for _ in range(2))
+    out, first = torch.empty(n, 4, dtype=torch.int32, device=DEV), torch.empty(n, dtype=torch.int32, device=DEV)
+    offsets, got = (ctypes.c_int64 * 28)(), ctypes.c_int64(0)
+    check(L.wcn_kmap_count_fill(ptr(table), n, slots, ptr(rows), n, k3, one, None, None, ptr(ws), 27 * n, ptr(ins), ptr(outs), s), "fill")
+    check(L.wcn_kmap_read_result(ptr(ws), n, 27, offsets, s), "read")
+    if since == "cells":
+        check(L.wcn_stride_unique_cells(ptr(table), n, slots, ptr(rows), two, ptr(other), ptr(out), ptr(first), s), "cells")
+        check(L.wcn_stride_unique_read_count(ptr(other), n, slots, ctypes.byref(got), s), "read")
+    elif since == "count":
+        check(L.wcn_kmap_count(ptr(table), n, slots, ptr(rows), n, k3, one, ptr(other), s), "count")
+        check(L.wcn_kmap_read_result(ptr(other), n, 27, offsets, s), "read")
+    elif since == "stride":
+        check(L.wcn_stride_unique(ptr(rows), n, three, ptr(other), slots, ptr(out), ptr(first), s), "stride")
+        check(L.wcn_stride_unique_read_count(ptr(other), n, slots, ctypes.byref(got), s), "read")
+    else:
+        torch.cuda.synchronize()
+        check(L.wcn_thread_release(), "release")
+    assert not L.wcn_kmap_take_event(ptr(ws))

@@ -1645,6 +1645,7 @@ static thread_local const void* g_filled = nullptr;  // the result block of such
 
 static void set_pending(Pending kind, int64_t sequence, const void* result) {
   g_pending = {sequence != 0 ? kind : Pending::none, sequence, result};
+  g_filled = nullptr;  // (the event is about to be another call's)
 }
 
 // The sequence of the mailbox write behind a result block, which is then collected; 0 if there is none.
