@@ -64,7 +64,8 @@ extern "C" {
 int wcn_version(void);
 
 /* Frees the calling thread's pinned staging buffers and events (see the conventions above); they
- * come back on the thread's next *_read_* call.  No counterpart in the reference. */
+ * come back on the thread's next *_read_* call.  The events of maps that have been handed back go too.  No counterpart in the
+ * reference. */
 int wcn_thread_release(void);
 
 /* Text for a status code; replaces gemm_status_to_string (warpconvnet_pybind.cpp:1207-1226). */
@@ -170,10 +171,15 @@ int wcn_kmap_count_fill(const void* table, int64_t n_keys, int64_t capacity, con
 
 /* An event (hipEvent_t, without timing) behind the kernels of this host thread's last wcn_kmap_count_fill(_apart), once its result
  * has been read from the same workspace (head): what work on another stream than the builder's has to wait for before it reads
- * lists or group starts.  The caller's to destroy; asked for at most once.  Null where there is none (the result came the slow way,
+ * lists or group starts.  Asked for at most once; the caller hands it back with the device that it is told (wcn_kmap_return_event), or
+ * destroys it.  Null where there is none (the result came the slow way,
  * another call on this thread since): then an event recorded on the builder's stream now serves, as it does behind a wcn_kmap_fill
  * that followed. */
-void* wcn_kmap_take_event(const void* workspace);
+void* wcn_kmap_take_event(const void* workspace, int32_t* device);
+
+/* Takes an event of wcn_kmap_take_event back, on any thread, for the maps to come: up to 64 of a device are kept by the process until
+ * they are used again or a thread calls wcn_thread_release. */
+void wcn_kmap_return_event(void* event, int32_t device);
 
 /* wcn_kmap_count_fill and the wcn_kmap_fill that may follow with the workspace in two pieces: `head`, the first
  * wcn_kmap_head_bytes of it (offsets, status and group starts: what wcn_kmap_read_result and wcn_kmap_group_start are given, and what

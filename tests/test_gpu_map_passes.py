@@ -276,4 +276,43 @@ def test_the_event_of_a_map_is_not_that_of_a_later_call(since):
     else:
         torch.cuda.synchronize()
         check(L.wcn_thread_release(), "release")
-    assert not L.wcn_kmap_take_event(ptr(ws))
+    device = ctypes.c_int32(-1)
+    assert not L.wcn_kmap_take_event(ptr(ws), ctypes.byref(device)) and device.value == -1
+
+
+def test_the_events_of_maps_are_handed_back():
+    """As many events as maps are alive; what is handed back, on whichever thread, is used again; a bounded number is kept."""
+    import threading
+
+    from warpconvnet_amd._lib import check, int3, lib, ptr, stream_ptr, workspace
+    from warpconvnet_amd.geometry.coords.search.torch_hashmap import TorchHashTable
+    dev, L = torch.device(DEV), lib()
+    rows = torch.as_tensor(_cube(9), device=DEV)
+    n, s = len(rows), stream_ptr(dev)
+    table, _, slots = TorchHashTable.from_keys(rows)._raw()
+    k3, one = int3((3, 3, 3)), int3((1, 1, 1))
+    ws = workspace(L.wcn_kmap_workspace_bytes(n, 27), dev)
+    ins, outs = (torch.empty(27 * n, dtype=torch.int32, device=DEV) for _ in range(2))
+    offsets, device = (ctypes.c_int64 * 28)(), ctypes.c_int32(-1)
+
+    def event():
+        check(L.wcn_kmap_count_fill(ptr(table), n, slots, ptr(rows), n, k3, one, None, None, ptr(ws), 27 * n, ptr(ins), ptr(outs), s),
+              "fill")
+        check(L.wcn_kmap_read_result(ptr(ws), n, 27, offsets, s), "read")
+        taken = L.wcn_kmap_take_event(ptr(ws), ctypes.byref(device))
+        assert taken and device.value == dev.index and not L.wcn_kmap_take_event(ptr(ws), ctypes.byref(device))
+        return taken
+
+    torch.cuda.synchronize()
+    check(L.wcn_thread_release(), "release")  # none are kept
+    alive = [event() for _ in range(100)]
+    assert len(set(alive)) == 100
+    other = threading.Thread(target=lambda: [L.wcn_kmap_return_event(e, dev.index) for e in alive])
+    other.start()
+    other.join()
+    again = [event() for _ in range(64)]
+    assert set(again) == set(alive[:64])  # the other 36 were destroyed
+    for e in again:
+        L.wcn_kmap_return_event(e, dev.index)
+    torch.cuda.synchronize()
+    check(L.wcn_thread_release(), "release")

@@ -31,7 +31,8 @@ SIGNATURES = {
     "wcn_kmap_count_dilated": (ctypes.c_int, [_vp, _i64, _i64, _vp, _i64, _i32p, _i32p, _i32p, _i32p, _vp, _vp]),
     "wcn_kmap_read_result": (ctypes.c_int, [_vp, _i64, _i32, _i64p, _vp]),
     "wcn_kmap_count_fill": (ctypes.c_int, [_vp, _i64, _i64, _vp, _i64, _i32p, _i32p, _i32p, _i32p, _vp, _i64, _vp, _vp, _vp]),
-    "wcn_kmap_take_event": (_vp, [_vp]),
+    "wcn_kmap_take_event": (_vp, [_vp, _i32p]),
+    "wcn_kmap_return_event": (None, [_vp, _i32]),
     "wcn_kmap_head_bytes": (_sz, [_i64, _i32]),
     "wcn_kmap_count_fill_apart": (ctypes.c_int, [_vp, _i64, _i64, _vp, _i64, _i32p, _i32p, _i32p, _i32p, _vp, _vp, _i64, _vp, _vp,
                                                  _vp]),

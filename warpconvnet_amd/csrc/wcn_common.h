@@ -371,7 +371,7 @@ int wcn_read_early_end(void* host_dst, const void* device_src, size_t bytes, hip
 // waits for `done` in any case (the kernel writes more than the mailbox, and the caller takes it for written).
 int wcn_mailbox_begin(int64_t** device_visible_box, int64_t* sequence);
 int wcn_mailbox_mark(hipStream_t stream);  // records `done` behind the writing kernel (and what was enqueued behind that)
-void* wcn_mailbox_take_event();            // `done` of a write that has been collected, to be destroyed by the caller; or null
+void* wcn_mailbox_take_event(int32_t* device);  // `done` of a write that has been collected, the caller's from there on; or null
 int wcn_mailbox_end(void* host_dst, size_t payload_bytes, int64_t sequence, bool kernel_over = false);
 
 // Output-row form of a pair list (rows of the map grouped by output row, inside a row ascending

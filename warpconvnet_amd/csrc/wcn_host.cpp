@@ -71,7 +71,8 @@ Tensor bytes_on(size_t n, const Tensor& like) {
 struct MadeOn {
   void* stream;
   hipEvent_t event = nullptr;
-  MadeOn(void* s, void* recorded) : stream(s), event(static_cast<hipEvent_t>(recorded)) {}
+  int32_t lent = -1;  // the device of an event that goes back to the map builder's
+  MadeOn(void* s, void* recorded, int32_t device) : stream(s), event(static_cast<hipEvent_t>(recorded)), lent(device) {}
   explicit MadeOn(void* s) : stream(s) {
     if (hipEventCreateWithFlags(&event, hipEventDisableTiming) != hipSuccess ||
         hipEventRecord(event, static_cast<hipStream_t>(s)) != hipSuccess) {
@@ -81,7 +82,8 @@ struct MadeOn {
   }
   MadeOn(const MadeOn&) = delete;
   ~MadeOn() {
-    if (event) (void)hipEventDestroy(event);
+    if (lent >= 0) wcn_kmap_return_event(event, lent);
+    else if (event) (void)hipEventDestroy(event);
   }
 
   static bool capturing(void* s) {
@@ -327,8 +329,9 @@ py::tuple kernel_map(const py::object& table, const Tensor& out4, const Int3& ks
     } else {
       in_buf = in_buf.narrow(0, 0, total);
       out_buf = out_buf.narrow(0, 0, total);
-      void* const behind = wcn_kmap_take_event(w);
-      made = behind ? std::make_shared<MadeOn>(stream, behind) : std::make_shared<MadeOn>(stream);
+      int32_t device = -1;
+      void* const behind = wcn_kmap_take_event(w, &device);
+      made = behind ? std::make_shared<MadeOn>(stream, behind, device) : std::make_shared<MadeOn>(stream);
     }
     break;
   }

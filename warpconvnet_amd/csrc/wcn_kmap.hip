@@ -1716,10 +1716,10 @@ static int kmap_count_impl(const void* table, int64_t n_keys, int64_t capacity, 
   return emitted ? WCN_OK : WCN_ERR_LAUNCH;
 }
 
-void* wcn_kmap_take_event(const void* workspace) {
-  if (!workspace || g_filled != workspace) return nullptr;
+void* wcn_kmap_take_event(const void* workspace, int32_t* device) {
+  if (!workspace || !device || g_filled != workspace) return nullptr;
   g_filled = nullptr;
-  return wcn_mailbox_take_event();
+  return wcn_mailbox_take_event(device);
 }
 
 int wcn_kmap_count_fill(const void* table, int64_t n_keys, int64_t capacity, const int32_t* out_coords, int64_t num_out,

@@ -24,6 +24,7 @@
 #include <mutex>
 #include <thread>
 #include <type_traits>
+#include <vector>
 
 #include <algorithm>
 
@@ -912,6 +913,30 @@ int wcn_read_early_end(void* host_dst, const void* device_src, size_t bytes, hip
 }
 
 namespace {
+// Events that maps have given back, by device, for the mailbox writes to come: created and destroyed with every map they took
+// 2 us of the host.  An event may be recorded again while an earlier record is still waited for: the wait is for that one.
+constexpr size_t kIdleEvents = 64;  // of a device; more are destroyed
+struct IdleEvents {
+  std::mutex mu;
+  std::vector<hipEvent_t> of[64];
+};
+IdleEvents& idle_events() {
+  static IdleEvents* const pool = new IdleEvents;  // (never destroyed: maps may outlive static objects)
+  return *pool;
+}
+hipError_t event_for(int device, hipEvent_t* event) {
+  if (device >= 0 && device < 64) {
+    IdleEvents& pool = idle_events();
+    std::lock_guard<std::mutex> hold(pool.mu);
+    if (!pool.of[device].empty()) {
+      *event = pool.of[device].back();
+      pool.of[device].pop_back();
+      return hipSuccess;
+    }
+  }
+  return hipEventCreateWithFlags(event, hipEventDisableTiming);
+}
+
 constexpr size_t kMailboxBytes = 16384;
 thread_local int64_t* g_box = nullptr;        // pinned, coherent, mapped
 thread_local hipEvent_t g_box_done = nullptr;
@@ -941,7 +966,7 @@ int wcn_mailbox_begin(int64_t** device_visible_box, int64_t* sequence) {
   }
   if (!g_box_done || g_box_device != device) {
     if (g_box_done) (void)hipEventDestroy(g_box_done);
-    if (hipEventCreateWithFlags(&g_box_done, hipEventDisableTiming) != hipSuccess) {
+    if (event_for(device, &g_box_done) != hipSuccess) {
       g_box_done = nullptr;
       return WCN_ERR_LAUNCH;
     }
@@ -983,10 +1008,11 @@ int wcn_mailbox_end(void* host_dst, size_t payload_bytes, int64_t sequence, bool
 }
 
 // The event behind the thread's last write, which has been collected, is the caller's from here on (the next write gets another).
-void* wcn_mailbox_take_event() {
+void* wcn_mailbox_take_event(int32_t* device) {
   if (g_box_open != 0) return nullptr;
   void* const event = (void*)g_box_done;
   g_box_done = nullptr;
+  *device = g_box_device;
   return event;
 }
 
@@ -1000,8 +1026,30 @@ extern "C" {
 
 int wcn_version(void) { return 200; }
 
+void wcn_kmap_return_event(void* event, int32_t device) {
+  if (!event) return;
+  if (device >= 0 && device < 64) {
+    IdleEvents& pool = idle_events();
+    std::lock_guard<std::mutex> hold(pool.mu);
+    if (pool.of[device].size() < kIdleEvents) {
+      pool.of[device].push_back((hipEvent_t)event);
+      return;
+    }
+  }
+  (void)hipEventDestroy((hipEvent_t)event);
+}
+
 int wcn_thread_release(void) {
   int st = WCN_OK;
+  {
+    IdleEvents& pool = idle_events();
+    std::lock_guard<std::mutex> hold(pool.mu);
+    for (auto& events : pool.of) {
+      for (hipEvent_t e : events)
+        if (hipEventDestroy(e) != hipSuccess) st = WCN_ERR_LAUNCH;
+      events.clear();
+    }
+  }
   if (g_small_done && hipEventDestroy(g_small_done) != hipSuccess) st = WCN_ERR_LAUNCH;
   if (g_early_done && hipEventDestroy(g_early_done) != hipSuccess) st = WCN_ERR_LAUNCH;
   if (g_box_done && hipEventDestroy(g_box_done) != hipSuccess) st = WCN_ERR_LAUNCH;

@@ -96,7 +96,9 @@ def _kernel_map_from_table(table: TorchHashTable, out_coords: Tensor, kernel_siz
     plain = (tuple(ks), tuple(st))
     kind = plain if dil is None else plain + (tuple(dil), tuple(centre))
     size, octave = kind + ((M ** 4).bit_length(),), kind + (-M.bit_length(),)
-    per_row = _PAIRS_PER_ROW.get(size, _PAIRS_PER_ROW.get(octave, _PAIRS_PER_ROW.get(plain + octave[-1:], 8.0)))
+    per_row = _PAIRS_PER_ROW.get(size)
+    if per_row is None:
+        per_row = _PAIRS_PER_ROW.get(octave, _PAIRS_PER_ROW.get(plain + octave[-1:], 8.0))
     in_maps, out_maps, offsets64, offsets, groups, address, device_offsets, flags, made = native().kernel_map(
         table, out4, ks, st, dil, centre, per_row, _KEEP_WORKSPACE_BYTES, ahead)
     if M > 0:
